@@ -26,11 +26,12 @@ constexpr int kCompactR = 8;   // 16-byte pieces each thread gathers per round
 #define ZP_SPLIT_ROWS 1024
 #endif
 constexpr int kSplitKvRows = ZP_SPLIT_ROWS;   // up to this many (layer, sequence, head) rows K and V get workgroups of their own
+constexpr int kWideThreads = 1024;            // of a workgroup where rows are few, see wide_parts
 // native vector types keep the staged pieces in VGPRs
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-__device__ __forceinline__ int block_exclusive_scan(int v, int* total, int* lds) {
+template <int NT> __device__ __forceinline__ int block_exclusive_scan(int v, int* total, int* lds) {
   const int lane = lane_id(), w = wave_id();
   int inc = v;
 #pragma unroll
@@ -42,7 +43,7 @@ __device__ __forceinline__ int block_exclusive_scan(int v, int* total, int* lds)
   __syncthreads();
   int woff = 0, tot = 0;
 #pragma unroll
-  for (int i = 0; i < kThreads / 64; ++i) {
+  for (int i = 0; i < NT / 64; ++i) {
     int c = lds[i];
     if (i < w) woff += c;
     tot += c;
@@ -75,6 +76,9 @@ struct CompactArgs {
   // !HAS_B with split_kv: the grid is twice n_items; workgroups n_items .. 2 n_items - 1 move
   // `b` (the values) with the same list, the first n_items move `a` (and the carried scores)
   int split_kv;
+  // wide form: a row's vectors are cut into `parts` column ranges of lpv pieces, each moved by a
+  // workgroup of its own (a byte only ever meets bytes of its own column, so parts need no order)
+  int parts;
 };
 
 // Survivors are written once and not read again by this kernel: non-temporal stores keep them
@@ -84,10 +88,12 @@ struct CompactArgs {
 #define ZP_NT_STORE(v, ptr) __builtin_nontemporal_store(v, ptr)
 // POW2: page size and pieces-per-vector are powers of two, so every index split is a shift.
 // CES: bytes of a carried-score element moved along with K and V by the same survivor list (0: none).
-template <typename P, int R, bool HAS_B, bool POW2, int CES = 0>
-__global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
+// NT: threads of a workgroup.
+template <typename P, int R, bool HAS_B, bool POW2, int CES = 0, int NT = kThreads>
+__global__ __launch_bounds__(NT) void compact_kernel(CompactArgs p) {
+  constexpr bool kWide = NT != kThreads;
   extern __shared__ __align__(16) char smem[];
-  __shared__ int scan_lds[kThreads / 64];
+  __shared__ int scan_lds[NT / 64];
   const int T = p.NB * p.BS;
   uint16_t* list = (uint16_t*)smem;
   int* tab = (int*)(smem + (((size_t)T * 2 + 15) & ~(size_t)15));
@@ -98,33 +104,35 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
   // works on one head's 256-byte slice of the token rows.  Measured against giving each XCD a
   // contiguous range of items (all heads of a sequence on one XCD: 2.5 % slower) and against
   // rotating the head index by the sequence index (4 % slower), inside one allocation.
-  const int which = (!HAS_B && p.split_kv && (int)blockIdx.x >= p.n_items) ? 1 : 0;
-  const int item = (int)blockIdx.x - which * p.n_items;
+  const int part = kWide ? (int)blockIdx.x % p.parts : 0;
+  const int unit = kWide ? (int)blockIdx.x / p.parts : (int)blockIdx.x;
+  const int which = (!HAS_B && p.split_kv && unit >= p.n_items) ? 1 : 0;
+  const int item = unit - which * p.n_items;
   if (item >= p.n_items) return;
   const int h = item % p.Hkv;
   const int b = (item / p.Hkv) % p.B;
   const int l = item / (p.Hkv * p.B);
 
-  for (int i = tid; i < p.NB; i += kThreads) {
+  for (int i = tid; i < p.NB; i += NT) {
     int code = p.table[(int64_t)b * p.NB + i];
     int pid = page_is_pad(code) ? -1 : page_id(code);
     tab[i] = (pid >= 0 && pid < p.num_pages) ? pid : -1;
   }
-  for (int i = tid; i < p.target_width; i += kThreads) {
+  for (int i = tid; i < p.target_width; i += NT) {
     int t = p.target[(int64_t)b * p.target_width + i];
     tgt[i] = (t >= 0 && t < p.num_pages) ? t : -1;
   }
   __syncthreads();
 
   // ---- phase 1: ordered survivor list
-  const int chunk = (T + kThreads - 1) / kThreads;
+  const int chunk = (T + NT - 1) / NT;
   const int s0 = min(tid * chunk, T), s1 = min(s0 + chunk, T);
   const uint8_t* f = p.flag + (((int64_t)l * p.B + b) * p.Hkv + h) * (int64_t)T;
   int cnt = 0;
   auto page_of = [&](int s) { return POW2 ? (s >> p.bs_shift) : (s / p.BS); };
   for (int s = s0; s < s1; ++s) cnt += (f[s] != 0 && tab[page_of(s)] >= 0) ? 1 : 0;
   int total;
-  int off = block_exclusive_scan(cnt, &total, scan_lds);
+  int off = block_exclusive_scan<NT>(cnt, &total, scan_lds);
   for (int s = s0; s < s1; ++s)
     if (f[s] != 0 && tab[page_of(s)] >= 0) list[off++] = (uint16_t)s;
   __syncthreads();
@@ -135,14 +143,15 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
   const int units = total * p.lpv;
   char* abase = which ? p.b + l * p.b_sl + h * p.b_sh : p.a + l * p.a_sl + h * p.a_sh;
   char* bbase = HAS_B ? p.b + l * p.b_sl + h * p.b_sh : nullptr;
+  if (kWide) abase += part * p.lpv * (int)sizeof(P);
   const int64_t a_sp = which ? p.b_sp : p.a_sp, a_ss = which ? p.b_ss : p.a_ss;
-  for (int base = 0; base < units; base += kThreads * R) {
+  for (int base = 0; base < units; base += NT * R) {
     P ra[R];
     P rb[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) {
       // out-of-range units re-load the last valid piece (never stored): no predicated loads
-      const int u = min(base + r * kThreads + tid, units - 1);
+      const int u = min(base + r * NT + tid, units - 1);
       const int i = POW2 ? (u >> p.lpv_shift) : (u / p.lpv), piece = u - i * p.lpv;
       const int s = list[i];
       const int j = page_of(s), slot = s - j * p.BS;
@@ -158,7 +167,7 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < R; ++r) {
-      const int u = base + r * kThreads + tid;
+      const int u = base + r * NT + tid;
       if (u < units) {
         const int i = POW2 ? (u >> p.lpv_shift) : (u / p.lpv), piece = u - i * p.lpv;
         const int j = page_of(i), slot = i - j * p.BS;
@@ -171,17 +180,17 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
       }
     }
   }
-  if (CES != 0 && which == 0) {
+  if (CES != 0 && which == 0 && part == 0) {
     // the carried score of every survivor follows its key: same list, same gather -> barrier ->
     // scatter rounds (the score cache aliases its own targets exactly as the key cache does)
     typedef typename std::conditional<CES == 4, uint32_t, uint16_t>::type E;
     constexpr int RC = 4;
     char* cbase = p.c + l * p.c_sl + h * p.c_sh;
-    for (int base = 0; base < total; base += kThreads * RC) {
+    for (int base = 0; base < total; base += NT * RC) {
       E rc[RC];
 #pragma unroll
       for (int r = 0; r < RC; ++r) {
-        const int s = list[min(base + r * kThreads + tid, total - 1)];
+        const int s = list[min(base + r * NT + tid, total - 1)];
         if (p.c_rows) {
           rc[r] = *(const E*)(p.c_rows + ((int64_t)item * T + s) * CES);
         } else {
@@ -193,7 +202,7 @@ __global__ __launch_bounds__(kThreads) void compact_kernel(CompactArgs p) {
       __syncthreads();
 #pragma unroll
       for (int r = 0; r < RC; ++r) {
-        const int i = base + r * kThreads + tid;
+        const int i = base + r * NT + tid;
         if (i < total) {
           const int j = page_of(i), slot = i - j * p.BS;
           const int64_t pid = tgt[j];
@@ -211,21 +220,21 @@ static int log2_exact(int v) {
   return s;
 }
 
-template <typename P, int R, bool HAS_B, bool POW2, int CES = 0>
+template <typename P, int R, bool HAS_B, bool POW2, int CES = 0, int NT = kThreads>
 int launch_compact_impl(CompactArgs a, int L, hipStream_t st) {
   a.n_items = L * a.B * a.Hkv;
   const int T = a.NB * a.BS;
   size_t smem = (((size_t)T * 2 + 15) & ~(size_t)15) + sizeof(int) * (a.NB + a.target_width);
-  dim3 grid((unsigned)((int64_t)L * a.B * a.Hkv * (!HAS_B && a.split_kv ? 2 : 1)));
+  dim3 grid((unsigned)((int64_t)L * a.B * a.Hkv * (!HAS_B && a.split_kv ? 2 : 1) * (NT != kThreads ? a.parts : 1)));
   if (smem > 64 * 1024) {
-    hipError_t e = hipFuncSetAttribute((const void*)compact_kernel<P, R, HAS_B, POW2, CES>,
+    hipError_t e = hipFuncSetAttribute((const void*)compact_kernel<P, R, HAS_B, POW2, CES, NT>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     if (e != hipSuccess) {
       zp_set_error("compaction: cannot reserve %zu bytes of LDS: %s", smem, hipGetErrorString(e));
       return ZP_EHIP;
     }
   }
-  hipLaunchKernelGGL((compact_kernel<P, R, HAS_B, POW2, CES>), grid, dim3(kThreads), smem, st, a);
+  hipLaunchKernelGGL((compact_kernel<P, R, HAS_B, POW2, CES, NT>), grid, dim3(NT), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -239,6 +248,21 @@ int launch_compact(CompactArgs a, int L, hipStream_t st) {
 }
 
 inline bool aligned_to(int64_t v, int n) { return (v % n) == 0; }
+
+// Few rows leave most of the chip idle, and a row is a chain of rounds (2 048 fp32 vectors of one tensor: sixteen
+// of 64 KB).  So up to kWideUnits (row, tensor) pairs get workgroups of sixteen waves, and a pair is cut into column
+// ranges of at least a cache line while that leaves at most one workgroup per CU.  Whole steps of one layer, general
+// -> wide form: 1 fp32 sequence of 8 heads 110 -> 59 us, 8 of them 130 -> 99, 32 of them (512 pairs) 323 -> 314; 1
+// bfloat16 sequence 64 -> 42, 16 of them 101 -> 91, 32 of them 171 -> 163.  At 1 024 pairs the general form has four
+// workgroups per CU and the wide one is within 1 % either way; cutting beyond 256 workgroups loses 1-3 %.
+// Returns the column ranges, 0: the general form.
+constexpr int kWideUnits = 512, kWideGrid = 256, kLinePieces = 8;
+inline int wide_parts(int64_t pairs, int lpv) {
+  if (pairs > kWideUnits) return 0;
+  int parts = 1;
+  while (pairs * parts * 2 <= kWideGrid && lpv % (parts * 2 * kLinePieces) == 0) parts *= 2;
+  return parts;
+}
 
 // ------------------------------------------------------------------ query ring store
 template <typename P>
@@ -303,10 +327,23 @@ int compress_kv_impl(void* key, void* value, const uint8_t* flag, const int32_t*
   ZP_REQUIRE((int64_t)target_width * BS * a.lpv < (int64_t)1 << 31, "compress_kv: row too large");
   hipStream_t st = (hipStream_t)stream;
   a.split_kv = 0;
+  a.parts = 1;
   // few rows: keys and values go to workgroups of their own (twice the workgroups per CU to hide
   // the gather's latency: 0.340 against 0.347 ms per step at 64 sequences x 8 heads; with many rows
   // the CUs are full either way and one survivor list per row is cheaper)
   const bool split = piece == 16 && (int64_t)L * B * Hkv <= kSplitKvRows;
+  const int parts = piece == 16 && log2_exact(BS) >= 0 && log2_exact(a.lpv) >= 0 ? wide_parts((int64_t)L * B * Hkv * 2, a.lpv) : 0;
+  if (parts) {
+    a.split_kv = 1;
+    a.parts = parts;
+    a.lpv /= parts;
+    a.lpv_shift = log2_exact(a.lpv);
+    a.bs_shift = log2_exact(BS);
+    if (!score_cache || !fused) return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 0, kWideThreads>(a, L, st);
+    *fused = true;
+    if (es == 4) return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 4, kWideThreads>(a, L, st);
+    return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 2, kWideThreads>(a, L, st);
+  }
   switch (piece) {
     case 16:
       if (score_cache && fused) {
@@ -388,6 +425,7 @@ extern "C" int zp_compress_score(void* score_cache, const void* scores_src, cons
   a.b_sl = a.b_sp = a.b_ss = a.b_sh = 0;
   a.c = nullptr; a.c_rows = nullptr; a.c_sl = a.c_sp = a.c_ss = a.c_sh = 0;
   a.split_kv = 0;
+  a.parts = 1;
   hipStream_t st = (hipStream_t)stream;
   if (es == 4) return launch_compact<uint32_t, 4, false>(a, L, st);
   return launch_compact<uint16_t, 4, false>(a, L, st);
