@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64 * NW) void delta_step_kernel(zp_delta a) {
 #pragma unroll
   for (int r = 0; r < RL; ++r) {
     S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (!fresh) S[r] = *(const f32x4*)(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
+    if (!fresh) S[r] = load_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
   }
   if (tid < cw) finish(tid, first);
   if (c2 < cw) finish(c2, second);
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64 * NW) void delta_step_kernel(zp_delta a) {
   for (int r = 0; r < RL; ++r) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) S[r][c] = fmaf(k4[r >> 2][r & 3], u[c], S[r][c]);
-    *(f32x4*)(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col) = S[r];
+    store_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col, S[r]);
   }
   ss = quads_sum(ss);
   if (lane == 0) red[wave] = ss;

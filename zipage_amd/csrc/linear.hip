@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
 #pragma unroll
   for (int r = 0; r < RL; ++r) {
     S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (sg.start > 0) S[r] = *(const f32x4*)(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
+    if (sg.start > 0) S[r] = load_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
   }
   for (int c = tid; c < dk; c += blockDim.x) {
     qs[c] = turned<T>(a, src + a.q_at + h * dk, c, half, sg.start) * a.q_scale;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
         s[c] = fmaf(k4[i], v[c], s[c] * g4[i]);
         o[c] = fmaf(s[c], q4[i], o[c]);
       }
-      *(f32x4*)(state + (int64_t)(at + i) * dv + col) = s;
+      store_once(state + (int64_t)(at + i) * dv + col, s);
     }
   }
   float ss = 0.f;
