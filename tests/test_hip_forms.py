@@ -2,6 +2,8 @@
 import pytest
 import torch
 
+from oracle import kapolorn_oracle as K
+from oracle import rutevik_oracle as R
 from oracle import zipage_oracle as O
 
 pytestmark = pytest.mark.gpu
@@ -39,3 +41,39 @@ def test_compaction_of_few_rows(dev, dtype, L, B, Hkv, D, style):
     compress_kv(gk, gv, flag.to(dev), enc.to(dev), target.to(dev))
     assert torch.equal(gk.cpu().view(torch.uint8), wk.view(torch.uint8))
     assert torch.equal(gv.cpu().view(torch.uint8), wv.view(torch.uint8))
+
+
+# ------------------------------------------------------------------ experts
+# rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup when
+# there are many; 256-row tiles are worked off whole from a contraction of 2048 on, in two halves below it.  Odd
+# numbers of steps, results that end inside a workgroup's columns, and experts without a token are among them.
+@pytest.mark.parametrize("n,width,E,top,ff", [(60, 96, 64, 2, 800), (61, 2080, 64, 2, 544), (1, 4096, 4, 2, 32),
+                                              (260, 160, 4, 1, 288), (1100, 2144, 3, 2, 96), (1100, 96, 2, 1, 2112),
+                                              (1300, 256, 2, 1, 96), (515, 2112, 1, 1, 48)])
+@pytest.mark.parametrize("act", ["clamped", "silu"])
+def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act):
+    from zipage_amd.layers import Experts
+    clamped = act == "clamped"
+    m = Experts(width, E, top, ff, 7.0, shared_ff=ff + 32 if clamped else None, shared_limit=5.0, act=act,
+                score="softmax" if clamped else "sigmoid")
+    w = {k: _rand(*s, seed=i, std=2.0 * s[-1] ** -0.5) for i, (k, s) in enumerate(m.shapes().items())}
+    if E > 2:
+        w["router"][E - 1] = w["router"][0] - 4.0 * w["router"][0].sign()     # hardly anyone's choice
+    m.load(w, BF16, dev)
+    h = torch.zeros(n, m.width_p, dtype=BF16, device=dev)
+    x = _rand(n, width, seed=99)
+    h[:, :width] = x.to(dev)
+    x64, w64 = x.double(), {k: v.double() for k, v in w.items()}
+    z = (x64 @ w64["router"].T).sort(-1, descending=True).values
+    sure = torch.ones(n, dtype=torch.bool) if top == E else z[:, top - 1] - z[:, top] > 1e-3
+    got = m.forward(h).double().sum(0)[:, :width].cpu()
+    groups = {"count": 1, "keep": 1}
+    if clamped:
+        want = K.experts(x64, w64, {"router": {"experts": E, "top": top, "groups": groups}, "expert": {"limit": 7.0},
+                                    "shared": {"limit": 5.0}})
+    else:
+        want = R.experts(x64, w64, {"router": {"experts": E, "top": top}})
+    assert int(sure.sum()) >= 0.8 * n
+    # bf16 activations and planes: each of top + 2 roundings is at most 2^-9 of its own value
+    err = (got - want)[sure].norm() / want[sure].norm()
+    assert float(err) < 2.0 ** -8 and bool(torch.isfinite(got).all())

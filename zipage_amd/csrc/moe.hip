@@ -307,11 +307,17 @@ template <typename T> __device__ __forceinline__ float gated(int act, float w, f
   return w * (g * sigmoid_of<T>(1.702f * g) * (u + 1.f));
 }
 
-// Few rows per expert: the weights are streamed straight into registers.  A workgroup owns 64 rows of W (gate_up:
-// two 16-row tiles of the gate and the two of `up` that belong to them) and up to 16 * MT tokens; its four waves
-// take every fourth step of the contraction and meet in LDS.
-constexpr int kRowsW = 4;                              // 16-row tiles of W
-template <typename T, int MT, bool UP>
+// Few rows per expert: the weights are streamed straight into registers.  A workgroup owns 16 * kRowsW rows of W
+// (gate_up: tiles of the gate and those of `up` that belong to them) and up to 16 * MT tokens; its four waves share
+// the steps of the contraction and meet in LDS.  What the weights' stream loses is what else passes the caches: 16
+// rows of tokens per kRowsW tiles of W, and twice as much where two waves take the two halves of a token's cache line.
+// One token tile (hardly any expert has a second): a wave takes pairs of steps, whole lines of x, and the workgroup
+// 128 rows of W where that leaves two workgroups per CU (64 tokens over 33 experts of 3 x 4096 x 3072: 516 -> 476 us,
+// 5.2 TB/s; with 64 rows 497; a single token, 192 workgroups of 128 rows: 72 against 81).  More token tiles keep 64
+// rows and single steps (256 tokens: 675 us; 687 with pairs, 876 with 128 rows).
+constexpr int kNarrowW = 4, kWideW = 8;                // 16-row tiles of W
+constexpr int kWideGrid = 512;                         // workgroups from which on 128 rows of W are better
+template <typename T, int MT, bool UP, int kRowsW>
 __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
@@ -340,8 +346,7 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   for (int k = 0; k < kRowsW; ++k)
 #pragma unroll
     for (int i = 0; i < MT; ++i) acc[k][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 4
-  for (int ks = wave; ks < steps; ks += 4) {
+  auto step = [&](int ks) {
     u32x4 wf[kRowsW], xf[MT];
 #pragma unroll
     for (int k = 0; k < kRowsW; ++k) {
@@ -355,6 +360,17 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
     for (int k = 0; k < kRowsW; ++k)
 #pragma unroll
       for (int i = 0; i < MT; ++i) acc[k][i] = Mma<T>::go(wf[k], xf[i], acc[k][i]);
+  };
+  if constexpr (MT == 1) {
+#pragma unroll kNarrowW * 2 / kRowsW
+    for (int ks = wave * 2; ks + 1 < steps; ks += 8) {
+      step(ks);
+      step(ks + 1);
+    }
+    if ((steps & 1) && (steps >> 1) % 4 == wave) step(steps - 1);
+  } else {
+#pragma unroll 4
+    for (int ks = wave; ks < steps; ks += 4) step(ks);
   }
 #pragma unroll
   for (int k = 0; k < kRowsW; ++k)
@@ -520,19 +536,23 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
     return ZP_OK;
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
-  const int64_t grid = (int64_t)a.max_tiles * ((Mw + 16 * kRowsW - 1) / (16 * kRowsW));
+  const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
+  const bool wide = rows == 16 && dtype == ZP_BF16 && grid_of(kWideW) >= kWideGrid;
+  const int64_t grid = grid_of(wide ? kWideW : kNarrowW);
   if (grid >= (1ll << 31)) {
     zp_set_error("moe: too many tiles");
     return ZP_EUNSUPPORTED;
   }
-#define ZP_EXPERTS(T, MT) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP>), dim3((unsigned)grid), dim3(256), 0, st, a)
-#define ZP_EXPERT_ROWS(T)                 \
-  do {                                    \
-    if (rows == 16) ZP_EXPERTS(T, 1);     \
-    else if (rows == 32) ZP_EXPERTS(T, 2);\
-    else ZP_EXPERTS(T, 4);                \
+#define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, a)
+#define ZP_EXPERT_ROWS(T)                            \
+  do {                                               \
+    if (rows == 16) ZP_EXPERTS(T, 1, kNarrowW);      \
+    else if (rows == 32) ZP_EXPERTS(T, 2, kNarrowW); \
+    else ZP_EXPERTS(T, 4, kNarrowW);                 \
   } while (0)
-  if (dtype == ZP_BF16) ZP_EXPERT_ROWS(BF16); else ZP_EXPERT_ROWS(F32);
+  if (wide) ZP_EXPERTS(BF16, 1, kWideW);
+  else if (dtype == ZP_BF16) ZP_EXPERT_ROWS(BF16);
+  else ZP_EXPERT_ROWS(F32);
 #undef ZP_EXPERT_ROWS
 #undef ZP_EXPERTS
   ZP_LAUNCH_CHECK();
