@@ -294,6 +294,7 @@ struct ExpertArgs {
   int64_t x_st, o_st, w_expert;   // w_expert: elements between experts
   int act;
   float limit, limit_shared;
+  int split;              // parts in which expert_tiles_kernel takes a tile
 };
 
 // ZP_GATE_CLAMPED: w g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
@@ -404,29 +405,64 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   }
 }
 
-// Many rows per expert: 128 tokens x 256 rows of W per workgroup, both streamed straight into LDS in the
-// order the matrix cores read them, 32 of the contraction at a time, two stages ahead of the products; one
-// barrier per stage.  A wave owns 64 tokens x 128 rows of W.
+// Many rows per expert: 128 or 256 tokens x 256 rows of W per workgroup, 32 of the contraction at a time.  A wave owns
+// 64 rows of W and all tokens.  W is kept in the order in which the matrix cores read it, so a wave's share goes from
+// memory straight into its registers; only tokens, which all four waves read, pass through LDS, by loads of their own;
+// one barrier per stage.  (With W through LDS too, reads and writes of LDS took longer than the products.)
+//   128 tokens: two workgroups per CU hide each other's set-up and results.  Stages are asked for two (W) and three
+//   (tokens) ahead.
+//   256 tokens: half the reads of W per product, one wave per SIMD, four and five stages ahead.  From averages of more
+//   than 512 rows per expert on, and only over long contractions, since nothing hides a workgroup's beginning and end.
+// 16 384 tokens over 33 experts of 3 x 4096 x 3072 (both products, 4.95 TFLOP): 5.66 ms with everything through LDS,
+// 5.36 with 128 tokens, 5.09 with 256; of 3 x 1024 x 768: 488, 473 and 526 us.  6 144 tokens of 4 of 32 large ones:
+// 2.29 ms with 128, 2.21 with 256.  What is left is the stream of W, which comes from memory once per XCD and 2 048
+// tokens: with every stage's W from the same addresses (wrong results) the large case took 0.9 ms less.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-constexpr int kBlockRows = 128;                        // tokens
-constexpr int kBlockW = 16;                            // 16-row tiles of W
-constexpr int kStageBytes = (kBlockRows / 16 + kBlockW) * 1024, kStages = 3;
+constexpr int kBlockW = 16, kWaveW = kBlockW / 4;      // 16-row tiles of W
+constexpr int kBigRows = 256, kBigContraction = 2048;
 
-template <bool UP>
-__global__ __launch_bounds__(256, 2) void expert_tiles_kernel(ExpertArgs a) {
+__device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, char* to, int lane_at, int at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)to, 16, lane_at, at, 0, 0);
+}
+__device__ __forceinline__ u32x4 load_16(__amdgpu_buffer_rsrc_t r, int lane_at, int at) {
+  return __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, lane_at, at, 0));
+}
+// acc += W x with the sum kept where it is, in the accumulation registers: with one wave per SIMD the compiler would
+// hold the sums in both register files and move them between every two products.  It neither reorders nor copies them
+// here (they are only touched by these products until `settled`), so the waits that it would put between a product and
+// another use of its result are not needed before that.
+__device__ __forceinline__ void mfma_in_place(f32x4& acc, const u32x4& w, const u32x4& x) {
+#ifdef __HIP_DEVICE_COMPILE__                            // the constraint means another register on the host
+  asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(acc) : "v"(w), "v"(x));
+#endif
+}
+__device__ __forceinline__ void settled(f32x4& acc) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+a"(acc));
+#endif
+}
+
+// HALVES of HT 16-token tiles
+template <bool UP, int HALVES, int HT>
+__global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(ExpertArgs a) {
+  constexpr int kTiles = HT * HALVES, kOwn = kTiles / 4, kStageBytes = kTiles * 1024, kGroup = 8;
+  constexpr int kLeadW = HALVES == 2 ? 4 : 2, kLeadX = HALVES == 2 ? 5 : 3, kStages = kLeadX + 1;      // stages ahead
   extern __shared__ __align__(16) char lds_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
-  // An XCD takes a contiguous share of the (tile, column block) pairs, in squares of eight by eight, so that
-  // what is in flight on it shares rows of x and of W in its L2.
-  const int nt = *a.ntiles;
+  // An XCD takes a contiguous share of the (tile, column block) pairs, eight tiles at a time, column block by column
+  // block, so that what is in flight on it shares rows of x and of W in its L2.
+  const int nt = *a.ntiles * a.split;
   const int Mx = max(a.M, a.M_shared) * (UP ? 2 : 1), cols = (Mx + 16 * kBlockW - 1) / (16 * kBlockW);
-  const int groups = (nt + 7) / 8, i_xcd = blockIdx.x >> 3;
-  if (i_xcd >= groups * cols) return;
-  const int lin = (blockIdx.x & 7) * groups * cols + i_xcd;
-  const int tg = lin / (8 * cols), rem = lin - tg * 8 * cols;
-  const int tile = tg * 8 + (rem & 7), cb = rem >> 3;
+  const int share = (nt + 7) / 8 * cols, i_xcd = blockIdx.x >> 3;
+  if (i_xcd >= share) return;
+  const int lin = (blockIdx.x & 7) * share + i_xcd;
+  const int tg = lin / (kGroup * cols), rem = lin - tg * kGroup * cols;
+  const int tile = tg * kGroup + rem % kGroup, cb = rem / kGroup;
   if (tile >= nt) return;
-  const int4 t = *(const int4*)(a.tiles + (int64_t)tile * 4);
+  int4 t = *(const int4*)(a.tiles + (int64_t)(tile / a.split) * 4);
+  t.y += tile % a.split * kTiles * 16;                   // a part of a larger tile
+  t.z = min(t.z - tile % a.split * kTiles * 16, kTiles * 16);
+  if (t.z <= 0) return;
   const bool shared = t.x == a.E;
   const int wtiles = (shared ? a.M_shared : a.M) / 16 * (UP ? 2 : 1), K = shared ? a.K_shared : a.K;
   const int w0 = cb * kBlockW;
@@ -438,52 +474,132 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_kernel(ExpertArgs a) {
   // gate_up gathers tokens from all of x, down reads consecutive rows
   const char* const xbase = (const char*)a.x + (UP ? 0 : t.y * a.x_st * 2);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)((UP ? a.n : t.z) * a.x_st * 2), 0x00020000);
-  // this wave's loads of a stage: two of the eight 16-token tiles, four of the sixteen of W
-  int xoff[2], woff[4];
+  int xoff[kOwn], woff[kWaveW];                          // this wave's loads of a stage
 #pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    const int r = min((wave * 2 + i) * 16 + l16, t.z - 1);
+  for (int i = 0; i < kOwn; ++i) {
+    const int r = min((wave * kOwn + i) * 16 + l16, t.z - 1);
     xoff[i] = (int)((UP ? a.sorted[t.y + r] / a.slots : r) * a.x_st * 2) + g * 16;
   }
 #pragma unroll
-  for (int i = 0; i < 4; ++i) woff[i] = min(wave * 4 + i, wtiles - w0 - 1) * steps * 1024;
-  auto request = [&](int ks) {
-    char* const st = lds_raw + (ks % kStages) * kStageBytes;
+  for (int i = 0; i < kWaveW; ++i) woff[i] = min(wave * kWaveW + i, wtiles - w0 - 1) * steps * 1024;
+  // where this lane's results go, and their weights: asked for now, used behind the products
+  int place[kTiles];
+  float wgt[kTiles];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rx, (lds_ptr_t)(st + (wave * 2 + i) * 1024), 16, xoff[i], ks * 64, 0, 0);
+  for (int j = 0; j < kTiles; ++j) place[j] = a.sorted[t.y + min(j * 16 + l16, t.z - 1)];
+  if constexpr (UP) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(st + (8 + wave * 4 + i) * 1024), 16, lane * 16,
-                                               woff[i] + ks * 1024, 0, 0);
+    for (int j = 0; j < kTiles; ++j) {
+      const int n = place[j] / a.slots, slot = place[j] - n * a.slots;
+      wgt[j] = slot < a.top ? a.weights[(int64_t)n * a.top + slot] : 1.f;
+    }
+  }
+  // Past the end the last stage is asked for again, so that the number of loads in flight is always the same.
+  auto token_tile = [&](int ks, int i) {
+    load_to_lds(rx, lds_raw + (ks % kStages) * kStageBytes + (wave * kOwn + i) * 1024, xoff[i], min(ks, steps - 1) * 64);
   };
-  const int th = wave & 1, wh = wave >> 1;
-  f32x4 acc[8][4];
+  auto tokens = [&](int ks) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-  request(0);
-  if (steps > 1) request(1);
-#pragma unroll 1
-  for (int ks = 0; ks < steps; ++ks) {
-    if (ks + 1 < steps) asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();                        // everyone's part of the stage is there
-    if (ks + 2 < steps) request(ks + 2);                 // over the stage that was used up before the barrier
-    const char* const st = lds_raw + (ks % kStages) * kStageBytes + lane * 16;
-    u32x4 xf[4];
-#pragma unroll
-    for (int j = 0; j < 4; ++j) xf[j] = *(const u32x4*)(st + (th * 4 + j) * 1024);
-    u32x4 wf[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) wf[i] = *(const u32x4*)(st + (8 + wh * 8 + i) * 1024);
-    __builtin_amdgcn_sched_barrier(0);                   // all reads on their way before the first product
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = mfma_bf16(wf[i], xf[j], acc[i][j]);
+    for (int i = 0; i < kOwn; ++i) token_tile(ks, i);
     __builtin_amdgcn_sched_barrier(0);
+  };
+  auto weights = [&](int i, int ks) { return load_16(rw, lane * 16, woff[i] + min(ks, steps - 1) * 1024); };
+  f32x4 acc[HALVES][kWaveW][HT];
+#pragma unroll
+  for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+    for (int i = 0; i < kWaveW; ++i)
+#pragma unroll
+      for (int j = 0; j < HT; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 wr[kLeadW][kWaveW], xf[HALVES][HT];
+  auto fill = [&](int ks, u32x4 (&w)[kWaveW]) {
+    tokens(ks);
+#pragma unroll
+    for (int i = 0; i < kWaveW; ++i) w[i] = weights(i, ks);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto read_tile = [&](int ks, int h, int j) {
+    xf[h][j] = *(const u32x4*)(lds_raw + (ks % kStages) * kStageBytes + (h * HT + j) * 1024 + lane * 16);
+  };
+  auto read = [&](int ks, int h) {
+#pragma unroll
+    for (int j = 0; j < HT; ++j) read_tile(ks, h, j);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  static_assert(HALVES == 1 || (kOwn == 4 && HT == 2 * kWaveW), "the waits count a wave's loads");
+  // the next tokens to be read are in LDS when all but the loads asked for after them have landed: three stages' (one
+  // stage's, of fewer tokens)
+  auto landed = [&]() {
+    if constexpr (HALVES == 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+    __builtin_amdgcn_s_barrier();                        // everyone's
+  };
+#pragma unroll
+  for (int s = 0; s < kLeadW; ++s) fill(s, wr[s]);
+  tokens(kLeadW);
+  if constexpr (HALVES == 2) {
+    asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    read(0, 0);
+  }
+  auto stage = [&](int ks, u32x4 (&w)[kWaveW]) {
+    if constexpr (HALVES == 2) {
+      // One wave per SIMD: whatever it issues between two products is time without products.  So reads and requests
+      // are spread over the products, a half ahead of their use.
+#pragma unroll
+      for (int i = 0; i < kWaveW; ++i)
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+          mfma_in_place(acc[0][i][j], w[i], xf[0][j]);
+          if (j == HT / 2 - 1) read_tile(ks, 1, 2 * i);
+          if (j == HT - 1) read_tile(ks, 1, 2 * i + 1);
+          if (j == HT / 2 - 1 || j == HT - 1) __builtin_amdgcn_sched_barrier(0);
+        }
+      landed();
+#pragma unroll
+      for (int i = 0; i < kWaveW; ++i) {
+#pragma unroll
+        for (int j = 0; j < HT; ++j) {
+          mfma_in_place(acc[1][i][j], w[i], xf[1][j]);
+          if (j == 1) token_tile(ks + kLeadX, i);             // over the stage before this one
+          if (j == 3) read_tile(ks + 1, 0, 2 * i);
+          if (j == 5) read_tile(ks + 1, 0, 2 * i + 1);
+          if (j & 1) __builtin_amdgcn_sched_barrier(0);
+        }
+        w[i] = weights(i, ks + kLeadW);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      landed();
+      tokens(ks + kLeadX);                               // over the stage before this one
+      read(ks, 0);
+#pragma unroll
+      for (int i = 0; i < kWaveW; ++i) {
+#pragma unroll
+        for (int j = 0; j < HT; ++j) acc[0][i][j] = mfma_bf16(w[i], xf[0][j], acc[0][i][j]);
+        w[i] = weights(i, ks + kLeadW);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  };
+  int ks = 0;
+#pragma unroll 1
+  for (; ks + kLeadW <= steps; ks += kLeadW) {
+#pragma unroll
+    for (int s = 0; s < kLeadW; ++s) stage(ks + s, wr[s]);
+  }
+#pragma unroll
+  for (int s = 0; s + 1 < kLeadW; ++s)
+    if (ks + s < steps) stage(ks + s, wr[s]);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // loads into LDS end before the workgroup does
+  if constexpr (HALVES == 2) {                           // the last products' results are in their registers
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int h = 0; h < HALVES; ++h)
+#pragma unroll
+      for (int i = 0; i < kWaveW; ++i)
+#pragma unroll
+        for (int j = 0; j < HT; ++j) settled(acc[h][i][j]);
   }
   // Two result tiles side by side hold 4 outputs per lane each; lanes of neighbouring groups swap halves, so that
   // each ends with 8 consecutive outputs of one of them: group g has tile (g & 1), outputs 8 (g >> 1) on.
@@ -493,45 +609,46 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_kernel(ExpertArgs a) {
     if (row && tile + (g & 1) < tiles)
       *(u32x4*)((uint16_t*)a.out + at + (tile + (g & 1)) * 16 + (g >> 1) * 8) = u32x4{a0[0], a1[0], a0[1], a1[1]};
   };
-  const int out_tiles = UP ? wtiles / 2 : wtiles;
+  const int out_tiles = UP ? wtiles / 2 : wtiles, own = w0 + wave * kWaveW;
 #pragma unroll
-  for (int j = 0; j < 4; ++j) {
-    const int r = (th * 4 + j) * 16 + l16;
+  for (int jj = 0; jj < kTiles; ++jj) {
+    const int j = jj % HT, h = jj / HT, r = jj * 16 + l16;
     const bool row = r < t.z;                          // every lane takes part in the swaps
-    const int pos = t.y + min(r, t.z - 1), as = a.sorted[pos], n = as / a.slots, slot = as - n * a.slots;
     if constexpr (UP) {
-      const float wgt = slot < a.top ? a.weights[(int64_t)n * a.top + slot] : 1.f;
       const float lim = shared ? a.limit_shared : a.limit;
+      float v[2][4];
 #pragma unroll
-      for (int i = 0; i < 8; i += 4) {
-        float v[2][4];
+      for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-          for (int k = 0; k < 4; ++k) v[u][k] = gated<BF16>(a.act, wgt, acc[i + 2 * u][j][k], acc[i + 2 * u + 1][j][k], lim);
-        store8(v[0], v[1], (int64_t)pos * a.o_st, (w0 + wh * 8 + i) / 2, out_tiles, row);
-      }
+        for (int k = 0; k < 4; ++k) v[u][k] = gated<BF16>(a.act, wgt[jj], acc[h][2 * u][j][k], acc[h][2 * u + 1][j][k], lim);
+      store8(v[0], v[1], (int64_t)(t.y + r) * a.o_st, own / 2, out_tiles, row);
     } else {
+      const int n = place[jj] / a.slots, slot = place[jj] - n * a.slots;
 #pragma unroll
-      for (int i = 0; i < 8; i += 2) {
-        const float lo[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]};
-        const float hi[4] = {acc[i + 1][j][0], acc[i + 1][j][1], acc[i + 1][j][2], acc[i + 1][j][3]};
-        store8(lo, hi, ((int64_t)slot * a.n + n) * a.o_st, w0 + wh * 8 + i, out_tiles, row);
+      for (int i = 0; i < kWaveW; i += 2) {
+        const float lo[4] = {acc[h][i][j][0], acc[h][i][j][1], acc[h][i][j][2], acc[h][i][j][3]};
+        const float hi[4] = {acc[h][i + 1][j][0], acc[h][i + 1][j][1], acc[h][i + 1][j][2], acc[h][i + 1][j][3]};
+        store8(lo, hi, ((int64_t)slot * a.n + n) * a.o_st, own + i, out_tiles, row);
       }
     }
   }
 }
 
 template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, hipStream_t st) {
-  if (rows == kBlockRows) {
+  if (rows == 128 || rows == kBigRows) {
     const int Mx = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
-    const int64_t grid = (int64_t)((a.max_tiles + 7) / 8) * 8 * ((Mx + 16 * kBlockW - 1) / (16 * kBlockW));
-    constexpr int smem = kStages * kStageBytes;
-    if (hipFuncSetAttribute((const void*)expert_tiles_kernel<UP>, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
+    const bool big = rows == kBigRows && a.K >= kBigContraction;
+    ExpertArgs b = a;
+    b.split = big ? 1 : rows / 128;
+    const int64_t grid = (int64_t)((b.max_tiles * b.split + 7) / 8) * 8 * ((Mx + 16 * kBlockW - 1) / (16 * kBlockW));
+    const void* const fn = big ? (const void*)expert_tiles_kernel<UP, 2, 8> : (const void*)expert_tiles_kernel<UP, 1, 8>;
+    const int smem = big ? 6 * 16 * 1024 : 4 * 8 * 1024;
+    if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
       zp_set_error("moe: cannot reserve %d bytes of LDS", smem);
       return ZP_EHIP;
     }
-    hipLaunchKernelGGL((expert_tiles_kernel<UP>), dim3((unsigned)grid), dim3(256), smem, st, a);
+    if (big) hipLaunchKernelGGL((expert_tiles_kernel<UP, 2, 8>), dim3((unsigned)grid), dim3(256), smem, st, b);
+    else hipLaunchKernelGGL((expert_tiles_kernel<UP, 1, 8>), dim3((unsigned)grid), dim3(256), smem, st, b);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }
@@ -562,7 +679,8 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
 // Rows per tile: enough for the average expert.
 int tile_rows(int n, int E, int top, int dtype) {
   const int64_t avg = ((int64_t)n * top + E - 1) / E;
-  if (dtype == ZP_BF16 && avg > 48) return kBlockRows;
+  if (dtype == ZP_BF16 && avg > 512) return kBigRows;
+  if (dtype == ZP_BF16 && avg > 48) return 128;
   return avg <= 8 ? 16 : (avg <= 16 ? 32 : 64);       // a second tile reads an expert's weights again
 }
 int tile_bound(int n, int E, int top, int shared, int rows) {
@@ -667,7 +785,7 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
              "moe experts: bad dims");
   ZP_MODEL_DTYPE("moe experts");
   if (K % 32 || K_shared % 32 || M % 16 || M_shared % 16 || x_stride % 8 || out_stride % 8 ||
-      (rows != 16 && rows != 32 && rows != 64 && (rows != kBlockRows || dtype != ZP_BF16))) {
+      (rows != 16 && rows != 32 && rows != 64 && ((rows != 128 && rows != kBigRows) || dtype != ZP_BF16))) {
     zp_set_error("moe experts: sizes %d x %d, shared %d x %d, %d rows per tile unsupported", M, K, M_shared, K_shared, rows);
     return ZP_EUNSUPPORTED;
   }
@@ -676,15 +794,15 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
   ZP_REQUIRE(aligned16(x) && aligned16(w) && aligned16(w_shared) && aligned16(out) && aligned16(tiles) &&
                  x_stride >= (K > K_shared ? K : K_shared) && out_stride >= (M > M_shared ? M : M_shared),
              "moe experts: unaligned or overlapping rows");
-  if (rows == kBlockRows) {       // 31-bit byte offsets into x and into a block of W
-    const int64_t xr = up ? n : kBlockRows, kx = K > K_shared ? K : K_shared;
+  if (rows >= 128) {              // 31-bit byte offsets into x and into a block of W
+    const int64_t xr = up ? n : rows, kx = K > K_shared ? K : K_shared;
     if (xr * x_stride * 2 >= (1ll << 31) || kx * 512 >= (1ll << 31)) {
       zp_set_error("moe experts: %lld rows of %lld elements in one step", (long long)xr, (long long)x_stride);
       return ZP_EUNSUPPORTED;
     }
   }
   ExpertArgs a = {x, w, w_shared, out, sorted, tiles, ntiles, weights, n, E, top, top + shared, max_tiles, K, K_shared,
-                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared};
+                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1};
   return up ? launch_experts<true>(a, rows, dtype, (hipStream_t)stream)
             : launch_experts<false>(a, rows, dtype, (hipStream_t)stream);
 }
