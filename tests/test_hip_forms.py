@@ -77,3 +77,41 @@ def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act):
     # bf16 activations and planes: each of top + 2 roundings is at most 2^-9 of its own value
     err = (got - want)[sure].norm() / want[sure].norm()
     assert float(err) < 2.0 ** -8 and bool(torch.isfinite(got).all())
+
+
+# ------------------------------------------------------------------ attention of runs
+def _attended(q, k, v, lens, scale):
+    """64-bit attention of runs: lens of (queries, keys), queries being the last positions."""
+    H, rep, want, a, b = q.shape[1], q.shape[1] // k.shape[1], [], 0, 0
+    for n, m in lens:
+        kk, vv = (t[b:b + m].double().repeat_interleave(rep, 1) for t in (k, v))
+        sc = torch.einsum("qhd,khd->hqk", q[a:a + n].double(), kk) * scale
+        seen = torch.arange(m)[None] <= torch.arange(m - n, m)[:, None]
+        want.append(torch.einsum("hqk,khd->qhd", torch.softmax(sc.masked_fill(~seen, float("-inf")), -1), vv))
+        a, b = a + n, b + m
+    return torch.cat(want)
+
+
+def _tiles(lens):
+    made, a, b = [], 0, 0
+    for n, m in lens:
+        made += [(a + i, min(128, n - i), b, m - n + i) for i in range(0, n, 128)]
+        a, b = a + n, b + m
+    return torch.tensor(made, dtype=torch.int32)
+
+
+# the scale joins the subtraction of the maximum: a negative one turns the queries round, zero takes them away
+@pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-30, 0.25])
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 40, 24), (4, 2, 128, 128), (3, 3, 136, 136)])
+def test_runs_of_any_scale(dev, H, G, D, V, scale):
+    from zipage_amd.layers import run_attention
+    lens = [(1, 1), (63, 63), (65, 65), (130, 200)]
+    N, M = (sum(t) for t in zip(*lens))
+    q, k = (_rand(N, H, D, seed=1), _rand(M, G, D, seed=2))
+    v = _rand(M, G, V, seed=3)
+    out = torch.empty(N, H * V, dtype=BF16, device=dev)
+    run_attention(q.flatten(1).to(dev), torch.cat([k.flatten(1), v.flatten(1)], 1).to(dev), H, G, D, V,
+                  _tiles(lens).to(dev), scale, out)
+    want = _attended(q, k, v, lens, scale)
+    # the result's rounding, and that of the weights: at most 2^-9 of each one's value's distance from the result
+    assert bool(((out.view(N, H, V).cpu().double() - want).abs() <= 2.0 ** -9 * want.abs() + 2.0 ** -8 * v.abs().max()).all())

@@ -20,6 +20,13 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 // key of operand element i (0..7) held by lane group g, within a step of 32 keys
 __device__ __forceinline__ int step_key(int g, int i) { return i < 4 ? 4 * g + i : 12 + 4 * g + i; }
 
+// A 4 x 16 block of 16-bit values in LDS, transposed: lane i of a group of sixteen names row i / 4, values 4 (i % 4) on,
+// and receives the four of column i.
+typedef short zp_s16x4 __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ uint2 read_transposed(const uint16_t* p) {
+  return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) zp_s16x4*)p));
+}
+
 // Eight rows (keys) of eight bf16 columns -> for column t the four dwords of its eight keys.
 __device__ __forceinline__ u32x4 column_of(const u32x4* rows, int t) {
   const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;

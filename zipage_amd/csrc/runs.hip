@@ -18,7 +18,7 @@ __global__ __launch_bounds__(256) void gather_rows_kernel(const char* src, const
 struct TilesArgs {
   const uint16_t* q;      // token rows of q_st elements, head h at h * maps * (D + P)
   const uint16_t* k;      // key rows of kv_st elements, head h at h * maps * D
-  const uint16_t* v;      // value rows of kv_st elements, head h at h * V
+  const uint16_t* v;      // value rows of v_st elements, head h at h * V
   const uint16_t* ks;     // rows of s_st elements: the last P of every head's key; null: P = 0
   uint16_t* out;          // token rows of o_st elements, head h at h * V
   const int32_t* tiles;   // (T, 4): first query row, queries, first key row of the run, position
@@ -26,7 +26,7 @@ struct TilesArgs {
   const float* sinks;     // (H,) logits that only join the denominator, or null
   int T, H, HK, D, P, V;  // HK key / value heads; query head h uses head h / (H / HK)
   int window, chunk;      // at most one is set, see first_seen
-  int64_t q_rows, k_rows, q_st, kv_st, s_st, o_st;
+  int64_t q_rows, k_rows, q_st, kv_st, v_st, s_st, o_st;
   float scale, out_scale;
   float cap;              // > 0: soft cap of the scores
   // two maps: rms(o1 - balance * o2) * out_scale * sigmoid(gate), the mean over vdim
@@ -42,7 +42,13 @@ constexpr int kTileK = 64;    // keys per LDS tile
 
 // A workgroup owns up to 128 queries of one head; key and value tiles pass through LDS once for all of
 // them (double-buffered, the next tile's loads in flight during the products), a wave owns 16 * kQT
-// queries at a time and skips the 32-key steps none of them sees.
+// queries at a time and skips the steps of 32 or 64 keys none of them sees.
+//
+// Bound by the vector units and by the latencies of a step's chain (products, maximum, exponentials, products) with two
+// waves per SIMD: matrix cores are busy a third of the time.  So the values are transposed by the LDS reads
+// themselves, operands are read a group ahead of their products, a step takes 64 keys where its scores fit the registers,
+// the maximum crosses lanes only when it has moved, and sums of weights are a product with ones.  8 prompts of 2048
+// tokens, 32 heads of 128 with 8 of keys and values: 531 -> 435 us without limit, 347 -> 296 in chunks of 1024.
 // First key position a query sees: the last `window` up to and including its own, or those of its own
 // block of `chunk` positions (key 0 of the run starts a block), or all.
 __device__ __forceinline__ int first_seen(int pos, int window, int chunk) {
@@ -54,7 +60,8 @@ __device__ __forceinline__ int first_seen(int pos, int window, int chunk) {
 constexpr int tile_waves(int maps) { return maps == 2 ? 8 : 4; }
 
 template <int DKS, int VCB, int MAPS> struct TileStage {
-  static constexpr int kK = MAPS * DKS * 32 + 8, kV = VCB * 128 + 8;    // row strides: rows 16 bytes apart in the banks
+  // row strides: rows of keys 16 bytes apart in the banks, those of values, which are read 32 bytes wide, 32
+  static constexpr int kK = MAPS * DKS * 32 + 8, kV = VCB * 128 + 16;
   static constexpr int kElems = kTileK * (kK + kV);
   static constexpr int kWaves = tile_waves(MAPS);
   static constexpr int kBuffers = MAPS == 2 || 8 * kElems <= 160 * 1024 ? 2 : 1;
@@ -65,11 +72,16 @@ enum { kNoCap, kCap, kBoundedCap };   // of the scores, see SoftCap
 
 // Column tile t of a wave: 16 queries, map t % MAPS of the head (differential attention has two, over the same
 // values; elsewhere there is one).  SHARED: the last P elements of every head's key are the row of a.ks.
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP>
+// FINE: softmax weights enter the value product as two bf16 planes (17 bits), elsewhere as one.
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE>
 __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(TilesArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef TileStage<DKS, VCB, MAPS> Stage;
   constexpr bool kTurns = MAPS == 1 && !SHARED && CAP == kNoCap;
+  // keys per step: 64 scores for each query where the registers hold them (8 prompts as above: 519 -> 463 us; keys of 192
+  // with a shared part spill: 1811 -> 1831)
+  constexpr int kStep = MAPS == 1 && VCB == 1 && CAP == kNoCap && DKS <= (SHARED ? 4 : 6) ? 64 : 32;
+  constexpr bool kPinned = DKS <= 4 && (VCB == 1 || MAPS == 1);   // reads ahead: wider heads would spill
   constexpr int kT = kQT * MAPS, kWaves = Stage::kWaves, kThreads = 64 * kWaves, kPass = 16 * kQT * kWaves;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
   const int h = blockIdx.x % a.H, tile = blockIdx.x / a.H;   // one head's tiles share an L2 when H % 8 == 0
@@ -79,9 +91,14 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
   if (q0 < 0 || kb < 0 || rel < 0 || (int64_t)q0 + nq > a.q_rows || (int64_t)kb + rel + nq > a.k_rows) return;
   const int DT = a.D + (SHARED ? a.P : 0);
   const SoftCap cap(a.scale, a.cap);
+  // without a cap the scale joins the subtraction of the maximum, for which it has to be positive: a negative one turns
+  // the queries round, zero takes them away
+  const uint32_t flip = CAP == kNoCap && a.scale < 0.f ? 0x80008000u : 0u, kept = CAP == kNoCap && cap.factor == 0.f ? 0u : ~0u;
+  const float factor = cap.factor == 0.f ? 1.f : fabsf(cap.factor);
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
   const int hk = h / (a.H / a.HK);
   const uint16_t* kbase = a.k + (int64_t)kb * a.kv_st + hk * MAPS * a.D;
-  const uint16_t* vbase = a.v + (int64_t)kb * a.kv_st + hk * a.V;
+  const uint16_t* vbase = a.v + (int64_t)kb * a.v_st + hk * a.V;
   const uint16_t* sbase = SHARED ? a.ks + (int64_t)kb * a.s_st : nullptr;
 
   for (int wg0 = 0; wg0 < nq; wg0 += kPass) {                 // uniform in the workgroup
@@ -104,7 +121,7 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
       for (int ks = 0; ks < DKS; ++ks) {
         // past the head's end: the key columns there hold other elements, against zeros here
         const int c = ks * 32 + g * 8;
-        qf[t][ks] = *(const u32x4*)(q + (c < DT ? c : 0));
+        qf[t][ks] = (*(const u32x4*)(q + (c < DT ? c : 0)) & kept) ^ flip;
         if (c >= DT) qf[t][ks] = u32x4{0u, 0u, 0u, 0u};
       }
     }
@@ -122,8 +139,8 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
     constexpr int kKN = kTileK * kKP / kThreads, kVN = kTileK * kVP / kThreads;
     u32x4 rk[kKN], rv[kVN];                                    // this thread's pieces of a tile
     auto fetch = [&](int k0) {                                 // offsets from the tile's first row: 32 bits
-      const uint16_t *kt = kbase + k0 * a.kv_st, *vt = vbase + k0 * a.kv_st, *st = SHARED ? sbase + k0 * a.s_st : nullptr;
-      const uint32_t kv_st = (uint32_t)a.kv_st, s_st = (uint32_t)a.s_st;
+      const uint16_t *kt = kbase + k0 * a.kv_st, *vt = vbase + k0 * a.v_st, *st = SHARED ? sbase + k0 * a.s_st : nullptr;
+      const uint32_t kv_st = (uint32_t)a.kv_st, v_st = (uint32_t)a.v_st, s_st = (uint32_t)a.s_st;
 #pragma unroll
       for (int j = 0; j < kKN; ++j) {
         const int id = tid + kThreads * j, pc = id % kKP, map = pc / (4 * DKS), c = (pc % (4 * DKS)) * 8;
@@ -139,7 +156,7 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
       for (int j = 0; j < kVN; ++j) {
         const int id = tid + kThreads * j, c = (id % kVP) * 8;
         const uint32_t r = min(id / kVP, last - k0);
-        rv[j] = *(const u32x4*)(vt + (r * kv_st + (c < a.V ? c : 0)));
+        rv[j] = *(const u32x4*)(vt + (r * v_st + (c < a.V ? c : 0)));
       }
     };
     fetch(first);
@@ -162,78 +179,128 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
       __syncthreads();
       if (t0 + kTileK <= last) fetch(t0 + kTileK);
 #pragma unroll 1
-      for (int sub = 0; sub < kTileK; sub += 32) {
+      for (int sub = 0; sub < kTileK; sub += kStep) {
         const int k0 = t0 + sub;
-        if (k0 > hi || k0 + 31 < lo) continue;                 // uniform in the wave
-        f32x4 s[kT][2];
+        if (k0 > hi || k0 + kStep - 1 < lo) continue;          // uniform in the wave
+        // operands leave LDS a group ahead of the products that use them; the barriers keep the compiler from moving each
+        // read to its use, where its latency would show (463 -> 421 us).  This wave's products go before the other's
+        // exponentials (441 -> 435)
+        float p[kT][kStep / 4];
+        u32x4 kf[2][DKS * MAPS];
+        const uint16_t* const ks0 = ldsk + (sub + l16) * Stage::kK + g * 8;
+        auto read_keys = [&](int tt) {
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
+          for (int i = 0; i < DKS * MAPS; ++i) kf[tt & 1][i] = *(const u32x4*)(ks0 + tt * 16 * Stage::kK + i * 32);
+        };
+        __builtin_amdgcn_s_setprio(1);
+        if constexpr (kPinned) read_keys(0);
 #pragma unroll
-          for (int t = 0; t < kT; ++t) s[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int tt = 0; tt < kStep / 16; ++tt) {
+          if (!kPinned) read_keys(tt);
+          else if (tt + 1 < kStep / 16) read_keys(tt + 1);
+          if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
+          f32x4 s[kT];
+#pragma unroll
+          for (int t = 0; t < kT; ++t) s[t] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
           for (int ks = 0; ks < DKS; ++ks)
 #pragma unroll
-            for (int map = 0; map < MAPS; ++map) {
-              const u32x4 kf = *(const u32x4*)(ldsk + (sub + tt * 16 + l16) * Stage::kK + (map * DKS + ks) * 32 + g * 8);
+            for (int t = 0; t < kT; ++t) s[t] = mfma_bf16(kf[tt & 1][t % MAPS * DKS + ks], qf[t][ks], s[t]);
 #pragma unroll
-              for (int t = map; t < kT; t += MAPS) s[t][tt] = mfma_bf16(kf, qf[t][ks], s[t][tt]);
+          for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) p[t][tt * 4 + i] = s[t][i];
+          if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
+        }
+        // value columns of 16, transposed on their way out of LDS: lane l16 gets column l16 of eight keys
+        const uint16_t* const vs = ldsv + (sub + 4 * g + (l16 >> 2)) * Stage::kV + (l16 & 3) * 4;
+        constexpr int kGroups = kStep / 32 * VCB * 2;          // of four such columns and 32 keys
+        u32x4 vf[2][4];
+        auto read_values = [&](int n) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint16_t* const at = vs + n / (VCB * 2) * 32 * Stage::kV + (n % (VCB * 2) * 4 + i) * 16;
+            const uint2 lo = read_transposed(at), hi = read_transposed(at + 16 * Stage::kV);
+            vf[n & 1][i] = u32x4{lo.x, lo.y, hi.x, hi.y};
+          }
+        };
+        __builtin_amdgcn_s_setprio(0);
+        if constexpr (kPinned) read_values(0);
+        if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
+        if (CAP != kNoCap) {
+#pragma unroll
+          for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int i = 0; i < kStep / 4; ++i) p[t][i] = cap.capped(p[t][i]);
+        }
+        if (k0 + kStep - 1 > rel + w0 || k0 < lo_last) {         // some query of the wave does not see all these keys
+#pragma unroll
+          for (int t = 0; t < kT; ++t)
+#pragma unroll
+            for (int i = 0; i < kStep / 4; ++i) {
+              const int key = k0 + (i >> 2) * 16 + 4 * g + (i & 3);
+              if (key > qpos[t / MAPS] || key < qlow[t / MAPS]) p[t][i] = -INFINITY;
             }
         }
-        // every query of the wave sees all 32 keys: no masks
-        const bool inner = k0 + 31 <= rel + w0 && k0 >= lo_last;
-        u32x4 pf[kT];
+        if (CAP != kBoundedCap) {
 #pragma unroll
-        for (int t = 0; t < kT; ++t) {
-          float p[8], sum = 0.f;
-#pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            const float x = s[t][i >> 2][i & 3];
-            p[i] = CAP == kNoCap ? x * cap.factor : cap.capped(x);
-          }
-          if (!inner) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              const int key = k0 + step_key(g, i);
-              if (key > qpos[t / MAPS] || key < qlow[t / MAPS]) p[i] = -INFINITY;
-            }
-          }
-          float ms = 0.f, f = 1.f;
-          if (CAP != kBoundedCap) {
+          for (int t = 0; t < kT; ++t) {
             float mx = -INFINITY;
 #pragma unroll
-            for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
-            mx = fmaxf(mx, lane_xor16(mx));
-            mx = fmaxf(mx, lane_xor32(mx));
-            const float mn = fmaxf(m[t], mx);
-            ms = mn == -INFINITY ? 0.f : mn;                    // a query whose window starts later
-            f = __builtin_amdgcn_exp2f(m[t] - ms);
-            m[t] = mn;
-          }
+            for (int i = 0; i < kStep / 4; ++i) mx = fmaxf(mx, p[t][i]);
+            if (CAP == kNoCap) mx *= factor;
+            if (__any(mx > m[t])) {                             // in any lane: hardly ever after the first keys
+              mx = fmaxf(m[t], mx);
+              mx = fmaxf(mx, lane_xor16(mx));
+              mx = fmaxf(mx, lane_xor32(mx));
+              const float f = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[t] - mx);
+              m[t] = mx;
+              l[t] *= f;
 #pragma unroll
-          for (int i = 0; i < 8; ++i) {
-            p[i] = __builtin_amdgcn_exp2f(CAP == kBoundedCap ? p[i] : p[i] - ms);
-            sum += p[i];
+              for (int i = 0; i < VCB * 8; ++i) o[t][i] *= f;
+            }
           }
-          l[t] = CAP == kBoundedCap ? l[t] + sum : l[t] * f + sum;
-          if (CAP != kBoundedCap && __any(f != 1.f)) {
+        }
+        u32x4 pf[kT][kStep / 32], pl[FINE ? kT : 1][kStep / 32];
 #pragma unroll
-            for (int i = 0; i < VCB * 8; ++i) o[t][i] *= f;
+        for (int t = 0; t < kT; ++t) {
+          const float ms = m[t] == -INFINITY ? 0.f : m[t];      // a query whose window starts later
+#pragma unroll
+          for (int i = 0; i < kStep / 4; ++i)
+            p[t][i] = __builtin_amdgcn_exp2f(CAP == kNoCap        ? fmaf(p[t][i], factor, -ms)
+                                             : CAP == kBoundedCap ? p[t][i]
+                                                                  : p[t][i] - ms);
+#pragma unroll
+          for (int d = 0; d < kStep / 8; ++d) {
+            const uint32_t w = pack_bf16(p[t][2 * d], p[t][2 * d + 1]);
+            pf[t][d / 4][d % 4] = w;
+            if constexpr (FINE)
+              pl[t][d / 4][d % 4] =
+                  pack_bf16(p[t][2 * d] - __uint_as_float(w << 16), p[t][2 * d + 1] - __uint_as_float(w & 0xffff0000u));
           }
-          pf[t] = u32x4{pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]),
-                        pack_bf16(p[6], p[7])};
+          // the sum of the weights as the values meet them: what rounding does to a weight that outweighs the others cancels
+          f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int d = 0; d < kStep / 32; ++d) {
+            sum = mfma_bf16(ones, pf[t][d], sum);
+            if constexpr (FINE) sum = mfma_bf16(ones, pl[t][d], sum);
+          }
+          l[t] += sum[0];
         }
 #pragma unroll
-        for (int cb = 0; cb < VCB; ++cb) {
-          u32x4 v[8];
+        for (int n = 0; n < kGroups; ++n) {
+          if (!kPinned) read_values(n);
+          else if (n + 1 < kGroups) read_values(n + 1);
+          if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
+          const int half = n / (VCB * 2), c0 = n % (VCB * 2) * 4;
 #pragma unroll
-          for (int i = 0; i < 8; ++i)
-            v[i] = *(const u32x4*)(ldsv + (sub + step_key(g, i)) * Stage::kV + cb * 128 + l16 * 8);
+          for (int i = 0; i < 4; ++i)
 #pragma unroll
-          for (int c = 0; c < 8; ++c) {
-            const u32x4 vf = column_of(v, c);
-#pragma unroll
-            for (int t = 0; t < kT; ++t) o[t][cb * 8 + c] = mfma_bf16(vf, pf[t], o[t][cb * 8 + c]);
-          }
+            for (int t = 0; t < kT; ++t) {
+              o[t][c0 + i] = mfma_bf16(vf[n & 1][i], pf[t][half], o[t][c0 + i]);
+              if constexpr (FINE) o[t][c0 + i] = mfma_bf16(vf[n & 1][i], pl[t][half], o[t][c0 + i]);
+            }
+          if constexpr (kPinned) __builtin_amdgcn_sched_barrier(0);
         }
       }
     }
@@ -243,8 +310,6 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
 #pragma unroll
       for (int map = 0; map < MAPS; ++map) {
         float lt = l[qt * MAPS + map];
-        lt += lane_xor16(lt);
-        lt += lane_xor32(lt);
         if (MAPS == 1 && a.sinks) lt += __builtin_amdgcn_exp2f(a.sinks[h] * 1.44269504088896f - m[qt]);
         inv[map] = lt > 0.f ? 1.f / lt : 0.f;
       }
@@ -259,50 +324,54 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
           for (int i = 0; i < 4; ++i) {
             const float r = o[qt * 2][j][i] * inv[0] - o[qt * 2 + 1][j][i] * second;
             o[qt * 2][j][i] = r;
-            if ((j >> 3) * 128 + (4 * g + i) * 8 < a.V) ss += r * r;
+            if (j * 16 + 4 * g + i < a.V) ss += r * r;
           }
         ss += lane_xor16(ss);
         ss += lane_xor32(ss);
         inv[0] = a.out_scale / sqrtf(ss / (float)a.vdim + a.eps);
       }
       const int qi = w0 + qt * 16 + l16;
-      if (qi >= nq) continue;
+      const bool row = qi < nq;                                // every lane takes part in the swaps
       uint16_t* out = a.out + (int64_t)(q0 + qi) * a.o_st + h * a.V;
       const float2* turns = a.turns;
       asm volatile("" : "+s"(turns));                          // nothing of the way back is computed before the loop
       const uint16_t* gate = MAPS == 2 && a.gate ? a.gate + (int64_t)(q0 + qi) * a.g_st + h * a.V : nullptr;
+      // a lane holds 4 columns of each of two tiles; groups g and g ^ 1 swap halves, so that each ends with 8 of one
 #pragma unroll
-      for (int cb = 0; cb < VCB; ++cb)
+      for (int c = 0; c < VCB * 8; c += 2) {
+        float r[8];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const int col = cb * 128 + (4 * g + i) * 8;
-          if (col < a.V) {
-            float r[8];
-#pragma unroll
-            for (int c = 0; c < 8; ++c) r[c] = o[qt * MAPS][cb * 8 + c][i] * inv[0];
-            if (kTurns && turns) turn_back8(r, turns + ((int64_t)(q0 + qi) * a.V + col) / 2);
-            if (MAPS == 2 && gate) {
-              float z[8];
-              Vec8<BF16>::ld(gate, col, z);
-#pragma unroll
-              for (int c = 0; c < 8; ++c) r[c] *= sigmoid_of<BF16>(z[c]);
-            }
-            Vec8<BF16>::st(out, col, r);
-          }
+          const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(o[qt * MAPS][c][i] * inv[0]),
+                                                             __float_as_uint(o[qt * MAPS][c + 1][i] * inv[0]), false, false);
+          r[i] = __uint_as_float(both[0]);
+          r[4 + i] = __uint_as_float(both[1]);
         }
+        const int col = (c + (g & 1)) * 16 + (g >> 1) * 8;
+        if (!row || col >= a.V) continue;
+        if (kTurns && turns) turn_back8(r, turns + ((int64_t)(q0 + qi) * a.V + col) / 2);
+        if (MAPS == 2 && gate) {
+          float z[8];
+          Vec8<BF16>::ld(gate, col, z);
+#pragma unroll
+          for (int i = 0; i < 8; ++i) r[i] *= sigmoid_of<BF16>(z[i]);
+        }
+        Vec8<BF16>::st(out, col, r);
+      }
     }
   }
 }
 
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP> int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
+int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
   constexpr int smem = TileStage<DKS, VCB, MAPS>::kBytes;
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP>,
+      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP>), dim3((unsigned)a.T * a.H),
+  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE>), dim3((unsigned)a.T * a.H),
                      dim3(64 * TileStage<DKS, VCB, MAPS>::kWaves), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
@@ -375,7 +444,7 @@ extern "C" int zp_run_attention(const void* q, const void* k, const void* v, con
                  kv_stride < (1ll << 26) && shared_stride < (1ll << 26),
              "run_attention: unaligned rows or too many tiles");
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)k_shared, (uint16_t*)out,
-                 tiles, sinks, T, H, HK, D, P, V, window, chunk, q_rows, k_rows, q_stride, kv_stride, shared_stride,
+                 tiles, sinks, T, H, HK, D, P, V, window, chunk, q_rows, k_rows, q_stride, kv_stride, kv_stride, shared_stride,
                  out_stride, scale, out_scale, f.softcap, f.balance, f.eps, f.vdim, (const uint16_t*)f.gate, f.gate_stride,
                  (const float2*)f.turns};
   hipStream_t st = (hipStream_t)stream;
