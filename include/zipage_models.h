@@ -101,6 +101,14 @@ int zp_run_attention(const void* q, const void* k, const void* v, const void* k_
                      int64_t shared_stride, int64_t out_stride, float scale, float out_scale,
                      int32_t dtype, void* stream);
 
+/* The same without window, chunk, sinks and form, for D = V <= 128 and keys and values with strides of their own; softmax
+ * weights keep 17 bits where they meet the values.  q rows q_stride, k rows k_stride, v rows v_stride apart, heads of D
+ * back to back. */
+int zp_causal_attention(const void* q, const void* k, const void* v, void* out, const int32_t* tiles, int32_t T,
+                        int32_t H, int32_t HK, int32_t D, int64_t q_rows, int64_t k_rows, int64_t q_stride,
+                        int64_t k_stride, int64_t v_stride, int64_t out_stride, float scale, int32_t dtype,
+                        void* stream);
+
 /* ------------------------------------------------------------------ libzipage_latent.so */
 
 /* in (n, q_width + c_width + p_width): the first part RMS-normed times q_weight goes to q_out; the second

@@ -3,8 +3,8 @@
 Only what the decode benchmark needs: bf16 weights drawn on the device and the fused qkv and
 gate/up projections through torch's GEMMs; everything between the GEMMs is this package's HIP
 kernels (residual add + RMSNorm, per-head q/k norm + rotary embedding + K/V scatter + window-query
-capture, paged decode attention, SiLU gate).  Prefill attention is torch's
-scaled_dot_product_attention.
+capture, paged decode attention, SiLU gate, causal attention of prompts).  In float16 prefill attention is
+torch's scaled_dot_product_attention.
 """
 from __future__ import annotations
 
@@ -14,7 +14,10 @@ import torch
 import torch.nn.functional as F
 
 from zipage_amd.kernel import store_query_cache
-from zipage_amd.layers import paged_decode_attention, qk_norm_rope_store, rms_norm, silu_and_mul
+from zipage_amd.layers import (causal_attention, gather_rows, paged_decode_attention, qk_norm_rope_store, rms_norm,
+                               silu_and_mul)
+
+from .inputs import plan_prompts
 
 
 @dataclass(frozen=True)
@@ -117,8 +120,27 @@ class Qwen3:
         self.k_cache, self.v_cache, self.q_cache = kv_cache[0], kv_cache[1], query_cache
 
     # ------------------------------------------------------------------ pieces
-    def _prefill_attention(self, li, q, k, v, ctx: StepContext) -> torch.Tensor:
+    def _plan_prefill(self, ctx: StepContext):
+        """Query tiles of a step of prompts, and the cache rows of its keys where prompts have a cached prefix; None where
+        the kernel does not cover the model."""
+        D = self.shape.head_dim
+        if not ctx.is_prefill or self.dtype != torch.bfloat16 or D % 8 or D > 128:
+            return None
+        tiles = torch.from_numpy(plan_prompts(ctx.seq_lens_q, ctx.seq_lens_k)).pin_memory().to(self.device, non_blocking=True)
+        if ctx.seq_lens_q == ctx.seq_lens_k:
+            return tiles, None
+        BS = self.k_cache.shape[2]
+        at = torch.arange(BS, dtype=torch.int32, device=self.device)
+        rows = [(ctx.block_tables[b, :-(-n // BS), None] * BS + at).flatten()[:n] for b, n in enumerate(ctx.seq_lens_k)]
+        return tiles, torch.cat(rows).int()
+
+    def _prefill_attention(self, li, q, k, v, ctx: StepContext, plan) -> torch.Tensor:
         s = self.shape
+        if plan is not None:
+            tiles, rows = plan
+            if rows is not None:   # cached prefixes: the whole contexts come back from the cache
+                k, v = (gather_rows(c[li].flatten(2), rows).view(-1, s.kv_heads, s.head_dim) for c in (self.k_cache, self.v_cache))
+            return causal_attention(q, k, v, tiles, self.scale)
         lens_q, lens_k = ctx.seq_lens_q, ctx.seq_lens_k
         if lens_q == lens_k and len(set(lens_q)) == 1:
             B, n = len(lens_q), lens_q[0]
@@ -147,7 +169,7 @@ class Qwen3:
             off += nq
         return out.view(-1, s.heads * s.head_dim)
 
-    def _attention(self, li, p, x, pos32, ctx: StepContext) -> torch.Tensor:
+    def _attention(self, li, p, x, pos32, ctx: StepContext, plan) -> torch.Tensor:
         """zipage/models/qwen3.py:72-88 + zipage/layers/attention.py:69-104."""
         s = self.shape
         N = x.shape[0]
@@ -163,7 +185,7 @@ class Qwen3:
             if ctx.query_slot_mapping is not None:
                 store_query_cache(q, self.q_cache[li], ctx.query_slot_mapping)
             v = qkv[:, q_sz + kv_sz:].view(N, s.kv_heads, s.head_dim)
-            o = self._prefill_attention(li, q, k, v, ctx)
+            o = self._prefill_attention(li, q, k, v, ctx, plan)
         else:
             q = qk_norm_rope_store(qkv, pos32, self.cos, self.sin, p["qn"], p["kn"], s.heads,
                                    s.kv_heads, s.head_dim, s.eps, kc, vc, ctx.slot_mapping,
@@ -182,12 +204,13 @@ class Qwen3:
         pos32 = positions.to(torch.int32)
         hidden = F.embedding(input_ids, self.embed)
         resid = None
+        plan = self._plan_prefill(ctx)
         for li, p in enumerate(self.layers):
             if resid is None:
                 resid, h = hidden, rms_norm(hidden, p["ln1"], s.eps)
             else:
                 h, resid = rms_norm(hidden, p["ln1"], s.eps, resid)
-            hidden = self._attention(li, p, h, pos32, ctx)
+            hidden = self._attention(li, p, h, pos32, ctx, plan)
             h, resid = rms_norm(hidden, p["ln2"], s.eps, resid)
             hidden = F.linear(silu_and_mul(F.linear(h, p["wgu"])), p["wd"])
         h, _ = rms_norm(hidden, self.final_norm, s.eps, resid)

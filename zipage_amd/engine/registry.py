@@ -25,7 +25,7 @@ class Architecture:
 
 
 ARCHITECTURES = {a.name: a for a in (
-    Architecture("Qwen3ForCausalLM", Qwen3, Qwen3Shape, Qwen3Shape.from_config, ("LIB",), loads_weights=False),
+    Architecture("Qwen3ForCausalLM", Qwen3, Qwen3Shape, Qwen3Shape.from_config, ("LIB", "MODELS_LIB"), loads_weights=False),
     Architecture("Pedivik", Pedivik, PedivikShape, PedivikShape.from_config, ("MODELS_LIB", "LATENT_LIB")),
     Architecture("Kapolorn", Kapolorn, KapolornShape, KapolornShape.from_config,
                  ("MODELS_LIB", "GROUPED_LIB", "RECURRENT_LIB", "MOE_LIB")),

@@ -6,4 +6,4 @@ from .moe import Experts, small_linear  # noqa: F401
 from .recurrent import ChannelDelta, LinearAttention, MatrixMemory  # noqa: F401
 from .residual import embed_norm, normed_powers, relu_square, residual_norm, softcap, xielu  # noqa: F401
 from .rotary import Rotary  # noqa: F401
-from .runs import attention_form, gather_rows, run_attention  # noqa: F401
+from .runs import attention_form, causal_attention, gather_rows, run_attention  # noqa: F401

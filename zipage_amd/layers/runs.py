@@ -54,3 +54,17 @@ def run_attention(q: torch.Tensor, kv: torch.Tensor, heads: int, kv_heads: int, 
                      tiles.shape[0], heads, kv_heads, dim, extra, vdim, window or 0, chunk or 0, q.shape[0],
                      kv.shape[0], q.stride(0), kv.stride(0), 0 if shared is None else shared.stride(0), out.stride(0), float(scale), float(out_scale), _lib.dtype_tag(q), _lib.stream_ptr(q))
     return out
+
+
+def causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, tiles: torch.Tensor, scale: float) -> torch.Tensor:
+    """q (N, H, D), k and v (Nk, HK, D), rows may be part of wider ones; tiles (T, 4) int32 as `inputs.plan_prompts` makes
+    them.  A query sees its own position and those before it in its run.  Returns (N, H * D)."""
+    (N, H, D), (Nk, HK, _) = q.shape, k.shape
+    assert k.shape == v.shape == (Nk, HK, D) and q.dtype == k.dtype == v.dtype
+    assert all(t.stride(2) == 1 and t.stride(1) == D for t in (q, k, v))
+    assert tiles.dtype == torch.int32 and tiles.is_contiguous() and tiles.shape[1] == 4
+    out = torch.empty((N, H * D), dtype=q.dtype, device=q.device)
+    _lib.call_models("zp_causal_attention", _lib.dev_ptr(q), _lib.dev_ptr(k), _lib.dev_ptr(v), _lib.dev_ptr(out),
+                     _lib.dev_ptr(tiles), tiles.shape[0], H, HK, D, N, Nk, q.stride(0), k.stride(0), v.stride(0), out.stride(0),
+                     float(scale), _lib.dtype_tag(q), _lib.stream_ptr(q))
+    return out
