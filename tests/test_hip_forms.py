@@ -138,3 +138,36 @@ def test_causal_attention(dev, H, G, D):
     # bf16 keeps 8 bits: 2^-8 of the result; two planes of it 16: 2^-16 of each weight times its value's distance from the
     # result, and as much for the fp32 sums of scores up to 32
     assert bool(((got.view(N, H, D).cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * vv.abs().max()).all())
+
+
+# ------------------------------------------------------------------ rotary store of heads of 128
+# aligned rows take sixteen lanes a vector, fewer than 2^18 of them with a workgroup per sixteen; others take a wave a vector
+@pytest.mark.parametrize("N,Hq,Hkv", [(1, 1, 1), (37, 32, 8), (700, 5, 2), (2047, 64, 32), (2048, 64, 32)])
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+def test_rotary_store_of_wide_rows(dev, dtype, N, Hq, Hkv):
+    from zipage_amd.layers import qk_norm_rope_store
+    D, total, max_pos = 128, Hq + 2 * Hkv, 300
+    rows = _rand(N, total * D + 16, seed=1, dtype=dtype).to(dev)
+    odd = torch.empty(N * (total * D + 17) + 1, dtype=dtype, device=dev)[1:].view(N, -1)     # not on 16 bytes
+    odd[:, :total * D] = rows[:, :total * D]
+    qn, kn = (1 + 0.1 * _rand(D, seed=2).float()).to(dtype).to(dev), (1 + 0.1 * _rand(D, seed=3).float()).to(dtype).to(dev)
+    ang = torch.arange(max_pos)[:, None] * 1e4 ** (-torch.arange(0, D, 2) / D)[None]
+    cos, sin = ang.cos().to(dev), ang.sin().to(dev)
+    pos = (torch.arange(N, dtype=torch.int32) * 7 % max_pos).to(dev)
+    slots = torch.randperm(N + 8, generator=torch.Generator().manual_seed(2))[:N].int()
+    slots[::5] = -1
+    ring = torch.tensor([[i, i % 3, i // 3] if i % 2 == 0 and i < 12 else [-1] * 3 for i in range(N)], dtype=torch.int32).to(dev)
+    got = []
+    for x in (rows[:, :total * D], odd[:, :total * D]):
+        kc, vc = (torch.zeros(N + 8, 1, Hkv, D, dtype=dtype, device=dev) for _ in range(2))
+        qc = torch.zeros(3, 4, Hq, D, dtype=dtype, device=dev)
+        q, k = qk_norm_rope_store(x, pos, cos, sin, qn, kn, Hq, Hkv, D, 1e-6, kc, vc, slots.to(dev), qc, ring, return_k=True)
+        got.append([t.cpu() for t in (q, k, kc, vc, qc)])
+    assert torch.equal(got[0][3], got[1][3])
+    for a, b in zip(*got):
+        # the sums of squares differ in order: now and then a rounding falls the other way, here and once more behind the
+        # rotation, each at most an ulp of the pair's larger element
+        a, b = a.float(), b.float()
+        pair = torch.maximum(b.abs(), b.abs().roll(D // 2, -1))
+        ulp = 2.0 ** (-7 if dtype == BF16 else -10)
+        assert float((a != b).float().mean()) < 0.01 and bool(((a - b).abs() <= 2 * ulp * pair + 1e-6).all())

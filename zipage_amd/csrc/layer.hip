@@ -194,6 +194,65 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(QkArgs a) {
   }
 }
 
+// The same for heads of 128 in aligned rows: sixteen lanes a vector, eight elements a lane, so that every access is 16
+// bytes wide; the other half of a rotated pair is eight lanes on.  Bound by HBM: 8192 tokens of 32 + 16 heads move
+// 218 MB (2-byte accesses, a wave a vector: 110 us; now
+// 42).
+constexpr int kVecHead = 128, kVecs = kThreads / 16;     // vectors of a workgroup at a time
+template <typename T>
+__global__ __launch_bounds__(kThreads) void qk_norm_rope_wide_kernel(QkArgs a) {
+  const int n = blockIdx.x, j = threadIdx.x & 15, total = a.Hq + 2 * a.Hkv;
+  const int pos = min(max(a.positions[n], 0), a.max_position - 1);
+  const float* const turn_c = a.cos + (int64_t)pos * (kVecHead / 2) + (j & 7) * 8;
+  const float* const turn_s = a.sin + (int64_t)pos * (kVecHead / 2) + (j & 7) * 8;
+  float c[8], s[8], w[8];
+#pragma unroll
+  for (int i = 0; i < 8; i += 4) {
+    const float4 x = *(const float4*)(turn_c + i), y = *(const float4*)(turn_s + i);
+    c[i] = x.x, c[i + 1] = x.y, c[i + 2] = x.z, c[i + 3] = x.w;
+    s[i] = y.x, s[i + 1] = y.y, s[i + 2] = y.z, s[i + 3] = y.w;
+  }
+  int64_t slot = a.slot_mapping ? a.slot_mapping[n] : -1;
+  if (slot >= a.num_slots) slot = -1;
+  int ring_seq = -1, ring_slot = -1;
+  if (a.ring && a.q_cache && a.ring[n * 3] == n) {
+    ring_seq = a.ring[n * 3 + 1];
+    ring_slot = a.ring[n * 3 + 2];
+    if (ring_seq < 0 || ring_seq >= a.max_seqs || ring_slot < 0 || ring_slot >= a.window) ring_seq = -1;
+  }
+  const uint16_t* const row = (const uint16_t*)a.qkv + (int64_t)n * a.qkv_st + j * 8;
+  for (int hv = blockIdx.y * kVecs + (threadIdx.x >> 4); hv < total; hv += gridDim.y * kVecs) {
+    const u32x4 raw = *(const u32x4*)(row + (int64_t)hv * kVecHead);
+    if (hv >= a.Hq + a.Hkv) {          // V: plain copy into the cache
+      if (slot >= 0) *(u32x4*)((uint16_t*)a.v_cache + (slot * a.Hkv + (hv - a.Hq - a.Hkv)) * kVecHead + j * 8) = raw;
+      continue;
+    }
+    const bool is_q = hv < a.Hq;
+    float x[8], other[8], ss = 0.f;
+    unpack8<T>(raw, x);
+    unpack8<T>(*(const u32x4*)((const uint16_t*)(is_q ? a.qn_w : a.kn_w) + j * 8), w);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
+    const float rs = rsqrtf(row16_sum(ss) / (float)kVecHead + a.eps);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      x[i] = Elem<T>::rnd(Elem<T>::rnd(x[i] * rs) * w[i]);
+      other[i] = dpp_row_ror<8>(x[i]);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = j < 8 ? x[i] * c[i] - other[i] * s[i] : x[i] * c[i] + other[i] * s[i];
+    const u32x4 y = pack8<T>(x);
+    if (is_q) {
+      *(u32x4*)((uint16_t*)a.q_out + ((int64_t)n * a.Hq + hv) * kVecHead + j * 8) = y;
+      if (ring_seq >= 0)
+        *(u32x4*)((uint16_t*)a.q_cache + ring_seq * a.qc_sseq + ring_slot * a.qc_sslot + (int64_t)hv * kVecHead + j * 8) = y;
+    } else {
+      if (slot >= 0) *(u32x4*)((uint16_t*)a.k_cache + (slot * a.Hkv + (hv - a.Hq)) * kVecHead + j * 8) = y;
+      if (a.k_out) *(u32x4*)((uint16_t*)a.k_out + ((int64_t)n * a.Hkv + (hv - a.Hq)) * kVecHead + j * 8) = y;
+    }
+  }
+}
+
 }  // namespace
 
 #define ZP_16BIT_ONLY(name)                                           \
@@ -288,6 +347,21 @@ extern "C" int zp_qk_norm_rope_store(const void* qkv, void* q_out, void* k_out, 
   a.num_slots = num_slots; a.qc_sseq = qc_stride_seq; a.qc_sslot = qc_stride_slot; a.eps = eps;
   hipStream_t st = (hipStream_t)stream;
   const int total = Hq + 2 * Hkv;
+  bool wide = D == kVecHead && qkv_stride % 8 == 0 && (!query_cache || (qc_stride_seq % 8 == 0 && qc_stride_slot % 8 == 0));
+  for (const void* p : {qkv, (const void*)q_out, (const void*)k_out, (const void*)k_cache, (const void*)v_cache,
+                        (const void*)query_cache, q_norm_weight, k_norm_weight, (const void*)cos, (const void*)sin})
+    wide = wide && (uintptr_t)p % 16 == 0;
+  if (wide) {
+    // a workgroup per sixteen vectors (32 + 8 + 8 heads, three times sixteen in brackets: 256 tokens 3.5 us [4.4], 2048
+    // tokens 11.8 [12.0]) until the caches no longer hold them all (8192 tokens 45.1 [41.7])
+    const unsigned per = (int64_t)n * total < (1 << 18) ? kVecs : 3 * kVecs, gy = (total + per - 1) / per;
+    if (dtype == ZP_BF16)
+      hipLaunchKernelGGL((qk_norm_rope_wide_kernel<BF16>), dim3(n, gy), dim3(kThreads), 0, st, a);
+    else
+      hipLaunchKernelGGL((qk_norm_rope_wide_kernel<F16>), dim3(n, gy), dim3(kThreads), 0, st, a);
+    ZP_LAUNCH_CHECK();
+    return ZP_OK;
+  }
   const unsigned gy = (unsigned)((total + 3 * kWaves - 1) / (3 * kWaves));   // ~3 vectors per wave
   if (dtype == ZP_BF16)
     hipLaunchKernelGGL((qk_norm_rope_kernel<BF16>), dim3(n, gy), dim3(kThreads), 0, st, a);
