@@ -102,10 +102,10 @@ def _tiles(lens):
 
 # the scale joins the subtraction of the maximum: a negative one turns the queries round, zero takes them away
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-30, 0.25])
-@pytest.mark.parametrize("H,G,D,V", [(2, 1, 40, 24), (4, 2, 128, 128), (3, 3, 136, 136)])
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 40, 24), (2, 2, 64, 64), (3, 1, 128, 56), (4, 2, 128, 128), (3, 3, 136, 136)])
 def test_runs_of_any_scale(dev, H, G, D, V, scale):
     from zipage_amd.layers import run_attention
-    lens = [(1, 1), (63, 63), (65, 65), (130, 200)]
+    lens = [(1, 1), (63, 63), (65, 65), (32, 64), (33, 129), (130, 200)]
     N, M = (sum(t) for t in zip(*lens))
     q, k = (_rand(N, H, D, seed=1), _rand(M, G, D, seed=2))
     v = _rand(M, G, V, seed=3)

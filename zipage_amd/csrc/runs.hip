@@ -68,6 +68,17 @@ template <int DKS, int VCB, int MAPS> struct TileStage {
   static constexpr int kBytes = kBuffers * kElems * 2;
 };
 
+// A lane holds 4 columns of each of two column tiles; groups of sixteen lanes swap halves with their neighbours, so that each
+// ends with 8 columns of one tile: those from (c + (g & 1)) * 16 + (g >> 1) * 8 on for tiles c and c + 1.
+__device__ __forceinline__ void eight_columns(const f32x4& even, const f32x4& odd, float by, float (&r)[8]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(even[i] * by), __float_as_uint(odd[i] * by), false, false);
+    r[i] = __uint_as_float(both[0]);
+    r[4 + i] = __uint_as_float(both[1]);
+  }
+}
+
 enum { kNoCap, kCap, kBoundedCap };   // of the scores, see SoftCap
 
 // Column tile t of a wave: 16 queries, map t % MAPS of the head (differential attention has two, over the same
@@ -336,17 +347,10 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
       const float2* turns = a.turns;
       asm volatile("" : "+s"(turns));                          // nothing of the way back is computed before the loop
       const uint16_t* gate = MAPS == 2 && a.gate ? a.gate + (int64_t)(q0 + qi) * a.g_st + h * a.V : nullptr;
-      // a lane holds 4 columns of each of two tiles; groups g and g ^ 1 swap halves, so that each ends with 8 of one
 #pragma unroll
       for (int c = 0; c < VCB * 8; c += 2) {
         float r[8];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const auto both = __builtin_amdgcn_permlane16_swap(__float_as_uint(o[qt * MAPS][c][i] * inv[0]),
-                                                             __float_as_uint(o[qt * MAPS][c + 1][i] * inv[0]), false, false);
-          r[i] = __uint_as_float(both[0]);
-          r[4 + i] = __uint_as_float(both[1]);
-        }
+        eight_columns(o[qt * MAPS][c], o[qt * MAPS][c + 1], inv[0], r);
         const int col = (c + (g & 1)) * 16 + (g >> 1) * 8;
         if (!row || col >= a.V) continue;
         if (kTurns && turns) turn_back8(r, turns + ((int64_t)(q0 + qi) * a.V + col) / 2);
@@ -361,6 +365,333 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
     }
   }
 }
+
+// ------------------------------------------------------------------ values of at most 64, one map, no cap
+// Here the products of a tile's keys run while the exponentials of the tile before take their turn, which needs the scores
+// of two tiles in registers: with 64 value columns they are there, with 128 they are not (heads of 128, 8 prompts of 2048
+// tokens: 435 -> 423 us, with weights of 17 bits 448 -> 470).  Rows go from memory into LDS without passing through
+// registers.  Bound by the vector units' issue (a product takes half of its 16 cycles there, too, an exponential 8).
+// Heads of 64, 8 prompts of about 1800 tokens, 16 heads, with the rotary store: 181 -> 145 us (236 before both kernels'
+// reads were ahead of their products); 4 of 2048, 32 heads: 163 -> 120 (222).
+//
+// Rows of CH 16-byte pieces (8 or 16) as loads leave them in LDS, 1 KB at a time with GAP bytes between: four rows after
+// one another interleave their pieces by four, so that a lane's pieces and the column tiles are immediate offsets.  With
+// eight rows per load the pieces of the second four lie FLIP apart.  What reads them falls into different banks: sixteen
+// rows of one piece (keys), twice four rows of two (values, transposed).
+template <int CH, int FLIP, int GAP> struct Staged {
+  static constexpr int kRows = 64 / CH;                        // per load
+  static constexpr int kLoad = 1024 + GAP, kBytes = kTileK / kRows * kLoad;
+  __device__ static __forceinline__ int row(int lane) { return CH == 16 ? lane >> 2 & 3 : (lane >> 5) * 4 + (lane >> 2 & 3); }
+  __device__ static __forceinline__ int piece(int lane) {
+    return CH == 16 ? (lane >> 4) * 4 + (lane & 3) : (lane >> 4 & 1) * 4 + ((lane & 3) ^ FLIP * (lane >> 5));
+  }
+  // where pieces p of 0 .. 3 of row r begin; those from 4 on are 256 bytes further for every four
+  __device__ static __forceinline__ int at(int r, int p) {
+    if (CH == 16) return (r >> 2) * kLoad + (r & 3) * 64 + p * 16;
+    return (r >> 3) * kLoad + (r >> 2 & 1) * 512 + (r & 3) * 64 + (p ^ FLIP * (r >> 2 & 1)) * 16;
+  }
+};
+constexpr int kFlowV = 64;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+// The row at `from` and those behind it; every lane reads within rows that are there: the bound is none of the buffer's.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const void* from) {
+  return __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, 0x7fffffff, 0x00020000);
+}
+__device__ __forceinline__ void rows_to_lds(__amdgpu_buffer_rsrc_t rows, char* to, int lane_at, int at) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_ptr_t)to, 16, lane_at, at, 0, 0);
+}
+
+// FINE as above.
+template <int DKS, bool FINE>
+__global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
+  extern __shared__ __align__(16) char lds_raw[];
+  typedef Staged<DKS * 4, 1, DKS == 4 ? 16 : 32> KL;
+  typedef Staged<8, 2, 0> VL;
+  constexpr int VT = kFlowV / 16;                              // column tiles of the values
+  constexpr int kQK = 4 * DKS * 2, kPV = VT * 2;               // products of a tile's keys, of half its values
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x % a.H, tile = blockIdx.x / a.H;     // one head's tiles share an L2 when H % 8 == 0
+  const int q0 = a.tiles[tile * 4], nq = min(a.tiles[tile * 4 + 1], kTileQ);
+  const int kb = a.tiles[tile * 4 + 2], rel = a.tiles[tile * 4 + 3];
+  // host-made descriptors: rows outside the buffers are not touched
+  if (q0 < 0 || nq <= 0 || kb < 0 || rel < 0 || (int64_t)q0 + nq > a.q_rows || (int64_t)kb + rel + nq > a.k_rows) return;
+  // the scale joins the subtraction of the maximum, for which it has to be positive: a negative one turns the queries
+  // round, zero takes them away
+  const float by = a.scale * 1.44269504088896f, factor = by == 0.f ? 1.f : fabsf(by);
+  const uint32_t flip = by < 0.f ? 0x80008000u : 0u, kept = by == 0.f ? 0u : ~0u;
+  const int hk = h / (a.H / a.HK);
+  const uint16_t* const kbase = a.k + (int64_t)kb * a.kv_st + hk * a.D;
+  const uint16_t* const vbase = a.v + (int64_t)kb * a.v_st + hk * a.V;
+
+  const int w0 = wave * 32;                                    // this wave's first query
+  const int first = first_seen(rel, a.window, a.chunk), last = rel + nq - 1;    // keys that any query sees
+  const int lo = first_seen(rel + w0, a.window, a.chunk), lo_last = first_seen(rel + w0 + 31, a.window, a.chunk);
+  const int tiles = (last - first) / kTileK + 1;
+  // tiles that queries of the wave see; none: they begin behind the last one
+  const int seen0 = w0 < nq ? (lo - first) / kTileK : tiles + 1;
+  const int seen1 = w0 < nq ? (rel + min(w0 + 32, nq) - 1 - first) / kTileK : tiles + 1;
+
+  u32x4 qf[2][DKS];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const int qi = min(w0 + t * 16 + l16, nq - 1);
+    const uint16_t* q = a.q + (int64_t)(q0 + qi) * a.q_st + h * a.D;
+#pragma unroll
+    for (int ks = 0; ks < DKS; ++ks) {
+      // past the head's end: the key columns there hold other elements, against zeros here
+      const int c = ks * 32 + g * 8;
+      qf[t][ks] = (*(const u32x4*)(q + (c < a.D ? c : 0)) & kept) ^ flip;
+      if (c >= a.D) qf[t][ks] = u32x4{0u, 0u, 0u, 0u};
+    }
+  }
+  f32x4 o[2][VT];
+  float m[2], l[2];
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    m[t] = -INFINITY;
+    l[t] = 0.f;
+#pragma unroll
+    for (int c = 0; c < VT; ++c) o[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+  }
+
+  // ---- a tile's rows from memory into LDS; rows past the last one are the last one again
+  char* const kl = lds_raw;
+  char* const vl = lds_raw + 2 * KL::kBytes;
+  // what follows from the lane is worked out anew: kept, it would not leave the products enough registers
+  auto lane_again = [&] {
+    int i = lane;
+    asm volatile("" : "+v"(i));
+    return i;
+  };
+  auto lane_at = [&](auto layout, int64_t stride, int cols) {
+    typedef decltype(layout) L;
+    const int i = lane_again();
+    return L::row(i) * (int)stride * 2 + (L::piece(i) * 8 < cols ? L::piece(i) * 16 : 0);
+  };
+  const int klane = lane_at(KL{}, a.kv_st, a.D), vlane = lane_at(VL{}, a.v_st, a.V);
+  auto stage = [&](auto layout, char* tile, const uint16_t* rows, int64_t stride, int cols, int k0, int whole) {
+    typedef decltype(layout) L;
+    constexpr int kLoads = kTileK / L::kRows / 4;              // of each wave
+    tile += wave * L::kLoad;
+    if (k0 + kTileK - 1 <= last && stride < 1 << 24) {
+      const __amdgpu_buffer_rsrc_t from = rows_at(rows + (int64_t)(k0 + wave * L::kRows) * stride);
+#pragma unroll
+      for (int n = 0; n < kLoads; ++n) rows_to_lds(from, tile + n * 4 * L::kLoad, whole, n * 8 * L::kRows * (int)stride);
+      return;
+    }
+    const int i = lane_again(), row = L::row(i), col = L::piece(i) * 8 < cols ? L::piece(i) * 16 : 0;
+#pragma unroll 1
+    for (int n = 0; n < kLoads; ++n) {
+      const int from = min(k0 + (n * 4 + wave) * L::kRows, last);
+      const int at = min(row, last - from) * (int)stride * 2 + col;
+      rows_to_lds(rows_at(rows + (int64_t)from * stride), tile + n * 4 * L::kLoad, at, 0);
+    }
+  };
+  auto stage_keys = [&](int j) { stage(KL{}, kl + (j & 1) * KL::kBytes, kbase, a.kv_st, a.D, first + j * kTileK, klane); };
+  auto stage_values = [&](int j) { stage(VL{}, vl + (j & 1) * VL::kBytes, vbase, a.v_st, a.V, first + j * kTileK, vlane); };
+
+  // ---- one tile: its weights and what its values add, and meanwhile the scores of the next one
+  // groups of lanes hold keys 16 (i / 4) + 4 g + i % 4; values leave LDS transposed, lane l16 with column l16 of four keys
+  const int kread = KL::at(l16, g);
+  const int vread = VL::at(4 * g + (l16 >> 2), (l16 & 3) >> 1) + (l16 & 1) * 8;
+  const int vread_odd = VL::at(4 * g + (l16 >> 2), 2 + ((l16 & 3) >> 1)) + (l16 & 1) * 8;      // of odd column tiles
+  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+  typedef float Scores[2][16];
+  auto step = [&](int j, auto here_, auto next_, Scores& p, Scores& after) {
+    constexpr bool HERE = here_.value, NEXT = next_.value;
+    const char* const kt = kl + ((j + 1) & 1) * KL::kBytes + kread;
+    const char* const vt = vl + (j & 1) * VL::kBytes;
+    f32x4 s[2][4];
+    // operands leave LDS kAhead ahead of their two products
+    constexpr int kAhead = 4, kRing = kAhead + 1;
+    u32x4 kf[kRing], vf[kRing];
+    // n: 16 keys n / DKS, step n % DKS
+    auto read_keys = [&](int n) {
+      if (n < 4 * DKS) kf[n % kRing] = *(const u32x4*)(kt + n / DKS * (16 / KL::kRows) * KL::kLoad + n % DKS * 256);
+    };
+    // n: 32 keys n / VT, column tile n % VT
+    auto read_values = [&](int n) {
+      if (n >= 2 * VT) return;
+      const int c = n % VT, r = n / VT * 32;
+      const char* const at = vt + (c >> 1) * 256 + (c & 1 ? vread_odd : vread);
+      const uint2 x = read_transposed((const uint16_t*)(at + r / VL::kRows * VL::kLoad));
+      const uint2 y = read_transposed((const uint16_t*)(at + (r + 16) / VL::kRows * VL::kLoad));
+      vf[n % kRing] = u32x4{x.x, x.y, y.x, y.y};
+    };
+    u32x4 pf[2][2], pl[2][2];
+    // product n of the next tile's keys: tile of keys n / (2 DKS), step, query tile
+    auto key_product = [&](int n) {
+      const int tt = n / (2 * DKS), ks = n / 2 % DKS, t = n & 1;
+      if (t == 0) read_keys(n / 2 + kAhead);
+      if (ks == 0) s[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      s[t][tt] = mfma_bf16(kf[n / 2 % kRing], qf[t][ks], s[t][tt]);
+    };
+    auto value_product = [&](int half, int n) {
+      const int c = n / 2, t = n & 1, v = half * VT + c;
+      if (t == 0) read_values(v + kAhead);
+      o[t][c] = mfma_bf16(vf[v % kRing], pf[t][half], o[t][c]);
+      if constexpr (FINE) o[t][c] = mfma_bf16(vf[v % kRing], pl[t][half], o[t][c]);
+    };
+    float ms[2];
+    // weights of keys pair d of half, both query tiles
+    auto weights = [&](int half, int n) {
+      const int t = n & 1, d = n / 2, i = half * 8 + d * 2;
+      const float x = __builtin_amdgcn_exp2f(fmaf(p[t][i], factor, -ms[t]));
+      const float y = __builtin_amdgcn_exp2f(fmaf(p[t][i + 1], factor, -ms[t]));
+      const uint32_t w = pack_bf16(x, y);
+      pf[t][half][d] = w;
+      if constexpr (FINE) pl[t][half][d] = pack_bf16(x - __uint_as_float(w << 16), y - __uint_as_float(w & 0xffff0000u));
+    };
+    if constexpr (NEXT)
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) read_keys(i);
+    if constexpr (HERE) {
+      const int k0 = first + j * kTileK;
+      if (k0 + kTileK - 1 > rel + w0 || k0 < lo_last) {        // some query of the wave does not see all these keys
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+          const int i0 = lane_again(), pos = rel + min(w0 + t * 16 + (i0 & 15), nq - 1);
+          const int low = first_seen(pos, a.window, a.chunk);
+          const int from = low - k0 - 4 * (i0 >> 4), span = pos - low;   // keys low .. pos are seen
+#pragma unroll
+          for (int i = 0; i < 16; ++i)
+            if ((unsigned)((i >> 2) * 16 + (i & 3) - from) > (unsigned)span) p[t][i] = -INFINITY;
+        }
+      }
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        float mx = -INFINITY;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, p[t][i]);
+        mx *= factor;
+        if (__any(mx > m[t])) {                                // in any lane: seldom after the first keys
+          mx = fmaxf(m[t], mx);
+          mx = fmaxf(mx, lane_xor16(mx));
+          mx = fmaxf(mx, lane_xor32(mx));
+          const float f = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[t] - mx);
+          m[t] = mx;
+          l[t] *= f;
+#pragma unroll
+          for (int c = 0; c < VT; ++c) o[t][c] *= f;
+        }
+        ms[t] = m[t] == -INFINITY ? 0.f : m[t];                // a query whose window starts later
+      }
+    }
+    constexpr int kEarly = kQK * 3 / 4, kLate = kQK - kEarly;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (NEXT)
+#pragma unroll
+        for (int e = i * kEarly / 8; e < (i + 1) * kEarly / 8; ++e) key_product(e);
+      if constexpr (HERE) weights(0, i);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (HERE)
+#pragma unroll
+      for (int i = 0; i < kAhead; ++i) read_values(i);
+    f32x4 sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    auto sums = [&](int half) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        sum[t] = mfma_bf16(ones, pf[t][half], sum[t]);
+        if constexpr (FINE) sum[t] = mfma_bf16(ones, pl[t][half], sum[t]);
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      constexpr int kAll = (NEXT ? kLate : 0) + (HERE ? kPV : 0);
+#pragma unroll
+      for (int e = i * kAll / 8; e < (i + 1) * kAll / 8; ++e) {
+        if (NEXT && e < kLate) key_product(kEarly + e);
+        else if constexpr (HERE) value_product(0, e - (NEXT ? kLate : 0));
+      }
+      if constexpr (HERE) {
+        if (i == 0) sums(0);
+        weights(1, i);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (HERE) {
+      sums(1);
+#pragma unroll
+      for (int e = 0; e < kPV; ++e) value_product(1, e);
+#pragma unroll
+      for (int t = 0; t < 2; ++t) l[t] += sum[t][0];
+    }
+    if constexpr (NEXT)
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) after[t][i] = s[t][i >> 2][i & 3];
+  };
+
+  typedef std::integral_constant<bool, true> yes;
+  typedef std::integral_constant<bool, false> no;
+  auto meet = [] {                                             // this wave's rows are there and its reads done, then everyone's
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Every wave takes the tiles from -1 on one by one, stages its share of what the next one needs (over what was used
+  // before the last barrier) and meets the others once for each; which of them it works on is its own matter.
+  int j = -1;
+  Scores p0, p1;
+  auto tile_of = [&](auto here, auto next, Scores& p, Scores& after) {
+    if (j + 2 < tiles) stage_keys(j + 2);
+    if (j + 1 < tiles) stage_values(j + 1);
+    step(j, here, next, p, after);
+    meet();
+    ++j;
+  };
+  stage_keys(0);
+  meet();
+#pragma unroll 1
+  while (j < tiles && j != seen0 - 1) tile_of(no{}, no{}, p0, p1);
+  if (j < tiles) {
+    tile_of(no{}, yes{}, p1, p0);
+#pragma unroll 1
+    while (j + 2 <= seen1) {
+      tile_of(yes{}, yes{}, p0, p1);
+      tile_of(yes{}, yes{}, p1, p0);
+    }
+    if (j < seen1) {
+      tile_of(yes{}, yes{}, p0, p1);
+      tile_of(yes{}, no{}, p1, p0);
+    } else {
+      tile_of(yes{}, no{}, p0, p1);
+    }
+#pragma unroll 1
+    while (j < tiles) tile_of(no{}, no{}, p0, p1);
+  }
+
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    if (a.sinks) l[t] += __builtin_amdgcn_exp2f(a.sinks[h] * 1.44269504088896f - m[t]);
+    const float inv = l[t] > 0.f ? a.out_scale / l[t] : 0.f;
+    const int qi = w0 + t * 16 + l16;
+    uint16_t* const out = a.out + (int64_t)(q0 + qi) * a.o_st + h * a.V;
+#pragma unroll
+    for (int c = 0; c < VT; c += 2) {
+      float r[8];
+      eight_columns(o[t][c], o[t][c + 1], inv, r);
+      const int col = (c + (g & 1)) * 16 + (g >> 1) * 8;
+      if (qi >= nq || col >= a.V) continue;                    // every lane took part in the swaps
+      if (a.turns) turn_back8(r, a.turns + ((int64_t)(q0 + qi) * a.V + col) / 2);
+      Vec8<BF16>::st(out, col, r);
+    }
+  }
+}
+
+template <int DKS, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
+  constexpr int smem = 2 * (Staged<DKS * 4, 1, DKS == 4 ? 16 : 32>::kBytes + Staged<8, 2, 0>::kBytes);
+  static_assert(smem <= 64 * 1024, "no attribute needed");
+  hipLaunchKernelGGL((run_flow_kernel<DKS, FINE>), dim3((unsigned)a.T * a.H), dim3(256), smem, st, a);
+  ZP_LAUNCH_CHECK();
+  return ZP_OK;
+}
+
 
 template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
 int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
@@ -379,6 +710,8 @@ int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
 
 template <bool SHARED, int CAP> int launch_one_map(const TilesArgs& a, hipStream_t st) {
   const int dk = (a.D + a.P + 31) / 32;
+  if constexpr (!SHARED && CAP == kNoCap)
+    if (dk <= 4 && a.V <= kFlowV) return dk <= 2 ? launch_flow<2, false>(a, st) : launch_flow<4, false>(a, st);
   if (a.V <= 128) {
     if (dk <= 2) return launch_run_tiles<2, 1, 2, 1, SHARED, CAP>(a, st);
     if (dk <= 4) return launch_run_tiles<4, 1, 2, 1, SHARED, CAP>(a, st);
@@ -474,6 +807,6 @@ extern "C" int zp_causal_attention(const void* q, const void* k, const void* v, 
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, tiles, nullptr, T, H, HK,
                  D, 0, D, 0, 0, q_rows, k_rows, q_stride, k_stride, v_stride, 0, out_stride, scale, 1.f, 0.f, 0.f, 0.f, D,
                  nullptr, 0, nullptr};
-  if (D <= 64) return launch_run_tiles<2, 1, 2, 1, false, kNoCap, true>(a, (hipStream_t)stream);
+  if (D <= kFlowV) return launch_flow<2, true>(a, (hipStream_t)stream);
   return launch_run_tiles<4, 1, 2, 1, false, kNoCap, true>(a, (hipStream_t)stream);
 }
