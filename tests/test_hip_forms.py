@@ -171,3 +171,45 @@ def test_rotary_store_of_wide_rows(dev, dtype, N, Hq, Hkv):
         pair = torch.maximum(b.abs(), b.abs().roll(D // 2, -1))
         ulp = 2.0 ** (-7 if dtype == BF16 else -10)
         assert float((a != b).float().mean()) < 0.01 and bool(((a - b).abs() <= 2 * ulp * pair + 1e-6).all())
+
+
+# ------------------------------------------------------------------ delta rule over runs
+# operands enter the bf16 matrix cores in three planes: the state has to stay as good as fp32's
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 128, 128), (2, 2, 32, 96), (3, 1, 64, 32), (1, 1, 128, 64)])
+def test_delta_state_of_runs(dev, H, G, D, V):
+    import types
+    from zipage_amd.engine.qwen3 import Segments
+    from zipage_amd.layers import ChannelDelta
+    W, taps, counts = 64, 2, [16, 47, 100]
+    m, n = ChannelDelta(W, H, G, D, V, taps, 1e-3), sum(counts)
+    r = lambda *s, seed, std=1.0: _rand(*s, seed=seed, std=std)
+    w = {"q": r(G * D, W, seed=1, std=.2), "k": r(G * D, W, seed=2, std=.2), "v": r(H * V, W, seed=3, std=.2),
+         "q.conv": r(G * D, taps, seed=4), "k.conv": r(G * D, taps, seed=5), "v.conv": r(H * V, taps, seed=6),
+         "b": r(H, W, seed=7, std=.2), "A_log": r(H, seed=8, std=.5), "norm": 1 + r(V, seed=9, std=.3),
+         "a1": r(5, W, seed=10, std=.1), "a2": r(H * D, 5, seed=11, std=.4), "dt_bias": -3 + 6 * r(H * D, seed=12),
+         "g1": r(7, W, seed=13, std=.1), "g2": r(H * V, 7, seed=14, std=.4), "o": r(W, H * V, seed=15)}
+    into, _ = m.load(w, BF16, dev, W)
+    proj = (r(n, W, seed=16).float() @ into.float().cpu().T).to(BF16).to(dev)
+    state = m.allocate(len(counts), BF16, dev)
+    rows = torch.tensor([sum(counts[:i]) for i in range(len(counts))], dtype=torch.int32)
+    at = lambda x: torch.as_tensor(x, dtype=torch.int32).to(dev)
+    seg = Segments(at(rows), at(counts), at(range(len(counts))), at([0] * len(counts)), first_row=0, longest=max(counts), max_count=0)
+    m.scan(proj, state, types.SimpleNamespace(segments=None, run_segments=seg), torch.empty(n, H * V, dtype=BF16, device=dev))
+    P, head = proj.double().cpu(), torch.arange(H) // (H // G)
+    low = torch.nn.functional.linear(proj[:, m.low_at:m.low_at + m.low_rank], m.low).double().cpu()
+    a = low[:, :H * D].view(n, H, D) + w["dt_bias"].double().view(H, D)
+    g = torch.exp(-torch.exp(w["A_log"].double())[None, :, None] * torch.nn.functional.softplus(a))
+    for i, c in enumerate(counts):
+        p, gg = P[rows[i]:rows[i] + c], g[rows[i]:rows[i] + c]
+        conv = lambda f, t, k: K.short_conv(p[:, f:t], w[k + ".conv"].double())
+        k = K.unit(conv(G * D, 2 * G * D, "k").view(c, G, D))[:, head]
+        v = conv(2 * G * D, 2 * G * D + H * V, "v").view(c, H, V)
+        beta, S = torch.sigmoid(p[:, m.b_at:m.b_at + H]), torch.zeros(H, D, V, dtype=torch.float64)
+        for t in range(c):
+            S = gg[t][:, :, None] * S
+            u = beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
+            S = S + k[t][:, :, None] * u[:, None, :]
+        # roundings of 2^-24 by the products, decays and unit vectors of the tokens that a state remembers; a product of
+        # planes that is left out costs 2^-17 and more
+        err = (state[0][i].double().cpu().view(H, D, V) - S).norm() / S.norm()
+        assert float(err) < 2.0 ** -19, float(err)

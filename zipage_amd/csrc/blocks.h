@@ -43,6 +43,80 @@ template <int KT, int NC> __device__ __forceinline__ void store_state(const f32x
       for (int r = 0; r < 4; ++r) state[(int64_t)(16 * kt + 4 * g + r) * dv + col0 + nc * 16 + l16] = S[kt][nc][r];
 }
 
+// An fp32 operand in three bf16 planes: each is what those before it leave, rounded to eight bits and a sign, so that they
+// hold more than its 24 bits, and the products of the first with all, of the second with the first two and of the third with
+// the first miss less than 2^-26 of a product.
+struct Planes {
+  uint2 hi, mid, lo;
+  __device__ __forceinline__ Planes(const f32x4& x) {
+    f32x4 r = x;
+    hi = rounded(r);
+    r = rest(r, hi);
+    mid = rounded(r);
+    lo = rounded(rest(r, mid));
+  }
+  __device__ static __forceinline__ uint2 rounded(const f32x4& x) { return uint2{pack_bf16(x[0], x[1]), pack_bf16(x[2], x[3])}; }
+  // x minus its rounded values, exactly: the dot product of a pair of them with (-1, 0) or (0, -1) is added to x, which saves
+  // taking the pair apart.  The factors are kept from the compiler, which would make an immediate of -1 that stands for
+  // another pair.
+  __device__ static __forceinline__ f32x4 rest(const f32x4& x, const uint2& p) {
+    uint32_t first = 0x0000bf80u, second = 0xbf800000u;
+#ifdef __HIP_DEVICE_COMPILE__
+    asm("" : "+s"(first));
+    asm("" : "+s"(second));
+#endif
+    return f32x4{plus_dot(p.x, first, x[0]), plus_dot(p.x, second, x[1]), plus_dot(p.y, first, x[2]), plus_dot(p.y, second, x[3])};
+  }
+  __device__ static __forceinline__ float plus_dot(uint32_t a, uint32_t b, float c) {
+    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(zp_bf16x2, a), __builtin_bit_cast(zp_bf16x2, b), c, false);
+  }
+};
+// A right operand of 16 of the contraction for left ones that lie as [64 lanes][hi 4, mid 4], [64][lo 4]: the bf16 matrix
+// cores take 32, so planes go in pairs.
+constexpr int kPairFloats = 384;               // of such a left operand
+struct PlanePairs {
+  u32x4 hh, mm, ll, hm;
+  __device__ __forceinline__ PlanePairs(const f32x4& x) {
+    const Planes p(x);
+    hh = u32x4{p.hi.x, p.hi.y, p.hi.x, p.hi.y};
+    mm = u32x4{p.mid.x, p.mid.y, p.mid.x, p.mid.y};
+    ll = u32x4{p.lo.x, p.lo.y, p.lo.x, p.lo.y};
+    hm = u32x4{p.hi.x, p.hi.y, p.mid.x, p.mid.y};
+  }
+  __device__ __forceinline__ void add(const u32x4& left, const uint2& lo, f32x4& c) const {
+    c = mfma_bf16(left, ll, c);
+    c = mfma_bf16(u32x4{lo.x, lo.y, lo.x, lo.y}, hm, c);
+    c = mfma_bf16(left, mm, c);
+    c = mfma_bf16(left, hh, c);
+  }
+  // two at a time: each waits for the one before
+  __device__ __forceinline__ void add(const u32x4 (&left)[2], const uint2 (&lo)[2], f32x4& c, f32x4& d) const {
+    c = mfma_bf16(left[0], ll, c);
+    d = mfma_bf16(left[1], ll, d);
+    c = mfma_bf16(u32x4{lo[0].x, lo[0].y, lo[0].x, lo[0].y}, hm, c);
+    d = mfma_bf16(u32x4{lo[1].x, lo[1].y, lo[1].x, lo[1].y}, hm, d);
+    c = mfma_bf16(left[0], mm, c);
+    d = mfma_bf16(left[1], mm, d);
+    c = mfma_bf16(left[0], hh, c);
+    d = mfma_bf16(left[1], hh, d);
+  }
+};
+// x is computed before what follows, whoever uses it.
+__device__ __forceinline__ void settle(u32x4& x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+v"(x));
+#endif
+}
+// A stretch with N products ends here: what else it holds is spread over them.
+template <int N, int PER> __device__ __forceinline__ void spread_over_products() {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);      // a product
+    __builtin_amdgcn_sched_group_barrier(0x002, PER, 0);    // vector instructions
+  }
+  __builtin_amdgcn_sched_barrier(0);
+}
+
 // Sum of squares of each of the block's 16 tokens over the wave's columns; lane l16 == 0 of group g leaves
 // tokens 4 g .. 4 g + 3 in `red` (16 floats per wave).
 template <int NC> __device__ __forceinline__ void block_squares(const f32x4 (&o)[NC], float* red, int wave) {

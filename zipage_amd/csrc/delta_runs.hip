@@ -21,9 +21,9 @@ struct RunArgs {
   int row0;      // first token row of the first segment
 };
 
-// [-W | G q] and the keys as left operands, U0 as a result tile, P, the block's decays; whole KBs
+// [-W | G q] and the keys as left operands, U0 as a result tile, P's planes, the block's decays; whole KBs
 __host__ __device__ inline constexpr int block_floats(int dk, int dv) {
-  return (kBlock * (3 * dk + dv) + kBlock * kBlock + dk + 255) / 256 * 256;
+  return (kBlock * (3 * dk + dv) + kPairFloats + dk + 255) / 256 * 256;
 }
 
 template <int TAPS>
@@ -178,8 +178,8 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
   float* const oWQ = ra.ws + base;             // [2][dk / 16][64 lanes][4]
   float* const oK = oWQ + 2 * kBlock * dk;     // [dk / 16][64][4]
   float* const oU = oK + kBlock * dk;          // [dv / 16][64][4]
-  float* const oP = oU + kBlock * dv;          // [64][4]
-  float* const oG = oP + kBlock * kBlock;      // [dk]
+  float* const oP = oU + kBlock * dv;          // [64][hi 4, mid 4], [64][lo 4]
+  float* const oG = oP + kPairFloats;          // [dk]
   float w[kBlock];
   auto substitute = [&](int t, float b) {      // w_t = b - sum_{s < t} A[t, s] w_s
     float x[4] = {b, 0.f, 0.f, 0.f};
@@ -225,7 +225,11 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
     for (int g = 0; g < 4; ++g)
       *(f32x4*)(oU + ((v >> 4) * 64 + g * 16 + (v & 15)) * 4) = f32x4{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
   }
-  if (tid < 64) *(f32x4*)(oP + tid * 4) = *(const f32x4*)(Ps + (tid & 15) * kBlock + (tid >> 4) * 4);
+  if (tid < 64) {
+    const Planes x(*(const f32x4*)(Ps + (tid & 15) * kBlock + (tid >> 4) * 4));
+    *(u32x4*)(oP + tid * 4) = u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y};
+    *(uint2*)(oP + 256 + tid * 2) = x.lo;
+  }
   __syncthreads();
   for (int i = tid; i < 2 * kBlock * dk / 4; i += 256) {       // lane (g, row) of tile kt: columns 16 kt + 4 g ..
     const int tile = i >> 6, l = i & 63, kt = tile & (dk / 16 - 1);
@@ -233,27 +237,37 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
   }
 }
 
-// A head's blocks, one after the other: a block's operands come straight into LDS while the block before it is
-// worked on; its rows are normed and stored behind the next meeting of the waves, which the norm needs too.
+// A head's blocks, one after the other, a wave 16 columns of the state.  On the fp32 matrix cores the products would be the
+// bound (208 of 32 cycles a block on each SIMD, which keep its vector units idle as well), so operands are split into
+// three bf16 planes: the products that count take a quarter of that, beside the vector units.  The state is split
+// where it is updated, what comes from memory by all waves together, a block ahead and under the products with the state;
+// rows are normed and stored behind the next meeting of the waves, which the norm needs too.  What bounds it now is a wave's
+// chain of work: two per SIMD are all there are (twice the columns per wave, one per SIMD: 2 to 12 % more time in all).
+// 8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1161 -> 1106 us, one of them 566 -> 491; error of the
+// state against 64 bits 4.0e-7 -> 3.6e-7 of its size.
 template <int KT, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
   const zp_delta& a = ra.d;
-  constexpr int NC = 2, dk = 16 * KT, dv = 32 * NW, size = block_floats(dk, dv);
+  constexpr int dk = 16 * KT, dv = 16 * NW, size = block_floats(dk, dv), J = KT / 2;
+  constexpr int kSplit = 3 * kBlock * dk, kRest = size - kSplit;      // floats of a block: operands to be split, the others
+  constexpr int kP = kBlock * dv, kG = kP + kPairFloats;              // in the rest, behind U0
+  constexpr int kPlanes = 3 * KT * 384, kMine = (3 * KT + NW - 1) / NW;      // floats of a block's planes; tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  float* const red = lds + 2 * size;           // [2][NW * 16]
+  float* const split = lds;                    // [2][kSplit]
+  float* const rest = split + 2 * kSplit;      // [3][kRest]
+  float* const planes = rest + 3 * kRest;      // [2][kPlanes]
+  float* const red = planes + 2 * kPlanes;     // [2][NW * 16]
   const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
   const Segment sg = segment_of(a.seg, seg);
   if (sg.count <= 0 || sg.row < ra.row0) return;
   const int64_t item = (int64_t)sg.slot * a.heads + h;
   float* const state = a.state + item * ((int64_t)dk * dv);
-  const int col0 = wave * 16 * NC;
-  f32x4 S[KT][NC];
-  load_state<KT, NC>(S, state, dv, col0, sg.start == 0);
-  float nrm[NC];
-#pragma unroll
-  for (int nc = 0; nc < NC; ++nc) nrm[nc] = a.norm[h * dv + col0 + nc * 16 + l16] * a.out_scale;
+  const int col0 = wave * 16;
+  f32x4 S[KT][1];
+  load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
+  const float nrm = a.norm[h * dv + col0 + l16] * a.out_scale;
   const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
   const int64_t stride = (int64_t)a.heads * size;
   const int blocks = (sg.count + kBlock - 1) / kBlock;
@@ -262,78 +276,145 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
 #pragma unroll
     for (int u = 0; u < (size / 256 + NW - 1) / NW; ++u) {
       const int i = min(wave + u * NW, size / 256 - 1);            // the last may come twice
-      from.ld(lds + (b & 1) * size + i * 256, lane * 16, i * 1024);
+      float* const to = i < kSplit / 256 ? split + (b & 1) * kSplit + i * 256 : rest + b % 3 * kRest + (i * 256 - kSplit);
+      from.ld(to, lane * 16, i * 1024);
     }
   };
-  f32x4 O[NC];
-  uint16_t gate[NC][4];
+  // Planes of a block's tiles: for pairs of those of -W and of G q [3][64 lanes][two tiles' 4], for those of keys
+  // [64][hi 4, mid 4], [64][lo 4].  A wave's tile u; the last may be made twice.
+  auto tile_of = [&](int b, int u) {
+    return *(const f32x4*)(split + (b & 1) * kSplit + min(wave + u * NW, 3 * KT - 1) * 256 + lane * 4);
+  };
+  auto put_planes = [&](int b, int u, const f32x4& x) {
+    const int i = min(wave + u * NW, 3 * KT - 1);
+    const int key = i >= 2 * KT;               // multiplied, not branched on: the products beside stay in one stretch
+    float* const to = planes + (b & 1) * kPlanes + (i >> 1) * 768 + (i & 1) * (2 + 382 * key) + lane * 4;
+    const Planes p(x);
+    *(uint2*)to = p.hi;
+    *(uint2*)(to + 256 - 254 * key) = p.mid;
+    *(uint2*)(to + 512 - (256 + lane * 2) * key) = p.lo;
+  };
+  f32x4 done = {0.f, 0.f, 0.f, 0.f};
+  uint16_t gate[4] = {0, 0, 0, 0};
   const float inv_v = 1.f / (float)a.vdim;
   const int out_at = (4 * g * (int)a.out_stride + h * dv + col0 + l16) * 2;
   const int low_at = (4 * g * (int)a.low_stride + a.g_at + h * dv + col0 + l16) * 2;
-  f32x4 done[NC];
-  auto finish = [&](int b) {                   // rows of block b, whose squares are in red; none of block -1
-    const f32x4 ss = block_squares_total<NW>(red + (b & 1) * NW * kBlock);
+  auto finish = [&](int b, int r, const f32x4& ss) {               // row r of block b, whose squares are ss; none of block -1
     const int cnt = b < 0 ? 0 : min(kBlock, sg.count - b * kBlock);
     const BlockRows out(a.out, sg.row + b * kBlock, cnt, a.out_stride);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float rs = __builtin_amdgcn_rsqf(ss[r] * inv_v + a.eps);
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc)
-        out.st(out_at + r * (int)a.out_stride * 2, nc * 16, done[nc][r] * rs * nrm[nc] * fast_sigmoid(bf16_bits_to_float(gate[nc][r])));
-    }
+    const float rs = __builtin_amdgcn_rsqf(ss[r] * inv_v + a.eps);
+    out.st(out_at + r * (int)a.out_stride * 2, 0, done[r] * rs * nrm * fast_sigmoid(bf16_bits_to_float(gate[r])));
+  };
+  u32x4 sp[3][J];                              // the state's planes, pairs of tiles
+  auto split_state = [&](int kt) {
+    const Planes x(S[kt][0]);
+    const int at = (kt & 1) * 2;
+    sp[0][kt >> 1][at] = x.hi.x, sp[0][kt >> 1][at + 1] = x.hi.y;
+    sp[1][kt >> 1][at] = x.mid.x, sp[1][kt >> 1][at + 1] = x.mid.y;
+    sp[2][kt >> 1][at] = x.lo.x, sp[2][kt >> 1][at + 1] = x.lo.y;
   };
   request(0);
   __builtin_amdgcn_s_waitcnt(0);               // the state is there: the loop's first use of it must not wait in every pass
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) split_state(kt);
+  wait_and_meet();
+  request(1);
+#pragma unroll
+  for (int u = 0; u < kMine; ++u) put_planes(0, u, tile_of(0, u));
 #pragma unroll 1
   for (int b = 0; b < blocks; ++b) {
     wait_and_meet();
-    request(b + 1);
-    finish(b - 1);
+    const float* const mine = rest + b % 3 * kRest;
+    const float* const pl = planes + (b & 1) * kPlanes + lane * 4;
+    u32x4 W[2][3], Q[2][3];
+    auto operands = [&](int j) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        W[j & 1][i] = *(const u32x4*)(pl + (j * 3 + i) * 256);
+        Q[j & 1][i] = *(const u32x4*)(pl + ((J + j) * 3 + i) * 256);
+      }
+    };
+    operands(0);
+    f32x4 U = *(const f32x4*)(mine + wave * 256 + lane * 4), O = {0.f, 0.f, 0.f, 0.f};
+    f32x4 tile = tile_of(b + 1, 0);
+    const f32x4 ss = block_squares_total<NW>(red + ((b - 1) & 1) * NW * kBlock);
+    request(b + 2);
     const int cnt = min(kBlock, sg.count - b * kBlock);
     const BlockRows low(a.low, sg.row + b * kBlock, cnt, a.low_stride);
+    uint16_t next[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+    for (int r = 0; r < 4; ++r) next[r] = low.ld(low_at + r * (int)a.low_stride * 2, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    u32x4 K[2][2];
+    uint2 Kl[2][2];
+    f32x4 dec[2][2];
+    auto keys = [&](int j) {
 #pragma unroll
-      for (int nc = 0; nc < NC; ++nc) gate[nc][r] = low.ld(low_at + r * (int)a.low_stride * 2, nc * 16);
-    const float* const blk = lds + (b & 1) * size + lane * 4;
-    f32x4 U[NC];
-#pragma unroll
-    for (int nc = 0; nc < NC; ++nc) {
-      U[nc] = *(const f32x4*)(blk + 3 * kBlock * dk + (wave * NC + nc) * 256);
-      O[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 W = *(const f32x4*)(blk + kt * 256), Q = *(const f32x4*)(blk + (KT + kt) * 256);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int nc = 0; nc < NC; ++nc) {
-          U[nc] = mfma_f32_step(W[j], S[kt][nc][j], U[nc]);
-          O[nc] = mfma_f32_step(Q[j], S[kt][nc][j], O[nc]);
-        }
-    }
-    const f32x4 P = *(const f32x4*)(blk + kBlock * (3 * dk + dv));
-    const float* const dec = blk - lane * 4 + kBlock * (3 * dk + dv) + kBlock * kBlock + 4 * g;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 d = *(const f32x4*)(dec + 16 * kt), K = *(const f32x4*)(blk + (2 * KT + kt) * 256);
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc) {
-        S[kt][nc] *= d;
-        mfma_f32_16(K, U[nc], S[kt][nc]);
+      for (int i = 0; i < 2; ++i) {
+        const float* const at = planes + (b & 1) * kPlanes + (2 * KT + 2 * j + i) * 384;
+        K[j & 1][i] = *(const u32x4*)(at + lane * 4);
+        Kl[j & 1][i] = *(const uint2*)(at + 256 + lane * 2);
+        dec[j & 1][i] = *(const f32x4*)(mine + kG + 16 * (2 * j + i) + 4 * g);
       }
+    };
+#pragma unroll
+    for (int j = 0; j < J; ++j) {              // beside: the block before is finished, the next one's planes are made
+      if (j + 1 < J) operands(j + 1);
+      else keys(0);
+#pragma unroll
+      for (int i = 2; i >= 0; --i)             // the smallest products first
+#pragma unroll
+        for (int k = 2 - i; k >= 0; --k) {
+          U = mfma_bf16(W[j & 1][i], sp[k][j], U);
+          O = mfma_bf16(Q[j & 1][i], sp[k][j], O);
+        }
+#pragma unroll
+      for (int r = j * 4 / J; r < (j + 1) * 4 / J; ++r) finish(b - 1, r, ss);
+#pragma unroll
+      for (int u = j * kMine / J; u < (j + 1) * kMine / J; ++u) {
+        put_planes(b + 1, u, tile);
+        if (u + 1 < kMine) tile = tile_of(b + 1, u + 1);
+      }
+      spread_over_products<12, 4>();
     }
 #pragma unroll
-    for (int nc = 0; nc < NC; ++nc) mfma_f32_16(P, U[nc], O[nc]);
-    block_squares<NC>(O, red + (b & 1) * NW * kBlock, wave);
+    for (int r = 0; r < 4; ++r) gate[r] = next[r];
+    const PlanePairs u(U);
+    const u32x4 P = *(const u32x4*)(mine + kP + lane * 4);
+    const uint2 Pl = *(const uint2*)(mine + kP + 256 + lane * 2);
+    __builtin_amdgcn_sched_barrier(0);
+    S[0][0] *= dec[0][0];
+    S[1][0] *= dec[0][1];
 #pragma unroll
-    for (int nc = 0; nc < NC; ++nc) done[nc] = O[nc];
+    for (int j = 0; j < J; ++j) {              // beside: two tiles before are split, the next two decay
+      if (j + 1 < J) {
+        keys(j + 1);
+        S[2 * j + 2][0] *= dec[(j + 1) & 1][0];
+        S[2 * j + 3][0] *= dec[(j + 1) & 1][1];
+      }
+      u.add(K[j & 1], Kl[j & 1], S[2 * j][0], S[2 * j + 1][0]);
+      if (j > 0) {
+        split_state(2 * j - 2);
+        split_state(2 * j - 1);
+      }
+      spread_over_products<8, 5>();
+    }
+    u.add(P, Pl, O);
+    split_state(KT - 2);
+    split_state(KT - 1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)                // here, not behind the squares
+#pragma unroll
+      for (int j = 0; j < J; ++j) settle(sp[i][j]);
+    f32x4 o[1] = {O};
+    block_squares<1>(o, red + (b & 1) * NW * kBlock, wave);
+    done = O;
   }
   wait_and_meet();
-  finish(blocks - 1);
-  store_state<KT, NC>(S, state, dv, col0);
+  const f32x4 ss = block_squares_total<NW>(red + ((blocks - 1) & 1) * NW * kBlock);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) finish(blocks - 1, r, ss);
+  store_state<KT, 1>(S, state, dv, col0);
   // the last inputs of the head's convolutions (runs are longer than a filter)
   const int taps = a.taps, cw = 2 * dk + dv, hk = h / (a.heads / a.kv_heads);
   char* const tail = (char*)a.conv_state + item * (taps - 1) * cw * 2;
@@ -345,7 +426,8 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
 }
 
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
-  constexpr int smem = (2 * block_floats(16 * KT, 32 * NW) + 2 * NW * kBlock) * 4;
+  constexpr int kSplit = 3 * kBlock * 16 * KT;
+  constexpr int smem = (3 * block_floats(16 * KT, 16 * NW) - kSplit + 2 * 3 * KT * 384 + 2 * NW * kBlock) * 4;
   if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)delta_blocks_kernel<KT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               smem) != hipSuccess) {
     zp_set_error("delta_runs: cannot reserve %d bytes of LDS", smem);
@@ -357,10 +439,10 @@ template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
 }
 template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   switch (ra.d.dv / 32) {
-    case 1: return launch_blocks<KT, 1>(ra, st);
-    case 2: return launch_blocks<KT, 2>(ra, st);
-    case 3: return launch_blocks<KT, 3>(ra, st);
-    default: return launch_blocks<KT, 4>(ra, st);
+    case 1: return launch_blocks<KT, 2>(ra, st);
+    case 2: return launch_blocks<KT, 4>(ra, st);
+    case 3: return launch_blocks<KT, 6>(ra, st);
+    default: return launch_blocks<KT, 8>(ra, st);
   }
 }
 
