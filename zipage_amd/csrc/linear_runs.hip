@@ -19,9 +19,9 @@ struct RunArgs {
   int row0;      // first token row of the first segment
 };
 
-// G q and the keys as left operands, P, the block's decays; whole KBs
+// G q and the keys as left operands, P's planes, the block's decays; whole KBs
 __host__ __device__ inline constexpr int block_floats(int dk) {
-  return (2 * kBlock * dk + kBlock * kBlock + dk + 255) / 256 * 256;
+  return (2 * kBlock * dk + kPairFloats + dk + 255) / 256 * 256;
 }
 
 __global__ __launch_bounds__(256, 4) void linear_prepare_kernel(RunArgs ra) {
@@ -99,8 +99,8 @@ __global__ __launch_bounds__(256, 4) void linear_prepare_kernel(RunArgs ra) {
   // ---- columns: a thread reads and writes its own only
   float* const oQ = ra.ws + (block_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * block_floats(dk);
   float* const oK = oQ + kBlock * dk;          // [dk / 16][64 lanes][4], as oQ
-  float* const oP = oK + kBlock * dk;          // [64][4]
-  float* const oG = oP + kBlock * kBlock;      // [dk]
+  float* const oP = oK + kBlock * dk;          // [64][hi 4, mid 4], [64][lo 4]
+  float* const oG = oP + kPairFloats;          // [dk]
   if (tid < dk) {                              // G q
     const int c = tid;
     float G = 1.f;
@@ -127,133 +127,204 @@ __global__ __launch_bounds__(256, 4) void linear_prepare_kernel(RunArgs ra) {
     }
   }
   __syncthreads();
-  if (tid < 64) *(f32x4*)(oP + tid * 4) = *(const f32x4*)(Ps + (tid & 15) * kBlock + (tid >> 4) * 4);
+  if (tid < 64) {
+    const Planes x(*(const f32x4*)(Ps + (tid & 15) * kBlock + (tid >> 4) * 4));
+    *(u32x4*)(oP + tid * 4) = u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y};
+    *(uint2*)(oP + 256 + tid * 2) = x.lo;
+  }
   for (int i = tid; i < kBlock * dk / 4; i += 256) {           // lane (g, row) of tile kt: columns 16 kt + 4 g ..
     const int l = i & 63, kt = i >> 6;
     *(f32x4*)(oQ + i * 4) = *(const f32x4*)(qs + (l & 15) * ld + kt * 16 + (l >> 4) * 4);
   }
 }
 
-// A head's blocks, one after the other: a block's operands and value rows come straight into LDS while the block
-// before it is worked on; its rows are normed and stored behind the next meeting of the waves, which the norm
-// needs too.
+// A head's blocks, one after the other, a wave 16 columns of the state.  Operands in fp32 enter the bf16 matrix cores in three
+// planes each, as in delta_blocks: the state is split where it is updated, what comes from memory by all waves together,
+// a block ahead; value rows are bf16 as they come.  Rows are normed and stored behind the next meeting of the
+// waves, which the norm needs too.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 677 -> 647 us,
+// 16 heads 422 -> 358; error of the state against 64 bits 2.0e-7 -> 1.8e-7 of its size.
 template <int KT, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void linear_blocks_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
   const zp_linear& a = ra.d;
-  constexpr int NC = 2, dk = 16 * KT, dv = 32 * NW, size = block_floats(dk), stage = size + kBlock * dv / 2;
+  constexpr int dk = 16 * KT, dv = 16 * NW, size = block_floats(dk), J = KT / 2;
+  constexpr int kSplit = 2 * kBlock * dk, kV = size - kSplit, kRest = kV + kBlock * dv / 2;   // floats to be split; the others
+  constexpr int kG = kPairFloats;                                     // in the others, behind P; then from kV on the value rows
+  constexpr int kPlanes = 2 * KT * 384, kMine = (2 * KT + NW - 1) / NW;      // floats of a block's planes; tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  float* const red = lds + 2 * stage;          // [2][NW * 16]
+  float* const split = lds;                    // [2][kSplit]
+  float* const rest = split + 2 * kSplit;      // [3][kRest]
+  float* const planes = rest + 3 * kRest;      // [2][kPlanes]
+  float* const red = planes + 2 * kPlanes;     // [2][NW * 16]
   const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
   const Segment sg = segment_of(a.seg, seg);
   if (sg.count <= 0 || sg.row < ra.row0) return;
   float* const state = a.state + ((int64_t)sg.slot * a.heads + h) * ((int64_t)dk * dv);
-  const int col0 = wave * 16 * NC;
-  f32x4 S[KT][NC];
-  load_state<KT, NC>(S, state, dv, col0, sg.start == 0);
-  float nrm[NC];
-#pragma unroll
-  for (int nc = 0; nc < NC; ++nc) nrm[nc] = a.norm[h * dv + col0 + nc * 16 + l16];
+  const int col0 = wave * 16;
+  f32x4 S[KT][1];
+  load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
+  const float nrm = a.norm[h * dv + col0 + l16];
   const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
   const int64_t stride = (int64_t)a.heads * size;
   const int blocks = (sg.count + kBlock - 1) / kBlock;
   auto request = [&](int b) {                  // a block behind the last: nothing is read
-    float* const st = lds + (b & 1) * stage;
     const int cnt = b < blocks ? min(kBlock, sg.count - b * kBlock) : 0;
     const StageLoads from(base + b * stride, cnt > 0 ? size * 4 : 0);
 #pragma unroll
     for (int u = 0; u < (size / 256 + NW - 1) / NW; ++u) {
       const int i = min(wave + u * NW, size / 256 - 1);            // the last may come twice
-      from.ld(st + i * 256, lane * 16, i * 1024);
+      float* const to = i < kSplit / 256 ? split + (b & 1) * kSplit + i * 256 : rest + b % 3 * kRest + (i * 256 - kSplit);
+      from.ld(to, lane * 16, i * 1024);
     }
     const StageLoads rows((const char*)a.in + (int64_t)(sg.row + b * kBlock) * a.in_stride * 2, cnt * a.in_stride * 2);
-    const int s = wave * 64 + lane, row = s / (dv / 8), pc = s - row * (dv / 8);
-    rows.ld(st + size + wave * 256, max(min(row, cnt - 1), 0) * (int)a.in_stride * 2 + pc * 16, (a.v_at + h * dv) * 2);
+    const int w = wave % (NW / 2), s = w * 64 + lane, row = s / (dv / 8), pc = s - row * (dv / 8);       // each comes twice
+    rows.ld(rest + b % 3 * kRest + kV + w * 256, max(min(row, cnt - 1), 0) * (int)a.in_stride * 2 + pc * 16, (a.v_at + h * dv) * 2);
   };
-  f32x4 O[NC], done[NC];
-  uint16_t gate[NC][4];
+  // Planes of a block's tiles: for pairs of those of G q [3][64 lanes][two tiles' 4], for those of keys [64][hi 4, mid 4],
+  // [64][lo 4].  A wave's tile u; the last may be made twice.
+  auto tile_of = [&](int b, int u) {
+    return *(const f32x4*)(split + (b & 1) * kSplit + min(wave + u * NW, 2 * KT - 1) * 256 + lane * 4);
+  };
+  auto put_planes = [&](int b, int u, const f32x4& x) {
+    const int i = min(wave + u * NW, 2 * KT - 1);
+    const int key = i >= KT;                   // multiplied, not branched on: the products beside stay in one stretch
+    float* const to = planes + (b & 1) * kPlanes + (i >> 1) * 768 + (i & 1) * (2 + 382 * key) + lane * 4;
+    const Planes p(x);
+    *(uint2*)to = p.hi;
+    *(uint2*)(to + 256 - 254 * key) = p.mid;
+    *(uint2*)(to + 512 - (256 + lane * 2) * key) = p.lo;
+  };
+  f32x4 done = {0.f, 0.f, 0.f, 0.f};
+  uint16_t gate[4] = {0, 0, 0, 0};
   const float inv_v = 1.f / (float)a.vdim;
   const int out_at = (4 * g * (int)a.out_stride + h * dv + col0 + l16) * 2;
   const int gate_at = (4 * g * (int)a.in_stride + a.g_at + h * dv + col0 + l16) * 2;
-  auto finish = [&](int b) {                   // rows of block b, whose squares are in red; none of block -1
-    const f32x4 ss = block_squares_total<NW>(red + (b & 1) * NW * kBlock);
+  auto finish = [&](int b, int r, const f32x4& ss) {               // row r of block b, whose squares are ss; none of block -1
     const int cnt = b < 0 ? 0 : min(kBlock, sg.count - b * kBlock);
     const BlockRows out(a.out, sg.row + b * kBlock, cnt, a.out_stride);
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const float rs = __builtin_amdgcn_rsqf(ss[r] * inv_v + a.eps);
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc) {
-        const float z = bf16_bits_to_float(gate[nc][r]);
-        out.st(out_at + r * (int)a.out_stride * 2, nc * 16, done[nc][r] * rs * nrm[nc] * z * fast_sigmoid(z));
-      }
-    }
+    const float rs = __builtin_amdgcn_rsqf(ss[r] * inv_v + a.eps), z = bf16_bits_to_float(gate[r]);
+    out.st(out_at + r * (int)a.out_stride * 2, 0, done[r] * rs * nrm * z * fast_sigmoid(z));
+  };
+  u32x4 sp[3][J];                              // the state's planes, pairs of tiles
+  auto split_state = [&](int kt) {
+    const Planes x(S[kt][0]);
+    const int at = (kt & 1) * 2;
+    sp[0][kt >> 1][at] = x.hi.x, sp[0][kt >> 1][at + 1] = x.hi.y;
+    sp[1][kt >> 1][at] = x.mid.x, sp[1][kt >> 1][at + 1] = x.mid.y;
+    sp[2][kt >> 1][at] = x.lo.x, sp[2][kt >> 1][at + 1] = x.lo.y;
   };
   request(0);
   __builtin_amdgcn_s_waitcnt(0);               // the state is there: the loop's first use of it must not wait in every pass
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) split_state(kt);
+  wait_and_meet();
+  request(1);
+#pragma unroll
+  for (int u = 0; u < kMine; ++u) put_planes(0, u, tile_of(0, u));
 #pragma unroll 1
   for (int b = 0; b < blocks; ++b) {
     wait_and_meet();
-    request(b + 1);
-    finish(b - 1);
-    const int cnt = min(kBlock, sg.count - b * kBlock);
-    const BlockRows gp(a.in, sg.row + b * kBlock, cnt, a.in_stride);
+    const float* const mine = rest + b % 3 * kRest;
+    const float* const pl = planes + (b & 1) * kPlanes;
+    u32x4 Q[2][3], K[2][2];
+    uint2 Kl[2][2];
+    f32x4 dec[2][2];
+    auto operands = [&](int j) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
+      for (int i = 0; i < 3; ++i) Q[j & 1][i] = *(const u32x4*)(pl + (j * 3 + i) * 256 + lane * 4);
+    };
+    auto keys = [&](int j) {
 #pragma unroll
-      for (int nc = 0; nc < NC; ++nc) gate[nc][r] = gp.ld(gate_at + r * (int)a.in_stride * 2, nc * 16);
-    const float* const blk = lds + (b & 1) * stage + lane * 4;
-    const uint16_t* const vs = (const uint16_t*)(lds + (b & 1) * stage + size);
-    f32x4 v[NC];
-#pragma unroll
-    for (int nc = 0; nc < NC; ++nc) {
-      v[nc] = read_columns((const char*)(vs + (4 * g + (l16 >> 2)) * dv + col0 + nc * 16 + (l16 & 3) * 4));
-      O[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
-    }
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 Q = *(const f32x4*)(blk + kt * 256);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int nc = 0; nc < NC; ++nc) O[nc] = mfma_f32_step(Q[j], S[kt][nc][j], O[nc]);
-    }
-    const f32x4 P = *(const f32x4*)(blk + 2 * kBlock * dk);
-#pragma unroll
-    for (int nc = 0; nc < NC; ++nc) mfma_f32_16(P, v[nc], O[nc]);
-    const float* const dec = blk - lane * 4 + 2 * kBlock * dk + kBlock * kBlock + 4 * g;
-#pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 d = *(const f32x4*)(dec + 16 * kt), K = *(const f32x4*)(blk + (KT + kt) * 256);
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc) {
-        S[kt][nc] *= d;
-        mfma_f32_16(K, v[nc], S[kt][nc]);
+      for (int i = 0; i < 2; ++i) {
+        const float* const at = pl + (KT + 2 * j + i) * kPairFloats;
+        K[j & 1][i] = *(const u32x4*)(at + lane * 4);
+        Kl[j & 1][i] = *(const uint2*)(at + 256 + lane * 2);
+        dec[j & 1][i] = *(const f32x4*)(mine + kG + 16 * (2 * j + i) + 4 * g);
       }
-    }
-    block_squares<NC>(O, red + (b & 1) * NW * kBlock, wave);
+    };
+    operands(0);
+    keys(0);
+    f32x4 tile = tile_of(b + 1, 0);
+    const f32x4 ss = block_squares_total<NW>(red + ((b - 1) & 1) * NW * kBlock);
+    const uint2 v4 = read_transposed((const uint16_t*)(mine + kV) + (4 * g + (l16 >> 2)) * dv + col0 + (l16 & 3) * 4);
+    const u32x4 v = {v4.x, v4.y, v4.x, v4.y};
+    const u32x4 P = *(const u32x4*)(mine + lane * 4);
+    const uint2 Pl = *(const uint2*)(mine + 256 + lane * 2);
+    request(b + 2);
+    const BlockRows gp(a.in, sg.row + b * kBlock, min(kBlock, sg.count - b * kBlock), a.in_stride);
+    uint16_t next[4];
 #pragma unroll
-    for (int nc = 0; nc < NC; ++nc) done[nc] = O[nc];
+    for (int r = 0; r < 4; ++r) next[r] = gp.ld(gate_at + r * (int)a.in_stride * 2, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x4 O[1] = {mfma_bf16(u32x4{Pl.x, Pl.y, 0u, 0u}, v, f32x4{0.f, 0.f, 0.f, 0.f})};
+    O[0] = mfma_bf16(P, v, O[0]);
+#pragma unroll
+    for (int j = 0; j < J; ++j) {              // beside: the block before is finished, the next one's planes are made
+      if (j + 1 < J) {
+        operands(j + 1);
+        keys(j + 1);
+      }
+#pragma unroll
+      for (int i = 2; i >= 0; --i)             // the smallest products first
+#pragma unroll
+        for (int k = 2 - i; k >= 0; --k) O[0] = mfma_bf16(Q[j & 1][i], sp[k][j], O[0]);
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {            // the state's tiles are behind their products
+        f32x4& s = S[2 * j + i][0];
+        s *= dec[j & 1][i];
+        s = mfma_bf16(u32x4{Kl[j & 1][i].x, Kl[j & 1][i].y, 0u, 0u}, v, s);
+        s = mfma_bf16(K[j & 1][i], v, s);
+      }
+#pragma unroll
+      for (int r = j * 4 / J; r < (j + 1) * 4 / J; ++r) finish(b - 1, r, ss);
+#pragma unroll
+      for (int u = j * kMine / J; u < (j + 1) * kMine / J; ++u) {
+        put_planes(b + 1, u, tile);
+        if (u + 1 < kMine) tile = tile_of(b + 1, u + 1);
+      }
+      if (j > 0) {
+        split_state(2 * j - 2);
+        split_state(2 * j - 1);
+      }
+      spread_over_products<10, 6>();
+    }
+    split_state(KT - 2);
+    split_state(KT - 1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i)                // here, not behind the squares
+#pragma unroll
+      for (int j = 0; j < J; ++j) settle(sp[i][j]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gate[r] = next[r];
+    block_squares<1>(O, red + (b & 1) * NW * kBlock, wave);
+    done = O[0];
   }
   wait_and_meet();
-  finish(blocks - 1);
-  store_state<KT, NC>(S, state, dv, col0);
+  const f32x4 ss = block_squares_total<NW>(red + ((blocks - 1) & 1) * NW * kBlock);
+#pragma unroll
+  for (int r = 0; r < 4; ++r) finish(blocks - 1, r, ss);
+  store_state<KT, 1>(S, state, dv, col0);
 }
 
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
-  constexpr int smem = (2 * (block_floats(16 * KT) + kBlock * 16 * NW) + 2 * NW * kBlock) * 4;
-  static_assert(smem <= 60 * 1024, "a stage outgrew the default LDS limit");
+  constexpr int kSplit = 2 * kBlock * 16 * KT;
+  constexpr int smem = (3 * (block_floats(16 * KT) + kBlock * 8 * NW) - kSplit + 2 * 2 * KT * 384 + 2 * NW * kBlock) * 4;
+  if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)linear_blocks_kernel<KT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              smem) != hipSuccess) {
+    zp_set_error("linear_runs: cannot reserve %d bytes of LDS", smem);
+    return ZP_EHIP;
+  }
   hipLaunchKernelGGL((linear_blocks_kernel<KT, NW>), dim3((unsigned)((int64_t)ra.d.seg.n * ra.d.heads)), dim3(64 * NW), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
 template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   switch (ra.d.dv / 32) {
-    case 1: return launch_blocks<KT, 1>(ra, st);
-    case 2: return launch_blocks<KT, 2>(ra, st);
-    case 3: return launch_blocks<KT, 3>(ra, st);
-    default: return launch_blocks<KT, 4>(ra, st);
+    case 1: return launch_blocks<KT, 2>(ra, st);
+    case 2: return launch_blocks<KT, 4>(ra, st);
+    case 3: return launch_blocks<KT, 6>(ra, st);
+    default: return launch_blocks<KT, 8>(ra, st);
   }
 }
 

@@ -9,8 +9,8 @@
 //   mlstm_prepare   D and the block's factors, for all blocks at once
 //   mlstm_blocks    a head's blocks one after the other, S in registers
 //
-// All fp32: the products q . k on the bf16 matrix cores are exact products of the projections, added up in
-// fp32; those with S run on the fp32 ones.  Projections in bfloat16.
+// All fp32, on the bf16 matrix cores: the products q . k are exact products of the projections, added up in fp32, and S, D
+// and the rows that are written are split into three bf16 planes each.  Projections in bfloat16.
 #include "blocks.h"
 #include <type_traits>
 
@@ -22,8 +22,8 @@ struct RunArgs {
   float4* scal;  // per token row from row0 on and head: F, x, m, m before the block
   int row0;
 };
-// D as a left operand (256), then a, write factors, e^{-m}, row sums of D (16 each), the keep factor
-constexpr int kAux = 512, kInter = 256, kWrite = 272, kFloor = 288, kSum = 304, kKeep = 320;
+// D's planes as a left operand, then a, write factors, e^{-m}, row sums of D (16 each), the keep factor
+constexpr int kAux = 512, kInter = kPairFloats, kWrite = kInter + 16, kFloor = kWrite + 16, kSum = kFloor + 16, kKeep = kSum + 16;
 
 __device__ __forceinline__ float lane_value(float v, int lane) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), lane));
@@ -108,7 +108,9 @@ __global__ __launch_bounds__(256) void mlstm_prepare_kernel(RunArgs ra) {
   sum += lane_xor32(sum);
   const float F_end = lane_value(sc.x, cnt - 1), m_end = lane_value(sc.z, cnt - 1);
   float* const aux = ra.aux + (block_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * kAux;
-  *(f32x4*)(aux + lane * 4) = P;
+  const Planes planes(P);
+  *(u32x4*)(aux + lane * 4) = u32x4{planes.hi.x, planes.hi.y, planes.mid.x, planes.mid.y};
+  *(uint2*)(aux + 256 + lane * 2) = planes.lo;
   if (g == 0) {
     aux[kInter + l16] = expf(sc.x + sc.w - sc.z);
     aux[kWrite + l16] = l16 < cnt ? expf(F_end + sc.y - m_end) : 0.f;
@@ -118,13 +120,13 @@ __global__ __launch_bounds__(256) void mlstm_prepare_kernel(RunArgs ra) {
   }
 }
 
-// LDS of a stage: Q and K rows, their 16-byte pieces xor-ed with the row so that neither operand order meets
+// A wave owns 16 columns of the state, which is split into planes where it is updated.  LDS of a stage: Q and K rows, their 16-byte pieces xor-ed with the row so that neither operand order meets
 // bank conflicts; V rows; the block's factors.  The next stage comes in while this one is worked on.
 template <int KT, int NW>
 __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   extern __shared__ __align__(16) char lds_raw[];
   const zp_mlstm& a = ra.d;
-  constexpr int NC = 2, dk = 16 * KT, dv = 32 * NW, PR = dk / 8;     // PR: pieces per row of Q and K
+  constexpr int dk = 16 * KT, dv = 16 * NW, PR = dk / 8, J = KT / 2;      // PR: pieces per row of Q and K
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
@@ -137,13 +139,11 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   float* const state = a.state + ((int64_t)sg.slot * a.heads + h) * ((int64_t)dk * dv + dk + 4);
   float* const nstate = state + (int64_t)dk * dv;
   const bool fresh = sg.start == 0;
-  const int col0 = wave * 16 * NC;
-  f32x4 S[KT][NC];
-  load_state<KT, NC>(S, state, dv, col0, fresh);
+  const int col0 = wave * 16;
+  f32x4 S[KT][1];
+  load_state<KT, 1>(S, state, dv, col0, fresh);
   for (int c = tid; c < dk; c += blockDim.x) nl[0][c] = fresh ? 0.f : nstate[c];
-  float nrm[NC];
-#pragma unroll
-  for (int nc = 0; nc < NC; ++nc) nrm[nc] = a.norm[h * dv + col0 + nc * 16 + l16] * a.out_scale;
+  const float nrm = a.norm[h * dv + col0 + l16] * a.out_scale;
   const int blocks = (sg.count + kBlock - 1) / kBlock;
   const float* const aux0 = ra.aux + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * kAux;
   constexpr int kQK = KT / 2;                  // KBs of Q, and of K
@@ -163,15 +163,14 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
       rows.ld(st + i * 1024, at, (a.q_at + h * dk) * 2);
       rows.ld(st + (kQK + i) * 1024, at, (a.k_at + h * dk) * 2);
     });
-    share(std::integral_constant<int, NW>(), [&](int i) {
+    share(std::integral_constant<int, NW / 2>(), [&](int i) {
       const int s = i * 64 + lane, row = s / (dv / 8), pc = s - row * (dv / 8);
       rows.ld(st + (2 * kQK + i) * 1024, max(min(row, cnt - 1), 0) * (int)a.in_stride * 2 + pc * 16, (a.v_at + h * dv) * 2);
     });
-    share(std::integral_constant<int, 2>(), [&](int i) { aux.ld(st + (2 * kQK + NW + i) * 1024, lane * 16, i * 1024); });
+    share(std::integral_constant<int, 2>(), [&](int i) { aux.ld(st + (2 * kQK + NW / 2 + i) * 1024, lane * 16, i * 1024); });
   };
-  f32x4 done[NC];
-  f32x4 O[NC];
-  uint16_t gate[NC][4];
+  f32x4 done = {0.f, 0.f, 0.f, 0.f};
+  uint16_t gate[4] = {0, 0, 0, 0};
   const float inv_v = 1.f / (float)a.vdim;
   const int out_at = (4 * g * (int)a.out_stride + h * dv + col0 + l16) * 2;
   const int gate_at = (4 * g * (int)a.in_stride + a.g_at + h * dv + col0 + l16) * 2;
@@ -183,13 +182,21 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const float f = a.q_scale * __builtin_amdgcn_rcpf(dn[r]), rs = f * __builtin_amdgcn_rsqf(ss[r] * f * f * inv_v + a.eps);
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc)
-        out.st(out_at + r * (int)a.out_stride * 2, nc * 16, done[nc][r] * rs * nrm[nc] * fast_sigmoid(bf16_bits_to_float(gate[nc][r])));
+      out.st(out_at + r * (int)a.out_stride * 2, 0, done[r] * rs * nrm * fast_sigmoid(bf16_bits_to_float(gate[r])));
     }
+  };
+  u32x4 sp[3][J];                              // the state's planes, pairs of tiles
+  auto split_state = [&](int kt) {
+    const Planes x(S[kt][0]);
+    const int at = (kt & 1) * 2;
+    sp[0][kt >> 1][at] = x.hi.x, sp[0][kt >> 1][at + 1] = x.hi.y;
+    sp[1][kt >> 1][at] = x.mid.x, sp[1][kt >> 1][at + 1] = x.mid.y;
+    sp[2][kt >> 1][at] = x.lo.x, sp[2][kt >> 1][at + 1] = x.lo.y;
   };
   request(0);
   __builtin_amdgcn_s_waitcnt(0);               // the state is there: the loop's first use of it must not wait in every pass
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) split_state(kt);
 #pragma unroll 1
   for (int b = 0; b < blocks; ++b) {
     wait_and_meet();
@@ -198,49 +205,45 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
     const int cnt = min(kBlock, sg.count - b * kBlock);
     const BlockRows gp(a.in, sg.row + b * kBlock, cnt, a.in_stride);
 #pragma unroll
-    for (int r = 0; r < 4; ++r)
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc) gate[nc][r] = gp.ld(gate_at + r * (int)a.in_stride * 2, nc * 16);
+    for (int r = 0; r < 4; ++r) gate[r] = gp.ld(gate_at + r * (int)a.in_stride * 2, 0);
     const char* const st = lds_raw + (b & 1) * stage;
     const char* const ks = st + kBlock * dk * 2;
     const uint16_t* const vs = (const uint16_t*)(ks + kBlock * dk * 2);
     const float* const aux = (const float*)((const char*)vs + v_bytes);
     // ---- read-outs
+    f32x4 O[1] = {f32x4{0.f, 0.f, 0.f, 0.f}};
+    const char* const qrow = st + l16 * dk * 2 + (g & 1) * 8;
 #pragma unroll
-    for (int nc = 0; nc < NC; ++nc) O[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < J; ++j) {
+      const uint2 q0 = *(const uint2*)(qrow + ((4 * j + (g >> 1)) ^ (l16 & (PR - 1))) * 16);
+      const uint2 q1 = *(const uint2*)(qrow + ((4 * j + 2 + (g >> 1)) ^ (l16 & (PR - 1))) * 16);
 #pragma unroll
-    for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 q = load4<BF16>(st + l16 * dk * 2 + (((2 * kt + (g >> 1)) ^ (l16 & (PR - 1))) * 16) + (g & 1) * 8, 0);
-#pragma unroll
-      for (int j = 0; j < 4; ++j)
-#pragma unroll
-        for (int nc = 0; nc < NC; ++nc) O[nc] = mfma_f32_step(q[j], S[kt][nc][j], O[nc]);
+      for (int k = 2; k >= 0; --k) O[0] = mfma_bf16(u32x4{q0.x, q0.y, q1.x, q1.y}, sp[k][j], O[0]);      // the smallest first
     }
-    const f32x4 P = *(const f32x4*)(aux + lane * 4), inter = *(const f32x4*)(aux + kInter + 4 * g), wr = *(const f32x4*)(aux + kWrite + 4 * g);
+    const u32x4 P = *(const u32x4*)(aux + lane * 4);
+    const uint2 Pl = *(const uint2*)(aux + 256 + lane * 2);
+    const f32x4 inter = *(const f32x4*)(aux + kInter + 4 * g), wr = *(const f32x4*)(aux + kWrite + 4 * g);
     const float keep = aux[kKeep];
-    f32x4 v[NC];
-#pragma unroll
-    for (int nc = 0; nc < NC; ++nc) {
-      v[nc] = read_columns((const char*)(vs + (4 * g + (l16 >> 2)) * dv + col0 + nc * 16 + (l16 & 3) * 4));
-      O[nc] *= inter;
-      mfma_f32_16(P, v[nc], O[nc]);
-      v[nc] *= wr;
-    }
+    const uint2 v4 = read_transposed(vs + (4 * g + (l16 >> 2)) * dv + col0 + (l16 & 3) * 4);
+    O[0] *= inter;
+    O[0] = mfma_bf16(u32x4{Pl.x, Pl.y, 0u, 0u}, u32x4{v4.x, v4.y, v4.x, v4.y}, O[0]);
+    O[0] = mfma_bf16(P, u32x4{v4.x, v4.y, v4.x, v4.y}, O[0]);
     // ---- the state behind the block
+    const f32x4 v = {__uint_as_float(v4.x << 16), __uint_as_float(v4.x & 0xffff0000u), __uint_as_float(v4.y << 16), __uint_as_float(v4.y & 0xffff0000u)};
+    const Planes vw(v * wr);
     const int kr = 4 * g + (l16 >> 2), kz = ((l16 & 3) >> 1) ^ (kr & (PR - 1));
     const char* const krow = ks + kr * dk * 2 + (l16 & 1) * 8;
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
-      const f32x4 kT = read_columns(krow + (((2 * kt) ^ kz) * 16));
-#pragma unroll
-      for (int nc = 0; nc < NC; ++nc) {
-        S[kt][nc] *= keep;
-        mfma_f32_16(kT, v[nc], S[kt][nc]);
-      }
+      const uint2 k4 = read_transposed((const uint16_t*)(krow + ((2 * kt) ^ kz) * 16));
+      S[kt][0] *= keep;
+      S[kt][0] = mfma_bf16(u32x4{k4.x, k4.y, 0u, 0u}, u32x4{vw.lo.x, vw.lo.y, 0u, 0u}, S[kt][0]);
+      S[kt][0] = mfma_bf16(u32x4{k4.x, k4.y, k4.x, k4.y}, u32x4{vw.hi.x, vw.hi.y, vw.mid.x, vw.mid.y}, S[kt][0]);
     }
-    block_squares<NC>(O, red[b & 1], wave);
 #pragma unroll
-    for (int nc = 0; nc < NC; ++nc) done[nc] = O[nc];
+    for (int kt = 0; kt < KT; ++kt) split_state(kt);
+    block_squares<1>(O, red[b & 1], wave);
+    done = O[0];
     // ---- the normaliser: 16 lanes a token
     const float* const n = nl[b & 1];
 #pragma unroll
@@ -271,12 +274,12 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   }
   wait_and_meet();
   finish(blocks - 1);
-  store_state<KT, NC>(S, state, dv, col0);
+  store_state<KT, 1>(S, state, dv, col0);
   for (int c = tid; c < dk; c += blockDim.x) nstate[c] = nl[blocks & 1][c];
 }
 
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
-  constexpr int dk = 16 * KT, dv = 32 * NW;
+  constexpr int dk = 16 * KT, dv = 16 * NW;
   constexpr size_t smem = 2 * (2 * kBlock * dk * 2 + kBlock * dv * 2 + kAux * 4) + 2 * 4 * (NW * kBlock + kBlock + dk);
   hipLaunchKernelGGL((mlstm_blocks_kernel<KT, NW>), dim3((unsigned)((int64_t)ra.d.seg.n * ra.d.heads)), dim3(64 * NW), smem, st, ra);
   ZP_LAUNCH_CHECK();
@@ -291,10 +294,10 @@ template <int KT> int launch_runs(const RunArgs& ra, int longest, hipStream_t st
                      dim3(256), 0, st, ra);
   ZP_LAUNCH_CHECK();
   switch (a.dv / 32) {
-    case 1: return launch_blocks<KT, 1>(ra, st);
-    case 2: return launch_blocks<KT, 2>(ra, st);
-    case 3: return launch_blocks<KT, 3>(ra, st);
-    default: return launch_blocks<KT, 4>(ra, st);
+    case 1: return launch_blocks<KT, 2>(ra, st);
+    case 2: return launch_blocks<KT, 4>(ra, st);
+    case 3: return launch_blocks<KT, 6>(ra, st);
+    default: return launch_blocks<KT, 8>(ra, st);
   }
 }
 
