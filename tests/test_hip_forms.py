@@ -173,12 +173,19 @@ def test_rotary_store_of_wide_rows(dev, dtype, N, Hq, Hkv):
         assert float((a != b).float().mean()) < 0.01 and bool(((a - b).abs() <= 2 * ulp * pair + 1e-6).all())
 
 
-# ------------------------------------------------------------------ delta rule over runs
+# ------------------------------------------------------------------ recurrences over runs
+def _run_segments(dev, counts):
+    import types
+    from zipage_amd.engine.qwen3 import Segments
+    at = lambda x: torch.as_tensor(x, dtype=torch.int32).to(dev)
+    rows = [sum(counts[:i]) for i in range(len(counts))]
+    seg = Segments(at(rows), at(counts), at(range(len(counts))), at([0] * len(counts)), first_row=0, longest=max(counts))
+    return rows, types.SimpleNamespace(segments=None, run_segments=seg)
+
+
 # operands enter the bf16 matrix cores in three planes: the state has to stay as good as fp32's
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 128, 128), (2, 2, 32, 96), (3, 1, 64, 32), (1, 1, 128, 64)])
 def test_delta_state_of_runs(dev, H, G, D, V):
-    import types
-    from zipage_amd.engine.qwen3 import Segments
     from zipage_amd.layers import ChannelDelta
     W, taps, counts = 64, 2, [16, 47, 100]
     m, n = ChannelDelta(W, H, G, D, V, taps, 1e-3), sum(counts)
@@ -191,10 +198,8 @@ def test_delta_state_of_runs(dev, H, G, D, V):
     into, _ = m.load(w, BF16, dev, W)
     proj = (r(n, W, seed=16).float() @ into.float().cpu().T).to(BF16).to(dev)
     state = m.allocate(len(counts), BF16, dev)
-    rows = torch.tensor([sum(counts[:i]) for i in range(len(counts))], dtype=torch.int32)
-    at = lambda x: torch.as_tensor(x, dtype=torch.int32).to(dev)
-    seg = Segments(at(rows), at(counts), at(range(len(counts))), at([0] * len(counts)), first_row=0, longest=max(counts), max_count=0)
-    m.scan(proj, state, types.SimpleNamespace(segments=None, run_segments=seg), torch.empty(n, H * V, dtype=BF16, device=dev))
+    rows, ctx = _run_segments(dev, counts)
+    m.scan(proj, state, ctx, torch.empty(n, H * V, dtype=BF16, device=dev))
     P, head = proj.double().cpu(), torch.arange(H) // (H // G)
     low = torch.nn.functional.linear(proj[:, m.low_at:m.low_at + m.low_rank], m.low).double().cpu()
     a = low[:, :H * D].view(n, H, D) + w["dt_bias"].double().view(H, D)
@@ -212,4 +217,50 @@ def test_delta_state_of_runs(dev, H, G, D, V):
         # roundings of 2^-24 by the products, decays and unit vectors of the tokens that a state remembers; a product of
         # planes that is left out costs 2^-17 and more
         err = (state[0][i].double().cpu().view(H, D, V) - S).norm() / S.norm()
+        assert float(err) < 2.0 ** -19, float(err)
+
+
+# linear attention and matrix memory likewise; rows of values, and of the memory's keys, are bf16 as they come
+@pytest.mark.parametrize("H,D,V", [(2, 128, 128), (2, 32, 96), (3, 64, 32), (1, 128, 64)])
+@pytest.mark.parametrize("mixer", ["linear", "memory"])
+def test_states_of_runs(dev, mixer, H, D, V):
+    from zipage_amd.layers import LinearAttention, MatrixMemory
+    W, counts, tau, cap = 64, [16, 47, 100], 8.0, 3.0
+    r = lambda *s, seed, std=1.0: _rand(*s, seed=seed, std=std)
+    w = {k: r(H * (V if k in "vg" else D), W, seed=i, std=.2) for i, k in enumerate("qkvg")} | {"o": r(W, H * V, seed=5)}
+    if mixer == "linear":
+        m = LinearAttention(W, H, D, V, 1e-3, k_scale=0.5, tau=tau, weighted=True)
+        w |= {"norm": r(V, seed=6), "a1": r(5, W, seed=7, std=.1), "a2": r(H * D, 5, seed=8, std=.4), "a2.b": 6 * r(H * D, seed=9)}
+    else:
+        m = MatrixMemory(W, H, D, V, cap, 1e-3)
+        w |= {"norm": r(H * V, seed=6), "i": r(H, W, seed=7, std=.3), "i.b": r(H, seed=8), "f": r(H, W, seed=9, std=.2),
+              "f.b": 3 + r(H, seed=10)}
+    into, _ = m.load(w, BF16, dev, W)
+    n = sum(counts)
+    h = r(n, W, seed=16)
+    proj = (h.float() @ into.float().cpu().T).to(BF16).to(dev)
+    state, out = m.allocate(len(counts), BF16, dev), torch.empty(n, H * V, dtype=BF16, device=dev)
+    rows, ctx = _run_segments(dev, counts)
+    m.scan(*([h.to(dev)] if mixer == "memory" else []), proj, state, ctx, out)
+    P, hh = proj.double().cpu(), h.double()
+    k, v = P[:, H * D:2 * H * D].view(n, H, D), P[:, 2 * H * D:2 * H * D + H * V].view(n, H, V)
+    if mixer == "linear":
+        low = torch.nn.functional.linear(proj[:, m.low_at:m.low_at + m.low_rank], m.low).double().cpu()
+        g = (torch.sigmoid(low.view(n, H, D) + w["a2.b"].double().view(H, D)) ** (1 / tau))[..., None]
+        k = k * 0.5
+    else:
+        i = cap * torch.tanh((hh @ w["i"].double().T + w["i.b"].double()) / cap)
+        f = torch.nn.functional.logsigmoid(cap * torch.tanh((hh @ w["f"].double().T + w["f.b"].double()) / cap))
+    for s, (a, c) in enumerate(zip(rows, counts)):
+        S, top = torch.zeros(H, D, V, dtype=torch.float64), torch.zeros(H, dtype=torch.float64)
+        for t in range(a, a + c):
+            if mixer == "linear":
+                S = g[t] * S + k[t][:, :, None] * v[t][:, None, :]
+            else:
+                new = torch.maximum(f[t] + top, i[t])
+                S = torch.exp(f[t] + top - new)[:, None, None] * S + (torch.exp(i[t] - new)[:, None] * k[t])[:, :, None] * v[t][:, None, :]
+                top = new
+        # as above; the memory's gates are sums of 64 products in fp32, whose error their exponentials take over
+        err = (state[s][..., :D * V].flatten(1).double().cpu().view(H, D, V) - S).norm() / S.norm() if mixer == "memory" else \
+            (state[s].double().cpu().view(H, D, V) - S).norm() / S.norm()
         assert float(err) < 2.0 ** -19, float(err)
