@@ -128,11 +128,12 @@ template <int NC> __device__ __forceinline__ void block_squares(const f32x4 (&o)
   for (int r = 0; r < 4; ++r) ss[r] = row16_sum(ss[r]);
   if (l16 == 0) *(f32x4*)(red + wave * kBlock + 4 * g) = ss;
 }
+// Each lane of a group of sixteen reads one wave's share.
 template <int NW> __device__ __forceinline__ f32x4 block_squares_total(const float* red) {
-  const int g = (threadIdx.x & 63) >> 4;
-  f32x4 ss = {0.f, 0.f, 0.f, 0.f};
+  const int l16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
+  f32x4 ss = *(const f32x4*)(red + min(l16, NW - 1) * kBlock + 4 * g);
 #pragma unroll
-  for (int w = 0; w < NW; ++w) ss += *(const f32x4*)(red + w * kBlock + 4 * g);
+  for (int r = 0; r < 4; ++r) ss[r] = row16_sum(l16 < NW ? ss[r] : 0.f);
   return ss;
 }
 
