@@ -264,3 +264,38 @@ def test_states_of_runs(dev, mixer, H, D, V):
         err = (state[s][..., :D * V].flatten(1).double().cpu().view(H, D, V) - S).norm() / S.norm() if mixer == "memory" else \
             (state[s].double().cpu().view(H, D, V) - S).norm() / S.norm()
         assert float(err) < 2.0 ** -19, float(err)
+
+
+# ------------------------------------------------------------------ latent rows
+# up to 32 heads of up to 256 columns a wave goes its own way; more of either: a ring of stages of 32 keys, page ids
+# fetched 64 at a time, a token's keys cut into ranges of at least four stages
+@pytest.mark.parametrize("H,R,P,BS,window", [(1, 288, 8, 16, None), (17, 512, 64, 16, 1100), (33, 128, 24, 16, None),
+                                             (48, 256, 0, 32, 65), (65, 384, 40, 16, 1), (32, 256, 8, 16, None),
+                                             (16, 512, 0, 64, None), (128, 32, 64, 16, 700)])
+def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
+    from zipage_amd.layers import latent_rows_attention
+    ctx = [0, 1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 130, 160, 193, 1023, 1024, 1025, 2080, 2500]
+    n, NB = len(ctx), -(-2500 // BS)
+    g = torch.Generator().manual_seed(H + R)
+    tables = torch.randperm(n * NB, generator=g).view(n, NB).int()
+    cache, q = _rand(n * NB, BS, R + P, seed=3), _rand(n, H, R + P, seed=4, std=4.0 * (R + P) ** -0.5)
+    want = torch.zeros(n, H, R, dtype=torch.double)
+    absolute = torch.zeros_like(want)
+    for i, c in enumerate(ctx):
+        low = max(0, c - window) if window else 0
+        if c:
+            rows = cache[tables[i].long()].reshape(-1, R + P)[low:c].double()
+            p = (q[i].double() @ rows.T).softmax(-1)
+            want[i], absolute[i] = p @ rows[:, :R], p @ rows[:, :R].abs()
+        tables[i, :low // BS] = -1                       # in front of the window: never read
+        tables[i, -(-c // BS):] = 1 << 30                # nor past the last key
+    t = lambda a: torch.as_tensor(a, dtype=torch.int32).to(dev)
+    qd, cd, td = q.to(dev), cache.to(dev), t(tables)
+    # probabilities in bf16 (2^-8 of a term and as much of the sum they are over), the result once more (2^-8)
+    allowed = (2 * 2.0 ** -8 * absolute + 2.0 ** -8 * want.abs()) * 1.01 + 1e-6
+    got = latent_rows_attention(qd, cd, td, t(ctx), 1.0, window, rank=R).cpu().double()
+    assert not got[0].any()
+    assert ((got - want).abs() <= allowed).all()
+    for i in (8, 16, 19):                                # alone: its keys cut into more ranges
+        one = latent_rows_attention(qd[i:i + 1], cd, td[i:i + 1], t(ctx[i:i + 1]), 1.0, window, rank=R).cpu().double()
+        assert ((one - want[i:i + 1]).abs() <= allowed[i:i + 1]).all()

@@ -171,24 +171,11 @@ __device__ __forceinline__ f32x4 read_columns(const char* p) {
                bf16_bits_to_float((uint16_t)v[3])};
 }
 
-// Loads straight into LDS: lane l's 16 bytes from `base` + offset (+ uniform) to `lds` + 16 l.  Written out,
-// because the compiler, which cannot tell the stage being filled from the stage being read, would wait for
-// them at the next LDS read; wait_and_meet() waits for them.
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
+// Loads straight into LDS; wait_and_meet() waits for them.
 struct StageLoads {
   u32x4 rs;
-  __device__ __forceinline__ StageLoads(const void* base, int64_t bytes) {
-    const uint64_t p = (uint64_t)base;
-    rs = u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(p >> 32) & 0xffffu)),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
-  }
-  __device__ __forceinline__ void ld(void* lds, int offset, int uniform) const {
-    const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
-    const int so = __builtin_amdgcn_readfirstlane(uniform);
-    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-                 :: "s"(to), "v"(offset), "s"(rs), "s"(so) : "memory", "m0");
-  }
+  __device__ __forceinline__ StageLoads(const void* base, int64_t bytes) : rs(rows_from(base, (uint32_t)bytes)) {}
+  __device__ __forceinline__ void ld(void* lds, int offset, int uniform) const { load_to_lds(rs, lds, offset, uniform); }
 };
 __device__ __forceinline__ void wait_and_meet() {
   asm volatile("" ::: "memory");

@@ -243,8 +243,7 @@ struct RowsArgs {
   int n, H, R, P, BS, bs_shift, B, NB, num_pages;   // P: elements that only join the scores
   int window;             // a token sees the last `window` tokens including itself; 0 = all
   int splits;             // key ranges handled by different workgroups
-  int hw;                 // waves of a workgroup on different heads (1, 2, 4); the others split keys
-  int lds_pages;          // page ids held in LDS
+  int lds_pages;          // narrow rows: page ids held in LDS
   float scale;
 };
 
@@ -252,8 +251,10 @@ __device__ __forceinline__ int page_of(const RowsArgs& a, int t) {
   return a.bs_shift >= 0 ? t >> a.bs_shift : t / a.BS;
 }
 
-// NCB column blocks of 128 cover R.  Workgroup: one token, 16 * HT * hw heads, one key range.  A wave
-// computes HT tiles of 16 heads on the same keys: with two, the second tile costs no key or value read.
+// Rows of at most 256 for up to 32 heads: a step of 32 keys is too little work to have the waves meet for it (256
+// sequences, 16 heads: 72 us; by the kernel below 75), so every wave goes its own way.  NCB column blocks of 128 cover R.
+// Workgroup: one token, one key range.  A wave computes HT tiles of 16 heads on the same keys: with two, the second tile
+// costs no key or value read.
 //
 // A wave takes 32 keys at a time.  They come from memory once, as whole 256-byte row pieces (lane: 8
 // keys x 8 columns), and stay in registers as the value operand; the key operand (lane: one key, 8
@@ -271,32 +272,25 @@ template <int NCB, int PK> struct RowsLds {
 __host__ __device__ inline int rows_merge_floats(int R) { return 16 * (R + 4) + 32; }   // per wave
 
 template <int NCB, int HT, int PK>
-__global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel(RowsArgs a) {
+__global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kernel(RowsArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef RowsLds<NCB, PK> Lds;
   int* pg = (int*)lds_raw;
   char* const shared = lds_raw + ((a.lds_pages * 4 + 15) & ~15);
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int l16 = lane & 15, g = lane >> 4;
-  const int hw = a.hw, kw = 4 / hw, hwi = wave % hw, kwi = wave / hw;
   uint16_t* const stage = (uint16_t*)(shared + wave * Lds::kStage);
   uint16_t* const qlds = (uint16_t*)(shared + 4 * Lds::kStage);
-  const int hgroups = (a.H + 16 * HT * hw - 1) / (16 * HT * hw);
-  int id = blockIdx.x;
-  const int split = id % a.splits;
-  id /= a.splits;
-  const int hg = id % hgroups;
-  const int row = id / hgroups;
-  const int head0 = hg * hw * HT * 16;
+  const int split = blockIdx.x % a.splits, row = blockIdx.x / a.splits;
   // queries to LDS, zeros past R and past the last head
   const int RW = a.R + a.P;
   constexpr int kQPieces = NCB * 16 + PK * 4;
-  for (int it = tid; it < hw * HT * 16 * kQPieces; it += 256) {
+  for (int it = tid; it < HT * 16 * kQPieces; it += 256) {
     const int hl = it / kQPieces, c = (it % kQPieces) * 8;
     const int p = c - NCB * 128;                                 // >= 0: of the rotated part
     u32x4 v = {0u, 0u, 0u, 0u};
-    if (head0 + hl < a.H && (p < 0 ? c < a.R : p < a.P))
-      v = *(const u32x4*)((const uint16_t*)a.q + ((int64_t)row * a.H + head0 + hl) * RW + (p < 0 ? c : a.R + p));
+    if (hl < a.H && (p < 0 ? c < a.R : p < a.P))
+      v = *(const u32x4*)((const uint16_t*)a.q + ((int64_t)row * a.H + hl) * RW + (p < 0 ? c : a.R + p));
     *(u32x4*)(qlds + hl * Lds::kQStride + c) = v;
   }
   const int seq = a.seq ? min(max(a.seq[row], 0), a.B - 1) : row;
@@ -329,7 +323,7 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel
     for (int i = 0; i < NCB * 8; ++i) o[ht][i] = f32x4{0.f, 0.f, 0.f, 0.f};
   }
   const float sc = a.scale * 1.44269504088896f;
-  const uint16_t* const qrow = qlds + (hwi * HT * 16 + l16) * Lds::kQStride + g * 8;
+  const uint16_t* const qrow = qlds + l16 * Lds::kQStride + g * 8;
   const int mask = a.BS - 1;
   u32x4 v[NCB][8], kr[2][PK ? PK : 1];
   int rot_off[PK ? PK : 1];                   // past P: the part's start again, against zeros in q
@@ -366,8 +360,8 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel
     }
   };
 
-  const int b1 = n > 0 ? (n - 1) >> 5 : -1, step = a.splits * kw;
-  int b = (lo >> 5) + split * kw + kwi;
+  const int b1 = n > 0 ? (n - 1) >> 5 : -1, step = a.splits * 4;
+  int b = (lo >> 5) + split * 4 + wave;
   if (b <= b1) {
     locate(b);
 #pragma unroll
@@ -493,21 +487,21 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel
     }
     __syncthreads();
     // per head: the common maximum, each key part's factor (over its maximum's place) and the sum
-    if (tid < hw * 16) {
-      float* const src = merge + (tid >> 4) * per + 16 * RS + (tid & 15);   // wave k * hw + tile: key part k
+    if (tid < 16) {
+      float* const src = merge + 16 * RS + tid;              // wave k: key part k
       float mx = src[0];
-      for (int k = 1; k < kw; ++k) mx = fmaxf(mx, src[k * hw * per]);
+      for (int k = 1; k < 4; ++k) mx = fmaxf(mx, src[k * per]);
       const float ms = mx == -INFINITY ? 0.f : mx;
       float sum = 0.f;
-      for (int k = 0; k < kw; ++k) {
-        float* const at = src + k * hw * per;
+      for (int k = 0; k < 4; ++k) {
+        float* const at = src + k * per;
         const float f = __builtin_amdgcn_exp2f(at[0] - ms);
         sum += at[16] * f;
         at[0] = f;
       }
       const float inv = a.splits > 1 ? 1.f : (sum > 0.f ? 1.f / sum : 0.f);
-      for (int k = 0; k < kw; ++k) src[k * hw * per] *= inv;
-      const int head = head0 + ((tid >> 4) * HT + ht) * 16 + (tid & 15);
+      for (int k = 0; k < 4; ++k) src[k * per] *= inv;
+      const int head = ht * 16 + tid;
       if (a.splits > 1 && head < a.H) {
         float* ml = a.part + (int64_t)a.n * a.H * a.splits * a.R + (((int64_t)row * a.H + head) * a.splits + split) * 2;
         ml[0] = mx;
@@ -516,17 +510,16 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel
     }
     __syncthreads();
 #pragma unroll 1
-    for (int it = tid; it < hw * 256 * NCB; it += 256) {
+    for (int it = tid; it < 256 * NCB; it += 256) {
       const int hl = it / (16 * NCB), c = it % (16 * NCB) * 8;
-      const int head = head0 + ((hl >> 4) * HT + ht) * 16 + (hl & 15);
+      const int head = ht * 16 + hl;
       if (head >= a.H || c >= a.R) continue;
-      const float* src = merge + (hl >> 4) * per;
       float r[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int k = 0; k < kw; ++k) {
-        const float* part = src + k * hw * per;
-        const float f = part[16 * RS + (hl & 15)];
+      for (int k = 0; k < 4; ++k) {
+        const float* part = merge + k * per;
+        const float f = part[16 * RS + hl];
         float x[8];
-        Vec8<F32>::ld(part, (hl & 15) * RS + c, x);
+        Vec8<F32>::ld(part, hl * RS + c, x);
 #pragma unroll
         for (int i = 0; i < 8; ++i) r[i] += x[i] * f;
       }
@@ -534,6 +527,235 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_rows_kernel
       if (a.splits == 1) Vec8<BF16>::st(a.out, item * a.R + c, r);
       else Vec8<F32>::st(a.part, (item * a.splits + split) * a.R + c, r);
     }
+  }
+}
+
+// NCB column blocks of 128 cover R; PK steps of 32 the rotated part, which is a key only, never a value.  Workgroup: one
+// token, HW tiles of 16 heads, one key range.  All four waves take the same 32 keys; waves on the same head tile
+// (4 / HW) share its value columns out and compute its scores each for itself, so that they meet only to hand over LDS.
+//
+// Bound by HBM, so what counts is how much is on its way: rows go from memory into LDS without passing through
+// registers, in a ring of stages of 32 keys of which all but one are in flight (128 KB per CU for rows of 576; held in
+// registers between its two uses, a block left its place only when its products were done: 256 sequences of 2050 tokens,
+// 32 heads 157 us, now 141; a window of 1024 76, now 60; 64 sequences, 128 heads 124, now 92).  The value operand is
+// transposed by the LDS reads.  An odd number of 16-byte pieces per staged row keeps both operands off each other's banks.
+constexpr int rows_ring(int NCB) { return NCB <= 2 ? 3 : 4; }       // two workgroups per CU where rows are short
+template <int NCB, int PK> struct RowsStage {
+  static constexpr int kMaxPieces = NCB * 16 + PK * 4 + 1;
+  static constexpr int kHalf = (kMaxPieces + 3) / 4 * 1024;           // bytes of 16 keys, whole loads
+  static constexpr int kLoads = ((kMaxPieces + 3) / 4 + 1) / 2;       // of a wave for a stage
+  static constexpr int kBytes = rows_ring(NCB) * 2 * kHalf;
+};
+
+template <int NCB, int HW, int PK>
+__global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_kernel(RowsArgs a) {
+  extern __shared__ __align__(16) char lds_raw[];
+  typedef RowsStage<NCB, PK> Stage;
+  constexpr int kRing = rows_ring(NCB), KS = 4 * NCB, VT = NCB * 8 / (4 / HW);     // value tiles of 16 columns of a wave
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
+  int id = blockIdx.x;
+  const int split = id % a.splits;
+  id /= a.splits;
+  const int row = id / hgroups, head = (id % hgroups * HW + wave % HW) * 16 + l16;
+  const int RW = a.R + a.P, pieces = RW / 8, staged = pieces | 1;
+  const int col0 = wave / HW * VT * 16;                          // of the wave's values
+
+  u32x4 q[KS + PK];
+#pragma unroll
+  for (int ks = 0; ks < KS + PK; ++ks) {
+    const int c = ks < KS ? ks * 32 + g * 8 : (ks - KS) * 32 + g * 8;
+    const bool there = head < a.H && c < (ks < KS ? a.R : a.P);
+    q[ks] = u32x4{0u, 0u, 0u, 0u};
+    if (there) q[ks] = *(const u32x4*)((const uint16_t*)a.q + ((int64_t)row * a.H + head) * RW + (ks < KS ? c : a.R + c));
+  }
+  const int seq = a.seq ? min(max(a.seq[row], 0), a.B - 1) : row;
+  const int n = min(a.ctx[row], a.NB * a.BS);
+  const int lo = a.window > 0 ? max(0, n - a.window) : 0;
+  const int b0 = (lo >> 5) + split, b1 = n > 0 ? (n - 1) >> 5 : -1;
+  const int blocks = b1 >= b0 ? (b1 - b0) / a.splits + 1 : 0;
+
+  // ---- rows into LDS: 16 keys of a page with `staged` pieces each, by loads of 64 pieces.  A wave has every other load of
+  // one half of the keys; its last may come twice.
+  const int half = wave & 1, loads = (staged + 3) / 4;
+  int piece_at[Stage::kLoads];                                   // byte of a lane's piece in 16 rows, row in the upper bits
+#pragma unroll
+  for (int k = 0; k < Stage::kLoads; ++k) {
+    const int p = min((wave >> 1) + 2 * k, loads - 1) * 64 + lane, r = min(p / staged, 15), pc = p - r * staged;
+    piece_at[k] = (r * RW * 2 + (pc < pieces ? pc : 0) * 16) | r << 20;
+  }
+  const int mask = a.BS - 1;
+  // page ids of the table from page0 on, one a lane; 64 are enough for a while
+  int page0 = lo >> a.bs_shift, ids;
+  auto fetch_ids = [&] {
+    const int at = page0 + lane, id = at < a.NB ? a.table[(int64_t)seq * a.NB + at] : 0;
+    ids = id >= 0 && id < a.num_pages ? id : 0;                  // whatever the table says, it is one of the cache's
+  };
+  fetch_ids();
+  // what the loads of stage j need, then load k of them
+  char* to;
+  int h0, from, upto;
+  bool whole;
+  u32x4 rows;
+  auto locate = [&](int j) {
+    const bool there = j < blocks;                               // past the last block nothing is read
+    h0 = (b0 + j * a.splits) * 32 + half * 16;
+    to = lds_raw + (j % kRing) * (2 * Stage::kHalf) + half * Stage::kHalf;
+    // keys outside the visible range repeat a visible row, with weight zero
+    from = h0 + 15 < lo ? lo : min(max(h0, lo), n - 1), upto = h0 + 15 < lo ? lo : max(min(h0 + 15, n - 1), from);
+    const int index = there ? from >> a.bs_shift : page0;
+    if (index >= page0 + 64) {                                   // uniform
+      page0 = index;
+      fetch_ids();
+    }
+    const char* const page = (const char*)a.cache + (int64_t)__builtin_amdgcn_readlane(ids, index - page0) * a.BS * RW * 2;
+    whole = from == h0 && upto == h0 + 15;
+    const int first = whole ? (h0 & mask) * RW * 2 : 0;
+    rows = rows_from(page + first, there ? (uint32_t)a.BS * RW * 2 - first : 0u);
+  };
+  auto load = [&](int k, bool all) {
+    char* const at = to + min((wave >> 1) + 2 * k, loads - 1) * 1024;
+    if (all) {
+      load_to_lds(rows, at, piece_at[k] & 0xfffff, 0);
+    } else {
+      const int r = piece_at[k] >> 20, key = min(max(h0 + r, from), upto);
+      load_to_lds(rows, at, (piece_at[k] & 0xfffff) + ((key & mask) - r) * RW * 2, 0);
+    }
+  };
+#pragma unroll
+  for (int j = 0; j < kRing - 1; ++j) {
+    locate(j);
+    if (whole)
+#pragma unroll
+      for (int k = 0; k < Stage::kLoads; ++k) load(k, true);
+    else
+#pragma unroll
+      for (int k = 0; k < Stage::kLoads; ++k) load(k, false);
+  }
+
+  f32x4 o[VT];
+#pragma unroll
+  for (int i = 0; i < VT; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m = -INFINITY, l = 0.f;
+  const float sc = a.scale * 1.44269504088896f;
+  // R may end inside the last column block: columns past it are others again, against zeros in q or in results that are not
+  // written
+  const int key_at = l16 * staged * 16 + g * 16, value_at = (4 * g + (l16 >> 2)) * staged * 16 + (l16 & 3) * 8;
+  int rot_at[PK ? PK : 1];
+#pragma unroll
+  for (int ks = 0; ks < PK; ++ks) rot_at[ks] = l16 * staged * 16 + (a.R / 8 + (ks * 32 + g * 8 < a.P ? ks * 4 + g : 0)) * 16;
+#pragma unroll 1
+  for (int j = 0; j < blocks; ++j) {
+    // this wave's share of block j has come when at most those of the blocks behind it are on their way
+    static_assert((kRing - 2) * Stage::kLoads < 64, "the counter's range");
+    constexpr int kOn = (kRing - 2) * Stage::kLoads;
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (kOn & 15) | (kOn >> 4) << 14);      // LDS reads of the block before are done, too
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    locate(j + kRing - 1);                                       // over what the block before was in
+    const int k0 = (b0 + j * a.splits) * 32;
+    const char* const at = lds_raw + (j % kRing) * (2 * Stage::kHalf);
+    // operands leave LDS kAhead products ahead; the barriers keep the compiler from moving a read to its use
+    constexpr int kAhead = 4, kRead = kAhead + 1, kKeys = KS + PK;
+    u32x4 kf[kRead];
+    auto read_key = [&](int i) {                                 // of half i / kKeys, step i % kKeys
+      if (i >= 2 * kKeys) return;
+      const int ks = i % kKeys;
+      const int c = ks < KS ? key_at + (ks < KS - 4 ? ks * 64 : min(ks * 64, a.R * 2 - 64)) : rot_at[ks < KS ? 0 : ks - KS];
+      kf[i % kRead] = *(const u32x4*)(at + i / kKeys * Stage::kHalf + c);
+    };
+    f32x4 part[2][2] = {};                                       // of both halves, even and odd steps
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) read_key(i);
+    auto scores = [&](bool loads_too) {
+#pragma unroll
+      for (int i = 0; i < 2 * kKeys; ++i) {
+        read_key(i + kAhead);
+        const int hf = i / kKeys, ks = i % kKeys;
+        part[hf][ks & 1] = mfma_bf16(kf[i % kRead], q[ks], part[hf][ks & 1]);
+        if (loads_too)
+#pragma unroll
+          for (int k = i * Stage::kLoads / (2 * kKeys); k < (i + 1) * Stage::kLoads / (2 * kKeys); ++k) load(k, true);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    if (whole) {                                                 // the loads are spread over the products
+      scores(true);
+    } else {
+#pragma unroll
+      for (int k = 0; k < Stage::kLoads; ++k) load(k, false);
+      scores(false);
+    }
+    const f32x4 s[2] = {part[0][0] + part[0][1], part[1][0] + part[1][1]};
+    u32x4 vf[kRead];
+    auto read_value = [&](int i) {
+      if (i >= VT) return;
+      const int c = col0 + i * 16;
+      const char* const v = at + value_at + (c < a.R ? c : 0) * 2;
+      const uint2 x = read_transposed((const uint16_t*)v), y = read_transposed((const uint16_t*)(v + Stage::kHalf));
+      vf[i % kRead] = u32x4{x.x, x.y, y.x, y.y};
+    };
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) read_value(i);
+    __builtin_amdgcn_sched_barrier(0);
+    float p[8], mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) p[i] = s[i >> 2][i & 3] * sc;
+    if (k0 < lo || k0 + 31 >= n) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int key = k0 + step_key(g, i);
+        if (key < lo || key >= n) p[i] = -INFINITY;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) mx = fmaxf(mx, p[i]);
+    if (__any(mx > m)) {                                         // in any lane: seldom after the first keys
+      mx = fmaxf(m, mx);
+      mx = fmaxf(mx, lane_xor16(mx));
+      mx = fmaxf(mx, lane_xor32(mx));                            // finite: every block holds a visible key
+      const float f = __builtin_amdgcn_exp2f(m - mx);
+      m = mx;
+      l *= f;
+#pragma unroll
+      for (int i = 0; i < VT; ++i) o[i] *= f;
+    }
+    float sum = 0.f;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      p[i] = __builtin_amdgcn_exp2f(p[i] - m);
+      sum += p[i];
+    }
+    l += sum;
+    const u32x4 pf = {pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7])};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < VT; ++i) {
+      read_value(i + kAhead);
+      o[i] = mfma_bf16(vf[i % kRead], pf, o[i]);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  }
+  __builtin_amdgcn_s_waitcnt(0);                                 // no load is left on its way to LDS
+  l += lane_xor16(l);
+  l += lane_xor32(l);
+  if (head >= a.H) return;
+  const int64_t item = (int64_t)row * a.H + head;
+  const float inv = a.splits > 1 ? 1.f : (l > 0.f ? 1.f / l : 0.f);
+#pragma unroll
+  for (int i = 0; i < VT; ++i) {
+    const int c = col0 + i * 16 + 4 * g;
+    if (c >= a.R) continue;
+    o[i] *= inv;
+    if (a.splits == 1) *(uint2*)((uint16_t*)a.out + item * a.R + c) = uint2{pack_bf16(o[i][0], o[i][1]), pack_bf16(o[i][2], o[i][3])};
+    else *(f32x4*)(a.part + (item * a.splits + split) * a.R + c) = o[i];
+  }
+  if (a.splits > 1 && wave < HW && g == 0) {
+    float* const ml = a.part + (int64_t)a.n * a.H * a.splits * a.R + (item * a.splits + split) * 2;
+    ml[0] = m;
+    ml[1] = l;
   }
 }
 
@@ -633,45 +855,75 @@ __global__ __launch_bounds__(256) void latent_plain_kernel(RowsArgs a) {
 
 constexpr int kMaxLdsPages = 4096, kMaxRotated = 64;
 
-// Head tiles per wave, and waves of a workgroup on different heads.
-int rows_ht(int H, int R) { return H > 16 && R <= 256 ? 2 : 1; }   // registers hold 2 x 256 columns
-int rows_hw(int H, int R) {
-  const int tiles = (H + 16 * rows_ht(H, R) - 1) / (16 * rows_ht(H, R));
-  return tiles >= 4 ? 4 : (tiles >= 2 ? 2 : 1);
-}
+// Which rows the narrow kernel takes, with its head tiles per wave.  Past 32 heads it would take a head's keys with fewer
+// waves and read a row twice (256 columns, 40 heads, a window of 300 keys: 49 us against 27), and wider rows don't fit
+// its registers with two tiles; up to 32 heads of 16 to 256 columns it is ahead by 2 to 20 per cent.
+bool rows_narrow(int H, int R) { return R <= 256 && H <= 32; }
+int rows_ht(int H) { return H > 16 ? 2 : 1; }
+// Head tiles of a workgroup of the other one.
+int rows_hw(int H) { return H > 32 ? 4 : (H > 16 ? 2 : 1); }
 
-// Key ranges per token: enough workgroups to cover the chip, at least two 32-key steps per wave.
+// Key ranges per token: enough workgroups to cover the chip, at least four 32-key steps each (of the narrow kernel two per
+// wave).
 int rows_splits(int n, int H, int R, int window, int NB, int BS) {
-  const int hw = rows_hw(H, R), kw = 4 / hw, per = 16 * rows_ht(H, R) * hw;
-  const int groups = n * ((H + per - 1) / per);
+  const bool narrow = rows_narrow(H, R);
+  const int groups = narrow ? n : n * ((H + 16 * rows_hw(H) - 1) / (16 * rows_hw(H)));
   int64_t keys = (int64_t)NB * BS;
   if (window > 0 && window < keys) keys = window;
   const int steps = (int)((keys + 31) / 32);
-  const int resident = (R + 127) / 128 * rows_ht(H, R) <= 2 ? 2 : 1;       // workgroups per CU
+  const int resident = (narrow ? (R + 127) / 128 * rows_ht(H) : (R + 127) / 128) <= 2 ? 2 : 1;       // workgroups per CU
+  const int least = narrow ? 8 : 4;
   int s = 256 * resident / (groups > 0 ? groups : 1);
-  s = s < steps / (2 * kw) ? s : steps / (2 * kw);
+  s = s < steps / least ? s : steps / least;
   s = s < 32 ? s : 32;
   return s < 1 ? 1 : s;
 }
 
-template <int NCB, int HT, int PK> int launch_latent_rows(RowsArgs a, hipStream_t st) {
-  const size_t merge = 4 * sizeof(float) * (size_t)rows_merge_floats(a.R);
-  const size_t work = 4 * RowsLds<NCB, PK>::kStage + (size_t)a.hw * HT * RowsLds<NCB, PK>::kQ;
-  const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + (merge > work ? merge : work);
-  if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)latent_rows_kernel<NCB, HT, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                          (int)smem) != hipSuccess) {
-    zp_set_error("latent_rows_attention: cannot reserve %zu bytes of LDS", smem);
-    return ZP_EHIP;
-  }
-  const int hgroups = (a.H + 16 * HT * a.hw - 1) / (16 * HT * a.hw);
-  hipLaunchKernelGGL((latent_rows_kernel<NCB, HT, PK>), dim3((unsigned)a.n * hgroups * a.splits), dim3(256), smem, st, a);
-  ZP_LAUNCH_CHECK();
+int launch_combine(const RowsArgs& a, hipStream_t st) {
   if (a.splits > 1) {
     hipLaunchKernelGGL(latent_rows_combine_kernel, dim3((unsigned)a.n * a.H), dim3(64), 0, st, a);
     ZP_LAUNCH_CHECK();
   }
   return ZP_OK;
+}
+template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
+  const size_t merge = 4 * sizeof(float) * (size_t)rows_merge_floats(a.R);
+  const size_t work = 4 * RowsLds<NCB, PK>::kStage + (size_t)HT * RowsLds<NCB, PK>::kQ;
+  const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + (merge > work ? merge : work);
+  if (smem > 64 * 1024 &&
+      hipFuncSetAttribute((const void*)latent_narrow_kernel<NCB, HT, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          (int)smem) != hipSuccess) {
+    zp_set_error("latent_rows_attention: cannot reserve %zu bytes of LDS", smem);
+    return ZP_EHIP;
+  }
+  hipLaunchKernelGGL((latent_narrow_kernel<NCB, HT, PK>), dim3((unsigned)a.n * a.splits), dim3(256), smem, st, a);
+  ZP_LAUNCH_CHECK();
+  return launch_combine(a, st);
+}
+template <int NCB, int HW, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
+  constexpr int smem = RowsStage<NCB, PK>::kBytes;
+  if (smem > 64 * 1024 &&
+      hipFuncSetAttribute((const void*)latent_rows_kernel<NCB, HW, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                          smem) != hipSuccess) {
+    zp_set_error("latent_rows_attention: cannot reserve %d bytes of LDS", smem);
+    return ZP_EHIP;
+  }
+  const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
+  hipLaunchKernelGGL((latent_rows_kernel<NCB, HW, PK>), dim3((unsigned)a.n * hgroups * a.splits), dim3(256), smem, st, a);
+  ZP_LAUNCH_CHECK();
+  return launch_combine(a, st);
+}
+template <int NCB, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
+  if constexpr (NCB <= 2) {
+    if (!rows_narrow(a.H, a.R)) return launch_latent_rows<NCB, 4, PK>(a, st);
+    return rows_ht(a.H) == 2 ? launch_latent_narrow<NCB, 2, PK>(a, st) : launch_latent_narrow<NCB, 1, PK>(a, st);
+  } else {
+    switch (rows_hw(a.H)) {
+      case 1: return launch_latent_rows<NCB, 1, PK>(a, st);
+      case 2: return launch_latent_rows<NCB, 2, PK>(a, st);
+      default: return launch_latent_rows<NCB, 4, PK>(a, st);
+    }
+  }
 }
 
 }  // namespace
@@ -799,10 +1051,11 @@ extern "C" int zp_latent_rows_attention(const void* q, const void* cache, const 
   a.num_pages = num_pages; a.window = window; a.scale = scale; a.bs_shift = -1;
   if ((BS & (BS - 1)) == 0)
     for (a.bs_shift = 0; (1 << a.bs_shift) < BS; ++a.bs_shift) {}
+  hipStream_t st = (hipStream_t)stream;
   int64_t pages = NB;
   if (window > 0 && (window - 1) / BS + 2 < pages) pages = (window - 1) / BS + 2;
-  hipStream_t st = (hipStream_t)stream;
-  if (dtype == ZP_F32 || R > 512 || P > kMaxRotated || pages > kMaxLdsPages || a.bs_shift < 4) {   // bs_shift -1: not a power of two
+  if (dtype == ZP_F32 || R > 512 || P > kMaxRotated || a.bs_shift < 4 || (rows_narrow(H, R) && pages > kMaxLdsPages) ||
+      (int64_t)BS * (R + P) * 2 >= 1ll << 31) {   // bs_shift -1: not a power of two
     const size_t smem = sizeof(float) * (R + P);
     if (dtype == ZP_BF16)
       hipLaunchKernelGGL((latent_plain_kernel<BF16>), dim3((unsigned)n * H), dim3(256), smem, st, a);
@@ -811,18 +1064,16 @@ extern "C" int zp_latent_rows_attention(const void* q, const void* cache, const 
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }
-  a.hw = rows_hw(H, R);
   a.lds_pages = (int)pages;
   a.splits = rows_splits(n, H, R, window, NB, BS);
   ZP_REQUIRE(a.splits == 1 || (workspace && workspace_bytes >= zp_latent_rows_workspace(n, H, R, window, NB, BS, dtype)),
              "latent_rows_attention: workspace too small");
-  const bool two = rows_ht(H, R) == 2;
-#define ZP_LATENT_ROWS(NCB, HT) (P ? launch_latent_rows<NCB, HT, 2>(a, st) : launch_latent_rows<NCB, HT, 0>(a, st))
+#define ZP_LATENT_ROWS(NCB) (P ? launch_latent_rows<NCB, 2>(a, st) : launch_latent_rows<NCB, 0>(a, st))
   switch ((R + 127) / 128) {
-    case 1: return two ? ZP_LATENT_ROWS(1, 2) : ZP_LATENT_ROWS(1, 1);
-    case 2: return two ? ZP_LATENT_ROWS(2, 2) : ZP_LATENT_ROWS(2, 1);
-    case 3: return ZP_LATENT_ROWS(3, 1);
-    default: return ZP_LATENT_ROWS(4, 1);
+    case 1: return ZP_LATENT_ROWS(1);
+    case 2: return ZP_LATENT_ROWS(2);
+    case 3: return ZP_LATENT_ROWS(3);
+    default: return ZP_LATENT_ROWS(4);
   }
 #undef ZP_LATENT_ROWS
 }

@@ -27,6 +27,24 @@ __device__ __forceinline__ uint2 read_transposed(const uint16_t* p) {
   return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) zp_s16x4*)p));
 }
 
+// A load straight into LDS: lane l's 16 bytes from `rows` + lane_at (+ at) to `lds` + 16 l.  Written out, because the compiler,
+// which cannot tell the stage being filled from the stage being read, would wait for it at the next LDS read; what
+// waits is the code that meets the other waves.
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
+__device__ __forceinline__ void load_to_lds(const u32x4& rows, void* lds, int lane_at, int at) {
+  const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
+  const int so = __builtin_amdgcn_readfirstlane(at);
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               :: "s"(to), "v"(lane_at), "s"(rows), "s"(so) : "memory", "m0");
+}
+// What such loads read: `bytes` from `base` on, zeros behind them.
+__device__ __forceinline__ u32x4 rows_from(const void* base, uint32_t bytes) {
+  const uint64_t p = (uint64_t)base;
+  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)p),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)((uint32_t)(p >> 32) & 0xffffu)),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)bytes), 0x00020000u};
+}
+
 // Eight rows (keys) of eight bf16 columns -> for column t the four dwords of its eight keys.
 __device__ __forceinline__ u32x4 column_of(const u32x4* rows, int t) {
   const uint32_t sel = (t & 1) ? 0x07060302u : 0x05040100u;

@@ -392,7 +392,6 @@ template <int CH, int FLIP, int GAP> struct Staged {
   }
 };
 constexpr int kFlowV = 64;
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // The row at `from` and those behind it; every lane reads within rows that are there: the bound is none of the buffer's.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const void* from) {
   return __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, 0x7fffffff, 0x00020000);
