@@ -299,3 +299,26 @@ def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
     for i in (8, 16, 19):                                # alone: its keys cut into more ranges
         one = latent_rows_attention(qd[i:i + 1], cd, td[i:i + 1], t(ctx[i:i + 1]), 1.0, window, rank=R).cpu().double()
         assert ((one - want[i:i + 1]).abs() <= allowed[i:i + 1]).all()
+
+
+# ------------------------------------------------------------------ per-head products
+# through LDS: tiles of 64 outputs by 16, 32 or 64 tokens, stages of 128 elements in a ring of four; straight from
+# memory: up to 16 tokens of one stage
+@pytest.mark.parametrize("n,H,K,M,tail", [(1, 2, 160, 16, 0), (16, 3, 128, 80, 8), (16, 65, 128, 272, 0), (17, 3, 544, 48, 0),
+                                          (33, 64, 128, 144, 64), (65, 8, 1056, 64, 0), (129, 130, 96, 112, 8),
+                                          (64, 256, 32, 16, 24), (200, 72, 640, 128, 0)])
+def test_headwise_by_tokens_and_contraction(dev, n, H, K, M, tail):
+    from zipage_amd.layers.latent import headwise_linear
+    x, w = _rand(n, H, K + tail, seed=6), _rand(H, M, K, seed=7)
+    x[n - 1, H - 1, :K] = float("inf")                   # a row of its own: nothing else may see it
+    got = headwise_linear(x.to(dev), w.to(dev)).cpu().double()
+    assert torch.equal(got[..., M:], x[..., K:].double())
+    live = torch.ones(n, H, dtype=torch.bool)
+    live[n - 1, H - 1] = False
+    a, b = x[..., :K].double().transpose(0, 1), w.double().transpose(1, 2)
+    a[H - 1, n - 1] = 0
+    want, absolute = (a @ b).transpose(0, 1), (a.abs() @ b.abs()).transpose(0, 1)
+    # fp32 sums of K products, then bf16
+    allowed = K * 2.0 ** -24 * absolute + 2.0 ** -8 * want.abs() + 1e-30
+    assert ((got[..., :M] - want).abs() <= allowed)[live].all()
+    assert not got[n - 1, H - 1, :M].isfinite().any()

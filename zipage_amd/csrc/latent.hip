@@ -157,6 +157,122 @@ struct HeadArgs {
   int n, H, K, M, tail, half;   // behind each head's part `tail` elements, of which 2 * half turn
 };
 
+// What lies behind head h's part in `tokens` tokens from n0 on: share `part` of `parts`, one of a workgroup (one workgroup
+// for all, and the others of its head waited for it: 256 tokens, 32 heads of 128 -> 512 with 64 behind them 19.2 us, 15.1).
+template <typename T>
+__device__ __forceinline__ void head_tails(const HeadArgs& a, int h, int n0, int tokens, int part, int parts) {
+  const int rest = a.tail - a.half;               // items of a token: the pairs, then what follows them
+  for (int it = part * 256 + threadIdx.x; it < tokens * rest; it += parts * 256) {
+    const int tok = it / rest, i = it - tok * rest, n = n0 + tok;
+    if (n >= a.n) break;
+    const int64_t from = ((int64_t)n * a.H + h) * (a.K + a.tail) + a.K, to = ((int64_t)n * a.H + h) * (a.M + a.tail) + a.M;
+    if (i < a.half) {
+      const float2 r = rotary_turn(a.positions[n], a.freqs[i]);
+      const float u = Elem<T>::ld(a.in, from + i), v = Elem<T>::ld(a.in, from + i + a.half);
+      Elem<T>::st(a.out, to + i, u * r.x - v * r.y);
+      Elem<T>::st(a.out, to + i + a.half, v * r.x + u * r.y);
+    } else {
+      Elem<T>::st(a.out, to + i + a.half, Elem<T>::ld(a.in, from + i + a.half));
+    }
+  }
+}
+
+// bf16.  Workgroup: 64 outputs of one head for 16 * TT tokens; a wave has MT tiles of 16 outputs for NT of 16 tokens.
+//
+// Operands pass through LDS: read from memory as they are multiplied, a load touches 16 rows for 64 bytes each and keeps
+// the L1 for some 70 cycles; whole rows are a quarter of that (256 tokens, 32 heads, 128 -> 512 with 64 behind: 15.1 us, now
+// 8.8; 512 -> 128: 13.4, now 7.2; 2048 tokens, 16 heads 45 and 39, now 25 and 23).  Stages hold 128 elements of a row, and
+// all of them are on their way at once where K is at most 512.  A row's sixteen 16-byte pieces lie in the order of
+// (piece ^ row), so that no two rows of an operand meet in a bank.  W is the row operand; the rows of two tiles alternate
+// by fours, so that a lane ends with eight consecutive outputs of a token.  Workgroups of a head follow one another on one
+// XCD, whose L2 holds its W and its tokens.
+constexpr int kHeadStage = 128, kHeadRing = 4;
+template <int TT> struct HeadTile {
+  static constexpr int MT = TT > 1 ? 2 : 1, NT = TT > 1 ? TT / 2 : 1;
+  static constexpr int kBytes = (64 + 16 * TT) * kHeadStage * 2, kLoads = 4 + TT;     // of a stage; of a wave for one
+};
+template <int kLeft> __device__ __forceinline__ void wait_loads_left() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x0f70 | (kLeft & 15) | (kLeft >> 4) << 14);
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+template <int TT>
+__global__ __launch_bounds__(256) void headwise_tile_kernel(HeadArgs a, int blocks_m, int blocks_n) {
+  extern __shared__ __align__(16) char lds_raw[];
+  typedef HeadTile<TT> Tile;
+  constexpr int MT = Tile::MT, NT = Tile::NT;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int total = gridDim.x;
+  int id = total % 8 == 0 ? (int)(blockIdx.x % 8) * (total / 8) + blockIdx.x / 8 : blockIdx.x;
+  const int bm = id % blocks_m;
+  id /= blocks_m;
+  const int n0 = id % blocks_n * 16 * TT, h = id / blocks_n;
+  const int x_row = a.H * (a.K + a.tail) * 2;                    // bytes from token to token
+  const u32x4 wr = rows_from((const uint16_t*)a.w + ((int64_t)h * a.M + bm * 64) * a.K, (uint32_t)min(64, a.M - bm * 64) * a.K * 2);
+  const u32x4 xr = rows_from((const uint16_t*)a.in + ((int64_t)n0 * a.H + h) * (a.K + a.tail),
+                             (uint32_t)(min(16 * TT, a.n - n0) - 1) * x_row + a.K * 2);
+  const int steps = a.K / 32, stages = (a.K + kHeadStage - 1) / kHeadStage, ring = min(stages, kHeadRing);
+  // loads of a stage: four rows each, first of W, then of the tokens; what is not there has an address past the end
+  auto issue = [&](int s) {
+    char* const to = lds_raw + s % kHeadRing * Tile::kBytes;
+#pragma unroll
+    for (int i = 0; i < Tile::kLoads; ++i) {
+      const int at = wave * Tile::kLoads + i, row = at * 4 + g;
+      const int c = s * 256 + (l16 ^ (row & 15)) * 16;           // byte of the row
+      const bool of_w = at < 16;                                 // uniform
+      int r = of_w ? row : row - 64;
+      if (of_w && MT == 2) r = (r & 32) + ((r & 12) << 1) + ((r & 16) >> 2) + (r & 3);
+      const bool there = c < a.K * 2 && (of_w ? bm * 64 + r < a.M : n0 + r < a.n);
+      if (of_w) load_to_lds(wr, to + at * 1024, there ? r * a.K * 2 + c : INT_MIN, 0);
+      else load_to_lds(xr, to + at * 1024, there ? r * x_row + c : INT_MIN, 0);
+    }
+  };
+  for (int s = 0; s < ring; ++s) issue(s);
+  if (a.tail) head_tails<BF16>(a, h, n0, 16 * TT, bm, blocks_m);
+  const int m_row = (MT == 2 ? (wave & 1) * 32 : wave * 16) + l16, x_first = (TT == 1 ? 0 : (wave >> 1) * 16 * NT) + l16;
+  f32x4 acc[MT][NT] = {};
+  for (int s = 0; s < stages; ++s) {
+    const int behind = min(stages - 1 - s, kHeadRing - 1);       // stages on their way behind this one
+    if (behind == 0) wait_loads_left<0>();
+    else if (behind == 1) wait_loads_left<Tile::kLoads>();
+    else if (behind == 2) wait_loads_left<2 * Tile::kLoads>();
+    else wait_loads_left<3 * Tile::kLoads>();
+    const char* const at = lds_raw + s % kHeadRing * Tile::kBytes;
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) {
+      if (s * 4 + ks >= steps) break;
+      const int piece = ((ks * 4 + g) ^ l16) * 16;
+      u32x4 wf[MT], xf[NT];
+#pragma unroll
+      for (int j = 0; j < MT; ++j) wf[j] = *(const u32x4*)(at + (m_row + j * 16) * 256 + piece);
+#pragma unroll
+      for (int t = 0; t < NT; ++t) xf[t] = *(const u32x4*)(at + (64 + x_first + t * 16) * 256 + piece);
+#pragma unroll
+      for (int j = 0; j < MT; ++j)
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[j][t] = mfma_bf16(wf[j], xf[t], acc[j][t]);
+    }
+    if (s + kHeadRing < stages) {
+      __builtin_amdgcn_s_waitcnt(0xc07f);                        // this stage has been read
+      wait_loads_left<63>();
+      issue(s + kHeadRing);
+    }
+  }
+  const int m = bm * 64 + (MT == 2 ? (wave & 1) * 32 + g * 8 : wave * 16 + g * 4);
+  if (m >= a.M) return;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) {
+    const int n = n0 + x_first + t * 16;
+    if (n >= a.n) continue;
+    uint16_t* const out = (uint16_t*)a.out + ((int64_t)n * a.H + h) * (a.M + a.tail) + m;
+    const f32x4 u = acc[0][t], v = acc[MT - 1][t];
+    if constexpr (MT == 2) *(u32x4*)out = u32x4{pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3]), pack_bf16(v[0], v[1]), pack_bf16(v[2], v[3])};
+    else *(uint2*)out = uint2{pack_bf16(u[0], u[1]), pack_bf16(u[2], u[3])};
+  }
+}
+
 // A wave owns 16 outputs of one head for 16 * kTokTiles tokens: W is the row operand, so a lane ends
 // with four consecutive outputs of one token.  Token rows past the end repeat the last one.
 template <typename T, int kTokTiles>
@@ -165,22 +281,7 @@ __global__ __launch_bounds__(256) void headwise_kernel(HeadArgs a) {
   const int m0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * 16;
   const int h = blockIdx.y;
   const int n0 = blockIdx.z * 16 * kTokTiles;
-  if (a.tail && blockIdx.x == 0) {
-    const int rest = a.tail - a.half;             // items of a token: the pairs, then what follows them
-    for (int it = threadIdx.x; it < 16 * kTokTiles * rest; it += 256) {
-      const int tok = it / rest, i = it - tok * rest, n = n0 + tok;
-      if (n >= a.n) break;
-      const int64_t from = ((int64_t)n * a.H + h) * (a.K + a.tail) + a.K, to = ((int64_t)n * a.H + h) * (a.M + a.tail) + a.M;
-      if (i < a.half) {
-        const float2 r = rotary_turn(a.positions[n], a.freqs[i]);
-        const float u = Elem<T>::ld(a.in, from + i), v = Elem<T>::ld(a.in, from + i + a.half);
-        Elem<T>::st(a.out, to + i, u * r.x - v * r.y);
-        Elem<T>::st(a.out, to + i + a.half, v * r.x + u * r.y);
-      } else {
-        Elem<T>::st(a.out, to + i + a.half, Elem<T>::ld(a.in, from + i + a.half));
-      }
-    }
-  }
+  if (a.tail) head_tails<T>(a, h, n0, 16 * kTokTiles, blockIdx.x, gridDim.x);
   if (m0 >= a.M) return;
   f32x4 acc[kTokTiles];
 #pragma unroll
@@ -879,6 +980,19 @@ int rows_splits(int n, int H, int R, int window, int NB, int BS) {
   return s < 1 ? 1 : s;
 }
 
+template <int TT> int launch_headwise(const HeadArgs& a, hipStream_t st) {
+  const int bm = (a.M + 63) / 64, bn = (a.n + 16 * TT - 1) / (16 * TT), stages = (a.K + kHeadStage - 1) / kHeadStage;
+  const int smem = (stages < kHeadRing ? stages : kHeadRing) * HeadTile<TT>::kBytes;
+  if (smem > 64 * 1024 &&
+      hipFuncSetAttribute((const void*)headwise_tile_kernel<TT>, hipFuncAttributeMaxDynamicSharedMemorySize, smem) !=
+          hipSuccess) {
+    zp_set_error("headwise_linear: cannot reserve %d bytes of LDS", smem);
+    return ZP_EHIP;
+  }
+  hipLaunchKernelGGL((headwise_tile_kernel<TT>), dim3((unsigned)bm * bn * a.H), dim3(256), smem, st, a, bm, bn);
+  ZP_LAUNCH_CHECK();
+  return ZP_OK;
+}
 int launch_combine(const RowsArgs& a, hipStream_t st) {
   if (a.splits > 1) {
     hipLaunchKernelGGL(latent_rows_combine_kernel, dim3((unsigned)a.n * a.H), dim3(64), 0, st, a);
@@ -999,13 +1113,21 @@ extern "C" int zp_headwise_linear(const void* in, const void* w, void* out, cons
   ZP_REQUIRE(in && w && out && aligned16(in) && aligned16(w) && aligned16(out),
              "headwise_linear: null or unaligned pointer");
   HeadArgs a = {in, w, out, positions, freqs, n, H, K, M, tail, rot / 2};
-  // as many tokens per wave (W is read once for them) as still leave two workgroups per CU
+  // The staged kernel, except for one stage of one token tile that has its CU to itself and nothing to pass the time with
+  // (1 token, 32 heads of 128 -> 512: 4.1 us, 3.6 without; 16 tokens 4.3 both; 8 tokens, 128 heads 7.1, 9.1 without), and
+  // what its 32-bit offsets don't span.
   const int64_t columns = (int64_t)((M + 63) / 64) * H;
-  int tt = 4;
-  while (tt > 1 && columns * ((n + 16 * tt - 1) / (16 * tt)) < 512) tt >>= 1;
+  const bool staged = dtype == ZP_BF16 && !(n <= 16 && K <= kHeadStage && columns <= 256) &&
+                      (int64_t)M * K * 2 < 1ll << 31 && (int64_t)64 * H * (K + tail) * 2 < 1ll << 31;
+  // as many tokens per wave (W is read once for them) as still leave two workgroups per CU; of the staged kernel as many as
+  // leave one (64 tokens, 32 heads of 512 -> 128: 6.9 us with 64 workgroups, 5.5 with 256), and no more than there are
+  int tt = staged && n <= 32 ? (n <= 16 ? 1 : 2) : 4;
+  while (tt > 1 && columns * ((n + 16 * tt - 1) / (16 * tt)) < (staged ? 256 : 512)) tt >>= 1;
   const dim3 grid((M + 63) / 64, H, (n + 16 * tt - 1) / (16 * tt));
   ZP_REQUIRE(grid.z <= 65535, "headwise_linear: too many tokens");
   hipStream_t st = (hipStream_t)stream;
+  if (staged && columns * grid.z < 1ll << 31)
+    return tt == 4 ? launch_headwise<4>(a, st) : (tt == 2 ? launch_headwise<2>(a, st) : launch_headwise<1>(a, st));
 #define ZP_HEADWISE(T)                                                                            \
   do {                                                                                            \
     if (tt == 4) hipLaunchKernelGGL((headwise_kernel<T, 4>), grid, dim3(256), 0, st, a);          \
