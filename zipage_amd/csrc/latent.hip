@@ -181,7 +181,7 @@ __device__ __forceinline__ void head_tails(const HeadArgs& a, int h, int n0, int
 //
 // Operands pass through LDS: read from memory as they are multiplied, a load touches 16 rows for 64 bytes each and keeps
 // the L1 for some 70 cycles; whole rows are a quarter of that (256 tokens, 32 heads, 128 -> 512 with 64 behind: 15.1 us, now
-// 8.8; 512 -> 128: 13.4, now 7.2; 2048 tokens, 16 heads 45 and 39, now 25 and 23).  Stages hold 128 elements of a row, and
+// 7.6; 512 -> 128: 13.4, now 6.1; 2048 tokens, 16 heads 45 and 39, now 22 and 18).  Stages hold 128 elements of a row, and
 // all of them are on their way at once where K is at most 512.  A row's sixteen 16-byte pieces lie in the order of
 // (piece ^ row), so that no two rows of an operand meet in a bank.  W is the row operand; the rows of two tiles alternate
 // by fours, so that a lane ends with eight consecutive outputs of a token.  Workgroups of a head follow one another on one
@@ -213,20 +213,25 @@ __global__ __launch_bounds__(256) void headwise_tile_kernel(HeadArgs a, int bloc
   const u32x4 wr = rows_from((const uint16_t*)a.w + ((int64_t)h * a.M + bm * 64) * a.K, (uint32_t)min(64, a.M - bm * 64) * a.K * 2);
   const u32x4 xr = rows_from((const uint16_t*)a.in + ((int64_t)n0 * a.H + h) * (a.K + a.tail),
                              (uint32_t)(min(16 * TT, a.n - n0) - 1) * x_row + a.K * 2);
-  const int steps = a.K / 32, stages = (a.K + kHeadStage - 1) / kHeadStage, ring = min(stages, kHeadRing);
+  const int stages = (a.K + kHeadStage - 1) / kHeadStage, ring = min(stages, kHeadRing);
   // loads of a stage: four rows each, first of W, then of the tokens; what is not there has an address past the end
+  int from[Tile::kLoads];
+#pragma unroll
+  for (int i = 0; i < Tile::kLoads; ++i) {
+    const int at = wave * Tile::kLoads + i, row = at * 4 + g;
+    int r = at < 16 ? row : row - 64;
+    if (at < 16 && MT == 2) r = (r & 32) + ((r & 12) << 1) + ((r & 16) >> 2) + (r & 3);
+    const bool there = at < 16 ? bm * 64 + r < a.M : n0 + r < a.n;
+    from[i] = (there ? r * (at < 16 ? a.K * 2 : x_row) : INT_MIN) + (l16 ^ (row & 15)) * 16;
+  }
   auto issue = [&](int s) {
-    char* const to = lds_raw + s % kHeadRing * Tile::kBytes;
+    char* const to = lds_raw + (s % kHeadRing * Tile::kBytes + wave * Tile::kLoads * 1024);
+    const bool whole = (s + 1) * kHeadStage <= a.K;
 #pragma unroll
     for (int i = 0; i < Tile::kLoads; ++i) {
-      const int at = wave * Tile::kLoads + i, row = at * 4 + g;
-      const int c = s * 256 + (l16 ^ (row & 15)) * 16;           // byte of the row
-      const bool of_w = at < 16;                                 // uniform
-      int r = of_w ? row : row - 64;
-      if (of_w && MT == 2) r = (r & 32) + ((r & 12) << 1) + ((r & 16) >> 2) + (r & 3);
-      const bool there = c < a.K * 2 && (of_w ? bm * 64 + r < a.M : n0 + r < a.n);
-      if (of_w) load_to_lds(wr, to + at * 1024, there ? r * a.K * 2 + c : INT_MIN, 0);
-      else load_to_lds(xr, to + at * 1024, there ? r * x_row + c : INT_MIN, 0);
+      int at = from[i] + s * 256;
+      if (!whole) at = s * 256 + (l16 ^ ((wave * Tile::kLoads + i) * 4 + g & 15)) * 16 < a.K * 2 ? at : INT_MIN;
+      load_to_lds(wave * Tile::kLoads + i < 16 ? wr : xr, to + i * 1024, at, 0);
     }
   };
   for (int s = 0; s < ring; ++s) issue(s);
@@ -240,20 +245,21 @@ __global__ __launch_bounds__(256) void headwise_tile_kernel(HeadArgs a, int bloc
     else if (behind == 2) wait_loads_left<2 * Tile::kLoads>();
     else wait_loads_left<3 * Tile::kLoads>();
     const char* const at = lds_raw + s % kHeadRing * Tile::kBytes;
+    u32x4 wf[4][MT], xf[4][NT];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) {
-      if (s * 4 + ks >= steps) break;
       const int piece = ((ks * 4 + g) ^ l16) * 16;
-      u32x4 wf[MT], xf[NT];
 #pragma unroll
-      for (int j = 0; j < MT; ++j) wf[j] = *(const u32x4*)(at + (m_row + j * 16) * 256 + piece);
+      for (int j = 0; j < MT; ++j) wf[ks][j] = *(const u32x4*)(at + (m_row + j * 16) * 256 + piece);
 #pragma unroll
-      for (int t = 0; t < NT; ++t) xf[t] = *(const u32x4*)(at + (64 + x_first + t * 16) * 256 + piece);
+      for (int t = 0; t < NT; ++t) xf[ks][t] = *(const u32x4*)(at + (64 + x_first + t * 16) * 256 + piece);
+    }
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks)                               // what lies behind the contraction's end is zero
 #pragma unroll
       for (int j = 0; j < MT; ++j)
 #pragma unroll
-        for (int t = 0; t < NT; ++t) acc[j][t] = mfma_bf16(wf[j], xf[t], acc[j][t]);
-    }
+        for (int t = 0; t < NT; ++t) acc[j][t] = mfma_bf16(wf[ks][j], xf[ks][t], acc[j][t]);
     if (s + kHeadRing < stages) {
       __builtin_amdgcn_s_waitcnt(0xc07f);                        // this stage has been read
       wait_loads_left<63>();
@@ -1114,7 +1120,7 @@ extern "C" int zp_headwise_linear(const void* in, const void* w, void* out, cons
              "headwise_linear: null or unaligned pointer");
   HeadArgs a = {in, w, out, positions, freqs, n, H, K, M, tail, rot / 2};
   // The staged kernel, except for one stage of one token tile that has its CU to itself and nothing to pass the time with
-  // (1 token, 32 heads of 128 -> 512: 4.1 us, 3.6 without; 16 tokens 4.3 both; 8 tokens, 128 heads 7.1, 9.1 without), and
+  // (1 token, 32 heads of 128 -> 512: 4.1 us, 3.6 without; 16 tokens 4.3 both; 8 tokens, 128 heads 6.6, 9.1 without), and
   // what its 32-bit offsets don't span.
   const int64_t columns = (int64_t)((M + 63) / 64) * H;
   const bool staged = dtype == ZP_BF16 && !(n <= 16 && K <= kHeadStage && columns <= 256) &&
