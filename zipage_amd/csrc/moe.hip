@@ -409,17 +409,18 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
 // 64 rows of W and all tokens.  W is kept in the order in which the matrix cores read it, so a wave's share goes from
 // memory straight into its registers; only tokens, which all four waves read, pass through LDS, by loads of their own;
 // one barrier per stage.  (With W through LDS too, reads and writes of LDS took longer than the products.)
-//   128 tokens: two workgroups per CU hide each other's set-up and results.  Stages are asked for two (W) and three
+//   128 tokens: two workgroups per CU hide each other's set-up and results.  Stages are asked for two (W) and four to five
 //   (tokens) ahead.
-//   256 tokens: half the reads of W per product, one wave per SIMD, four and five stages ahead.  From averages of more
-//   than 512 rows per expert on, and only over long contractions, since nothing hides a workgroup's beginning and end.
-// 16 384 tokens over 33 experts of 3 x 4096 x 3072 (both products, 4.95 TFLOP): 5.66 ms with everything through LDS,
-// 5.36 with 128 tokens, 5.09 with 256; of 3 x 1024 x 768: 488, 473 and 526 us.  6 144 tokens of 4 of 32 large ones:
-// 2.29 ms with 128, 2.21 with 256.  What is left is the stream of W, which comes from memory once per XCD and 2 048
-// tokens: with every stage's W from the same addresses (wrong results) the large case took 0.9 ms less.
+//   256 tokens: half the reads of W per product, one wave per SIMD, four and six to seven stages ahead.  From averages of
+//   more than 512 rows per expert on, and only over long contractions, since nothing hides a workgroup's beginning and end.
+// The L1 takes four to five cycles for every line that a load touches, whole or in part, and a stage's loads as long as its
+// products if each touches whole lines: so tokens come for two stages at a time, 128 bytes of a row (64 for one stage were
+// half as much again in lines).  16 384 tokens over 33 experts of 3 x 4096 x 3072 (both products, 4.95 TFLOP; the layer):
+// 5.66 ms with everything through LDS, 5.24 with 256 tokens and half lines, now 4.40 (128 tokens: 4.64); of
+// 3 x 2048 x 1536: 1.51 at first, 1.27 with 128 tokens, 1.31 with 256; of 3 x 1024 x 768: 488, 429 and 509 us.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 constexpr int kBlockW = 16, kWaveW = kBlockW / 4;      // 16-row tiles of W
-constexpr int kBigRows = 256, kBigContraction = 2048;
+constexpr int kBigRows = 256, kBigContraction = 2560;
 
 __device__ __forceinline__ void load_to_lds(__amdgpu_buffer_rsrc_t r, char* to, int lane_at, int at) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr_t)to, 16, lane_at, at, 0, 0);
@@ -445,8 +446,8 @@ __device__ __forceinline__ void settled(f32x4& acc) {
 // HALVES of HT 16-token tiles
 template <bool UP, int HALVES, int HT>
 __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(ExpertArgs a) {
-  constexpr int kTiles = HT * HALVES, kOwn = kTiles / 4, kStageBytes = kTiles * 1024, kGroup = 8;
-  constexpr int kLeadW = HALVES == 2 ? 4 : 2, kLeadX = HALVES == 2 ? 5 : 3, kStages = kLeadX + 1;      // stages ahead
+  constexpr int kTiles = HT * HALVES, kOwn = kTiles / 4, kPairBytes = kTiles * 2048, kGroup = 8;
+  constexpr int kLeadW = HALVES == 2 ? 4 : 2, kLeadX = HALVES == 2 ? 3 : 2, kPairs = kLeadX + 1;      // stages, pairs ahead
   extern __shared__ __align__(16) char lds_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
   // An XCD takes a contiguous share of the (tile, column block) pairs, eight tiles at a time, column block by column
@@ -474,11 +475,12 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   // gate_up gathers tokens from all of x, down reads consecutive rows
   const char* const xbase = (const char*)a.x + (UP ? 0 : t.y * a.x_st * 2);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc((void*)xbase, 0, (int)((UP ? a.n : t.z) * a.x_st * 2), 0x00020000);
-  int xoff[kOwn], woff[kWaveW];                          // this wave's loads of a stage
+  int xoff[2 * kOwn], woff[kWaveW];                      // this wave's loads of a pair of stages; of a stage
+  // a row's eight pieces of a pair lie in the order of (piece ^ row): rows of an operand don't meet in a bank
 #pragma unroll
-  for (int i = 0; i < kOwn; ++i) {
-    const int r = min((wave * kOwn + i) * 16 + l16, t.z - 1);
-    xoff[i] = (int)((UP ? a.sorted[t.y + r] / a.slots : r) * a.x_st * 2) + g * 16;
+  for (int i = 0; i < 2 * kOwn; ++i) {
+    const int r = min(wave * kOwn * 16 + i * 8 + (lane >> 3), t.z - 1);
+    xoff[i] = (int)((UP ? a.sorted[t.y + r] / a.slots : r) * a.x_st * 2) + ((lane & 7) ^ (lane >> 3)) * 16;
   }
 #pragma unroll
   for (int i = 0; i < kWaveW; ++i) woff[i] = min(wave * kWaveW + i, wtiles - w0 - 1) * steps * 1024;
@@ -495,12 +497,14 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
     }
   }
   // Past the end the last stage is asked for again, so that the number of loads in flight is always the same.
-  auto token_tile = [&](int ks, int i) {
-    load_to_lds(rx, lds_raw + (ks % kStages) * kStageBytes + (wave * kOwn + i) * 1024, xoff[i], min(ks, steps - 1) * 64);
+  const int pairs = (steps + 1) / 2, second = ((lane & 7) ^ (lane >> 3)) & 4 ? 64 : 0;
+  auto token_rows = [&](int pair, int i) {
+    const int back = (steps & 1) && pair >= pairs - 1 ? second : 0;      // a last stage alone: nothing behind the row's end
+    load_to_lds(rx, lds_raw + (pair % kPairs) * kPairBytes + (wave * 2 * kOwn + i) * 1024, xoff[i] - back, min(pair, pairs - 1) * 128);
   };
-  auto tokens = [&](int ks) {
+  auto tokens = [&](int pair, int half) {
 #pragma unroll
-    for (int i = 0; i < kOwn; ++i) token_tile(ks, i);
+    for (int i = 0; i < kOwn; ++i) token_rows(pair, half * kOwn + i);
     __builtin_amdgcn_sched_barrier(0);
   };
   auto weights = [&](int i, int ks) { return load_16(rw, lane * 16, woff[i] + min(ks, steps - 1) * 1024); };
@@ -513,13 +517,13 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
       for (int j = 0; j < HT; ++j) acc[h][i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   u32x4 wr[kLeadW][kWaveW], xf[HALVES][HT];
   auto fill = [&](int ks, u32x4 (&w)[kWaveW]) {
-    tokens(ks);
 #pragma unroll
     for (int i = 0; i < kWaveW; ++i) w[i] = weights(i, ks);
     __builtin_amdgcn_sched_barrier(0);
   };
+  const int lane_at = l16 * 128 + (g ^ (l16 & 7)) * 16;
   auto read_tile = [&](int ks, int h, int j) {
-    xf[h][j] = *(const u32x4*)(lds_raw + (ks % kStages) * kStageBytes + (h * HT + j) * 1024 + lane * 16);
+    xf[h][j] = *(const u32x4*)(lds_raw + (ks / 2 % kPairs) * kPairBytes + (h * HT + j) * 2048 + (lane_at ^ (ks & 1) * 64));
   };
   auto read = [&](int ks, int h) {
 #pragma unroll
@@ -527,22 +531,33 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
     __builtin_amdgcn_sched_barrier(0);
   };
   static_assert(HALVES == 1 || (kOwn == 4 && HT == 2 * kWaveW), "the waits count a wave's loads");
-  // the next tokens to be read are in LDS when all but the loads asked for after them have landed: three stages' (one
-  // stage's, of fewer tokens)
-  auto landed = [&]() {
-    if constexpr (HALVES == 2) asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
-    else asm volatile("s_waitcnt vmcnt(6)" ::: "memory");
+  // A pair of stages is in LDS when all but the loads asked for after it have landed.  256 tokens: the pair behind an odd
+  // stage is first read in it, three stages' loads behind; 128: in its own first stage, two stages' and a half.
+  auto landed = [&](int odd) {
+    if constexpr (HALVES == 2) { if (odd) asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); }
+    else if (!odd) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
+    asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();                        // everyone's
   };
 #pragma unroll
-  for (int s = 0; s < kLeadW; ++s) fill(s, wr[s]);
-  tokens(kLeadW);
+  for (int s = 0; s < kLeadX; ++s) {
+    tokens(s, 0);
+    tokens(s, 1);
+    if constexpr (HALVES == 2) {
+      if (2 * s < kLeadW) { fill(2 * s, wr[2 * s]); fill(2 * s + 1, wr[2 * s + 1]); }
+    } else {
+      fill(s, wr[s]);
+    }
+  }
   if constexpr (HALVES == 2) {
-    asm volatile("s_waitcnt vmcnt(24)" ::: "memory");
+    asm volatile("s_waitcnt vmcnt(32)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     read(0, 0);
+  } else {
+    asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   }
-  auto stage = [&](int ks, u32x4 (&w)[kWaveW]) {
+  auto stage = [&](int ks, int odd, u32x4 (&w)[kWaveW]) {      // odd: ks % 2
+    const int next = ks / 2 + kLeadX;                    // its tokens come over the pair before this one
     if constexpr (HALVES == 2) {
       // One wave per SIMD: whatever it issues between two products is time without products.  So reads and requests
       // are spread over the products, a half ahead of their use.
@@ -555,13 +570,13 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
           if (j == HT - 1) read_tile(ks, 1, 2 * i + 1);
           if (j == HT / 2 - 1 || j == HT - 1) __builtin_amdgcn_sched_barrier(0);
         }
-      landed();
+      landed(odd);
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
           mfma_in_place(acc[1][i][j], w[i], xf[1][j]);
-          if (j == 1) token_tile(ks + kLeadX, i);             // over the stage before this one
+          if (j == 1) token_rows(next, odd * kOwn + i);
           if (j == 3) read_tile(ks + 1, 0, 2 * i);
           if (j == 5) read_tile(ks + 1, 0, 2 * i + 1);
           if (j & 1) __builtin_amdgcn_sched_barrier(0);
@@ -570,8 +585,8 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      landed();
-      tokens(ks + kLeadX);                               // over the stage before this one
+      landed(odd);
+      tokens(next, odd);
       read(ks, 0);
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
@@ -586,11 +601,11 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
 #pragma unroll 1
   for (; ks + kLeadW <= steps; ks += kLeadW) {
 #pragma unroll
-    for (int s = 0; s < kLeadW; ++s) stage(ks + s, wr[s]);
+    for (int s = 0; s < kLeadW; ++s) stage(ks + s, s & 1, wr[s]);
   }
 #pragma unroll
   for (int s = 0; s + 1 < kLeadW; ++s)
-    if (ks + s < steps) stage(ks + s, wr[s]);
+    if (ks + s < steps) stage(ks + s, s & 1, wr[s]);
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // loads into LDS end before the workgroup does
   if constexpr (HALVES == 2) {                           // the last products' results are in their registers
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
@@ -642,7 +657,7 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
     b.split = big ? 1 : rows / 128;
     const int64_t grid = (int64_t)((b.max_tiles * b.split + 7) / 8) * 8 * ((Mx + 16 * kBlockW - 1) / (16 * kBlockW));
     const void* const fn = big ? (const void*)expert_tiles_kernel<UP, 2, 8> : (const void*)expert_tiles_kernel<UP, 1, 8>;
-    const int smem = big ? 6 * 16 * 1024 : 4 * 8 * 1024;
+    const int smem = big ? 4 * 32 * 1024 : 3 * 16 * 1024;
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
       zp_set_error("moe: cannot reserve %d bytes of LDS", smem);
       return ZP_EHIP;
