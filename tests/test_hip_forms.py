@@ -323,3 +323,15 @@ def test_headwise_by_tokens_and_contraction(dev, n, H, K, M, tail):
     allowed = K * 2.0 ** -24 * absolute + 2.0 ** -8 * want.abs() + 1e-30
     assert ((got[..., :M] - want).abs() <= allowed)[live].all()
     assert not got[n - 1, H - 1, :M].isfinite().any()
+
+
+# ------------------------------------------------------------------ few outputs
+# from 4 081 rows and 17 outputs on through LDS: 32 tokens by 32 or 64 outputs, stages of 128 elements
+@pytest.mark.parametrize("n,K,M", [(4080, 160, 20), (4081, 32, 20), (4099, 160, 32), (4095, 1056, 36), (4100, 96, 100),
+                                   (5000, 640, 64), (4113, 4128, 132)])
+def test_small_linear_of_many_rows(dev, n, K, M):
+    from zipage_amd.layers import small_linear
+    x, w = _rand(n, K + 8, seed=8)[:, :K], _rand(M, K, seed=9)
+    got = small_linear(x.to(dev)[:, :K], w.to(dev)).cpu().double()
+    want, absolute = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    assert ((got - want).abs() <= K * 2.0 ** -24 * absolute + 1e-30).all()

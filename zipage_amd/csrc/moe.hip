@@ -90,6 +90,87 @@ __global__ __launch_bounds__(64 * NW) void small_linear_kernel(SmallArgs a) {
   }
 }
 
+// Many rows, bf16: 16 * TT tokens x 16 * MT outputs, operands through LDS.  A row read as it is multiplied gives 64 bytes of
+// a line to a load, and the L1 takes four to five cycles for every line touched (16 384 tokens, 32 outputs of 4096: 69 us,
+// now 31; 128 outputs 148, now 65).  A stage is 128 elements of every row, a step for each of the four waves: the same share of the contraction
+// that each has above, so that sums are the same to the last bit.  A row's sixteen pieces lie in the order of (piece ^ row).
+template <int TT, int MT> struct SmallTile {
+  static constexpr int kRing = MT > 2 ? 3 : 4, kBytes = (TT + MT) * 4096, kLoads = TT + MT;   // of a stage; of a wave
+};
+template <int TT, int MT>
+__global__ __launch_bounds__(256, 2) void small_tile_kernel(SmallArgs a) {
+  extern __shared__ __align__(16) char lds_raw[];
+  typedef SmallTile<TT, MT> Tile;
+  constexpr int L = Tile::kLoads, R = Tile::kRing;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = blockIdx.x * 16 * TT, m0 = blockIdx.y * 16 * MT, steps = a.K / 32, stages = (steps + 3) / 4;
+  const int x_row = (int)a.x_st * 2;                     // bytes
+  const u32x4 xr = rows_from((const uint16_t*)a.x + n0 * a.x_st, (uint32_t)(min(16 * TT, a.n - n0) - 1) * x_row + a.K * 2);
+  const u32x4 wr = rows_from((const uint16_t*)a.w + (int64_t)m0 * a.K, (uint32_t)min(16 * MT, a.M - m0) * a.K * 2);
+  int from[L];                                           // of four rows a load; what is not there lies past the end
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int at = wave * L + i, row = at * 4 + g, r = at < 4 * MT ? row : row - 16 * MT;
+    const bool there = at < 4 * MT ? m0 + r < a.M : n0 + r < a.n;
+    from[i] = (there ? r * (at < 4 * MT ? a.K * 2 : x_row) : INT_MIN) + (l16 ^ (row & 15)) * 16;
+  }
+  auto issue = [&](int s) {                              // past the last stage zeros come, so that the count stays
+    char* const to = lds_raw + (s % R * Tile::kBytes + wave * L * 1024);
+    const bool whole = s * 4 + 4 <= steps;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      int at = from[i] + s * 256;
+      if (!whole) at = s * 256 + (l16 ^ ((wave * L + i) * 4 + g & 15)) * 16 < a.K * 2 ? at : INT_MIN;
+      load_to_lds(wave * L + i < 4 * MT ? wr : xr, to + i * 1024, at, 0);
+    }
+  };
+#pragma unroll
+  for (int s = 0; s < R - 1; ++s) issue(s);
+  f32x4 acc[TT][MT] = {};
+  const int read_at = l16 * 256 + ((wave * 4 + g) ^ l16) * 16;
+#pragma unroll 1
+  for (int s = 0; s < stages; ++s) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070 | (R - 2) * L);    // this stage is there, and the one before has been read
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(s + R - 1);
+    if (s * 4 + wave >= steps) continue;
+    const char* const at = lds_raw + s % R * Tile::kBytes + read_at;
+    u32x4 wf[MT], xf[TT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) wf[j] = *(const u32x4*)(at + j * 4096);
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xf[t] = *(const u32x4*)(at + (MT + t) * 4096);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[t][j] = mfma_bf16(wf[j], xf[t], acc[t][j]);
+  }
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0);                         // no load is left on its way to LDS
+  __syncthreads();
+  f32x4* const red = (f32x4*)lds_raw;
+  if (wave > 0) {
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) red[((wave - 1) * TT * MT + t * MT + j) * 64 + lane] = acc[t][j];
+  }
+  __syncthreads();
+  if (wave > 0) return;
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) {
+#pragma unroll
+      for (int k = 0; k < 3; ++k) acc[t][j] += red[(k * TT * MT + t * MT + j) * 64 + lane];
+      const int n = n0 + t * 16 + l16, m = m0 + j * 16 + g * 4;
+      if (n < a.n && m < a.M) *(f32x4*)(a.out + (int64_t)n * a.M + m) = acc[t][j];
+    }
+}
+
 // ------------------------------------------------------------------ selection
 constexpr int kMaxExperts = 1024;
 
@@ -721,6 +802,19 @@ extern "C" int zp_small_linear(const void* x, const void* w, float* out, int32_t
   const unsigned gx = (unsigned)((n + 15) / 16);
   const bool wide = gx >= 256 && M > 16;
   const dim3 grid(gx, (unsigned)(wide ? (M + 63) / 64 : (M + 15) / 16));
+  if (wide && dtype == ZP_BF16 && 32 * x_stride * 2 < 1ll << 31 && (int64_t)64 * K * 2 < 1ll << 31) {
+    const dim3 tiles((unsigned)((n + 31) / 32), (unsigned)(M <= 32 ? 1 : (M + 63) / 64));
+    const int smem = M <= 32 ? SmallTile<2, 2>::kRing * SmallTile<2, 2>::kBytes : SmallTile<2, 4>::kRing * SmallTile<2, 4>::kBytes;
+    const void* const fn = M <= 32 ? (const void*)small_tile_kernel<2, 2> : (const void*)small_tile_kernel<2, 4>;
+    if (smem > 64 * 1024 && hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
+      zp_set_error("small_linear: cannot reserve %d bytes of LDS", smem);
+      return ZP_EHIP;
+    }
+    if (M <= 32) hipLaunchKernelGGL((small_tile_kernel<2, 2>), tiles, dim3(256), smem, st, a);
+    else hipLaunchKernelGGL((small_tile_kernel<2, 4>), tiles, dim3(256), smem, st, a);
+    ZP_LAUNCH_CHECK();
+    return ZP_OK;
+  }
 #define ZP_SMALL(T)                                                                              \
   do {                                                                                           \
     if (wide) hipLaunchKernelGGL((small_linear_kernel<T, 4, 4>), grid, dim3(256), 0, st, a);     \
