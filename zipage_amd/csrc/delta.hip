@@ -155,7 +155,7 @@ __global__ __launch_bounds__(64 * NW) void delta_scan_kernel(zp_delta a) {
 }
 
 // One token per segment (decoding): the state passes through once.
-template <typename T, int RL, int NW>
+template <typename T, int RL, int NW, bool PAST>
 __global__ __launch_bounds__(64 * NW) void delta_step_kernel(zp_delta a) {
   extern __shared__ __align__(16) float lds[];
   __shared__ float red[NW];
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64 * NW) void delta_step_kernel(zp_delta a) {
 #pragma unroll
   for (int r = 0; r < RL; ++r) {
     S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (!fresh) S[r] = load_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
+    if (!fresh) S[r] = load_state<PAST>(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
   }
   if (tid < cw) finish(tid, first);
   if (c2 < cw) finish(c2, second);
@@ -269,7 +269,7 @@ __global__ __launch_bounds__(64 * NW) void delta_step_kernel(zp_delta a) {
   for (int r = 0; r < RL; ++r) {
 #pragma unroll
     for (int c = 0; c < 4; ++c) S[r][c] = fmaf(k4[r >> 2][r & 3], u[c], S[r][c]);
-    store_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col, S[r]);
+    store_state<PAST>(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col, S[r]);
   }
   ss = quads_sum(ss);
   if (lane == 0) red[wave] = ss;
@@ -290,8 +290,11 @@ template <typename T, int RL> int launch_delta(const zp_delta& a, hipStream_t st
   const dim3 grid((unsigned)((int64_t)a.seg.n * a.heads)), block(a.dv * 2);
   if (a.seg.max_count == 1) {
     const size_t step = sizeof(float) * (3 * a.dk + a.dv);
-    if (a.dv <= 128) hipLaunchKernelGGL((delta_step_kernel<T, RL, 4>), grid, block, step, st, a);
-    else hipLaunchKernelGGL((delta_step_kernel<T, RL, 8>), grid, block, step, st, a);
+    const bool past = past_cache((int64_t)a.seg.n * a.heads, a.dk, a.dv);
+    if (a.dv <= 128 && past) hipLaunchKernelGGL((delta_step_kernel<T, RL, 4, true>), grid, block, step, st, a);
+    else if (a.dv <= 128) hipLaunchKernelGGL((delta_step_kernel<T, RL, 4, false>), grid, block, step, st, a);
+    else if (past) hipLaunchKernelGGL((delta_step_kernel<T, RL, 8, true>), grid, block, step, st, a);
+    else hipLaunchKernelGGL((delta_step_kernel<T, RL, 8, false>), grid, block, step, st, a);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }

@@ -84,7 +84,7 @@ __global__ __launch_bounds__(64 * NW) void linear_scan_kernel(zp_linear a) {
   for (int r = 0; r < RL; ++r) *(f32x4*)(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col) = S[r];
 }
 
-template <typename T, int RL, int NW>
+template <typename T, int RL, int NW, bool PAST>
 __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
   constexpr int dk = 8 * RL;
   __shared__ __align__(16) float qs[dk], ks[dk], gs[dk];
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
 #pragma unroll
   for (int r = 0; r < RL; ++r) {
     S[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (sg.start > 0) S[r] = load_once(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
+    if (sg.start > 0) S[r] = load_state<PAST>(state + (int64_t)(4 * (8 * (r >> 2) + rg) + (r & 3)) * dv + col);
   }
   for (int c = tid; c < dk; c += blockDim.x) {
     qs[c] = turned<T>(a, src + a.q_at + h * dk, c, half, sg.start) * a.q_scale;
@@ -128,7 +128,7 @@ __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
         s[c] = fmaf(k4[i], v[c], s[c] * g4[i]);
         o[c] = fmaf(s[c], q4[i], o[c]);
       }
-      store_once(state + (int64_t)(at + i) * dv + col, s);
+      store_state<PAST>(state + (int64_t)(at + i) * dv + col, s);
     }
   }
   float ss = 0.f;
@@ -154,8 +154,11 @@ __global__ __launch_bounds__(64 * NW) void linear_step_kernel(zp_linear a) {
 template <typename T, int RL> int launch_linear(const zp_linear& a, hipStream_t st) {
   const dim3 grid((unsigned)((int64_t)a.seg.n * a.heads)), block(a.dv * 2);
   if (a.seg.max_count == 1) {
-    if (a.dv <= 128) hipLaunchKernelGGL((linear_step_kernel<T, RL, 4>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((linear_step_kernel<T, RL, 8>), grid, block, 0, st, a);
+    const bool past = past_cache((int64_t)a.seg.n * a.heads, a.dk, a.dv);
+    if (a.dv <= 128 && past) hipLaunchKernelGGL((linear_step_kernel<T, RL, 4, true>), grid, block, 0, st, a);
+    else if (a.dv <= 128) hipLaunchKernelGGL((linear_step_kernel<T, RL, 4, false>), grid, block, 0, st, a);
+    else if (past) hipLaunchKernelGGL((linear_step_kernel<T, RL, 8, true>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((linear_step_kernel<T, RL, 8, false>), grid, block, 0, st, a);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }

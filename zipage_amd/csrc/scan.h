@@ -31,12 +31,20 @@ __device__ __forceinline__ Segment segment_of(const zp_segments& s, int i) {
 __device__ __forceinline__ int lane_cq() { return threadIdx.x & 7; }
 __device__ __forceinline__ int lane_rg() { return (threadIdx.x & 63) >> 3; }
 
-// A decoded token passes over the state once, and the next reads it after every other layer's: non-temporal both ways
-// (256 sequences, heads of 128 x 128: linear attention with 32 heads 226 -> 215 us, delta rule with 32 246 -> 203;
-// 128 sequences, retention with 16 heads 64 -> 50; non-temporal stores alone change nothing).  Not for the matrix
-// memory, whose states do not begin on a cache line: 133 -> 215 us, 190 with the loads alone.
-__device__ __forceinline__ f32x4 load_once(const float* p) { return __builtin_nontemporal_load((const f32x4*)p); }
-__device__ __forceinline__ void store_once(float* p, const f32x4& v) { __builtin_nontemporal_store(v, (f32x4*)p); }
+// A decoded token passes over the state once, and the next reads it after every other layer's.  A layer's states that the
+// last-level cache (256 MB) cannot hold until then go past it, non-temporal both ways (256 sequences, heads of 128 x 128:
+// linear attention with 32 heads 226 -> 215 us, delta rule with 32 244 -> 203; 180 sequences 154 -> 150 and 176 -> 147);
+// smaller ones may still be there (128 sequences, 32 heads: linear 94 us, 110 past it; 62, retention with 16: 22 and 23).
+// Not for the matrix memory, whose states do not begin on a cache line: 133 -> 215 us, 190 with the loads alone.
+inline bool past_cache(int64_t states, int dk, int dv) { return states * dk * dv * 4 >= 320ll << 20; }
+template <bool PAST> __device__ __forceinline__ f32x4 load_state(const float* p) {
+  if constexpr (PAST) return __builtin_nontemporal_load((const f32x4*)p);
+  return *(const f32x4*)p;
+}
+template <bool PAST> __device__ __forceinline__ void store_state(float* p, const f32x4& v) {
+  if constexpr (PAST) __builtin_nontemporal_store(v, (f32x4*)p);
+  else *(f32x4*)p = v;
+}
 
 // Sum over the eight row groups, in every lane.
 __device__ __forceinline__ float rows_sum(float v) {
