@@ -45,12 +45,14 @@ def test_compaction_of_few_rows(dev, dtype, L, B, Hkv, D, style):
 
 # ------------------------------------------------------------------ experts
 # rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup when
-# there are many; 256-row tiles are worked off whole from a contraction of 2048 on, in two halves below it.  Odd
+# there are many and tokens come to six per expert; 256-row tiles are worked off whole from a contraction of 2560 on, in
+# two halves below it.  Odd
 # numbers of steps, results that end inside a workgroup's columns, and experts without a token are among them.
 @pytest.mark.parametrize("n,width,E,top,ff", [(60, 96, 64, 2, 800), (61, 2080, 64, 2, 544), (1, 4096, 4, 2, 32),
                                               (260, 160, 4, 1, 288), (1100, 2144, 3, 2, 96), (1100, 96, 2, 1, 2112),
                                               (1300, 256, 2, 1, 96), (515, 2112, 1, 1, 48),
-                                              (1100, 2592, 3, 2, 96), (1100, 96, 2, 1, 2592), (515, 2624, 1, 1, 48)])
+                                              (1100, 2592, 3, 2, 96), (1100, 96, 2, 1, 2592), (515, 2624, 1, 1, 48),
+                                              (200, 96, 64, 2, 800), (225, 2080, 64, 2, 544)])
 @pytest.mark.parametrize("act", ["clamped", "silu"])
 def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act):
     from zipage_amd.layers import Experts

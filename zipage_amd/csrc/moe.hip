@@ -394,11 +394,13 @@ template <typename T> __device__ __forceinline__ float gated(int act, float w, f
 // the steps of the contraction and meet in LDS.  What the weights' stream loses is what else passes the caches: 16
 // rows of tokens per kRowsW tiles of W, and twice as much where two waves take the two halves of a token's cache line.
 // One token tile (hardly any expert has a second): a wave takes pairs of steps, whole lines of x, and the workgroup
-// 128 rows of W where that leaves two workgroups per CU (64 tokens over 33 experts of 3 x 4096 x 3072: 516 -> 476 us,
-// 5.2 TB/s; with 64 rows 497; a single token, 192 workgroups of 128 rows: 72 against 81).  More token tiles keep 64
-// rows and single steps (256 tokens: 675 us; 687 with pairs, 876 with 128 rows).
+// 128 rows of W where that leaves two workgroups per CU and tokens come to six per expert (64 tokens over 33 experts of
+// 3 x 4096 x 3072: 516 -> 476 us, 5.2 TB/s; with 64 rows 497; 48 tokens of 4 of 32: 405, 394, 400).  With fewer tokens
+// there is less of x to read again, and the last workgroups are half as long with 64 rows (9 tokens: 314, 317, 306; 24:
+// 385, 390, 385; widths of 2048: 95, 97, 94).  More token tiles keep 64 rows and single steps (256 tokens: 675 us; 687
+// with pairs, 876 with 128 rows).
 constexpr int kNarrowW = 4, kWideW = 8;                // 16-row tiles of W
-constexpr int kWideGrid = 512;                         // workgroups from which on 128 rows of W are better
+constexpr int kWideGrid = 512, kWideRows = 6;          // workgroups and average rows from which on 128 rows of W are better
 template <typename T, int MT, bool UP, int kRowsW>
 __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
@@ -750,7 +752,7 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
   const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
-  const bool wide = rows == 16 && dtype == ZP_BF16 && grid_of(kWideW) >= kWideGrid;
+  const bool wide = rows == 16 && dtype == ZP_BF16 && grid_of(kWideW) >= kWideGrid && (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
   const int64_t grid = grid_of(wide ? kWideW : kNarrowW);
   if (grid >= (1ll << 31)) {
     zp_set_error("moe: too many tiles");
