@@ -196,9 +196,11 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_kernel(QkArgs a) {
 
 // The same for heads of 128 in aligned rows: sixteen lanes a vector, eight elements a lane, so that every access is 16
 // bytes wide; the other half of a rotated pair is eight lanes on.  Bound by HBM: 8192 tokens of 32 + 16 heads move
-// 218 MB (2-byte accesses, a wave a vector: 110 us; now
-// 42).
+// 218 MB (2-byte accesses, a wave a vector: 110 us; now 42).
 constexpr int kVecHead = 128, kVecs = kThreads / 16;     // vectors of a workgroup at a time
+template <int kControl> __device__ __forceinline__ float dpp(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), kControl, 0xf, 0xf, false));
+}
 template <typename T>
 __global__ __launch_bounds__(kThreads) void qk_norm_rope_wide_kernel(QkArgs a) {
   const int n = blockIdx.x, j = threadIdx.x & 15, total = a.Hq + 2 * a.Hkv;
@@ -228,12 +230,21 @@ __global__ __launch_bounds__(kThreads) void qk_norm_rope_wide_kernel(QkArgs a) {
       continue;
     }
     const bool is_q = hv < a.Hq;
-    float x[8], other[8], ss = 0.f;
+    float x[8], other[8], sq[8];
     unpack8<T>(raw, x);
     unpack8<T>(*(const u32x4*)((const uint16_t*)(is_q ? a.qn_w : a.kn_w) + j * 8), w);
+    // squares meet in the order of the kernel above, lane k of which has elements k and k + 64, so that where rows lie
+    // doesn't change a bit: first those two, then those of k ^ 8 (the next lane's), 4, 2 and 1 (this lane's), 16 and 32
 #pragma unroll
-    for (int i = 0; i < 8; ++i) ss += x[i] * x[i];
-    const float rs = rsqrtf(row16_sum(ss) / (float)kVecHead + a.eps);
+    for (int i = 0; i < 8; ++i) {
+      sq[i] = x[i] * x[i];
+      sq[i] += dpp_row_ror<8>(sq[i]);
+      sq[i] += dpp<0xB1>(sq[i]);                               // [1,0,3,2]
+    }
+    float ss = ((sq[0] + sq[4]) + (sq[2] + sq[6])) + ((sq[1] + sq[5]) + (sq[3] + sq[7]));
+    ss += dpp<0x4E>(ss);                                       // [2,3,0,1]
+    ss += dpp<0x141>(ss);                                      // half mirror
+    const float rs = rsqrtf(ss / (float)kVecHead + a.eps);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
       x[i] = Elem<T>::rnd(Elem<T>::rnd(x[i] * rs) * w[i]);
