@@ -54,10 +54,10 @@ def test_compaction_of_few_rows(dev, dtype, L, B, Hkv, D, style):
                                               (1100, 2592, 3, 2, 96), (1100, 96, 2, 1, 2592), (515, 2624, 1, 1, 48),
                                               (200, 96, 64, 2, 800), (225, 2080, 64, 2, 544)])
 @pytest.mark.parametrize("act", ["clamped", "silu"])
-def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act):
+def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act, shared_ff=None):
     from zipage_amd.layers import Experts
     clamped = act == "clamped"
-    m = Experts(width, E, top, ff, 7.0, shared_ff=ff + 32 if clamped else None, shared_limit=5.0, act=act,
+    m = Experts(width, E, top, ff, 7.0, shared_ff=(shared_ff or ff + 32) if clamped else None, shared_limit=5.0, act=act,
                 score="softmax" if clamped else "sigmoid")
     w = {k: _rand(*s, seed=i, std=2.0 * s[-1] ** -0.5) for i, (k, s) in enumerate(m.shapes().items())}
     if E > 2:
@@ -80,6 +80,16 @@ def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act):
     # bf16 activations and planes: each of top + 2 roundings is at most 2^-9 of its own value
     err = (got - want)[sure].norm() / want[sure].norm()
     assert float(err) < 2.0 ** -8 and bool(torch.isfinite(got).all())
+
+
+# 256-row tiles whose contraction leaves 0 to 3 steps behind the loop, which takes four at a time, in either product; a
+# shared expert that has fewer steps than the loop takes
+@pytest.mark.parametrize("n,width,ff,shared_ff", [(530, 2560, 48, 0), (530, 2592, 48, 0), (530, 2624, 48, 0), (530, 2656, 48, 0),
+                                                  (530, 2688, 48, 0), (530, 96, 2656, 0), (700, 160, 2688, 32),
+                                                  (700, 160, 2656, 64), (700, 2656, 2592, 96), (530, 96, 2624, 128),
+                                                  (530, 96, 2560, 160), (530, 96, 2560, 224)])
+def test_experts_of_long_contractions(dev, n, width, ff, shared_ff):
+    test_experts_by_rows_and_contraction(dev, n, width, 1, 1, ff, "clamped" if shared_ff else "silu", shared_ff)
 
 
 # ------------------------------------------------------------------ attention of runs

@@ -16,6 +16,7 @@
 // wave's operand is then one contiguous KB.  W is the row operand: a lane ends with four consecutive
 // outputs of one token.
 #include "mfma.h"
+#include <type_traits>
 
 namespace {
 
@@ -579,7 +580,8 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
       wgt[j] = slot < a.top ? a.weights[(int64_t)n * a.top + slot] : 1.f;
     }
   }
-  // Past the end the last stage is asked for again, so that the number of loads in flight is always the same.
+  // Past the end the last stage is asked for again, so that the number of loads in flight is the same in every pass of the
+  // loop.  Stages behind it ask for nothing, and wait for all.
   const int pairs = (steps + 1) / 2, second = ((lane & 7) ^ (lane >> 3)) & 4 ? 64 : 0;
   auto token_rows = [&](int pair, int i) {
     const int back = (steps & 1) && pair >= pairs - 1 ? second : 0;      // a last stage alone: nothing behind the row's end
@@ -615,9 +617,13 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   };
   static_assert(HALVES == 1 || (kOwn == 4 && HT == 2 * kWaveW), "the waits count a wave's loads");
   // A pair of stages is in LDS when all but the loads asked for after it have landed.  256 tokens: the pair behind an odd
-  // stage is first read in it, three stages' loads behind; 128: in its own first stage, two stages' and a half.
-  auto landed = [&](int odd) {
-    if constexpr (HALVES == 2) { if (odd) asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); }
+  // stage is first read in it, three stages' loads behind; 128: in its own first stage, two stages' and a half.  Behind the
+  // loop there are fewer (weights that no stage would use are not loaded, whatever is written here).
+  typedef std::integral_constant<bool, true> yes;
+  typedef std::integral_constant<bool, false> no;
+  auto landed = [&](int odd, auto loop) {
+    if constexpr (!loop.value) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    else if constexpr (HALVES == 2) { if (odd) asm volatile("s_waitcnt vmcnt(24)" ::: "memory"); }
     else if (!odd) asm volatile("s_waitcnt vmcnt(16)" ::: "memory");
     asm volatile("" ::: "memory");
     __builtin_amdgcn_s_barrier();                        // everyone's
@@ -639,7 +645,8 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   } else {
     asm volatile("s_waitcnt vmcnt(12)" ::: "memory");
   }
-  auto stage = [&](int ks, int odd, u32x4 (&w)[kWaveW]) {      // odd: ks % 2
+  auto stage = [&](int ks, int odd, u32x4 (&w)[kWaveW], auto loop) {      // odd: ks % 2
+    constexpr bool kAsk = loop.value;
     const int next = ks / 2 + kLeadX;                    // its tokens come over the pair before this one
     if constexpr (HALVES == 2) {
       // One wave per SIMD: whatever it issues between two products is time without products.  So reads and requests
@@ -653,29 +660,29 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
           if (j == HT - 1) read_tile(ks, 1, 2 * i + 1);
           if (j == HT / 2 - 1 || j == HT - 1) __builtin_amdgcn_sched_barrier(0);
         }
-      landed(odd);
+      landed(odd, loop);
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
 #pragma unroll
         for (int j = 0; j < HT; ++j) {
           mfma_in_place(acc[1][i][j], w[i], xf[1][j]);
-          if (j == 1) token_rows(next, odd * kOwn + i);
+          if (kAsk && j == 1) token_rows(next, odd * kOwn + i);
           if (j == 3) read_tile(ks + 1, 0, 2 * i);
           if (j == 5) read_tile(ks + 1, 0, 2 * i + 1);
           if (j & 1) __builtin_amdgcn_sched_barrier(0);
         }
-        w[i] = weights(i, ks + kLeadW);
+        if (kAsk) w[i] = weights(i, ks + kLeadW);
         __builtin_amdgcn_sched_barrier(0);
       }
     } else {
-      landed(odd);
-      tokens(next, odd);
+      landed(odd, loop);
+      if (kAsk) tokens(next, odd);
       read(ks, 0);
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
 #pragma unroll
         for (int j = 0; j < HT; ++j) acc[0][i][j] = mfma_bf16(w[i], xf[0][j], acc[0][i][j]);
-        w[i] = weights(i, ks + kLeadW);
+        if (kAsk) w[i] = weights(i, ks + kLeadW);
         __builtin_amdgcn_sched_barrier(0);
       }
     }
@@ -684,11 +691,11 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
 #pragma unroll 1
   for (; ks + kLeadW <= steps; ks += kLeadW) {
 #pragma unroll
-    for (int s = 0; s < kLeadW; ++s) stage(ks + s, s & 1, wr[s]);
+    for (int s = 0; s < kLeadW; ++s) stage(ks + s, s & 1, wr[s], yes{});
   }
 #pragma unroll
   for (int s = 0; s + 1 < kLeadW; ++s)
-    if (ks + s < steps) stage(ks + s, s & 1, wr[s]);
+    if (ks + s < steps) stage(ks + s, s & 1, wr[s], no{});
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // loads into LDS end before the workgroup does
   if constexpr (HALVES == 2) {                           // the last products' results are in their registers
     asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");
