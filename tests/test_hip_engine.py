@@ -77,6 +77,33 @@ def test_cached_prefix_prefill_equals_dense(dev):
     assert (h.float() - dense[n0:]).abs().max() < 6e-2
 
 
+def test_prompts_with_and_without_a_cached_prefix_in_one_step(dev):
+    """A step of new prompts beside one that continues a cached prefix.  New prompts attend their own rows: they need
+    neither slots nor pages (-1 in both)."""
+    from zipage_amd.engine import Qwen3, StepContext
+    s = _tiny()
+    BS, pages = 16, 12
+    model = Qwen3(s, dev, seed=3, init_std=0.05)
+    kv = torch.zeros(2, s.layers, pages, BS, s.kv_heads, s.head_dim, device=dev, dtype=torch.bfloat16)
+    qc = torch.zeros(s.layers, 3, 4, s.heads, s.head_dim, device=dev, dtype=torch.bfloat16)
+    lens_q, lens_k, n0 = [37, 18, 130], [37, 50, 130], 32
+    prompts = [torch.randint(0, s.vocab, (n,), device=dev) for n in lens_k]
+    at = [torch.arange(n, device=dev) for n in lens_k]
+    dense = [model.forward(p, a, StepContext(True, None, None, None, None, [len(p)], [len(p)])).float() for p, a in zip(prompts, at)]
+    model.attach_caches(kv, qc)
+    table = torch.tensor([7, 2, 9, 4], dtype=torch.int32)
+    slots = (table.long()[:, None] * BS + torch.arange(BS)[None, :]).flatten().int().to(dev)
+    model.forward(prompts[1][:n0], at[1][:n0], StepContext(True, slots[:n0], None, None, None, [n0], [n0]))
+    none = lambda n: torch.full((n,), -1, dtype=torch.int32, device=dev)
+    tables = torch.full((3, 9), -1, dtype=torch.int32)
+    tables[1, :4] = table
+    first = [0, n0, 0]
+    h = model.forward(torch.cat([p[f:] for p, f in zip(prompts, first)]), torch.cat([a[f:] for a, f in zip(at, first)]),
+                      StepContext(True, torch.cat([none(37), slots[n0:50], none(130)]), None, None, tables.to(dev), lens_q, lens_k))
+    want = torch.cat([d[f:] for d, f in zip(dense, first)])
+    assert (h.float() - want).abs().max() < 6e-2
+
+
 def _generate(cfg, prompts, max_tokens):
     from zipage_amd.engine import SamplingParams, ZipageEngine
     eng = ZipageEngine(cfg)

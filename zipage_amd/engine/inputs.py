@@ -140,13 +140,16 @@ def plan_runs(portions: list[Portion], block_size: int, sight) -> Runs:
                 None if own else np.concatenate(slots).astype(np.int32))
 
 
-def plan_prompts(lens_q: list[int], lens_k: list[int]) -> np.ndarray:
-    """Query tiles of prompts whose query rows and whose key rows follow one another, a prompt's queries being its last
-    positions.  Tiles with many keys come first, so that the last workgroups to start are short ones."""
-    tiles, q, k = [], 0, 0
-    for nq, nk in zip(lens_q, lens_k):
+def plan_prompts(lens_q: list[int], lens_k: list[int], starts_k: list[int] | None = None) -> np.ndarray:
+    """Query tiles of prompts whose query rows follow one another, a prompt's queries being its last positions.  Its key
+    rows begin at its entry of `starts_k` (None: they follow one another, too).  Tiles with many keys come first, so that
+    the last workgroups to start are short ones."""
+    if starts_k is None:
+        starts_k = np.cumsum([0, *lens_k])
+    tiles, q = [], 0
+    for nq, nk, k in zip(lens_q, lens_k, starts_k):
         tiles += [(q + off, min(RUN_TILE, nq - off), k, nk - nq + off) for off in range(0, nq, RUN_TILE)]
-        q, k = q + nq, k + nk
+        q += nq
     tiles.sort(key=lambda t: -t[3])
     return np.asarray(tiles, dtype=np.int32).reshape(-1, 4)
 

@@ -121,25 +121,34 @@ class Qwen3:
 
     # ------------------------------------------------------------------ pieces
     def _plan_prefill(self, ctx: StepContext):
-        """Query tiles of a step of prompts, and the cache rows of its keys where prompts have a cached prefix; None where
-        the kernel does not cover the model."""
+        """Query tiles of a step of prompts, and the cache rows of the prompts with a cached prefix, whose whole contexts are
+        read back: they come first among the keys, the step's own rows, which the other prompts attend, behind them (None
+        where no prompt does).  None where the kernel does not cover the model."""
         D = self.shape.head_dim
         if not ctx.is_prefill or self.dtype != torch.bfloat16 or D % 8 or D > 128:
             return None
-        tiles = torch.from_numpy(plan_prompts(ctx.seq_lens_q, ctx.seq_lens_k)).pin_memory().to(self.device, non_blocking=True)
-        if ctx.seq_lens_q == ctx.seq_lens_k:
-            return tiles, None
+        lens = list(zip(ctx.seq_lens_q, ctx.seq_lens_k))
+        cached = [b for b, (nq, nk) in enumerate(lens) if nq != nk]
+        back = sum(lens[b][1] for b in cached)
+        starts, read, own = [], 0, back
+        for nq, nk in lens:
+            starts.append(own if nq == nk else read)
+            own, read = own + nq, read + (nk if nq != nk else 0)
+        tiles = torch.from_numpy(plan_prompts(ctx.seq_lens_q, ctx.seq_lens_k, starts)).pin_memory().to(self.device, non_blocking=True)
+        if not cached:
+            return tiles, None, True
         BS = self.k_cache.shape[2]
         at = torch.arange(BS, dtype=torch.int32, device=self.device)
-        rows = [(ctx.block_tables[b, :-(-n // BS), None] * BS + at).flatten()[:n] for b, n in enumerate(ctx.seq_lens_k)]
-        return tiles, torch.cat(rows).int()
+        rows = [(ctx.block_tables[b, :-(-lens[b][1] // BS), None] * BS + at).flatten()[:lens[b][1]] for b in cached]
+        return tiles, torch.cat(rows).int(), len(cached) < len(lens)
 
     def _prefill_attention(self, li, q, k, v, ctx: StepContext, plan) -> torch.Tensor:
         s = self.shape
         if plan is not None:
-            tiles, rows = plan
-            if rows is not None:   # cached prefixes: the whole contexts come back from the cache
-                k, v = (gather_rows(c[li].flatten(2), rows).view(-1, s.kv_heads, s.head_dim) for c in (self.k_cache, self.v_cache))
+            tiles, rows, own = plan
+            if rows is not None:
+                back = (gather_rows(c[li].flatten(2), rows).view(-1, s.kv_heads, s.head_dim) for c in (self.k_cache, self.v_cache))
+                k, v = (torch.cat([b, t]) if own else b for b, t in zip(back, (k, v)))
             return causal_attention(q, k, v, tiles, self.scale)
         lens_q, lens_k = ctx.seq_lens_q, ctx.seq_lens_k
         if lens_q == lens_k and len(set(lens_q)) == 1:
