@@ -104,6 +104,37 @@ def test_prompts_with_and_without_a_cached_prefix_in_one_step(dev):
     assert (h.float() - want).abs().max() < 6e-2
 
 
+@pytest.mark.parametrize("lens_q,lens_k", [([64, 64], [64, 64]), ([37, 130], [37, 130]), ([37, 18], [37, 50])])
+def test_captured_prefill_equals_eager(dev, lens_q, lens_k):
+    """Prompts of one length, of several, and one that continues a cached prefix; every replay is on other tokens, behind
+    eager steps of the same prompts and of others."""
+    from zipage_amd.engine import Qwen3, StepContext
+    s = _tiny()
+    BS, pages = 16, 12
+    model = Qwen3(s, dev, seed=5, init_std=0.05)
+    kv = torch.randn(2, s.layers, pages, BS, s.kv_heads, s.head_dim, device=dev).to(torch.bfloat16)
+    model.attach_caches(kv, torch.zeros(s.layers, 2, 4, s.heads, s.head_dim, device=dev, dtype=torch.bfloat16))
+    tables = torch.arange(10, dtype=torch.int32).view(2, 5)
+    slot = lambda b, t: int(tables[b, t // BS]) * BS + t % BS if t < 5 * BS else -1
+    at = [(b, t) for b, (q, k) in enumerate(zip(lens_q, lens_k)) for t in range(k - q, k)]
+    slots = torch.tensor([slot(*x) for x in at], dtype=torch.int32, device=dev)
+    ctx = StepContext(True, slots, None, None, tables.to(dev), lens_q, lens_k)
+    pos, ids = torch.tensor([t for _, t in at], device=dev), torch.zeros(len(at), dtype=torch.long, device=dev)
+    model.forward(ids, pos, ctx)                     # lazy initialisations happen outside capture
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g), torch.inference_mode():
+        got = model.forward(ids, pos, ctx)
+    for _ in range(4):
+        ids.copy_(torch.randint(0, s.vocab, (len(at),), device=dev))
+        want = model.forward(ids, pos, ctx).float()
+        for cut in (20, 41, 3, 50):                  # as many tokens, other prompts
+            model.forward(ids, pos, StepContext(True, None, None, None, None, [cut, len(at) - cut], [cut, len(at) - cut]))
+        torch.cuda.synchronize()
+        g.replay()
+        torch.cuda.synchronize()
+        assert (got.float() - want).abs().max() < 6e-2
+
+
 def _generate(cfg, prompts, max_tokens):
     from zipage_amd.engine import SamplingParams, ZipageEngine
     eng = ZipageEngine(cfg)

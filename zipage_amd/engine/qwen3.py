@@ -3,8 +3,8 @@
 Only what the decode benchmark needs: bf16 weights drawn on the device and the fused qkv and
 gate/up projections through torch's GEMMs; everything between the GEMMs is this package's HIP
 kernels (residual add + RMSNorm, per-head q/k norm + rotary embedding + K/V scatter + window-query
-capture, paged decode attention, SiLU gate, causal attention of prompts).  In float16 prefill attention is
-torch's scaled_dot_product_attention.
+capture, paged decode attention, SiLU gate, causal attention of prompts).  In float16, and in a captured step,
+prefill attention is torch's scaled_dot_product_attention.
 """
 from __future__ import annotations
 
@@ -123,9 +123,10 @@ class Qwen3:
     def _plan_prefill(self, ctx: StepContext):
         """Query tiles of a step of prompts, and the cache rows of the prompts with a cached prefix, whose whole contexts are
         read back: they come first among the keys, the step's own rows, which the other prompts attend, behind them (None
-        where no prompt does).  None where the kernel does not cover the model."""
+        where no prompt does).  None where the kernel does not cover the model, and during a capture: a replay would copy the
+        plan from host memory that is gone."""
         D = self.shape.head_dim
-        if not ctx.is_prefill or self.dtype != torch.bfloat16 or D % 8 or D > 128:
+        if not ctx.is_prefill or self.dtype != torch.bfloat16 or D % 8 or D > 128 or torch.cuda.is_current_stream_capturing():
             return None
         lens = list(zip(ctx.seq_lens_q, ctx.seq_lens_k))
         cached = [b for b, (nq, nk) in enumerate(lens) if nq != nk]
