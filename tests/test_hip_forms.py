@@ -43,6 +43,24 @@ def test_compaction_of_few_rows(dev, dtype, L, B, Hkv, D, style):
     assert torch.equal(gv.cpu().view(torch.uint8), wv.view(torch.uint8))
 
 
+# the list of 65 536 tokens and its pages, which fill the LDS but for 16 or 64 bytes: the former leaves no room for the
+# sums of sixteen waves
+@pytest.mark.parametrize("width", [4092, 4080])
+def test_compaction_of_the_longest_list(dev, width):
+    from zipage_amd.kernel import compress_kv
+    BS, NB, D = 16, 4096, 64
+    g = torch.Generator().manual_seed(width)
+    table = torch.randperm(NB, generator=g).tolist()
+    enc, target = O.encode_block_table([table]), torch.tensor([table[:width]], dtype=torch.int32)
+    k, v = (_rand(1, NB, BS, 1, D, seed=s) for s in (1, 2))
+    flag = (torch.rand((1, 1, 1, NB, BS), generator=g) < 0.9)
+    wk, wv = k.clone(), v.clone()
+    O.compress_kv(wk, wv, flag, enc, target)
+    gk, gv = k.to(dev), v.to(dev)
+    compress_kv(gk, gv, flag.to(dev), enc.to(dev), target.to(dev))
+    assert torch.equal(gk.cpu(), wk) and torch.equal(gv.cpu(), wv)
+
+
 # ------------------------------------------------------------------ experts
 # rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup when
 # there are many and tokens come to six per expert; 256-row tiles are worked off whole from a contraction of 2560 on, in

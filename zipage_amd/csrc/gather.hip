@@ -220,11 +220,14 @@ static int log2_exact(int v) {
   return s;
 }
 
+// of a workgroup: the list, and the pages of both tables
+inline size_t compact_lds(const CompactArgs& a) {
+  return (((size_t)a.NB * a.BS * 2 + 15) & ~(size_t)15) + sizeof(int) * ((size_t)a.NB + a.target_width);
+}
 template <typename P, int R, bool HAS_B, bool POW2, int CES = 0, int NT = kThreads>
 int launch_compact_impl(CompactArgs a, int L, hipStream_t st) {
   a.n_items = L * a.B * a.Hkv;
-  const int T = a.NB * a.BS;
-  size_t smem = (((size_t)T * 2 + 15) & ~(size_t)15) + sizeof(int) * (a.NB + a.target_width);
+  const size_t smem = compact_lds(a);
   dim3 grid((unsigned)((int64_t)L * a.B * a.Hkv * (!HAS_B && a.split_kv ? 2 : 1) * (NT != kThreads ? a.parts : 1)));
   if (smem > 64 * 1024) {
     hipError_t e = hipFuncSetAttribute((const void*)compact_kernel<P, R, HAS_B, POW2, CES, NT>,
@@ -255,10 +258,11 @@ inline bool aligned_to(int64_t v, int n) { return (v % n) == 0; }
 // -> wide form: 1 fp32 sequence of 8 heads 110 -> 59 us, 8 of them 130 -> 99, 32 of them (512 pairs) 323 -> 314; 1
 // bfloat16 sequence 64 -> 42, 16 of them 101 -> 91, 32 of them 171 -> 163.  At 1 024 pairs the general form has four
 // workgroups per CU and the wide one is within 1 % either way; cutting beyond 256 workgroups loses 1-3 %.
-// Returns the column ranges, 0: the general form.
-constexpr int kWideUnits = 512, kWideGrid = 256, kLinePieces = 8;
-inline int wide_parts(int64_t pairs, int lpv) {
-  if (pairs > kWideUnits) return 0;
+// Returns the column ranges, 0: the general form, also for the longest lists, which leave no room for the sums of sixteen
+// waves beside them.
+constexpr int kWideUnits = 512, kWideGrid = 256, kLinePieces = 8, kLds = 160 * 1024;
+inline int wide_parts(int64_t pairs, int lpv, size_t lds) {
+  if (pairs > kWideUnits || lds + kWideThreads / 64 * sizeof(int) > kLds) return 0;
   int parts = 1;
   while (pairs * parts * 2 <= kWideGrid && lpv % (parts * 2 * kLinePieces) == 0) parts *= 2;
   return parts;
@@ -332,7 +336,7 @@ int compress_kv_impl(void* key, void* value, const uint8_t* flag, const int32_t*
   // the gather's latency: 0.340 against 0.347 ms per step at 64 sequences x 8 heads; with many rows
   // the CUs are full either way and one survivor list per row is cheaper)
   const bool split = piece == 16 && (int64_t)L * B * Hkv <= kSplitKvRows;
-  const int parts = piece == 16 && log2_exact(BS) >= 0 && log2_exact(a.lpv) >= 0 ? wide_parts((int64_t)L * B * Hkv * 2, a.lpv) : 0;
+  const int parts = piece == 16 && log2_exact(BS) >= 0 && log2_exact(a.lpv) >= 0 ? wide_parts((int64_t)L * B * Hkv * 2, a.lpv, compact_lds(a)) : 0;
   if (parts) {
     a.split_kv = 1;
     a.parts = parts;
