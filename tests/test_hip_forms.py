@@ -70,7 +70,8 @@ def test_compaction_of_the_longest_list(dev, width):
                                               (260, 160, 4, 1, 288), (1100, 2144, 3, 2, 96), (1100, 96, 2, 1, 2112),
                                               (1300, 256, 2, 1, 96), (515, 2112, 1, 1, 48),
                                               (1100, 2592, 3, 2, 96), (1100, 96, 2, 1, 2592), (515, 2624, 1, 1, 48),
-                                              (200, 96, 64, 2, 800), (225, 2080, 64, 2, 544)])
+                                              (200, 96, 64, 2, 800), (225, 2080, 64, 2, 544),
+                                              (200, 96, 64, 2, 1120)])
 @pytest.mark.parametrize("act", ["clamped", "silu"])
 def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act, shared_ff=None):
     from zipage_amd.layers import Experts

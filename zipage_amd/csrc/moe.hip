@@ -394,14 +394,16 @@ template <typename T> __device__ __forceinline__ float gated(int act, float w, f
 // (gate_up: tiles of the gate and those of `up` that belong to them) and up to 16 * MT tokens; its four waves share
 // the steps of the contraction and meet in LDS.  What the weights' stream loses is what else passes the caches: 16
 // rows of tokens per kRowsW tiles of W, and twice as much where two waves take the two halves of a token's cache line.
-// One token tile (hardly any expert has a second): a wave takes pairs of steps, whole lines of x, and the workgroup
-// 128 rows of W where that leaves two workgroups per CU and tokens come to six per expert (64 tokens over 33 experts of
-// 3 x 4096 x 3072: 516 -> 476 us, 5.2 TB/s; with 64 rows 497; 48 tokens of 4 of 32: 405, 394, 400).  With fewer tokens
-// there is less of x to read again, and the last workgroups are half as long with 64 rows (9 tokens: 314, 317, 306; 24:
-// 385, 390, 385; widths of 2048: 95, 97, 94).  More token tiles keep 64 rows and single steps (256 tokens: 675 us; 687
-// with pairs, 876 with 128 rows).
+// One token tile (hardly any expert has a second): a wave takes pairs of steps, whole lines of x.  The workgroup has 128
+// rows of W from six tokens per expert on (with fewer there is less of x to read again: 42 tokens of 3 of 32 experts, 3 x
+// 4096 x 3072 each, 397 us, 399 with 128 rows; 53: 424, 429) and where at least two and a half rounds of workgroups (two per
+// CU) are asked for, as the last round is twice as long.  With 64 rows and with 128, whole layers of 6, 7 and 8 tokens per
+// expert, 3 of 32 with a shared expert: 4096 wide 495 and 475 us, 449 and 450, 474 and 480; 4 of 32 without one 395 and 388,
+// 393 and 390, 387 and 386.  Single products: the first, 3 x 5120 x 3840 and 3 x 6144 x 4608, -1 to +3 %; 3 x 3072 x 2304 +4 to
+// -3 %; 3 x 2048 x 1536, whose products stay below the line, +3 to -4 %, the last -13 to +1 %.
+// More token tiles keep 64 rows and single steps (256 tokens: 675 us; 687 with pairs, 876 with 128 rows).
 constexpr int kNarrowW = 4, kWideW = 8;                // 16-row tiles of W
-constexpr int kWideGrid = 512, kWideRows = 6;          // workgroups and average rows from which on 128 rows of W are better
+constexpr int kWideGrid = 1280, kWideRows = 6;         // workgroups and average rows from which on 128 rows of W are better
 template <typename T, int MT, bool UP, int kRowsW>
 __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
