@@ -351,9 +351,11 @@ def test_headwise_by_tokens_and_contraction(dev, n, H, K, M, tail):
 
 
 # ------------------------------------------------------------------ few outputs
-# from 4 081 rows and 17 outputs on through LDS: 32 tokens by 32 or 64 outputs, stages of 128 elements
+# from 4 081 rows, 17 outputs, a contraction of 256 and 2.2 million elements of x on through LDS: 32 tokens by 32 or 64
+# outputs, stages of 128 elements
 @pytest.mark.parametrize("n,K,M", [(4080, 160, 20), (4081, 32, 20), (4099, 160, 32), (4095, 1056, 36), (4100, 96, 100),
-                                   (5000, 640, 64), (4113, 4128, 132)])
+                                   (5000, 640, 64), (4113, 4128, 132), (8594, 256, 20), (8593, 256, 20), (8100, 224, 36),
+                                   (6900, 320, 100), (4099, 544, 32)])
 def test_small_linear_of_many_rows(dev, n, K, M):
     from zipage_amd.layers import small_linear
     x, w = _rand(n, K + 8, seed=8)[:, :K], _rand(M, K, seed=9)

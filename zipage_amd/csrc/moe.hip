@@ -93,8 +93,9 @@ __global__ __launch_bounds__(64 * NW) void small_linear_kernel(SmallArgs a) {
 
 // Many rows, bf16: 16 * TT tokens x 16 * MT outputs, operands through LDS.  A row read as it is multiplied gives 64 bytes of
 // a line to a load, and the L1 takes four to five cycles for every line touched (16 384 tokens, 32 outputs of 4096: 69 us,
-// now 31; 128 outputs 148, now 65).  A stage is 128 elements of every row, a step for each of the four waves: the same share of the contraction
-// that each has above, so that sums are the same to the last bit.  A row's sixteen pieces lie in the order of (piece ^ row).
+// now 31; 128 outputs 148, now 65).  A stage is 128 elements of every row, a step for each of the four waves: the same share
+// of the contraction that each has above, so that sums are the same to the last bit.  A row's sixteen pieces lie in the
+// order of (piece ^ row).
 template <int TT, int MT> struct SmallTile {
   static constexpr int kRing = MT > 2 ? 3 : 4, kBytes = (TT + MT) * 4096, kLoads = TT + MT;   // of a stage; of a wave
 };
@@ -813,7 +814,11 @@ extern "C" int zp_small_linear(const void* x, const void* w, float* out, int32_t
   const unsigned gx = (unsigned)((n + 15) / 16);
   const bool wide = gx >= 256 && M > 16;
   const dim3 grid(gx, (unsigned)(wide ? (M + 63) / 64 : (M + 15) / 16));
-  if (wide && dtype == ZP_BF16 && 32 * x_stride * 2 < 1ll << 31 && (int64_t)64 * K * 2 < 1ll << 31) {
+  // through LDS where there are stages enough to pass the time with (us of both, this one second: K 128, 4081 rows of 64
+  // outputs 4.1 and 4.9, 16 384 of 256 14.3 and 15.2; K 160, 5.4 and 6.3; K 256, 4081 rows of 36 outputs 4.5 and 5.1, 8192
+  // 5.2 and 5.1, 16 384 6.9 and 5.9; K 512, 4081 of 36 5.5 and 5.8, of 128 8.0 and 6.1), and offsets are within 31 bits
+  if (wide && dtype == ZP_BF16 && K >= 256 && (int64_t)n * K >= 2200000 && 32 * x_stride * 2 < 1ll << 31 &&
+      (int64_t)64 * K * 2 < 1ll << 31) {
     const dim3 tiles((unsigned)((n + 31) / 32), (unsigned)(M <= 32 ? 1 : (M + 63) / 64));
     const int smem = M <= 32 ? SmallTile<2, 2>::kRing * SmallTile<2, 2>::kBytes : SmallTile<2, 4>::kRing * SmallTile<2, 4>::kBytes;
     const void* const fn = M <= 32 ? (const void*)small_tile_kernel<2, 2> : (const void*)small_tile_kernel<2, 4>;
