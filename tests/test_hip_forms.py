@@ -329,10 +329,12 @@ def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
 
 # ------------------------------------------------------------------ per-head products
 # through LDS: tiles of 64 outputs by 16, 32 or 64 tokens, stages of 128 elements in a ring of four; straight from
-# memory: up to 16 tokens of one stage
+# memory: contractions below 256 (512 with fewer than 64 outputs) and below 8192 matrix products
 @pytest.mark.parametrize("n,H,K,M,tail", [(1, 2, 160, 16, 0), (16, 3, 128, 80, 8), (16, 65, 128, 272, 0), (17, 3, 544, 48, 0),
                                           (33, 64, 128, 144, 64), (65, 8, 1056, 64, 0), (129, 130, 96, 112, 8),
-                                          (64, 256, 32, 16, 24), (200, 72, 640, 128, 0)])
+                                          (64, 256, 32, 16, 24), (200, 72, 640, 128, 0), (9, 3, 256, 64, 8), (9, 3, 224, 64, 8),
+                                          (40, 171, 64, 128, 0), (39, 171, 64, 128, 0), (33, 4, 480, 48, 0), (24, 512, 128, 48, 8),
+                                          (1300, 33, 32, 64, 8), (70, 3, 192, 80, 40), (200, 70, 64, 64, 64)])
 def test_headwise_by_tokens_and_contraction(dev, n, H, K, M, tail):
     from zipage_amd.layers.latent import headwise_linear
     x, w = _rand(n, H, K + tail, seed=6), _rand(H, M, K, seed=7)

@@ -1119,12 +1119,18 @@ extern "C" int zp_headwise_linear(const void* in, const void* w, void* out, cons
   ZP_REQUIRE(in && w && out && aligned16(in) && aligned16(w) && aligned16(out),
              "headwise_linear: null or unaligned pointer");
   HeadArgs a = {in, w, out, positions, freqs, n, H, K, M, tail, rot / 2};
-  // The staged kernel, except for one stage of one token tile that has its CU to itself and nothing to pass the time with
-  // (1 token, 32 heads of 128 -> 512: 4.1 us, 3.6 without; 16 tokens 4.3 both; 8 tokens, 128 heads 6.6, 9.1 without), and
-  // what its 32-bit offsets don't span.
+  // The staged kernel, except for what its 32-bit offsets don't span and for little work in one or two stages, whose set-up
+  // nothing hides: from 8192 matrix products on it is ahead (us of both, the staged one second: K 160, 16 heads of M 64, 1 to
+  // 200 tokens 2.9 to 3.3 and 3.5 to 3.8, 1000 tokens 5.6 and 4.5; K 128, 16 heads of M 64, 200 tokens 3.3 and 3.4, 1000 5.4
+  // and 3.9; K 96, 64 heads of M 112, 17 tokens 2.9 and 3.4, 64 tokens 3.5 and 3.7, 200 6.6 and 4.5; K 64, 64 heads of M 256,
+  // 17 tokens 3.1 and 3.6, 64 tokens 4.0 and 3.8; K 32, 64 heads of M 64, 200 tokens 3.2 and 3.8, 1000 6.7 and 6.3), if its
+  // rows of W hold at least 3 KB (M 16, K 32, 64 heads, 4000 tokens: 10.0 and 13.3) and the tails are not most of it (K 64, M
+  // 64, 64 behind them, 128 heads, 4000 tokens: 96 and 122).  K 256: 17 tokens 4.2 and 3.7; 512: 5.8 and 4.6; with M 16 3.4
+  // and 3.6, 4.5 and 4.5
   const int64_t columns = (int64_t)((M + 63) / 64) * H;
-  const bool staged = dtype == ZP_BF16 && !(n <= 16 && K <= kHeadStage && columns <= 256) &&
-                      (int64_t)M * K * 2 < 1ll << 31 && (int64_t)64 * H * (K + tail) * 2 < 1ll << 31;
+  const int64_t products = (int64_t)(K / 32) * (M / 16) * H * (n < 24 ? 1 : (n + 8) / 16);
+  const bool much = K >= (M < 64 ? 512 : 256) || (products >= 8192 && (M < 64 ? M : 64) * K >= 1536 && (tail < K || tail < M));
+  const bool staged = dtype == ZP_BF16 && much && (int64_t)M * K * 2 < 1ll << 31 && (int64_t)64 * H * (K + tail) * 2 < 1ll << 31;
   // as many tokens per wave (W is read once for them) as still leave two workgroups per CU; of the staged kernel as many as
   // leave one (64 tokens, 32 heads of 512 -> 128: 6.9 us with 64 workgroups, 5.5 with 256), and no more than there are
   int tt = staged && n <= 32 ? (n <= 16 ? 1 : 2) : 4;
