@@ -397,14 +397,16 @@ template <typename T> __device__ __forceinline__ float gated(int act, float w, f
 // rows of tokens per kRowsW tiles of W, and twice as much where two waves take the two halves of a token's cache line.
 // One token tile (hardly any expert has a second): a wave takes pairs of steps, whole lines of x.  The workgroup has 128
 // rows of W from six tokens per expert on (with fewer there is less of x to read again: 42 tokens of 3 of 32 experts, 3 x
-// 4096 x 3072 each, 397 us, 399 with 128 rows; 53: 424, 429) and where at least two and a half rounds of workgroups (two per
-// CU) are asked for, as the last round is twice as long.  With 64 rows and with 128, whole layers of 6, 7 and 8 tokens per
-// expert, 3 of 32 with a shared expert: 4096 wide 495 and 475 us, 449 and 450, 474 and 480; 4 of 32 without one 395 and 388,
-// 393 and 390, 387 and 386.  Single products: the first, 3 x 5120 x 3840 and 3 x 6144 x 4608, -1 to +3 %; 3 x 3072 x 2304 +4 to
-// -3 %; 3 x 2048 x 1536, whose products stay below the line, +3 to -4 %, the last -13 to +1 %.
+// 4096 x 3072 each, 397 us, 399 with 128 rows; 53: 424, 429), and where 40 tiles and 1280 workgroups are asked for: with few
+// experts, or two rounds of workgroups (two per CU), the last one, twice as long, costs more.  With 64 rows and with 128,
+// whole layers of 6, 7 and 8 tokens per expert, 3 of 32 with a shared expert: 4096 wide 495 and 475 us, 449 and 450, 474 and
+// 480; 4 of 32 without one 395 and 388, 393 and 390, 387 and 386.  Single products above the line, of 32 and 64 experts, are
+// 3 % slower to 6 % faster (on average 1.5 % faster); below it, 8 experts of 3 x 3072 x 8192, the first, 124 and 132; 16 of
+// 3 x 1536 x 4096, 66 and 69; 32 of 3 x 2048 x 1536 +3 to -4 %, the last -13 to +1 %.
 // More token tiles keep 64 rows and single steps (256 tokens: 675 us; 687 with pairs, 876 with 128 rows).
 constexpr int kNarrowW = 4, kWideW = 8;                // 16-row tiles of W
-constexpr int kWideGrid = 1280, kWideRows = 6;         // workgroups and average rows from which on 128 rows of W are better
+constexpr int kWideGrid = 1280, kWideTiles = 40, kWideRows = 6;    // workgroups, token tiles and average rows from which on
+                                                                   // 128 rows of W are better
 template <typename T, int MT, bool UP, int kRowsW>
 __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
@@ -762,7 +764,8 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
   const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
-  const bool wide = rows == 16 && dtype == ZP_BF16 && grid_of(kWideW) >= kWideGrid && (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
+  const bool wide = rows == 16 && dtype == ZP_BF16 && a.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
+                    (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
   const int64_t grid = grid_of(wide ? kWideW : kNarrowW);
   if (grid >= (1ll << 31)) {
     zp_set_error("moe: too many tiles");
