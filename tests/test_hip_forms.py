@@ -135,9 +135,8 @@ def _tiles(lens):
 # the scale joins the subtraction of the maximum: a negative one turns the queries round, zero takes them away
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-30, 0.25])
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 40, 24), (2, 2, 64, 64), (3, 1, 128, 56), (4, 2, 128, 128), (3, 3, 136, 136)])
-def test_runs_of_any_scale(dev, H, G, D, V, scale):
+def test_runs_of_any_scale(dev, H, G, D, V, scale, lens=((1, 1), (63, 63), (65, 65), (32, 64), (33, 129), (130, 200))):
     from zipage_amd.layers import run_attention
-    lens = [(1, 1), (63, 63), (65, 65), (32, 64), (33, 129), (130, 200)]
     N, M = (sum(t) for t in zip(*lens))
     q, k = (_rand(N, H, D, seed=1), _rand(M, G, D, seed=2))
     v = _rand(M, G, V, seed=3)
@@ -149,12 +148,24 @@ def test_runs_of_any_scale(dev, H, G, D, V, scale):
     assert bool(((out.view(N, H, V).cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -7 * v.abs().max()).all())
 
 
+# up to 256 keys, and up to 32 per tile on average: steps of 32 keys, whatever a run has
+FEW_KEYS = [(1, 1)] * 5 + [(16, 16), (17, 33), (64, 65), (96, 137)]
+
+
+@pytest.mark.parametrize("H,G,D,V", [(2, 1, 128, 128), (3, 3, 136, 128), (4, 2, 40, 72), (2, 2, 64, 64), (2, 1, 200, 256)])
+def test_runs_of_few_keys(dev, H, G, D, V):
+    test_runs_of_any_scale(dev, H, G, D, V, 0.25, FEW_KEYS)
+
+
+def test_causal_attention_of_few_keys(dev):
+    test_causal_attention(dev, 8, 2, 128, FEW_KEYS)
+
+
 @pytest.mark.parametrize("H,G,D", [(2, 1, 8), (4, 4, 64), (6, 2, 72), (8, 2, 128)])
-def test_causal_attention(dev, H, G, D):
+def test_causal_attention(dev, H, G, D, lens=((1, 1), (31, 31), (128, 128), (129, 129), (5, 300), (64, 65), (257, 257))):
     """Prompts with and without cached context, of lengths about a tile's and a step's; queries that point at one key."""
     from zipage_amd.engine.inputs import plan_prompts
     from zipage_amd.layers import causal_attention
-    lens = [(1, 1), (31, 31), (128, 128), (129, 129), (5, 300), (64, 65), (257, 257)]
     N, M = (sum(t) for t in zip(*lens))
     qkv = _rand(N, (H + 2 * G) * D, seed=1)
     k, v = _rand(M, G, D, seed=2), _rand(M, (H + 2 * G) * D, seed=3)

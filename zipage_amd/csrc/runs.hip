@@ -80,18 +80,20 @@ __device__ __forceinline__ void eight_columns(const f32x4& even, const f32x4& od
 }
 
 enum { kNoCap, kCap, kBoundedCap };   // of the scores, see SoftCap
+// Keys per step: 64 scores for each query where the registers hold them (8 prompts as above: 519 -> 463 us; keys of 192
+// with a shared part spill: 1811 -> 1831).
+constexpr int long_step(int DKS, int VCB, int MAPS, bool SHARED, int CAP) {
+  return MAPS == 1 && VCB == 1 && CAP == kNoCap && DKS <= (SHARED ? 4 : 6) ? 64 : 32;
+}
 
 // Column tile t of a wave: 16 queries, map t % MAPS of the head (differential attention has two, over the same
 // values; elsewhere there is one).  SHARED: the last P elements of every head's key are the row of a.ks.
 // FINE: softmax weights enter the value product as two bf16 planes (17 bits), elsewhere as one.
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE>
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
 __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(TilesArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef TileStage<DKS, VCB, MAPS> Stage;
   constexpr bool kTurns = MAPS == 1 && !SHARED && CAP == kNoCap;
-  // keys per step: 64 scores for each query where the registers hold them (8 prompts as above: 519 -> 463 us; keys of 192
-  // with a shared part spill: 1811 -> 1831)
-  constexpr int kStep = MAPS == 1 && VCB == 1 && CAP == kNoCap && DKS <= (SHARED ? 4 : 6) ? 64 : 32;
   constexpr bool kPinned = DKS <= 4 && (VCB == 1 || MAPS == 1);   // reads ahead: wider heads would spill
   constexpr int kT = kQT * MAPS, kWaves = Stage::kWaves, kThreads = 64 * kWaves, kPass = 16 * kQT * kWaves;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
@@ -692,19 +694,28 @@ template <int DKS, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st
 }
 
 
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
-int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
+int launch_steps(const TilesArgs& a, hipStream_t st) {
   constexpr int smem = TileStage<DKS, VCB, MAPS>::kBytes;
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE>,
+      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE>), dim3((unsigned)a.T * a.H),
+  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>), dim3((unsigned)a.T * a.H),
                      dim3(64 * TileStage<DKS, VCB, MAPS>::kWaves), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
+}
+// Steps of 32 keys where tiles have no more on average: a prompt of 16 tokens, 32 heads of 128 5.2 us (5.8 with 64), of 32
+// 5.5 (6.1); of 64 6.4 (6.3).  Not among many keys, where one long run may decide (31 prompts of 16 tokens and one of 512
+// 23.1, 20.3 with 64).
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
+int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
+  constexpr int kLong = long_step(DKS, VCB, MAPS, SHARED, CAP);
+  if (a.k_rows <= 256 && a.k_rows <= 32 * (int64_t)a.T) return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, 32>(a, st);
+  return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kLong>(a, st);
 }
 
 template <bool SHARED, int CAP> int launch_one_map(const TilesArgs& a, hipStream_t st) {
