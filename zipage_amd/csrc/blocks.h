@@ -1,11 +1,11 @@
-// The recurrent mixers over long runs of tokens: 16 tokens at a time on the fp32 matrix cores, the state
-// of a head in registers.
+// The recurrent mixers over long runs of tokens: 16 tokens at a time on the bf16 matrix cores, fp32 operands in three
+// planes, the state of a head in registers.
 //
-// A wave owns 16 * NC columns of the state.  S lies in the result layout of the 16x16 products (lane (g,
-// l16) holds rows 16 kt + 4 g + r of column l16 in element r), which is also the layout of a right operand
-// if step j of the contraction takes index 4 g + j from lane group g.  So S, and the rows u derived from
-// it, enter the next product from the registers they were computed in; left operands give a lane the four
-// elements 4 g .. 4 g + 3 of its row.
+// A wave owns 16 * NC columns of the state.  S lies in the result layout of the 16x16 products (lane (g, l16) holds rows 16 kt
+// + 4 g + r of column l16 in element r), which is also the layout of a right operand if the contraction is numbered
+// accordingly: of 32, lane group g has rows 4 g .. 4 g + 3 of one tile and those of the next.  So S, and the rows u derived
+// from it, enter the next product from the registers they were computed in; left operands give a lane the same elements
+// of its row.
 #pragma once
 #include "scan.h"
 #include "mfma.h"
@@ -13,15 +13,6 @@
 namespace {
 
 constexpr int kBlock = 16;
-
-__device__ __forceinline__ f32x4 mfma_f32_step(float a, float b, const f32x4& c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-// c += A B over sixteen of the contraction: a is the left operand's four elements, b a result tile.
-__device__ __forceinline__ void mfma_f32_16(const f32x4& a, const f32x4& b, f32x4& c) {
-#pragma unroll
-  for (int j = 0; j < 4; ++j) c = mfma_f32_step(a[j], b[j], c);
-}
 
 template <int KT, int NC> __device__ __forceinline__ void load_state(f32x4 (&S)[KT][NC], const float* state, int dv, int col0, bool fresh) {
   const int l16 = threadIdx.x & 15, g = (threadIdx.x & 63) >> 4;
@@ -43,9 +34,10 @@ template <int KT, int NC> __device__ __forceinline__ void store_state(const f32x
       for (int r = 0; r < 4; ++r) state[(int64_t)(16 * kt + 4 * g + r) * dv + col0 + nc * 16 + l16] = S[kt][nc][r];
 }
 
-// An fp32 operand in three bf16 planes: each is what those before it leave, rounded to eight bits and a sign, so that they
-// hold more than its 24 bits, and the products of the first with all, of the second with the first two and of the third with
-// the first miss less than 2^-26 of a product.
+// An fp32 operand in three bf16 planes: each is what those before it leave, rounded to eight bits and a sign.  Together they
+// are its 24 bits: the second is at most 2^-8 of x, the third 2^-17.  Six products (the first plane with all, the second
+// with the first two, the third with the first) miss up to 2^-24 of the product of two operands' leading bits, as much as
+// an fp32 product is rounded by; eight (all but the third with the third) up to 2^-34.
 struct Planes {
   uint2 hi, mid, lo;
   __device__ __forceinline__ Planes(const f32x4& x) {
@@ -72,7 +64,7 @@ struct Planes {
   }
 };
 // A right operand of 16 of the contraction for left ones that lie as [64 lanes][hi 4, mid 4], [64][lo 4]: the bf16 matrix
-// cores take 32, so planes go in pairs.
+// cores take 32, so planes go in pairs, eight products in four.
 constexpr int kPairFloats = 384;               // of such a left operand
 struct PlanePairs {
   u32x4 hh, mm, ll, hm;

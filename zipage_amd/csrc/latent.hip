@@ -642,7 +642,7 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
 // (4 / HW) share its value columns out and compute its scores each for itself, so that they meet only to hand over LDS.
 //
 // Bound by HBM, so what counts is how much is on its way: rows go from memory into LDS without passing through
-// registers, in a ring of stages of 32 keys of which all but one are in flight (128 KB per CU for rows of 576; held in
+// registers, in a ring of stages of 32 keys of which all but one are in flight (108 KB per CU for rows of 576; held in
 // registers between its two uses, a block left its place only when its products were done: 256 sequences of 2050 tokens,
 // 32 heads 157 us, now 141; a window of 1024 76, now 60; 64 sequences, 128 heads 124, now 92).  The value operand is
 // transposed by the LDS reads.  An odd number of 16-byte pieces per staged row keeps both operands off each other's banks.

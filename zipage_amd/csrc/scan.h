@@ -31,10 +31,13 @@ __device__ __forceinline__ Segment segment_of(const zp_segments& s, int i) {
 __device__ __forceinline__ int lane_cq() { return threadIdx.x & 7; }
 __device__ __forceinline__ int lane_rg() { return (threadIdx.x & 63) >> 3; }
 
-// A decoded token passes over the state once, and the next reads it after every other layer's.  A layer's states that the
-// last-level cache (256 MB) cannot hold until then go past it, non-temporal both ways (256 sequences, heads of 128 x 128:
-// linear attention with 32 heads 226 -> 215 us, delta rule with 32 244 -> 203; 180 sequences 154 -> 150 and 176 -> 147);
-// smaller ones may still be there (128 sequences, 32 heads: linear 94 us, 110 past it; 62, retention with 16: 22 and 23).
+// A decoded token passes over the state once.  A layer's states that the last-level cache (256 MB) cannot hold until the
+// next token go past it, non-temporal both ways (256 sequences, heads of 128 x 128: linear attention with 32 heads 227 -> 215
+// us, delta rule with 32 245 -> 203; 180 sequences 154 -> 150 and 177 -> 148).  Smaller ones stay with the caches, where a
+// layer called by itself finds them again (128 sequences, 32 heads: linear 92 us, 109 past it; 96: 67, 83; delta 78, 86;
+// retention with 16 heads, 180 sequences 60, 71).  Where other layers' states come in between, up to 3 GB in all, they are
+// gone by then and going past would be the faster way at every size (linear, 128 sequences 121 us, 110 past it; 62: 68, 58;
+// delta 138, 112 and 79, 64; retention, 62 sequences 34, 25): a call sees one layer and cannot tell.
 // Not for the matrix memory, whose states do not begin on a cache line: 133 -> 215 us, 190 with the loads alone.
 inline bool past_cache(int64_t states, int dk, int dv) { return states * dk * dv * 4 >= 320ll << 20; }
 template <bool PAST> __device__ __forceinline__ f32x4 load_state(const float* p) {
