@@ -646,6 +646,10 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
 // registers between its two uses, a block left its place only when its products were done: 256 sequences of 2050 tokens,
 // 32 heads 157 us, now 141; a window of 1024 76, now 60; 64 sequences, 128 heads 124, now 92).  The value operand is
 // transposed by the LDS reads.  An odd number of 16-byte pieces per staged row keeps both operands off each other's banks.
+//
+// Softmax weights meet the values in two bf16 planes.  With one, results were up to 0.5 % further from 64-bit ones than those
+// of waves with maxima of their own (the weight of a maximum is 1 and loses nothing, and here there are fewer); with two
+// they are 2 to 3 % nearer, for 5 % of the kernel's time (141 -> 147 us of the first).
 constexpr int rows_ring(int NCB) { return NCB <= 2 ? 3 : 4; }       // two workgroups per CU where rows are short
 template <int NCB, int PK> struct RowsStage {
   static constexpr int kMaxPieces = NCB * 16 + PK * 4 + 1;
@@ -805,7 +809,7 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
       vf[i % kRead] = u32x4{x.x, x.y, y.x, y.y};
     };
 #pragma unroll
-    for (int i = 0; i < kAhead; ++i) read_value(i);
+    for (int i = 0; i < kRead; ++i) read_value(i);
     __builtin_amdgcn_sched_barrier(0);
     float p[8], mx = -INFINITY;
 #pragma unroll
@@ -836,12 +840,21 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
       sum += p[i];
     }
     l += sum;
-    const u32x4 pf = {pack_bf16(p[0], p[1]), pack_bf16(p[2], p[3]), pack_bf16(p[4], p[5]), pack_bf16(p[6], p[7])};
+    u32x4 pf, pl;                                                // planes
+#pragma unroll
+    for (int d = 0; d < 4; ++d) {
+      pf[d] = pack_bf16(p[2 * d], p[2 * d + 1]);
+      pl[d] = pack_bf16(p[2 * d] - __uint_as_float(pf[d] << 16), p[2 * d + 1] - __uint_as_float(pf[d] & 0xffff0000u));
+    }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int i = 0; i < VT; ++i) {
-      read_value(i + kAhead);
+    for (int i = 0; i < VT; i += 2) {                            // no product waits for the one before it
       o[i] = mfma_bf16(vf[i % kRead], pf, o[i]);
+      o[i + 1] = mfma_bf16(vf[(i + 1) % kRead], pf, o[i + 1]);
+      o[i] = mfma_bf16(vf[i % kRead], pl, o[i]);
+      o[i + 1] = mfma_bf16(vf[(i + 1) % kRead], pl, o[i + 1]);
+      read_value(i + kRead);
+      read_value(i + 1 + kRead);
       __builtin_amdgcn_sched_barrier(0);
     }
   }
