@@ -363,8 +363,8 @@ extern "C" int zp_qk_norm_rope_store(const void* qkv, void* q_out, void* k_out, 
                         (const void*)query_cache, q_norm_weight, k_norm_weight, (const void*)cos, (const void*)sin})
     wide = wide && (uintptr_t)p % 16 == 0;
   if (wide) {
-    // a workgroup per sixteen vectors (32 + 8 + 8 heads, three times sixteen in brackets: 256 tokens 3.5 us [4.4], 2048
-    // tokens 11.8 [12.0]) until the caches no longer hold them all (8192 tokens 45.1 [41.7])
+    // a workgroup per sixteen vectors (32 + 8 + 8 heads, three times sixteen in brackets: 256 tokens 3.8 us [4.3], 2048
+    // tokens 12.2 [12.4]) until the caches no longer hold them all (8192 tokens 45.0 [41.9])
     const unsigned per = (int64_t)n * total < (1 << 18) ? kVecs : 3 * kVecs, gy = (total + per - 1) / per;
     if (dtype == ZP_BF16)
       hipLaunchKernelGGL((qk_norm_rope_wide_kernel<BF16>), dim3(n, gy), dim3(kThreads), 0, st, a);
