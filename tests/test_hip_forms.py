@@ -62,10 +62,10 @@ def test_compaction_of_the_longest_list(dev, width):
 
 
 # ------------------------------------------------------------------ experts
-# rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup when
-# there are many and tokens come to six per expert; 256-row tiles are worked off whole from a contraction of 2560 on, in
-# two halves below it.  Odd
-# numbers of steps, results that end inside a workgroup's columns, and experts without a token are among them.
+# rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup from six
+# tokens per expert, 40 tiles and 1280 workgroups on; 256-row tiles are worked off whole from a contraction of 2560 on, in
+# two halves below it.  Odd numbers of steps, results that end inside a workgroup's columns, and experts without a token are
+# among them.
 @pytest.mark.parametrize("n,width,E,top,ff", [(60, 96, 64, 2, 800), (61, 2080, 64, 2, 544), (1, 4096, 4, 2, 32),
                                               (260, 160, 4, 1, 288), (1100, 2144, 3, 2, 96), (1100, 96, 2, 1, 2112),
                                               (1300, 256, 2, 1, 96), (515, 2112, 1, 1, 48),
