@@ -61,6 +61,27 @@ def test_compaction_of_the_longest_list(dev, width):
     assert torch.equal(gk.cpu(), wk) and torch.equal(gv.cpu(), wv)
 
 
+# ------------------------------------------------------------------ redundancy inside pages
+# 16-bit caches: workgroups walk whole rows where 512 of them, or a multiple, are at least 90 % full (461 rows on), and
+# take a page each otherwise; fp32 always does.  Same bits for a sequence alone, in a batch that is walked and in one
+# that is not; pages the caller did not list score as none.
+@pytest.mark.parametrize("dtype", [BF16, torch.float16, torch.float32])
+@pytest.mark.parametrize("B", [57, 58, 64, 65, 116])
+def test_redundancy_of_pages_walked_or_alone(dev, dtype, B):
+    from zipage_amd.kernel import lightning_redudancy_score
+    BS, Hkv, D, NB = 64, 8, 32, 3
+    g = torch.Generator().manual_seed(B)
+    pages = torch.randperm(B * NB, generator=g).tolist()
+    enc = O.encode_block_table([[pages.pop() for _ in range(1 + b % NB)] for b in range(B)]).contiguous()
+    k = _rand(1, B * NB, BS, Hkv, D, seed=B, dtype=dtype).to(dev)
+    got = lightning_redudancy_score(k, enc.to(dev))
+    for b in (0, 1, 2, B - 1):
+        alone = lightning_redudancy_score(k, enc[b:b + 1].contiguous().to(dev))
+        assert torch.equal(got[:, b:b + 1], alone)
+    want = O.lightning_redudancy_score(k.cpu()[:, :, :, :1].contiguous(), enc[:3])
+    torch.testing.assert_close(got[:, :3, :1].cpu().float(), want.float(), atol=1e-7, rtol=2.0 ** -6 if dtype != torch.float32 else 1e-4)
+
+
 # ------------------------------------------------------------------ experts
 # rows per tile go by the average expert (16, 32, 64, 128, 256); 16-row tiles take 128 rows of W per workgroup from six
 # tokens per expert, 40 tiles and 1280 workgroups on; 256-row tiles are worked off whole from a contraction of 2560 on, in

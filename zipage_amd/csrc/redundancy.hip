@@ -12,8 +12,8 @@
 //   gram_kernel        fp32 caches, both variants, any page size and table length:
 //                      v_mfma_f32_32x32x2_f32 on keys divided by their norm in fp32, full matrix,
 //                      a wave owns 32 rows for all columns.
-//   gram_page_f32_kernel  fp32 caches, lightning, pages of at most 256 keys: a workgroup walks the
-//                      pages of a row; the normalised page resident in LDS as two fp16 planes per
+//   gram_page_f32_kernel  fp32 caches, lightning, pages of at most 256 keys: one per workgroup; the
+//                      normalised page resident in LDS as two fp16 planes per
 //                      element (fp32-grade products on the 16-bit matrix instructions), one
 //                      barrier, both operands read from that copy, every pair of key blocks once.
 //   gram_raw_sym_f32_kernel  fp32 caches, raw, pages of at most 256 keys and tables of at most 16
@@ -31,6 +31,7 @@
 //                      accumulated in the cache dtype chunk by chunk as the reference does.
 //   red_softmax_kernel claim corrections of the raw variant and the softmax of both.
 #include "common.h"
+#include <algorithm>
 #include <type_traits>
 #include <math.h>
 
@@ -154,6 +155,8 @@ struct GramArgs {
   int B, NB, BS, Hkv, D, num_pages;
   int64_t k_sl, k_sp;
   float threshold, eps;
+  int parts;       // gram_page_kernel: workgroups per row; each walks every parts-th entry of its block table
+  int64_t pages;   // gram_page_f32_kernel: entries of all rows
 };
 
 template <typename T, bool RAW, int NW>
@@ -644,11 +647,12 @@ __global__ __launch_bounds__(kSymWaves * 64) void gram_raw_sym_f32_kernel(GramAr
 }
 
 // ------------------------------------------------------------------ fp32 caches, lightning, whole page in LDS
-// Pages of at most 256 keys; one workgroup per (layer, sequence, head) row walks the row's pages:
-// a page is loaded once with coalesced 16-byte loads into registers (requested under the tiles of
-// the page before), normalised on the way into LDS (132 KB), and after ONE barrier every wave
-// multiplies its 32 rows (A operand read from the same LDS copy) with its share of the column
-// blocks (every unordered pair of blocks once): no tile pipeline, no strided row loads.
+// Pages of at most 256 keys, one per workgroup: loaded once with coalesced 16-byte loads, normalised on the way
+// into LDS (132 KB), and after ONE barrier every wave multiplies its 32 rows (A operand read from the same LDS
+// copy) with its share of the column blocks (every unordered pair of blocks once): no tile pipeline, no strided
+// row loads.  A workgroup per row of pages, which requested the next page under the tiles of this one, was no faster
+// where rows fill the CUs evenly (1024 rows of 9 pages: 497 us, 496 like this) and left them idle everywhere else (320
+// rows: 237 us, 172; 8 rows of 10: 108, 17.5; all with the softmax).
 constexpr int kPage32Rows = 256;
 constexpr int kPage32Threads = 512;
 __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs p) {
@@ -662,62 +666,37 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
   unsigned long long* l_claim = l_corr + kPage32Rows;       // (claimed index + 1) << 32 | value bits
   float* l_sum = (float*)(l_claim + kPage32Rows);
   float* l_csum = l_sum + kPage32Rows;                        // [4][256] column sums per distance
-  int* l_code = (int*)(l_csum + 4 * kPage32Rows);             // [NB] the block table row
 
-  const int tid0 = threadIdx.x;
-  // a workgroup walks the pages of one (layer, sequence, kv head) row: the next page's keys are
-  // requested into registers under the tiles of this one (a page fills the LDS a CU has, so
-  // nothing else could overlap its load)
-  const int h = blockIdx.x % p.Hkv;
-  const int b = (blockIdx.x / p.Hkv) % p.B;
-  const int l = blockIdx.x / (p.Hkv * p.B);
-  const int Tn = p.NB * p.BS;
-  const int64_t rowbase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  // one page of a (layer, sequence, kv head) row; the heads of a page side by side
+#pragma unroll 1
+  for (int64_t at = blockIdx.x; at < p.pages; at += gridDim.x) {
+  const int h = (int)(at % p.Hkv);
+  const int jp = (int)(at / p.Hkv % p.NB);
+  const int b = (int)(at / ((int64_t)p.Hkv * p.NB) % p.B);
+  const int64_t l = at / ((int64_t)p.Hkv * p.NB * p.B);
+  const int64_t obase = (((l * p.B + b) * p.Hkv + h) * p.NB + jp) * p.BS;
   const int dpieces = p.D / 4;
   const int64_t k_row = (int64_t)p.Hkv * p.D * 4;
-  const char* layer = p.k + l * p.k_sl * 4 + (int64_t)h * p.D * 4;
 
-  for (int j = tid0; j < p.NB; j += kPage32Threads) l_code[j] = p.table[(int64_t)b * p.NB + j];
-  __syncthreads();
-  auto page_of = [&](int j) {     // page id of table entry j, or -1 (uniform)
-    const int code = __builtin_amdgcn_readfirstlane(l_code[j]);
-    const int pid = page_is_pad(code) ? -1 : page_id(code);
-    return pid < p.num_pages ? pid : -1;
-  };
-  auto next_valid = [&](int j) {
-    while (j < p.NB && page_of(j) < 0) ++j;
-    return j;
-  };
-  for (int j = 0; j < p.NB; ++j) {      // entries without a page score -inf
-    if (page_of(j) >= 0) continue;
-    for (int s = tid0; s < p.BS; s += kPage32Threads) Elem<T>::st(p.r_out, rowbase + (int64_t)j * p.BS + s, -INFINITY);
+  const int code = p.table[(int64_t)b * p.NB + jp];
+  const int pid = page_is_pad(code) ? -1 : page_id(code);
+  if (pid < 0 || pid >= p.num_pages) {      // an entry without a page scores -inf
+    for (int s = tid; s < p.BS; s += kPage32Threads) Elem<T>::st(p.r_out, obase + s, -INFINITY);
+    continue;
   }
-  float4 raw[ITERS];
-  auto request = [&](int j, int piece, int prow0) {
-    const char* page = layer + (int64_t)page_of(j) * p.k_sp * 4;
+  // ---- stage: norms and the normalised copy of the page
+  {
+    const char* page = p.k + (l * p.k_sl + (int64_t)h * p.D + (int64_t)pid * p.k_sp) * 4;
+    const int piece = tid % PIECES, row0 = tid / PIECES;
+    float4 raw[ITERS];
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-      const int row = it * ROWS_PER_IT + prow0;
+      const int row = it * ROWS_PER_IT + row0;
       raw[it] = *(const float4*)(page + (int64_t)(row < p.BS ? row : 0) * k_row +
                                  (piece < dpieces ? piece : 0) * 16);
     }
-  };
-  int jp = next_valid(0);
-  if (jp < p.NB) request(jp, tid0 % PIECES, tid0 / PIECES);
-#pragma unroll 1
-  while (jp < p.NB) {
-  // The thread id is made opaque once per page: what is derived from it (LDS addresses, row
-  // indices) is then computed where a page uses it, not before the loop and held in registers
-  // through all of it, where the prefetched page needs them.
-  int tid = tid0;
-  asm volatile("" : "+v"(tid));
-  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, col = lane & 31;
-  const int piece = tid % PIECES, prow0 = tid / PIECES;
-  const int64_t obase = rowbase + (int64_t)jp * p.BS;
-  // ---- stage: norms and the normalised copy of the page requested a page ago
-  {
-    const int row0 = prow0;
     if (tid < kPage32Rows) { l_corr[tid] = 0ull; l_claim[tid] = 0ull; }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -735,8 +714,6 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
     }
   }
   __syncthreads();
-  const int nj = next_valid(jp + 1);
-  if (nj < p.NB) request(nj, piece, prow0);
 
   // ---- Gram tiles, every unordered pair of 32-key blocks once: wave a multiplies its block with
   // the blocks (a + d) mod n, d = 0 .. n/2 (the last distance only for the lower half of the
@@ -851,8 +828,7 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
     }
     Elem<T>::st(p.r_out, obase + i, sv - from_fixed32(l_corr[i]));
   }
-  __syncthreads();   // the page and the per-key slots in LDS are free for the next page
-  jp = nj;
+  __syncthreads();   // LDS is free for the next page, where there is one
   }
 }
 
@@ -1231,10 +1207,11 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
   long long st_[10];
   int nst = 0;
 #endif
-  // a workgroup walks the pages of one (layer, sequence, kv head) row
+  // a workgroup walks its share of the pages of one (layer, sequence, kv head) row
   const int h = blockIdx.x % p.Hkv;
-  const int b = (blockIdx.x / p.Hkv) % p.B;
-  const int l = blockIdx.x / (p.Hkv * p.B);
+  const int part = (blockIdx.x / p.Hkv) % p.parts;
+  const int b = (blockIdx.x / (p.Hkv * p.parts)) % p.B;
+  const int l = blockIdx.x / (p.Hkv * p.parts * p.B);
   const int Tn = p.NB * p.BS;
   const int64_t rowbase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
   const float epsr = Elem<T>::rnd(p.eps);
@@ -1256,11 +1233,11 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
     const int pid = page_is_pad(code) ? -1 : page_id(code);
     return pid < p.num_pages ? pid : -1;
   };
-  auto next_valid = [&](int j) {
-    while (j < p.NB && page_of(j) < 0) ++j;
+  auto next_valid = [&](int j) {        // of this workgroup's entries
+    while (j < p.NB && page_of(j) < 0) j += p.parts;
     return j;
   };
-  for (int j = 0; j < p.NB; ++j) {      // entries without a page score -inf
+  for (int j = part; j < p.NB; j += p.parts) {      // entries without a page score -inf
     if (page_of(j) >= 0) continue;
     for (int s = tid; s < p.BS; s += kPageThreads) Elem<T>::st(p.r_out, rowbase + (int64_t)j * p.BS + s, -INFINITY);
   }
@@ -1280,7 +1257,7 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
     }
   };
 
-  int jp = next_valid(0);
+  int jp = next_valid(part);
   if (jp < p.NB) request(jp, __builtin_amdgcn_readfirstlane(tid >> 6), tid & 63);
   int par = 0;
 #pragma unroll 1
@@ -1519,7 +1496,7 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
 
     // ---- nothing below reads the page in LDS: the next page of the row is requested now and
     // lands while this one finishes
-    const int nj = next_valid(jp + 1);
+    const int nj = next_valid(jp + p.parts);
     if (nj < p.NB) request(nj, wave, lane);
 
     // ---- row sums without the matrix: sum_{j != i} e_i.e_j = rn_i (k_i . S) - |e_i|^2, the products
@@ -2541,38 +2518,47 @@ inline bool raw_f32_symmetric(int NB, int BS) {
   return BS <= 256 && BS % TN == 0 && NB / 2 <= kSymMaxDist;
 }
 
+constexpr int64_t kMostPages = 1 << 22;      // workgroups of a launch that has one per page
+
 template <typename T, bool RAW>
 int launch_gram(const GramArgs& a, int L, hipStream_t st) {
   dim3 grid((unsigned)((int64_t)L * a.B * a.Hkv * a.NB));
   const size_t tail = (RAW ? 0 : (size_t)a.BS * 20) + sizeof(int) * 2 * a.NB;
   if constexpr (T::bytes == 2 && !RAW) {
-    // one workgroup per (layer, sequence, kv head) row; the block table row sits in LDS
+    // the block table row sits in LDS
     const size_t smem = (size_t)kPgBytes + 4 * kDmax * 2 + 4 * kPageRows * 2 +
                         (size_t)kPageRows * (2 * 8 + 2 * 4 + 4 + 4) + sizeof(int) * (kPageWaves + a.NB);
     if (a.BS <= kPageRows && a.BS % 32 == 0 && smem <= 80 * 1024) {
-      grid = dim3((unsigned)((int64_t)L * a.B * a.Hkv));
+      // Workgroups walk whole rows where these fill the CUs, two to each, in rounds that are at least 90 % full: a page
+      // then lands while the one before is finished (512 rows of 9 pages: 86 us, 93 with a page each; 1024: 180,
+      // 183).  Otherwise a page each, so that few rows or a thin last round leave no CU idle (8 rows of 10: 49 us by
+      // rows, 13; 256: 63, 51; 768 of 9: 149, 140; all with the softmax).
+      const int64_t rows = (int64_t)L * a.B * a.Hkv, slots = 2 * 256;
+      GramArgs w = a;
+      w.parts = (rows + slots - 1) / slots * slots * 9 <= rows * 10 || rows * a.NB > kMostPages ? 1 : a.NB;
+      grid = dim3((unsigned)(rows * w.parts));
       if (hipFuncSetAttribute((const void*)gram_page_kernel<T>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
         zp_set_error("redundancy: cannot reserve %zu bytes of LDS", smem);
         return ZP_EHIP;
       }
-      hipLaunchKernelGGL((gram_page_kernel<T>), grid, dim3(kPageThreads), smem, st, a);
+      hipLaunchKernelGGL((gram_page_kernel<T>), grid, dim3(kPageThreads), smem, st, w);
       ZP_LAUNCH_CHECK();
       return ZP_OK;
     }
   }
   if constexpr (T::bytes == 4 && !RAW) {
     if (a.BS <= kPage32Rows && a.BS % 32 == 0 && a.NB <= 1024) {
-      // one workgroup per (layer, sequence, kv head) row
-      grid = dim3((unsigned)((int64_t)L * a.B * a.Hkv));
-      const size_t smem = (size_t)kPage32Rows * ROWF * 4 + (size_t)kPage32Rows * (8 + 8 + 4 + 4 * 4) +
-                          sizeof(int) * a.NB;
+      GramArgs w = a;
+      w.pages = (int64_t)L * a.B * a.Hkv * a.NB;
+      grid = dim3((unsigned)std::min(w.pages, kMostPages));
+      const size_t smem = (size_t)kPage32Rows * ROWF * 4 + (size_t)kPage32Rows * (8 + 8 + 4 + 4 * 4);
       if (hipFuncSetAttribute((const void*)gram_page_f32_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
         zp_set_error("redundancy: cannot reserve %zu bytes of LDS", smem);
         return ZP_EHIP;
       }
-      hipLaunchKernelGGL(gram_page_f32_kernel, grid, dim3(kPage32Threads), smem, st, a);
+      hipLaunchKernelGGL(gram_page_f32_kernel, grid, dim3(kPage32Threads), smem, st, w);
       ZP_LAUNCH_CHECK();
       return ZP_OK;
     }
