@@ -12,8 +12,8 @@
 //   gram_kernel        fp32 caches, both variants, any page size and table length:
 //                      v_mfma_f32_32x32x2_f32 on keys divided by their norm in fp32, full matrix,
 //                      a wave owns 32 rows for all columns.
-//   gram_page_f32_kernel  fp32 caches, lightning, pages of at most 256 keys: one per workgroup; the
-//                      normalised page resident in LDS as two fp16 planes per
+//   gram_page_f32_kernel  fp32 caches, lightning, pages of at most 256 keys: a workgroup walks its share of
+//                      the pages of a row; the normalised page resident in LDS as two fp16 planes per
 //                      element (fp32-grade products on the 16-bit matrix instructions), one
 //                      barrier, both operands read from that copy, every pair of key blocks once.
 //   gram_raw_sym_f32_kernel  fp32 caches, raw, pages of at most 256 keys and tables of at most 16
@@ -31,7 +31,6 @@
 //                      accumulated in the cache dtype chunk by chunk as the reference does.
 //   red_softmax_kernel claim corrections of the raw variant and the softmax of both.
 #include "common.h"
-#include <algorithm>
 #include <type_traits>
 #include <math.h>
 
@@ -155,8 +154,7 @@ struct GramArgs {
   int B, NB, BS, Hkv, D, num_pages;
   int64_t k_sl, k_sp;
   float threshold, eps;
-  int parts;       // gram_page_kernel: workgroups per row; each walks every parts-th entry of its block table
-  int64_t pages;   // gram_page_f32_kernel: entries of all rows
+  int parts;       // the page kernels: workgroups per row; each walks every parts-th entry of its block table
 };
 
 template <typename T, bool RAW, int NW>
@@ -647,12 +645,11 @@ __global__ __launch_bounds__(kSymWaves * 64) void gram_raw_sym_f32_kernel(GramAr
 }
 
 // ------------------------------------------------------------------ fp32 caches, lightning, whole page in LDS
-// Pages of at most 256 keys, one per workgroup: loaded once with coalesced 16-byte loads, normalised on the way
-// into LDS (132 KB), and after ONE barrier every wave multiplies its 32 rows (A operand read from the same LDS
-// copy) with its share of the column blocks (every unordered pair of blocks once): no tile pipeline, no strided
-// row loads.  A workgroup per row of pages, which requested the next page under the tiles of this one, was no faster
-// where rows fill the CUs evenly (1024 rows of 9 pages: 497 us, 496 like this) and left them idle everywhere else (320
-// rows: 237 us, 172; 8 rows of 10: 108, 17.5; all with the softmax).
+// Pages of at most 256 keys; a workgroup walks its share of the pages of a (layer, sequence, head) row:
+// a page is loaded once with coalesced 16-byte loads into registers (requested under the tiles of
+// the page before), normalised on the way into LDS (132 KB), and after ONE barrier every wave
+// multiplies its 32 rows (A operand read from the same LDS copy) with its share of the column
+// blocks (every unordered pair of blocks once): no tile pipeline, no strided row loads.
 constexpr int kPage32Rows = 256;
 constexpr int kPage32Threads = 512;
 __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs p) {
@@ -666,37 +663,63 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
   unsigned long long* l_claim = l_corr + kPage32Rows;       // (claimed index + 1) << 32 | value bits
   float* l_sum = (float*)(l_claim + kPage32Rows);
   float* l_csum = l_sum + kPage32Rows;                        // [4][256] column sums per distance
+  int* l_code = (int*)(l_csum + 4 * kPage32Rows);             // [NB] the block table row
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int half = lane >> 5, col = lane & 31;
-  // one page of a (layer, sequence, kv head) row; the heads of a page side by side
-#pragma unroll 1
-  for (int64_t at = blockIdx.x; at < p.pages; at += gridDim.x) {
-  const int h = (int)(at % p.Hkv);
-  const int jp = (int)(at / p.Hkv % p.NB);
-  const int b = (int)(at / ((int64_t)p.Hkv * p.NB) % p.B);
-  const int64_t l = at / ((int64_t)p.Hkv * p.NB * p.B);
-  const int64_t obase = (((l * p.B + b) * p.Hkv + h) * p.NB + jp) * p.BS;
+  const int tid0 = threadIdx.x;
+  // a workgroup walks the pages of one (layer, sequence, kv head) row: the next page's keys are
+  // requested into registers under the tiles of this one (a page fills the LDS a CU has, so
+  // nothing else could overlap its load)
+  const int h = blockIdx.x % p.Hkv;
+  const int part = (blockIdx.x / p.Hkv) % p.parts;
+  const int b = (blockIdx.x / (p.Hkv * p.parts)) % p.B;
+  const int l = blockIdx.x / (p.Hkv * p.parts * p.B);
+  const int Tn = p.NB * p.BS;
+  const int64_t rowbase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
   const int dpieces = p.D / 4;
   const int64_t k_row = (int64_t)p.Hkv * p.D * 4;
+  const char* layer = p.k + l * p.k_sl * 4 + (int64_t)h * p.D * 4;
 
-  const int code = p.table[(int64_t)b * p.NB + jp];
-  const int pid = page_is_pad(code) ? -1 : page_id(code);
-  if (pid < 0 || pid >= p.num_pages) {      // an entry without a page scores -inf
-    for (int s = tid; s < p.BS; s += kPage32Threads) Elem<T>::st(p.r_out, obase + s, -INFINITY);
-    continue;
+  for (int j = tid0; j < p.NB; j += kPage32Threads) l_code[j] = p.table[(int64_t)b * p.NB + j];
+  __syncthreads();
+  auto page_of = [&](int j) {     // page id of table entry j, or -1 (uniform)
+    const int code = __builtin_amdgcn_readfirstlane(l_code[j]);
+    const int pid = page_is_pad(code) ? -1 : page_id(code);
+    return pid < p.num_pages ? pid : -1;
+  };
+  auto next_valid = [&](int j) {        // of this workgroup's entries
+    while (j < p.NB && page_of(j) < 0) j += p.parts;
+    return j;
+  };
+  for (int j = part; j < p.NB; j += p.parts) {      // entries without a page score -inf
+    if (page_of(j) >= 0) continue;
+    for (int s = tid0; s < p.BS; s += kPage32Threads) Elem<T>::st(p.r_out, rowbase + (int64_t)j * p.BS + s, -INFINITY);
   }
-  // ---- stage: norms and the normalised copy of the page
-  {
-    const char* page = p.k + (l * p.k_sl + (int64_t)h * p.D + (int64_t)pid * p.k_sp) * 4;
-    const int piece = tid % PIECES, row0 = tid / PIECES;
-    float4 raw[ITERS];
+  float4 raw[ITERS];
+  auto request = [&](int j, int piece, int prow0) {
+    const char* page = layer + (int64_t)page_of(j) * p.k_sp * 4;
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
-      const int row = it * ROWS_PER_IT + row0;
+      const int row = it * ROWS_PER_IT + prow0;
       raw[it] = *(const float4*)(page + (int64_t)(row < p.BS ? row : 0) * k_row +
                                  (piece < dpieces ? piece : 0) * 16);
     }
+  };
+  int jp = next_valid(part);
+  if (jp < p.NB) request(jp, tid0 % PIECES, tid0 / PIECES);
+#pragma unroll 1
+  while (jp < p.NB) {
+  // The thread id is made opaque once per page: what is derived from it (LDS addresses, row
+  // indices) is then computed where a page uses it, not before the loop and held in registers
+  // through all of it, where the prefetched page needs them.
+  int tid = tid0;
+  asm volatile("" : "+v"(tid));
+  const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int half = lane >> 5, col = lane & 31;
+  const int piece = tid % PIECES, prow0 = tid / PIECES;
+  const int64_t obase = rowbase + (int64_t)jp * p.BS;
+  // ---- stage: norms and the normalised copy of the page requested a page ago
+  {
+    const int row0 = prow0;
     if (tid < kPage32Rows) { l_corr[tid] = 0ull; l_claim[tid] = 0ull; }
 #pragma unroll
     for (int it = 0; it < ITERS; ++it) {
@@ -714,6 +737,8 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
     }
   }
   __syncthreads();
+  const int nj = next_valid(jp + p.parts);
+  if (nj < p.NB) request(nj, piece, prow0);
 
   // ---- Gram tiles, every unordered pair of 32-key blocks once: wave a multiplies its block with
   // the blocks (a + d) mod n, d = 0 .. n/2 (the last distance only for the lower half of the
@@ -828,7 +853,8 @@ __global__ __launch_bounds__(kPage32Threads) void gram_page_f32_kernel(GramArgs 
     }
     Elem<T>::st(p.r_out, obase + i, sv - from_fixed32(l_corr[i]));
   }
-  __syncthreads();   // LDS is free for the next page, where there is one
+  __syncthreads();   // the page and the per-key slots in LDS are free for the next page
+  jp = nj;
   }
 }
 
@@ -2518,7 +2544,17 @@ inline bool raw_f32_symmetric(int NB, int BS) {
   return BS <= 256 && BS % TN == 0 && NB / 2 <= kSymMaxDist;
 }
 
-constexpr int64_t kMostPages = 1 << 22;      // workgroups of a launch that has one per page
+// Workgroups of the page kernels, `per_cu` of which a CU holds, walk whole rows where these fill the CUs in rounds that are at
+// least 90 % full: a page then lands while the one before is finished (512 16-bit rows of 9 pages: 86 us, 93 with a page
+// each; 1024 fp32 rows: 435, 486).  Otherwise a page each, so that few rows or a thin last round leave no CU idle (8 rows of
+// 10 pages: 49 us by rows, 13, fp32 108, 18; 768 16-bit rows of 9: 149, 140; 320 fp32 rows: 237, 172; all but the 435 and 486
+// with the softmax).
+GramArgs page_walks(GramArgs a, int L, int per_cu) {
+  const int64_t rows = (int64_t)L * a.B * a.Hkv, slots = 256 * per_cu;
+  const bool walk = (rows + slots - 1) / slots * slots * 9 <= rows * 10 || rows * a.NB > (1 << 22);
+  a.parts = walk ? 1 : a.NB;
+  return a;
+}
 
 template <typename T, bool RAW>
 int launch_gram(const GramArgs& a, int L, hipStream_t st) {
@@ -2529,14 +2565,8 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
     const size_t smem = (size_t)kPgBytes + 4 * kDmax * 2 + 4 * kPageRows * 2 +
                         (size_t)kPageRows * (2 * 8 + 2 * 4 + 4 + 4) + sizeof(int) * (kPageWaves + a.NB);
     if (a.BS <= kPageRows && a.BS % 32 == 0 && smem <= 80 * 1024) {
-      // Workgroups walk whole rows where these fill the CUs, two to each, in rounds that are at least 90 % full: a page
-      // then lands while the one before is finished (512 rows of 9 pages: 86 us, 93 with a page each; 1024: 180,
-      // 183).  Otherwise a page each, so that few rows or a thin last round leave no CU idle (8 rows of 10: 49 us by
-      // rows, 13; 256: 63, 51; 768 of 9: 149, 140; all with the softmax).
-      const int64_t rows = (int64_t)L * a.B * a.Hkv, slots = 2 * 256;
-      GramArgs w = a;
-      w.parts = (rows + slots - 1) / slots * slots * 9 <= rows * 10 || rows * a.NB > kMostPages ? 1 : a.NB;
-      grid = dim3((unsigned)(rows * w.parts));
+      const GramArgs w = page_walks(a, L, 2);
+      grid = dim3((unsigned)((int64_t)L * a.B * a.Hkv * w.parts));
       if (hipFuncSetAttribute((const void*)gram_page_kernel<T>,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
         zp_set_error("redundancy: cannot reserve %zu bytes of LDS", smem);
@@ -2549,10 +2579,10 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
   }
   if constexpr (T::bytes == 4 && !RAW) {
     if (a.BS <= kPage32Rows && a.BS % 32 == 0 && a.NB <= 1024) {
-      GramArgs w = a;
-      w.pages = (int64_t)L * a.B * a.Hkv * a.NB;
-      grid = dim3((unsigned)std::min(w.pages, kMostPages));
-      const size_t smem = (size_t)kPage32Rows * ROWF * 4 + (size_t)kPage32Rows * (8 + 8 + 4 + 4 * 4);
+      const GramArgs w = page_walks(a, L, 1);
+      grid = dim3((unsigned)((int64_t)L * a.B * a.Hkv * w.parts));
+      const size_t smem = (size_t)kPage32Rows * ROWF * 4 + (size_t)kPage32Rows * (8 + 8 + 4 + 4 * 4) +
+                          sizeof(int) * a.NB;
       if (hipFuncSetAttribute((const void*)gram_page_f32_kernel,
                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
         zp_set_error("redundancy: cannot reserve %zu bytes of LDS", smem);
