@@ -61,6 +61,25 @@ def test_compaction_of_the_longest_list(dev, width):
     assert torch.equal(gk.cpu(), wk) and torch.equal(gv.cpu(), wv)
 
 
+# ------------------------------------------------------------------ attention scores
+# pages of 256 tokens with groups of two or four heads and a mean over the window have forms of their own; the same
+# tokens in pages of 128 take the general one: same bits.
+@pytest.mark.parametrize("dtype", [BF16, torch.float16, torch.float32])
+@pytest.mark.parametrize("group,W", [(2, 32), (2, 16), (2, 5), (4, 32), (3, 20)])
+def test_scores_by_page_size_and_group(dev, dtype, group, W):
+    from zipage_amd.kernel import attention_score
+    B, Hkv, D, P = 3, 2, 128, 9
+    g = torch.Generator().manual_seed(group * 64 + W)
+    pages = torch.randperm(P, generator=g).tolist()
+    tables = [[pages.pop() for _ in range(n)] for n in (4, 3, 1)]
+    k, q = _rand(1, P, 256, Hkv, D, seed=W, dtype=dtype).to(dev), _rand(1, B, W, group * Hkv, D, seed=W + 1, dtype=dtype).to(dev)
+    seq = torch.arange(B, dtype=torch.int32, device=dev)
+    whole, halves = (O.encode_block_table(t).to(dev) for t in (tables, [[2 * p + i for p in t for i in (0, 1)] for t in tables]))
+    got = attention_score(k, q, seq, whole)
+    want = attention_score(k.view(1, 2 * P, 128, Hkv, D), q, seq, halves)
+    assert torch.equal(got.reshape(want.shape), want)
+
+
 # ------------------------------------------------------------------ redundancy inside pages
 # 16-bit caches: workgroups walk whole rows where 512 of them, or a multiple, are at least 90 % full (461 rows on), and
 # take a page each otherwise; fp32 always does.  Same bits for a sequence alone, in a batch that is walked and in one

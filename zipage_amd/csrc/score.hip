@@ -1579,10 +1579,13 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
     const size_t smem = (size_t)kWaves * 2 * kSubBytes + sizeof(float) * kWaves * 32;
     const unsigned units = (unsigned)(((int64_t)a.n_items + 7) / 8 * 8 * RB);
     const dim3 cgrid((unsigned)a.n_items, (unsigned)((NB * BS / 4 + 255) / 256));
+    // The common groups get straight-line epilogues (groups of two, window 32, the whole compression step: 1 sequence
+    // 53 -> 42 us, 64 sequences 330 -> 312, 200 1039 -> 1009).
 #define ZP_RESIDENT_LAUNCH(TT)                                                                   \
   do {                                                                                           \
     void (*fn)(ScoreArgs) = score_resident_kernel<TT, 0, -1, 0>;                                 \
     if (Gp == 4 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 4, 0, 2>;          \
+    else if (Gp == 2 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 2, 0, 2>;     \
     if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,         \
                             (int)smem) != hipSuccess) {                                          \
       zp_set_error("attention_score: cannot reserve %zu bytes of LDS", smem);                    \
