@@ -63,7 +63,9 @@ int zp_store_query(const void* query, void* query_cache, const int32_t* slot_map
  * (zp_attention_score_workspace(): the upper bound over the dtypes).  With no logits_out, a
  * positive scale and at most 2560 tokens per sequence that scratch lets the library keep the
  * logits in registers and sweep K once (fp32 window partials per block of 32 query rows -- 16
- * for fp32 caches -- go through the scratch); with less scratch (NULL is fine up to 128 window x
+ * for fp32 caches -- go through the scratch); zp_attention_score_workspace_few(..., dtype) bytes,
+ * which are more for calls with at most 64 such blocks, let it spread a block's tokens over the
+ * chip, with the same bits; with less scratch (NULL is fine up to 128 window x
  * group rows) the same entry point sweeps K three times (twice for fp32 caches).  The kernels
  * round at the same points and differ only in the fp32 order of the row sums (fp32 caches: also
  * in the last bit of the probabilities, e / sum against 2^(x log2 e - log2 sum)). */
@@ -78,6 +80,8 @@ int zp_attention_score(const void* k_cache, const void* query_cache, const int32
 int64_t zp_attention_score_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                      int32_t Hkv, int32_t Hq, int32_t W);
 int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_t NB, int32_t BS,
+                                         int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype);
+int64_t zp_attention_score_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                          int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype);
 
 /* global_score(reduced_scores, score_cache, block_table, compressed, decay_factor,

@@ -80,6 +80,29 @@ def test_scores_by_page_size_and_group(dev, dtype, group, W):
     assert torch.equal(got.reshape(want.shape), want)
 
 
+# up to 64 blocks of query rows (32, fp32: 16) have their tiles side by side, more walk them: same bits for a sequence alone and
+# in a batch, and where the scratch holds only what the walk needs.
+@pytest.mark.parametrize("dtype", [BF16, torch.float16, torch.float32])
+@pytest.mark.parametrize("group,W,BS,D,reduced,B", [(1, 32, 256, 128, "mean", 65), (2, 16, 256, 128, "mean", 65), (3, 9, 128, 64, "mean", 65),
+                                                    (4, 32, 256, 96, "max", 17), (8, 5, 256, 128, "mean", 33), (8, 3, 128, 40, "max", 65),
+                                                    (16, 4, 128, 128, "mean", 33), (1, 20, 128, 128, "max", 65)])
+def test_scores_of_few_sequences(dev, dtype, group, W, BS, D, reduced, B):
+    from zipage_amd import _lib
+    from zipage_amd.kernel import attention_score
+    NB = 6
+    g = torch.Generator().manual_seed(group * 64 + W)
+    pages = torch.randperm(B * NB, generator=g).tolist()
+    enc = O.encode_block_table([[pages.pop() for _ in range(NB - b % 5)] for b in range(B)])
+    k, q = _rand(1, B * NB, BS, 1, D, seed=W, dtype=dtype, std=2.0).to(dev), _rand(1, B, W, group, D, seed=W + 1, dtype=dtype).to(dev)
+    seq = torch.randperm(B, generator=g).int().to(dev)
+    many = attention_score(k, q, seq, enc.to(dev), reduced=reduced)
+    for n in (1, 3):
+        few = attention_score(k, q, seq[:n].contiguous(), enc[:n].contiguous().to(dev), reduced=reduced)
+        assert torch.equal(few, many[:, :n])
+    want = O.attention_score(k[:, :, :, :, :].cpu(), q.cpu(), seq[:3].cpu(), enc[:3], reduced=reduced)
+    torch.testing.assert_close(many[:, :3].cpu().float(), want.float(), rtol=2.0 ** -6 if dtype != torch.float32 else 1e-4, atol=1e-6)
+
+
 # ------------------------------------------------------------------ redundancy inside pages
 # 16-bit caches: workgroups walk whole rows where 512 of them, or a multiple, are at least 90 % full (461 rows on), and
 # take a page each otherwise; fp32 always does.  Same bits for a sequence alone, in a batch that is walked and in one

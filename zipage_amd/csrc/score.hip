@@ -5,13 +5,14 @@
 // to the cache dtype), so bf16/fp16 results agree with it to the last bit except where fp32
 // accumulation order moves a value across a rounding boundary.
 //
-// Three kernels:
+// Kernels:
 //   score_resident_kernel  16-bit caches, at most 2560 tokens per sequence, no logits requested:
 //       ONE sweep over K.  A workgroup is one block of 32 query rows of a (layer, sequence, head);
 //       its rounded logits stay in registers (two per word) and the row maximum, the row sum and
 //       the output come from the registers.  Described above the kernel.
 //   score_resident_f32_kernel  the same for fp32 caches: blocks of 16 query rows, one fp32 logit
 //       per register, v_mfma_f32_16x16x4_f32.  Described above the kernel.
+//   score_tiles_kernel, score_rows_kernel  the work of those two spread out where there are few blocks of rows.
 //   score_kernel           everything else (longer sequences, logits, no scratch):
 //       one workgroup per (layer, sequence, kv head).  The softmax normaliser spans the whole
 //       sequence, so it makes three passes over the sequence's pages, recomputing QK^T each time:
@@ -31,6 +32,7 @@
 // one cross-half step; the row blocks' shares meet in LDS (score_kernel: wave v owns row block v,
 // tiles of 128 or 64 tokens are shared by all waves) or in the scratch (score_resident_kernel).
 #include "common.h"
+#include <algorithm>
 #include <math.h>
 #include <type_traits>
 
@@ -88,7 +90,9 @@ struct ScoreArgs {
   int RB;  // row blocks of 32
   int gs;  // log2(Gp)
   int RW;  // waves along the row axis: 1, 2 or 4
-  float* part;    // register-resident kernel: fp32 window partials (L*B*Hkv, RB, NB*BS)
+  float* part;    // register-resident kernels: fp32 window partials (L*B*Hkv, RB, NB*BS)
+  void* lg;       // tiles side by side: the logits
+  int tiles;      // and the tiles of a full table
   int n_items;    // L*B*Hkv
 };
 
@@ -832,6 +836,21 @@ __device__ __forceinline__ float group_window_reduce(float (&pv)[16], int Gp, bo
   return red;
 }
 
+// Every wave builds the list of usable pages for itself (no LDS, no barrier): `code` is table entry `lane`, a ballot ranks
+// the usable ones, and a lane permute leaves entry n of the list in lane n as (page id, table index | last << 30).  Returns
+// their number.
+__device__ __forceinline__ int list_pages(int code, int num_pages, int2& mine) {
+  const int lane = threadIdx.x & 63;
+  const int pid = page_is_pad(code) ? -1 : page_id(code);
+  const bool ok = pid >= 0 && pid < num_pages;
+  const unsigned long long okm = __builtin_amdgcn_ballot_w64(ok);
+  const int n = __builtin_popcountll(okm);
+  const int dst = ok ? __builtin_popcountll(okm & lanemask_lt()) : n + __builtin_popcountll(~okm & lanemask_lt());
+  mine.x = __builtin_amdgcn_ds_permute(dst << 2, pid);
+  mine.y = __builtin_amdgcn_ds_permute(dst << 2, lane | (page_is_last(code) ? (1 << 30) : 0));
+  return n;
+}
+
 // TPP: 128-token tiles per page when known at compile time (0: from the arguments); with it
 // the page of every unrolled tile is a constant and its id comes from a lane of a register.
 template <typename T, int GPC, int RMAXC, int TPP>
@@ -874,23 +893,10 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   const int l = item / (p.Hkv * p.B);
   const int Tn = p.NB * p.BS;
 
-  // Every wave builds the list of usable pages for itself (no LDS, no barrier): lane j reads table
-  // entry j, a ballot ranks the usable ones, and a lane permute leaves entry n of the list in lane
-  // n as (page id, table index | last << 30).
   const int code = lane < p.NB ? p.table[(int64_t)b * p.NB + lane] : -1;
   int seq = p.seq_idx[b];
   int2 myinfo;
-  int nvalid;
-  {
-    const int pid = page_is_pad(code) ? -1 : page_id(code);
-    const bool ok = pid >= 0 && pid < p.num_pages;
-    const unsigned long long okm = __builtin_amdgcn_ballot_w64(ok);
-    nvalid = __builtin_popcountll(okm);
-    const int dst = ok ? __builtin_popcountll(okm & lanemask_lt())
-                       : nvalid + __builtin_popcountll(~okm & lanemask_lt());
-    myinfo.x = __builtin_amdgcn_ds_permute(dst << 2, pid);
-    myinfo.y = __builtin_amdgcn_ds_permute(dst << 2, lane | (page_is_last(code) ? (1 << 30) : 0));
-  }
+  const int nvalid = list_pages(code, p.num_pages, myinfo);
   const int dpieces = p.D * T::bytes / 16;
   char* kb = smem + wave * 2 * kSubBytes;    // this wave's two K blocks
   if (dpieces < 16) {   // the tail of every staged row must read as zero
@@ -1160,21 +1166,10 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_f32_kernel(ScoreAr
   const int l = item / (p.Hkv * p.B);
   const int Tn = p.NB * p.BS;
 
-  // per-wave list of usable pages: entry n in lane n as (page id, table index | last << 30)
   const int code = lane < p.NB ? p.table[(int64_t)b * p.NB + lane] : -1;
   int seq = p.seq_idx[b];
   int2 myinfo;
-  int nvalid;
-  {
-    const int pid = page_is_pad(code) ? -1 : page_id(code);
-    const bool ok = pid >= 0 && pid < p.num_pages;
-    const unsigned long long okm = __builtin_amdgcn_ballot_w64(ok);
-    nvalid = __builtin_popcountll(okm);
-    const int dst = ok ? __builtin_popcountll(okm & lanemask_lt())
-                       : nvalid + __builtin_popcountll(~okm & lanemask_lt());
-    myinfo.x = __builtin_amdgcn_ds_permute(dst << 2, pid);
-    myinfo.y = __builtin_amdgcn_ds_permute(dst << 2, lane | (page_is_last(code) ? (1 << 30) : 0));
-  }
+  const int nvalid = list_pages(code, p.num_pages, myinfo);
   const int dpieces = p.D / 4;               // 16-byte pieces of a key row
   char* kb = smem + wave * 2 * kF32Sub;      // this wave's two key blocks
   if (dpieces < 32) {   // the tail of every staged row must read as zero
@@ -1392,14 +1387,262 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_f32_kernel(ScoreAr
   }
 }
 
+// ------------------------------------------------------------------ few sequences: tiles side by side
+// A unit of the kernels above walks up to 20 (fp32: 40) tiles one after the other, 24 (33) us however few units there are.
+// With few of them the same arithmetic is spread out: score_tiles has a workgroup per tile of an item and leaves the
+// logits of all its units in the scratch, score_rows has four workgroups per unit with a quarter of its rows each (a lane's four rows of a
+// 16-bit unit; a lane group's four of an fp32 one) and leaves the quarters' window sums, which score_combine adds up as
+// the kernels above do.  Every sum has the same terms in the same order, so the bits are theirs.
+// Logits [unit][quarter][wave][tile][64 lanes], 8 bytes a lane (two rounded pairs) or 4 (a row of 16 tokens each).
+template <typename T> struct Tiles;            // tokens of a tile, tiles of a row
+template <> struct Tiles<BF16> { static constexpr int tokens = 128, most = kResTiles; };
+template <> struct Tiles<F16> { static constexpr int tokens = 128, most = kResTiles; };
+template <> struct Tiles<F32> { static constexpr int tokens = 64, most = kF32Tiles; };
+
+// What both kernels ask of a unit: its place and its pages.
+template <typename T, int TPP> struct TiledUnit {
+  int item, h, b, l, n, tpp;                   // n: tiles of the sequence; tpp: of a page (TPP, where that is not 0)
+  int2 pages;
+  __device__ __forceinline__ TiledUnit(const ScoreArgs& p, int item_) {
+    item = item_;
+    const int row = item / p.Hkv;
+    h = item - row * p.Hkv;
+    l = row / p.B;
+    b = row - l * p.B;
+    tpp = TPP > 0 ? TPP : p.BS / Tiles<T>::tokens;
+    const int lane = threadIdx.x & 63;
+    n = list_pages(lane < p.NB ? p.table[(int64_t)b * p.NB + lane] : -1, p.num_pages, pages) * tpp;
+  }
+  __device__ __forceinline__ int page_of(int tile) const { return __builtin_amdgcn_readlane(pages.x, tile / tpp); }
+  __device__ __forceinline__ int place_of(int tile) const { return __builtin_amdgcn_readlane(pages.y, tile / tpp); }
+  __device__ __forceinline__ int first_token(int tile) const { return tile % tpp * Tiles<T>::tokens; }
+};
+
+template <typename T, int TPP> __global__ __launch_bounds__(kThreads) void score_tiles_kernel(ScoreArgs p) {
+  typedef Mma<T> M;
+  __shared__ __align__(16) char smem[T::bytes == 2 ? kWaves * kSubBytes : 16];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int rb = blockIdx.y, unit = blockIdx.z * p.RB + rb, it = blockIdx.x;
+  const TiledUnit<T, TPP> u(p, blockIdx.z);
+  int seq = p.seq_idx[u.b];
+  const bool seq_ok = seq >= 0 && seq < p.max_seqs;
+  if (!seq_ok) seq = 0;
+  if (it >= u.n) return;
+  constexpr int kRows = T::bytes == 2 ? 32 : 16, kWaveTokens = Tiles<T>::tokens / kWaves;
+  const int col = lane % kRows, g = lane / kRows;      // query row and token of this lane; its half or lane group
+  const int64_t k_row = (int64_t)p.Hkv * p.D * T::bytes;
+  const int toff = u.first_token(it) + wave * kWaveTokens;
+  const char* const keys = p.k + (u.l * p.k_sl + (int64_t)u.h * p.D + (int64_t)u.page_of(it) * p.k_sp) * T::bytes + toff * k_row;
+  const int mrow = rb * kRows + col, a_w = mrow >> p.gs, a_g = mrow & (p.Gp - 1);
+  const bool a_ok = seq_ok && a_w < p.W && a_g < p.G;
+  const char* const qrow = p.q + ((int64_t)u.l * p.q_sl + (int64_t)seq * p.q_ss +
+                                  ((int64_t)a_w * p.Hq + (int64_t)u.h * p.G + a_g) * p.D) * T::bytes;
+  // causal mask: tail of the last page
+  const bool masked = ((u.place_of(it) >> 30) & 1) && toff + kWaveTokens - 1 > p.BS - p.W;
+  const int slot = toff + col - (p.BS - p.W);          // windows below it do not see this token
+  const int64_t quarter = (int64_t)kWaves * p.tiles * 64;      // lanes' words of a quarter
+  const int64_t at = (int64_t)unit * 4 * quarter + ((int64_t)wave * p.tiles + it) * 64;
+  if constexpr (T::bytes == 2) {
+    typedef typename M::Frag Frag;
+    char* const kb = smem + wave * kSubBytes;          // as in the kernel above: pieces of four rows, 1040 bytes apart
+    const int dpieces = p.D * 2 / 16;
+    if (dpieces < 16) {
+      for (int i = lane; i < kSubBytes / 4; i += 64) ((uint32_t*)kb)[i] = 0u;
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    }
+    const int st_g = (lane >> 4) * 4 + (lane & 3), st_r = (lane >> 2) & 3;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)keys, 0, (int)(32 * k_row), 0x00020000);
+    typedef void __attribute__((address_space(3))) * lptr_t;
+    if (st_g < dpieces) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lptr_t)(kb + i * kGrp), 16, (int)(st_r * k_row + st_g * 16),
+                                                 i * (int)(4 * k_row), 0, 0);
+    }
+    Frag q[M::KS];
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) {
+      const int k0 = s * M::KPI + g * M::EPL;
+      if (a_ok && k0 < p.D) q[s] = *(const Frag*)(qrow + (int64_t)k0 * 2);
+      else zero_frag<T>(q[s]);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const char* const cur = kb + (col >> 2) * kGrp + (col & 3) * 64 + g * 16;
+    f32x16_t acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+#pragma unroll
+    for (int s = 0; s < M::KS; ++s) acc = M::mma(q[s], *(const Frag*)(cur + (s >> 1) * 256 + (s & 1) * 32), acc);
+    uint2* const dst = (uint2*)p.lg + at + lane;
+#pragma unroll
+    for (int v = 0; v < 4; ++v) {
+      uint32_t w[2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int r = 4 * v + 2 * i, row = rb * 32 + 8 * v + 4 * g + 2 * i;
+        if (masked && slot > (row >> p.gs)) acc[r] = -INFINITY;
+        if (masked && slot > ((row + 1) >> p.gs)) acc[r + 1] = -INFINITY;
+        w[i] = Pack2<T>::pack(acc[r] * p.scale, acc[r + 1] * p.scale);
+      }
+      dst[v * quarter] = make_uint2(w[0], w[1]);
+    }
+  } else {
+    f32x4_t q[8], k[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      const int k0 = 16 * j + 4 * g;
+      const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+      k[j] = k0 < p.D ? *(const f32x4_t*)(keys + col * k_row + (int64_t)k0 * 4) : zero;
+      q[j] = a_ok && k0 < p.D ? *(const f32x4_t*)(qrow + (int64_t)k0 * 4) : zero;
+    }
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(q[j][i], k[j][i], acc, 0, 0, 0);
+    float* const dst = (float*)p.lg + at + g * quarter + col;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      if (masked && slot > ((rb * 16 + 4 * g + r) >> p.gs)) acc[r] = -INFINITY;
+      dst[r * 16] = acc[r] * p.scale;
+    }
+  }
+}
+
+template <typename T, int TPP> __global__ __launch_bounds__(kThreads) void score_rows_kernel(ScoreArgs p) {
+  __shared__ float stat[2][kWaves][8];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int v = blockIdx.x, rb = blockIdx.y, unit = blockIdx.z * p.RB + rb;
+  const TiledUnit<T, TPP> u(p, blockIdx.z);
+  constexpr int NT = Tiles<T>::most, kRows = T::bytes == 2 ? 4 : 1;      // rows of a lane
+  const bool rmax = p.reduce_max != 0;
+  // lanes of a row: 32 that hold four rows, or 16 that hold one
+  const int g = T::bytes == 2 ? lane >> 5 : lane >> 4, col = T::bytes == 2 ? lane & 31 : lane & 15;
+  const int row0 = T::bytes == 2 ? rb * 32 + 8 * v + 4 * g : rb * 16 + 4 * v + g;
+  typedef typename std::conditional<T::bytes == 2, uint2, float>::type Word;
+  Word lg[NT];
+  {
+    const Word* const src = (const Word*)p.lg + (((int64_t)unit * 4 + v) * kWaves + wave) * p.tiles * 64 + lane;
+#pragma unroll
+    for (int it = 0; it < NT; ++it)           // all that there is room for: nothing waits for the table
+      if (it < p.tiles) lg[it] = src[it * 64];
+  }
+  float run[kRows], mx[kRows], last[kRows];
+  // what a wave found for its rows meets in LDS; the waves' shares are taken in their order, whichever wave does it
+  auto share = [&](int n, const float (&x)[kRows]) {
+    if (col == 0)
+#pragma unroll
+      for (int r = 0; r < kRows; ++r) stat[n][wave][g * kRows + r] = x[r];
+    __syncthreads();
+  };
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) run[r] = -INFINITY;
+#pragma unroll
+  for (int it = 0; it < NT; ++it) {
+    if (it < u.n) {
+      if constexpr (T::bytes == 2) {
+        run[0] = vmax(run[0], Pack2<T>::lo(lg[it].x));
+        run[1] = vmax(run[1], Pack2<T>::hi(lg[it].x));
+        run[2] = vmax(run[2], Pack2<T>::lo(lg[it].y));
+        run[3] = vmax(run[3], Pack2<T>::hi(lg[it].y));
+      } else {
+        run[0] = vmax(run[0], lg[it]);
+      }
+    }
+  }
+  // rounding and a positive factor keep the order: the largest rounded logit is the rounded largest
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) run[r] = T::bytes == 2 ? half_max(run[r]) : row16_max(run[r]);
+  share(0, run);
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    mx[r] = run[r];
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) mx[r] = fmaxf(mx[r], stat[0][w][g * kRows + r]);
+    run[r] = 0.f;
+  }
+#pragma unroll
+  for (int it = 0; it < NT; ++it) {
+    if (it < u.n) {
+      if constexpr (T::bytes == 2) {
+        const uint32_t a = Pack2<T>::pack(Pack2<T>::lo(lg[it].x) - mx[0], Pack2<T>::hi(lg[it].x) - mx[1]);
+        const uint32_t b = Pack2<T>::pack(Pack2<T>::lo(lg[it].y) - mx[2], Pack2<T>::hi(lg[it].y) - mx[3]);
+        lg[it] = make_uint2(a, b);
+        run[0] += exp_neg(Pack2<T>::lo(a));
+        run[1] += exp_neg(Pack2<T>::hi(a));
+        run[2] += exp_neg(Pack2<T>::lo(b));
+        run[3] += exp_neg(Pack2<T>::hi(b));
+      } else {
+        const float e = exp_neg(lg[it] - mx[0]);
+        lg[it] = e;
+        run[0] += e;
+      }
+    }
+  }
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) run[r] = T::bytes == 2 ? half_sum(run[r]) : row16_sum(run[r]);
+  share(1, run);
+#pragma unroll
+  for (int r = 0; r < kRows; ++r) {
+    float sum = stat[1][0][g * kRows + r];
+#pragma unroll
+    for (int w = 1; w < kWaves; ++w) sum += stat[1][w][g * kRows + r];
+    const bool ok = ((row0 + r) >> p.gs) < p.W && ((row0 + r) & (p.Gp - 1)) < p.G;
+    // rows outside the window or group never win a maximum, or contribute 0
+    if constexpr (T::bytes == 2) last[r] = ok ? -__builtin_amdgcn_logf(sum) : -INFINITY;
+    else last[r] = ok ? 1.f / sum : 0.f;
+  }
+  // ---- output: this quarter's share of the window reduction, halves apart where they hold different windows
+  constexpr int kShares = T::bytes == 2 ? 8 : 4;
+  float* const part = p.part + ((int64_t)unit * kShares + (T::bytes == 2 ? 2 * v + g : v)) * p.NB * p.BS + wave * (Tiles<T>::tokens / kWaves) + col;
+#pragma unroll
+  for (int it = 0; it < NT; ++it) {
+    if (it < u.n) {
+      float red;
+      if constexpr (T::bytes == 2) {
+        float pv[4];
+        pv[0] = __builtin_fmaf(Pack2<T>::lo(lg[it].x), 1.44269504088896340736f, last[0]);
+        pv[1] = __builtin_fmaf(Pack2<T>::hi(lg[it].x), 1.44269504088896340736f, last[1]);
+        pv[2] = __builtin_fmaf(Pack2<T>::lo(lg[it].y), 1.44269504088896340736f, last[2]);
+        pv[3] = __builtin_fmaf(Pack2<T>::hi(lg[it].y), 1.44269504088896340736f, last[3]);
+        if (p.Gp >= 4) {
+          red = vmax4(pv[0], pv[1], pv[2], pv[3]);
+          if (p.Gp >= 8) red = vmax(red, lane_xor32(red));
+          float none = red = exp2_hw(red);
+          Rnd<T>::pair(red, none);
+        } else if (p.Gp == 2) {
+          float a = exp2_hw(vmax(pv[0], pv[1])), b = exp2_hw(vmax(pv[2], pv[3]));
+          Rnd<T>::pair(a, b);
+          red = rmax ? vmax(a, b) : a + b;
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) pv[r] = exp2_hw(pv[r]);
+          Rnd<T>::pair(pv[0], pv[1]);
+          Rnd<T>::pair(pv[2], pv[3]);
+          red = rmax ? vmax4(pv[0], pv[1], pv[2], pv[3]) : (pv[0] + pv[1]) + (pv[2] + pv[3]);
+        }
+      } else {
+        red = lg[it] * last[0];
+        float o = lane_xor16(red);
+        red = p.Gp >= 2 || rmax ? vmax(red, o) : red + o;
+        o = lane_xor32(red);
+        red = p.Gp >= 4 || rmax ? vmax(red, o) : red + o;
+      }
+      const int j = u.place_of(it) & 0xffff;
+      if (T::bytes == 2 || g == 0) part[j * p.BS + u.first_token(it)] = red;
+    }
+  }
+}
+
 // Adds the row blocks' window partials of every (layer, sequence, head) in block order, divides by
-// the window length, rounds to the cache dtype; pad pages score exactly 0.
-template <typename T>
+// the window length, rounds to the cache dtype; pad pages score exactly 0.  SHARES: a block's partials lie as
+// score_rows_kernel leaves them, quarters (16-bit caches: and halves) apart.
+template <typename T, int SHARES>
 __global__ __launch_bounds__(256) void score_combine_kernel(const float* __restrict__ part,
                                                             void* __restrict__ out,
                                                             const int32_t* __restrict__ table,
                                                             int B, int NB, int BS, int Hkv, int RB,
-                                                            int W, int num_pages, int rmax) {
+                                                            int W, int num_pages, int rmax, int Gp) {
   // four consecutive tokens per thread (a page is a multiple of 128 tokens)
   const int item = blockIdx.x;
   const int b = (item / Hkv) % B;
@@ -1411,13 +1654,24 @@ __global__ __launch_bounds__(256) void score_combine_kernel(const float* __restr
   typedef float f4 __attribute__((ext_vector_type(4)));
   f4 v = {0.f, 0.f, 0.f, 0.f};
   if (pid >= 0 && pid < num_pages) {
-    const float* src = part + (int64_t)item * RB * Tn + t;
-    v = __builtin_nontemporal_load((const f4*)src);
-    for (int r = 1; r < RB; ++r) {
-      const f4 o = __builtin_nontemporal_load((const f4*)(src + (int64_t)r * Tn));
-      if (rmax) { v.x = fmaxf(v.x, o.x); v.y = fmaxf(v.y, o.y); v.z = fmaxf(v.z, o.z); v.w = fmaxf(v.w, o.w); }
-      else { v.x += o.x; v.y += o.y; v.z += o.z; v.w += o.w; }
-    }
+    auto join = [&](bool largest, const f4& x, const f4& o) {
+      return largest ? f4{fmaxf(x.x, o.x), fmaxf(x.y, o.y), fmaxf(x.z, o.z), fmaxf(x.w, o.w)} : x + o;
+    };
+    auto block = [&](int r) -> f4 {
+      const float* src = part + ((int64_t)item * RB + r) * SHARES * Tn + t;
+      f4 x[SHARES];
+#pragma unroll
+      for (int i = 0; i < SHARES; ++i) x[i] = __builtin_nontemporal_load((const f4*)(src + (int64_t)i * Tn));
+      if constexpr (SHARES == 1) return x[0];
+      if constexpr (SHARES == 4)      // rows 4 i .. of a block of 16: groups of eight span two quarters, of sixteen all
+        return join(rmax || Gp >= 16, join(rmax || Gp >= 8, x[0], x[1]), join(rmax || Gp >= 8, x[2], x[3]));
+      f4 half[2];                     // of 32: rows 8 i .. of a quarter are the lower half's four and the upper's
+#pragma unroll
+      for (int g = 0; g < 2; ++g) half[g] = join(rmax, join(rmax, x[g], x[2 + g]), join(rmax, x[4 + g], x[6 + g]));
+      return Gp < 8 ? join(rmax, half[0], half[1]) : half[0];
+    };
+    v = block(0);
+    for (int r = 1; r < RB; ++r) v = join(rmax, v, block(r));
     if (!rmax) {
       v.x = Elem<T>::rnd(v.x / (float)W); v.y = Elem<T>::rnd(v.y / (float)W);
       v.z = Elem<T>::rnd(v.z / (float)W); v.w = Elem<T>::rnd(v.w / (float)W);
@@ -1486,6 +1740,19 @@ static int64_t resident_need(int L, int B, int NB, int BS, int Hkv, int Hq, int 
   return (int64_t)L * B * Hkv * ((W * Gp + 31) / 32) * NB * BS * 4;
 }
 
+// Few units spread their tiles over the chip (score_tiles_kernel); what that needs, or 0.  The line lies where they
+// occupy a quarter of the CUs: the whole compression step of one fp32 sequence, 16 heads, window 32 (32 units) 59 -> 47 us, of
+// two 66 -> 61; 16-bit, window 16 (8) 42 -> 33, four sequences (32) 51 -> 43, eight (64) 65 -> 58; but 32 heads, window 32: two
+// sequences (64) 47 -> 44, three 47 -> 52, as logits through memory cost more with every unit.
+constexpr int64_t kFewUnits = 64;
+static int64_t tiled_need(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype) {
+  if (!resident_need(L, B, NB, BS, Hkv, Hq, W, dtype)) return 0;
+  const int Gp = pow2_ceil(Hq / Hkv);
+  const int64_t units = (int64_t)L * B * Hkv * (dtype == ZP_F32 ? (W * Gp + 15) / 16 : (W * Gp + 31) / 32);
+  if (units > kFewUnits || (dtype != ZP_F32 && Gp > 8)) return 0;
+  return units * NB * BS * (64 + (dtype == ZP_F32 ? 4 : 8) * 4);      // logits, and partials of a unit's quarters
+}
+
 extern "C" int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                                     int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype) {
   if (Hkv <= 0 || Hq <= 0 || L < 0 || B < 0 || NB <= 0 || BS <= 0 || W <= 0) return 0;
@@ -1493,6 +1760,12 @@ extern "C" int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_
   const int64_t floor_bytes = sweep_workspace(L, B, NB, BS, Hkv, Hq, W);
   const int64_t res = resident_need(L, B, NB, BS, Hkv, Hq, W, dtype);
   return res > floor_bytes ? res : floor_bytes;
+}
+
+extern "C" int64_t zp_attention_score_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS,
+                                                    int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype) {
+  const int64_t usual = zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, dtype);
+  return usual <= 0 ? usual : std::max(usual, tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype));
 }
 
 extern "C" int64_t zp_attention_score_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS,
@@ -1575,6 +1848,28 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
   hipStream_t st = (hipStream_t)stream;
   a.n_items = L * B * Hkv;
   a.part = (float*)workspace;
+  const int64_t tiled = tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype);
+  if ((resident || resident32) && tiled && workspace_bytes >= tiled) {
+    if (resident32) a.RB = (W * Gp + 15) / 16;
+    const unsigned units = (unsigned)(a.n_items * a.RB);
+    a.tiles = NB * (BS / (resident ? 128 : 64));
+    a.lg = (char*)workspace + (int64_t)units * NB * BS * (resident ? 32 : 16);
+    const dim3 cgrid((unsigned)a.n_items, (unsigned)((NB * BS / 4 + 255) / 256));
+#define ZP_TILED_LAUNCH(TPP)                                                                                          \
+  do {                                                                                                                \
+    hipLaunchKernelGGL((score_tiles_kernel<T, TPP>), dim3(a.tiles, a.RB, a.n_items), dim3(kThreads), 0, st, a);       \
+    hipLaunchKernelGGL((score_rows_kernel<T, TPP>), dim3(4, a.RB, a.n_items), dim3(kThreads), 0, st, a);              \
+  } while (0)
+    ZP_DISPATCH_DTYPE(dtype, {
+      if (BS == 256) ZP_TILED_LAUNCH(T::bytes == 2 ? 2 : 4);
+      else ZP_TILED_LAUNCH(0);
+      hipLaunchKernelGGL((score_combine_kernel<T, T::bytes == 2 ? 8 : 4>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
+                         B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max, Gp);
+    });
+#undef ZP_TILED_LAUNCH
+    ZP_LAUNCH_CHECK();
+    return ZP_OK;
+  }
   if (resident) {
     const size_t smem = (size_t)kWaves * 2 * kSubBytes + sizeof(float) * kWaves * 32;
     const unsigned units = (unsigned)(((int64_t)a.n_items + 7) / 8 * 8 * RB);
@@ -1592,8 +1887,8 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
       return ZP_EHIP;                                                                            \
     }                                                                                            \
     hipLaunchKernelGGL(fn, dim3(units), dim3(kThreads), smem, st, a);                            \
-    hipLaunchKernelGGL(score_combine_kernel<TT>, cgrid, dim3(256), 0, st, a.part, scores_out,    \
-                       block_table, B, NB, BS, Hkv, RB, W, num_pages, a.reduce_max);             \
+    hipLaunchKernelGGL((score_combine_kernel<TT, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, \
+                       block_table, B, NB, BS, Hkv, RB, W, num_pages, a.reduce_max, Gp);         \
   } while (0)
     if (dtype == ZP_BF16) ZP_RESIDENT_LAUNCH(BF16);
     else ZP_RESIDENT_LAUNCH(F16);
@@ -1615,8 +1910,8 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
       return ZP_EHIP;
     }
     hipLaunchKernelGGL(fn, dim3(units), dim3(kThreads), smem, st, a);
-    hipLaunchKernelGGL(score_combine_kernel<F32>, cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
-                       B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max);
+    hipLaunchKernelGGL((score_combine_kernel<F32, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
+                       B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max, Gp);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }
