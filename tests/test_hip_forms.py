@@ -211,6 +211,14 @@ def test_runs_of_any_scale(dev, H, G, D, V, scale, lens=((1, 1), (63, 63), (65, 
     assert bool(((out.view(N, H, V).cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -7 * v.abs().max()).all())
 
 
+# The launch hands key heads and tiles to eight parts: heads that divide into them, tiles that do not; key heads that share a
+# part; key and value rows of 8 and 16 pieces in each combination, not all of them there
+@pytest.mark.parametrize("H,G,D,V", [(16, 8, 128, 128), (32, 16, 64, 128), (12, 12, 72, 40), (10, 10, 40, 24), (6, 2, 64, 64),
+                                     (9, 3, 128, 104), (5, 1, 56, 72)])
+def test_runs_over_the_parts_of_a_launch(dev, H, G, D, V):
+    test_runs_of_any_scale(dev, H, G, D, V, 0.25, ((385, 385), (1, 900), (127, 191), (128, 192), (129, 193), (33, 600)))
+
+
 # up to 256 keys, and up to 32 per tile on average: steps of 32 keys, whatever a run has
 FEW_KEYS = [(1, 1)] * 5 + [(16, 16), (17, 33), (64, 65), (96, 137)]
 

@@ -81,9 +81,9 @@ __device__ __forceinline__ void eight_columns(const f32x4& even, const f32x4& od
 
 enum { kNoCap, kCap, kBoundedCap };   // of the scores, see SoftCap
 // Keys per step: 64 scores for each query where the registers hold them (8 prompts as above: 519 -> 463 us; keys of 192
-// with a shared part spill: 1811 -> 1831).
+// with a shared part spill: 1811 -> 1831) and many keys come here (heads of at most 128 have a kernel of their own).
 constexpr int long_step(int DKS, int VCB, int MAPS, bool SHARED, int CAP) {
-  return MAPS == 1 && VCB == 1 && CAP == kNoCap && DKS <= (SHARED ? 4 : 6) ? 64 : 32;
+  return MAPS == 1 && VCB == 1 && CAP == kNoCap && (SHARED ? DKS <= 4 : DKS == 6) ? 64 : 32;
 }
 
 // Column tile t of a wave: 16 queries, map t % MAPS of the head (differential attention has two, over the same
@@ -368,18 +368,23 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
   }
 }
 
-// ------------------------------------------------------------------ values of at most 64, one map, no cap
+// ------------------------------------------------------------------ heads of at most 128, one map, no cap
 // Here the products of a tile's keys run while the exponentials of the tile before take their turn, which needs the scores
-// of two tiles in registers: with 64 value columns they are there, with 128 they are not (heads of 128, 8 prompts of 2048
-// tokens: 435 -> 423 us, with weights of 17 bits 448 -> 470).  Rows go from memory into LDS without passing through
-// registers.  Bound by the vector units' issue (a product takes half of its 16 cycles there, too, an exponential 8).
-// Heads of 64, 8 prompts of about 1800 tokens, 16 heads, with the rotary store: 181 -> 145 us (236 before both kernels'
-// reads were ahead of their products); 4 of 2048, 32 heads: 163 -> 120 (222).
+// of two tiles in registers.  A 32 x 32 product takes 8 of its 32 cycles at the vector issue, a 16 x 16 one 8 of 16: with the
+// wide ones there is room for the exponentials, and for 128 value columns (16 x 16, those of a head of 128 did not pay).
+// Rows go from memory into LDS without passing through registers, one load at a time between the products: eight in a row
+// held a wave for 870 cycles a tile.  Queries and the first keys are asked for together.
+// Bound by the vector issue (300 of 3390 cycles a tile and SIMD pair are waits) at the clock that the power limit leaves
+// (1.9 GHz); a tenth of the time a CU has one workgroup or none.  Heads of 128, 32 over 8 of keys and values, 8 prompts of
+// 2048 tokens: window of 1024 309 -> 278 us, all keys 371 -> 327; one prompt 52 -> 44, of 300 tokens 12.7 -> 10.6; heads of
+// 64: 198 -> 181, 240 -> 216, 33 -> 29, 9.0 -> 8.2; causal with two planes of weights 452 -> 448, one prompt of 300 14.7 -> 12.5.  Tried: eight waves of two heads that share their rows, in turns at
+// the matrix cores and the vector units (322 us: a wave alone issues a vector instruction every six cycles) or side by side
+// (347: they meet at the same unit); whole rows next to one another in LDS (281).
 //
 // Rows of CH 16-byte pieces (8 or 16) as loads leave them in LDS, 1 KB at a time with GAP bytes between: four rows after
 // one another interleave their pieces by four, so that a lane's pieces and the column tiles are immediate offsets.  With
 // eight rows per load the pieces of the second four lie FLIP apart.  What reads them falls into different banks: sixteen
-// rows of one piece (keys), twice four rows of two (values, transposed).
+// rows of one piece (keys), four rows of four (values, transposed).
 template <int CH, int FLIP, int GAP> struct Staged {
   static constexpr int kRows = 64 / CH;                        // per load
   static constexpr int kLoad = 1024 + GAP, kBytes = kTileK / kRows * kLoad;
@@ -393,26 +398,78 @@ template <int CH, int FLIP, int GAP> struct Staged {
     return (r >> 3) * kLoad + (r >> 2 & 1) * 512 + (r & 3) * 64 + (p ^ FLIP * (r >> 2 & 1)) * 16;
   }
 };
-constexpr int kFlowV = 64;
-// The row at `from` and those behind it; every lane reads within rows that are there: the bound is none of the buffer's.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t rows_at(const void* from) {
-  return __builtin_amdgcn_make_buffer_rsrc((void*)from, 0, 0x7fffffff, 0x00020000);
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16 mfma32_bf16(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
-__device__ __forceinline__ void rows_to_lds(__amdgpu_buffer_rsrc_t rows, char* to, int lane_at, int at) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(rows, (lds_ptr_t)to, 16, lane_at, at, 0, 0);
+template <int KS, int VB> struct FlowStage {                   // 16 KS elements of a key, 32 VB of a value
+  typedef Staged<2 * KS, 1, KS == 8 ? 16 : 32> K;
+  typedef Staged<4 * VB, 2, 0> V;
+  static constexpr int kBytes = 2 * (K::kBytes + V::kBytes);
+};
+
+// Which head and tile a workgroup takes.  Those of one L2 (x, eighths of the launch) have the query heads of a key head next
+// to one another and its tiles behind, the last ones first: what reads the same keys at the same time reads them from there.
+struct FlowPlace {
+  int h, hk, tile;
+  __host__ __device__ static int part_bits(int heads) { return heads % 8 == 0 ? 3 : heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0; }
+  __host__ __device__ static int tiles_of(int T, int bits) { return (T + (8 >> bits) - 1) >> (3 - bits); }
+  __host__ static dim3 grid(const TilesArgs& a) {
+    const int bits = part_bits(a.HK);
+    return dim3(8, a.H / a.HK, (unsigned)tiles_of(a.T, bits) * (a.HK >> bits));
+  }
+  __device__ __forceinline__ FlowPlace(const TilesArgs& a) {
+    const int bits = part_bits(a.HK), part = blockIdx.x, tiles = tiles_of(a.T, bits);
+    int at = blockIdx.z, from = 0;
+    if (at >= tiles) {
+      from = at / tiles;
+      at -= from * tiles;
+    }
+    hk = (from << bits) + (part & ((1 << bits) - 1));
+    h = hk * (int)gridDim.y + blockIdx.y;
+    tile = ((tiles - 1 - at) << (3 - bits)) + (part >> bits);  // past the last one: nothing to do
+  }
+};
+
+// A wave's results on their way out: lane l32 of either half has a query's columns 8 (i / 4) + 4 half + i % 4 of each 32.
+template <int VB>
+__device__ __forceinline__ void flow_out(const TilesArgs& a, int h, int64_t row, bool there, f32x16 (&o)[VB], float m, float l) {
+  const int half = (threadIdx.x & 63) >> 5;
+  if (a.sinks) l += __builtin_amdgcn_exp2f(a.sinks[h] * 1.44269504088896f - m);
+  const float inv = l > 0.f ? a.out_scale / l : 0.f;
+  uint16_t* const out = a.out + row * a.o_st + h * a.V;
+#pragma unroll
+  for (int c = 0; c < VB; ++c)
+#pragma unroll
+    for (int i = 0; i < 16; i += 8) {                          // halves swap four columns: each ends with eight neighbours
+      float r[8];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[c][i + e] * inv), __float_as_uint(o[c][i + 4 + e] * inv),
+                                                           false, false);
+        r[e] = __uint_as_float(both[0]);
+        r[4 + e] = __uint_as_float(both[1]);
+      }
+      const int col = c * 32 + (i + half * 4) * 2;
+      if (!there || col >= a.V) continue;                    // every lane took part in the swaps
+      if (a.turns) turn_back8(r, a.turns + (row * a.V + col) / 2);
+      Vec8<BF16>::st(out, col, r);
+    }
 }
 
-// FINE as above.
-template <int DKS, bool FINE>
+// FINE as above.  A wave's 32 queries are the columns of 32 x 32 products: lane l32 of either half holds one query's scores
+// for keys 8 (i / 4) + 4 half + i % 4 of a tile of 32, which are its operand elements of the products with values.
+template <int KS, int VB, bool FINE>
 __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
-  typedef Staged<DKS * 4, 1, DKS == 4 ? 16 : 32> KL;
-  typedef Staged<8, 2, 0> VL;
-  constexpr int VT = kFlowV / 16;                              // column tiles of the values
-  constexpr int kQK = 4 * DKS * 2, kPV = VT * 2;               // products of a tile's keys, of half its values
-  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  typedef typename FlowStage<KS, VB>::K KL;
+  typedef typename FlowStage<KS, VB>::V VL;
+  constexpr int kQK = 2 * KS, kPV = 2 * VB;                    // products of a tile's keys, of half its values
+  const int lane = threadIdx.x & 63, l16 = lane & 15, l32 = lane & 31, g = lane >> 4, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = blockIdx.x % a.H, tile = blockIdx.x / a.H;     // one head's tiles share an L2 when H % 8 == 0
+  const FlowPlace place(a);
+  const int h = place.h, tile = place.tile;
+  if (tile >= a.T) return;
   const int q0 = a.tiles[tile * 4], nq = min(a.tiles[tile * 4 + 1], kTileQ);
   const int kb = a.tiles[tile * 4 + 2], rel = a.tiles[tile * 4 + 3];
   // host-made descriptors: rows outside the buffers are not touched
@@ -421,7 +478,7 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   // round, zero takes them away
   const float by = a.scale * 1.44269504088896f, factor = by == 0.f ? 1.f : fabsf(by);
   const uint32_t flip = by < 0.f ? 0x80008000u : 0u, kept = by == 0.f ? 0u : ~0u;
-  const int hk = h / (a.H / a.HK);
+  const int hk = place.hk;
   const uint16_t* const kbase = a.k + (int64_t)kb * a.kv_st + hk * a.D;
   const uint16_t* const vbase = a.v + (int64_t)kb * a.v_st + hk * a.V;
 
@@ -433,30 +490,7 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   const int seen0 = w0 < nq ? (lo - first) / kTileK : tiles + 1;
   const int seen1 = w0 < nq ? (rel + min(w0 + 32, nq) - 1 - first) / kTileK : tiles + 1;
 
-  u32x4 qf[2][DKS];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int qi = min(w0 + t * 16 + l16, nq - 1);
-    const uint16_t* q = a.q + (int64_t)(q0 + qi) * a.q_st + h * a.D;
-#pragma unroll
-    for (int ks = 0; ks < DKS; ++ks) {
-      // past the head's end: the key columns there hold other elements, against zeros here
-      const int c = ks * 32 + g * 8;
-      qf[t][ks] = (*(const u32x4*)(q + (c < a.D ? c : 0)) & kept) ^ flip;
-      if (c >= a.D) qf[t][ks] = u32x4{0u, 0u, 0u, 0u};
-    }
-  }
-  f32x4 o[2][VT];
-  float m[2], l[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    m[t] = -INFINITY;
-    l[t] = 0.f;
-#pragma unroll
-    for (int c = 0; c < VT; ++c) o[t][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-
-  // ---- a tile's rows from memory into LDS; rows past the last one are the last one again
+  // ---- a tile's rows from memory into LDS; in place of rows past the last one come zeros, which nothing sees
   char* const kl = lds_raw;
   char* const vl = lds_raw + 2 * KL::kBytes;
   // what follows from the lane is worked out anew: kept, it would not leave the products enough registers
@@ -471,78 +505,94 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
     return L::row(i) * (int)stride * 2 + (L::piece(i) * 8 < cols ? L::piece(i) * 16 : 0);
   };
   const int klane = lane_at(KL{}, a.kv_st, a.D), vlane = lane_at(VL{}, a.v_st, a.V);
-  auto stage = [&](auto layout, char* tile, const uint16_t* rows, int64_t stride, int cols, int k0, int whole) {
-    typedef decltype(layout) L;
-    constexpr int kLoads = kTileK / L::kRows / 4;              // of each wave
-    tile += wave * L::kLoad;
-    if (k0 + kTileK - 1 <= last && stride < 1 << 24) {
-      const __amdgpu_buffer_rsrc_t from = rows_at(rows + (int64_t)(k0 + wave * L::kRows) * stride);
-#pragma unroll
-      for (int n = 0; n < kLoads; ++n) rows_to_lds(from, tile + n * 4 * L::kLoad, whole, n * 8 * L::kRows * (int)stride);
-      return;
-    }
-    const int i = lane_again(), row = L::row(i), col = L::piece(i) * 8 < cols ? L::piece(i) * 16 : 0;
-#pragma unroll 1
-    for (int n = 0; n < kLoads; ++n) {
-      const int from = min(k0 + (n * 4 + wave) * L::kRows, last);
-      const int at = min(row, last - from) * (int)stride * 2 + col;
-      rows_to_lds(rows_at(rows + (int64_t)from * stride), tile + n * 4 * L::kLoad, at, 0);
-    }
+  // rows k0 + wave * kRows on of a tile, as far as they are there
+  auto rows_of = [&](auto layout, const uint16_t* rows, int64_t stride, int cols, int k0) {
+    const int from = k0 + wave * decltype(layout)::kRows, left = last - from;
+    const uint32_t bytes = left >= kTileK ? 0x7fffffffu : left < 0 ? 0u : (uint32_t)(left * (int)stride + cols) * 2;
+    return rows_from(rows + (int64_t)from * stride, bytes);
   };
-  auto stage_keys = [&](int j) { stage(KL{}, kl + (j & 1) * KL::kBytes, kbase, a.kv_st, a.D, first + j * kTileK, klane); };
-  auto stage_values = [&](int j) { stage(VL{}, vl + (j & 1) * VL::kBytes, vbase, a.v_st, a.V, first + j * kTileK, vlane); };
+  constexpr int kKeyLoads = kTileK / KL::kRows / 4, kValueLoads = kTileK / VL::kRows / 4;      // of a wave
+  u32x4 krows, vrows;
+  auto rows_of_keys = [&](int j) { krows = rows_of(KL{}, kbase, a.kv_st, a.D, first + min(j, tiles) * kTileK); };
+  auto rows_of_values = [&](int j) { vrows = rows_of(VL{}, vbase, a.v_st, a.V, first + min(j, tiles) * kTileK); };
+  auto stage_keys = [&](int j, int n) {
+    load_to_lds(krows, kl + (j & 1) * KL::kBytes + (wave + n * 4) * KL::kLoad, klane + n * 8 * KL::kRows * (int)a.kv_st, 0);
+  };
+  auto stage_values = [&](int j, int n) {
+    load_to_lds(vrows, vl + (j & 1) * VL::kBytes + (wave + n * 4) * VL::kLoad, vlane + n * 8 * VL::kRows * (int)a.v_st, 0);
+  };
+  rows_of_keys(0);
+#pragma unroll
+  for (int n = 0; n < kKeyLoads; ++n) stage_keys(0, n);
+
+  u32x4 qf[KS];
+  {
+    const int qi = min(w0 + l32, nq - 1);
+    const uint16_t* q = a.q + (int64_t)(q0 + qi) * a.q_st + h * a.D;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+      // past the head's end: the key columns there hold other elements, against zeros here
+      const int c = ks * 16 + half * 8;
+      qf[ks] = *(const u32x4*)(q + (c < a.D ? c : 0));
+      if (c >= a.D) qf[ks] = u32x4{0u, 0u, 0u, 0u};
+    }
+    if (by <= 0.f)
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) qf[ks] = (qf[ks] & kept) ^ flip;
+  }
+  f32x16 o[VB];
+  float m = -INFINITY, l = 0.f;
+#pragma unroll
+  for (int c = 0; c < VB; ++c) o[c] = f32x16{};
 
   // ---- one tile: its weights and what its values add, and meanwhile the scores of the next one
-  // groups of lanes hold keys 16 (i / 4) + 4 g + i % 4; values leave LDS transposed, lane l16 with column l16 of four keys
-  const int kread = KL::at(l16, g);
-  const int vread = VL::at(4 * g + (l16 >> 2), (l16 & 3) >> 1) + (l16 & 1) * 8;
-  const int vread_odd = VL::at(4 * g + (l16 >> 2), 2 + ((l16 & 3) >> 1)) + (l16 & 1) * 8;      // of odd column tiles
-  const u32x4 ones = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
-  typedef float Scores[2][16];
-  auto step = [&](int j, auto here_, auto next_, Scores& p, Scores& after) {
+  const int kread = KL::at(l32, half);
+  // values leave LDS transposed, lane l32 with a column of four keys
+  const int vread = VL::at(4 * half + (l16 >> 2), 2 * (g & 1) + ((l16 & 3) >> 1)) + (l16 & 1) * 8;
+  // Sums of weights are 16 x 16 products, which take the same registers as sixteen queries of four groups of keys: ones
+  // where a group of rows and a group of keys belong to the same half of the queries.
+  const uint32_t one = ((l16 >> 2) & 1) == (g & 1) ? 0x3f803f80u : 0u;
+  const u32x4 ones = {one, one, one, one};
+  float mx = -INFINITY;                                        // largest score of the tile whose turn is next
+  auto step = [&](int j, auto here_, auto next_, f32x16 (&p)[2], f32x16 (&s)[2]) {
     constexpr bool HERE = here_.value, NEXT = next_.value;
     const char* const kt = kl + ((j + 1) & 1) * KL::kBytes + kread;
-    const char* const vt = vl + (j & 1) * VL::kBytes;
-    f32x4 s[2][4];
-    // operands leave LDS kAhead ahead of their two products
-    constexpr int kAhead = 4, kRing = kAhead + 1;
+    const char* const vt = vl + (j & 1) * VL::kBytes + vread;
+    // operands leave LDS kAhead ahead of their product
+    constexpr int kAhead = VB == 4 ? 3 : 4, kRing = kAhead + 1;
     u32x4 kf[kRing], vf[kRing];
-    // n: 16 keys n / DKS, step n % DKS
+    // n: step n / 2, 32 keys n % 2
     auto read_keys = [&](int n) {
-      if (n < 4 * DKS) kf[n % kRing] = *(const u32x4*)(kt + n / DKS * (16 / KL::kRows) * KL::kLoad + n % DKS * 256);
+      if (n < kQK) kf[n % kRing] = *(const u32x4*)(kt + (n & 1) * (32 / KL::kRows) * KL::kLoad + (n >> 2) * 256 + (n >> 1 & 1) * 32);
     };
-    // n: 32 keys n / VT, column tile n % VT
+    // n: 16 keys n / VB, column tile n % VB
     auto read_values = [&](int n) {
-      if (n >= 2 * VT) return;
-      const int c = n % VT, r = n / VT * 32;
-      const char* const at = vt + (c >> 1) * 256 + (c & 1 ? vread_odd : vread);
-      const uint2 x = read_transposed((const uint16_t*)(at + r / VL::kRows * VL::kLoad));
-      const uint2 y = read_transposed((const uint16_t*)(at + (r + 16) / VL::kRows * VL::kLoad));
+      if (n >= 4 * VB) return;
+      const char* const at = vt + n % VB * 256 + n / VB * (16 / VL::kRows) * VL::kLoad;
+      const uint2 x = read_transposed((const uint16_t*)at);
+      const uint2 y = read_transposed((const uint16_t*)(at + 8 / VL::kRows * VL::kLoad));
       vf[n % kRing] = u32x4{x.x, x.y, y.x, y.y};
     };
-    u32x4 pf[2][2], pl[2][2];
-    // product n of the next tile's keys: tile of keys n / (2 DKS), step, query tile
+    u32x4 pf[4], pl[4];
     auto key_product = [&](int n) {
-      const int tt = n / (2 * DKS), ks = n / 2 % DKS, t = n & 1;
-      if (t == 0) read_keys(n / 2 + kAhead);
-      if (ks == 0) s[t][tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-      s[t][tt] = mfma_bf16(kf[n / 2 % kRing], qf[t][ks], s[t][tt]);
+      read_keys(n + kAhead);
+      if (n < 2) s[n] = f32x16{};
+      s[n & 1] = mfma32_bf16(kf[n % kRing], qf[n >> 1], s[n & 1]);
     };
-    auto value_product = [&](int half, int n) {
-      const int c = n / 2, t = n & 1, v = half * VT + c;
-      if (t == 0) read_values(v + kAhead);
-      o[t][c] = mfma_bf16(vf[v % kRing], pf[t][half], o[t][c]);
-      if constexpr (FINE) o[t][c] = mfma_bf16(vf[v % kRing], pl[t][half], o[t][c]);
+    auto value_product = [&](int n) {
+      read_values(n + kAhead);
+      o[n % VB] = mfma32_bf16(vf[n % kRing], pf[n / VB], o[n % VB]);
+      if constexpr (FINE) o[n % VB] = mfma32_bf16(vf[n % kRing], pl[n / VB], o[n % VB]);
     };
-    float ms[2];
-    // weights of keys pair d of half, both query tiles
-    auto weights = [&](int half, int n) {
-      const int t = n & 1, d = n / 2, i = half * 8 + d * 2;
-      const float x = __builtin_amdgcn_exp2f(fmaf(p[t][i], factor, -ms[t]));
-      const float y = __builtin_amdgcn_exp2f(fmaf(p[t][i + 1], factor, -ms[t]));
-      const uint32_t w = pack_bf16(x, y);
-      pf[t][half][d] = w;
-      if constexpr (FINE) pl[t][half][d] = pack_bf16(x - __uint_as_float(w << 16), y - __uint_as_float(w & 0xffff0000u));
+    float ms = 0.f;
+    // weights of pair d of the 32 keys t
+    auto weights = [&](int t, int d) {
+      const float x = __builtin_amdgcn_exp2f(fmaf(p[t][2 * d], factor, -ms));
+      const float y = __builtin_amdgcn_exp2f(fmaf(p[t][2 * d + 1], factor, -ms));
+      uint32_t w = pack_bf16(x, y);
+      asm volatile("" : "+v"(w));                              // made here, not at its use
+      pf[2 * t + d / 4][d % 4] = w;
+      if constexpr (FINE) pl[2 * t + d / 4][d % 4] = pack_bf16(x - __uint_as_float(w << 16), y - __uint_as_float(w & 0xffff0000u));
     };
     if constexpr (NEXT)
 #pragma unroll
@@ -550,82 +600,77 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
     if constexpr (HERE) {
       const int k0 = first + j * kTileK;
       if (k0 + kTileK - 1 > rel + w0 || k0 < lo_last) {        // some query of the wave does not see all these keys
+        const int i0 = lane_again(), pos = rel + min(w0 + (i0 & 31), nq - 1);
+        const int low = first_seen(pos, a.window, a.chunk);
+        const int from = low - k0 - 4 * (i0 >> 5), span = pos - low;     // keys low .. pos are seen
+        mx = -INFINITY;
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
-          const int i0 = lane_again(), pos = rel + min(w0 + t * 16 + (i0 & 15), nq - 1);
-          const int low = first_seen(pos, a.window, a.chunk);
-          const int from = low - k0 - 4 * (i0 >> 4), span = pos - low;   // keys low .. pos are seen
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int i = 0; i < 16; ++i)
-            if ((unsigned)((i >> 2) * 16 + (i & 3) - from) > (unsigned)span) p[t][i] = -INFINITY;
-        }
+          for (int i = 0; i < 16; ++i) {
+            if ((unsigned)(t * 32 + (i >> 2) * 8 + (i & 3) - from) > (unsigned)span) p[t][i] = -INFINITY;
+            mx = fmaxf(mx, p[t][i]);
+          }
       }
+      mx *= factor;
+      if (__any(mx > m)) {                                     // in any lane: seldom after the first keys
+        mx = fmaxf(m, mx);
+        mx = fmaxf(mx, lane_xor32(mx));
+        const float f = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m - mx);
+        m = mx;
+        l *= f;
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        float mx = -INFINITY;
-#pragma unroll
-        for (int i = 0; i < 16; ++i) mx = fmaxf(mx, p[t][i]);
-        mx *= factor;
-        if (__any(mx > m[t])) {                                // in any lane: seldom after the first keys
-          mx = fmaxf(m[t], mx);
-          mx = fmaxf(mx, lane_xor16(mx));
-          mx = fmaxf(mx, lane_xor32(mx));
-          const float f = mx == -INFINITY ? 1.f : __builtin_amdgcn_exp2f(m[t] - mx);
-          m[t] = mx;
-          l[t] *= f;
-#pragma unroll
-          for (int c = 0; c < VT; ++c) o[t][c] *= f;
-        }
-        ms[t] = m[t] == -INFINITY ? 0.f : m[t];                // a query whose window starts later
+        for (int c = 0; c < VB; ++c) o[c] *= f;
       }
+      ms = m == -INFINITY ? 0.f : m;                           // a query whose window starts later
     }
-    constexpr int kEarly = kQK * 3 / 4, kLate = kQK - kEarly;
+    rows_of_keys(j + 2);
+    rows_of_values(j + 1);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
+      // what the next step needs, over what was used before the last barrier; one by one, as loads block in a row
+      if (i < kKeyLoads) stage_keys(j + 2, i);
+      else if (i - kKeyLoads < kValueLoads) stage_values(j + 1, i - kKeyLoads);
       if constexpr (NEXT)
 #pragma unroll
-        for (int e = i * kEarly / 8; e < (i + 1) * kEarly / 8; ++e) key_product(e);
+        for (int e = i * kQK / 8; e < (i + 1) * kQK / 8; ++e) key_product(e);
       if constexpr (HERE) weights(0, i);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (HERE)
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    auto sums = [&](int t) {
 #pragma unroll
-      for (int i = 0; i < kAhead; ++i) read_values(i);
-    f32x4 sum[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-    auto sums = [&](int half) {
-#pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        sum[t] = mfma_bf16(ones, pf[t][half], sum[t]);
-        if constexpr (FINE) sum[t] = mfma_bf16(ones, pl[t][half], sum[t]);
+      for (int i = 2 * t; i < 2 * t + 2; ++i) {
+        sum = mfma_bf16(ones, pf[i], sum);
+        if constexpr (FINE) sum = mfma_bf16(ones, pl[i], sum);
       }
     };
+    if constexpr (HERE) {
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      constexpr int kAll = (NEXT ? kLate : 0) + (HERE ? kPV : 0);
+      for (int i = 0; i < kAhead; ++i) read_values(i);
 #pragma unroll
-      for (int e = i * kAll / 8; e < (i + 1) * kAll / 8; ++e) {
-        if (NEXT && e < kLate) key_product(kEarly + e);
-        else if constexpr (HERE) value_product(0, e - (NEXT ? kLate : 0));
-      }
-      if constexpr (HERE) {
+      for (int i = 0; i < 8; ++i) {
+#pragma unroll
+        for (int e = i * kPV / 8; e < (i + 1) * kPV / 8; ++e) value_product(e);
         if (i == 0) sums(0);
         weights(1, i);
+        __builtin_amdgcn_sched_barrier(0);
       }
+      sums(1);
+    }
+    if constexpr (NEXT) mx = -INFINITY;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      if constexpr (HERE)
+#pragma unroll
+        for (int e = i * kPV / 8; e < (i + 1) * kPV / 8; ++e) value_product(kPV + e);
+      if constexpr (NEXT)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx = fmaxf(mx, s[i >> 2][(i & 3) * 4 + e]);
       __builtin_amdgcn_sched_barrier(0);
     }
-    if constexpr (HERE) {
-      sums(1);
-#pragma unroll
-      for (int e = 0; e < kPV; ++e) value_product(1, e);
-#pragma unroll
-      for (int t = 0; t < 2; ++t) l[t] += sum[t][0];
-    }
-    if constexpr (NEXT)
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int i = 0; i < 16; ++i) after[t][i] = s[t][i >> 2][i & 3];
+    if constexpr (HERE) l += sum[0];
   };
 
   typedef std::integral_constant<bool, true> yes;
@@ -635,18 +680,15 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  // Every wave takes the tiles from -1 on one by one, stages its share of what the next one needs (over what was used
-  // before the last barrier) and meets the others once for each; which of them it works on is its own matter.
+  // Every wave takes the tiles from -1 on one by one, stages its share of what the next one needs and meets the others once
+  // for each; which of them it works on is its own matter.
   int j = -1;
-  Scores p0, p1;
-  auto tile_of = [&](auto here, auto next, Scores& p, Scores& after) {
-    if (j + 2 < tiles) stage_keys(j + 2);
-    if (j + 1 < tiles) stage_values(j + 1);
+  f32x16 p0[2], p1[2];
+  auto tile_of = [&](auto here, auto next, f32x16 (&p)[2], f32x16 (&after)[2]) {
     step(j, here, next, p, after);
     meet();
     ++j;
   };
-  stage_keys(0);
   meet();
 #pragma unroll 1
   while (j < tiles && j != seen0 - 1) tile_of(no{}, no{}, p0, p1);
@@ -667,32 +709,34 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
     while (j < tiles) tile_of(no{}, no{}, p0, p1);
   }
 
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    if (a.sinks) l[t] += __builtin_amdgcn_exp2f(a.sinks[h] * 1.44269504088896f - m[t]);
-    const float inv = l[t] > 0.f ? a.out_scale / l[t] : 0.f;
-    const int qi = w0 + t * 16 + l16;
-    uint16_t* const out = a.out + (int64_t)(q0 + qi) * a.o_st + h * a.V;
-#pragma unroll
-    for (int c = 0; c < VT; c += 2) {
-      float r[8];
-      eight_columns(o[t][c], o[t][c + 1], inv, r);
-      const int col = (c + (g & 1)) * 16 + (g >> 1) * 8;
-      if (qi >= nq || col >= a.V) continue;                    // every lane took part in the swaps
-      if (a.turns) turn_back8(r, a.turns + ((int64_t)(q0 + qi) * a.V + col) / 2);
-      Vec8<BF16>::st(out, col, r);
-    }
-  }
+  const int qi = w0 + l32;
+  flow_out(a, h, q0 + qi, qi < nq, o, m, l);
 }
 
-template <int DKS, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
-  constexpr int smem = 2 * (Staged<DKS * 4, 1, DKS == 4 ? 16 : 32>::kBytes + Staged<8, 2, 0>::kBytes);
-  static_assert(smem <= 64 * 1024, "no attribute needed");
-  hipLaunchKernelGGL((run_flow_kernel<DKS, FINE>), dim3((unsigned)a.T * a.H), dim3(256), smem, st, a);
+template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
+  constexpr int smem = FlowStage<KS, VB>::kBytes;
+  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)run_flow_kernel<KS, VB, FINE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              smem) != hipSuccess) {
+    zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
+    return ZP_EHIP;
+  }
+  hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE>), FlowPlace::grid(a), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
-
+// Steps of 32 keys where tiles have no more on average: a prompt of 16 tokens, 32 heads of 128 5.2 us (5.7 in the flow), of
+// 64 6.2 (6.1).  Not among many keys, where one long run may decide (31 prompts of 16 tokens and one of 512 23.1, 20.3 with 64).
+inline bool few_keys(const TilesArgs& a) { return a.k_rows <= 256 && a.k_rows <= 32 * (int64_t)a.T; }
+// Offsets within a tile are 32 bits, the launch is three-dimensional.
+inline bool flow_takes(const TilesArgs& a) {
+  const dim3 grid = FlowPlace::grid(a);
+  return a.D <= 128 && a.V <= 128 && (a.V <= 64 || !few_keys(a)) && a.kv_st < 1 << 24 && a.v_st < 1 << 24 && grid.y < 65536 &&
+         grid.z < 65536;
+}
+template <bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
+  if (a.V <= 64) return a.D <= 64 ? launch_flow<4, 2, FINE>(a, st) : launch_flow<8, 2, FINE>(a, st);
+  return a.D <= 64 ? launch_flow<4, 4, FINE>(a, st) : launch_flow<8, 4, FINE>(a, st);
+}
 
 template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
 int launch_steps(const TilesArgs& a, hipStream_t st) {
@@ -708,20 +752,17 @@ int launch_steps(const TilesArgs& a, hipStream_t st) {
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
-// Steps of 32 keys where tiles have no more on average: a prompt of 16 tokens, 32 heads of 128 5.2 us (5.8 with 64), of 32
-// 5.5 (6.1); of 64 6.4 (6.3).  Not among many keys, where one long run may decide (31 prompts of 16 tokens and one of 512
-// 23.1, 20.3 with 64).
 template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
 int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
   constexpr int kLong = long_step(DKS, VCB, MAPS, SHARED, CAP);
-  if (a.k_rows <= 256 && a.k_rows <= 32 * (int64_t)a.T) return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, 32>(a, st);
+  if (few_keys(a)) return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, 32>(a, st);
   return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kLong>(a, st);
 }
 
 template <bool SHARED, int CAP> int launch_one_map(const TilesArgs& a, hipStream_t st) {
   const int dk = (a.D + a.P + 31) / 32;
   if constexpr (!SHARED && CAP == kNoCap)
-    if (dk <= 4 && a.V <= kFlowV) return dk <= 2 ? launch_flow<2, false>(a, st) : launch_flow<4, false>(a, st);
+    if (flow_takes(a)) return launch_flow<false>(a, st);
   if (a.V <= 128) {
     if (dk <= 2) return launch_run_tiles<2, 1, 2, 1, SHARED, CAP>(a, st);
     if (dk <= 4) return launch_run_tiles<4, 1, 2, 1, SHARED, CAP>(a, st);
@@ -817,6 +858,6 @@ extern "C" int zp_causal_attention(const void* q, const void* k, const void* v, 
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, tiles, nullptr, T, H, HK,
                  D, 0, D, 0, 0, q_rows, k_rows, q_stride, k_stride, v_stride, 0, out_stride, scale, 1.f, 0.f, 0.f, 0.f, D,
                  nullptr, 0, nullptr};
-  if (D <= kFlowV) return launch_flow<2, true>(a, (hipStream_t)stream);
+  if (flow_takes(a)) return launch_flow<true>(a, (hipStream_t)stream);
   return launch_run_tiles<4, 1, 2, 1, false, kNoCap, true>(a, (hipStream_t)stream);
 }
