@@ -377,9 +377,10 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
 // Bound by the vector issue (300 of 3390 cycles a tile and SIMD pair are waits) at the clock that the power limit leaves
 // (1.9 GHz); a tenth of the time a CU has one workgroup or none.  Heads of 128, 32 over 8 of keys and values, 8 prompts of
 // 2048 tokens: window of 1024 309 -> 278 us, all keys 371 -> 327; one prompt 52 -> 44, of 300 tokens 12.7 -> 10.6; heads of
-// 64: 198 -> 181, 240 -> 216, 33 -> 29, 9.0 -> 8.2; causal with two planes of weights 452 -> 448, one prompt of 300 14.7 -> 12.5.  Tried: eight waves of two heads that share their rows, in turns at
-// the matrix cores and the vector units (322 us: a wave alone issues a vector instruction every six cycles) or side by side
-// (347: they meet at the same unit); whole rows next to one another in LDS (281).
+// 64: 198 -> 181, 240 -> 216, 33 -> 29, 9.0 -> 8.2; causal with weights of 17 bits 452 -> 448, one prompt of 300 14.7 -> 12.5.
+// Tried: eight waves of two heads that share their rows, in turns at the matrix cores and the vector units (322 us: a wave
+// alone issues a vector instruction every six cycles) or side by side (347: they meet at the same unit); whole rows next
+// to one another in LDS (281).
 //
 // Rows of CH 16-byte pieces (8 or 16) as loads leave them in LDS, 1 KB at a time with GAP bytes between: four rows after
 // one another interleave their pieces by four, so that a lane's pieces and the column tiles are immediate offsets.  With
