@@ -13,6 +13,13 @@ __device__ __forceinline__ f32x4 mfma_bf16(const u32x4& a, const u32x4& b, const
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a),
                                                  __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
+// 32 x 32 x 16: lane (half, l32) gives row or column l32 at elements 8 half .., and ends with rows 8 (i / 4) + 4 half + i % 4 of
+// column l32.  Half the operand reads of 16 x 16 x 32 for the same products, and a quarter of its cycles at the vector issue
+// instead of a half.
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+__device__ __forceinline__ f32x16 mfma32_bf16(const u32x4& a, const u32x4& b, const f32x16& c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
+}
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   const zp_f32x2 f = {lo, hi};
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, zp_bf16x2));

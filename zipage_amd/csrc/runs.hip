@@ -399,10 +399,6 @@ template <int CH, int FLIP, int GAP> struct Staged {
     return (r >> 3) * kLoad + (r >> 2 & 1) * 512 + (r & 3) * 64 + (p ^ FLIP * (r >> 2 & 1)) * 16;
   }
 };
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-__device__ __forceinline__ f32x16 mfma32_bf16(const u32x4& a, const u32x4& b, const f32x16& c) {
-  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-}
 template <int KS, int VB> struct FlowStage {                   // 16 KS elements of a key, 32 VB of a value
   typedef Staged<2 * KS, 1, KS == 8 ? 16 : 32> K;
   typedef Staged<4 * VB, 2, 0> V;
