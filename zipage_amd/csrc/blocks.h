@@ -181,4 +181,53 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
   return (sg.row - row0) / kBlock + seg + b;
 }
 
+// ------------------------------------------------------------------ runs in pieces
+// A head walks its blocks one after the other, 2.5 us each whatever else the chip does, and a few heads leave most CUs idle.
+// The state behind a piece of a run is (decays of the piece) * (the state before it) + what the piece adds to none, so few
+// heads walk their runs in pieces side by side:
+//
+//   sums     what each piece but the last adds, and its decays: a wave 16 rows of the state, nothing waits for a state
+//   states   the states between pieces, from the first to the last, an element of the state per thread and element
+//   blocks   as without pieces, each from its state on
+//
+// Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) allow.  Blocks of the sums cost about
+// 0.3 of the others', the two launches as much as four blocks: where that is more than what is saved, runs stay whole.
+constexpr int kPieceGroups = 256, kPieceStates = 512, kLeastPiece = 4;
+struct Pieces {
+  int blocks = 0, most = 1;      // of a piece, 0: runs are whole; pieces of the longest run at most
+  float* states = nullptr;
+};
+inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest) {
+  Pieces p;
+  const int64_t all = (longest + kBlock - 1) / kBlock;
+  if (segments * heads * 2 > kPieceGroups) return p;
+  for (int64_t m = kLeastPiece; m < all; ++m) {
+    const int64_t most = (all + m - 1) / m, slots = rows / (kBlock * m) + segments;
+    if ((segments * most < slots ? segments * most : slots) * heads > kPieceGroups || slots * heads > kPieceStates) continue;
+    if (m * 13 + 40 < all * 10) p.blocks = (int)m, p.most = (int)most;
+    return p;
+  }
+  return p;
+}
+// Piece c of a run: the segment that it is, whether it is the last; of segments that have fewer none is left.  Its place among
+// the states, a run's pieces one after the other: enough room, as with the blocks.
+struct Piece {
+  Segment sg;
+  bool last;
+  int64_t slot;
+  __device__ __forceinline__ Piece(const Pieces& p, int row0, const Segment& whole, int seg, int c) : sg(whole), last(true), slot(0) {
+    if (p.blocks == 0) return;
+    const int tokens = p.blocks * kBlock, from = c * tokens;
+    sg.row += from;
+    sg.count = min(whole.count - from, tokens);
+    last = from + tokens >= whole.count;
+    slot = (whole.row - row0) / tokens + seg + c;
+  }
+};
+// States between pieces lie as the waves that own 16 columns hold them: [columns / 16][rows / 16][64 lanes][4].
+template <int KT> __device__ __forceinline__ void load_piece_state(f32x4 (&S)[KT][1], const float* state, int wave) {
+#pragma unroll
+  for (int kt = 0; kt < KT; ++kt) S[kt][0] = *(const f32x4*)(state + ((wave * KT + kt) * 64 + (threadIdx.x & 63)) * 4);
+}
+
 }  // namespace

@@ -17,6 +17,7 @@ struct RunArgs {
   zp_linear d;
   float* ws;
   int row0;      // first token row of the first segment
+  Pieces pieces;
 };
 
 // G q and the keys as left operands, P's planes, the block's decays; whole KBs
@@ -138,6 +139,111 @@ __global__ __launch_bounds__(256, 4) void linear_prepare_kernel(RunArgs ra) {
   }
 }
 
+// ------------------------------------------------------------------ runs in pieces
+// A piece's state: its sums, or the state before it, then its decays.
+__host__ __device__ inline constexpr int piece_floats(int dk, int dv) { return dk * dv + dk; }
+
+// What a piece adds to the state and its decays; pieces behind which there is another, whose blocks are whole.  A wave 16
+// rows of the state, so that every key is split once; value rows of four blocks come into LDS while four are worked on.
+template <int KT, int NW>
+__global__ __launch_bounds__(64 * KT) void linear_sums_kernel(RunArgs ra) {
+  constexpr int kAhead = 4, dk = 16 * KT, dv = 16 * NW, size = block_floats(dk), kRows = kBlock * dv;
+  __shared__ __align__(16) uint16_t rows[2][kAhead * kRows];
+  const zp_linear& a = ra.d;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int kt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = blockIdx.x % (ra.pieces.most - 1), unit = blockIdx.x / (ra.pieces.most - 1), h = unit % a.heads, seg = unit / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const Piece piece(ra.pieces, ra.row0, whole, seg, c);
+  if (piece.last) return;
+  const Segment& sg = piece.sg;
+  const int blocks = ra.pieces.blocks;
+  const int64_t stride = (int64_t)a.heads * size;
+  const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
+  const float* const keys = base + kBlock * dk + (kt * 64 + lane) * 4;
+  const float* const decays = base + 2 * kBlock * dk + kPairFloats + 16 * kt + 4 * g;
+  f32x4 k[2][kAhead], dec[2][kAhead];
+  auto request = [&](int b0, int to) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int b = min(b0 + i, blocks - 1);                   // the last may come again
+      k[to][i] = *(const f32x4*)(keys + b * stride);
+      dec[to][i] = *(const f32x4*)(decays + b * stride);
+    }
+    for (int u = kt; u < kAhead * NW / 2; u += KT) {
+      const int i = u / (NW / 2), part = u % (NW / 2), b = min(b0 + i, blocks - 1), s = part * 64 + lane, row = s / (dv / 8);
+      const StageLoads from((const char*)a.in + (int64_t)(sg.row + b * kBlock) * a.in_stride * 2, kBlock * a.in_stride * 2);
+      from.ld(rows[to] + i * kRows + part * 512, row * (int)a.in_stride * 2 + (s - row * (dv / 8)) * 16, (a.v_at + h * dv) * 2);
+    }
+  };
+  f32x4 S[NW], D = {1.f, 1.f, 1.f, 1.f};
+#pragma unroll
+  for (int nc = 0; nc < NW; ++nc) S[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto work = [&](int b0, int at) {
+    wait_and_meet();
+    if (b0 + kAhead < blocks) request(b0 + kAhead, at ^ 1);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (b0 + i >= blocks) break;
+      const Planes x(k[at][i]);
+      const uint16_t* const from = rows[at] + i * kRows + (4 * g + (l16 >> 2)) * dv + (l16 & 3) * 4;
+      D *= dec[at][i];
+#pragma unroll
+      for (int nc = 0; nc < NW; ++nc) {
+        const uint2 v = read_transposed(from + nc * 16);
+        S[nc] *= dec[at][i];
+        S[nc] = mfma_bf16(u32x4{x.lo.x, x.lo.y, 0u, 0u}, u32x4{v.x, v.y, v.x, v.y}, S[nc]);
+        S[nc] = mfma_bf16(u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y}, u32x4{v.x, v.y, v.x, v.y}, S[nc]);
+      }
+    }
+  };
+  request(0, 0);
+#pragma unroll 1
+  for (int b0 = 0; b0 < blocks; b0 += 2 * kAhead) {
+    work(b0, 0);
+    if (b0 + kAhead < blocks) work(b0 + kAhead, 1);
+  }
+  float* const to = ra.pieces.states + (piece.slot * a.heads + h) * piece_floats(dk, dv);
+#pragma unroll
+  for (int nc = 0; nc < NW; ++nc) *(f32x4*)(to + ((nc * KT + kt) * 64 + lane) * 4) = S[nc];
+  if (l16 == 0) *(f32x4*)(to + dk * dv + 16 * kt + 4 * g) = D;
+}
+
+// From sums to the states before the pieces, in place; a thread four rows of a column.
+template <int KT, int NW>
+__global__ __launch_bounds__(256) void linear_states_kernel(RunArgs ra) {
+  constexpr int dk = 16 * KT, dv = 16 * NW, kAhead = 4;
+  const zp_linear& a = ra.d;
+  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads, f = blockIdx.y * 256 + threadIdx.x;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const int lane = f & 63, kt = (f >> 6) % KT, nc = (f >> 6) / KT, row = 16 * kt + 4 * (lane >> 4);
+  const float* const state = a.state + ((int64_t)whole.slot * a.heads + h) * ((int64_t)dk * dv) + row * dv + nc * 16 + (lane & 15);
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  if (whole.start != 0)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = state[r * dv];
+  const int tokens = ra.pieces.blocks * kBlock, count = (whole.count + tokens - 1) / tokens;
+  const int64_t stride = (int64_t)a.heads * piece_floats(dk, dv);
+  float* const at = ra.pieces.states + Piece(ra.pieces, ra.row0, whole, seg, 0).slot * stride + (int64_t)h * piece_floats(dk, dv);
+  for (int c0 = 0; c0 < count; c0 += kAhead) {
+    f32x4 x[kAhead], D[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int c = min(c0 + i, max(count - 2, 0));            // the last piece has no sums
+      x[i] = *(const f32x4*)(at + c * stride + f * 4);
+      D[i] = *(const f32x4*)(at + c * stride + dk * dv + row);
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+      if (c0 + i < count) {
+        *(f32x4*)(at + (c0 + i) * stride + f * 4) = S;
+        S = S * D[i] + x[i];
+      }
+  }
+}
+
 // A head's blocks, one after the other, a wave 16 columns of the state.  Operands in fp32 enter the bf16 matrix cores in three
 // planes each, as in delta_blocks: the state is split where it is updated, what comes from memory by all waves together,
 // a block ahead; value rows are bf16 as they come.  Rows are normed and stored behind the next meeting of the
@@ -157,13 +263,17 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_blocks_kernel(RunArgs ra) {
   float* const rest = split + 2 * kSplit;      // [3][kRest]
   float* const planes = rest + 3 * kRest;      // [2][kPlanes]
   float* const red = planes + 2 * kPlanes;     // [2][NW * 16]
-  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
-  const Segment sg = segment_of(a.seg, seg);
-  if (sg.count <= 0 || sg.row < ra.row0) return;
+  const int unit = blockIdx.x / ra.pieces.most, h = unit % a.heads, seg = unit / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const Piece piece(ra.pieces, ra.row0, whole, seg, blockIdx.x % ra.pieces.most);
+  const Segment& sg = piece.sg;
+  if (sg.count <= 0) return;
   float* const state = a.state + ((int64_t)sg.slot * a.heads + h) * ((int64_t)dk * dv);
   const int col0 = wave * 16;
   f32x4 S[KT][1];
-  load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
+  if (ra.pieces.blocks) load_piece_state(S, ra.pieces.states + (piece.slot * a.heads + h) * piece_floats(dk, dv), wave);
+  else load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
   const float nrm = a.norm[h * dv + col0 + l16];
   const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
   const int64_t stride = (int64_t)a.heads * size;
@@ -304,7 +414,7 @@ __global__ __launch_bounds__(64 * NW, 2) void linear_blocks_kernel(RunArgs ra) {
   const f32x4 ss = block_squares_total<NW>(red + ((blocks - 1) & 1) * NW * kBlock);
 #pragma unroll
   for (int r = 0; r < 4; ++r) finish(blocks - 1, r, ss);
-  store_state<KT, 1>(S, state, dv, col0);
+  if (piece.last) store_state<KT, 1>(S, state, dv, col0);
 }
 
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
@@ -315,7 +425,14 @@ template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
     zp_set_error("linear_runs: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((linear_blocks_kernel<KT, NW>), dim3((unsigned)((int64_t)ra.d.seg.n * ra.d.heads)), dim3(64 * NW), smem, st, ra);
+  const int64_t units = (int64_t)ra.d.seg.n * ra.d.heads;
+  if (ra.pieces.blocks) {
+    hipLaunchKernelGGL((linear_sums_kernel<KT, NW>), dim3((unsigned)(units * (ra.pieces.most - 1))), dim3(64 * KT), 0, st, ra);
+    ZP_LAUNCH_CHECK();
+    hipLaunchKernelGGL((linear_states_kernel<KT, NW>), dim3((unsigned)units, KT * NW / 4), dim3(256), 0, st, ra);
+    ZP_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL((linear_blocks_kernel<KT, NW>), dim3((unsigned)(units * ra.pieces.most)), dim3(64 * NW), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -330,9 +447,15 @@ template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
 
 }  // namespace
 
+static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads, int dk) {
+  return (rows / kBlock + segments) * heads * block_floats(dk) * 4;
+}
+
+// With room for the states between pieces of few heads' runs, whatever the values' size and the longest run.
 extern "C" int64_t zp_linear_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk) {
   if (rows < 0 || segments < 0 || heads <= 0 || dk <= 0) return -1;
-  return ((int64_t)rows / kBlock + segments) * heads * block_floats(dk) * 4;
+  const bool pieces = (int64_t)segments * heads * 2 <= kPieceGroups && dk <= 128;
+  return blocks_bytes(rows, segments, heads, dk) + (pieces ? (int64_t)kPieceStates * piece_floats(dk, 128) * 4 : 0);
 }
 
 extern "C" int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t longest, void* workspace,
@@ -350,9 +473,12 @@ extern "C" int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t 
   ZP_REQUIRE(a.in && a.decay && (a.rot == 0 || a.freqs) && a.norm && a.state && a.out && a.seg.rows && a.seg.counts &&
                  a.seg.slots && a.seg.starts && aligned16(a.in) && aligned16(a.low) && (!a.low || aligned16(a.decay)) &&
                  aligned16(a.state) && aligned16(workspace), "linear_runs: null or unaligned pointer");
-  ZP_REQUIRE(workspace && workspace_bytes >= zp_linear_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk),
-             "linear_runs: workspace too small");
-  RunArgs ra = {a, (float*)workspace, first_row};
+  const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk);
+  ZP_REQUIRE(workspace && workspace_bytes >= whole, "linear_runs: workspace too small");
+  RunArgs ra = {a, (float*)workspace, first_row, {}};
+  if (workspace_bytes >= zp_linear_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk))    // else runs stay whole
+    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest);
+  ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   hipStream_t st = (hipStream_t)stream;
   hipLaunchKernelGGL(linear_prepare_kernel, dim3((unsigned)((longest + kBlock - 1) / kBlock), (unsigned)a.heads, (unsigned)a.seg.n),

@@ -21,6 +21,7 @@ struct RunArgs {
   float* aux;    // per block and head: kAux floats
   float4* scal;  // per token row from row0 on and head: F, x, m, m before the block
   int row0;
+  Pieces pieces;
 };
 // D's planes as a left operand, then a, write factors, e^{-m}, row sums of D (16 each), the keep factor
 constexpr int kAux = 512, kInter = kPairFloats, kWrite = kInter + 16, kFloor = kWrite + 16, kSum = kFloor + 16, kKeep = kSum + 16;
@@ -120,6 +121,133 @@ __global__ __launch_bounds__(256) void mlstm_prepare_kernel(RunArgs ra) {
   }
 }
 
+// ------------------------------------------------------------------ runs in pieces
+// A piece's state: its sums, or the state before it; the same of the normaliser; the factor that keeps what was before.
+__host__ __device__ inline constexpr int piece_floats(int dk, int dv) { return dk * dv + dk + 4; }
+
+// What a piece adds to the state and the normaliser; pieces behind which there is another, whose blocks are whole.  A wave 16
+// rows of the state, so that every key is weighted and split once; key and value rows of four blocks come into LDS while
+// four are worked on.
+template <int KT, int NW>
+__global__ __launch_bounds__(64 * KT) void mlstm_sums_kernel(RunArgs ra) {
+  constexpr int kAhead = 4, dk = 16 * KT, dv = 16 * NW, kKeys = kBlock * dk, kRows = kBlock * dv;
+  __shared__ __align__(16) uint16_t krows[2][kAhead * kKeys], vrows[2][kAhead * kRows];
+  const zp_mlstm& a = ra.d;
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int kt = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = blockIdx.x % (ra.pieces.most - 1), unit = blockIdx.x / (ra.pieces.most - 1), h = unit % a.heads, seg = unit / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const Piece piece(ra.pieces, ra.row0, whole, seg, c);
+  if (piece.last) return;
+  const Segment& sg = piece.sg;
+  const int blocks = ra.pieces.blocks;
+  const float* const aux = ra.aux + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * kAux;
+  const int64_t stride = (int64_t)a.heads * kAux;
+  f32x4 wr[2][kAhead];
+  float keep[2][kAhead];
+  // rows of `cols` columns from column `at` on
+  auto stage = [&](auto cols_, uint16_t* to, int b, int part, int at) {
+    constexpr int cols = cols_.value;
+    const int s = part * 64 + lane, row = s / (cols / 8);
+    const StageLoads from((const char*)a.in + (int64_t)(sg.row + b * kBlock) * a.in_stride * 2, kBlock * a.in_stride * 2);
+    from.ld(to + part * 512, row * (int)a.in_stride * 2 + (s - row * (cols / 8)) * 16, at * 2);
+  };
+  auto request = [&](int b0, int to) {
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int b = min(b0 + i, blocks - 1);                   // the last may come again
+      wr[to][i] = *(const f32x4*)(aux + b * stride + kWrite + 4 * g);
+      keep[to][i] = aux[b * stride + kKeep];
+    }
+    for (int u = kt; u < kAhead * KT / 2; u += KT)
+      stage(std::integral_constant<int, dk>(), krows[to] + u / (KT / 2) * kKeys, min(b0 + u / (KT / 2), blocks - 1), u % (KT / 2), a.k_at + h * dk);
+    for (int u = kt; u < kAhead * NW / 2; u += KT)
+      stage(std::integral_constant<int, dv>(), vrows[to] + u / (NW / 2) * kRows, min(b0 + u / (NW / 2), blocks - 1), u % (NW / 2), a.v_at + h * dv);
+  };
+  f32x4 S[NW];
+  float n = 0.f, kept = 1.f;
+#pragma unroll
+  for (int nc = 0; nc < NW; ++nc) S[nc] = f32x4{0.f, 0.f, 0.f, 0.f};
+  auto work = [&](int b0, int at) {
+    wait_and_meet();
+    if (b0 + kAhead < blocks) request(b0 + kAhead, at ^ 1);
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      if (b0 + i >= blocks) break;
+      const float f = keep[at][i];
+      const int row = 4 * g + (l16 >> 2);
+      const f32x4 k = read_columns((const char*)(krows[at] + i * kKeys + row * dk + 16 * kt + (l16 & 3) * 4)) * wr[at][i];
+      const uint16_t* const from = vrows[at] + i * kRows + row * dv + (l16 & 3) * 4;
+      const Planes x(k);
+      n = fmaf(n, f, (k[0] + k[1]) + (k[2] + k[3]));
+      kept *= f;
+#pragma unroll
+      for (int nc = 0; nc < NW; ++nc) {
+        const uint2 v = read_transposed(from + nc * 16);
+        S[nc] *= f;
+        S[nc] = mfma_bf16(u32x4{x.lo.x, x.lo.y, 0u, 0u}, u32x4{v.x, v.y, v.x, v.y}, S[nc]);
+        S[nc] = mfma_bf16(u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y}, u32x4{v.x, v.y, v.x, v.y}, S[nc]);
+      }
+    }
+  };
+  request(0, 0);
+#pragma unroll 1
+  for (int b0 = 0; b0 < blocks; b0 += 2 * kAhead) {
+    work(b0, 0);
+    if (b0 + kAhead < blocks) work(b0 + kAhead, 1);
+  }
+  n += lane_xor16(n);
+  n += lane_xor32(n);
+  float* const to = ra.pieces.states + (piece.slot * a.heads + h) * piece_floats(dk, dv);
+#pragma unroll
+  for (int nc = 0; nc < NW; ++nc) *(f32x4*)(to + ((nc * KT + kt) * 64 + lane) * 4) = S[nc];
+  if (g == 0) to[dk * dv + 16 * kt + l16] = n;
+  if (threadIdx.x == 0) to[dk * dv + dk] = kept;
+}
+
+// From sums to the states before the pieces, in place; a thread four rows of a column, or a row of the normaliser.
+template <int KT, int NW>
+__global__ __launch_bounds__(256) void mlstm_states_kernel(RunArgs ra) {
+  constexpr int dk = 16 * KT, dv = 16 * NW, kAhead = 4;
+  const zp_mlstm& a = ra.d;
+  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads, f = blockIdx.y * 256 + threadIdx.x;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const int lane = f & 63, kt = (f >> 6) % KT, nc = (f >> 6) / KT;
+  const float* const state = a.state + ((int64_t)whole.slot * a.heads + h) * ((int64_t)dk * dv + dk + 4);
+  const bool fresh = whole.start == 0, norm = f < dk;
+  f32x4 S = {0.f, 0.f, 0.f, 0.f};
+  float n = 0.f;
+  if (!fresh) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) S[r] = state[(16 * kt + 4 * (lane >> 4) + r) * dv + nc * 16 + (lane & 15)];
+    if (norm) n = state[dk * dv + f];
+  }
+  const int tokens = ra.pieces.blocks * kBlock, count = (whole.count + tokens - 1) / tokens;
+  const int64_t stride = (int64_t)a.heads * piece_floats(dk, dv);
+  float* const at = ra.pieces.states + Piece(ra.pieces, ra.row0, whole, seg, 0).slot * stride + (int64_t)h * piece_floats(dk, dv);
+  for (int c0 = 0; c0 < count; c0 += kAhead) {
+    f32x4 x[kAhead];
+    float y[kAhead], kept[kAhead];
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i) {
+      const int c = min(c0 + i, max(count - 2, 0));            // the last piece has no sums
+      x[i] = *(const f32x4*)(at + c * stride + f * 4);
+      y[i] = norm ? at[c * stride + dk * dv + f] : 0.f;
+      kept[i] = at[c * stride + dk * dv + dk];
+    }
+#pragma unroll
+    for (int i = 0; i < kAhead; ++i)
+      if (c0 + i < count) {
+        *(f32x4*)(at + (c0 + i) * stride + f * 4) = S;
+        if (norm) at[(c0 + i) * stride + dk * dv + f] = n;
+        S = S * kept[i] + x[i];
+        n = fmaf(n, kept[i], y[i]);
+      }
+  }
+}
+
 // A wave owns 16 columns of the state, which is split into planes where it is updated (8 prompts of 2048 tokens, 16 heads
 // of 128 x 128, with the kernels above: 595 us with products on the fp32 matrix cores, 440; error of the state against 64
 // bits 3.1e-7 -> 2.9e-7 of its size).  What bounds it is a wave's chain of work from meeting to meeting: the normaliser is
@@ -133,9 +261,12 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   constexpr int dk = 16 * KT, dv = 16 * NW, PR = dk / 8, J = KT / 2;      // PR: pieces per row of Q and K
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
-  const Segment sg = segment_of(a.seg, seg);
-  if (sg.count <= 0 || sg.row < ra.row0) return;
+  const int unit = blockIdx.x / ra.pieces.most, h = unit % a.heads, seg = unit / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const Piece piece(ra.pieces, ra.row0, whole, seg, blockIdx.x % ra.pieces.most);
+  const Segment& sg = piece.sg;
+  if (sg.count <= 0) return;
   constexpr int v_bytes = kBlock * dv * 2, stage = 2 * kBlock * dk * 2 + v_bytes + kAux * 4;
   float (*const red)[NW * kBlock] = (float (*)[NW * kBlock])(lds_raw + 2 * stage);
   float (*const den)[kBlock] = (float (*)[kBlock])(red + 2);
@@ -145,8 +276,14 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   const bool fresh = sg.start == 0;
   const int col0 = wave * 16;
   f32x4 S[KT][1];
-  load_state<KT, 1>(S, state, dv, col0, fresh);
-  for (int c = tid; c < dk; c += blockDim.x) nl[0][c] = fresh ? 0.f : nstate[c];
+  if (ra.pieces.blocks) {
+    const float* const from = ra.pieces.states + (piece.slot * a.heads + h) * piece_floats(dk, dv);
+    load_piece_state(S, from, wave);
+    for (int c = tid; c < dk; c += blockDim.x) nl[0][c] = from[dk * dv + c];
+  } else {
+    load_state<KT, 1>(S, state, dv, col0, fresh);
+    for (int c = tid; c < dk; c += blockDim.x) nl[0][c] = fresh ? 0.f : nstate[c];
+  }
   const float nrm = a.norm[h * dv + col0 + l16] * a.out_scale;
   const int blocks = (sg.count + kBlock - 1) / kBlock;
   const float* const aux0 = ra.aux + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * kAux;
@@ -287,6 +424,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
   }
   wait_and_meet();
   finish(blocks - 1);
+  if (!piece.last) return;
   store_state<KT, 1>(S, state, dv, col0);
   for (int c = tid; c < dk; c += blockDim.x) nstate[c] = nl[blocks & 1][c];
 }
@@ -294,7 +432,14 @@ __global__ __launch_bounds__(64 * NW, 2) void mlstm_blocks_kernel(RunArgs ra) {
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   constexpr int dk = 16 * KT, dv = 16 * NW;
   constexpr size_t smem = 2 * (2 * kBlock * dk * 2 + kBlock * dv * 2 + kAux * 4) + 2 * 4 * (NW * kBlock + kBlock + dk);
-  hipLaunchKernelGGL((mlstm_blocks_kernel<KT, NW>), dim3((unsigned)((int64_t)ra.d.seg.n * ra.d.heads)), dim3(64 * NW), smem, st, ra);
+  const int64_t units = (int64_t)ra.d.seg.n * ra.d.heads;
+  if (ra.pieces.blocks) {
+    hipLaunchKernelGGL((mlstm_sums_kernel<KT, NW>), dim3((unsigned)(units * (ra.pieces.most - 1))), dim3(64 * KT), 0, st, ra);
+    ZP_LAUNCH_CHECK();
+    hipLaunchKernelGGL((mlstm_states_kernel<KT, NW>), dim3((unsigned)units, KT * NW / 4), dim3(256), 0, st, ra);
+    ZP_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL((mlstm_blocks_kernel<KT, NW>), dim3((unsigned)(units * ra.pieces.most)), dim3(64 * NW), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -316,9 +461,15 @@ template <int KT> int launch_runs(const RunArgs& ra, int longest, hipStream_t st
 
 }  // namespace
 
+static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads) {
+  return ((rows / kBlock + segments) * kAux + rows * 4) * heads * 4;
+}
+
+// With room for the states between pieces of few heads' runs, whatever the sizes and the longest run.
 extern "C" int64_t zp_mlstm_runs_workspace(int32_t rows, int32_t segments, int32_t heads) {
   if (rows < 0 || segments < 0 || heads <= 0) return -1;
-  return (((int64_t)rows / kBlock + segments) * kAux + (int64_t)rows * 4) * heads * 4;
+  const bool pieces = (int64_t)segments * heads * 2 <= kPieceGroups;
+  return blocks_bytes(rows, segments, heads) + (pieces ? (int64_t)kPieceStates * piece_floats(128, 128) * 4 : 0);
 }
 
 extern "C" int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t longest, void* workspace,
@@ -337,9 +488,12 @@ extern "C" int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t lo
   ZP_REQUIRE(a.in && a.gates && a.i_bias && a.f_bias && a.norm && a.state && a.out && a.seg.rows && a.seg.counts &&
                  a.seg.slots && a.seg.starts && aligned16(a.in) && aligned16(a.state) && aligned16(workspace),
              "mlstm_runs: null or unaligned pointer");
-  ZP_REQUIRE(workspace && workspace_bytes >= zp_mlstm_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads),
-             "mlstm_runs: workspace too small");
-  RunArgs ra = {a, (float*)workspace, nullptr, first_row};
+  const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads);
+  ZP_REQUIRE(workspace && workspace_bytes >= whole, "mlstm_runs: workspace too small");
+  RunArgs ra = {a, (float*)workspace, nullptr, first_row, {}};
+  if (workspace_bytes >= zp_mlstm_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads))           // else runs stay whole
+    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest);
+  ra.pieces.states = (float*)workspace + whole / 4;
   ra.scal = (float4*)(ra.aux + ((int64_t)(a.seg.num_rows - first_row) / kBlock + a.seg.n) * a.heads * kAux);
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   hipStream_t st = (hipStream_t)stream;
