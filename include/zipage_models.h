@@ -215,7 +215,9 @@ typedef struct {
 int zp_mlstm_scan(const zp_mlstm* args, int32_t dtype, void* stream);
 /* The same for long runs, 16 tokens at a time on the matrix cores (fp32): bfloat16, dk 32, 64 or 128, dv up
  * to 128, rows given in rising order from first_row on, none longer than `longest`.  `workspace`:
- * zp_mlstm_runs_workspace() bytes for the rows from first_row to the end. */
+ * zp_mlstm_runs_workspace() bytes for the rows from first_row to the end.  Of those, up to 128 (run, head) pairs have room
+ * for states between pieces of runs, which are then worked on side by side; without it (the first ((rows / 16 + segments)
+ * * 512 + rows * 4) * heads * 4 bytes are needed) runs stay whole. */
 int64_t zp_mlstm_runs_workspace(int32_t rows, int32_t segments, int32_t heads);
 int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t longest, void* workspace,
                   int64_t workspace_bytes, int32_t dtype, void* stream);
@@ -239,7 +241,8 @@ typedef struct {
 int zp_delta_scan(const zp_delta* args, int32_t dtype, void* stream);
 /* The same for long runs (of taps - 1 tokens at least), 16 tokens at a time on the matrix cores (fp32):
  * bfloat16, dk 32, 64 or 128, dv up to 128, rows given in rising order from first_row on, none longer than
- * `longest`.  `workspace`: zp_delta_runs_workspace() bytes for the rows from first_row to the end. */
+ * `longest`.  `workspace`: zp_delta_runs_workspace() bytes for the rows from first_row to the end, with
+ * room for pieces of runs as above where dk == dv. */
 int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk, int32_t dv);
 int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
                   int64_t workspace_bytes, int32_t dtype, void* stream);
@@ -265,7 +268,7 @@ typedef struct {
 int zp_linear_scan(const zp_linear* args, int32_t dtype, void* stream);
 /* The same for long runs, 16 tokens at a time on the matrix cores (fp32): bfloat16, dk 32, 64 or 128, dv up
  * to 128, rows given in rising order from first_row on, none longer than `longest`.  `workspace`:
- * zp_linear_runs_workspace() bytes for the rows from first_row to the end. */
+ * zp_linear_runs_workspace() bytes for the rows from first_row to the end, with room for pieces of runs as above. */
 int64_t zp_linear_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk);
 int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t longest, void* workspace,
                    int64_t workspace_bytes, int32_t dtype, void* stream);

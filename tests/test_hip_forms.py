@@ -254,6 +254,59 @@ def test_causal_attention(dev, H, G, D, lens=((1, 1), (31, 31), (128, 128), (129
     assert bool(((got.view(N, H, D).cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * vv.abs().max()).all())
 
 
+# ------------------------------------------------------------------ recurrences over runs, in pieces
+# Few heads walk long runs in pieces of at least four blocks of 16 tokens: one run, runs of which some have fewer pieces than
+# others or none, pieces whose last has one token or a whole block, states of earlier tokens and none; key and value sizes
+# apart (the delta rule stays whole there).  Token by token in fp32 the same sums stand in another order.
+@pytest.mark.parametrize("kind", ["delta", "memory", "linear", "retention"])
+@pytest.mark.parametrize("H,D,V,lens", [(1, 128, 128, (700,)), (16, 128, 128, (705, 161, 64, 1377)), (2, 32, 32, (16, 1025, 31)),
+                                        (24, 64, 96, (1024, 496)), (40, 64, 64, (400, 15, 401)), (128, 32, 32, (640,))])
+def test_recurrences_in_pieces(dev, kind, H, D, V, lens):
+    import types
+    from zipage_amd.engine.qwen3 import Segments
+    from zipage_amd.layers import ChannelDelta, LinearAttention, MatrixMemory, Rotary
+    W, n, rows = 64, len(lens), sum(lens)
+    m = {"delta": lambda: ChannelDelta(W, H, H // 2 if H % 2 == 0 else H, D, V, 4, 1e-3),
+         "memory": lambda: MatrixMemory(W, H, D, V, 15.0, 1e-3),
+         "linear": lambda: LinearAttention(W, H, D, V, 1e-3, q_scale=D ** -0.5, tau=16.0, weighted=True),
+         "retention": lambda: LinearAttention(W, H, D, V, 1e-3, k_scale=D ** -0.5, rotary=Rotary(1e4, D),
+                                              decay=tuple(1 - 2.0 ** (-3 - 4 * i / H) for i in range(H)))}[kind]()
+    shapes = m.shapes(8, 8) if kind == "delta" else m.shapes(8) if kind == "linear" else m.shapes()
+    w = {k: _rand(*s, seed=i) * s[-1] ** -0.5 for i, (k, s) in enumerate(shapes.items())}
+    if kind == "memory":
+        w["f.b"] = (3 + _rand(H, seed=50).float()).to(BF16)
+    if kind == "linear":
+        w["a2.b"] = (1 + _rand(H * D, seed=51).float()).to(BF16)
+    if kind == "delta":
+        w["dt_bias"] = (_rand(H * D, seed=52).float() - 3).to(BF16)
+    into, _ = m.load(w, BF16, dev, W)
+    h = _rand(rows, W, seed=60).to(dev)
+    proj = (h.float() @ into.to(dev).float().T).to(BF16)
+    t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
+    first, starts = [sum(lens[:i]) for i in range(n)], [0 if i % 2 == 0 else 333 for i in range(n)]
+
+    def scan(runs):
+        state = m.allocate(n + 1, BF16, dev)
+        S = state[0] if kind == "delta" else state
+        S.copy_((0.1 * _rand(*S.shape, seed=61).float()).to(dev))
+        if kind == "delta":
+            state[1].copy_(_rand(*state[1].shape, seed=62))
+        seg = Segments(t(first), t(lens), t(list(range(n, 0, -1))), t(starts), longest=max(lens))
+        out = torch.empty(rows, m.out_columns, dtype=BF16, device=dev)
+        ctx = types.SimpleNamespace(segments=None if runs else seg, run_segments=seg if runs else None)
+        m.scan(*([h] if kind == "memory" else []), proj, state, ctx, out)
+        return out.float(), S.double(), state[1] if kind == "delta" else None
+    (got, gs, gt), (want, ws, wt) = scan(True), scan(False)
+    # the state: sums of up to 1400 terms in fp32, each way within 2^-24 sqrt(1400) of their size, decays of 2^-23 each token
+    # that forgets little; the token-by-token form takes its exponentials from another function
+    assert float((gs - ws).norm() / ws.norm()) < 2.0 ** -13
+    # rows: bf16 rounds both to 2^-9, one step apart where they lie on either side; small denominators amplify the rest
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -8
+    assert bool(((got - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -6 * want.square().mean().sqrt()).float().mean() > 0.999)
+    if gt is not None:
+        assert torch.equal(gt[1:], wt[1:])       # the convolutions' last inputs
+
+
 # ------------------------------------------------------------------ rotary store of heads of 128
 # aligned rows take sixteen lanes a vector, fewer than 2^18 of them with a workgroup per sixteen; others take a wave a vector
 @pytest.mark.parametrize("N,Hq,Hkv", [(1, 1, 1), (37, 32, 8), (700, 5, 2), (2047, 64, 32), (2048, 64, 32)])

@@ -183,28 +183,30 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 
 // ------------------------------------------------------------------ runs in pieces
 // A head walks its blocks one after the other, 2.5 us each whatever else the chip does, and a few heads leave most CUs idle.
-// The state behind a piece of a run is (decays of the piece) * (the state before it) + what the piece adds to none, so few
+// The state behind a piece of a run is (what the piece keeps) * (the state before it) + what the piece adds to none, so few
 // heads walk their runs in pieces side by side:
 //
-//   sums     what each piece but the last adds, and its decays: a wave 16 rows of the state, nothing waits for a state
-//   states   the states between pieces, from the first to the last, an element of the state per thread and element
+//   sums     what each piece but the last adds and keeps: nothing waits for a state
+//   states   the states between pieces, from the first to the last
 //   blocks   as without pieces, each from its state on
 //
-// Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) allow.  Blocks of the sums cost about
-// 0.3 of the others', the two launches as much as four blocks: where that is more than what is saved, runs stay whole.
-constexpr int kPieceGroups = 256, kPieceStates = 512, kLeastPiece = 4;
+// Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) allow.  Where the sums and the two
+// launches cost more than what is saved, runs stay whole.
+constexpr int kPieceGroups = 256, kPieceStates = 384, kLeastPiece = 4;
 struct Pieces {
   int blocks = 0, most = 1;      // of a piece, 0: runs are whole; pieces of the longest run at most
   float* states = nullptr;
 };
-inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest) {
+inline bool few_heads(int64_t segments, int64_t heads) { return segments * heads * 2 <= kPieceGroups; }
+// The sums take `groups` workgroups per piece and, in tenths of a block, `sum` per block; the rest `fixed` and `state` per piece.
+inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest, int groups, int sum, int fixed, int state) {
   Pieces p;
   const int64_t all = (longest + kBlock - 1) / kBlock;
-  if (segments * heads * 2 > kPieceGroups) return p;
+  if (!few_heads(segments, heads)) return p;
   for (int64_t m = kLeastPiece; m < all; ++m) {
-    const int64_t most = (all + m - 1) / m, slots = rows / (kBlock * m) + segments;
-    if ((segments * most < slots ? segments * most : slots) * heads > kPieceGroups || slots * heads > kPieceStates) continue;
-    if (m * 13 + 40 < all * 10) p.blocks = (int)m, p.most = (int)most;
+    const int64_t most = (all + m - 1) / m, slots = rows / (kBlock * m) + segments, pieces = segments * most < slots ? segments * most : slots;
+    if (pieces * heads > kPieceGroups || (pieces - segments) * heads * groups > kPieceGroups || slots * heads > kPieceStates) continue;
+    if (m * (10 + sum) + fixed + most * state < all * 10) p.blocks = (int)m, p.most = (int)most;
     return p;
   }
   return p;

@@ -19,6 +19,7 @@ struct RunArgs {
   zp_delta d;
   float* ws;
   int row0;      // first token row of the first segment
+  Pieces pieces;
 };
 
 // [-W | G q] and the keys as left operands, U0 as a result tile, P's planes, the block's decays; whole KBs
@@ -244,6 +245,91 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
   }
 }
 
+// ------------------------------------------------------------------ runs in pieces, of heads with as many keys as values
+// A piece keeps M S of a state S before it, M the product of its blocks' (diag(G_15) - keys^T W).  Its columns walk through
+// the piece as those of a state do, from one on, with nothing of the values.  A piece's state: its sums, or the state before
+// it, then M as a left operand, [rows / 16][columns / 16][64 lanes][4].
+__host__ __device__ inline constexpr int piece_floats(int dk) { return 2 * dk * dk; }
+
+// From sums to the states before the pieces, in place; a wave 16 columns.  The products are those of the blocks, M split by
+// all waves together while the piece before is worked on: 2.4 us a piece.
+template <int KT>
+__global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
+  extern __shared__ __align__(16) float planes[];              // [rows / 16][pairs of columns / 16][3][64 lanes][4]
+  constexpr int dk = 16 * KT, J = KT / 2;
+  const zp_delta& a = ra.d;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  f32x4 S[KT][1], x[KT], add[KT];
+  load_state<KT, 1>(S, a.state + ((int64_t)whole.slot * a.heads + h) * ((int64_t)dk * dk), dk, wave * 16, whole.start == 0);
+  const int tokens = ra.pieces.blocks * kBlock, count = (whole.count + tokens - 1) / tokens;
+  const int64_t stride = (int64_t)a.heads * piece_floats(dk);
+  float* const at = ra.pieces.states + Piece(ra.pieces, ra.row0, whole, seg, 0).slot * stride + (int64_t)h * piece_floats(dk) + lane * 4;
+  auto load = [&](int c) {                                     // this wave's columns of M, for all waves
+#pragma unroll
+    for (int t = 0; t < KT; ++t) x[t] = *(const f32x4*)(at + c * stride + dk * dk + (t * KT + wave) * 256);
+  };
+  auto meet = [] {                                             // LDS alone: what comes from memory and goes there stays on its way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto load_sums = [&](int c, int t) { add[t] = *(const f32x4*)(at + c * stride + (wave * KT + t) * 256); };
+  if (count > 1) {
+    load(0);
+#pragma unroll
+    for (int t = 0; t < KT; ++t) load_sums(0, t);
+  }
+#pragma unroll 1
+  for (int c = 0; c < count; ++c) {
+    const bool more = c + 1 < count;                           // the last piece has no sums
+    u32x4 sp[3][J];
+    meet();                                                    // the planes before these are used up
+    if (more) {
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+        const Planes p(x[t]);
+        float* const to = planes + (t * J + (wave >> 1)) * 768 + lane * 4 + (wave & 1) * 2;
+        *(uint2*)to = p.hi;
+        *(uint2*)(to + 256) = p.mid;
+        *(uint2*)(to + 512) = p.lo;
+      }
+      load(min(c + 1, count - 2));
+    }
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      *(f32x4*)(at + c * stride + (wave * KT + kt) * 256) = S[kt][0];
+      const Planes p(S[kt][0]);
+      const int e = (kt & 1) * 2;
+      sp[0][kt >> 1][e] = p.hi.x, sp[0][kt >> 1][e + 1] = p.hi.y;
+      sp[1][kt >> 1][e] = p.mid.x, sp[1][kt >> 1][e + 1] = p.mid.y;
+      sp[2][kt >> 1][e] = p.lo.x, sp[2][kt >> 1][e + 1] = p.lo.y;
+    }
+    meet();
+    if (!more) break;
+#pragma unroll
+    for (int t = 0; t < KT; t += 2) {                          // two rows of tiles: each product waits for the one before
+      f32x4 y[2] = {add[t], add[t + 1]};
+      load_sums(min(c + 1, count - 2), t);
+      load_sums(min(c + 1, count - 2), t + 1);
+#pragma unroll
+      for (int i = 2; i >= 0; --i)                             // the smallest products first
+#pragma unroll
+        for (int k = 2 - i; k >= 0; --k)
+#pragma unroll
+          for (int j = 0; j < J; ++j)
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+              y[u] = mfma_bf16(*(const u32x4*)(planes + (((t + u) * J + j) * 3 + i) * 256 + lane * 4), sp[k][j], y[u]);
+      S[t][0] = y[0];
+      S[t + 1][0] = y[1];
+    }
+  }
+}
+
 // A head's blocks, one after the other, a wave 16 columns of the state.  On the fp32 matrix cores the products would be the
 // bound (208 of 32 cycles a block on each SIMD, which keep its vector units idle as well), so operands are split into
 // three bf16 planes: the products that count take a quarter of that, beside the vector units.  The state is split
@@ -252,37 +338,54 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
 // chain of work: two per SIMD are all there are (twice the columns per wave, one per SIMD: 2 to 12 % more time in all).
 // 8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1161 -> 1106 us, one of them 566 -> 491; error of the
 // state against 64 bits 4.0e-7 -> 3.6e-7 of its size.
-template <int KT, int NW>
+// SUMS: no state comes in and no rows go out; every second workgroup takes what the piece keeps, where values are none.
+template <int KT, int NW, bool SUMS>
 __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
   const zp_delta& a = ra.d;
   constexpr int dk = 16 * KT, dv = 16 * NW, size = block_floats(dk, dv), J = KT / 2;
   constexpr int kSplit = 3 * kBlock * dk, kRest = size - kSplit;      // floats of a block: operands to be split, the others
   constexpr int kP = kBlock * dv, kG = kP + kPairFloats;              // in the rest, behind U0
-  constexpr int kPlanes = 3 * KT * 384, kMine = (3 * KT + NW - 1) / NW;      // floats of a block's planes; tiles of a wave
+  constexpr int kPlanes = 3 * KT * 384, kMine = ((SUMS ? 2 : 3) * KT + NW - 1) / NW;    // floats of a block's planes; tiles of a wave
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   float* const split = lds;                    // [2][kSplit]
   float* const rest = split + 2 * kSplit;      // [3][kRest]
   float* const planes = rest + 3 * kRest;      // [2][kPlanes]
   float* const red = planes + 2 * kPlanes;     // [2][NW * 16]
-  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
-  const Segment sg = segment_of(a.seg, seg);
-  if (sg.count <= 0 || sg.row < ra.row0) return;
+  const bool keeps = SUMS && blockIdx.x & 1;
+  const int id = SUMS ? blockIdx.x >> 1 : blockIdx.x, most = ra.pieces.most - SUMS, unit = id / most, h = unit % a.heads, seg = unit / a.heads;
+  const Segment whole = segment_of(a.seg, seg);
+  if (whole.count <= 0 || whole.row < ra.row0) return;
+  const Piece piece(ra.pieces, ra.row0, whole, seg, id % most);
+  const Segment& sg = piece.sg;
+  if (SUMS ? piece.last : sg.count <= 0) return;
   const int64_t item = (int64_t)sg.slot * a.heads + h;
   float* const state = a.state + item * ((int64_t)dk * dv);
+  float* const between = ra.pieces.states + (piece.slot * a.heads + h) * piece_floats(dk);
   const int col0 = wave * 16;
   f32x4 S[KT][1];
-  load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) S[kt][0][r] = keeps && 16 * kt + 4 * g + r == col0 + l16 ? 1.f : 0.f;
+  } else if (ra.pieces.blocks) {
+    load_piece_state(S, between, wave);
+  } else {
+    load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
+  }
   const float nrm = a.norm[h * dv + col0 + l16] * a.out_scale;
   const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
   const int64_t stride = (int64_t)a.heads * size;
   const int blocks = (sg.count + kBlock - 1) / kBlock;
+  auto tile_at = [](int i) { return SUMS && i >= KT ? i + KT : i; };      // without those of G q
   auto request = [&](int b) {                  // a block behind the last: nothing is read
     const StageLoads from(base + b * stride, b < blocks ? size * 4 : 0);
+    constexpr int kKBs = size / 256 - (SUMS ? KT : 0);
 #pragma unroll
-    for (int u = 0; u < (size / 256 + NW - 1) / NW; ++u) {
-      const int i = min(wave + u * NW, size / 256 - 1);            // the last may come twice
+    for (int u = 0; u < (kKBs + NW - 1) / NW; ++u) {
+      const int i = tile_at(min(wave + u * NW, kKBs - 1));         // the last may come twice
       float* const to = i < kSplit / 256 ? split + (b & 1) * kSplit + i * 256 : rest + b % 3 * kRest + (i * 256 - kSplit);
       from.ld(to, lane * 16, i * 1024);
     }
@@ -290,10 +393,10 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
   // Planes of a block's tiles: for pairs of those of -W and of G q [3][64 lanes][two tiles' 4], for those of keys
   // [64][hi 4, mid 4], [64][lo 4].  A wave's tile u; the last may be made twice.
   auto tile_of = [&](int b, int u) {
-    return *(const f32x4*)(split + (b & 1) * kSplit + min(wave + u * NW, 3 * KT - 1) * 256 + lane * 4);
+    return *(const f32x4*)(split + (b & 1) * kSplit + tile_at(min(wave + u * NW, (SUMS ? 2 : 3) * KT - 1)) * 256 + lane * 4);
   };
   auto put_planes = [&](int b, int u, const f32x4& x) {
-    const int i = min(wave + u * NW, 3 * KT - 1);
+    const int i = tile_at(min(wave + u * NW, (SUMS ? 2 : 3) * KT - 1));
     const int key = i >= 2 * KT;               // multiplied, not branched on: the products beside stay in one stretch
     float* const to = planes + (b & 1) * kPlanes + (i >> 1) * 768 + (i & 1) * (2 + 382 * key) + lane * 4;
     const Planes p(x);
@@ -338,17 +441,19 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
         W[j & 1][i] = *(const u32x4*)(pl + (j * 3 + i) * 256);
-        Q[j & 1][i] = *(const u32x4*)(pl + ((J + j) * 3 + i) * 256);
+        if constexpr (!SUMS) Q[j & 1][i] = *(const u32x4*)(pl + ((J + j) * 3 + i) * 256);
       }
     };
     operands(0);
     f32x4 U = *(const f32x4*)(mine + wave * 256 + lane * 4), O = {0.f, 0.f, 0.f, 0.f};
-    f32x4 tile = tile_of(b + 1, 0);
-    const f32x4 ss = block_squares_total<NW>(red + ((b - 1) & 1) * NW * kBlock);
+    if (keeps) U = f32x4{0.f, 0.f, 0.f, 0.f};
+    f32x4 tile = tile_of(b + 1, 0), ss;
+    if constexpr (!SUMS) ss = block_squares_total<NW>(red + ((b - 1) & 1) * NW * kBlock);
     request(b + 2);
     const int cnt = min(kBlock, sg.count - b * kBlock);
     const BlockRows low(a.low, sg.row + b * kBlock, cnt, a.low_stride);
     uint16_t next[4];
+    if constexpr (!SUMS)
 #pragma unroll
     for (int r = 0; r < 4; ++r) next[r] = low.ld(low_at + r * (int)a.low_stride * 2, 0);
     __builtin_amdgcn_sched_barrier(0);
@@ -373,22 +478,27 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
 #pragma unroll
         for (int k = 2 - i; k >= 0; --k) {
           U = mfma_bf16(W[j & 1][i], sp[k][j], U);
-          O = mfma_bf16(Q[j & 1][i], sp[k][j], O);
+          if constexpr (!SUMS) O = mfma_bf16(Q[j & 1][i], sp[k][j], O);
         }
+      if constexpr (!SUMS)
 #pragma unroll
-      for (int r = j * 4 / J; r < (j + 1) * 4 / J; ++r) finish(b - 1, r, ss);
+        for (int r = j * 4 / J; r < (j + 1) * 4 / J; ++r) finish(b - 1, r, ss);
 #pragma unroll
       for (int u = j * kMine / J; u < (j + 1) * kMine / J; ++u) {
         put_planes(b + 1, u, tile);
         if (u + 1 < kMine) tile = tile_of(b + 1, u + 1);
       }
-      spread_over_products<12, 4>();
+      spread_over_products<SUMS ? 6 : 12, 4>();
     }
+    u32x4 P;
+    uint2 Pl;
+    if constexpr (!SUMS) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) gate[r] = next[r];
+      for (int r = 0; r < 4; ++r) gate[r] = next[r];
+      P = *(const u32x4*)(mine + kP + lane * 4);
+      Pl = *(const uint2*)(mine + kP + 256 + lane * 2);
+    }
     const PlanePairs u(U);
-    const u32x4 P = *(const u32x4*)(mine + kP + lane * 4);
-    const uint2 Pl = *(const uint2*)(mine + kP + 256 + lane * 2);
     __builtin_amdgcn_sched_barrier(0);
     S[0][0] *= dec[0][0];
     S[1][0] *= dec[0][1];
@@ -406,21 +516,37 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
       }
       spread_over_products<8, 5>();
     }
-    u.add(P, Pl, O);
+    if constexpr (!SUMS) u.add(P, Pl, O);
     split_state(KT - 2);
     split_state(KT - 1);
 #pragma unroll
     for (int i = 0; i < 3; ++i)                // here, not behind the squares
 #pragma unroll
       for (int j = 0; j < J; ++j) settle(sp[i][j]);
-    f32x4 o[1] = {O};
-    block_squares<1>(o, red + (b & 1) * NW * kBlock, wave);
-    done = O;
+    if constexpr (!SUMS) {
+      f32x4 o[1] = {O};
+      block_squares<1>(o, red + (b & 1) * NW * kBlock, wave);
+      done = O;
+    }
   }
   wait_and_meet();
+  if constexpr (SUMS) {
+#pragma unroll
+    for (int kt = 0; kt < KT; ++kt) {
+      if (keeps) {
+        float* const to = between + dk * dk + ((kt * KT + wave) * 64 + (l16 >> 2) * 16 + 4 * g) * 4 + (l16 & 3);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) to[r * 4] = S[kt][0][r];
+      } else {
+        *(f32x4*)(between + ((wave * KT + kt) * 64 + lane) * 4) = S[kt][0];
+      }
+    }
+    return;
+  }
   const f32x4 ss = block_squares_total<NW>(red + ((blocks - 1) & 1) * NW * kBlock);
 #pragma unroll
   for (int r = 0; r < 4; ++r) finish(blocks - 1, r, ss);
+  if (!piece.last) return;
   store_state<KT, 1>(S, state, dv, col0);
   // the last inputs of the head's convolutions (runs are longer than a filter)
   const int taps = a.taps, cw = 2 * dk + dv, hk = h / (a.heads / a.kv_heads);
@@ -428,21 +554,30 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
   for (int i = tid; i < (taps - 1) * cw; i += blockDim.x) {
     const int e = i / cw, c = i - e * cw;
     const int at = c < dk ? hk * dk + c : (c < 2 * dk ? a.kv_heads * dk + hk * dk + c - dk : 2 * a.kv_heads * dk + h * dv + c - 2 * dk);
-    Elem<BF16>::st(tail, i, Elem<BF16>::ld(a.in, (int64_t)(sg.row + max(sg.count - (taps - 1) + e, 0)) * a.in_stride + at));
+    Elem<BF16>::st(tail, i, Elem<BF16>::ld(a.in, (int64_t)(whole.row + max(whole.count - (taps - 1) + e, 0)) * a.in_stride + at));
   }
 }
 
-template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
-  constexpr int kSplit = 3 * kBlock * 16 * KT;
-  constexpr int smem = (3 * block_floats(16 * KT, 16 * NW) - kSplit + 2 * 3 * KT * 384 + 2 * NW * kBlock) * 4;
-  if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)delta_blocks_kernel<KT, NW>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                              smem) != hipSuccess) {
+template <typename F> int launch_kernel(F* kernel, int64_t groups, int threads, int smem, const RunArgs& ra, hipStream_t st) {
+  if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
     zp_set_error("delta_runs: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((delta_blocks_kernel<KT, NW>), dim3((unsigned)((int64_t)ra.d.seg.n * ra.d.heads)), dim3(64 * NW), smem, st, ra);
+  hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3(threads), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
+}
+template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
+  constexpr int kSplit = 3 * kBlock * 16 * KT;
+  constexpr int smem = (3 * block_floats(16 * KT, 16 * NW) - kSplit + 2 * 3 * KT * 384 + 2 * NW * kBlock) * 4;
+  const int64_t units = (int64_t)ra.d.seg.n * ra.d.heads;
+  if constexpr (KT == NW)
+    if (ra.pieces.blocks) {
+      int rc = launch_kernel(delta_blocks_kernel<KT, NW, true>, units * (ra.pieces.most - 1) * 2, 64 * NW, smem, ra, st);
+      if (rc == ZP_OK) rc = launch_kernel(delta_states_kernel<KT>, units, 64 * KT, KT * KT / 2 * 3072, ra, st);
+      if (rc != ZP_OK) return rc;
+    }
+  return launch_kernel(delta_blocks_kernel<KT, NW, false>, units * ra.pieces.most, 64 * NW, smem, ra, st);
 }
 template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   switch (ra.d.dv / 32) {
@@ -480,9 +615,15 @@ int launch_runs(const RunArgs& ra, int longest, hipStream_t st) {
 
 }  // namespace
 
+static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads, int dk, int dv) {
+  return (rows / kBlock + segments) * heads * block_floats(dk, dv) * 4;
+}
+
+// With room for the states between pieces of few heads' runs, whatever the longest run.
 extern "C" int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk, int32_t dv) {
   if (rows < 0 || segments < 0 || heads <= 0 || dk <= 0 || dv <= 0) return -1;
-  return ((int64_t)rows / kBlock + segments) * heads * block_floats(dk, dv) * 4;
+  const bool pieces = dk == dv && dk <= 128 && few_heads(segments, heads);
+  return blocks_bytes(rows, segments, heads, dk, dv) + (pieces ? (int64_t)kPieceStates * piece_floats(dk) * 4 : 0);
 }
 
 extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
@@ -503,9 +644,12 @@ extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t lo
                  a.seg.rows && a.seg.counts && a.seg.slots && a.seg.starts && aligned16(a.state) && aligned16(a.in) && aligned16(a.low) &&
                  aligned16(a.dt_bias) && aligned16(workspace),
              "delta_runs: null or unaligned pointer");
-  ZP_REQUIRE(workspace && workspace_bytes >= zp_delta_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk, a.dv),
-             "delta_runs: workspace too small");
-  RunArgs ra = {a, (float*)workspace, first_row};
+  const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk, a.dv);
+  ZP_REQUIRE(workspace && workspace_bytes >= whole, "delta_runs: workspace too small");
+  RunArgs ra = {a, (float*)workspace, first_row, {}};
+  if (a.dk == a.dv && workspace_bytes >= zp_delta_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk, a.dv))
+    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 2, 8, 40, 10);     // else runs stay whole
+  ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   return launch_runs(ra, longest, (hipStream_t)stream);
 }
