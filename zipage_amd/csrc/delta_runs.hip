@@ -648,7 +648,7 @@ extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t lo
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "delta_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, first_row, {}};
   if (a.dk == a.dv && workspace_bytes >= zp_delta_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk, a.dv))
-    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 2, 8, 75, 10);     // else runs stay whole
+    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 2, 8, 60, 10);     // else runs stay whole
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   return launch_runs(ra, longest, (hipStream_t)stream);

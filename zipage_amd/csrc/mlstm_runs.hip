@@ -80,11 +80,13 @@ __global__ __launch_bounds__(kGateTokens) void mlstm_gates_kernel(RunArgs ra) {
     if (tid < 64) {
       const float Fe = ends[0][lane], te = ends[1][lane];
       float mine = m;
+#pragma unroll 1
+      for (int b0 = 0; b0 * kBlock < cnt; b0 += 8)             // blocks behind the end change nothing
 #pragma unroll
-      for (int b = 0; b < 64; ++b) {                           // blocks behind the end change nothing
-        if (lane == b) mine = m;
-        m = lane_value(Fe, b) + fmaxf(m, lane_value(te, b));
-      }
+        for (int b = b0; b < b0 + 8; ++b) {
+          if (lane == b) mine = m;
+          m = lane_value(Fe, b) + fmaxf(m, lane_value(te, b));
+        }
       before[lane] = mine;
       if (lane == 0) before[64] = m;
     }
