@@ -66,6 +66,10 @@ int zp_softcap(const void* in, float* out, int64_t count, float cap, int32_t dty
 int zp_gather_rows(const void* src, const int32_t* rows, void* out, int32_t n, int32_t row_bytes,
                    int64_t num_rows, void* stream);
 
+/* out (n, M) = x (n, K) w^T, w (M, K) contiguous, sums in fp32: 16-bit, up to 64 rows, K a multiple of 32, M of 4. */
+int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                       int64_t out_stride, int32_t dtype, void* stream);
+
 /* What an attention does beyond the softmax of scaled products; NULL stands for {0, 1}.
  * softcap > 0: scores s (after the scale) enter the softmax as softcap * tanh(s / softcap).
  * maps 2 (differential attention): a query head holds two queries of D and a key head two keys of D, back to

@@ -254,6 +254,42 @@ def test_causal_attention(dev, H, G, D, lens=((1, 1), (31, 31), (128, 128), (129
     assert bool(((got.view(N, H, D).cpu().double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -14 * vv.abs().max()).all())
 
 
+# ------------------------------------------------------------------ products of few rows
+# token tiles of 1, 2 and 4, row tiles of 1, 2 and 4; contractions of one step, of stages that end early and of more than
+# the ring; outputs that end inside a tile; rows of x further apart than they are long
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+@pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("K,M", [(32, 4), (96, 20), (128, 4096), (1056, 4100), (1312, 68), (2048, 4128), (160, 16388), (2176, 16400)])
+def test_products_of_few_rows(dev, dtype, n, K, M):
+    from zipage_amd import _lib
+    wide = _rand(n, K + 24, seed=1, dtype=dtype).to(dev)
+    x, w = wide[:, 8:8 + K], (_rand(M, K, seed=2).float() * K ** -0.5).to(dtype).to(dev)
+    out = torch.full((n, M + 4), 7.0, dtype=dtype, device=dev)
+    _lib.call_models("zp_few_rows_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, K, M, x.stride(0), out.stride(0),
+                     _lib.dtype_tag(x), _lib.stream_ptr(x))
+    assert bool((out[:, M:] == 7).all())
+    want = x.double() @ w.double().T
+    # rounding to 8 or 11 bits, and K terms in fp32, each sum within 2^-24 sqrt(K) of its terms' root of squares
+    bits = 2.0 ** (-8 if dtype == BF16 else -11)
+    assert bool(((out[:, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
+
+
+def test_which_products_are_of_few_rows(dev):
+    from zipage_amd.layers import linear
+    w = (_rand(96, 64, seed=1).float() / 8).to(BF16).to(dev)
+    for x in (_rand(5, 64, seed=2).to(dev), _rand(64, 64, seed=3).to(dev), _rand(65, 64, seed=4).to(dev), _rand(5, 128, seed=5).to(dev)[:, ::2],
+              _rand(5, 65, seed=6).to(dev)[:, 1:], _rand(2, 3, 64, seed=7).to(dev), _rand(0, 64, seed=8).to(dev), _rand(64, 5, seed=9).to(dev).T):
+        want = torch.nn.functional.linear(x, w)
+        got = linear(x, w)
+        assert got.shape == want.shape and got.dtype == want.dtype
+        assert bool(((got.double() - want.double()).abs() <= 2.0 ** -7 * want.double().abs() + 2.0 ** -18).all())
+    grad = w.clone().requires_grad_()
+    linear(_rand(5, 64, seed=2).to(dev), grad).sum().backward()
+    assert grad.grad is not None
+    half = w.float()
+    assert linear(_rand(5, 64, seed=2).float().to(dev), half).dtype == torch.float32
+
+
 # ------------------------------------------------------------------ recurrences over runs, in pieces
 # Few heads walk long runs in pieces of at least four blocks of 16 tokens: one run, runs of which some have fewer pieces than
 # others or none, pieces whose last has one token or a whole block, states of earlier tokens and none; key and value sizes

@@ -34,7 +34,7 @@ FLAGS = BASE_FLAGS + ["-ffp-contract=off"]
 
 # sources of the model-side libraries, beside the error reporting; the rest is the compression library
 MODEL_SOURCES = {
-    MODELS_LIB: ("residual.hip", "runs.hip"),
+    MODELS_LIB: ("residual.hip", "runs.hip", "few_rows.hip"),
     LATENT_LIB: ("latent.hip",),
     GROUPED_LIB: ("grouped.hip",),
     RECURRENT_LIB: ("mlstm.hip", "mlstm_runs.hip", "delta.hip", "delta_runs.hip"),

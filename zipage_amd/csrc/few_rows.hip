@@ -1,0 +1,157 @@
+// y = x W^T for few rows of x, 16-bit: what a decode step asks of its weights.
+#include "mfma.h"
+#include <climits>
+
+namespace {
+
+typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
+template <typename T> __device__ __forceinline__ f32x4 product(const u32x4& w, const u32x4& x, const f32x4& c);
+template <> __device__ __forceinline__ f32x4 product<BF16>(const u32x4& w, const u32x4& x, const f32x4& c) { return mfma_bf16(w, x, c); }
+template <> __device__ __forceinline__ f32x4 product<F16>(const u32x4& w, const u32x4& x, const f32x4& c) {
+  return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(f16x8, w), __builtin_bit_cast(f16x8, x), c, 0, 0, 0);
+}
+
+struct FewArgs {
+  const uint16_t* x;   // rows of x_st elements
+  const uint16_t* w;   // (M, K)
+  uint16_t* out;       // rows of o_st elements
+  int n, K, M;
+  int64_t x_st, o_st;
+};
+
+// 16 * TT rows of x and 16 * MT of W per workgroup, four waves that share the contraction.  Both pass through LDS in stages of
+// 128 elements of every row, a step of 32 for each wave: loads of whole cache lines, for the L1 takes four to five cycles for
+// every line touched, whole or in part.  A row's sixteen pieces lie in the order of (piece ^ row).  Bound by the weights'
+// stream: what counts is bytes in flight, so the ring takes what LDS there is, for two workgroups where the tiles are small.
+// 1 to 31 rows, weights from memory, us (the library, which costs 18 us of host time a call, 5 here): 1024 -> 4096 4.2 to 4.9
+// (7.5 to 11.2), 2048 -> 1024 5.2 to 6.1 (8.1), 3072 -> 1024 6.5 to 7.8 (9.5), 4096 -> 4096 9.5 to 10.8 (15.8 to 13.4), 4096 ->
+// 6144 12.8 to 14.4 (16.1 to 15.7), 4096 -> 24 576 45.7 to 48.3 (47.8 to 48.8), 12 288 -> 4096 21.4 to 26.9 (23.1 to 26.8);
+// errors the same.  48 rows: 1024 -> 4096 6.5 (11.1), 3072 -> 1024 11.0 (10.7), but 4096 -> 6144 27.2 (17.7).
+template <int TT, int MT> struct FewTile {
+  static constexpr int kLoads = TT + MT, kBytes = kLoads * 4096;       // of a wave; of a stage
+  static constexpr int kRing = kLoads <= 2 ? 9 : kLoads == 3 ? 6 : kLoads == 4 ? 9 : kLoads == 5 ? 7 : 6;
+};
+template <typename T, int TT, int MT>
+__global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
+  extern __shared__ __align__(16) char lds_raw[];
+  typedef FewTile<TT, MT> Tile;
+  constexpr int L = Tile::kLoads, R = Tile::kRing;
+  static_assert((R - 2) * L < 64, "loads that a wait can count");
+  const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = blockIdx.x * 16 * MT, steps = a.K / 32, stages = (steps + 3) / 4;
+  const int x_row = (int)a.x_st * 2;                     // bytes
+  const u32x4 xr = rows_from(a.x, (uint32_t)(a.n - 1) * x_row + a.K * 2);
+  const u32x4 wr = rows_from(a.w + (int64_t)m0 * a.K, (uint32_t)min(16 * MT, a.M - m0) * a.K * 2);
+  int from[L];                                           // of four rows a load; what is not there lies past the end
+#pragma unroll
+  for (int i = 0; i < L; ++i) {
+    const int at = wave * L + i, row = at * 4 + g, r = at < 4 * MT ? row : row - 16 * MT;
+    const bool there = at < 4 * MT ? m0 + r < a.M : r < a.n;
+    from[i] = (there ? r * (at < 4 * MT ? a.K * 2 : x_row) : INT_MIN) + (l16 ^ (row & 15)) * 16;
+  }
+  auto issue = [&](int s) {                              // past the last stage zeros come, so that the count stays
+    char* const to = lds_raw + (s % R * Tile::kBytes + wave * L * 1024);
+    const bool whole = s * 4 + 4 <= steps;
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      int at = from[i] + s * 256;
+      if (!whole) at = s * 256 + (l16 ^ ((wave * L + i) * 4 + g & 15)) * 16 < a.K * 2 ? at : INT_MIN;
+      load_to_lds(wave * L + i < 4 * MT ? wr : xr, to + i * 1024, at, 0);
+    }
+  };
+#pragma unroll 1
+  for (int s = 0; s < R - 1; ++s) issue(s);
+  f32x4 acc[TT][MT] = {};
+  const int read_at = l16 * 256 + ((wave * 4 + g) ^ l16) * 16;
+#pragma unroll 1
+  for (int s = 0; s < stages; ++s) {
+    // this stage is there, and the one before has been read
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"((R - 2) * L) : "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    issue(s + R - 1);
+    if (s * 4 + wave >= steps) continue;
+    const char* const at = lds_raw + s % R * Tile::kBytes + read_at;
+    u32x4 wf[MT], xf[TT];
+#pragma unroll
+    for (int j = 0; j < MT; ++j) wf[j] = *(const u32x4*)(at + j * 4096);
+#pragma unroll
+    for (int t = 0; t < TT; ++t) xf[t] = *(const u32x4*)(at + (MT + t) * 4096);
+#pragma unroll
+    for (int t = 0; t < TT; ++t)
+#pragma unroll
+      for (int j = 0; j < MT; ++j) acc[t][j] = product<T>(wf[j], xf[t], acc[t][j]);
+  }
+  asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");    // no load is left on its way to LDS
+  __syncthreads();
+  // tile i of the TT * MT goes to wave i % 4, which adds up the others' shares in the order of the waves
+  f32x4* const red = (f32x4*)lds_raw;
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int j = 0; j < MT; ++j) red[((t * MT + j) * 4 + wave) * 64 + lane] = acc[t][j];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < (TT * MT + 3) / 4; ++i) {
+    const int id = i * 4 + wave, t = id / MT, j = id - t * MT;
+    if (id >= TT * MT) break;
+    f32x4 y = red[id * 256 + lane];
+#pragma unroll
+    for (int k = 1; k < 4; ++k) y += red[id * 256 + k * 64 + lane];
+    const int n = t * 16 + l16, m = m0 + j * 16 + g * 4;
+    if (n >= a.n || m >= a.M) continue;
+    uint2 o;
+    if constexpr (std::is_same<T, BF16>::value) {
+      o = uint2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+    } else {
+      typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
+      o = uint2{__builtin_bit_cast(uint32_t, f16x2{(_Float16)y[0], (_Float16)y[1]}),
+                __builtin_bit_cast(uint32_t, f16x2{(_Float16)y[2], (_Float16)y[3]})};
+    }
+    *(uint2*)(a.out + n * a.o_st + m) = o;
+  }
+}
+
+template <typename T, int TT, int MT> int launch_few(const FewArgs& a, hipStream_t st) {
+  constexpr int ring = FewTile<TT, MT>::kRing * FewTile<TT, MT>::kBytes, sums = TT * MT * 4096, smem = ring > sums ? ring : sums;
+  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)few_rows_kernel<T, TT, MT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                              smem) != hipSuccess) {
+    zp_set_error("few_rows_linear: cannot reserve %d bytes of LDS", smem);
+    return ZP_EHIP;
+  }
+  hipLaunchKernelGGL((few_rows_kernel<T, TT, MT>), dim3((unsigned)((a.M + 16 * MT - 1) / (16 * MT))), dim3(256), smem, st, a);
+  ZP_LAUNCH_CHECK();
+  return ZP_OK;
+}
+// Rows of W per workgroup: 16 where that makes at most a workgroup per CU, else 32, since each workgroup reads all of x (16
+// rows of x, us with 16, 32 and 64 rows of W: 1024 -> 4096 4.4, 4.8, 6.8; 4096 -> 4096 9.7, 11.0, 16.0; 1024 -> 6144 6.2, 5.2,
+// 7.1; 4096 -> 24 576 46.3, 45.2, 52.9).  64 where many short ones would spend their time on beginning (31 rows, 1024 -> 32 768:
+// 23.9, 21.7, 17.9).
+template <typename T, int TT> int launch_few(const FewArgs& a, hipStream_t st) {
+  if (a.M <= 4096) return launch_few<T, TT, 1>(a, st);
+  if constexpr (TT == 2)
+    if (a.M >= 16384 && a.K < 2048) return launch_few<T, 2, 4>(a, st);
+  return launch_few<T, TT, 2>(a, st);
+}
+template <typename T> int launch_few(const FewArgs& a, hipStream_t st) {
+  if (a.n <= 16) return launch_few<T, 1>(a, st);
+  return a.n <= 32 ? launch_few<T, 2>(a, st) : launch_few<T, 4>(a, st);
+}
+
+}  // namespace
+
+extern "C" int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                                  int64_t out_stride, int32_t dtype, void* stream) {
+  ZP_REQUIRE(n >= 0 && K > 0 && M > 0 && x_stride >= K && out_stride >= M, "few_rows_linear: bad dims");
+  if ((dtype != ZP_BF16 && dtype != ZP_F16) || n > 64 || K % 32 || M % 4 || x_stride % 8 || out_stride % 4 ||
+      x_stride > (1 << 23) || K > (1 << 23)) {
+    zp_set_error("few_rows_linear: 16-bit, %d rows (at most 64) of %d elements (a multiple of 32), %d outputs (a multiple of 4) unsupported",
+                 n, K, M);
+    return ZP_EUNSUPPORTED;
+  }
+  if (n == 0) return ZP_OK;
+  ZP_REQUIRE(x && w && out && aligned16(x) && aligned16(w) && ((uintptr_t)out & 7) == 0, "few_rows_linear: null or unaligned pointer");
+  const FewArgs a = {(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, n, K, M, x_stride, out_stride};
+  return dtype == ZP_BF16 ? launch_few<BF16>(a, (hipStream_t)stream) : launch_few<F16>(a, (hipStream_t)stream);
+}

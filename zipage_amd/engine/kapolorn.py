@@ -11,10 +11,9 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
-import torch.nn.functional as F
 
 from zipage_amd.layers.grouped import GroupedAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
 from zipage_amd.layers.moe import Experts
 from zipage_amd.layers.recurrent import ChannelDelta, MatrixMemory
 from zipage_amd.layers.residual import embed_norm, residual_norm, softcap
@@ -297,7 +296,7 @@ class Kapolorn:
         for run, i in enumerate(order):
             p, mixer, mlp = self.layers[i], self.mixers[i], self.mlps[i]
             mixed = torch.empty((N, mixer.out_columns), dtype=self.dtype, device=self.device)
-            mixer.mix(h, F.linear(h, p["into"]), positions, self.caches[run], ctx, mixed)
+            mixer.mix(h, linear(h, p["into"]), positions, self.caches[run], ctx, mixed)
             y, w = p["out"].forward(mixed), p["norm1b"]
             if mlp is not None:
                 h = residual_norm(x, y, p["norm2"], s.eps, s.width, x_out=x, y_weight=w)
@@ -310,4 +309,4 @@ class Kapolorn:
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
         """fp32 logits under the soft cap."""
-        return softcap(F.linear(hidden, self.embed), self.shape.logit_softcap)
+        return softcap(linear(hidden, self.embed), self.shape.logit_softcap)

@@ -13,10 +13,9 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
-import torch.nn.functional as F
 
 from zipage_amd.layers.grouped import GroupedAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
 from zipage_amd.layers.recurrent import LinearAttention
 from zipage_amd.layers.residual import embed_norm, normed_powers, residual_norm
 from zipage_amd.layers.rotary import Rotary
@@ -258,7 +257,7 @@ class Layer:
 
     def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, ctx) -> list:
         """The branches that join the stream, with the weights of their norms."""
-        proj = F.linear(h, self.into)
+        proj = linear(h, self.into)
         rows = [torch.empty((h.shape[0], o.w.shape[1]), dtype=h.dtype, device=h.device) for o in self.outs]
         self.mixer.mix(proj[:, :self.mixed], positions, cache, ctx, [r[:, :n] for r, n in zip(rows, self.spans)])
         if self.ff is not None:
@@ -372,4 +371,4 @@ class Mefupel:
 
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.head)
+        return linear(hidden, self.head)

@@ -13,10 +13,9 @@ import math
 from dataclasses import dataclass
 
 import torch
-import torch.nn.functional as F
 
 from zipage_amd.layers.latent import LatentAttention
-from zipage_amd.layers.linear import ResidualLinear, fit
+from zipage_amd.layers.linear import ResidualLinear, fit, linear
 from zipage_amd.layers.residual import embed_norm, residual_norm, xielu
 
 
@@ -184,7 +183,7 @@ class Pedivik:
             y = mixer.forward(h, self.caches[i], ctx)
             if "up" in p:
                 h = residual_norm(x, y, p["norm2"], s.eps, s.width, weight_offset=1.0, x_out=inner)
-                x, y = inner, p["down"].forward(xielu(F.linear(h, p["up"]), *p["act"]))
+                x, y = inner, p["down"].forward(xielu(linear(h, p["up"]), *p["act"]))
             h = residual_norm(x, y, norms[i + 1], s.eps, s.width, weight_offset=1.0, out_scale=scales[i + 1],
                               x_out=after, result=history[i + 1], history=history, mix=p["dwa"])
             x = after
@@ -194,4 +193,4 @@ class Pedivik:
 
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.embed)
+        return linear(hidden, self.embed)

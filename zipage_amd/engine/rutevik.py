@@ -11,11 +11,10 @@ from __future__ import annotations
 from dataclasses import dataclass
 
 import torch
-import torch.nn.functional as F
 
 from zipage_amd.layers.grouped import GroupedAttention
 from zipage_amd.layers.latent import LatentAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
 from zipage_amd.layers.moe import Experts
 from zipage_amd.layers.residual import embed_norm, relu_square, residual_norm
 from zipage_amd.layers.rotary import Rotary
@@ -155,7 +154,7 @@ class Differential:
 
     def forward(self, h, cache, ctx, positions, held):
         mixed = torch.empty((h.shape[0], self.core.out_columns), dtype=h.dtype, device=h.device)
-        self.core.attend(F.linear(h, self.into), positions, cache, ctx, mixed)
+        self.core.attend(linear(h, self.into), positions, cache, ctx, mixed)
         return self.out.forward(mixed)
 
 
@@ -178,7 +177,7 @@ class Dense:
                    for k, s in self.shapes().items()}, dtype, device)
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return self.down.forward(relu_square(F.linear(h, self.up)))
+        return self.down.forward(relu_square(linear(h, self.up)))
 
 
 class Rutevik:
@@ -305,4 +304,4 @@ class Rutevik:
 
     @torch.inference_mode()
     def compute_logits(self, hidden: torch.Tensor) -> torch.Tensor:
-        return F.linear(hidden, self.head)
+        return linear(hidden, self.head)

@@ -4,6 +4,8 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
+from zipage_amd import _lib
+
 
 def pad_to_multiple(n: int, to: int) -> int:
     return -(-n // to) * to
@@ -14,6 +16,27 @@ def fit(t: torch.Tensor, *shape: int) -> torch.Tensor:
     out = torch.zeros(shape, dtype=t.dtype, device=t.device)
     out[tuple(slice(0, n) for n in t.shape)] = t
     return out
+
+
+def _few_rows(n: int, k: int, m: int) -> bool:
+    """Whether a product of n rows of k elements and (m, k) weights goes to the kernel for few rows.  Up to 32 rows it is as
+    fast as the library on the GPU or faster (csrc/few_rows.hip has both), and costs a quarter of the host's time; up to 64
+    where the weights are few, since each workgroup reads all of x."""
+    return (n <= 32 or n <= 64 and m * k <= 1 << 23) and n > 0 and k % 32 == 0 and m % 4 == 0 and 0 < k <= 1 << 23
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w) without a bias."""
+    if x.is_cuda and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == w.dtype and w.dim() == 2 and \
+            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+        (n, k), m, stride = x.shape, w.shape[0], x.stride(0)
+        if _few_rows(n, k, m) and w.shape[1] == k and x.stride(1) == 1 and k <= stride <= 1 << 23 and stride % 8 == 0 and \
+                w.is_contiguous() and w.device == x.device and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
+            out = x.new_empty(n, m)
+            _lib.call_models("zp_few_rows_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, k, m, stride, m,
+                             _lib.dtype_tag(x), _lib.stream_ptr(x))
+            return out
+    return F.linear(x, w)
 
 
 class ResidualLinear:
@@ -39,6 +62,6 @@ class ResidualLinear:
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         N = x.shape[0]
         if self.parts is None or N > self.SPLIT_ROWS:
-            return F.linear(x, self.w).unsqueeze(0)
+            return linear(x, self.w).unsqueeze(0)
         P, k, _ = self.parts.shape
         return torch.bmm(x.view(N, P, k).transpose(0, 1), self.parts)
