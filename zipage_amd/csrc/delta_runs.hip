@@ -53,41 +53,44 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
     return c < dk ? hk * dk + c : (c < 2 * dk ? a.kv_heads * dk + hk * dk + c - dk : 2 * a.kv_heads * dk + h * dv + c - 2 * dk);
   };
   // ---- requests first: the decays' pre-activations (two pieces a thread at most), the step sizes'
+  const int piece_bits = 31 - __builtin_clz(dk / 4);           // pieces of four channels: 8, 16 or 32 a row
   f32x4 z[2], zb[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int i = tid + u * 256, t = i / (dk / 4), c = (i - t * (dk / 4)) * 4;
-    z[u] = zb[u] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (t < cnt) {
-      z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t0 + t) * a.low_stride + h * dk + c);
-      zb[u] = *(const f32x4*)(a.dt_bias + h * dk + c);
-    }
+    const int i = tid + u * 256, t = min(i >> piece_bits, cnt - 1), c = (i & ((1 << piece_bits) - 1)) * 4;
+    z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t0 + t) * a.low_stride + h * dk + c);
+    zb[u] = *(const f32x4*)(a.dt_bias + h * dk + c);
   }
   const float b_in = tid < cnt ? Elem<BF16>::ld(a.in, (int64_t)(sg.row + t0 + tid) * a.in_stride + a.b_at + h) : 0.f;
   const float rate = __expf(a.a_log[h]);
-  // ---- convolutions: a thread's two channels, the block's 16 tokens from a sliding window
-  // rows from t0 - (TAPS - 1) on; those outside the run read as zero, those before it come from the history
-  const int back = min(TAPS - 1, t0);
+  // ---- convolutions: a thread's two channels, the block's 16 tokens from a sliding window.  Rows behind the run's end read
+  // as zero, and those before its beginning too, unless they come from the history.
+  const int row_bytes = (int)a.in_stride * 2;
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)((const char*)a.in + (int64_t)(sg.row + t0 - back) * a.in_stride * 2), 0, (int)((cnt + back) * a.in_stride * 2), 0x00020000);
-  for (int c = 2 * tid; c < cw; c += 512) {
+      (void*)((const char*)a.in + (int64_t)(sg.row + t0) * row_bytes), 0, cnt * row_bytes, 0x00020000);
+  const __amdgpu_buffer_rsrc_t before = __builtin_amdgcn_make_buffer_rsrc(
+      (void*)((const char*)a.in + (int64_t)(sg.row + t0 - (TAPS - 1)) * row_bytes), 0, t0 > 0 ? (TAPS - 1) * row_bytes : 0, 0x00020000);
+  if (const int c = 2 * tid; c < cw) {         // at most 384 channels
     const int at = place(c);
     uint32_t x[kBlock + TAPS - 1];             // two channels' bf16
 #pragma unroll
-    for (int i = 0; i < kBlock + TAPS - 1; ++i) {
-      const int u = i - (TAPS - 1) + back;     // row of the buffer
-      x[i] = u >= 0 ? (uint32_t)__builtin_amdgcn_raw_buffer_load_b32(rows, at * 2, u * (int)a.in_stride * 2, 0) : 0u;
-    }
+    for (int i = 0; i < kBlock + TAPS - 1; ++i)
+      x[i] = (uint32_t)(i < TAPS - 1 ? __builtin_amdgcn_raw_buffer_load_b32(before, at * 2, i * row_bytes, 0)
+                                     : __builtin_amdgcn_raw_buffer_load_b32(rows, at * 2, (i - (TAPS - 1)) * row_bytes, 0));
+    float f[2][TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j)                            // f[.][j]: j tokens back
+#pragma unroll
+      for (int e = 0; e < 2; ++e) f[e][j] = a.filters[(int64_t)max(taps - 1 - j, 0) * channels + at + e];
+#pragma unroll
+    for (int j = 1; j < TAPS; ++j)
+#pragma unroll
+      for (int e = 0; e < 2; ++e) f[e][j] = j < taps ? f[e][j] : 0.f;
     if (t0 == 0 && sg.start > 0) {
 #pragma unroll
       for (int i = 0; i < TAPS - 1; ++i)
         if (i >= TAPS - taps) x[i] = *(const uint32_t*)(tail + ((int64_t)(taps - TAPS + i) * cw + c) * 2);
     }
-    float f[2][TAPS];
-#pragma unroll
-    for (int j = 0; j < TAPS; ++j)                            // f[.][j]: j tokens back
-#pragma unroll
-      for (int e = 0; e < 2; ++e) f[e][j] = j < taps ? a.filters[(int64_t)(taps - 1 - j) * channels + at + e] : 0.f;
     float* const dst = c < dk ? qs + c : (c < 2 * dk ? ks + c - dk : vs + c - 2 * dk);
 #pragma unroll
     for (int t = 0; t < kBlock; ++t) {
@@ -98,21 +101,20 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
         y.x = fmaf(f[0][j], __uint_as_float(v << 16), y.x);
         y.y = fmaf(f[1][j], __uint_as_float(v & 0xffff0000u), y.y);
       }
-      y.x = t < cnt ? y.x * fast_sigmoid(y.x) : 0.f;
-      y.y = t < cnt ? y.y * fast_sigmoid(y.y) : 0.f;
+      y.x *= fast_sigmoid(y.x);
+      y.y *= fast_sigmoid(y.y);
       *(float2*)(dst + t * ld) = y;
       if (t % 4 == 3) __builtin_amdgcn_sched_barrier(0);
     }
+    for (int t = cnt; t < kBlock; ++t) *(float2*)(dst + t * ld) = float2{0.f, 0.f};
   }
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int i = tid + u * 256, t = i / (dk / 4), c = (i - t * (dk / 4)) * 4;
+    const int i = tid + u * 256, t = i >> piece_bits, c = (i & ((1 << piece_bits) - 1)) * 4;
     if (t < kBlock) {
-      f32x4 g = {1.f, 1.f, 1.f, 1.f};
-      if (t < cnt) {
+      f32x4 g;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) g[e] = __expf(-rate * fast_softplus(z[u][e] + zb[u][e]));
-      }
+      for (int e = 0; e < 4; ++e) g[e] = t < cnt ? __expf(-rate * fast_softplus(z[u][e] + zb[u][e])) : 1.f;
       *(f32x4*)(gs + t * ld + c) = g;
     }
   }
