@@ -59,13 +59,17 @@ __device__ __forceinline__ float rows_sum(float v) {
 __device__ __forceinline__ float sigmoid_f(float x) { return 1.f / (1.f + expf(-x)); }
 __device__ __forceinline__ float softplus_f(float x) { return fmaxf(x, 0.f) + log1pf(expf(-fabsf(x))); }
 
-// Sum over the eight column quads of a wave (lanes of one row group), in every one of them.
-__device__ __forceinline__ float quads_sum(float v) {
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x141, 0xf, 0xf, false));  // half mirror
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0xB1, 0xf, 0xf, false));   // [1,0,3,2]
-  v += __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x4E, 0xf, 0xf, false));   // [2,3,0,1]
-  return v;
+template <int CTRL> __device__ __forceinline__ float dpp_moved(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xf, 0xf, false));
 }
+__device__ __forceinline__ float half_row_mirror(float v) { return dpp_moved<0x141>(v); }        // lane i of eight <- lane 7 - i
+// Sum over four lanes, in every one of them.
+__device__ __forceinline__ float quad_sum(float v) {
+  v += dpp_moved<0xB1>(v);   // [1,0,3,2]
+  return v + dpp_moved<0x4E>(v);   // [2,3,0,1]
+}
+// Sum over the eight column quads of a wave (lanes of one row group), in every one of them.
+__device__ __forceinline__ float quads_sum(float v) { return quad_sum(v + half_row_mirror(v)); }
 
 // Four consecutive elements as fp32.
 template <typename T> __device__ __forceinline__ f32x4 load4(const void* p, int64_t i);
