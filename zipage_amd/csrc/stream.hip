@@ -30,16 +30,30 @@ __global__ __launch_bounds__(kThreads) void global_score_kernel(
   const int64_t sbase = (((int64_t)l * B + b) * Hkv) * (int64_t)NB * BS + (int64_t)j * BS;
   const int64_t cbase = l * c_sl + pid * c_sp;
   const int n = BS * Hkv;
-  for (int c = threadIdx.x; c < n; c += kThreads) {
-    const int slot = c / Hkv, h = c - slot * Hkv;
-    const int64_t si = sbase + (int64_t)h * NB * BS + slot;
-    float v = Elem<T>::ld(scores, si);
-    if (carry) {
-      const float old = Elem<T>::ld(cache, cbase + c) * decay;
-      v = Elem<T>::rnd(method == ZP_ACTIVATE_MAX ? fmaxf(v, old) : v + old);
-      Elem<T>::st(scores, si, v);
+  // eight elements' loads side by side: one after the other, each waits for memory (2 layers of 2 sequences 7.3 us, now 6.4;
+  // 64 sequences 11.0, now 8.4)
+  constexpr int kAhead = 8;
+  for (int c0 = threadIdx.x; c0 < n; c0 += kAhead * kThreads) {
+    float v[kAhead], old[kAhead];
+    int64_t si[kAhead];
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int c = min(c0 + u * kThreads, n - 1), slot = c / Hkv, h = c - slot * Hkv;
+      si[u] = sbase + (int64_t)h * NB * BS + slot;
+      v[u] = Elem<T>::ld(scores, si[u]);
+      old[u] = carry ? Elem<T>::ld(cache, cbase + c) : 0.f;
     }
-    if (write_cache) Elem<T>::st(cache, cbase + c, v);
+#pragma unroll
+    for (int u = 0; u < kAhead; ++u) {
+      const int c = c0 + u * kThreads;
+      if (c >= n) break;
+      if (carry) {
+        const float o = old[u] * decay;
+        v[u] = Elem<T>::rnd(method == ZP_ACTIVATE_MAX ? fmaxf(v[u], o) : v[u] + o);
+        Elem<T>::st(scores, si[u], v[u]);
+      }
+      if (write_cache) Elem<T>::st(cache, cbase + c, v[u]);
+    }
   }
 }
 
