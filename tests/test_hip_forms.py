@@ -468,7 +468,8 @@ def test_states_of_runs(dev, mixer, H, D, V):
 # fetched 64 at a time, a token's keys cut into ranges of at least four stages
 @pytest.mark.parametrize("H,R,P,BS,window", [(1, 288, 8, 16, None), (17, 512, 64, 16, 1100), (33, 128, 24, 16, None),
                                              (48, 256, 0, 32, 65), (65, 384, 40, 16, 1), (32, 256, 8, 16, None),
-                                             (16, 512, 0, 64, None), (128, 32, 64, 16, 700)])
+                                             (16, 512, 0, 64, None), (128, 32, 64, 16, 700), (24, 352, 24, 16, 300),
+                                             (9, 416, 16, 32, None)])
 def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
     from zipage_amd.layers import latent_rows_attention
     ctx = [0, 1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129, 130, 160, 193, 1023, 1024, 1025, 2080, 2500]

@@ -639,20 +639,24 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
 
 // NCB column blocks of 128 cover R; PK steps of 32 the rotated part, which is a key only, never a value.  Workgroup: one
 // token, HW tiles of 16 heads, one key range.  All four waves take the same 32 keys; waves on the same head tile
-// (4 / HW) share its value columns out and compute its scores each for itself, so that they meet only to hand over LDS.
+// (4 / HW) share its value columns out, and its scores: two take 16 keys each, four also every other step of the contraction,
+// and hand them over through LDS (each for itself read all keys: 16 heads, 256 sequences of 1800 to 2304 tokens 123 us,
+// now 115; 32 heads 134, now 121; the same sums).
 //
 // Bound by HBM, so what counts is how much is on its way: rows go from memory into LDS without passing through
 // registers, in a ring of stages of 32 keys of which all but one are in flight (108 KB per CU for rows of 576; held in
 // registers between its two uses, a block left its place only when its products were done: 256 sequences of 2050 tokens,
 // 32 heads 157 us, now 141; a window of 1024 76, now 60; 64 sequences, 128 heads 124, now 92).  The value operand is
-// transposed by the LDS reads.  An odd number of 16-byte pieces per staged row keeps both operands off each other's banks.
+// transposed by the LDS reads.  Staged rows are twice an odd number of 16-byte pieces apart: of a read of 16 bytes lanes 0 to 3,
+// 12 to 15 and 20 to 27 go together, and then the two quarters of a wave have every other piece of the banks each (an odd
+// number had half of the LDS cycles in conflicts; 100 to 4096 tokens, 32 heads 174 us, 167 without them).
 //
 // Softmax weights meet the values in two bf16 planes.  With one, results were up to 0.5 % further from 64-bit ones than those
 // of waves with maxima of their own (the weight of a maximum is 1 and loses nothing, and here there are fewer); with two
 // they are 2 to 3 % nearer, for 5 % of the kernel's time (141 -> 147 us of the first).
 constexpr int rows_ring(int NCB) { return NCB <= 2 ? 3 : 4; }       // two workgroups per CU where rows are short
 template <int NCB, int PK> struct RowsStage {
-  static constexpr int kMaxPieces = NCB * 16 + PK * 4 + 1;
+  static constexpr int kMaxPieces = NCB * 16 + PK * 4 + 2;
   static constexpr int kHalf = (kMaxPieces + 3) / 4 * 1024;           // bytes of 16 keys, whole loads
   static constexpr int kLoads = ((kMaxPieces + 3) / 4 + 1) / 2;       // of a wave for a stage
   static constexpr int kBytes = rows_ring(NCB) * 2 * kHalf;
@@ -662,7 +666,8 @@ template <int NCB, int HW, int PK>
 __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_kernel(RowsArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef RowsStage<NCB, PK> Stage;
-  constexpr int kRing = rows_ring(NCB), KS = 4 * NCB, VT = NCB * 8 / (4 / HW);     // value tiles of 16 columns of a wave
+  constexpr int kRing = rows_ring(NCB), KS = 4 * NCB, SH = 4 / HW, VT = NCB * 8 / SH;     // value tiles of 16 columns of a wave
+  constexpr int kKeys = KS + PK, kDots = 2 * kKeys / SH, kOdd = SH == 4 ? 2 : 1;   // products of a wave for the scores of a block
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
@@ -670,16 +675,18 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
   const int split = id % a.splits;
   id /= a.splits;
   const int row = id / hgroups, head = (id % hgroups * HW + wave % HW) * 16 + l16;
-  const int RW = a.R + a.P, pieces = RW / 8, staged = pieces | 1;
-  const int col0 = wave / HW * VT * 16;                          // of the wave's values
+  const int RW = a.R + a.P, pieces = RW / 8, staged = ((pieces + 1) | 3) - 1;
+  const int share = wave / HW, col0 = share * VT * 16;           // of the wave's values
+  const int mine = SH > 1 ? share & 1 : 0, odd = SH == 4 ? share >> 1 : 0;      // of the scores: its 16 keys, its steps
 
-  u32x4 q[KS + PK];
+  u32x4 q[kKeys / kOdd];
 #pragma unroll
-  for (int ks = 0; ks < KS + PK; ++ks) {
+  for (int i = 0; i < kKeys / kOdd; ++i) {
+    const int ks = kOdd * i + odd;
     const int c = ks < KS ? ks * 32 + g * 8 : (ks - KS) * 32 + g * 8;
     const bool there = head < a.H && c < (ks < KS ? a.R : a.P);
-    q[ks] = u32x4{0u, 0u, 0u, 0u};
-    if (there) q[ks] = *(const u32x4*)((const uint16_t*)a.q + ((int64_t)row * a.H + head) * RW + (ks < KS ? c : a.R + c));
+    q[i] = u32x4{0u, 0u, 0u, 0u};
+    if (there) q[i] = *(const u32x4*)((const uint16_t*)a.q + ((int64_t)row * a.H + head) * RW + (ks < KS ? c : a.R + c));
   }
   const int seq = a.seq ? min(max(a.seq[row], 0), a.B - 1) : row;
   const int n = min(a.ctx[row], a.NB * a.BS);
@@ -752,10 +759,14 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
   const float sc = a.scale * 1.44269504088896f;
   // R may end inside the last column block: columns past it are others again, against zeros in q or in results that are not
   // written
-  const int key_at = l16 * staged * 16 + g * 16, value_at = (4 * g + (l16 >> 2)) * staged * 16 + (l16 & 3) * 8;
-  int rot_at[PK ? PK : 1];
+  const int key_at = mine * Stage::kHalf + l16 * staged * 16 + g * 16, value_at = (4 * g + (l16 >> 2)) * staged * 16 + (l16 & 3) * 8;
+  int rot_at[PK ? PK / kOdd : 1];
 #pragma unroll
-  for (int ks = 0; ks < PK; ++ks) rot_at[ks] = l16 * staged * 16 + (a.R / 8 + (ks * 32 + g * 8 < a.P ? ks * 4 + g : 0)) * 16;
+  for (int i = 0; i < PK / kOdd; ++i) {
+    const int ks = kOdd * i + odd;
+    rot_at[i] = key_at + (a.R / 8 - g + (ks * 32 + g * 8 < a.P ? ks * 4 + g : 0)) * 16;
+  }
+  f32x4* const shared = (f32x4*)(lds_raw + Stage::kBytes) + wave % HW * SH * 64 + lane;     // scores of the wave's heads
 #pragma unroll 1
   for (int j = 0; j < blocks; ++j) {
     // this wave's share of block j has come when at most those of the blocks behind it are on their way
@@ -769,26 +780,27 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
     const int k0 = (b0 + j * a.splits) * 32;
     const char* const at = lds_raw + (j % kRing) * (2 * Stage::kHalf);
     // operands leave LDS kAhead products ahead; the barriers keep the compiler from moving a read to its use
-    constexpr int kAhead = 4, kRead = kAhead + 1, kKeys = KS + PK;
+    constexpr int kAhead = 4, kRead = kAhead + 1, kSteps = kKeys / kOdd;
     u32x4 kf[kRead];
-    auto read_key = [&](int i) {                                 // of half i / kKeys, step i % kKeys
-      if (i >= 2 * kKeys) return;
-      const int ks = i % kKeys;
-      const int c = ks < KS ? key_at + (ks < KS - 4 ? ks * 64 : min(ks * 64, a.R * 2 - 64)) : rot_at[ks < KS ? 0 : ks - KS];
-      kf[i % kRead] = *(const u32x4*)(at + i / kKeys * Stage::kHalf + c);
+    auto read_key = [&](int i) {                                 // of the wave's half i / kSteps, its step i % kSteps
+      if (i >= kDots) return;
+      const int own = i % kSteps, first = kOdd * own, ks = first + odd;
+      const int c = first < KS ? key_at + (first < KS - 4 ? ks * 64 : min(ks * 64, a.R * 2 - 64))
+                               : rot_at[first < KS ? 0 : own - KS / kOdd];
+      kf[i % kRead] = *(const u32x4*)(at + i / kSteps * Stage::kHalf + c);
     };
     f32x4 part[2][2] = {};                                       // of both halves, even and odd steps
 #pragma unroll
     for (int i = 0; i < kAhead; ++i) read_key(i);
     auto scores = [&](bool loads_too) {
 #pragma unroll
-      for (int i = 0; i < 2 * kKeys; ++i) {
+      for (int i = 0; i < kDots; ++i) {
         read_key(i + kAhead);
-        const int hf = i / kKeys, ks = i % kKeys;
-        part[hf][ks & 1] = mfma_bf16(kf[i % kRead], q[ks], part[hf][ks & 1]);
+        const int hf = i / kSteps, own = i % kSteps, chain = SH == 4 ? 0 : own & 1;
+        part[hf][chain] = mfma_bf16(kf[i % kRead], q[own], part[hf][chain]);
         if (loads_too)
 #pragma unroll
-          for (int k = i * Stage::kLoads / (2 * kKeys); k < (i + 1) * Stage::kLoads / (2 * kKeys); ++k) load(k, true);
+          for (int k = i * Stage::kLoads / kDots; k < (i + 1) * Stage::kLoads / kDots; ++k) load(k, true);
         __builtin_amdgcn_sched_barrier(0);
       }
     };
@@ -799,7 +811,8 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
       for (int k = 0; k < Stage::kLoads; ++k) load(k, false);
       scores(false);
     }
-    const f32x4 s[2] = {part[0][0] + part[0][1], part[1][0] + part[1][1]};
+    f32x4 s[2] = {part[0][0] + part[0][1], part[1][0] + part[1][1]};
+    if constexpr (SH > 1) shared[share * 64] = SH == 4 ? part[0][0] : s[0];
     u32x4 vf[kRead];
     auto read_value = [&](int i) {
       if (i >= VT) return;
@@ -811,6 +824,14 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
 #pragma unroll
     for (int i = 0; i < kRead; ++i) read_value(i);
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (SH > 1) {
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_s_waitcnt(0xc07f);                        // in LDS; loads from memory go on
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      s[0] = shared[0], s[1] = shared[64];
+      if constexpr (SH == 4) s[0] += shared[128], s[1] += shared[192];
+    }
     float p[8], mx = -INFINITY;
 #pragma unroll
     for (int i = 0; i < 8; ++i) p[i] = s[i >> 2][i & 3] * sc;
@@ -1034,7 +1055,8 @@ template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, h
   return launch_combine(a, st);
 }
 template <int NCB, int HW, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
-  constexpr int smem = RowsStage<NCB, PK>::kBytes;
+  constexpr int smem = RowsStage<NCB, PK>::kBytes + (HW < 4 ? 4096 : 0);
+  static_assert(smem <= 160 * 1024, "LDS of a CU");
   if (smem > 64 * 1024 &&
       hipFuncSetAttribute((const void*)latent_rows_kernel<NCB, HW, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           smem) != hipSuccess) {
