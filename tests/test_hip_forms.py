@@ -501,6 +501,24 @@ def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
         assert ((one - want[i:i + 1]).abs() <= allowed[i:i + 1]).all()
 
 
+# a pool and tables of 320 MB and more: rows are asked for past the last-level cache, by the same sums
+@pytest.mark.parametrize("H,R,P", [(16, 512, 64), (20, 384, 8), (33, 512, 64), (40, 128, 64), (65, 512, 0)])
+def test_latent_rows_past_the_cache(dev, H, R, P):
+    from zipage_amd.layers import latent_rows_attention
+    BS, used, ctx = 1024, 8, [0, 1, 33, 700, 1024, 2500]
+    pages = (320 << 20) // (BS * (R + P) * 2) + 1
+    cache = torch.zeros(pages, BS, R + P, dtype=torch.bfloat16, device=dev)
+    cache[:used] = _rand(used, BS, R + P, seed=H).to(dev)
+    tables = torch.full((len(ctx), pages), -1, dtype=torch.int32)
+    for i, c in enumerate(ctx):
+        tables[i, :-(-c // BS)] = (torch.arange(-(-c // BS)) * 3 + i).int() % used
+    q = _rand(len(ctx), H, R + P, seed=R, std=4.0 * (R + P) ** -0.5).to(dev)
+    t, n = tables.to(dev), torch.tensor(ctx, dtype=torch.int32, device=dev)
+    past = latent_rows_attention(q, cache, t, n, 1.0, None, rank=R)
+    assert torch.equal(past, latent_rows_attention(q, cache[:used].clone(), t, n, 1.0, None, rank=R))
+    assert past[1:].any(-1).all()
+
+
 # ------------------------------------------------------------------ per-head products
 # through LDS: tiles of 64 outputs by 16, 32 or 64 tokens, stages of 128 elements in a ring of four; straight from
 # memory: contractions below 256 (512 with fewer than 64 outputs) and below 8192 matrix products

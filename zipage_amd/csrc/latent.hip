@@ -20,6 +20,7 @@
 // eight keys x eight columns by v_perm; the column order that results (MFMA t, row m <-> column
 // 8m + t) leaves eight consecutive output columns in each lane.
 #include "mfma.h"
+#include <algorithm>
 #include <math.h>
 
 namespace {
@@ -662,7 +663,7 @@ template <int NCB, int PK> struct RowsStage {
   static constexpr int kBytes = rows_ring(NCB) * 2 * kHalf;
 };
 
-template <int NCB, int HW, int PK>
+template <int NCB, int HW, int PK, bool PAST>
 __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_kernel(RowsArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef RowsStage<NCB, PK> Stage;
@@ -735,10 +736,10 @@ __global__ __launch_bounds__(256, NCB <= 2 || HW <= 2 ? 2 : 1) void latent_rows_
   auto load = [&](int k, bool all) {
     char* const at = to + min((wave >> 1) + 2 * k, loads - 1) * 1024;
     if (all) {
-      load_to_lds(rows, at, piece_at[k] & 0xfffff, 0);
+      load_to_lds<PAST>(rows, at, piece_at[k] & 0xfffff, 0);
     } else {
       const int r = piece_at[k] >> 20, key = min(max(h0 + r, from), upto);
-      load_to_lds(rows, at, (piece_at[k] & 0xfffff) + ((key & mask) - r) * RW * 2, 0);
+      load_to_lds<PAST>(rows, at, (piece_at[k] & 0xfffff) + ((key & mask) - r) * RW * 2, 0);
     }
   };
 #pragma unroll
@@ -1054,19 +1055,30 @@ template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, h
   ZP_LAUNCH_CHECK();
   return launch_combine(a, st);
 }
-template <int NCB, int HW, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
+// Whether rows are asked for past the last-level cache: one workgroup reads a key, and all that may be read do not fit.  Rows
+// of 576, 256 sequences of 1800 to 2304 tokens, 16 heads 115 us through it and 103 past it, 32 heads 122 and 115, 64 heads
+// 181 and 176; with two workgroups on a token (128 heads) 324 and 338, and where rows fit, 40 sequences, 42 and 43.
+bool rows_past(const RowsArgs& a, int hgroups) {
+  const int64_t keys = a.window > 0 ? std::min<int64_t>(a.window, (int64_t)a.NB * a.BS) : (int64_t)a.NB * a.BS;
+  return hgroups == 1 && std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * (a.R + a.P) * 2 >= 320ll << 20;
+}
+template <int NCB, int HW, int PK, bool PAST> int launch_latent_rows(const RowsArgs& a, int hgroups, hipStream_t st) {
   constexpr int smem = RowsStage<NCB, PK>::kBytes + (HW < 4 ? 4096 : 0);
   static_assert(smem <= 160 * 1024, "LDS of a CU");
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)latent_rows_kernel<NCB, HW, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)latent_rows_kernel<NCB, HW, PK, PAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           smem) != hipSuccess) {
     zp_set_error("latent_rows_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
-  hipLaunchKernelGGL((latent_rows_kernel<NCB, HW, PK>), dim3((unsigned)a.n * hgroups * a.splits), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((latent_rows_kernel<NCB, HW, PK, PAST>), dim3((unsigned)a.n * hgroups * a.splits), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return launch_combine(a, st);
+}
+template <int NCB, int HW, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
+  const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
+  return rows_past(a, hgroups) ? launch_latent_rows<NCB, HW, PK, true>(a, hgroups, st)
+                               : launch_latent_rows<NCB, HW, PK, false>(a, hgroups, st);
 }
 template <int NCB, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
   if constexpr (NCB <= 2) {

@@ -38,11 +38,16 @@ __device__ __forceinline__ uint2 read_transposed(const uint16_t* p) {
 // which cannot tell the stage being filled from the stage being read, would wait for it at the next LDS read; what
 // waits is the code that meets the other waves.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
+template <bool PAST = false>      // past the last-level cache
 __device__ __forceinline__ void load_to_lds(const u32x4& rows, void* lds, int lane_at, int at) {
   const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
   const int so = __builtin_amdgcn_readfirstlane(at);
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
-               :: "s"(to), "v"(lane_at), "s"(rows), "s"(so) : "memory", "m0");
+  if constexpr (PAST)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds"
+                 :: "s"(to), "v"(lane_at), "s"(rows), "s"(so) : "memory", "m0");
+  else
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+                 :: "s"(to), "v"(lane_at), "s"(rows), "s"(so) : "memory", "m0");
 }
 // What such loads read: `bytes` from `base` on, zeros behind them.
 __device__ __forceinline__ u32x4 rows_from(const void* base, uint32_t bytes) {
