@@ -147,6 +147,35 @@ def test_turning_values_are_stored(dev, dtype, H, G, D, V, vdim, rot):
     _check_slots(cache, kv)
 
 
+# 320 MB and more in one call: rows that are not read next pass the last-level cache by; parts of it take the other form
+@pytest.mark.parametrize("form", ["plain", "bias", "turning", "norms", "tied"])
+def test_rows_past_the_cache_are_stored_alike(dev, form):
+    from zipage_amd.layers import rotary_store, store_form
+    n, H, G, D = 11_721, 32, 8, 128
+    assert n * (2 * H + 3 * 2 * G) * D * 2 >= 320 << 20 > 4000 * (2 * H + 3 * 2 * G) * D * 2
+    x = _rand(dev, torch.bfloat16, n, (H + 2 * G) * D, seed=1)
+    g = torch.Generator().manual_seed(2)
+    pos = torch.randint(0, 5000, (n,), generator=g).int().to(dev)
+    slots = torch.randperm(n + 9, generator=g)[:n].int()
+    slots[::7] = -1
+    slots = slots.to(dev)
+    bias = _rand(dev, F32, (H + 2 * G) * D, seed=3) if form == "bias" else None
+    weights = _rand(dev, F32, (H + G) * D, seed=4)
+
+    def store(parts):
+        cache, out = torch.full((1, n + 9, 2 * G * D), 7.0, dtype=torch.bfloat16, device=dev), []
+        for a, b in parts:
+            turns = torch.zeros(b - a, D // 2, 2, device=dev)
+            f = {"turning": lambda: store_form(value_freqs=_freqs(dev, D // 2, 40.0), turns=turns),
+                 "norms": lambda: store_form(norm=weights, q_norm=H * D, k_norm=G * D, eps=1e-6),
+                 "tied": lambda: store_form(tied=True)}.get(form, lambda: None)()
+            q, kv = rotary_store(x[a:b], pos[a:b], _freqs(dev, 32), H, G, D, D, cache, slots[a:b], return_kv=True, bias=bias, form=f)
+            out.append((q, kv, turns))
+        return [torch.cat(t) for t in zip(*out)] + [cache]
+    for a, b in zip(store([(0, n)]), store([(i, min(n, i + 4000)) for i in range(0, n, 4000)])):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("dtype", DTYPES, ids=ids)
 @pytest.mark.parametrize("H,G,D,dim,rot", [(4, 2, 32, 32, 32), (6, 3, 32, 20, 10), (8, 8, 16, 9, 0), (20, 1, 80, 72, 48), (2, 2, 256, 250, 250)])
 def test_keys_that_are_values_and_norms_over_all_heads(dev, dtype, H, G, D, dim, rot):
