@@ -502,7 +502,8 @@ def test_latent_rows_by_width_and_heads(dev, H, R, P, BS, window):
 
 
 # a pool and tables of 320 MB and more: rows are asked for past the last-level cache, by the same sums
-@pytest.mark.parametrize("H,R,P", [(16, 512, 64), (20, 384, 8), (33, 512, 64), (40, 128, 64), (65, 512, 0)])
+@pytest.mark.parametrize("H,R,P", [(16, 512, 64), (20, 320, 64), (33, 512, 64), (40, 128, 64), (65, 512, 0),
+                                   (20, 256, 64), (16, 128, 0), (32, 256, 0)])
 def test_latent_rows_past_the_cache(dev, H, R, P):
     from zipage_amd.layers import latent_rows_attention
     BS, used, ctx = 1024, 8, [0, 1, 33, 700, 1024, 2500]
@@ -517,6 +518,24 @@ def test_latent_rows_past_the_cache(dev, H, R, P):
     past = latent_rows_attention(q, cache, t, n, 1.0, None, rank=R)
     assert torch.equal(past, latent_rows_attention(q, cache[:used].clone(), t, n, 1.0, None, rank=R))
     assert past[1:].any(-1).all()
+
+
+@pytest.mark.parametrize("H,G,D,V", [(8, 2, 128, 128), (16, 1, 64, 64), (6, 2, 96, 256), (34, 2, 128, 128)])
+def test_grouped_rows_past_the_cache(dev, H, G, D, V):
+    from zipage_amd.layers.grouped import grouped_rows_attention
+    BS, used, ctx, row = 1024, 8, [0, 1, 33, 700, 1024, 2500], G * (D + V)
+    pages = (320 << 20) // (BS * row * 2) + 1
+    cache = torch.zeros(pages, BS, row, dtype=torch.bfloat16, device=dev)
+    cache[:used] = _rand(used, BS, row, seed=H).to(dev)
+    tables = torch.full((len(ctx), pages), -1, dtype=torch.int32)
+    for i, c in enumerate(ctx):
+        tables[i, :-(-c // BS)] = (torch.arange(-(-c // BS)) * 3 + i).int() % used
+    q = _rand(len(ctx), H * D, seed=D).to(dev)
+    t, n = tables.to(dev), torch.tensor(ctx, dtype=torch.int32, device=dev)
+    got = [torch.empty(len(ctx), H * V, dtype=torch.bfloat16, device=dev) for _ in range(2)]
+    for out, c in zip(got, (cache, cache[:used].clone())):
+        grouped_rows_attention(q, c, H, G, D, V, t, n, D ** -0.5, out)
+    assert torch.equal(*got) and got[0][1:].any(-1).all()
 
 
 # ------------------------------------------------------------------ per-head products

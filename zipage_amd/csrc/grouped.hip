@@ -13,6 +13,7 @@
 // other one's elements are, so that keys and values are still read once.  Values that turned with their
 // position turn back with the query's in the last step of a kernel.
 #include "mfma.h"
+#include <algorithm>
 
 namespace {
 
@@ -243,8 +244,9 @@ __device__ __forceinline__ int first_key(const RowsArgs& a, int n) {   // n toke
 // are flash loops of their own over every fourth 32-key step and meet in LDS at the end.  Keys are the
 // row operand straight from memory (64-byte pieces), values are loaded as rows and turned into column
 // operands by v_perm.  The next step's keys are requested once the scores are done, its values once the
-// value products are.
-template <int DKS, int VCB, int MAPS>
+// value products are.  PAST: values, of which a load reads whole lines, pass the last-level cache by; keys, read as operands in
+// parts of lines, don't (256 sequences, 32 heads over 8 of 128: 393 us, values past it 363, both 386).
+template <int DKS, int VCB, int MAPS, bool PAST>
 __global__ __launch_bounds__(256, 2) void grouped_rows_kernel(RowsArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   int* const pg = (int*)lds_raw;
@@ -308,7 +310,7 @@ __global__ __launch_bounds__(256, 2) void grouped_rows_kernel(RowsArgs a) {
     for (int i = 0; i < 8; ++i) {
       const uint16_t* v = vc + row_at(b * 32 + step_key(g, i));
 #pragma unroll
-      for (int cb = 0; cb < VCB; ++cb) vf[cb][i] = *(const u32x4*)(v + col[cb]);
+      for (int cb = 0; cb < VCB; ++cb) vf[cb][i] = load_piece<PAST>(v + col[cb]);
     }
   };
   f32x4 o[VCB * 8];
@@ -621,15 +623,15 @@ int rows_splits(int n, int H, int HK, int window, int chunk, int NB, int BS) {
   return s < 1 ? 1 : s;
 }
 
-template <int DKS, int VCB, int MAPS> int launch_rows(const RowsArgs& a, hipStream_t st) {
+template <int DKS, int VCB, int MAPS, bool PAST> int launch_rows(const RowsArgs& a, hipStream_t st) {
   const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + 4 * sizeof(float) * (16 * (a.V + 4) + 32);
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)grouped_rows_kernel<DKS, VCB, MAPS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)grouped_rows_kernel<DKS, VCB, MAPS, PAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)smem) != hipSuccess) {
     zp_set_error("grouped_rows_attention: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((grouped_rows_kernel<DKS, VCB, MAPS>), dim3((unsigned)a.n * a.HK * a.htiles * a.splits), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((grouped_rows_kernel<DKS, VCB, MAPS, PAST>), dim3((unsigned)a.n * a.HK * a.htiles * a.splits), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   if (a.splits > 1) {
     if (MAPS == 2) hipLaunchKernelGGL(grouped_pair_combine_kernel, dim3((unsigned)a.n * a.H / 2), dim3(64), 0, st, a);
@@ -637,6 +639,19 @@ template <int DKS, int VCB, int MAPS> int launch_rows(const RowsArgs& a, hipStre
     ZP_LAUNCH_CHECK();
   }
   return ZP_OK;
+}
+// Values go past the last-level cache where one workgroup reads them, in whole lines, and all rows that may be read do not
+// fit: 40 sequences of about 2050 tokens, 32 heads over 8 of 128 89 us and 80, 256 of them 393 and 363, heads of 64 over 4
+// 112 and 96, 256 of 100 to 4096 tokens 456 and 428.
+bool rows_past(const RowsArgs& a) {
+  int64_t keys = (int64_t)a.NB * a.BS;
+  if (a.window > 0) keys = std::min<int64_t>(keys, a.window);
+  if (a.chunk > 0) keys = std::min<int64_t>(keys, a.chunk);
+  return a.htiles == 1 && a.V % 64 == 0 && (int64_t)a.HK * a.D % 64 == 0 &&
+         past_cache(std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * a.HK * (a.D + a.V) * 2);
+}
+template <int DKS, int VCB, int MAPS> int launch_rows(const RowsArgs& a, hipStream_t st) {
+  return rows_past(a) ? launch_rows<DKS, VCB, MAPS, true>(a, st) : launch_rows<DKS, VCB, MAPS, false>(a, st);
 }
 template <int MAPS> int dispatch_rows(const RowsArgs& a, hipStream_t st) {
   const int dk = (a.D + 31) / 32;
@@ -681,7 +696,7 @@ extern "C" int zp_rotary_store(const void* in, const float* bias, const int32_t*
   // and the attention behind it 298 -> 285.  Without kv_out the attention reads the cache's rows.
   const int64_t kvw = (int64_t)HK * D + VT;
   const bool past = kv_out && tokens == 4 && dtype == ZP_BF16 && rot % 16 == 0 &&
-                    (2 * (int64_t)H * D + 3 * kvw) * n * 2 >= 320ll << 20;
+                    past_cache((2 * (int64_t)H * D + 3 * kvw) * n * 2);
   const unsigned grid = (unsigned)((n + tokens - 1) / tokens);
   const size_t smem = ((sizeof(float2) * tokens * (rot / 2 + (f.value_freqs ? f.V / 2 : 0)) + 15) & ~(size_t)15) + tokens * a.staged;
   hipStream_t st = (hipStream_t)stream;

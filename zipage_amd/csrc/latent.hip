@@ -379,7 +379,7 @@ template <int NCB, int PK> struct RowsLds {
 };
 __host__ __device__ inline int rows_merge_floats(int R) { return 16 * (R + 4) + 32; }   // per wave
 
-template <int NCB, int HT, int PK>
+template <int NCB, int HT, int PK, bool PAST>
 __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kernel(RowsArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef RowsLds<NCB, PK> Lds;
@@ -464,7 +464,7 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
       const int key = min(max(b * 32 + hf * 16 + l16, from[hf]), upto[hf]);
       const uint32_t ro = (uint32_t)((key & mask) * RW * 2);
 #pragma unroll
-      for (int ks = 0; ks < PK; ++ks) kr[hf][ks] = *(const u32x4*)(base[hf] + (ro + rot_off[ks]));
+      for (int ks = 0; ks < PK; ++ks) kr[hf][ks] = load_piece<PAST>(base[hf] + (ro + rot_off[ks]));
     }
   };
 
@@ -476,7 +476,7 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
     for (int i = 0; i < 8; ++i) {
       const uint32_t ro = row_off(b, i);
 #pragma unroll
-      for (int cb = 0; cb < NCB; ++cb) v[cb][i] = *(const u32x4*)(base[i >> 2] + (ro + col_off[cb]));
+      for (int cb = 0; cb < NCB; ++cb) v[cb][i] = load_piece<PAST>(base[i >> 2] + (ro + col_off[cb]));
     }
     load_rotated(b);
   }
@@ -564,7 +564,7 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
         for (int ht = 0; ht < HT; ++ht) o[ht][cb * 8 + t] = mfma_bf16(vf, pf[ht], o[ht][cb * 8 + t]);
       }
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[cb][i] = *(const u32x4*)(base[i >> 2] + (ro[i] + col_off[cb]));
+      for (int i = 0; i < 8; ++i) v[cb][i] = load_piece<PAST>(base[i >> 2] + (ro[i] + col_off[cb]));
     }
   }
 
@@ -1041,26 +1041,31 @@ int launch_combine(const RowsArgs& a, hipStream_t st) {
   }
   return ZP_OK;
 }
-template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
+// Whether rows are asked for past the last-level cache: one workgroup reads a key, in whole lines, and all that may be read do
+// not fit.  256 sequences of 1800 to 2304 tokens: rows of 576, 16 heads 115 us through it and 103 past it, 32 heads 122 and
+// 115, 64 heads 181 and 176; rows of 320, 32 heads 78 and 73, 16 heads 71 and 65.  With two workgroups on a token (128
+// heads) 324 and 338; where rows fit, 40 sequences, 42 and 43; rows of 192, 200 MB, 42 and 47.
+bool rows_past(const RowsArgs& a, int hgroups) {
+  const int64_t keys = a.window > 0 ? std::min<int64_t>(a.window, (int64_t)a.NB * a.BS) : (int64_t)a.NB * a.BS;
+  return hgroups == 1 && (a.R + a.P) % 64 == 0 &&
+         past_cache(std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * (a.R + a.P) * 2);
+}
+template <int NCB, int HT, int PK, bool PAST> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
   const size_t merge = 4 * sizeof(float) * (size_t)rows_merge_floats(a.R);
   const size_t work = 4 * RowsLds<NCB, PK>::kStage + (size_t)HT * RowsLds<NCB, PK>::kQ;
   const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + (merge > work ? merge : work);
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)latent_narrow_kernel<NCB, HT, PK>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)latent_narrow_kernel<NCB, HT, PK, PAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)smem) != hipSuccess) {
     zp_set_error("latent_rows_attention: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((latent_narrow_kernel<NCB, HT, PK>), dim3((unsigned)a.n * a.splits), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((latent_narrow_kernel<NCB, HT, PK, PAST>), dim3((unsigned)a.n * a.splits), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return launch_combine(a, st);
 }
-// Whether rows are asked for past the last-level cache: one workgroup reads a key, and all that may be read do not fit.  Rows
-// of 576, 256 sequences of 1800 to 2304 tokens, 16 heads 115 us through it and 103 past it, 32 heads 122 and 115, 64 heads
-// 181 and 176; with two workgroups on a token (128 heads) 324 and 338, and where rows fit, 40 sequences, 42 and 43.
-bool rows_past(const RowsArgs& a, int hgroups) {
-  const int64_t keys = a.window > 0 ? std::min<int64_t>(a.window, (int64_t)a.NB * a.BS) : (int64_t)a.NB * a.BS;
-  return hgroups == 1 && std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * (a.R + a.P) * 2 >= 320ll << 20;
+template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
+  return rows_past(a, 1) ? launch_latent_narrow<NCB, HT, PK, true>(a, st) : launch_latent_narrow<NCB, HT, PK, false>(a, st);
 }
 template <int NCB, int HW, int PK, bool PAST> int launch_latent_rows(const RowsArgs& a, int hgroups, hipStream_t st) {
   constexpr int smem = RowsStage<NCB, PK>::kBytes + (HW < 4 ? 4096 : 0);

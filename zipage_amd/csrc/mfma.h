@@ -38,7 +38,13 @@ __device__ __forceinline__ uint2 read_transposed(const uint16_t* p) {
 // which cannot tell the stage being filled from the stage being read, would wait for it at the next LDS read; what
 // waits is the code that meets the other waves.
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
-template <bool PAST = false>      // past the last-level cache
+// PAST: past the last-level cache, where more is read once than that holds
+template <bool PAST> __device__ __forceinline__ u32x4 load_piece(const void* p) {
+  if constexpr (PAST) return __builtin_nontemporal_load((const u32x4*)p);
+  return *(const u32x4*)p;
+}
+inline bool past_cache(int64_t bytes) { return bytes >= 320ll << 20; }
+template <bool PAST = false>
 __device__ __forceinline__ void load_to_lds(const u32x4& rows, void* lds, int lane_at, int at) {
   const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
   const int so = __builtin_amdgcn_readfirstlane(at);
