@@ -250,10 +250,16 @@ enum {
 };
 
 /* Bytes of device workspace zp_compress_layers needs for these dims (scores, redundancy, the
- * stages' own scratch, and the keep flags when flag_in_workspace != 0); -1 on bad arguments. */
+ * stages' own scratch, and the keep flags when flag_in_workspace != 0); -1 on bad arguments.  More
+ * sequences need more, so what serves the largest batch serves every other.  With
+ * zp_compress_layers_workspace_few() bytes, which are more for few sequences, their scores are
+ * spread over the chip (see zp_attention_score): the same bits, sooner. */
 int64_t zp_compress_layers_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv,
                                      int32_t Hq, int32_t W, int32_t dtype,
                                      const zp_compress_config* cfg, int32_t flag_in_workspace);
+int64_t zp_compress_layers_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv,
+                                         int32_t Hq, int32_t W, int32_t dtype,
+                                         const zp_compress_config* cfg, int32_t flag_in_workspace);
 
 /* k_cache / v_cache (L, num_pages, BS, Hkv, D), compacted in place; query_cache
  * (L, max_seqs, W, Hq, D); score_cache (L, num_pages, BS, Hkv) or NULL (required with

@@ -96,3 +96,16 @@ def test_product_has_no_cpu_fallback():
     from zipage_amd.kernel import topk_mask
     with pytest.raises(RuntimeError, match="device tensors"):
         topk_mask(torch.zeros(2, 8), 3)
+
+
+def test_a_workspace_for_the_largest_batch_serves_every_other():
+    from zipage_amd import _lib
+    from zipage_amd.compress import CompressConfig, c_config
+    lib = _lib.load()
+    for kw in (dict(), dict(use_redudancy=True, use_global_score=True, decay_factor=0.8)):
+        cc = c_config(CompressConfig(budget_blocks=8, query_cache_len=16, **kw))
+        for dtype, heads, window in ((0, 32, 32), (1, 16, 16), (2, 16, 32)):
+            sizes = [lib.zp_compress_layers_workspace(1, b, 9, 256, 8, heads, window, dtype, ctypes.byref(cc), 0) for b in range(1, 70)]
+            assert sizes == sorted(sizes)
+            few = [lib.zp_compress_layers_workspace_few(1, b, 9, 256, 8, heads, window, dtype, ctypes.byref(cc), 0) for b in range(1, 70)]
+            assert few[0] > sizes[0] and few[-1] == sizes[-1] and all(f >= s for f, s in zip(few, sizes))

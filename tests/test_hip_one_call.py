@@ -112,6 +112,31 @@ def test_one_call_rejects_a_short_workspace(dev):
                   ctypes.byref(cc), ws.data_ptr(), need - 256, None, 0)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("name", ["pooling", "scripts", "max-reduced"])
+def test_one_call_with_the_workspace_of_a_larger_batch(dev, dtype, name):
+    """Two sequences in the workspace that five need without room for the scores of few, and in one with it: same bits."""
+    import ctypes
+    from zipage_amd import _lib
+    from zipage_amd.compress import CompressConfig, c_config, layer_chunk_args
+    tensors = _inputs(dtype, L=1, B=2, Hkv=4, Hq=16)
+    cc, lib, outs = c_config(CompressConfig(budget_blocks=2, query_cache_len=16, **SWITCHES[name])), _lib.load(), []
+    for batch, size in ((5, lib.zp_compress_layers_workspace), (2, lib.zp_compress_layers_workspace), (2, lib.zp_compress_layers_workspace_few)):
+        k, v, q, sc, qid, enc, comp, target = (t.clone().to(dev) for t in tensors)
+        dims, strides = layer_chunk_args(k, v, q, sc, qid, enc, comp, target)
+        L, B, NB, BS, Hkv, Hq, D, W = dims[:8]
+        tag = _lib.dtype_tag(k)
+        bytes_ = size(L, batch, NB, BS, Hkv, Hq, W, tag, ctypes.byref(cc), 0)
+        ws, flag = (torch.zeros(s, dtype=torch.uint8, device=dev) for s in (bytes_, L * B * Hkv * NB * BS))
+        _lib.call("zp_compress_layers", *(t.data_ptr() for t in (k, v, q, sc, qid, enc, comp, target, flag)), *dims, strides, tag,
+                  ctypes.byref(cc), ws.data_ptr(), bytes_, None, _lib.stream_ptr(k))
+        torch.cuda.synchronize()
+        outs.append([t.cpu() for t in (flag, k, v, sc)])
+    for other in outs[1:]:
+        for a, b in zip(outs[0], other):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+
+
 @pytest.mark.parametrize("kw", [dict(enable_pooling=True, pooling_size=5),
                                 dict(use_global_score=True, decay_factor=0.8)],
                          ids=["pooling", "global-score"])

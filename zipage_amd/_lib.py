@@ -79,6 +79,8 @@ STATIC_SCRATCH_BYTES = 32 << 20
 I64_RETURNING = {
     "zp_compress_layers_workspace": [i32, i32, i32, i32, i32, i32, i32, i32,
                                      C.POINTER(CompressConfigC), i32],
+    "zp_compress_layers_workspace_few": [i32, i32, i32, i32, i32, i32, i32, i32,
+                                         C.POINTER(CompressConfigC), i32],
     "zp_attention_score_workspace": [i32, i32, i32, i32, i32, i32, i32],
     "zp_attention_score_workspace_for": [i32, i32, i32, i32, i32, i32, i32, i32],
     "zp_attention_score_workspace_few": [i32, i32, i32, i32, i32, i32, i32, i32],

@@ -270,7 +270,7 @@ def _compress_layers_one_call(k_cache, v_cache, query_cache, score_cache, query_
     cc = c_config(cfg, deterministic_carry)
     lib = _lib.load()
     tag = _lib.dtype_tag(k_cache)
-    ws_bytes = lib.zp_compress_layers_workspace(L, B, NB, BS, Hkv, Hq, W, tag, ctypes.byref(cc), 0)
+    ws_bytes = lib.zp_compress_layers_workspace_few(L, B, NB, BS, Hkv, Hq, W, tag, ctypes.byref(cc), 0)
     ws = torch.empty(ws_bytes, device=k_cache.device, dtype=torch.uint8)
     running = {"attention_score", FUSED_SELECT_STAGE, "compress_kv"}
     if cfg.use_global_score:

@@ -26,8 +26,8 @@ struct Plan {
 // Rows the one-launch selection holds in LDS (zp_select_topk's own limit).
 inline bool select_fits(int64_t Tn) { return Tn * 8 <= 150 * 1024; }
 
-// What the scorer gets.  Callers with a fixed scratch budget go down the list: logits of few sequences in memory; one sweep
-// over K with the logits in registers; only what it cannot do without, for three sweeps.
+// What the scorer gets.  Callers with less scratch go down the list: logits of few sequences in memory; one sweep over K with
+// the logits in registers; only what it cannot do without, for three sweeps.
 enum class Scratch { all, one_sweep, floor };
 Plan make_plan(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype,
                const zp_compress_config* c, bool own_flag, Scratch scratch = Scratch::all) {
@@ -289,14 +289,26 @@ extern "C" int zp_static_scratch_init(void) {
   return static_scratch(&ws);
 }
 
+static int64_t layers_workspace(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype, const zp_compress_config* cfg,
+                                bool own_flag, Scratch scratch) {
+  if (!cfg || L < 0 || B < 0 || NB <= 0 || BS <= 0 || Hkv <= 0 || Hq <= 0 || W <= 0 ||
+      dtype < ZP_BF16 || dtype > ZP_F32)
+    return -1;
+  return make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, own_flag, scratch).total;
+}
+
 extern "C" int64_t zp_compress_layers_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                                 int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype,
                                                 const zp_compress_config* cfg,
                                                 int32_t flag_in_workspace) {
-  if (!cfg || L < 0 || B < 0 || NB <= 0 || BS <= 0 || Hkv <= 0 || Hq <= 0 || W <= 0 ||
-      dtype < ZP_BF16 || dtype > ZP_F32)
-    return -1;
-  return make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_in_workspace != 0).total;
+  return layers_workspace(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_in_workspace != 0, Scratch::one_sweep);
+}
+
+extern "C" int64_t zp_compress_layers_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS,
+                                                    int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype,
+                                                    const zp_compress_config* cfg,
+                                                    int32_t flag_in_workspace) {
+  return layers_workspace(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_in_workspace != 0, Scratch::all);
 }
 
 extern "C" int zp_compress_layers(void* k_cache, void* v_cache, const void* query_cache,
@@ -316,7 +328,9 @@ extern "C" int zp_compress_layers(void* k_cache, void* v_cache, const void* quer
   ZP_REQUIRE(k_cache && v_cache && query_cache && seq_idx && block_table && compressed &&
                  target_block_table && strides, "compress_layers: null pointer");
   if (L == 0 || B == 0) return ZP_OK;
-  const Plan p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr);
+  // the scores of few sequences are faster with more scratch, but a workspace that serves the largest batch serves all
+  Plan p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr);
+  if (workspace_bytes < p.total) p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr, Scratch::one_sweep);
   ZP_REQUIRE(workspace && workspace_bytes >= p.total,
              "compress_layers: workspace of %lld bytes required, %lld given", (long long)p.total,
              (long long)workspace_bytes);
