@@ -1,5 +1,6 @@
 // Attention of runs of prompt tokens, and the gather of the cached rows they look back on.
 #include "mfma.h"
+#include "launch_order.h"
 
 namespace {
 
@@ -35,6 +36,7 @@ struct TilesArgs {
   const uint16_t* gate;   // token rows of g_st elements, head h at h * V; or null
   int64_t g_st;
   const float2* turns;    // one map: (q_rows, V / 2) cos and sin, results turn back by them; or null
+  bool rising;            // a run's tiles come in the order of their keys; otherwise those with many keys first
 };
 
 constexpr int kTileQ = 128;   // queries per workgroup
@@ -405,29 +407,6 @@ template <int KS, int VB> struct FlowStage {                   // 16 KS elements
   static constexpr int kBytes = 2 * (K::kBytes + V::kBytes);
 };
 
-// Which head and tile a workgroup takes.  Those of one L2 (x, eighths of the launch) have the query heads of a key head next
-// to one another and its tiles behind, the last ones first: what reads the same keys at the same time reads them from there.
-struct FlowPlace {
-  int h, hk, tile;
-  __host__ __device__ static int part_bits(int heads) { return heads % 8 == 0 ? 3 : heads % 4 == 0 ? 2 : heads % 2 == 0 ? 1 : 0; }
-  __host__ __device__ static int tiles_of(int T, int bits) { return (T + (8 >> bits) - 1) >> (3 - bits); }
-  __host__ static dim3 grid(const TilesArgs& a) {
-    const int bits = part_bits(a.HK);
-    return dim3(8, a.H / a.HK, (unsigned)tiles_of(a.T, bits) * (a.HK >> bits));
-  }
-  __device__ __forceinline__ FlowPlace(const TilesArgs& a) {
-    const int bits = part_bits(a.HK), part = blockIdx.x, tiles = tiles_of(a.T, bits);
-    int at = blockIdx.z, from = 0;
-    if (at >= tiles) {
-      from = at / tiles;
-      at -= from * tiles;
-    }
-    hk = (from << bits) + (part & ((1 << bits) - 1));
-    h = hk * (int)gridDim.y + blockIdx.y;
-    tile = ((tiles - 1 - at) << (3 - bits)) + (part >> bits);  // past the last one: nothing to do
-  }
-};
-
 // A wave's results on their way out: lane l32 of either half has a query's columns 8 (i / 4) + 4 half + i % 4 of each 32.
 template <int VB>
 __device__ __forceinline__ void flow_out(const TilesArgs& a, int h, int64_t row, bool there, f32x16 (&o)[VB], float m, float l) {
@@ -464,9 +443,9 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   constexpr int kQK = 2 * KS, kPV = 2 * VB;                    // products of a tile's keys, of half its values
   const int lane = threadIdx.x & 63, l16 = lane & 15, l32 = lane & 31, g = lane >> 4, half = lane >> 5;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const FlowPlace place(a);
-  const int h = place.h, tile = place.tile;
-  if (tile >= a.T) return;
+  const FlowPlace place(a.T, a.HK, a.rising, blockIdx.x, blockIdx.z);
+  const int h = place.hk * (int)gridDim.y + blockIdx.y, tile = place.tile;
+  if (tile >= a.T) return;                                     // a part that has fewer
   const int q0 = a.tiles[tile * 4], nq = min(a.tiles[tile * 4 + 1], kTileQ);
   const int kb = a.tiles[tile * 4 + 2], rel = a.tiles[tile * 4 + 3];
   // host-made descriptors: rows outside the buffers are not touched
@@ -710,6 +689,7 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   flow_out(a, h, q0 + qi, qi < nq, o, m, l);
 }
 
+inline dim3 flow_grid(const TilesArgs& a) { return dim3(8, a.H / a.HK, (unsigned)FlowPlace::depth(a.T, a.HK)); }
 template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
   constexpr int smem = FlowStage<KS, VB>::kBytes;
   if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)run_flow_kernel<KS, VB, FINE>, hipFuncAttributeMaxDynamicSharedMemorySize,
@@ -717,7 +697,7 @@ template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& a, hipStre
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE>), FlowPlace::grid(a), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE>), flow_grid(a), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -726,7 +706,7 @@ template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& a, hipStre
 inline bool few_keys(const TilesArgs& a) { return a.k_rows <= 256 && a.k_rows <= 32 * (int64_t)a.T; }
 // Offsets within a tile are 32 bits, the launch is three-dimensional.
 inline bool flow_takes(const TilesArgs& a) {
-  const dim3 grid = FlowPlace::grid(a);
+  const dim3 grid = flow_grid(a);
   return a.D <= 128 && a.V <= 128 && (a.V <= 64 || !few_keys(a)) && a.kv_st < 1 << 24 && a.v_st < 1 << 24 && grid.y < 65536 &&
          grid.z < 65536;
 }
@@ -827,7 +807,7 @@ extern "C" int zp_run_attention(const void* q, const void* k, const void* v, con
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, (const uint16_t*)k_shared, (uint16_t*)out,
                  tiles, sinks, T, H, HK, D, P, V, window, chunk, q_rows, k_rows, q_stride, kv_stride, kv_stride, shared_stride,
                  out_stride, scale, out_scale, f.softcap, f.balance, f.eps, f.vdim, (const uint16_t*)f.gate, f.gate_stride,
-                 (const float2*)f.turns};
+                 (const float2*)f.turns, true};
   hipStream_t st = (hipStream_t)stream;
   if (P) return launch_one_map<true, kNoCap>(a, st);
   if (!(f.softcap > 0.f)) return launch_forms<kNoCap>(a, two, st);
@@ -854,7 +834,7 @@ extern "C" int zp_causal_attention(const void* q, const void* k, const void* v, 
              "causal_attention: unaligned rows or too many tiles");
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, tiles, nullptr, T, H, HK,
                  D, 0, D, 0, 0, q_rows, k_rows, q_stride, k_stride, v_stride, 0, out_stride, scale, 1.f, 0.f, 0.f, 0.f, D,
-                 nullptr, 0, nullptr};
+                 nullptr, 0, nullptr, false};
   if (flow_takes(a)) return launch_flow<true>(a, (hipStream_t)stream);
   return launch_run_tiles<4, 1, 2, 1, false, kNoCap, true>(a, (hipStream_t)stream);
 }
