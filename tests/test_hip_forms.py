@@ -228,6 +228,21 @@ def test_runs_of_few_keys(dev, H, G, D, V):
     test_runs_of_any_scale(dev, H, G, D, V, 0.25, FEW_KEYS)
 
 
+# launches of many workgroups take runs of up to 128 keys apart from 1024 workgroups on, of up to 64 from 512 on; beside them
+# longer runs, and runs with cached context
+MANY_SHORT = [(n, n) for n in (1, 16, 31, 33, 63, 64, 65, 100, 127, 128, 129)] * 6 + [(40, 90), (3, 300), (200, 264), (300, 300)]
+
+
+@pytest.mark.parametrize("H,G,D,V", [(16, 8, 128, 128), (15, 5, 72, 104), (8, 8, 56, 128), (4, 2, 128, 72)])
+def test_many_short_runs(dev, H, G, D, V):
+    test_runs_of_any_scale(dev, H, G, D, V, -0.25 if G == 8 else 0.25, MANY_SHORT)
+
+
+@pytest.mark.parametrize("H,G,D", [(16, 4, 128), (8, 2, 104)])
+def test_causal_attention_of_many_short_prompts(dev, H, G, D):
+    test_causal_attention(dev, H, G, D, MANY_SHORT)
+
+
 def test_causal_attention_of_few_keys(dev):
     test_causal_attention(dev, 8, 2, 128, FEW_KEYS)
 

@@ -37,6 +37,7 @@ struct TilesArgs {
   int64_t g_st;
   const float2* turns;    // one map: (q_rows, V / 2) cos and sin, results turn back by them; or null
   bool rising;            // a run's tiles come in the order of their keys; otherwise those with many keys first
+  int few_tiles;          // tiles of keys up to which a workgroup takes the form that stages no tile ahead
 };
 
 constexpr int kTileQ = 128;   // queries per workgroup
@@ -92,14 +93,12 @@ constexpr int long_step(int DKS, int VCB, int MAPS, bool SHARED, int CAP) {
 // values; elsewhere there is one).  SHARED: the last P elements of every head's key are the row of a.ks.
 // FINE: softmax weights enter the value product as two bf16 planes (17 bits), elsewhere as one.
 template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
-__global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(TilesArgs a) {
-  extern __shared__ __align__(16) char lds_raw[];
+__device__ __forceinline__ void run_tile(const TilesArgs& a, char* lds_raw, int h, int tile) {
   typedef TileStage<DKS, VCB, MAPS> Stage;
   constexpr bool kTurns = MAPS == 1 && !SHARED && CAP == kNoCap;
   constexpr bool kPinned = DKS <= 4 && (VCB == 1 || MAPS == 1);   // reads ahead: wider heads would spill
   constexpr int kT = kQT * MAPS, kWaves = Stage::kWaves, kThreads = 64 * kWaves, kPass = 16 * kQT * kWaves;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, g = lane >> 4;
-  const int h = blockIdx.x % a.H, tile = blockIdx.x / a.H;   // one head's tiles share an L2 when H % 8 == 0
   const int q0 = a.tiles[tile * 4], nq = min(a.tiles[tile * 4 + 1], kTileQ);
   const int kb = a.tiles[tile * 4 + 2], rel = a.tiles[tile * 4 + 3];
   // host-made descriptors: rows outside the buffers are not touched
@@ -370,6 +369,12 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
   }
 }
 
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
+__global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(TilesArgs a) {
+  extern __shared__ __align__(16) char lds_raw[];
+  run_tile<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>(a, lds_raw, blockIdx.x % a.H, blockIdx.x / a.H);   // one head's tiles share an L2 when H % 8 == 0
+}
+
 // ------------------------------------------------------------------ heads of at most 128, one map, no cap
 // Here the products of a tile's keys run while the exponentials of the tile before take their turn, which needs the scores
 // of two tiles in registers.  A 32 x 32 product takes 8 of its 32 cycles at the vector issue, a 16 x 16 one 8 of 16: with the
@@ -462,6 +467,8 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   const int first = first_seen(rel, a.window, a.chunk), last = rel + nq - 1;    // keys that any query sees
   const int lo = first_seen(rel + w0, a.window, a.chunk), lo_last = first_seen(rel + w0 + 31, a.window, a.chunk);
   const int tiles = (last - first) / kTileK + 1;
+  if constexpr (VB == 4)
+    if (tiles <= a.few_tiles) return run_tile<KS / 2, 1, 2, 1, false, kNoCap, FINE, 32>(a, lds_raw, h, tile);
   // tiles that queries of the wave see; none: they begin behind the last one
   const int seen0 = w0 < nq ? (lo - first) / kTileK : tiles + 1;
   const int seen1 = w0 < nq ? (rel + min(w0 + 32, nq) - 1 - first) / kTileK : tiles + 1;
@@ -690,13 +697,24 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
 }
 
 inline dim3 flow_grid(const TilesArgs& a) { return dim3(8, a.H / a.HK, (unsigned)FlowPlace::depth(a.T, a.HK)); }
-template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
-  constexpr int smem = FlowStage<KS, VB>::kBytes;
+// Values of more than 64, few keys: the flow has one tile on its way, sets up for one behind it and counts keys by 64, which pays from
+// three tiles on, and in small launches, where a workgroup's own time counts, from two or one.  Heads over 8 of 128, us in the
+// flow alone and with short tiles in the other form: 32 heads, 256 prompts of 64 tokens 139 and 110, 128 of 128 106 and 91,
+// 64 of 256 117 and 113, 512 of 32 206 and 162; 16 heads, 128 of 128 54 and 49; 2 tiles, 512 workgroups (16 of 128 tokens, 32
+// heads) 16.9 and 18.6; one tile, 512 workgroups 11.1 and 10.6, 256 8.8 and 8.9, one prompt of 64 8.1 and 8.4.
+inline int few_tiles(const TilesArgs& a) {
+  const int64_t groups = (int64_t)a.T * a.H;
+  return groups >= 1024 ? 2 : groups >= 512 ? 1 : 0;
+}
+template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& args, hipStream_t st) {
+  constexpr int flow = FlowStage<KS, VB>::kBytes, steps = VB == 4 ? TileStage<KS / 2, 1, 1>::kBytes : 0, smem = flow > steps ? flow : steps;
   if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)run_flow_kernel<KS, VB, FINE>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               smem) != hipSuccess) {
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
+  TilesArgs a = args;
+  a.few_tiles = few_tiles(a);
   hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE>), flow_grid(a), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
