@@ -289,20 +289,55 @@ def test_products_of_few_rows(dev, dtype, n, K, M):
     assert bool(((out[:, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
 
 
-def test_which_products_are_of_few_rows(dev):
+@pytest.fixture
+def few_rows_calls(monkeypatch):
+    """Says whether the kernel for few rows was called since it last did."""
+    from zipage_amd import _lib
+    made, call = [], _lib.call_models
+    monkeypatch.setattr(_lib, "call_models", lambda name, *args: (made.append(name), call(name, *args))[1])
+
+    def called():
+        n = made.count("zp_few_rows_linear")
+        made.clear()
+        return n > 0
+    return called
+
+
+def test_which_products_are_of_few_rows(dev, few_rows_calls):
     from zipage_amd.layers import linear
     w = (_rand(96, 64, seed=1).float() / 8).to(BF16).to(dev)
-    for x in (_rand(5, 64, seed=2).to(dev), _rand(64, 64, seed=3).to(dev), _rand(65, 64, seed=4).to(dev), _rand(5, 128, seed=5).to(dev)[:, ::2],
-              _rand(5, 65, seed=6).to(dev)[:, 1:], _rand(2, 3, 64, seed=7).to(dev), _rand(0, 64, seed=8).to(dev), _rand(64, 5, seed=9).to(dev).T):
+    wide = _rand(5, 96, seed=10).to(dev)
+    for few, x in ((True, _rand(5, 64, seed=2).to(dev)), (True, _rand(1, 64, seed=2).to(dev)), (True, wide[:, 8:72]),
+                   (False, _rand(65, 64, seed=4).to(dev)), (False, _rand(5, 128, seed=5).to(dev)[:, ::2]),
+                   (False, _rand(5, 65, seed=6).to(dev)[:, 1:]), (False, wide[:, 1:65]), (False, _rand(2, 3, 64, seed=7).to(dev)),
+                   (False, _rand(0, 64, seed=8).to(dev)), (False, _rand(64, 5, seed=9).to(dev).T)):
         want = torch.nn.functional.linear(x, w)
         got = linear(x, w)
+        assert few_rows_calls() == few, x.shape
         assert got.shape == want.shape and got.dtype == want.dtype
         assert bool(((got.double() - want.double()).abs() <= 2.0 ** -7 * want.double().abs() + 2.0 ** -18).all())
+    x = _rand(5, 64, seed=2).to(dev)
+    with torch.inference_mode():
+        linear(x, w)
+    assert few_rows_calls()
     grad = w.clone().requires_grad_()
-    linear(_rand(5, 64, seed=2).to(dev), grad).sum().backward()
-    assert grad.grad is not None
-    half = w.float()
-    assert linear(_rand(5, 64, seed=2).float().to(dev), half).dtype == torch.float32
+    linear(x, grad).sum().backward()
+    assert grad.grad is not None and not few_rows_calls()
+    with torch.no_grad():
+        linear(x, grad)
+    assert few_rows_calls()
+    assert linear(x.float(), w.float()).dtype == torch.float32 and not few_rows_calls()
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert linear(x, w).dtype == torch.float16 and not few_rows_calls()
+
+
+def test_products_of_few_rows_keep_tangents(dev, few_rows_calls):
+    import torch.autograd.forward_ad as fwd
+    from zipage_amd.layers import linear
+    x, t, w = (_rand(*s, seed=i, dtype=torch.float16).to(dev) / 8 for i, s in enumerate([(5, 64), (5, 64), (96, 64)]))
+    with fwd.dual_level():
+        got = fwd.unpack_dual(linear(fwd.make_dual(x, t), w)).tangent
+    assert torch.equal(got, torch.nn.functional.linear(t, w)) and not few_rows_calls()
 
 
 # ------------------------------------------------------------------ recurrences over runs, in pieces

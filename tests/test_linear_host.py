@@ -1,0 +1,83 @@
+"""Which calls of `linear` may pass torch's dispatcher by: those that nothing else looks at."""
+import pytest
+import torch
+import torch.autograd.forward_ad as fwd
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.overrides import TorchFunctionMode
+
+from zipage_amd.layers import linear
+from zipage_amd.layers.linear import ResidualLinear, _seen_by_others
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+class _Mode(TorchFunctionMode):
+    def __torch_function__(self, func, types, args=(), kwargs=None):
+        return func(*args, **(kwargs or {}))
+
+
+def _under_vmap(x, w, look):
+    torch.func.vmap(lambda a: (look(a, w), a)[1])(x.expand(2, -1, -1))
+
+
+def _under_jvp(x, w, look):
+    torch.func.jvp(lambda a: (look(a, w), a)[1], (x,), (x,))
+
+
+def _under_dual(x, w, look):
+    with fwd.dual_level():
+        look(fwd.make_dual(x, x), w)
+
+
+def _under_grad(x, w, look):
+    look(x, w.clone().requires_grad_())
+
+
+def _under_autocast(x, w, look):
+    torch.set_autocast_enabled("cuda", True)                  # torch.autocast asks for a device that is there
+    try:
+        look(x, w)
+    finally:
+        torch.set_autocast_enabled("cuda", False)
+
+
+def _under_fx(x, w, look):
+    make_fx(lambda a: (look(a, w), a + 1)[1])(x)
+
+
+def _under_jit(x, w, look):
+    torch.jit.trace(lambda a: (look(a, w), a + 1)[1], x, check_trace=False)
+
+
+def _under_fake(x, w, look):
+    with FakeTensorMode() as m:
+        look(m.from_tensor(x), m.from_tensor(w))
+
+
+def _as_subclass(x, w, look):
+    look(x.as_subclass(_Sub), w)
+
+
+def _under_mode(x, w, look):
+    with _Mode():
+        look(x, w)
+
+
+@pytest.mark.filterwarnings("ignore")
+@pytest.mark.parametrize("under", [_under_vmap, _under_jvp, _under_dual, _under_grad, _under_autocast, _under_fx, _under_jit, _under_fake, _as_subclass,
+                                   _under_mode])
+def test_calls_that_others_look_at(under):
+    x, w, seen = torch.randn(5, 64), torch.randn(96, 64), []
+    under(x, w, lambda a, b: seen.append(_seen_by_others(a, b)))
+    assert seen == [True]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_device_tensors_without_storage(dtype):
+    with FakeTensorMode():
+        x, w = torch.empty(5, 64, dtype=dtype, device="cuda"), torch.empty(96, 64, dtype=dtype, device="cuda")
+        assert linear(x, w).shape == (5, 96)
+        assert ResidualLinear(w).forward(x).shape == (1, 5, 96)

@@ -3,8 +3,11 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from zipage_amd import _lib
+
+_TENSORS = (torch.Tensor, torch.nn.Parameter)
 
 
 def pad_to_multiple(n: int, to: int) -> int:
@@ -25,10 +28,22 @@ def _few_rows(n: int, k: int, m: int) -> bool:
     return (n <= 32 or n <= 64 and m * k <= 1 << 23) and n > 0 and k % 32 == 0 and m % 4 == 0 and 0 < k <= 1 << 23
 
 
+def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether something beside the product looks at the call, which only the library's passes through torch's dispatcher:
+    gradients of either mode, vmap and its like, autocast, modes, subclasses, tracing and compilation; or another device than the current
+    one is meant."""
+    return (type(x) not in _TENSORS or type(w) not in _TENSORS
+            or torch.is_grad_enabled() and (x.requires_grad or w.requires_grad) or forward_ad._current_level >= 0
+            or torch._C._functorch.peek_interpreter_stack() is not None or torch.is_autocast_enabled("cuda")
+            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
+            or x.device.index != torch._C._cuda_getDevice())
+
+
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) without a bias."""
-    if x.is_cuda and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == w.dtype and w.dim() == 2 and \
-            not (torch.is_grad_enabled() and (x.requires_grad or w.requires_grad)):
+    if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == w.dtype \
+            and w.dim() == 2 and x.layout == w.layout == torch.strided:
         (n, k), m, stride = x.shape, w.shape[0], x.stride(0)
         if _few_rows(n, k, m) and w.shape[1] == k and x.stride(1) == 1 and k <= stride <= 1 << 23 and stride % 8 == 0 and \
                 w.is_contiguous() and w.device == x.device and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
