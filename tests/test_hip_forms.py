@@ -662,3 +662,27 @@ def test_decoded_states_past_the_cache(dev, mixer):
     close = lambda x, y: float((x - y).norm()) <= (0.0 if mixer == "linear" else 2.0 ** -7) * float(x.norm())
     # linear: the same sums.  The delta rule's low-rank products are the library's, which may round other row counts otherwise
     assert close(a, b) and all(close(x, y) for x, y in zip(sa, sb)) and a.any()
+
+
+# ------------------------------------------------------------------ products of a step
+@pytest.mark.parametrize("model", ["kapolorn", "mefupel", "pedivik", "rutevik"])
+def test_prompts_keep_the_librarys_products(dev, few_rows_calls, tmp_path, model):
+    """Portions of prompts, attended as runs or token by token, and a portion beside a decoded token: none of their products is one of few
+    rows, as none of a whole prompt is; those of decoded tokens alone are."""
+    import importlib
+    import json
+    from zipage_amd.engine import EngineConfig, ZipageEngine, read_shape
+    from zipage_amd.engine.weights import write_safetensors
+    C = importlib.import_module(f"tests.{model}_cases")
+    cfg, w = C.case("wide" if "wide" in C.CONFIGS else sorted(C.CONFIGS)[0])
+    (tmp_path / "config.json").write_text(json.dumps(cfg))
+    write_safetensors(str(tmp_path / "model.safetensors"), w)
+    eng = ZipageEngine(EngineConfig(shape=read_shape(str(tmp_path)), model_folder=str(tmp_path), dtype=BF16, num_kvcache_blocks=64,
+                                    kvcache_block_size=16, max_concurrency=6, use_graph=False))
+    toks = C.tokens(cfg, 60, 1)
+    a, b = eng.open_request(), eng.open_request()
+    for step in ([(a, toks[:24], [])], [(a, toks[24:29], [])], [(a, toks[29:30], []), (b, toks[:20], [])]):
+        eng.feed(step)
+        assert not few_rows_calls(), [len(t) for _, t, _ in step]
+    eng.feed([(a, toks[30:31], []), (b, toks[20:21], [])])
+    assert few_rows_calls()

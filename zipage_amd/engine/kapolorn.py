@@ -13,7 +13,7 @@ from dataclasses import dataclass
 import torch
 
 from zipage_amd.layers.grouped import GroupedAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple, step_product
 from zipage_amd.layers.moe import Experts
 from zipage_amd.layers.recurrent import ChannelDelta, MatrixMemory
 from zipage_amd.layers.residual import embed_norm, residual_norm, softcap
@@ -289,15 +289,15 @@ class Kapolorn:
         after every layer run."""
         s, W, N = self.shape, self.padded_width, input_ids.shape[0]
         positions = positions.to(torch.int32)
-        order = s.order
+        order, product = s.order, step_product(ctx)
         x = torch.empty((N, W), dtype=torch.float32, device=self.device)
         norms = [self.layers[i]["norm1"] for i in order] + [self.final_norm]
         h = embed_norm(input_ids, positions, self.embed, None, x, norms[0], s.eps, s.width, embed_scale=s.embed_scale)
         for run, i in enumerate(order):
             p, mixer, mlp = self.layers[i], self.mixers[i], self.mlps[i]
             mixed = torch.empty((N, mixer.out_columns), dtype=self.dtype, device=self.device)
-            mixer.mix(h, linear(h, p["into"]), positions, self.caches[run], ctx, mixed)
-            y, w = p["out"].forward(mixed), p["norm1b"]
+            mixer.mix(h, product(h, p["into"]), positions, self.caches[run], ctx, mixed)
+            y, w = p["out"].forward(mixed, product), p["norm1b"]
             if mlp is not None:
                 h = residual_norm(x, y, p["norm2"], s.eps, s.width, x_out=x, y_weight=w)
                 y, w = mlp.forward(h), p["norm2b"]

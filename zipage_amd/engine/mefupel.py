@@ -15,7 +15,7 @@ from dataclasses import dataclass
 import torch
 
 from zipage_amd.layers.grouped import GroupedAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple, step_product
 from zipage_amd.layers.recurrent import LinearAttention
 from zipage_amd.layers.residual import embed_norm, normed_powers, residual_norm
 from zipage_amd.layers.rotary import Rotary
@@ -257,12 +257,13 @@ class Layer:
 
     def forward(self, h: torch.Tensor, positions: torch.Tensor, cache, ctx) -> list:
         """The branches that join the stream, with the weights of their norms."""
-        proj = linear(h, self.into)
+        product = step_product(ctx)
+        proj = product(h, self.into)
         rows = [torch.empty((h.shape[0], o.w.shape[1]), dtype=h.dtype, device=h.device) for o in self.outs]
         self.mixer.mix(proj[:, :self.mixed], positions, cache, ctx, [r[:, :n] for r, n in zip(rows, self.spans)])
         if self.ff is not None:
             normed_powers(proj[:, self.mixed:], self.act, self.eps, self.ff, rows[-1][:, self.spans[-1]:])
-        return [(o.forward(r), n) for o, r, n in zip(self.outs, rows, self.norms)]
+        return [(o.forward(r, product), n) for o, r, n in zip(self.outs, rows, self.norms)]
 
 
 class Mefupel:

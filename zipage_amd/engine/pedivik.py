@@ -15,7 +15,7 @@ from dataclasses import dataclass
 import torch
 
 from zipage_amd.layers.latent import LatentAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, linear
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, step_product
 from zipage_amd.layers.residual import embed_norm, residual_norm, xielu
 
 
@@ -169,7 +169,7 @@ class Pedivik:
         """Normed and scaled output rows (N, padded width) for compute_logits.  `trace`, when given,
         receives the stream after every layer."""
         s, W = self.shape, self.padded_width
-        N, L = input_ids.shape[0], len(self.layers)
+        N, L, product = input_ids.shape[0], len(self.layers), step_product(ctx)
         # plane j holds the embedding output (0) or the result of layer j - 1
         history = torch.empty((L + 1, N, W), dtype=torch.float32, device=self.device)
         x = history[0]
@@ -183,7 +183,7 @@ class Pedivik:
             y = mixer.forward(h, self.caches[i], ctx)
             if "up" in p:
                 h = residual_norm(x, y, p["norm2"], s.eps, s.width, weight_offset=1.0, x_out=inner)
-                x, y = inner, p["down"].forward(xielu(linear(h, p["up"]), *p["act"]))
+                x, y = inner, p["down"].forward(xielu(product(h, p["up"]), *p["act"]), product)
             h = residual_norm(x, y, norms[i + 1], s.eps, s.width, weight_offset=1.0, out_scale=scales[i + 1],
                               x_out=after, result=history[i + 1], history=history, mix=p["dwa"])
             x = after

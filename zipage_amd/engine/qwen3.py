@@ -15,7 +15,7 @@ import torch.nn.functional as F
 
 from zipage_amd.kernel import store_query_cache
 from zipage_amd.layers import (causal_attention, gather_rows, linear, paged_decode_attention, qk_norm_rope_store, rms_norm,
-                               silu_and_mul)
+                               silu_and_mul, step_product)
 
 from .inputs import plan_prompts
 
@@ -120,12 +120,6 @@ class Qwen3:
         self.k_cache, self.v_cache, self.q_cache = kv_cache[0], kv_cache[1], query_cache
 
     # ------------------------------------------------------------------ pieces
-    @staticmethod
-    def _product(ctx: StepContext):
-        """Decode steps have few rows.  What a prefix cache leaves of a prompt may be few as well, and keeps the products of
-        whole prompts, so that both round alike."""
-        return F.linear if ctx.is_prefill else linear
-
     def _plan_prefill(self, ctx: StepContext):
         """Query tiles of a step of prompts, and the cache rows of the prompts with a cached prefix, whose whole contexts are
         read back: they come first among the keys, the step's own rows, which the other prompts attend, behind them (None
@@ -189,7 +183,7 @@ class Qwen3:
         """zipage/models/qwen3.py:72-88 + zipage/layers/attention.py:69-104."""
         s = self.shape
         N = x.shape[0]
-        product = self._product(ctx)
+        product = step_product(ctx)
         qkv = product(x, p["wqkv"])
         q_sz, kv_sz = s.heads * s.head_dim, s.kv_heads * s.head_dim
         cached = self.k_cache is not None and self.k_cache.numel() > 0 and ctx.slot_mapping is not None
@@ -221,7 +215,7 @@ class Qwen3:
         pos32 = positions.to(torch.int32)
         hidden = F.embedding(input_ids, self.embed)
         resid = None
-        plan, product = self._plan_prefill(ctx), self._product(ctx)
+        plan, product = self._plan_prefill(ctx), step_product(ctx)
         for li, p in enumerate(self.layers):
             if resid is None:
                 resid, h = hidden, rms_norm(hidden, p["ln1"], s.eps)

@@ -14,7 +14,7 @@ import torch
 
 from zipage_amd.layers.grouped import GroupedAttention
 from zipage_amd.layers.latent import LatentAttention
-from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple
+from zipage_amd.layers.linear import ResidualLinear, fit, linear, pad_to_multiple, step_product
 from zipage_amd.layers.moe import Experts
 from zipage_amd.layers.residual import embed_norm, relu_square, residual_norm
 from zipage_amd.layers.rotary import Rotary
@@ -154,8 +154,9 @@ class Differential:
 
     def forward(self, h, cache, ctx, positions, held):
         mixed = torch.empty((h.shape[0], self.core.out_columns), dtype=h.dtype, device=h.device)
-        self.core.attend(linear(h, self.into), positions, cache, ctx, mixed)
-        return self.out.forward(mixed)
+        product = step_product(ctx)
+        self.core.attend(product(h, self.into), positions, cache, ctx, mixed)
+        return self.out.forward(mixed, product)
 
 
 class Dense:
@@ -176,8 +177,8 @@ class Dense:
         self.load({k: torch.empty(*s, dtype=dtype, device=device).normal_(0.0, std, generator=generator)
                    for k, s in self.shapes().items()}, dtype, device)
 
-    def forward(self, h: torch.Tensor) -> torch.Tensor:
-        return self.down.forward(relu_square(linear(h, self.up)))
+    def forward(self, h: torch.Tensor, product=linear) -> torch.Tensor:
+        return self.down.forward(relu_square(product(h, self.up)), product)
 
 
 class Rutevik:
@@ -290,13 +291,14 @@ class Rutevik:
         # the last norm's rows leave with the logits' scale
         after = [n[0] for n in self.norms[1:]] + [dict(self.final_norm, out_scale=s.logit_scale)]
         held: list[dict] = [{} for _ in self.mixers]
+        product = step_product(ctx)
         h = embed_norm(input_ids, positions, self.embed, None, x, eps=s.eps, norm_width=s.width, **self.norms[0][0])
         for i, (mixer, mlp) in enumerate(zip(self.mixers, self.mlps)):
             j = self.source[i]
             y = mixer.forward(h, self.caches[j], ctx, positions, held[j])
             if mlp is not None:
                 h = residual_norm(x, y, eps=s.eps, norm_width=s.width, x_out=x, **self.norms[i][1])
-                y = mlp.forward(h)
+                y = mlp.forward(h, product) if isinstance(mlp, Dense) else mlp.forward(h)
             h = residual_norm(x, y, eps=s.eps, norm_width=s.width, x_out=x, **after[i])
             if trace is not None:
                 trace.append(x[:, :s.width].clone())

@@ -9,7 +9,7 @@ import torch.nn.functional as F
 
 from zipage_amd import _lib
 
-from .linear import ResidualLinear, fit, linear, pad_to_multiple
+from .linear import ResidualLinear, fit, pad_to_multiple, step_product
 from .rotary import Rotary
 from .runs import gather_rows, run_attention
 
@@ -202,7 +202,8 @@ class LatentAttention:
         singles = ctx.context_lens.numel()
         runs = ctx.runs[self.window] if singles < N else None
         direct = runs is not None and runs.key_slots is None    # the runs' keys are this step's own tokens
-        down = linear(h, self.down)
+        product = step_product(ctx)
+        down = product(h, self.down)
         if self.own_latent:
             norms = latent_norm_store(down, self.q_norm, self.c_norm, self.q_rank, self.kv_rank, self.eps, cache,
                                       ctx.slot_mapping, direct, positions, self.freqs)
@@ -211,7 +212,7 @@ class LatentAttention:
                 held["rows"] = norms[1][singles:] if direct else gather_rows(cache, runs.key_slots)
         else:
             cq = latent_norm_store(down, self.q_norm, None, self.q_rank, 0, self.eps, None, None)
-        q = linear(cq, self.uq)
+        q = product(cq, self.uq)
         mixed = torch.empty((N, H * self.vdim_p), dtype=h.dtype, device=h.device)
         if runs is not None:
             rows, qr, shared = held["rows"], q[singles:], None
@@ -226,4 +227,4 @@ class LatentAttention:
             ol = latent_rows_attention(ql, cache, ctx.block_tables, ctx.context_lens, self.scale, self.window,
                                        ctx.table_rows, self.kv_rank_p)
             headwise_linear(ol, self.uv, mixed[:singles])
-        return self.o.forward(mixed)
+        return self.o.forward(mixed, product)

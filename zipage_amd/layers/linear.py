@@ -54,6 +54,15 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return F.linear(x, w)
 
 
+def step_product(ctx):
+    """What a step's layers multiply with: `linear` where every sequence has one token.  What a step holds of a prompt may be few rows as
+    well, and keeps the library's products, as the same rows of a whole prompt do, so that both round alike."""
+    segments = getattr(ctx, "segments", None)
+    prompts = getattr(ctx, "is_prefill", False) or getattr(ctx, "runs", None) or getattr(ctx, "run_segments", None) is not None or \
+        segments is not None and segments.max_count != 1
+    return F.linear if prompts else linear
+
+
 class ResidualLinear:
     """y = W x, returned as planes of partial sums (planes, N, out) that `residual_norm` adds up in
     fp32.
@@ -74,9 +83,10 @@ class ResidualLinear:
         if w.dtype == torch.bfloat16 and inn >= self.MIN_CONTRACTION and inn % (8 * self.PARTS) == 0:
             self.parts = w.t().contiguous().view(self.PARTS, inn // self.PARTS, out)
 
-    def forward(self, x: torch.Tensor) -> torch.Tensor:
+    def forward(self, x: torch.Tensor, product=linear) -> torch.Tensor:
+        """`product`: see `step_product`."""
         N = x.shape[0]
         if self.parts is None or N > self.SPLIT_ROWS:
-            return linear(x, self.w).unsqueeze(0)
+            return product(x, self.w).unsqueeze(0)
         P, k, _ = self.parts.shape
         return torch.bmm(x.view(N, P, k).transpose(0, 1), self.parts)

@@ -9,7 +9,7 @@ import torch
 
 from zipage_amd import _lib
 
-from .linear import fit, linear, pad_to_multiple
+from .linear import fit, pad_to_multiple, step_product
 from .moe import small_linear
 from .rotary import Rotary
 
@@ -167,7 +167,7 @@ class ChannelDelta:
         S, tail = state
         H, D = self.heads, self.dim_p
         assert proj.stride(1) == out.stride(1) == 1 and proj.dtype == out.dtype == tail.dtype and S.is_contiguous()
-        low = linear(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
+        low = step_product(ctx)(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
         tag, stream = _lib.dtype_tag(proj), _lib.stream_ptr(proj)
         for segments, runs in ((ctx.segments, False), (ctx.run_segments, self.can_run and proj.dtype == torch.bfloat16)):
             if segments is None:
@@ -250,7 +250,7 @@ class LinearAttention:
         """proj: this mixer's columns of the projections, out: of the output rows."""
         H, D, V = self.heads, self.dim_p, self.vdim_p
         assert proj.stride(1) == out.stride(1) == 1 and proj.dtype == out.dtype and state.is_contiguous()
-        low = None if self.low is None else linear(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
+        low = None if self.low is None else step_product(ctx)(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
         tag, stream = _lib.dtype_tag(proj), _lib.stream_ptr(proj)
         for segments, runs in ((ctx.segments, False), (ctx.run_segments, self.can_run and proj.dtype == torch.bfloat16)):
             if segments is None:
