@@ -274,7 +274,7 @@ def test_causal_attention(dev, H, G, D, lens=((1, 1), (31, 31), (128, 128), (129
 # the ring; outputs that end inside a tile; rows of x further apart than they are long
 @pytest.mark.parametrize("dtype", [BF16, torch.float16])
 @pytest.mark.parametrize("n", [1, 16, 17, 32, 33, 64])
-@pytest.mark.parametrize("K,M", [(32, 4), (96, 20), (128, 4096), (1056, 4100), (1312, 68), (2048, 4128), (160, 16388), (2176, 16400)])
+@pytest.mark.parametrize("K,M", [(32, 4), (96, 20), (128, 4096), (1056, 4100), (1312, 68), (2048, 4128), (160, 16388), (2176, 16400), (1984, 8196)])
 def test_products_of_few_rows(dev, dtype, n, K, M):
     from zipage_amd import _lib
     wide = _rand(n, K + 24, seed=1, dtype=dtype).to(dev)

@@ -81,3 +81,16 @@ def test_device_tensors_without_storage(dtype):
         x, w = torch.empty(5, 64, dtype=dtype, device="cuda"), torch.empty(96, 64, dtype=dtype, device="cuda")
         assert linear(x, w).shape == (5, 96)
         assert ResidualLinear(w).forward(x).shape == (1, 5, 96)
+
+
+# on either side of the lines that measuring drew, with weights from memory
+@pytest.mark.parametrize("n,k,m,few", [(1, 1024, 4096, True), (16, 4096, 4096, True), (8, 12288, 4096, True), (8, 12288, 1024, False), (8, 12288, 9216, False),
+                                       (8, 8192, 4096, False), (16, 128, 32768, False), (16, 256, 32768, True), (8, 1024, 65536, False),
+                                       (8, 2048, 151936, True), (17, 4096, 4096, True), (17, 4096, 6144, False), (32, 4096, 24576, False),
+                                       (24, 1024, 16384, True), (24, 1024, 20480, False), (24, 2048, 8192, True), (24, 2048, 9216, False),
+                                       (32, 64, 5120, False), (48, 1024, 4096, True), (48, 3072, 1024, True), (48, 3072, 2048, False),
+                                       (48, 3072, 256, False), (48, 64, 8192, False), (64, 1024, 16384, False), (65, 1024, 1024, False),
+                                       (0, 64, 64, False), (4, 48, 64, False), (4, 64, 66, False)])
+def test_which_sizes_are_few_rows(n, k, m, few):
+    from zipage_amd.layers.linear import _few_rows
+    assert _few_rows(n, k, m) == few

@@ -23,10 +23,9 @@ struct FewArgs {
 // 128 elements of every row, a step of 32 for each wave: loads of whole cache lines, for the L1 takes four to five cycles for
 // every line touched, whole or in part.  A row's sixteen pieces lie in the order of (piece ^ row).  Bound by the weights'
 // stream: what counts is bytes in flight, so the ring takes what LDS there is, for two workgroups where the tiles are small.
-// 1 to 31 rows, weights from memory, us (the library, which costs 18 us of host time a call, 5 here): 1024 -> 4096 4.2 to 4.9
-// (7.5 to 11.2), 2048 -> 1024 5.2 to 6.1 (8.1), 3072 -> 1024 6.5 to 7.8 (9.5), 4096 -> 4096 9.5 to 10.8 (15.8 to 13.4), 4096 ->
-// 6144 12.8 to 14.4 (16.1 to 15.7), 4096 -> 24 576 45.7 to 48.3 (47.8 to 48.8), 12 288 -> 4096 21.4 to 26.9 (23.1 to 26.8);
-// errors the same.  48 rows: 1024 -> 4096 6.5 (11.1), 3072 -> 1024 11.0 (10.7), but 4096 -> 6144 27.2 (17.7).
+// Weights from memory, us (the library): 16 rows, 1024 -> 4096 4.4 (7.6), 2048 -> 1024 5.5 (11.0), 3072 -> 1024 6.7 (12.0), 4096
+// -> 4096 9.6 (15.8), 4096 -> 24 576 45 (46), 12 288 -> 4096 22.5 (22.7); 32 rows, 1024 -> 4096 5.0 (11.4), 4096 -> 4096 10.9
+// (13.4); 48 rows, 1024 -> 4096 6.6 (11.4), 3072 -> 1024 11.2 (11.7); errors the same.  The caller's rule has where it is slower.
 template <int TT, int MT> struct FewTile {
   static constexpr int kLoads = TT + MT, kBytes = kLoads * 4096;       // of a wave; of a stage
   static constexpr int kRing = kLoads <= 2 ? 9 : kLoads == 3 ? 6 : kLoads == 4 ? 9 : kLoads == 5 ? 7 : 6;
@@ -126,12 +125,13 @@ template <typename T, int TT, int MT> int launch_few(const FewArgs& a, hipStream
 }
 // Rows of W per workgroup: 16 where that makes at most a workgroup per CU, else 32, since each workgroup reads all of x (16
 // rows of x, us with 16, 32 and 64 rows of W: 1024 -> 4096 4.4, 4.8, 6.8; 4096 -> 4096 9.7, 11.0, 16.0; 1024 -> 6144 6.2, 5.2,
-// 7.1; 4096 -> 24 576 46.3, 45.2, 52.9).  64 where many short ones would spend their time on beginning (31 rows, 1024 -> 32 768:
-// 23.9, 21.7, 17.9).
+// 7.1; 4096 -> 24 576 46.3, 45.2, 52.9).  64 where more rows of x leave one workgroup's ring on a CU and that makes one round of
+// what were two, with contractions short enough to be bound by the beginning of a workgroup (24 rows, us with 32 and 64 rows of
+// W: 128 -> 12 288 6.2, 4.4; 512 -> 9216 8.4, 6.3; 1024 -> 12 288 11.6, 9.0; 1536 -> 14 336 15.0, 12.6).
 template <typename T, int TT> int launch_few(const FewArgs& a, hipStream_t st) {
   if (a.M <= 4096) return launch_few<T, TT, 1>(a, st);
   if constexpr (TT == 2)
-    if (a.M >= 16384 && a.K < 2048) return launch_few<T, 2, 4>(a, st);
+    if (a.M > 8192 && a.K < 2048) return launch_few<T, 2, 4>(a, st);
   return launch_few<T, TT, 2>(a, st);
 }
 template <typename T> int launch_few(const FewArgs& a, hipStream_t st) {

@@ -22,10 +22,26 @@ def fit(t: torch.Tensor, *shape: int) -> torch.Tensor:
 
 
 def _few_rows(n: int, k: int, m: int) -> bool:
-    """Whether a product of n rows of k elements and (m, k) weights goes to the kernel for few rows.  Up to 32 rows it is as
-    fast as the library on the GPU or faster (csrc/few_rows.hip has both), and costs a quarter of the host's time; up to 64
-    where the weights are few, since each workgroup reads all of x."""
-    return (n <= 32 or n <= 64 and m * k <= 1 << 23) and n > 0 and k % 32 == 0 and m % 4 == 0 and 0 < k <= 1 << 23
+    """Whether a product of n rows of k elements and (m, k) weights goes to the kernel for few rows: where that is no slower on the GPU, with
+    weights from memory (us of both, the library second; a call of the library costs 18 us of host time, of the kernel 8).
+
+    Up to 16 rows: nearly everywhere (8 rows, 1024 -> 4096 4.3 and 7.7, 4096 -> 4096 9.1 and 15.8, 2048 -> 151 936 121 and 212).
+    Long contractions need outputs that fill one round of workgroups (12 288 -> 4096 21.6 and 22.5, but -> 1024 18.6 and 17.0,
+    -> 9216 59 and 50), and rows that are not a multiple of 16 KB apart (8192 -> 4096 17.2 and 16.2); many outputs a
+    contraction that is worth a workgroup's beginning (128 -> 32 768 6.6 and 6.2, 1024 -> 65 536 29 and 27.5).
+    Up to 32: as far as one round of workgroups goes (24 rows, 1024 -> 16 384 9.5 and 13.0, -> 20 480 15.1 and 14.4; 2048
+    -> 8192 11.2 and 14.6, -> 9216 17.0 and 14.1; 4096 -> 4096 10.4 and 13.6, -> 6144 16.5 and 15.4).
+    Up to 64, since each workgroup reads all rows: 48 rows, 1024 -> 4096 6.6 and 11.3, 3072 -> 1024 11.3 and 11.7, but -> 2048
+    11.4 and 10.3, -> 256 10.6 and 9.3; 64 -> 8192 4.0 and 3.8."""
+    if n <= 0 or k <= 0 or k % 32 or m % 4 or k > 1 << 23:
+        return False
+    if n <= 16:
+        if k > 4096:
+            return (1024 if k <= 6144 else 4096) <= m <= 8192 and k % 8192 != 0
+        return m <= 16384 or k >= (192 if m <= 32768 else 2048)
+    if n <= 32:
+        return k <= 4608 if m <= 4096 else 128 <= k and (k <= 2048 and m <= 8192 or k < 2048 and m <= 16384)
+    return n <= 64 and m * k <= 1 << 23 and m <= 8192 and (96 <= k <= 1024 or 512 <= m and 1024 < k <= 2048 or 512 <= m <= 1280 and 2048 < k <= 4096)
 
 
 def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
