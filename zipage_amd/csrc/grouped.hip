@@ -246,8 +246,7 @@ __device__ __forceinline__ int first_key(const RowsArgs& a, int n) {   // n toke
 // operands by v_perm.  The next step's keys are requested once the scores are done, its values once the
 // value products are.  PAST: values, of which a load reads whole lines, pass the last-level cache by; keys, read as operands in
 // parts of lines, don't (256 sequences, 32 heads over 8 of 128: 393 us, values past it 363, both 386).
-template <int DKS, int VCB, int MAPS, bool PAST>
-__global__ __launch_bounds__(256, 2) void grouped_rows_kernel(RowsArgs a) {
+template <int DKS, int VCB, int MAPS, bool PAST> __device__ __forceinline__ void grouped_rows(const RowsArgs& a) {
   extern __shared__ __align__(16) char lds_raw[];
   int* const pg = (int*)lds_raw;
   float* const merge = (float*)(lds_raw + ((a.lds_pages * 4 + 15) & ~15));
@@ -457,6 +456,20 @@ __global__ __launch_bounds__(256, 2) void grouped_rows_kernel(RowsArgs a) {
   }
 }
 
+// Whether values go past the last-level cache.  How much of their tables a call's tokens use is known here alone: a workgroup takes all
+// of them to see as many keys as its own does.
+__device__ __forceinline__ bool rows_past(const RowsArgs& a, int row) {
+  const int n = min(max(a.ctx[row], 0), a.NB * a.BS);
+  return past_cache(min((int64_t)a.n * (n - first_key(a, n)), (int64_t)a.num_pages * a.BS) * a.HK * (a.D + a.V) * 2);
+}
+// MAY: they may (see may_pass)
+template <int DKS, int VCB, int MAPS, bool MAY>
+__global__ __launch_bounds__(256, 2) void grouped_rows_kernel(RowsArgs a) {
+  if constexpr (MAY)
+    if (rows_past(a, blockIdx.x / (a.splits * a.htiles * a.HK))) return grouped_rows<DKS, VCB, MAPS, true>(a);
+  grouped_rows<DKS, VCB, MAPS, false>(a);
+}
+
 __global__ __launch_bounds__(64) void grouped_combine_kernel(RowsArgs a) {
   const int64_t item = blockIdx.x;       // (row, head)
   const int h = (int)(item % a.H);
@@ -623,15 +636,15 @@ int rows_splits(int n, int H, int HK, int window, int chunk, int NB, int BS) {
   return s < 1 ? 1 : s;
 }
 
-template <int DKS, int VCB, int MAPS, bool PAST> int launch_rows(const RowsArgs& a, hipStream_t st) {
+template <int DKS, int VCB, int MAPS, bool MAY> int launch_rows(const RowsArgs& a, hipStream_t st) {
   const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + 4 * sizeof(float) * (16 * (a.V + 4) + 32);
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)grouped_rows_kernel<DKS, VCB, MAPS, PAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)grouped_rows_kernel<DKS, VCB, MAPS, MAY>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)smem) != hipSuccess) {
     zp_set_error("grouped_rows_attention: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((grouped_rows_kernel<DKS, VCB, MAPS, PAST>), dim3((unsigned)a.n * a.HK * a.htiles * a.splits), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((grouped_rows_kernel<DKS, VCB, MAPS, MAY>), dim3((unsigned)a.n * a.HK * a.htiles * a.splits), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   if (a.splits > 1) {
     if (MAPS == 2) hipLaunchKernelGGL(grouped_pair_combine_kernel, dim3((unsigned)a.n * a.H / 2), dim3(64), 0, st, a);
@@ -640,10 +653,11 @@ template <int DKS, int VCB, int MAPS, bool PAST> int launch_rows(const RowsArgs&
   }
   return ZP_OK;
 }
-// Values go past the last-level cache where one workgroup reads them, in whole lines, and all rows that may be read do not
+// Values may go past the last-level cache where one workgroup reads them, in whole lines, and all rows that may be read do not
 // fit: 40 sequences of about 2050 tokens, 32 heads over 8 of 128 89 us and 80, 256 of them 393 and 363, heads of 64 over 4
-// 112 and 96, 256 of 100 to 4096 tokens 456 and 428.
-bool rows_past(const RowsArgs& a) {
+// 112 and 96, 256 of 100 to 4096 tokens 456 and 428.  Where the tables hold more than the contexts, workgroups ask themselves (64
+// sequences of 700 tokens in tables of 10 240, heads of 128 over 8: 33 us through it, 35 past it, now 33).
+bool may_pass(const RowsArgs& a) {
   int64_t keys = (int64_t)a.NB * a.BS;
   if (a.window > 0) keys = std::min<int64_t>(keys, a.window);
   if (a.chunk > 0) keys = std::min<int64_t>(keys, a.chunk);
@@ -651,7 +665,7 @@ bool rows_past(const RowsArgs& a) {
          past_cache(std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * a.HK * (a.D + a.V) * 2);
 }
 template <int DKS, int VCB, int MAPS> int launch_rows(const RowsArgs& a, hipStream_t st) {
-  return rows_past(a) ? launch_rows<DKS, VCB, MAPS, true>(a, st) : launch_rows<DKS, VCB, MAPS, false>(a, st);
+  return may_pass(a) ? launch_rows<DKS, VCB, MAPS, true>(a, st) : launch_rows<DKS, VCB, MAPS, false>(a, st);
 }
 template <int MAPS> int dispatch_rows(const RowsArgs& a, hipStream_t st) {
   const int dk = (a.D + 31) / 32;

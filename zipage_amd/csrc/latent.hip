@@ -379,8 +379,7 @@ template <int NCB, int PK> struct RowsLds {
 };
 __host__ __device__ inline int rows_merge_floats(int R) { return 16 * (R + 4) + 32; }   // per wave
 
-template <int NCB, int HT, int PK, bool PAST>
-__global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kernel(RowsArgs a) {
+template <int NCB, int HT, int PK, bool PAST> __device__ __forceinline__ void latent_narrow(const RowsArgs& a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef RowsLds<NCB, PK> Lds;
   int* pg = (int*)lds_raw;
@@ -636,6 +635,21 @@ __global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kern
       else Vec8<F32>::st(a.part, (item * a.splits + split) * a.R + c, r);
     }
   }
+}
+
+// Whether rows are asked for past the last-level cache.  How much of their tables a call's tokens use is known here alone: a workgroup
+// takes all of them to see as many keys as its own does.  (May be and is not: 0.1 to 0.3 us.)
+__device__ __forceinline__ bool rows_past(const RowsArgs& a, int row) {
+  int keys = min(max(a.ctx[row], 0), a.NB * a.BS);
+  if (a.window > 0) keys = min(keys, a.window);
+  return past_cache(min((int64_t)a.n * keys, (int64_t)a.num_pages * a.BS) * (a.R + a.P) * 2);
+}
+// MAY: it may be (see may_pass)
+template <int NCB, int HT, int PK, bool MAY>
+__global__ __launch_bounds__(256, NCB * HT <= 2 ? 2 : 1) void latent_narrow_kernel(RowsArgs a) {
+  if constexpr (MAY)
+    if (rows_past(a, blockIdx.x / a.splits)) return latent_narrow<NCB, HT, PK, true>(a);
+  latent_narrow<NCB, HT, PK, false>(a);
 }
 
 // NCB column blocks of 128 cover R; PK steps of 32 the rotated part, which is a key only, never a value.  Workgroup: one
@@ -1041,31 +1055,34 @@ int launch_combine(const RowsArgs& a, hipStream_t st) {
   }
   return ZP_OK;
 }
-// Whether rows are asked for past the last-level cache: one workgroup reads a key, in whole lines, and all that may be read do
+// Whether rows may be asked for past the last-level cache: one workgroup reads a key, in whole lines, and all that may be read do
 // not fit.  256 sequences of 1800 to 2304 tokens: rows of 576, 16 heads 115 us through it and 103 past it, 32 heads 122 and
 // 115, 64 heads 181 and 176; rows of 320, 32 heads 78 and 73, 16 heads 71 and 65.  With two workgroups on a token (128
-// heads) 324 and 338; where rows fit, 40 sequences, 42 and 43; rows of 192, 200 MB, 42 and 47.
-bool rows_past(const RowsArgs& a, int hgroups) {
+// heads) 324 and 338; where rows fit, 40 sequences, 42 and 43; rows of 192, 200 MB, 42 and 47.  What may be read is as much as the
+// tables hold.  Where contexts are shorter, the narrow kernel asks itself (rows of 320, 16 heads, 256 sequences of 1000 tokens
+// in tables of 4096: 34 us through it, 37 past it, now 34.5); the other one goes past it all the same (rows of 576, 32
+// heads, 700 tokens 47 us for 44; with both forms in one kernel 64 heads took 2 % longer wherever they are).
+bool may_pass(const RowsArgs& a, int hgroups) {
   const int64_t keys = a.window > 0 ? std::min<int64_t>(a.window, (int64_t)a.NB * a.BS) : (int64_t)a.NB * a.BS;
   return hgroups == 1 && (a.R + a.P) % 64 == 0 &&
          past_cache(std::min(a.n * keys, (int64_t)a.num_pages * a.BS) * (a.R + a.P) * 2);
 }
-template <int NCB, int HT, int PK, bool PAST> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
+template <int NCB, int HT, int PK, bool MAY> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
   const size_t merge = 4 * sizeof(float) * (size_t)rows_merge_floats(a.R);
   const size_t work = 4 * RowsLds<NCB, PK>::kStage + (size_t)HT * RowsLds<NCB, PK>::kQ;
   const size_t smem = (((size_t)a.lds_pages * 4 + 15) & ~(size_t)15) + (merge > work ? merge : work);
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)latent_narrow_kernel<NCB, HT, PK, PAST>, hipFuncAttributeMaxDynamicSharedMemorySize,
+      hipFuncSetAttribute((const void*)latent_narrow_kernel<NCB, HT, PK, MAY>, hipFuncAttributeMaxDynamicSharedMemorySize,
                           (int)smem) != hipSuccess) {
     zp_set_error("latent_rows_attention: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((latent_narrow_kernel<NCB, HT, PK, PAST>), dim3((unsigned)a.n * a.splits), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((latent_narrow_kernel<NCB, HT, PK, MAY>), dim3((unsigned)a.n * a.splits), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return launch_combine(a, st);
 }
 template <int NCB, int HT, int PK> int launch_latent_narrow(const RowsArgs& a, hipStream_t st) {
-  return rows_past(a, 1) ? launch_latent_narrow<NCB, HT, PK, true>(a, st) : launch_latent_narrow<NCB, HT, PK, false>(a, st);
+  return may_pass(a, 1) ? launch_latent_narrow<NCB, HT, PK, true>(a, st) : launch_latent_narrow<NCB, HT, PK, false>(a, st);
 }
 template <int NCB, int HW, int PK, bool PAST> int launch_latent_rows(const RowsArgs& a, int hgroups, hipStream_t st) {
   constexpr int smem = RowsStage<NCB, PK>::kBytes + (HW < 4 ? 4096 : 0);
@@ -1082,7 +1099,7 @@ template <int NCB, int HW, int PK, bool PAST> int launch_latent_rows(const RowsA
 }
 template <int NCB, int HW, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {
   const int hgroups = (a.H + 16 * HW - 1) / (16 * HW);
-  return rows_past(a, hgroups) ? launch_latent_rows<NCB, HW, PK, true>(a, hgroups, st)
+  return may_pass(a, hgroups) ? launch_latent_rows<NCB, HW, PK, true>(a, hgroups, st)
                                : launch_latent_rows<NCB, HW, PK, false>(a, hgroups, st);
 }
 template <int NCB, int PK> int launch_latent_rows(const RowsArgs& a, hipStream_t st) {

@@ -43,7 +43,7 @@ template <bool PAST> __device__ __forceinline__ u32x4 load_piece(const void* p) 
   if constexpr (PAST) return __builtin_nontemporal_load((const u32x4*)p);
   return *(const u32x4*)p;
 }
-inline bool past_cache(int64_t bytes) { return bytes >= 320ll << 20; }
+__host__ __device__ inline bool past_cache(int64_t bytes) { return bytes >= 320ll << 20; }
 template <bool PAST = false>
 __device__ __forceinline__ void load_to_lds(const u32x4& rows, void* lds, int lane_at, int at) {
   const uint32_t to = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(uintptr_t)(lds_ptr_t)lds);
