@@ -219,9 +219,9 @@ typedef struct {
 int zp_mlstm_scan(const zp_mlstm* args, int32_t dtype, void* stream);
 /* The same for long runs, 16 tokens at a time on the matrix cores (fp32): bfloat16, dk 32, 64 or 128, dv up
  * to 128, rows given in rising order from first_row on, none longer than `longest`.  `workspace`:
- * zp_mlstm_runs_workspace() bytes for the rows from first_row to the end.  Of those, up to 128 (run, head) pairs have room
- * for states between pieces of runs, which are then worked on side by side; without it (the first ((rows / 16 + segments)
- * * 512 + rows * 4) * heads * 4 bytes are needed) runs stay whole. */
+ * zp_mlstm_runs_workspace() bytes for the rows from first_row to the end.  Of those, up to 128 (run, head) pairs of more than
+ * 192 rows have room for states between pieces of runs, which are then worked on side by side; without it (the first ((rows
+ * / 16 + segments) * 512 + rows * 4) * heads * 4 bytes are needed) runs stay whole. */
 int64_t zp_mlstm_runs_workspace(int32_t rows, int32_t segments, int32_t heads);
 int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t longest, void* workspace,
                   int64_t workspace_bytes, int32_t dtype, void* stream);

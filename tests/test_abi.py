@@ -109,3 +109,20 @@ def test_a_workspace_for_the_largest_batch_serves_every_other():
             assert sizes == sorted(sizes)
             few = [lib.zp_compress_layers_workspace_few(1, b, 9, 256, 8, heads, window, dtype, ctypes.byref(cc), 0) for b in range(1, 70)]
             assert few[0] > sizes[0] and few[-1] == sizes[-1] and all(f >= s for f, s in zip(few, sizes))
+
+
+def test_room_for_pieces_of_runs_follows_the_rows():
+    """Blocks of 16 tokens alone where no run can be cut, as many states as rows, runs and heads can ask for beyond, and never more
+    than 384."""
+    from zipage_amd import _lib
+    recurrent, linear = _lib.load_models("recurrent"), _lib.load_models("linear")
+    for size, state in ((lambda *a: recurrent.zp_delta_runs_workspace(*a, 128, 128), 2 * 128 * 128 * 4),
+                        (lambda *a: linear.zp_linear_runs_workspace(*a, 128), (128 * 128 + 128) * 4),
+                        (lambda *a: recurrent.zp_mlstm_runs_workspace(*a), (128 * 128 + 128 + 4) * 4)):
+        blocks = lambda rows, runs, heads: size(rows, runs, 1000) // 1000 * heads        # so many heads' runs stay whole
+        for heads in (1, 8, 32, 128):
+            assert size(16, 1, heads) == blocks(16, 1, heads) and size(192, 1, heads) == blocks(192, 1, heads)
+        for rows, runs, heads in ((700, 1, 16), (1025, 3, 2), (2048, 1, 32), (16384, 8, 16)):
+            room = size(rows, runs, heads) - blocks(rows, runs, heads)
+            assert room == min(384, (rows // 64 + runs) * heads) * state
+        assert size(2048, 8, 32) == blocks(2048, 8, 32)                                   # 256 pairs

@@ -343,12 +343,14 @@ def test_products_of_few_rows_keep_tangents(dev, few_rows_calls):
 # ------------------------------------------------------------------ recurrences over runs, in pieces
 # Few heads walk long runs in pieces of at least four blocks of 16 tokens: one run, runs of which some have fewer pieces than
 # others or none, pieces whose last has one token or a whole block, states of earlier tokens and none; key and value sizes
-# apart (the delta rule stays whole there).  Token by token in fp32 the same sums stand in another order.
+# apart (the delta rule stays whole there).  The same kernels take runs whole where the workspace has room for blocks alone; token by
+# token in fp32 the same sums stand in another order.
 @pytest.mark.parametrize("kind", ["delta", "memory", "linear", "retention"])
 @pytest.mark.parametrize("H,D,V,lens", [(1, 128, 128, (700,)), (16, 128, 128, (705, 161, 64, 1377)), (2, 32, 32, (16, 1025, 31)),
                                         (24, 64, 96, (1024, 496)), (40, 64, 64, (400, 15, 401)), (128, 32, 32, (640,))])
-def test_recurrences_in_pieces(dev, kind, H, D, V, lens):
+def test_recurrences_in_pieces(dev, monkeypatch, kind, H, D, V, lens):
     import types
+    from zipage_amd import _lib
     from zipage_amd.engine.qwen3 import Segments
     from zipage_amd.layers import ChannelDelta, LinearAttention, MatrixMemory, Rotary
     W, n, rows = 64, len(lens), sum(lens)
@@ -371,7 +373,14 @@ def test_recurrences_in_pieces(dev, kind, H, D, V, lens):
     t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
     first, starts = [sum(lens[:i]) for i in range(n)], [0 if i % 2 == 0 else 333 for i in range(n)]
 
-    def scan(runs):
+    lib = _lib.load_models("recurrent" if kind in ("delta", "memory") else "linear")
+    name = {"delta": "zp_delta_runs_workspace", "memory": "zp_mlstm_runs_workspace"}.get(kind, "zp_linear_runs_workspace")
+    size = getattr(lib, name)
+
+    def scan(runs, left=None):
+        # so many heads' runs stay whole: the room that their blocks take, and `left` bytes
+        room = size if left is None else lambda rows, segments, heads, *dims: size(rows, segments, 1000, *dims) // 1000 * heads + left
+        monkeypatch.setattr(lib, name, room)
         state = m.allocate(n + 1, BF16, dev)
         S = state[0] if kind == "delta" else state
         S.copy_((0.1 * _rand(*S.shape, seed=61).float()).to(dev))
@@ -383,6 +392,16 @@ def test_recurrences_in_pieces(dev, kind, H, D, V, lens):
         m.scan(*([h] if kind == "memory" else []), proj, state, ctx, out)
         return out.float(), S.double(), state[1] if kind == "delta" else None
     (got, gs, gt), (want, ws, wt) = scan(True), scan(False)
+    for left in (0, 64):                         # and too little for the first state
+        one, os, ot = scan(True, left)
+        # whole runs and pieces: the planes' products leave out 2^-24 of each, sums of up to 1400 terms in fp32 stand in another order
+        assert float((gs - os).norm() / os.norm()) < 2.0 ** -20, float((gs - os).norm() / os.norm())
+        # rows: one in 2^12 lies so near the middle of two bf16 values that 2^-20 moves it to the other, 2^-8 away
+        assert float((got - one).norm() / one.norm()) < 2.0 ** -13, float((got - one).norm() / one.norm())
+        if gt is not None:
+            assert torch.equal(gt[1:], ot[1:])
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        scan(True, -4)
     # the state: sums of up to 1400 terms in fp32, each way within 2^-24 sqrt(1400) of their size, decays of 2^-23 each token
     # that forgets little; the token-by-token form takes its exponentials from another function
     assert float((gs - ws).norm() / ws.norm()) < 2.0 ** -13

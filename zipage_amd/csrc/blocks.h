@@ -191,9 +191,10 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 //   blocks   as without pieces, each from its state on
 //
 // Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) allow.  Where the sums and the two
-// launches cost more than what is saved, runs stay whole: a block of the sums takes 0.3 of one with rows (0.8 for the delta
-// rule), the launches 18 us, states of the delta rule 2.4 us a piece (matrix memory, 8 heads, a prompt of 155 tokens: whole
-// 41.8 us, in pieces 42.8; linear attention, 32 heads, 200 tokens: 53, 46).  Whole scans: linear attention, 32 heads of 128,
+// launches cost more than what is saved, runs stay whole (PieceCost): a block of the sums takes 0.3 of one with rows (0.8 for the
+// delta rule), the launches 19 us (15 for the delta rule, whose blocks are the longer ones), states of the delta rule 2.4 us a
+// piece (matrix memory, 8 heads, a prompt of 155 tokens: whole 41.8 us, in pieces 42.8; linear attention, 32 heads, 200
+// tokens: 53, 46).  Whole scans: linear attention, 32 heads of 128,
 // 4 prompts of 500 to 2048 tokens 374 -> 287 us; 16 heads, 8 prompts of 2048, retention 429 -> 332 and matrix memory 369
 // -> 285; retention, a prompt of 700 126 -> 45; delta rule, 32 heads, a prompt of 2048 477 -> 269, two of about 1250 384 -> 314.
 constexpr int kPieceGroups = 256, kPieceStates = 384, kLeastPiece = 4;
@@ -203,14 +204,23 @@ struct Pieces {
 };
 inline bool few_heads(int64_t segments, int64_t heads) { return segments * heads * 2 <= kPieceGroups; }
 // The sums take `groups` workgroups per piece and, in tenths of a block, `sum` per block; the rest `fixed` and `state` per piece.
-inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest, int groups, int sum, int fixed, int state) {
+struct PieceCost { int groups, sum, fixed, state; };
+inline int64_t piece_slots(int64_t rows, int64_t segments, int64_t blocks) { return rows / (kBlock * blocks) + segments; }
+// States that runs in so many rows can ask for, whatever the longest: none where the longest that fits stays whole.
+inline int64_t most_states(int64_t rows, int64_t segments, int64_t heads, const PieceCost& cost) {
+  if (!few_heads(segments, heads) || (rows + kBlock - 1) / kBlock * 10 <= kLeastPiece * (10 + cost.sum) + cost.fixed) return 0;
+  const int64_t states = piece_slots(rows, segments, kLeastPiece) * heads;
+  return states < kPieceStates ? states : kPieceStates;
+}
+// Runs stay whole, too, where `room` states are not enough.
+inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest, const PieceCost& cost, int64_t room) {
   Pieces p;
   const int64_t all = (longest + kBlock - 1) / kBlock;
   if (!few_heads(segments, heads)) return p;
   for (int64_t m = kLeastPiece; m < all; ++m) {
-    const int64_t most = (all + m - 1) / m, slots = rows / (kBlock * m) + segments, pieces = segments * most < slots ? segments * most : slots;
-    if (pieces * heads > kPieceGroups || (pieces - segments) * heads * groups > kPieceGroups || slots * heads > kPieceStates) continue;
-    if (m * (10 + sum) + fixed + most * state < all * 10) p.blocks = (int)m, p.most = (int)most;
+    const int64_t most = (all + m - 1) / m, slots = piece_slots(rows, segments, m), pieces = segments * most < slots ? segments * most : slots;
+    if (pieces * heads > kPieceGroups || (pieces - segments) * heads * cost.groups > kPieceGroups || slots * heads > kPieceStates) continue;
+    if (m * (10 + cost.sum) + cost.fixed + most * cost.state < all * 10 && slots * heads <= room) p.blocks = (int)m, p.most = (int)most;
     return p;
   }
   return p;

@@ -634,11 +634,13 @@ static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads, int d
   return (rows / kBlock + segments) * heads * block_floats(dk, dv) * 4;
 }
 
+constexpr PieceCost kCost = {2, 8, 60, 10};
+
 // With room for the states between pieces of few heads' runs, whatever the longest run.
 extern "C" int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk, int32_t dv) {
   if (rows < 0 || segments < 0 || heads <= 0 || dk <= 0 || dv <= 0) return -1;
-  const bool pieces = dk == dv && dk <= 128 && few_heads(segments, heads);
-  return blocks_bytes(rows, segments, heads, dk, dv) + (pieces ? (int64_t)kPieceStates * piece_floats(dk) * 4 : 0);
+  return blocks_bytes(rows, segments, heads, dk, dv) +
+         (dk == dv && dk <= 128 ? most_states(rows, segments, heads, kCost) * piece_floats(dk) * 4 : 0);
 }
 
 extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
@@ -662,8 +664,7 @@ extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t lo
   const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk, a.dv);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "delta_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, first_row, {}};
-  if (a.dk == a.dv && workspace_bytes >= zp_delta_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk, a.dv))
-    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 2, 8, 60, 10);     // else runs stay whole
+  if (a.dk == a.dv) ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   return launch_runs(ra, longest, (hipStream_t)stream);

@@ -456,11 +456,12 @@ static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads, int d
   return (rows / kBlock + segments) * heads * block_floats(dk) * 4;
 }
 
+constexpr PieceCost kCost = {1, 3, 75, 0};
+
 // With room for the states between pieces of few heads' runs, whatever the values' size and the longest run.
 extern "C" int64_t zp_linear_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk) {
   if (rows < 0 || segments < 0 || heads <= 0 || dk <= 0) return -1;
-  const bool pieces = few_heads(segments, heads) && dk <= 128;
-  return blocks_bytes(rows, segments, heads, dk) + (pieces ? (int64_t)kPieceStates * piece_floats(dk, 128) * 4 : 0);
+  return blocks_bytes(rows, segments, heads, dk) + (dk <= 128 ? most_states(rows, segments, heads, kCost) * piece_floats(dk, 128) * 4 : 0);
 }
 
 extern "C" int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t longest, void* workspace,
@@ -481,8 +482,7 @@ extern "C" int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t 
   const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "linear_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, first_row, {}};
-  if (workspace_bytes >= zp_linear_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads, a.dk))    // else runs stay whole
-    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 1, 3, 75, 0);
+  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   hipStream_t st = (hipStream_t)stream;

@@ -484,11 +484,12 @@ static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads) {
   return ((rows / kBlock + segments) * kAux + rows * 4) * heads * 4;
 }
 
+constexpr PieceCost kCost = {1, 3, 75, 0};
+
 // With room for the states between pieces of few heads' runs, whatever the sizes and the longest run.
 extern "C" int64_t zp_mlstm_runs_workspace(int32_t rows, int32_t segments, int32_t heads) {
   if (rows < 0 || segments < 0 || heads <= 0) return -1;
-  const bool pieces = few_heads(segments, heads);
-  return blocks_bytes(rows, segments, heads) + (pieces ? (int64_t)kPieceStates * piece_floats(128, 128) * 4 : 0);
+  return blocks_bytes(rows, segments, heads) + most_states(rows, segments, heads, kCost) * piece_floats(128, 128) * 4;
 }
 
 extern "C" int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t longest, void* workspace,
@@ -510,8 +511,7 @@ extern "C" int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t lo
   const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "mlstm_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, nullptr, first_row, {}};
-  if (workspace_bytes >= zp_mlstm_runs_workspace(a.seg.num_rows - first_row, a.seg.n, a.heads))           // else runs stay whole
-    ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, 1, 3, 75, 0);
+  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.scal = (float4*)(ra.aux + ((int64_t)(a.seg.num_rows - first_row) / kBlock + a.seg.n) * a.heads * kAux);
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
