@@ -7,7 +7,10 @@ from torch.autograd import forward_ad
 
 from zipage_amd import _lib
 
-_TENSORS = (torch.Tensor, torch.nn.Parameter)
+_TENSORS, _FEW_TYPES = (torch.Tensor, torch.nn.Parameter), (torch.bfloat16, torch.float16)
+_is_compiling, _is_autocast_enabled, _is_tracing = torch.compiler.is_compiling, torch.is_autocast_enabled, torch._C._is_tracing
+_transforms, _current_device = torch._C._functorch.peek_interpreter_stack, torch._C._cuda_getDevice
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 
 
 def pad_to_multiple(n: int, to: int) -> int:
@@ -23,7 +26,7 @@ def fit(t: torch.Tensor, *shape: int) -> torch.Tensor:
 
 def _few_rows(n: int, k: int, m: int) -> bool:
     """Whether a product of n rows of k elements and (m, k) weights goes to the kernel for few rows: where that is no slower on the GPU, with
-    weights from memory (us of both, the library second; a call of the library costs 18 us of host time, of the kernel 8).
+    weights from memory (us of both, the library second; a call of the library costs 18 us of host time, of the kernel 7).
 
     Up to 16 rows: nearly everywhere (8 rows, 1024 -> 4096 4.3 and 7.7, 4096 -> 4096 9.1 and 15.8, 2048 -> 151 936 121 and 212).
     Long contractions need outputs that fill one round of workgroups (12 288 -> 4096 21.6 and 22.5, but -> 1024 18.6 and 17.0,
@@ -48,25 +51,22 @@ def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether something beside the product looks at the call, which only the library's passes through torch's dispatcher:
     gradients of either mode, vmap and its like, autocast, modes, subclasses, tracing and compilation; or another device than the current
     one is meant."""
-    return (type(x) not in _TENSORS or type(w) not in _TENSORS
-            or torch.is_grad_enabled() and (x.requires_grad or w.requires_grad) or forward_ad._current_level >= 0
-            or torch._C._functorch.peek_interpreter_stack() is not None or torch.is_autocast_enabled("cuda")
-            or torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
-            or torch._C._get_tracing_state() is not None or torch.compiler.is_compiling()
-            or x.device.index != torch._C._cuda_getDevice())
+    return (_is_compiling() or type(x) not in _TENSORS or type(w) not in _TENSORS or forward_ad._current_level >= 0
+            or _transforms() is not None or _is_autocast_enabled() or _dispatch_modes() > 0 or _function_modes() > 0 or _is_tracing()
+            or (x.requires_grad or w.requires_grad) and torch.is_grad_enabled() or x.device.index != _current_device())
 
 
 def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) without a bias."""
-    if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 and x.dtype in (torch.bfloat16, torch.float16) and x.dtype == w.dtype \
-            and w.dim() == 2 and x.layout == w.layout == torch.strided:
-        (n, k), m, stride = x.shape, w.shape[0], x.stride(0)
-        if _few_rows(n, k, m) and w.shape[1] == k and x.stride(1) == 1 and k <= stride <= 1 << 23 and stride % 8 == 0 and \
-                w.is_contiguous() and w.device == x.device and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-            out = x.new_empty(n, m)
-            _lib.call_models("zp_few_rows_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, k, m, stride, m,
-                             _lib.dtype_tag(x), _lib.stream_ptr(x))
-            return out
+    if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 == w.dim() and x.layout == w.layout == torch.strided:
+        (n, k), (m, wk), (stride, one) = x.shape, w.shape, x.stride()
+        if k == wk and x.dtype == w.dtype in _FEW_TYPES and _few_rows(n, k, m) and one == 1 and k <= stride <= 1 << 23 and \
+                stride % 8 == 0 and w.is_contiguous() and w.device == x.device:
+            at, w_at = x.data_ptr(), w.data_ptr()
+            if (at | w_at) % 16 == 0:
+                out = x.new_empty(n, m)
+                _lib.call_models("zp_few_rows_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, _lib.dtype_tag(x), _lib.stream_ptr(x))
+                return out
     return F.linear(x, w)
 
 
