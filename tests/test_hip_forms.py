@@ -63,11 +63,13 @@ def test_compaction_of_the_longest_list(dev, width):
 
 # ------------------------------------------------------------------ attention scores
 # pages of 256 tokens with groups of two or four heads and a mean over the window have forms of their own; the same
-# tokens in pages of 128 take the general one: same bits.
+# tokens in pages of 128 take the general one: same bits.  Of few blocks of rows, too, whose tiles lie side by side where there is
+# room, and which walk them where there is not.
 @pytest.mark.parametrize("dtype", [BF16, torch.float16, torch.float32])
 @pytest.mark.parametrize("group,W", [(2, 32), (2, 16), (2, 5), (4, 32), (3, 20)])
 def test_scores_by_page_size_and_group(dev, dtype, group, W):
     from zipage_amd.kernel import attention_score
+    from tests.test_hip_kernels import _score_one_sweep
     B, Hkv, D, P = 3, 2, 128, 9
     g = torch.Generator().manual_seed(group * 64 + W)
     pages = torch.randperm(P, generator=g).tolist()
@@ -75,9 +77,10 @@ def test_scores_by_page_size_and_group(dev, dtype, group, W):
     k, q = _rand(1, P, 256, Hkv, D, seed=W, dtype=dtype).to(dev), _rand(1, B, W, group * Hkv, D, seed=W + 1, dtype=dtype).to(dev)
     seq = torch.arange(B, dtype=torch.int32, device=dev)
     whole, halves = (O.encode_block_table(t).to(dev) for t in (tables, [[2 * p + i for p in t for i in (0, 1)] for t in tables]))
-    got = attention_score(k, q, seq, whole)
-    want = attention_score(k.view(1, 2 * P, 128, Hkv, D), q, seq, halves)
-    assert torch.equal(got.reshape(want.shape), want)
+    want = _score_one_sweep(k.view(1, 2 * P, 128, Hkv, D), q, seq, halves)
+    for got in (_score_one_sweep(k, q, seq, whole), attention_score(k, q, seq, whole),
+                attention_score(k.view(1, 2 * P, 128, Hkv, D), q, seq, halves)):
+        assert torch.equal(got.reshape(want.shape), want)
 
 
 # up to 64 blocks of query rows (32, fp32: 16) have their tiles side by side, more walk them: same bits for a sequence alone and
@@ -87,8 +90,8 @@ def test_scores_by_page_size_and_group(dev, dtype, group, W):
                                                     (4, 32, 256, 96, "max", 17), (8, 5, 256, 128, "mean", 33), (8, 3, 128, 40, "max", 65),
                                                     (16, 4, 128, 128, "mean", 33), (1, 20, 128, 128, "max", 65)])
 def test_scores_of_few_sequences(dev, dtype, group, W, BS, D, reduced, B):
-    from zipage_amd import _lib
     from zipage_amd.kernel import attention_score
+    from tests.test_hip_kernels import _score_one_sweep
     NB = 6
     g = torch.Generator().manual_seed(group * 64 + W)
     pages = torch.randperm(B * NB, generator=g).tolist()
@@ -97,15 +100,16 @@ def test_scores_of_few_sequences(dev, dtype, group, W, BS, D, reduced, B):
     seq = torch.randperm(B, generator=g).int().to(dev)
     many = attention_score(k, q, seq, enc.to(dev), reduced=reduced)
     for n in (1, 3):
-        few = attention_score(k, q, seq[:n].contiguous(), enc[:n].contiguous().to(dev), reduced=reduced)
-        assert torch.equal(few, many[:, :n])
+        args = (k, q, seq[:n].contiguous(), enc[:n].contiguous().to(dev), reduced)
+        for few in (attention_score(*args[:4], reduced=reduced), _score_one_sweep(*args)):
+            assert torch.equal(few, many[:, :n])
     want = O.attention_score(k[:, :, :, :, :].cpu(), q.cpu(), seq[:3].cpu(), enc[:3], reduced=reduced)
     torch.testing.assert_close(many[:, :3].cpu().float(), want.float(), rtol=2.0 ** -6 if dtype != torch.float32 else 1e-4, atol=1e-6)
 
 
 # ------------------------------------------------------------------ redundancy inside pages
-# 16-bit caches: workgroups walk whole rows where 512 of them, or a multiple, are at least 90 % full (461 rows on), and
-# take a page each otherwise; fp32 always does.  Same bits for a sequence alone, in a batch that is walked and in one
+# workgroups walk whole rows where 512 of them (fp32: 256), or a multiple, are at least 90 % full (461 rows on), and
+# take a page each otherwise.  Same bits for a sequence alone, in a batch that is walked and in one
 # that is not; pages the caller did not list score as none.
 @pytest.mark.parametrize("dtype", [BF16, torch.float16, torch.float32])
 @pytest.mark.parametrize("B", [57, 58, 64, 65, 116])

@@ -338,6 +338,30 @@ def test_attention_score_fp32_logit_range(dev, boost):
     assert torch.isfinite(got.float()).all()
 
 
+def _score_in(scratch, k, q, seq_idx, enc, reduced="mean"):
+    """zp_attention_score with so many bytes of scratch."""
+    from zipage_amd import _lib
+    L, P, BS, Hkv, D = k.shape
+    _, S, W, Hq, _ = q.shape
+    B, NB = enc.shape
+    out = torch.empty((L, B, Hkv, NB, BS), device=k.device, dtype=k.dtype)
+    ws = torch.empty(max(scratch, 1), device=k.device, dtype=torch.uint8)
+    _lib.call("zp_attention_score", _lib.dev_ptr(k), _lib.dev_ptr(q), _lib.dev_ptr(seq_idx),
+              _lib.dev_ptr(enc), _lib.dev_ptr(out), 0, L, B, NB, BS, Hkv, Hq, D, W, P, S,
+              k.stride(0), k.stride(1), q.stride(0), q.stride(1), float(D ** -0.5),
+              {"mean": 0, "max": 1}[reduced], _lib.dtype_tag(k), _lib.dev_ptr(ws) if scratch else 0,
+              scratch, _lib.stream_ptr(k))
+    return out
+
+
+def _score_one_sweep(k, q, seq_idx, enc, reduced="mean"):
+    """With the scratch for the window partials alone: a block of query rows walks its sequence's tiles, however
+    few blocks there are."""
+    from zipage_amd import _lib
+    (L, _, BS, Hkv, _), (_, _, W, Hq, _), (B, NB) = k.shape, q.shape, enc.shape
+    return _score_in(_lib.load().zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, _lib.dtype_tag(k)), k, q, seq_idx, enc, reduced)
+
+
 def _score_three_sweeps(k, q, seq_idx, enc, reduced="mean"):
     """zp_attention_score without the scratch for the window partials: the library then takes
     the kernel that sweeps K three times."""
@@ -346,7 +370,6 @@ def _score_three_sweeps(k, q, seq_idx, enc, reduced="mean"):
     _, S, W, Hq, _ = q.shape
     B, NB = enc.shape
     lib = _lib.load()
-    out = torch.empty((L, B, Hkv, NB, BS), device=k.device, dtype=k.dtype)
     full = lib.zp_attention_score_workspace(L, B, NB, BS, Hkv, Hq, W)
     assert full > 0
     # more than 128 window x group rows: the three-sweep kernel keeps fp32 partial sums of its
@@ -356,13 +379,7 @@ def _score_three_sweeps(k, q, seq_idx, enc, reduced="mean"):
         gp *= 2
     floor = L * B * Hkv * NB * BS * 4 if (W * gp + 31) // 32 > 4 else 0
     assert floor < full
-    ws = torch.empty(max(floor, 1), device=k.device, dtype=torch.uint8)
-    _lib.call("zp_attention_score", _lib.dev_ptr(k), _lib.dev_ptr(q), _lib.dev_ptr(seq_idx),
-              _lib.dev_ptr(enc), _lib.dev_ptr(out), 0, L, B, NB, BS, Hkv, Hq, D, W, P, S,
-              k.stride(0), k.stride(1), q.stride(0), q.stride(1), float(D ** -0.5),
-              {"mean": 0, "max": 1}[reduced], _lib.dtype_tag(k), _lib.dev_ptr(ws) if floor else 0,
-              floor, _lib.stream_ptr(k))
-    return out
+    return _score_in(floor, k, q, seq_idx, enc, reduced)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
@@ -379,13 +396,15 @@ def test_attention_score_one_sweep_matches_three_sweeps(dev, dtype, shape, reduc
     """16-bit caches, sequences of at most 2560 tokens: the kernel that keeps the rounded logits
     in registers (one sweep over K) against the three-sweep kernel and against the oracle.  Same
     rounding points; the row sums are added in another order, which moves a few values across a
-    rounding boundary."""
+    rounding boundary.  So few blocks of rows have their tiles side by side where there is room for their
+    logits: the same bits."""
     from zipage_amd.kernel import attention_score
     shape = dict(shape)
     nb = shape.pop("nb_choices")
     s = _setup(71, dtype, L=2, B=4, nb_choices=nb, num_pages=48, **shape)
     args = tuple(a.to(dev) for a in (s["k"], s["q"], s["seq_idx"], s["enc"]))
-    one = attention_score(*args, reduced=reduced)
+    one = _score_one_sweep(*args, reduced=reduced)
+    assert torch.equal(attention_score(*args, reduced=reduced), one)
     three = _score_three_sweeps(*args, reduced=reduced)
     ulps = 2 if reduced == "mean" else 16
     _ulp_close(one, three.cpu(), dtype, ulps=ulps, frac_exact=0.98)
@@ -423,7 +442,8 @@ def test_attention_score_fp32_one_sweep_matches_two_sweeps(dev, shape, reduced):
     need = lib.zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, 2)
     assert need == L * B * Hkv * -(-W * max(1, 1 << (Hq // Hkv - 1).bit_length()) // 16) * NB * BS * 4
     assert need <= lib.zp_attention_score_workspace(L, B, NB, BS, Hkv, Hq, W)
-    one = attention_score(*args, reduced=reduced)
+    one = _score_one_sweep(*args, reduced=reduced)
+    assert torch.equal(attention_score(*args, reduced=reduced), one)
     two = _score_three_sweeps(*args, reduced=reduced)
     _rel_close(one, two.cpu(), rel=1e-4, abs_floor=1e-9)
     want = O.attention_score(s["k"], s["q"], s["seq_idx"], s["enc"], reduced=reduced)
