@@ -415,6 +415,36 @@ def test_recurrences_in_pieces(dev, monkeypatch, kind, H, D, V, lens):
     if gt is not None:
         assert torch.equal(gt[1:], wt[1:])       # the convolutions' last inputs
 
+# The gates of matrix memories: as many waves as the longest run keeps busy.  A wave's remainder, all that it has, one token more; runs
+# shorter than the longest; the same bits as with the sixteen that a longest run of 1100 tokens gets (whole runs: no room for pieces).
+@pytest.mark.parametrize("lens", [(1,), (63, 64, 5), (65, 16), (128, 129, 17), (449, 448), (960, 961, 2), (1023,), (1025, 1024)])
+def test_matrix_memory_gates_by_the_longest_run(dev, monkeypatch, lens):
+    import types
+    from zipage_amd import _lib
+    from zipage_amd.engine.qwen3 import Segments
+    from zipage_amd.layers import MatrixMemory
+    W, H, D, n, rows = 64, 3, 32, len(lens), sum(lens)
+    m = MatrixMemory(W, H, D, D, 15.0, 1e-3)
+    w = {k: _rand(*s, seed=i) * s[-1] ** -0.5 for i, (k, s) in enumerate(m.shapes().items())}
+    into, _ = m.load(w, BF16, dev, W)
+    h = _rand(rows, W, seed=60).to(dev)
+    proj = (h.float() @ into.to(dev).float().T).to(BF16)
+    t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
+    lib = _lib.load_models("recurrent")
+    size = lib.zp_mlstm_runs_workspace
+    monkeypatch.setattr(lib, "zp_mlstm_runs_workspace", lambda rows, segments, heads: size(rows, segments, 1000) // 1000 * heads)
+
+    def scan(longest):
+        S = m.allocate(n + 1, BF16, dev)
+        S.copy_((0.1 * _rand(*S.shape, seed=61).float()).to(dev))
+        seg = Segments(t([sum(lens[:i]) for i in range(n)]), t(lens), t(list(range(n, 0, -1))), t([7 * i for i in range(n)]), longest=longest)
+        out = torch.empty(rows, m.out_columns, dtype=BF16, device=dev)
+        m.scan(h, proj, S, types.SimpleNamespace(segments=None, run_segments=seg), out)
+        return out, S
+    for got, want in zip(scan(max(lens)), scan(1100)):
+        assert bool(torch.isfinite(got).all()) and torch.equal(got, want)
+
+
 
 # ------------------------------------------------------------------ rotary store of heads of 128
 # aligned rows take sixteen lanes a vector, fewer than 2^18 of them with a workgroup per sixteen; others take a wave a vector

@@ -36,10 +36,12 @@ template <int N> __device__ __forceinline__ float row_shr(float v, float edge) {
                                                                0xf, 0xf, false));
 }
 
-// A workgroup per head and run, a wave 64 tokens of every 1024: sums and maxima of blocks side by side, then one wave takes the
-// maximum from block to block.  (One wave for all, 64 tokens at a time: 14.2 us for 970 tokens of 16 heads, now 7.4; three runs of 844 to 2043 21.2, now 9.7.)
-constexpr int kGateWaves = 16, kGateTokens = 64 * kGateWaves;
-__global__ __launch_bounds__(kGateTokens) void mlstm_gates_kernel(RunArgs ra) {
+// A workgroup per head and run, a wave 64 tokens of every stretch: sums and maxima of blocks side by side, then one wave takes the
+// maximum from block to block.  As many waves as the longest run keeps busy, up to 16.  (One wave for all, 64 tokens at a
+// time: 14.2 us for 970 tokens of 16 heads, now 7.4; three runs of 844 to 2043 21.2, now 9.7.  With 16 waves for any run 40 runs of
+// 17 tokens, 64 heads of 64, took 57.9 us with the kernels behind; with one wave each 45.3.)
+constexpr int kGateWaves = 16;
+__global__ __launch_bounds__(64 * kGateWaves) void mlstm_gates_kernel(RunArgs ra) {
   __shared__ float ends[2][64], before[65];                    // of 64 blocks: F and the maximum of x at the last token; m before it
   const zp_mlstm& a = ra.d;
   const int tid = threadIdx.x, lane = tid & 63, block = tid >> 4, h = blockIdx.x % a.heads;
@@ -55,11 +57,12 @@ __global__ __launch_bounds__(kGateTokens) void mlstm_gates_kernel(RunArgs ra) {
     zf = a.gates[src + a.heads];
   };
   fetch(0);
-  for (int t0 = 0; t0 < sg.count; t0 += kGateTokens) {
-    const int cnt = min(kGateTokens, sg.count - t0);
+  const int stretch = blockDim.x;
+  for (int t0 = 0; t0 < sg.count; t0 += stretch) {
+    const int cnt = min(stretch, sg.count - t0);
     const float gi = a.cap * tanhf((zi + ib) * icap), x = a.cap * tanhf((zf + fb) * icap);
     const float gf = fminf(x, 0.f) - log1pf(expf(-fabsf(x)));
-    if (t0 + kGateTokens < sg.count) fetch(t0 + kGateTokens);
+    if (t0 + stretch < sg.count) fetch(t0 + stretch);
     // sums and maxima inside each block of 16 lanes: m_t = F_t + max(m before the block, max_{s <= t} x_s)
     float F = tid < cnt ? gf : 0.f;
     F += row_shr<1>(F, 0.f);
@@ -78,7 +81,8 @@ __global__ __launch_bounds__(kGateTokens) void mlstm_gates_kernel(RunArgs ra) {
     }
     __syncthreads();
     if (tid < 64) {
-      const float Fe = ends[0][lane], te = ends[1][lane];
+      const bool there = lane * kBlock < stretch;
+      const float Fe = there ? ends[0][lane] : 0.f, te = there ? ends[1][lane] : -INFINITY;
       float mine = m;
 #pragma unroll 1
       for (int b0 = 0; b0 * kBlock < cnt; b0 += 8)             // blocks behind the end change nothing
@@ -466,7 +470,8 @@ template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
 template <int KT> int launch_runs(const RunArgs& ra, int longest, hipStream_t st) {
   const zp_mlstm& a = ra.d;
   const unsigned grid = (unsigned)((int64_t)a.seg.n * a.heads);
-  hipLaunchKernelGGL(mlstm_gates_kernel, dim3(grid), dim3(kGateTokens), 0, st, ra);
+  const int waves = longest < 64 * kGateWaves ? (longest + 63) / 64 : kGateWaves;
+  hipLaunchKernelGGL(mlstm_gates_kernel, dim3(grid), dim3(64 * waves), 0, st, ra);
   hipLaunchKernelGGL((mlstm_prepare_kernel<KT>), dim3((unsigned)((longest + kBlock - 1) / kBlock), (unsigned)((a.heads + 3) / 4), (unsigned)a.seg.n),
                      dim3(256), 0, st, ra);
   ZP_LAUNCH_CHECK();
