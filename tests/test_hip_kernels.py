@@ -338,14 +338,14 @@ def test_attention_score_fp32_logit_range(dev, boost):
     assert torch.isfinite(got.float()).all()
 
 
-def _score_in(scratch, k, q, seq_idx, enc, reduced="mean"):
+def _score_in(scratch, k, q, seq_idx, enc, reduced="mean", ws=None):
     """zp_attention_score with so many bytes of scratch."""
     from zipage_amd import _lib
     L, P, BS, Hkv, D = k.shape
     _, S, W, Hq, _ = q.shape
     B, NB = enc.shape
     out = torch.empty((L, B, Hkv, NB, BS), device=k.device, dtype=k.dtype)
-    ws = torch.empty(max(scratch, 1), device=k.device, dtype=torch.uint8)
+    ws = torch.empty(max(scratch, 1), device=k.device, dtype=torch.uint8) if ws is None else ws
     _lib.call("zp_attention_score", _lib.dev_ptr(k), _lib.dev_ptr(q), _lib.dev_ptr(seq_idx),
               _lib.dev_ptr(enc), _lib.dev_ptr(out), 0, L, B, NB, BS, Hkv, Hq, D, W, P, S,
               k.stride(0), k.stride(1), q.stride(0), q.stride(1), float(D ** -0.5),
@@ -380,6 +380,28 @@ def _score_three_sweeps(k, q, seq_idx, enc, reduced="mean"):
     floor = L * B * Hkv * NB * BS * 4 if (W * gp + 31) // 32 > 4 else 0
     assert floor < full
     return _score_in(floor, k, q, seq_idx, enc, reduced)
+
+
+@pytest.mark.parametrize("dtype,per_unit", [(torch.bfloat16, 32), (torch.float16, 32), (torch.float32, 16)])
+@pytest.mark.parametrize("G,units,NB,BS,reduced,side_by_side", [
+    (4, 32, 6, 256, "mean", True), (4, 40, 6, 256, "mean", False), (4, 40, 7, 256, "mean", True), (2, 64, 1, 256, "mean", False),
+    (2, 64, 7, 256, "mean", True), (4, 64, 2, 256, "max", True), (1, 64, 2, 256, "mean", True), (4, 64, 4, 128, "mean", True)])
+def test_attention_score_route_of_few_units(dev, dtype, per_unit, G, units, NB, BS, reduced, side_by_side):
+    """Tiles side by side leave their logits behind the room that the walk uses; either way the walk's bits."""
+    from zipage_amd import _lib
+    W, B, Hkv = per_unit // G, 1, units             # a window and its group fill one block of rows
+    g = torch.Generator().manual_seed(units + NB)
+    k = torch.randn(1, B * NB, BS, Hkv, 128, generator=g).to(dtype).to(dev)
+    q = torch.randn(1, B, W, Hkv * G, 128, generator=g).to(dtype).to(dev)
+    enc = O.encode_block_table([list(range(NB))]).to(dev)
+    seq = torch.zeros(B, dtype=torch.int32, device=dev)
+    size = lambda f: f(1, B, NB, BS, Hkv, Hkv * G, W, _lib.dtype_tag(k))
+    few, walk = size(_lib.load().zp_attention_score_workspace_few), size(_lib.load().zp_attention_score_workspace_for)
+    assert few > walk
+    ws = torch.zeros(few, dtype=torch.uint8, device=dev)
+    got = _score_in(few, k, q, seq, enc, reduced, ws)
+    assert bool(ws[walk:].any()) == side_by_side
+    assert torch.equal(got, _score_one_sweep(k, q, seq, enc, reduced))
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])

@@ -1741,10 +1741,17 @@ static int64_t resident_need(int L, int B, int NB, int BS, int Hkv, int Hq, int 
 }
 
 // Few units spread their tiles over the chip (score_tiles_kernel); what that needs, or 0.  The line lies where they
-// occupy a quarter of the CUs: the whole compression step of one fp32 sequence, 16 heads, window 32 (32 units) 59 -> 47 us, of
-// two 66 -> 61; 16-bit, window 16 (8) 42 -> 33, four sequences (32) 51 -> 43, eight (64) 65 -> 58; but 32 heads, window 32: two
-// sequences (64) 47 -> 44, three 47 -> 52, as logits through memory cost more with every unit.
+// occupy a quarter of the CUs: the whole compression step of one fp32 sequence, 16 heads, window 32 (32 units) 59 -> 49 us, of
+// two (64) 65 -> 61; 16-bit, window 16, four sequences (32) 53 -> 45, eight (64) 64 -> 58; 32 heads, window 32: two sequences
+// (64) 46 as before, three 47 -> 52, as logits through memory cost more with every unit.
 constexpr int64_t kFewUnits = 64;
+// The walk with a straight-line epilogue (groups of two and four, pages of 256) catches up sooner where it has few tiles to
+// walk: scores alone, keys from memory, 16-bit, groups of four, window 32, tiles against the walk: 32 units, 2 pages 14.2 against
+// 14.6 us, 5 pages 18.1 / 20.5; 64 units, 3 pages 18.0 / 16.5, 5 pages 21.4 / 20.7, 7 pages 23.4 / 24.3, 10 pages 25.9 / 29.9
+// (keys in the caches: 5 pages 20.6 / 17.7, 10 pages 26.0 / 25.8); fp32, 5 pages, 32 units 20.1 / 25.3, 64 units 26.9 / 27.2
+// (26.5 / 24.5).
+constexpr int64_t kFewUnitsShort = 32;
+constexpr int kShortPages = 6;
 static int64_t tiled_need(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype) {
   if (!resident_need(L, B, NB, BS, Hkv, Hq, W, dtype)) return 0;
   const int Gp = pow2_ceil(Hq / Hkv);
@@ -1849,11 +1856,12 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
   a.n_items = L * B * Hkv;
   a.part = (float*)workspace;
   const int64_t tiled = tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype);
-  if ((resident || resident32) && tiled && workspace_bytes >= tiled) {
+  const bool straight = BS == 256 && !a.reduce_max && (Gp == 2 || Gp == 4);
+  const int64_t walks = (int64_t)a.n_items * (resident32 ? (W * Gp + 15) / 16 : RB);
+  if ((resident || resident32) && tiled && workspace_bytes >= tiled && !(straight && NB <= kShortPages && walks > kFewUnitsShort)) {
     if (resident32) a.RB = (W * Gp + 15) / 16;
-    const unsigned units = (unsigned)(a.n_items * a.RB);
     a.tiles = NB * (BS / (resident ? 128 : 64));
-    a.lg = (char*)workspace + (int64_t)units * NB * BS * (resident ? 32 : 16);
+    a.lg = (char*)workspace + walks * NB * BS * (resident ? 32 : 16);
     const dim3 cgrid((unsigned)a.n_items, (unsigned)((NB * BS / 4 + 255) / 256));
 #define ZP_TILED_LAUNCH(TPP)                                                                                          \
   do {                                                                                                                \
