@@ -78,7 +78,10 @@ int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32
  * gate (rows gate_stride elements apart, heads of V back to back, of the call's dtype) or NULL: no gate.
  * Sinks are for one map only.
  * turns: (rows of q, V / 2) pairs cos, sin of one map whose values turned by angles of their positions; elements 2 i
- * and 2 i + 1 of every head's output turn back by the query's.  16-byte aligned; NULL: nothing turns. */
+ * and 2 i + 1 of every head's output turn back by the query's.  16-byte aligned; NULL: nothing turns.
+ * q_turns: (q_half / 2) planes of (rows of q, 2) pairs cos, sin, a plane q_plane rows on, of one map without a soft cap or shared keys, whose queries come as projected:
+ * elements j < q_half of every head of q turn with j + q_half by them, and are rounded as a stored q is.  q_half 32 or 64,
+ * 2 q_half <= D <= 128, V <= 128; 16-byte aligned; NULL: q is as it is.  Attention of runs only. */
 typedef struct {
   float softcap;
   int32_t maps;
@@ -87,6 +90,9 @@ typedef struct {
   const void* gate;
   int64_t gate_stride;
   const float* turns;
+  const float* q_turns;
+  int64_t q_plane;
+  int32_t q_half;
 } zp_attention_form;
 
 /* Attention of runs of tokens, bfloat16.  tiles (T, 4) int32, one entry per up to 128 queries of one
@@ -157,7 +163,9 @@ int zp_latent_rows_attention(const void* q, const void* cache, const int32_t* ta
  * elements), before they turn.
  * tied: the values are the keys as they are in `in`, which has no value columns; VT = HK * D.
  * value_freqs (V / 2): the values' heads of V turn too, elements 2 i and 2 i + 1 by positions[.] * value_freqs[i];
- * turns (n, V / 2) receives cos and sin of these angles. */
+ * turns (n, V / 2) receives cos and sin of these angles.
+ * q_turns (rot / 4, n, 2): q goes to q_out for the first q_rows rows only; for the others cos and sin of its angles, two in a
+ * plane, come here, for zp_run_attention to turn it by.  rot a multiple of 4.  Without norm and bias; NULL: q goes to q_out for all. */
 typedef struct {
   const float* norm;
   int32_t q_norm, k_norm;
@@ -166,6 +174,8 @@ typedef struct {
   int32_t V;
   const float* value_freqs;
   float* turns;
+  float* q_turns;
+  int32_t q_rows;
 } zp_store_form;
 
 /* Rows `in` (in_stride elements apart) hold q (H heads of D), k (HK of D) and VT value columns; with `bias`

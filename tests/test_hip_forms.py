@@ -199,6 +199,37 @@ def _tiles(lens):
     return torch.tensor(made, dtype=torch.int32)
 
 
+# queries as projected, which the attention turns itself, against queries that the store has turned: heads as long as what turns
+# and longer, 8 and 16 steps of a key, runs that take either form and both
+@pytest.mark.parametrize("H,G,D,V,rot", [(4, 2, 64, 64, 64), (2, 1, 128, 128, 128), (3, 3, 128, 64, 64), (4, 1, 72, 128, 64), (2, 2, 104, 56, 64),
+                                         (16, 8, 128, 128, 128)])
+@pytest.mark.parametrize("lens", ["few", "short", "long"])
+def test_runs_turn_their_queries(dev, H, G, D, V, rot, lens, first=5):
+    from zipage_amd.layers import run_attention
+    from zipage_amd.layers.grouped import rotary_store, store_form
+    from zipage_amd.layers.runs import attention_form
+    lens = {"few": FEW_KEYS, "short": MANY_SHORT, "long": [(385, 385), (1, 900), (129, 193), (33, 600)]}[lens]
+    N, M = (sum(t) for t in zip(*lens))
+    rows, edge = first + N, H * D
+    proj = _rand(rows, edge + G * (D + V) + 8, seed=1).to(dev)[:, :edge + G * (D + V)]
+    pos = torch.randint(0, 3000, (rows,), generator=torch.Generator().manual_seed(2), dtype=torch.int32).to(dev)
+    freqs = (1e4 ** (-torch.arange(0, rot, 2) / rot)).float().to(dev)
+    slots = torch.arange(rows, dtype=torch.int32, device=dev)
+    cache, other = (torch.zeros(rows, 1, G * (D + V), dtype=BF16, device=dev) for _ in range(2))
+    q = rotary_store(proj, pos, freqs, H, G, D, V, cache, slots)
+    turns = torch.full((rot // 4, rows, 2, 2), float("nan"), device=dev)
+    some, kv = rotary_store(proj, pos, freqs, H, G, D, V, other, slots, return_kv=True, form=store_form(q_turns=turns, q_rows=first))
+    assert torch.equal(some, q[:first]) and torch.equal(cache, other) and torch.equal(kv, cache[:, 0])
+    keys, sinks = _rand(M, G * (D + V), seed=3).to(dev), _rand(H, seed=4, dtype=torch.float32).to(dev)
+    for scale in (D ** -0.5, -0.1):
+        got, want = (torch.empty(N, H * V, dtype=BF16, device=dev) for _ in range(2))
+        run_attention(q[first:], keys, H, G, D, V, _tiles(lens).to(dev), scale, want, window=200, sinks=sinks)
+        run_attention(proj[first:, :edge], keys, H, G, D, V, _tiles(lens).to(dev), scale, got, window=200, sinks=sinks,
+                      form=attention_form(q_turns=turns[:, first:]))
+        # both turn in 32 bits and round once, but a compiler may round a product on the way: seldom another last bit of a query
+        assert (got != want).float().mean() < 1e-3 and (got.float() - want.float()).abs().max() <= 2.0 ** -6 * want.float().abs().max()
+
+
 # the scale joins the subtraction of the maximum: a negative one turns the queries round, zero takes them away
 @pytest.mark.parametrize("scale", [-0.25, 0.0, 1e-30, 0.25])
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 40, 24), (2, 2, 64, 64), (3, 1, 128, 56), (4, 2, 128, 128), (3, 3, 136, 136)])

@@ -129,13 +129,13 @@ class LinearArgs(C.Structure):
 class AttentionForm(C.Structure):
     """zp_attention_form."""
     _fields_ = [("softcap", f32), ("maps", i32), ("balance", f32), ("eps", f32), ("vdim", i32), ("gate", ptr),
-                ("gate_stride", i64), ("turns", ptr)]
+                ("gate_stride", i64), ("turns", ptr), ("q_turns", ptr), ("q_plane", i64), ("q_half", i32)]
 
 
 class StoreForm(C.Structure):
     """zp_store_form."""
     _fields_ = [("norm", ptr), ("q_norm", i32), ("k_norm", i32), ("eps", f32), ("tied", i32), ("V", i32),
-                ("value_freqs", ptr), ("turns", ptr)]
+                ("value_freqs", ptr), ("turns", ptr), ("q_turns", ptr), ("q_rows", i32)]
 
 
 SCORE_SOFTMAX, SCORE_SIGMOID = 0, 1      # ZP_SCORE_*

@@ -37,6 +37,8 @@ struct RotaryArgs {
   int V;                    // of a value head
   const float* vfreqs;      // (V / 2,): values turn, elements 2 i and 2 i + 1 with frequency i; or null
   float2* turns;            // (n, V / 2): cos and sin of the values' angles, for the way back
+  float2* q_turns;          // (half / 2, n, 2): cos and sin of q's angles, or null; then
+  int q_rows;               // q is stored for so many rows, the others' turns are
   int staged;               // bytes of q and k that wait in LDS while their norms are taken; 0: they are read twice
 };
 
@@ -64,7 +66,10 @@ __global__ __launch_bounds__(256) void rotary_store_kernel(RotaryArgs a) {
     };
     if (NORM && a.norm) fetch(tid * 8);
     const int position = a.positions[row];
-    for (int i = tid; i < a.half; i += kPer) cs[i] = rotary_turn(position, a.freqs[i]);
+    for (int i = tid; i < a.half; i += kPer) {
+      cs[i] = rotary_turn(position, a.freqs[i]);
+      if (a.q_turns && row >= a.q_rows) a.q_turns[((int64_t)(i >> 1) * a.n + row) * 2 + (i & 1)] = cs[i];
+    }
     if (TURN)
       for (int i = tid; i < a.V / 2; i += kPer) {
         vcs[i] = rotary_turn(position, a.vfreqs[i]);
@@ -158,7 +163,7 @@ __global__ __launch_bounds__(256) void rotary_store_kernel(RotaryArgs a) {
       else Elem<T>::st(a.cache, slot * kvw + kc, o[0]);
     }
   };
-  for (int it = tid; it < items; it += kPer) {
+  for (int it = tid + (a.q_turns && row >= a.q_rows ? a.H * per_head : 0); it < items; it += kPer) {
     float x[VEC], y[VEC];
     if (it >= rotated) {
       const int v = (it - rotated) * VEC, c = end + v;
@@ -693,7 +698,8 @@ extern "C" int zp_rotary_store(const void* in, const float* bias, const int32_t*
     return ZP_EUNSUPPORTED;
   }
   if (n == 0) return ZP_OK;
-  ZP_REQUIRE(in && positions && q_out && cache && slots && (rot == 0 || freqs), "rotary_store: null pointer");
+  ZP_REQUIRE(in && positions && (q_out || (f.q_turns && f.q_rows == 0)) && cache && slots && (rot == 0 || freqs), "rotary_store: null pointer");
+  ZP_REQUIRE(!f.q_turns || (!f.norm && !bias && rot > 0 && rot % 4 == 0 && f.q_rows >= 0), "rotary_store: queries that stay as projected go without norms and bias");
   ZP_REQUIRE(aligned16(in) && aligned16(q_out) && aligned16(kv_out) && aligned16(cache) && aligned16(bias) && aligned16(f.norm),
              "rotary_store: tensors must be 16-byte aligned");
   ZP_REQUIRE(!f.norm || (!bias && f.q_norm > 0 && f.k_norm > 0), "rotary_store: norms of whole projections go without a bias");
@@ -702,7 +708,7 @@ extern "C" int zp_rotary_store(const void* in, const float* bias, const int32_t*
   ZP_REQUIRE(!f.value_freqs || (f.turns && f.V > 0 && f.V % 8 == 0 && f.V <= 1024 && VT % f.V == 0),
              "rotary_store: values that turn need their head size and room for the turns");
   RotaryArgs a = {in, bias, positions, freqs, q_out, kv_out, cache, slots, n, H, HK, D, VT, rot / 2, in_stride, num_slots,
-                  f.norm, f.q_norm, f.k_norm, f.eps, f.tied != 0, f.V, f.value_freqs, (float2*)f.turns};
+                  f.norm, f.q_norm, f.k_norm, f.eps, f.tied != 0, f.V, f.value_freqs, (float2*)f.turns, (float2*)f.q_turns, f.q_rows};
   const int tokens = n < 2048 ? 1 : 4;
   const int64_t row = (int64_t)(H + HK) * D * zp_dtype_bytes(dtype);
   if (f.norm && row * tokens <= 32 * 1024) a.staged = (int)row;
@@ -766,7 +772,7 @@ extern "C" int zp_grouped_rows_attention(const void* q, const void* cache, const
                                          int32_t NB, int32_t num_pages, int32_t window, int32_t chunk,
                                          int64_t out_stride, float scale, float out_scale, int32_t dtype,
                                          void* workspace, int64_t workspace_bytes, void* stream) {
-  const zp_attention_form plain = {0.f, 1, 0.f, 0.f, 0, nullptr, 0, nullptr}, f = form ? *form : plain;
+  const zp_attention_form plain = {0.f, 1, 0.f, 0.f, 0, nullptr, 0, nullptr, nullptr, 0, 0}, f = form ? *form : plain;
   const bool two = f.maps == 2;
   ZP_REQUIRE(n >= 0 && H > 0 && HK > 0 && H % HK == 0 && D > 0 && V > 0 && BS > 0 && B > 0 && NB > 0 &&
                  num_pages > 0 && window >= 0 && chunk >= 0 && !(window && chunk) && (f.maps == 1 || two) &&
@@ -779,6 +785,7 @@ extern "C" int zp_grouped_rows_attention(const void* q, const void* cache, const
   if (n == 0) return ZP_OK;
   ZP_REQUIRE(q && cache && table && context_lens && out, "grouped_rows_attention: null pointer");
   ZP_REQUIRE(table_rows || n <= B, "grouped_rows_attention: more tokens than table rows");
+  ZP_REQUIRE(!f.q_turns, "grouped_rows_attention: queries come turned");
   ZP_REQUIRE(!two || (!sinks && !f.turns && f.vdim > 0 && f.vdim <= V && (!f.gate || f.gate_stride >= (int64_t)H * V)),
              "grouped_rows_attention: two maps go without sinks and turns, with a mean over the values");
   ZP_REQUIRE(aligned16(q) && aligned16(cache) && aligned16(out) && aligned16(workspace) && aligned16(f.gate) &&

@@ -24,7 +24,7 @@ def rotary_store(proj: torch.Tensor, positions: torch.Tensor, freqs: torch.Tenso
     """proj (N, >= maps * (heads + kv_heads) * dim + kv_heads * vdim), rows may be part of wider ones: q, k, v, to
     which `bias` (fp32, one row) is added.  Rotates the first 2 * len(freqs) dimensions of every map of q's and
     k's heads (i with i + len(freqs)); [k | v] goes to the flat cache slots (-1 skips) and is returned too with
-    `return_kv`.  `form` see store_form.  Returns q (N, heads * maps * dim)."""
+    `return_kv`.  `form` see store_form.  Returns q (N, heads * maps * dim), or its rows that are stored."""
     values, heads, kv_heads = kv_heads * vdim, heads * maps, kv_heads * maps
     N, row = proj.shape[0], kv_heads * dim + values
     assert proj.stride(1) == 1 and proj.shape[1] >= heads * dim + (kv_heads * dim if form is not None and form.tied else row)
@@ -33,7 +33,8 @@ def rotary_store(proj: torch.Tensor, positions: torch.Tensor, freqs: torch.Tenso
     assert positions.numel() == slot_mapping.numel() == N and freqs.dtype == torch.float32
     assert cache.is_contiguous() and cache.dtype == proj.dtype and cache.shape[-1] == row
     assert form is None or not form.V or form.V == vdim
-    q = torch.empty((N, heads * dim), dtype=proj.dtype, device=proj.device)
+    assert form is None or not form.q_turns or (bias is None and form.held[3].shape == (freqs.numel() // 2, N, 2, 2))
+    q = torch.empty((N if form is None or not form.q_turns else form.q_rows, heads * dim), dtype=proj.dtype, device=proj.device)
     kv = torch.empty((N, row), dtype=proj.dtype, device=proj.device) if return_kv else None
     _lib.call_models("zp_rotary_store", _lib.dev_ptr(proj), _lib.dev_ptr(bias), _lib.dev_ptr(positions),
                      _lib.dev_ptr(freqs), form and C.byref(form), _lib.dev_ptr(q), _lib.dev_ptr(kv), _lib.dev_ptr(cache),
@@ -43,21 +44,24 @@ def rotary_store(proj: torch.Tensor, positions: torch.Tensor, freqs: torch.Tenso
 
 
 def store_form(norm: torch.Tensor | None = None, q_norm: int = 0, k_norm: int = 0, eps: float = 0.0, tied: bool = False,
-               value_freqs: torch.Tensor | None = None, turns: torch.Tensor | None = None):
+               value_freqs: torch.Tensor | None = None, turns: torch.Tensor | None = None,
+               q_turns: torch.Tensor | None = None, q_rows: int = 0):
     """What else a store does (zp_store_form), or None.  norm: fp32 weights of RMS norms over the whole of q and
     the whole of k, whose means run over q_norm and k_norm elements; tied: the values are the keys as projected;
     value_freqs (V / 2,) fp32: values turn too, adjacent elements a pair, and `turns` (N, V / 2, 2) fp32 receives
-    cos and sin."""
-    if norm is None and not tied and value_freqs is None:
+    cos and sin.  q_turns (rotated / 4, N, 2, 2) fp32: q is stored for the first q_rows tokens only, for the others cos
+    and sin of its angles go there (see attention_form); without norm and bias."""
+    if norm is None and not tied and value_freqs is None and q_turns is None:
         return None
+    assert q_turns is None or (q_turns.dtype == torch.float32 and q_turns.is_contiguous() and norm is None and 0 <= q_rows <= q_turns.shape[1])
     assert norm is None or (norm.dtype == torch.float32 and norm.is_contiguous())
     if value_freqs is not None:
         assert value_freqs.dtype == turns.dtype == torch.float32 and value_freqs.is_contiguous() and turns.is_contiguous()
         assert turns.shape[1:] == (value_freqs.numel(), 2)
     form = _lib.StoreForm(_lib.dev_ptr(norm) or None, q_norm, k_norm, float(eps), int(tied),
                           0 if value_freqs is None else 2 * value_freqs.numel(), _lib.dev_ptr(value_freqs) or None,
-                          _lib.dev_ptr(turns) or None)
-    form.held = (norm, value_freqs, turns)    # the form alone has their addresses
+                          _lib.dev_ptr(turns) or None, _lib.dev_ptr(q_turns) or None, q_rows)
+    form.held = (norm, value_freqs, turns, q_turns)    # the form alone has their addresses
     return form
 
 
@@ -86,6 +90,12 @@ def grouped_rows_attention(q: torch.Tensor, cache: torch.Tensor, heads: int, kv_
                      _lib.dev_ptr(out), N, heads, kv_heads, dim, vdim, BS, B, NB, pages, w, c, out.stride(0), float(scale),
                      float(out_scale), tag, _lib.dev_ptr(ws), max(size, 0), _lib.stream_ptr(q))
     return out
+
+
+def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
+    """Whether two tensors of rows may share memory."""
+    end = lambda t: t.data_ptr() + (t.shape[0] * t.stride(0) + t.shape[1]) * t.element_size()
+    return a.data_ptr() < end(b) and b.data_ptr() < end(a)
 
 
 class GroupedAttention:
@@ -141,6 +151,14 @@ class GroupedAttention:
         """Sizes the run form's kernel covers; others run token by token."""
         return self.maps * self.dim_p <= 256 and self.vdim_p <= 256
 
+    def _turns_late(self, n: int) -> bool:
+        """Whether the attention of n tokens in runs takes queries as projected (zp_attention_form.q_turns), where it can: the store
+        neither reads nor writes them then, but each head's workgroups read the angles.  From 28 MB of queries on (us before and
+        after: 32 heads over 8 of 128, all keys, 3950 tokens 102 and 96, 5900 152 and 143; 16 384, window of 1024, values that turn
+        347 and 332; 16 heads of 64, 15 800 tokens 132 and 124; but 16 heads of 128, 6000 tokens, window of 512, 62.8 and 63.9)."""
+        return n * self.heads * self.dim_p * 2 >= 28 << 20 and self.maps == 1 and not (self.qk_norm or self.has_bias or self.softcap) and \
+            self.rotary.dims in (64, 128) and self.dim_p <= 128 and self.vdim_p <= 128
+
     def shapes(self) -> dict:
         H, G, D, V = self.heads, self.kv_heads, self.dim, self.vdim
         rows = {"q": H * self.maps * D, "k": G * self.maps * D, **({} if self.tied else {"v": G * V})}
@@ -193,18 +211,21 @@ class GroupedAttention:
         direct = runs is not None and runs.key_slots is None      # the runs' keys are this step's own tokens
         sizes = (self.heads, self.kv_heads, self.dim_p, self.vdim_p)
         turns = torch.empty((N, self.vdim_p // 2, 2), dtype=torch.float32, device=proj.device) if self.turn_values else None
+        late = runs is not None and self._turns_late(N - singles) and not _overlap(proj, out)
+        q_turns = torch.empty((self.freqs.numel() // 2, N, 2, 2), dtype=torch.float32, device=proj.device) if late else None
         store = store_form(self.norm, self.heads * self.dim, self.kv_heads * self.dim, self.eps, self.tied, self.value_freqs,
-                           turns)
+                           turns, q_turns, singles)
         q = rotary_store(proj, positions, self.freqs, *sizes, cache, ctx.slot_mapping, return_kv=direct,
                          maps=self.maps, bias=self.bias, form=store)
         q, kv = q if direct else (q, None)
-        form = lambda rows: attention_form(self.softcap, self.maps, self.balance, self.eps, self.vdim,
-                                           proj[rows, self.gate_at:self.columns] if self.gated else None,
-                                           None if turns is None else turns[rows])
+        form = lambda rows, late=None: attention_form(self.softcap, self.maps, self.balance, self.eps, self.vdim,
+                                                      proj[rows, self.gate_at:self.columns] if self.gated else None,
+                                                      None if turns is None else turns[rows], late)
         if runs is not None:
             kv = kv[singles:] if direct else gather_rows(cache, runs.key_slots)
-            run_attention(q[singles:], kv, *sizes, runs.tiles, self.scale, out[singles:], sinks=self.sinks,
-                          out_scale=self.out_scale, form=form(slice(singles, N)), **self._see)
+            run_attention(proj[singles:, :self.heads * self.dim_p] if late else q[singles:], kv, *sizes, runs.tiles, self.scale,
+                          out[singles:], sinks=self.sinks, out_scale=self.out_scale,
+                          form=form(slice(singles, N), q_turns[:, singles:] if late else None), **self._see)
         if singles:
             grouped_rows_attention(q[:singles], cache, *sizes, ctx.block_tables, ctx.context_lens, self.scale,
                                    out[:singles], sinks=self.sinks, table_rows=ctx.table_rows,

@@ -9,17 +9,20 @@ from zipage_amd import _lib
 
 
 def attention_form(softcap: float = 0.0, maps: int = 1, balance: float = 0.0, eps: float = 0.0, vdim: int = 0,
-                   gate: torch.Tensor | None = None, turns: torch.Tensor | None = None):
+                   gate: torch.Tensor | None = None, turns: torch.Tensor | None = None, q_turns: torch.Tensor | None = None):
     """What an attention does beyond the softmax of scaled products (zp_attention_form), or None.  maps 2: two
     softmaxes over the same values, o = rms(o1 - balance o2) (mean over `vdim`) times sigmoid(gate).  turns (N,
-    V / 2, 2) fp32: cos and sin by which adjacent elements of every head's output turn back."""
-    if not softcap and maps == 1 and turns is None:
+    V / 2, 2) fp32: cos and sin by which adjacent elements of every head's output turn back.  q_turns (16 or 32, N, 2,
+    2) fp32: the queries of runs come as projected, and elements j and j + 32 or 64 of every head turn by these first."""
+    if not softcap and maps == 1 and turns is None and q_turns is None:
         return None
+    assert q_turns is None or (q_turns.dtype == torch.float32 and q_turns.shape[2:] == (2, 2) and q_turns.stride()[1:] == (4, 2, 1))
     assert gate is None or gate.stride(1) == 1
     assert turns is None or (turns.dtype == torch.float32 and turns.is_contiguous() and turns.shape[2] == 2)
     form = _lib.AttentionForm(float(softcap), maps, float(balance), float(eps), vdim, _lib.dev_ptr(gate) or None,
-                              0 if gate is None else gate.stride(0), _lib.dev_ptr(turns) or None)
-    form.held = (gate, turns)                 # the form alone has their addresses
+                              0 if gate is None else gate.stride(0), _lib.dev_ptr(turns) or None, _lib.dev_ptr(q_turns) or None,
+                              *((0, 0) if q_turns is None else (q_turns.stride(0) // 4, 2 * q_turns.shape[0])))
+    form.held = (gate, turns, q_turns)                 # the form alone has their addresses
     return form
 
 
