@@ -458,6 +458,36 @@ def test_experts(dev, dtype, n, E, top, groups, keep, W, ff, sff):
         _close(got, O.route(z, top, groups, keep), F32, 16.0)
 
 
+# an expert's tiles of 128 have as many rows each, in quarters; of 256 the last one of the second product is cut in quarters
+# from a half on (rows 128: 2300 / 24 rows on average; 256: more than 512)
+@pytest.mark.parametrize("K,M,counts", [(96, 64, [1, 15, 16, 17, 31, 32, 33, 48, 63, 64, 65, 80, 96, 97, 112, 113, 127, 128, 129, 143, 144, 145, 257, 294]),
+                                        (2592, 48, [513, 600, 704, 705, 960, 961, 1024, 1])])
+def test_tiles_of_experts_in_parts(dev, K, M, counts):
+    from zipage_amd.layers import Experts
+    from zipage_amd.layers.moe import Plan
+    E, n = len(counts), sum(counts)
+    ids_ = torch.cat([torch.full((c,), e, dtype=torch.int32) for e, c in enumerate(counts)])[torch.randperm(n, generator=torch.Generator().manual_seed(1))]
+    m = Experts(M, E, 1, K, 7.0)
+    w = _expert_weights(E, M, K, None, BF16)
+    m.load(w, BF16, dev)
+    p = Plan(ids_[:, None].to(dev), torch.zeros(E + 1, dtype=torch.int32, device=dev), E, False, BF16)
+    rows = [t[2] for t in p.tiles[:int(p.ntiles)].tolist()]
+    assert p.rows == (128 if K == 96 else 256) and len(rows) == sum(-(-c // p.rows) for c in counts) and sum(rows) == n
+    h, a = _rand(dev, BF16, n, m.width_p, seed=2), _rand(dev, BF16, n, K, seed=3)
+    h[:, M:] = 0
+    order = p.sorted.cpu().long()
+    act = m.gate_up_rows(h, p, torch.ones(n, 1, device=dev))
+    down = m.down_planes(a, p)[0].cpu()
+    for e in range(E):
+        at = order[ids_[order] == e]                               # positions of this expert's rows follow one another
+        first = sum(counts[:e])
+        x = h[at.to(dev), :M].double().cpu()
+        g, u = x @ w[f"e{e}.gate"].double().T, x @ w[f"e{e}.up"].double().T
+        g, u = g.clamp(max=7.0), u.clamp(-7.0, 7.0)
+        _close(act[first:first + counts[e], :K], g * torch.sigmoid(1.702 * g) * (u + 1), BF16, 2.0)
+        _close(down[at, :M], a[first:first + counts[e]].double().cpu() @ w[f"e{e}.down"].double().T, BF16, 2.0)
+
+
 # ------------------------------------------------------------------ the model
 def _engine(name, dtype, tmp, **kw):
     from zipage_amd.engine import EngineConfig, ZipageEngine, read_shape

@@ -298,13 +298,15 @@ __device__ __forceinline__ void offsets_and_tiles(const PlanArgs& a, const int* 
   int at = block_prefix(c, red);
   at = min(at, a.n * (a.top + a.shared));             // counters that were not cleared stay in bounds
   c = min(c, a.n * (a.top + a.shared) - at);
-  const int t = (c + a.rows - 1) / a.rows;
+  // no more tiles than full ones make, of as many rows each as the expert has for them
+  const int full = (c + a.rows - 1) / a.rows, per = a.rows != 128 || full < 2 ? a.rows : ((c + full - 1) / full + 15) & ~15;
+  const int t = (c + per - 1) / per;
   const int first = block_prefix(t, red);
   if (e <= a.E) {
     offsets[e] = at;
     for (int i = 0; i < t; ++i)
       if (first + i < a.max_tiles)
-        *(int4*)(a.tiles + (int64_t)(first + i) * 4) = make_int4(e, at + i * a.rows, min(a.rows, c - i * a.rows), 0);
+        *(int4*)(a.tiles + (int64_t)(first + i) * 4) = make_int4(e, at + i * per, min(per, c - i * per), 0);
     if (e == a.E) *a.ntiles = min(first + t, a.max_tiles);
   }
   __syncthreads();
@@ -535,27 +537,18 @@ __device__ __forceinline__ void settled(f32x4& acc) {
 #endif
 }
 
-// HALVES of HT 16-token tiles
-template <bool UP, int HALVES, int HT>
-__global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(ExpertArgs a) {
-  constexpr int kTiles = HT * HALVES, kOwn = kTiles / 4, kPairBytes = kTiles * 2048, kGroup = 8;
+// HALVES of HT 16-token tiles, of which the first NT are worked on: products and LDS reads of tiles that an expert has no rows for
+// are left out, and the plan gives an expert's tiles of up to 128 as many rows each (262 rows: 96, 96 and 70 instead of 128,
+// 128 and 6).  Whole layers, 3 of 32 experts and a shared one of 3 x 4096 x 3072, us: 2800 tokens 1265 -> 1090, 1900 799 -> 765,
+// 1500 814 -> 757, 3300 1237 -> 1203, 5000 1556 -> 1549; 3 x 1024 x 768, 1700 tokens 78 -> 73.  Of 256 rows: tiles are full but an
+// expert's last one, and only the second product has them in parts (16 384 tokens 1412 -> 1385; the first one, whose weights
+// take registers, 2710 -> 2760).  Dividing the launch among XCDs by such costs instead of tiles lost up to 16 %.
+template <bool UP, int HALVES, int HT, int NT>
+__device__ __forceinline__ void expert_tile(const ExpertArgs& a, char* lds_raw, const int4& t, int cb) {
+  constexpr int kTiles = HT * HALVES, kOwn = kTiles / 4, kPairBytes = kTiles * 2048;
   constexpr int kLeadW = HALVES == 2 ? 4 : 2, kLeadX = HALVES == 2 ? 3 : 2, kPairs = kLeadX + 1;      // stages, pairs ahead
-  extern __shared__ __align__(16) char lds_raw[];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g = lane >> 4;
-  // An XCD takes a contiguous share of the (tile, column block) pairs, eight tiles at a time, column block by column
-  // block, so that what is in flight on it shares rows of x and of W in its L2.
-  const int nt = *a.ntiles * a.split;
-  const int Mx = max(a.M, a.M_shared) * (UP ? 2 : 1), cols = (Mx + 16 * kBlockW - 1) / (16 * kBlockW);
-  const int share = (nt + 7) / 8 * cols, i_xcd = blockIdx.x >> 3;
-  if (i_xcd >= share) return;
-  const int lin = (blockIdx.x & 7) * share + i_xcd;
-  const int tg = lin / (kGroup * cols), rem = lin - tg * kGroup * cols;
-  const int tile = tg * kGroup + rem % kGroup, cb = rem / kGroup;
-  if (tile >= nt) return;
-  int4 t = *(const int4*)(a.tiles + (int64_t)(tile / a.split) * 4);
-  t.y += tile % a.split * kTiles * 16;                   // a part of a larger tile
-  t.z = min(t.z - tile % a.split * kTiles * 16, kTiles * 16);
-  if (t.z <= 0) return;
+  constexpr int N0 = NT < HT ? NT : HT, N1 = NT - N0;      // of the halves
   const bool shared = t.x == a.E;
   const int wtiles = (shared ? a.M_shared : a.M) / 16 * (UP ? 2 : 1), K = shared ? a.K_shared : a.K;
   const int w0 = cb * kBlockW;
@@ -571,19 +564,20 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   // a row's eight pieces of a pair lie in the order of (piece ^ row): rows of an operand don't meet in a bank
 #pragma unroll
   for (int i = 0; i < 2 * kOwn; ++i) {
-    const int r = min(wave * kOwn * 16 + i * 8 + (lane >> 3), t.z - 1);
+    const int at = wave * kOwn * 16 + i * 8 + (lane >> 3), r = min(at, t.z - 1);
     xoff[i] = (int)((UP ? a.sorted[t.y + r] / a.slots : r) * a.x_st * 2) + ((lane & 7) ^ (lane >> 3)) * 16;
+    if (at >= (t.z + 15 & ~15)) xoff[i] = -(1 << 28);      // past the end: nothing is read
   }
 #pragma unroll
   for (int i = 0; i < kWaveW; ++i) woff[i] = min(wave * kWaveW + i, wtiles - w0 - 1) * steps * 1024;
   // where this lane's results go, and their weights: asked for now, used behind the products
-  int place[kTiles];
-  float wgt[kTiles];
+  int place[NT];
+  float wgt[NT];
 #pragma unroll
-  for (int j = 0; j < kTiles; ++j) place[j] = a.sorted[t.y + min(j * 16 + l16, t.z - 1)];
+  for (int j = 0; j < NT; ++j) place[j] = a.sorted[t.y + min(j * 16 + l16, t.z - 1)];
   if constexpr (UP) {
 #pragma unroll
-    for (int j = 0; j < kTiles; ++j) {
+    for (int j = 0; j < NT; ++j) {
       const int n = place[j] / a.slots, slot = place[j] - n * a.slots;
       wgt[j] = slot < a.top ? a.weights[(int64_t)n * a.top + slot] : 1.f;
     }
@@ -620,7 +614,7 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   };
   auto read = [&](int ks, int h) {
 #pragma unroll
-    for (int j = 0; j < HT; ++j) read_tile(ks, h, j);
+    for (int j = 0; j < N0; ++j) read_tile(ks, h, j);
     __builtin_amdgcn_sched_barrier(0);
   };
   static_assert(HALVES == 1 || (kOwn == 4 && HT == 2 * kWaveW), "the waits count a wave's loads");
@@ -662,21 +656,21 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i)
 #pragma unroll
-        for (int j = 0; j < HT; ++j) {
+        for (int j = 0; j < N0; ++j) {
           mfma_in_place(acc[0][i][j], w[i], xf[0][j]);
-          if (j == HT / 2 - 1) read_tile(ks, 1, 2 * i);
-          if (j == HT - 1) read_tile(ks, 1, 2 * i + 1);
+          if (j == HT / 2 - 1 && 2 * i < N1) read_tile(ks, 1, 2 * i);
+          if (j == HT - 1 && 2 * i < N1) read_tile(ks, 1, 2 * i + 1);
           if (j == HT / 2 - 1 || j == HT - 1) __builtin_amdgcn_sched_barrier(0);
         }
       landed(odd, loop);
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
 #pragma unroll
-        for (int j = 0; j < HT; ++j) {
-          mfma_in_place(acc[1][i][j], w[i], xf[1][j]);
-          if (kAsk && j == 1) token_rows(next, odd * kOwn + i);
-          if (j == 3) read_tile(ks + 1, 0, 2 * i);
-          if (j == 5) read_tile(ks + 1, 0, 2 * i + 1);
+        for (int j = 0; j < (N1 ? N1 : 1); ++j) {
+          if constexpr (N1 > 0) mfma_in_place(acc[1][i][j], w[i], xf[1][j]);
+          if (kAsk && j == (N1 ? 1 : 0)) token_rows(next, odd * kOwn + i);
+          if (j == (N1 ? 3 : 0)) read_tile(ks + 1, 0, 2 * i);
+          if (j == (N1 > 4 ? 5 : N1 ? 3 : 0)) read_tile(ks + 1, 0, 2 * i + 1);
           if (j & 1) __builtin_amdgcn_sched_barrier(0);
         }
         if (kAsk) w[i] = weights(i, ks + kLeadW);
@@ -689,7 +683,7 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
 #pragma unroll
       for (int i = 0; i < kWaveW; ++i) {
 #pragma unroll
-        for (int j = 0; j < HT; ++j) acc[0][i][j] = mfma_bf16(w[i], xf[0][j], acc[0][i][j]);
+        for (int j = 0; j < N0; ++j) acc[0][i][j] = mfma_bf16(w[i], xf[0][j], acc[0][i][j]);
         if (kAsk) w[i] = weights(i, ks + kLeadW);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -728,7 +722,7 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   auto activated = [&](auto act) {
     const float lim = shared ? a.limit_shared : a.limit;
 #pragma unroll
-    for (int jj = 0; jj < kTiles; ++jj) {
+    for (int jj = 0; jj < NT; ++jj) {
       const int j = jj % HT, h = jj / HT, r = jj * 16 + l16;
       float v[2][4];
 #pragma unroll
@@ -744,7 +738,7 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
     return;
   }
 #pragma unroll
-  for (int jj = 0; jj < kTiles; ++jj) {
+  for (int jj = 0; jj < NT; ++jj) {
     const int j = jj % HT, h = jj / HT;
     const bool row = jj * 16 + l16 < t.z;
     const int n = place[jj] / a.slots, slot = place[jj] - n * a.slots;
@@ -755,6 +749,34 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
       store8(lo, hi, ((int64_t)slot * a.n + n) * a.o_st, own + i, out_tiles, row);
     }
   }
+}
+
+template <bool UP, int HALVES, int HT>
+__global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(ExpertArgs a) {
+  constexpr int kTiles = HT * HALVES, kGroup = 8;
+  extern __shared__ __align__(16) char lds_raw[];
+  // An XCD takes a contiguous share of the (tile, column block) pairs, eight tiles at a time, column block by column
+  // block, so that what is in flight on it shares rows of x and of W in its L2.
+  const int nt = *a.ntiles * a.split;
+  const int Mx = max(a.M, a.M_shared) * (UP ? 2 : 1), cols = (Mx + 16 * kBlockW - 1) / (16 * kBlockW);
+  const int share = (nt + 7) / 8 * cols, i_xcd = blockIdx.x >> 3;
+  if (i_xcd >= share) return;
+  const int lin = (blockIdx.x & 7) * share + i_xcd;
+  const int tg = lin / (kGroup * cols), rem = lin - tg * kGroup * cols;
+  const int tile = tg * kGroup + rem % kGroup, cb = rem / kGroup;
+  if (tile >= nt) return;
+  int4 t = *(const int4*)(a.tiles + (int64_t)(tile / a.split) * 4);
+  // a part of a larger tile
+  const int per = a.split > 1 ? ((t.z + a.split - 1) / a.split + 15) & ~15 : kTiles * 16;
+  t.y += tile % a.split * per;
+  t.z = min(t.z - tile % a.split * per, per);
+  if (t.z <= 0) return;
+  constexpr int kPart = kTiles / 4;
+  if constexpr (HALVES == 2 && UP) return expert_tile<UP, HALVES, HT, kTiles>(a, lds_raw, t, cb);
+  if (t.z > 48 * kPart) expert_tile<UP, HALVES, HT, 4 * kPart>(a, lds_raw, t, cb);
+  else if (t.z > 32 * kPart) expert_tile<UP, HALVES, HT, 3 * kPart>(a, lds_raw, t, cb);
+  else if (HALVES == 2 || t.z > 16 * kPart) expert_tile<UP, HALVES, HT, 2 * kPart>(a, lds_raw, t, cb);
+  else if constexpr (HALVES == 1) expert_tile<UP, HALVES, HT, kPart>(a, lds_raw, t, cb);
 }
 
 template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, hipStream_t st) {
