@@ -2,7 +2,8 @@
 ``include/zipage_hip.h`` and ``include/zipage_models.h``).
 
 The product path has no CPU fallback: if the shared object is missing or a symbol cannot
-be resolved, importing a kernel wrapper raises.  ctypes releases the GIL for the duration
+be resolved, importing a kernel wrapper raises.  Wrappers call through ``libzipage_calls.so``, which
+converts arguments in native code; like ctypes it releases the GIL for the duration
 of every call, so the wrappers can be driven from a worker thread while another thread
 runs the model forward (the reference calls this path from a ThreadPoolExecutor worker,
 zipage/engine/zipage_engine.py:153-166).
@@ -10,6 +11,8 @@ zipage/engine/zipage_engine.py:153-166).
 from __future__ import annotations
 
 import ctypes as C
+import importlib.machinery
+import importlib.util
 import os
 
 import torch
@@ -195,10 +198,13 @@ MODEL_LIBS = {
         "zp_moe_plan_workspace": [i32, i32, i32]}),
 }
 MODEL_EXPORTS = {lib: sorted([*calls, *sizes]) for lib, (calls, sizes) in MODEL_LIBS.items()}
-_LIB_OF = {name: lib for lib, (calls, _) in MODEL_LIBS.items() for name in calls}
+_LIB_OF = {name: lib for lib, names in MODEL_EXPORTS.items() for name in names}
 
+CALLS_PATH = os.path.join(_HERE, "libzipage_calls.so")
 _lib = None
 _models: dict[str, C.CDLL] = {}
+_calls = None
+_entries: dict = {}
 
 
 def _open(path: str, signatures: dict, i64_returning: dict) -> C.CDLL:
@@ -242,14 +248,40 @@ def _check(lib, name: str, rc: int) -> None:
         raise RuntimeError(f"{name} failed ({rc}): {lib.zp_last_error().decode()}")
 
 
+def load_calls():
+    """The module that ``csrc/calls.cpp`` becomes."""
+    global _calls
+    if _calls is None:
+        if not os.path.exists(CALLS_PATH):
+            raise RuntimeError(f"{CALLS_PATH} is missing: build it with `python -m zipage_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("zipage_calls", CALLS_PATH)
+        _calls = importlib.util.module_from_spec(importlib.util.spec_from_loader("zipage_calls", loader))
+        loader.exec_module(_calls)
+    return _calls
+
+
+def _entry(name: str, lib: C.CDLL):
+    _entries[name] = load_calls().entry(name, C.cast(getattr(lib, name), C.c_void_p).value)
+    return _entries[name]
+
+
 def call(name: str, *args) -> None:
-    lib = load()
-    _check(lib, name, getattr(lib, name)(*args))
+    """Numbers for numbers; for pointers an address, None, or a ctypes structure or array."""
+    rc = (_entries.get(name) or _entry(name, load()))(*args)
+    if rc:
+        _check(load(), name, rc)
 
 
 def call_models(name: str, *args) -> None:
-    lib = load_models(_LIB_OF[name])
-    _check(lib, name, getattr(lib, name)(*args))
+    """The same for a model-side library."""
+    rc = (_entries.get(name) or _entry(name, load_models(_LIB_OF[name])))(*args)
+    if rc:
+        _check(load_models(_LIB_OF[name]), name, rc)
+
+
+def size(name: str, *args) -> int:
+    """The same for an entry point that returns a count."""
+    return (_entries.get(name) or _entry(name, load_models(_LIB_OF[name]) if name in _LIB_OF else load()))(*args)
 
 
 def dtype_tag(t: torch.Tensor) -> int:
@@ -260,11 +292,10 @@ def dtype_tag(t: torch.Tensor) -> int:
 
 
 def dev_ptr(t) -> int:
-    if t is None:
-        return 0
-    if not t.is_cuda:
-        raise RuntimeError("the compression kernels need device tensors (no CPU fallback)")
-    return t.data_ptr()
+    """Address of a device tensor, 0 of None."""
+    global dev_ptr
+    dev_ptr = load_calls().pointer
+    return dev_ptr(t)
 
 
 def stream_ptr(t: torch.Tensor) -> int:

@@ -4,7 +4,8 @@ Run as ``python -m zipage_amd.build``.  Shared objects with a plain C ABI, none 
 torch: ``libzipage_hip.so`` (``include/zipage_hip.h``: the compression path and the kernels of the
 models that use it) and, for the other models, ``libzipage_models.so``, ``libzipage_latent.so``,
 ``libzipage_grouped.so``, ``libzipage_recurrent.so``, ``libzipage_linear.so`` and ``libzipage_moe.so``
-(``include/zipage_models.h``), so that a model compiles only what it runs.
+(``include/zipage_models.h``), so that a model compiles only what it runs.  ``libzipage_calls.so``
+makes Python functions of their entry points.
 """
 from __future__ import annotations
 
@@ -12,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
@@ -22,6 +24,7 @@ GROUPED_LIB = os.path.join(HERE, "libzipage_grouped.so")
 RECURRENT_LIB = os.path.join(HERE, "libzipage_recurrent.so")
 LINEAR_LIB = os.path.join(HERE, "libzipage_linear.so")
 MOE_LIB = os.path.join(HERE, "libzipage_moe.so")
+CALLS_LIB = os.path.join(HERE, "libzipage_calls.so")      # host code
 
 # packed fp32 VALU ops are disabled on purpose (some forms misbehave on this fleet)
 BASE_FLAGS = [
@@ -42,7 +45,7 @@ MODEL_SOURCES = {
     MOE_LIB: ("moe.hip",),
 }
 COMMON_SOURCES = ("runtime.hip",)
-LIBS = (LIB, *MODEL_SOURCES)
+LIBS = (LIB, *MODEL_SOURCES, CALLS_LIB)
 
 
 def sources(lib: str = LIB) -> list[str]:
@@ -73,6 +76,11 @@ def build(verbose: bool = True, jobs: int | None = None, libs: tuple[str, ...] =
     extra = os.environ.get("ZP_EXTRA_HIPCC_FLAGS", "").split()
     work, links = [], []
     for lib in libs:
+        if lib == CALLS_LIB:
+            work.append([shutil.which("g++") or hipcc, "-O2", "-std=c++17", "-fPIC", "-shared", "-I" + sysconfig.get_path("include"),
+                         os.path.join(CSRC, "calls.cpp"), "-o", lib + ".tmp"])
+            links.append((lib, None))
+            continue
         models = lib in MODEL_SOURCES
         objdir = os.path.join(HERE, "build", os.path.basename(lib)[len("libzipage_"):-3] if models else "")
         os.makedirs(objdir, exist_ok=True)
@@ -86,13 +94,15 @@ def build(verbose: bool = True, jobs: int | None = None, libs: tuple[str, ...] =
     with ThreadPoolExecutor(max_workers=jobs) as pool:
         list(pool.map(lambda cmd: _run(cmd, verbose), work))
     for lib, objs in links:
-        _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", lib + ".tmp"], verbose)
+        if objs is not None:
+            _run([hipcc, "--offload-arch=gfx950", "-shared", "-fPIC", *objs, "-o", lib + ".tmp"], verbose)
         os.replace(lib + ".tmp", lib)
     return libs[0]
 
 
 def ensure(*libs: str) -> None:
-    """Build those of ``libs`` that are not there yet (one process at a time)."""
+    """Build those of ``libs``, and what calls them, that are not there yet (one process at a time)."""
+    libs = (*libs, CALLS_LIB)
     if not all(os.path.exists(lib) for lib in libs):
         import fcntl
         os.makedirs(os.path.join(HERE, "build"), exist_ok=True)

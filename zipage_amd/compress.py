@@ -268,9 +268,8 @@ def _compress_layers_one_call(k_cache, v_cache, query_cache, score_cache, query_
     if flag.numel() == 0:
         return flag
     cc = c_config(cfg, deterministic_carry)
-    lib = _lib.load()
     tag = _lib.dtype_tag(k_cache)
-    ws_bytes = lib.zp_compress_layers_workspace_few(L, B, NB, BS, Hkv, Hq, W, tag, ctypes.byref(cc), 0)
+    ws_bytes = _lib.size("zp_compress_layers_workspace_few", L, B, NB, BS, Hkv, Hq, W, tag, cc, 0)
     ws = torch.empty(ws_bytes, device=k_cache.device, dtype=torch.uint8)
     running = {"attention_score", FUSED_SELECT_STAGE, "compress_kv"}
     if cfg.use_global_score:
@@ -283,5 +282,5 @@ def _compress_layers_one_call(k_cache, v_cache, query_cache, score_cache, query_
               _lib.dev_ptr(query_cache), _lib.dev_ptr(score_cache), _lib.dev_ptr(query_ids),
               _lib.dev_ptr(block_tables), _lib.dev_ptr(compressed),
               _lib.dev_ptr(target_block_tables), _lib.dev_ptr(flag), *dims, strides, tag,
-              ctypes.byref(cc), _lib.dev_ptr(ws), ws_bytes, events, _lib.stream_ptr(k_cache))
+              cc, _lib.dev_ptr(ws), ws_bytes, events, _lib.stream_ptr(k_cache))
     return flag

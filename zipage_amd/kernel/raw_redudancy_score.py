@@ -22,8 +22,7 @@ def raw_redudancy_score(key_cache: torch.Tensor, block_table: torch.Tensor,
     logits = torch.empty((L, B, Hkv, NB * BS), device=dev, dtype=dt) if return_logits else None
     if red.numel() == 0:
         return (logits, red) if return_logits else red
-    lib = _lib.load()
-    ws_bytes = lib.zp_redundancy_raw_workspace(L, B, NB, BS, Hkv)
+    ws_bytes = _lib.size("zp_redundancy_raw_workspace", L, B, NB, BS, Hkv)
     ws = torch.empty(ws_bytes, device=dev, dtype=torch.uint8) if ws_bytes else None
     _lib.call("zp_redundancy_raw", _lib.dev_ptr(key_cache), _lib.dev_ptr(block_table),
               _lib.dev_ptr(red), _lib.dev_ptr(logits), L, B, NB, BS, Hkv, D, num_pages,

@@ -5,7 +5,6 @@ wants (`project`), is handed the columns of the common product, and writes its p
 output rows."""
 from __future__ import annotations
 
-import ctypes as C
 import math
 
 import torch
@@ -37,7 +36,7 @@ def rotary_store(proj: torch.Tensor, positions: torch.Tensor, freqs: torch.Tenso
     q = torch.empty((N if form is None or not form.q_turns else form.q_rows, heads * dim), dtype=proj.dtype, device=proj.device)
     kv = torch.empty((N, row), dtype=proj.dtype, device=proj.device) if return_kv else None
     _lib.call_models("zp_rotary_store", _lib.dev_ptr(proj), _lib.dev_ptr(bias), _lib.dev_ptr(positions),
-                     _lib.dev_ptr(freqs), form and C.byref(form), _lib.dev_ptr(q), _lib.dev_ptr(kv), _lib.dev_ptr(cache),
+                     _lib.dev_ptr(freqs), form, _lib.dev_ptr(q), _lib.dev_ptr(kv), _lib.dev_ptr(cache),
                      _lib.dev_ptr(slot_mapping), N, heads, kv_heads, dim, values, 2 * freqs.numel(), proj.stride(0), cache.numel() // row,
                      _lib.dtype_tag(proj), _lib.stream_ptr(proj))
     return (q, kv) if return_kv else q
@@ -83,10 +82,10 @@ def grouped_rows_attention(q: torch.Tensor, cache: torch.Tensor, heads: int, kv_
     B, NB = block_tables.shape
     pages, BS, _ = cache.shape
     w, c, tag = window or 0, chunk or 0, _lib.dtype_tag(q)
-    size = _lib.load_models("grouped").zp_grouped_rows_workspace(N, heads, kv_heads, dim, vdim, maps, w, c, NB, BS, tag)
+    size = _lib.size("zp_grouped_rows_workspace", N, heads, kv_heads, dim, vdim, maps, w, c, NB, BS, tag)
     ws = torch.empty(size, dtype=torch.uint8, device=q.device) if size > 0 else None
     _lib.call_models("zp_grouped_rows_attention", _lib.dev_ptr(q), _lib.dev_ptr(cache), _lib.dev_ptr(block_tables),
-                     _lib.dev_ptr(context_lens), _lib.dev_ptr(table_rows), _lib.dev_ptr(sinks), form and C.byref(form),
+                     _lib.dev_ptr(context_lens), _lib.dev_ptr(table_rows), _lib.dev_ptr(sinks), form,
                      _lib.dev_ptr(out), N, heads, kv_heads, dim, vdim, BS, B, NB, pages, w, c, out.stride(0), float(scale),
                      float(out_scale), tag, _lib.dev_ptr(ws), max(size, 0), _lib.stream_ptr(q))
     return out

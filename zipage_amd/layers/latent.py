@@ -91,7 +91,7 @@ def latent_rows_attention(q: torch.Tensor, cache: torch.Tensor, block_tables: to
     B, NB = block_tables.shape
     pages, BS, _ = cache.shape
     w, tag = window or 0, _lib.dtype_tag(q)
-    size = _lib.load_models("latent").zp_latent_rows_workspace(N, H, R, w, NB, BS, tag)
+    size = _lib.size("zp_latent_rows_workspace", N, H, R, w, NB, BS, tag)
     ws = torch.empty(max(size, 0), dtype=torch.uint8, device=q.device) if size > 0 else None
     out = torch.empty((N, H, R), dtype=q.dtype, device=q.device)
     _lib.call_models("zp_latent_rows_attention", _lib.dev_ptr(q), _lib.dev_ptr(cache),

@@ -3,8 +3,6 @@ linear attention with decay.  All keep a float32 matrix per head and sequence sl
 segments (`StepContext.segments`, and `.run_segments` where 16 tokens at a time pay)."""
 from __future__ import annotations
 
-import ctypes
-
 import torch
 
 from zipage_amd import _lib
@@ -93,12 +91,11 @@ class MatrixMemory:
                 _lib.dev_ptr(out), proj.stride(0), gates.stride(0), out.stride(0), H, D, V, self.vdim, 0, H * D,
                 2 * H * D, 2 * H * D + H * V, self.gate_cap, self.dim ** -0.5, self.eps, self.out_scale)
             if not runs:
-                _lib.call_models("zp_mlstm_scan", ctypes.byref(args), tag, stream)
+                _lib.call_models("zp_mlstm_scan", args, tag, stream)
                 continue
-            size = _lib.load_models("recurrent").zp_mlstm_runs_workspace(h.shape[0] - segments.first_row,
-                                                                      segments.counts.numel(), H)
+            size = _lib.load_models("recurrent").zp_mlstm_runs_workspace(h.shape[0] - segments.first_row, segments.counts.numel(), H)
             ws = torch.empty(size, dtype=torch.uint8, device=proj.device)
-            _lib.call_models("zp_mlstm_runs", ctypes.byref(args), segments.first_row, segments.longest, _lib.dev_ptr(ws),
+            _lib.call_models("zp_mlstm_runs", args, segments.first_row, segments.longest, _lib.dev_ptr(ws),
                              size, tag, stream)
 
 
@@ -179,12 +176,11 @@ class ChannelDelta:
                 self.kv_heads, D, self.vdim_p, self.vdim, self.taps, self.b_at, H * D, self.dim ** -0.5, self.eps,
                 self.out_scale)
             if not runs:
-                _lib.call_models("zp_delta_scan", ctypes.byref(args), tag, stream)
+                _lib.call_models("zp_delta_scan", args, tag, stream)
                 continue
-            size = _lib.load_models("recurrent").zp_delta_runs_workspace(proj.shape[0] - segments.first_row,
-                                                                      segments.counts.numel(), H, D, self.vdim_p)
+            size = _lib.load_models("recurrent").zp_delta_runs_workspace(proj.shape[0] - segments.first_row, segments.counts.numel(), H, D, self.vdim_p)
             ws = torch.empty(size, dtype=torch.uint8, device=proj.device)
-            _lib.call_models("zp_delta_runs", ctypes.byref(args), segments.first_row, segments.longest,
+            _lib.call_models("zp_delta_runs", args, segments.first_row, segments.longest,
                              _lib.dev_ptr(ws), size, tag, stream)
 
 
@@ -262,10 +258,9 @@ class LinearAttention:
                 0 if self.freqs is None else 2 * self.freqs.numel(), 0, H * D, 2 * H * D, 2 * H * D + H * V, self.q_scale,
                 self.k_scale, 0.0 if self.tau is None else 1.0 / self.tau, self.eps)
             if not runs:
-                _lib.call_models("zp_linear_scan", ctypes.byref(args), tag, stream)
+                _lib.call_models("zp_linear_scan", args, tag, stream)
                 continue
-            size = _lib.load_models("linear").zp_linear_runs_workspace(proj.shape[0] - segments.first_row,
-                                                                    segments.counts.numel(), H, D)
+            size = _lib.load_models("linear").zp_linear_runs_workspace(proj.shape[0] - segments.first_row, segments.counts.numel(), H, D)
             ws = torch.empty(size, dtype=torch.uint8, device=proj.device)
-            _lib.call_models("zp_linear_runs", ctypes.byref(args), segments.first_row, segments.longest, _lib.dev_ptr(ws),
+            _lib.call_models("zp_linear_runs", args, segments.first_row, segments.longest, _lib.dev_ptr(ws),
                              size, tag, stream)

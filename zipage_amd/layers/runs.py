@@ -1,8 +1,6 @@
 """Attention of runs of prompt tokens, and the gather of the cached rows they look back on."""
 from __future__ import annotations
 
-import ctypes as C
-
 import torch
 
 from zipage_amd import _lib
@@ -53,7 +51,7 @@ def run_attention(q: torch.Tensor, kv: torch.Tensor, heads: int, kv_heads: int, 
     assert sinks is None or (sinks.dtype == torch.float32 and sinks.numel() == heads)
     v = kv[:, kv_heads * maps * dim:]
     _lib.call_models("zp_run_attention", _lib.dev_ptr(q), _lib.dev_ptr(kv), v.data_ptr(), _lib.dev_ptr(shared),
-                     _lib.dev_ptr(out), _lib.dev_ptr(tiles), _lib.dev_ptr(sinks), form and C.byref(form),
+                     _lib.dev_ptr(out), _lib.dev_ptr(tiles), _lib.dev_ptr(sinks), form,
                      tiles.shape[0], heads, kv_heads, dim, extra, vdim, window or 0, chunk or 0, q.shape[0],
                      kv.shape[0], q.stride(0), kv.stride(0), 0 if shared is None else shared.stride(0), out.stride(0), float(scale), float(out_scale), _lib.dtype_tag(q), _lib.stream_ptr(q))
     return out
