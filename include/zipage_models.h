@@ -69,6 +69,9 @@ int zp_gather_rows(const void* src, const int32_t* rows, void* out, int32_t n, i
 /* out (n, M) = x (n, K) w^T, w (M, K) contiguous, sums in fp32: 16-bit, up to 64 rows, K a multiple of 32, M of 4. */
 int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
                        int64_t out_stride, int32_t dtype, void* stream);
+/* The same for up to 256 rows. */
+int zp_row_tiles_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                        int64_t out_stride, int32_t dtype, void* stream);
 
 /* What an attention does beyond the softmax of scaled products; NULL stands for {0, 1}.
  * softcap > 0: scores s (after the scale) enter the softmax as softcap * tanh(s / softcap).

@@ -324,6 +324,28 @@ def test_products_of_few_rows(dev, dtype, n, K, M):
     assert bool(((out[:, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
 
 
+# up to 256 rows: each of the four tile sizes at the most outputs that make 256 workgroups with it and at more; rows that leave one,
+# 33 and 63 of a tile of 64; a contraction of less than a stage, and of one step more than whole stages
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+@pytest.mark.parametrize("n", [65, 97, 127, 128, 193, 256])
+@pytest.mark.parametrize("K,M", [(96, 4), (128, 340), (160, 2048), (1056, 4100), (1312, 1364), (2048, 516), (384, 8196)])
+def test_products_of_row_tiles(dev, dtype, n, K, M):
+    from zipage_amd import _lib
+    wide = _rand(n, K + 24, seed=1, dtype=dtype).to(dev)
+    x, w = wide[:, 8:8 + K], (_rand(M, K, seed=2).float() * K ** -0.5).to(dtype).to(dev)
+    out = torch.full((n + 1, M + 4), 7.0, dtype=dtype, device=dev)
+    args = (K, M, x.stride(0), out.stride(0), _lib.dtype_tag(x), _lib.stream_ptr(x))
+    _lib.call_models("zp_row_tiles_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, *args)
+    assert bool((out[:n, M:] == 7).all()) and bool((out[n:] == 7).all())
+    want = x.double() @ w.double().T                           # bounds as for few rows
+    bits = 2.0 ** (-8 if dtype == BF16 else -11)
+    assert bool(((out[:n, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
+    with pytest.raises(RuntimeError, match="at most 256"):
+        _lib.call_models("zp_row_tiles_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), 257, *args)
+    with pytest.raises(RuntimeError, match="at most 64"):
+        _lib.call_models("zp_few_rows_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, *args)
+
+
 @pytest.fixture
 def few_rows_calls(monkeypatch):
     """Says whether the kernel for few rows was called since it last did."""

@@ -94,3 +94,14 @@ def test_device_tensors_without_storage(dtype):
 def test_which_sizes_are_few_rows(n, k, m, few):
     from zipage_amd.layers.linear import _few_rows
     assert _few_rows(n, k, m) == few
+
+
+@pytest.mark.parametrize("n,k,m,tiles", [(64, 1024, 1024, False), (65, 1024, 1024, True), (256, 1024, 1024, True), (257, 1024, 1024, False),
+                                         (65, 64, 1024, False), (65, 96, 1024, True), (128, 1024, 8192, True), (128, 1024, 8196, False),
+                                         (129, 1024, 5440, True), (129, 1024, 5444, False), (256, 1024, 4096, True), (256, 1056, 4096, False),
+                                         (256, 1056, 2048, True), (128, 2048, 8192, True), (128, 2080, 4096, True), (128, 2080, 4128, False),
+                                         (96, 2080, 4096, False), (129, 2080, 1024, False), (112, 4096, 4096, False), (113, 4096, 4096, True),
+                                         (128, 4128, 1024, False), (100, 48, 64, False), (100, 128, 66, False), (100, 144, 64, False)])
+def test_which_sizes_are_row_tiles(n, k, m, tiles):
+    from zipage_amd.layers.linear import _few_rows, _row_tiles
+    assert _row_tiles(n, k, m) == tiles and not (_row_tiles(n, k, m) and _few_rows(n, k, m))

@@ -4,6 +4,7 @@
 
 namespace {
 
+constexpr int kCUs = 256;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 template <typename T> __device__ __forceinline__ f32x4 product(const u32x4& w, const u32x4& x, const f32x4& c);
 template <> __device__ __forceinline__ f32x4 product<BF16>(const u32x4& w, const u32x4& x, const f32x4& c) { return mfma_bf16(w, x, c); }
@@ -19,7 +20,7 @@ struct FewArgs {
   int64_t x_st, o_st;
 };
 
-// 16 * TT rows of x and 16 * MT of W per workgroup, four waves that share the contraction.  Both pass through LDS in stages of
+// 16 * TT rows of x (tiles of them side by side, which share W in the L2) and 16 * MT of W per workgroup, four waves that share the contraction.  Both pass through LDS in stages of
 // 128 elements of every row, a step of 32 for each wave: loads of whole cache lines, for the L1 takes four to five cycles for
 // every line touched, whole or in part.  A row's sixteen pieces lie in the order of (piece ^ row).  Bound by the weights'
 // stream: what counts is bytes in flight, so the ring takes what LDS there is, for two workgroups where the tiles are small.
@@ -28,7 +29,7 @@ struct FewArgs {
 // (13.4); 48 rows, 1024 -> 4096 6.6 (11.4), 3072 -> 1024 11.2 (11.7); errors the same.  The caller's rule has where it is slower.
 template <int TT, int MT> struct FewTile {
   static constexpr int kLoads = TT + MT, kBytes = kLoads * 4096;       // of a wave; of a stage
-  static constexpr int kRing = kLoads <= 2 ? 9 : kLoads == 3 ? 6 : kLoads == 4 ? 9 : kLoads == 5 ? 7 : 6;
+  static constexpr int kRing = kLoads <= 2 ? 9 : kLoads == 3 ? 6 : kLoads == 4 ? 9 : kLoads == 5 ? 7 : kLoads == 6 ? 6 : 5;
 };
 template <typename T, int TT, int MT>
 __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
@@ -38,15 +39,16 @@ __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
   static_assert((R - 2) * L < 64, "loads that a wait can count");
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int m0 = blockIdx.x * 16 * MT, steps = a.K / 32, stages = (steps + 3) / 4;
+  const int row_tiles = (a.n + 16 * TT - 1) / (16 * TT), n0 = (int)(blockIdx.x % row_tiles) * 16 * TT, rows = min(16 * TT, a.n - n0);
+  const int m0 = (int)(blockIdx.x / row_tiles) * 16 * MT, steps = a.K / 32, stages = (steps + 3) / 4;
   const int x_row = (int)a.x_st * 2;                     // bytes
-  const u32x4 xr = rows_from(a.x, (uint32_t)(a.n - 1) * x_row + a.K * 2);
+  const u32x4 xr = rows_from(a.x + n0 * a.x_st, (uint32_t)(rows - 1) * x_row + a.K * 2);
   const u32x4 wr = rows_from(a.w + (int64_t)m0 * a.K, (uint32_t)min(16 * MT, a.M - m0) * a.K * 2);
   int from[L];                                           // of four rows a load; what is not there lies past the end
 #pragma unroll
   for (int i = 0; i < L; ++i) {
     const int at = wave * L + i, row = at * 4 + g, r = at < 4 * MT ? row : row - 16 * MT;
-    const bool there = at < 4 * MT ? m0 + r < a.M : r < a.n;
+    const bool there = at < 4 * MT ? m0 + r < a.M : r < rows;
     from[i] = (there ? r * (at < 4 * MT ? a.K * 2 : x_row) : INT_MIN) + (l16 ^ (row & 15)) * 16;
   }
   auto issue = [&](int s) {                              // past the last stage zeros come, so that the count stays
@@ -98,7 +100,7 @@ __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
     f32x4 y = red[id * 256 + lane];
 #pragma unroll
     for (int k = 1; k < 4; ++k) y += red[id * 256 + k * 64 + lane];
-    const int n = t * 16 + l16, m = m0 + j * 16 + g * 4;
+    const int n = n0 + t * 16 + l16, m = m0 + j * 16 + g * 4;
     if (n >= a.n || m >= a.M) continue;
     uint2 o;
     if constexpr (std::is_same<T, BF16>::value) {
@@ -119,7 +121,7 @@ template <typename T, int TT, int MT> int launch_few(const FewArgs& a, hipStream
     zp_set_error("few_rows_linear: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((few_rows_kernel<T, TT, MT>), dim3((unsigned)((a.M + 16 * MT - 1) / (16 * MT))), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((few_rows_kernel<T, TT, MT>), dim3((unsigned)((a.M + 16 * MT - 1) / (16 * MT) * ((a.n + 16 * TT - 1) / (16 * TT)))), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -138,20 +140,39 @@ template <typename T> int launch_few(const FewArgs& a, hipStream_t st) {
   if (a.n <= 16) return launch_few<T, 1>(a, st);
   return a.n <= 32 ? launch_few<T, 2>(a, st) : launch_few<T, 4>(a, st);
 }
+// More than 64 rows: the smallest tiles that make at most a workgroup per CU.  Weights from memory, us (the library): 128 rows,
+// 1024 -> 4096 7.8 (12.3), 2048 -> 1024 6.5 (8.5), 1024 -> 6144 9.8 (12.6), 512 -> 2048 5.2 (7.9), 4096 -> 4096 18.2 (23.6); 256 rows, 1024
+// -> 4096 10.1 (11.9), 512 -> 3072 7.4 (9.0), 1024 -> 768 6.0 (8.1), 128 -> 4096 5.5 (5.5).
+template <typename T> int launch_row_tiles(const FewArgs& a, hipStream_t st) {
+  const auto groups = [&](int rows, int outs) { return (int64_t)((a.n + rows - 1) / rows) * ((a.M + outs - 1) / outs); };
+  if (groups(32, 16) <= kCUs) return launch_few<T, 2, 1>(a, st);
+  if (groups(32, 32) <= kCUs) return launch_few<T, 2, 2>(a, st);
+  if (groups(64, 32) <= kCUs) return launch_few<T, 4, 2>(a, st);
+  return launch_few<T, 4, 4>(a, st);
+}
 
 }  // namespace
 
-extern "C" int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
-                                  int64_t out_stride, int32_t dtype, void* stream) {
-  ZP_REQUIRE(n >= 0 && K > 0 && M > 0 && x_stride >= K && out_stride >= M, "few_rows_linear: bad dims");
-  if ((dtype != ZP_BF16 && dtype != ZP_F16) || n > 64 || K % 32 || M % 4 || x_stride % 8 || out_stride % 4 ||
+static int few_linear(const char* name, int most, const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                      int64_t out_stride, int32_t dtype, hipStream_t st) {
+  ZP_REQUIRE(n >= 0 && K > 0 && M > 0 && x_stride >= K && out_stride >= M, "%s: bad dims", name);
+  if ((dtype != ZP_BF16 && dtype != ZP_F16) || n > most || K % 32 || M % 4 || x_stride % 8 || out_stride % 4 ||
       x_stride > (1 << 23) || K > (1 << 23)) {
-    zp_set_error("few_rows_linear: 16-bit, %d rows (at most 64) of %d elements (a multiple of 32), %d outputs (a multiple of 4) unsupported",
-                 n, K, M);
+    zp_set_error("%s: 16-bit, %d rows (at most %d) of %d elements (a multiple of 32), %d outputs (a multiple of 4) unsupported",
+                 name, n, most, K, M);
     return ZP_EUNSUPPORTED;
   }
   if (n == 0) return ZP_OK;
-  ZP_REQUIRE(x && w && out && aligned16(x) && aligned16(w) && ((uintptr_t)out & 7) == 0, "few_rows_linear: null or unaligned pointer");
+  ZP_REQUIRE(x && w && out && aligned16(x) && aligned16(w) && ((uintptr_t)out & 7) == 0, "%s: null or unaligned pointer", name);
   const FewArgs a = {(const uint16_t*)x, (const uint16_t*)w, (uint16_t*)out, n, K, M, x_stride, out_stride};
-  return dtype == ZP_BF16 ? launch_few<BF16>(a, (hipStream_t)stream) : launch_few<F16>(a, (hipStream_t)stream);
+  if (n <= 64) return dtype == ZP_BF16 ? launch_few<BF16>(a, st) : launch_few<F16>(a, st);
+  return dtype == ZP_BF16 ? launch_row_tiles<BF16>(a, st) : launch_row_tiles<F16>(a, st);
+}
+extern "C" int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                                  int64_t out_stride, int32_t dtype, void* stream) {
+  return few_linear("few_rows_linear", 64, x, w, out, n, K, M, x_stride, out_stride, dtype, (hipStream_t)stream);
+}
+extern "C" int zp_row_tiles_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                                   int64_t out_stride, int32_t dtype, void* stream) {
+  return few_linear("row_tiles_linear", 256, x, w, out, n, K, M, x_stride, out_stride, dtype, (hipStream_t)stream);
 }

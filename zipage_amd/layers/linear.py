@@ -47,6 +47,21 @@ def _few_rows(n: int, k: int, m: int) -> bool:
     return n <= 64 and m * k <= 1 << 23 and m <= 8192 and (96 <= k <= 1024 or 512 <= m and 1024 < k <= 2048 or 512 <= m <= 1280 and 2048 < k <= 4096)
 
 
+def _row_tiles(n: int, k: int, m: int) -> bool:
+    """The same for 65 to 256 rows, in tiles of up to 64 x 64: what makes one round of workgroups, over contractions that are not much
+    longer than their beginning and end (us of both: 65 to 128 rows, 1024 -> 4096 7.7 and 12.0, 2048 -> 1024 6.5 and 8.3, 2048 -> 4096
+    11.4 and 12.8, 128 -> 2048 4.1 and 4.0; 129 to 256, 1024 -> 4096 9.8 and 12.4, 2048 -> 2048 10.5 and 11.8).  The largest tiles for
+    short ones, since a CU has one workgroup with them (256 rows, 1536 -> 4096 12.7 and 11.2, 2048 -> 4096 18.1 and 13.2); longer
+    contractions up to 128 rows, where the library's tiles leave most of the chip idle (128 rows, 4096 -> 4096 18.2 and 23.5, 3072 ->
+    4096 14.9 and 20.2; 100 rows 17.7 and 16.5, 13.6 and 16.5; 4096 -> 6144 25.4 and 25.3)."""
+    if not 64 < n <= 256 or k % 32 or m % 4 or k < 96:
+        return False
+    tiles = lambda outs: -(-n // 64) * -(-m // outs)
+    if tiles(32) > 256 and (tiles(64) > 256 or k > (2048 if n <= 128 else 1024)):
+        return False
+    return k <= 2048 or n <= 128 and (n > 96 and k <= 3072 or n > 112 and k <= 4096)
+
+
 def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether something beside the product looks at the call, which only the library's passes through torch's dispatcher:
     gradients of either mode, vmap and its like, autocast, modes, subclasses, tracing and compilation; or another device than the current
@@ -60,12 +75,12 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) without a bias."""
     if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 == w.dim() and x.layout == w.layout == torch.strided:
         (n, k), (m, wk), (stride, one) = x.shape, w.shape, x.stride()
-        if k == wk and x.dtype == w.dtype in _FEW_TYPES and _few_rows(n, k, m) and one == 1 and k <= stride <= 1 << 23 and \
-                stride % 8 == 0 and w.is_contiguous() and w.device == x.device:
+        if k == wk and x.dtype == w.dtype in _FEW_TYPES and (_few_rows(n, k, m) or _row_tiles(n, k, m)) and one == 1 and \
+                k <= stride <= 1 << 23 and stride % 8 == 0 and w.is_contiguous() and w.device == x.device:
             at, w_at = x.data_ptr(), w.data_ptr()
             if (at | w_at) % 16 == 0:
                 out = x.new_empty(n, m)
-                _lib.call_models("zp_few_rows_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, _lib.dtype_tag(x), _lib.stream_ptr(x))
+                _lib.call_models("zp_few_rows_linear" if n <= 64 else "zp_row_tiles_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, _lib.dtype_tag(x), _lib.stream_ptr(x))
                 return out
     return F.linear(x, w)
 
