@@ -397,6 +397,31 @@ def test_products_of_few_rows_keep_tangents(dev, few_rows_calls):
     assert torch.equal(got, torch.nn.functional.linear(t, w)) and not few_rows_calls()
 
 
+# ------------------------------------------------------------------ raw redundancy of few sequences
+# pages of few sequences are worked on in parts (five, three, two; the claims' in eight and four), of twelve whole: the same bits.  Odd and
+# even numbers of pages, padding, near copies of keys in their own page, in others and across the parts' edges
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+@pytest.mark.parametrize("BS,pages", [(128, (9, 9, 8, 9)), (256, (3, 4, 4, 1)), (384, (2, 1, 2, 2))])
+def test_raw_redundancy_in_parts(dev, dtype, BS, pages):
+    from zipage_amd.kernel import raw_redudancy_score
+    B, G, D = 12, 8, 64
+    g = torch.Generator().manual_seed(BS)
+    lens = [pages[b % 4] for b in range(B)]
+    order = iter(torch.randperm(sum(lens), generator=g).tolist())
+    enc = O.encode_block_table([[next(order) for _ in range(n)] for n in lens])
+    keys = torch.randn(sum(lens) * BS, G, D, generator=g)
+    copies = torch.randint(0, len(keys), (2, len(keys) // 4), generator=g)
+    keys[copies[0]] = keys[copies[1]] + 0.3 * torch.randn(len(keys) // 4, G, D, generator=g)
+    keys[BS:BS + 30] = keys[:30]
+    k = keys.view(1, sum(lens), BS, G, D).to(dtype).to(dev)
+    logits, red = raw_redudancy_score(k, enc.to(dev), threshold=0.5, temperature=0.4, return_logits=True)
+    assert bool(torch.isfinite(logits).any())
+    for first, n in ((0, 1), (1, 1), (3, 1), (0, 2), (2, 2), (1, 3), (4, 4), (0, 8)):
+        few = enc[first:first + n].contiguous().to(dev)
+        a, b = raw_redudancy_score(k, few, threshold=0.5, temperature=0.4, return_logits=True)
+        assert torch.equal(a.view(1, n, G, -1), logits.view(1, B, G, -1)[:, first:first + n]) and torch.equal(b, red[:, first:first + n]), (first, n)
+
+
 # ------------------------------------------------------------------ recurrences over runs, in pieces
 # Few heads walk long runs in pieces of at least four blocks of 16 tokens: one run, runs of which some have fewer pieces than
 # others or none, pieces whose last has one token or a whole block, states of earlier tokens and none; key and value sizes

@@ -154,7 +154,7 @@ struct GramArgs {
   int B, NB, BS, Hkv, D, num_pages;
   int64_t k_sl, k_sp;
   float threshold, eps;
-  int parts;       // the page kernels: workgroups per row; each walks every parts-th entry of its block table
+  int parts;       // the page kernels: workgroups per row; each walks every parts-th entry of its block table.  All pairs, 16 bit: per page
 };
 
 template <typename T, bool RAW, int NW>
@@ -1917,10 +1917,11 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, col = lane & 31;
-  const int jp = blockIdx.x % p.NB;
-  const int h = (blockIdx.x / p.NB) % p.Hkv;
-  const int b = (blockIdx.x / (p.NB * p.Hkv)) % p.B;
-  const int l = blockIdx.x / (p.NB * p.Hkv * p.B);
+  const unsigned pages = gridDim.x / p.parts, page = blockIdx.x % pages, part = blockIdx.x / pages;
+  const int jp = page % p.NB;
+  const int h = (page / p.NB) % p.Hkv;
+  const int b = (page / (p.NB * p.Hkv)) % p.B;
+  const int l = page / (p.NB * p.Hkv * p.B);
   const int Tn = p.NB * p.BS;
   const int64_t obase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
 
@@ -1939,7 +1940,7 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int nv = nvalid_s, ia = mine_s;
   const int nd = nv / 2 + (((nv & 1) || ia < nv / 2) ? 1 : 0);   // page distances 0 .. nd-1
   const int tiles_per_page = p.BS / TNc;
-  const int ntiles = nd * tiles_per_page;
+  const int from = nd * tiles_per_page * part / p.parts, to = nd * tiles_per_page * (part + 1) / p.parts;   // its tiles
   const int k_row = p.Hkv * p.D * 2;
   const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2;
   const float* rn_all = p.ws_val + obase;           // written by raw_prep_kernel
@@ -2019,8 +2020,8 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dcol0[r] = -1; dcol1[r] = -1; }
 
-    if (ntiles > 0) request(0, buf0);
-    for (int tile = 0; tile < ntiles; ++tile) {
+    if (from < to) request(from, (from & 1) ? buf1 : buf0);
+    for (int tile = from; tile < to; ++tile) {
       char* cur = (tile & 1) ? buf1 : buf0;
       char* nxt = (tile & 1) ? buf0 : buf1;
       // this wave's share of the tile (and its A fragments, the first time) has landed; after the
@@ -2028,8 +2029,8 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       if (tid < TNc) l_rn[(tile & 1) * TNc + tid] = pre_rn;
       __syncthreads();
-      if (tile + 1 < ntiles) request(tile + 1, nxt);
-      if (tile > 0) flush_cside(tile - 1);   // its slot is next written two tiles from now
+      if (tile + 1 < to) request(tile + 1, nxt);
+      if (tile > from) flush_cside(tile - 1);   // its slot is next written two tiles from now
       int d, toff;
       const int ic = tile_page(tile, d, toff);
       const int jc = vidx[ic];
@@ -2088,7 +2089,7 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
       }
     }
     __syncthreads();   // everybody is done with the last tile
-    if (ntiles > 0) flush_cside(ntiles - 1);
+    if (from < to) flush_cside(to - 1);
     bool any_mine = false;
 #pragma unroll
     for (int r = 0; r < 16; ++r) any_mine |= dcol0[r] >= 0 || dcol1[r] >= 0;
@@ -2111,10 +2112,11 @@ __global__ __launch_bounds__(kThreads) void raw_claim_value_kernel(GramArgs p) {
   constexpr int PIECES = kDmax / 8, GROUPS = kThreads / PIECES;
   const int tid = threadIdx.x;
   const int piece = tid % PIECES, g = tid / PIECES;
-  const int jp = blockIdx.x % p.NB;
-  const int h = (blockIdx.x / p.NB) % p.Hkv;
-  const int b = (blockIdx.x / (p.NB * p.Hkv)) % p.B;
-  const int l = blockIdx.x / (p.NB * p.Hkv * p.B);
+  const unsigned pages = gridDim.x / p.parts, page = blockIdx.x % pages, part = blockIdx.x / pages;
+  const int jp = page % p.NB;
+  const int h = (page / p.NB) % p.Hkv;
+  const int b = (page / (p.NB * p.Hkv)) % p.B;
+  const int l = page / (p.NB * p.Hkv * p.B);
   const int Tn = p.NB * p.BS;
   const int64_t obase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
   const float epsr = Elem<T>::rnd(p.eps);
@@ -2125,7 +2127,7 @@ __global__ __launch_bounds__(kThreads) void raw_claim_value_kernel(GramArgs p) {
   const bool pok = piece < p.D / 8;
   const int64_t k_row = (int64_t)p.Hkv * p.D * 2;
   const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2 + (pok ? piece : 0) * 16;
-  for (int slot = g; slot < p.BS; slot += GROUPS) {
+  for (int slot = part * GROUPS + g; slot < p.BS; slot += GROUPS * p.parts) {
     const int64_t oi = obase + (int64_t)jp * p.BS + slot;
     const int c = p.ws_col[oi];
     if (c < 0 || c >= Tn) continue;     // uniform over the 16 lanes of a key
@@ -2572,6 +2574,26 @@ GramArgs page_walks(GramArgs a, int L, int per_cu) {
   return a;
 }
 
+// All pairs, 16 bit: the column tiles of a page are divided among workgroups where that ends the launch earlier, in rounds of two
+// workgroups per CU whose beginning takes as long as two tiles; claims are integer maxima whatever the order.  Pages of 1, 2, 3, 4
+// and 8 sequences of 8 heads, us whole and in parts: 54.6 and 22.6 (5), 56.5 and 33.8 (3), 58.0 and 41.9 (2), 79.2 and 64.5
+// (3), 118.8 and 104.9 (2); of 6, 12, 24 and 40 best whole (74.5 and 80.0 with 2; 143 and 145; 267 and 275; 412 and 440).
+GramArgs tile_parts(GramArgs a, int64_t pages) {
+  const int tiles = (a.NB / 2 + 1) * (a.BS / kRawTile);
+  int64_t least = INT64_MAX;
+  for (int n = 1; n <= 5 && n <= tiles && pages * n <= INT32_MAX; ++n) {
+    const int64_t cost = (pages * n + 511) / 512 * (2 * n + tiles) * (60 / n);
+    if (cost < least) least = cost, a.parts = n;
+  }
+  return a;
+}
+// The keys of a page, whose claims are looked up one after the other (us with 1, 2, 4 and 8 workgroups: 80 pages 15.5, 9.4, 6.0, 5.0;
+// 320 21.1, 13.2, 9.7, 10.2; 1152 28.5, 25.4, 23.8, 26.9; 2880 53.0, 49.8, 52.3, 61.9).
+GramArgs claim_parts(GramArgs a, int64_t pages) {
+  a.parts = pages <= 256 ? 8 : pages <= 2048 ? 4 : pages <= INT32_MAX / 2 ? 2 : 1;
+  return a;
+}
+
 template <typename T, bool RAW>
 int launch_gram(const GramArgs& a, int L, hipStream_t st) {
   dim3 grid((unsigned)((int64_t)L * a.B * a.Hkv * a.NB));
@@ -2649,10 +2671,11 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
       return ZP_EHIP;
     }
     hipLaunchKernelGGL((raw_prep_kernel<T>), grid, dim3(kThreads), 0, st, a);
-    if (wide) hipLaunchKernelGGL((gram_raw_wide_kernel<T>), grid, dim3(256), smemw, st, a);
+    const GramArgs cut = tile_parts(a, grid.x), claims = claim_parts(a, grid.x);
+    if (wide) hipLaunchKernelGGL((gram_raw_wide_kernel<T>), dim3(grid.x * cut.parts), dim3(256), smemw, st, cut);
     else if (tn == 128) hipLaunchKernelGGL((gram_raw_kernel<T, 128>), grid, dim3(512), smem1, st, a);
     else hipLaunchKernelGGL((gram_raw_kernel<T, TN>), grid, dim3(512), smem1, st, a);
-    hipLaunchKernelGGL((raw_claim_value_kernel<T>), grid, dim3(kThreads), 0, st, a);
+    hipLaunchKernelGGL((raw_claim_value_kernel<T>), dim3(grid.x * claims.parts), dim3(kThreads), 0, st, claims);
     hipLaunchKernelGGL((raw_chain_kernel<T>), grid, dim3(512), smem2, st, a);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
