@@ -168,3 +168,33 @@ def test_one_call_on_rows_too_long_for_the_one_launch_selection(dev, kw):
     for a, b in zip(*outs):
         assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
     assert (outs[0][0].flatten(3).sum(-1) == budget * 256).all()
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("BS, W, G, pages, reduced, method", [
+    (256, 16, 2, [3, 4], "mean", "max"),      # one block of query rows
+    (256, 32, 4, [10], "mean", "sum"),        # four (fp32: eight), the longest row of the selection in registers
+    (256, 32, 4, [10, 11], "mean", "max"),    # one page more
+    (128, 32, 5, [3, 6], "max", "sum"),      # a block's remainder
+    (256, 16, 16, [3, 5], "max", "max"),
+])
+def test_selection_of_what_the_scorer_leaves(dev, dtype, BS, W, G, pages, reduced, method):
+    """One call adds the scorer's partials, and the scores of earlier steps, inside the selection: same bits as launch by launch."""
+    from zipage_amd.compress import CompressConfig, StageTimer, compress_layers
+    L, B, Hkv, P = 2, 24, 4, 12 * 24
+    _, enc, target = cases.random_tables(31 + W, B, P, pages, 2)
+    k, v, q, sc = cases.make_caches(33 + G, L, P, BS, Hkv, Hkv * G, 128, W, B + 1, dtype, touched=cases.touched_pages(enc),
+                                    with_score_cache=True)
+    qid, comp = torch.arange(B, dtype=torch.int32), torch.tensor([b % 3 != 1 for b in range(B)])
+    for carried in (True, False):
+        cfg = CompressConfig(budget_blocks=2, query_cache_len=W, reduced=reduced, use_global_score=carried, activate_method=method,
+                             decay_factor=0.9, enable_pooling=True, pooling_size=3)
+        outs = []
+        for one_call in (True, False):
+            gk, gv, gsc = k.clone().to(dev), v.clone().to(dev), sc.clone().to(dev)
+            res = compress_layers(gk, gv, q.to(dev), gsc, qid.to(dev), enc.to(dev), comp.to(dev), target.to(dev), cfg,
+                                  timer=StageTimer(False), return_intermediates=not one_call)
+            outs.append([t.cpu() for t in (res if one_call else res[0], gk, gv, gsc)])
+        for a, b in zip(*outs):
+            assert torch.equal(a.view(torch.uint8), b.view(torch.uint8))
+        assert (outs[0][0].flatten(3).sum(-1) == 2 * BS).all()

@@ -40,6 +40,32 @@ extern "C" int64_t zp_attention_score_workspace_few(int32_t L, int32_t B, int32_
 // brings less than zp_attention_score_workspace() asks for).  Library-internal.
 int64_t zp_attention_score_workspace_floor(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv,
                                            int32_t Hq, int32_t W);
+// Library-internal: what the walks of one sweep leave of a row, fp32 partials of RB blocks of query rows, where the selection adds them
+// up itself; part null: the scores are there.
+struct ScoreParts {
+  const float* part = nullptr;
+  int RB = 0, W = 0, rmax = 0, Gp = 0;
+};
+int zp_attention_score_parts(const void* k_cache, const void* query_cache, const int32_t* seq_idx, const int32_t* block_table,
+                             void* scores_out, int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
+                             int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl, int64_t k_sp, int64_t q_sl,
+                             int64_t q_ss, float softmax_scale, int32_t reduced, int32_t dtype, void* workspace,
+                             int64_t workspace_bytes, ScoreParts* left, void* stream);
+// The scores of earlier steps join those of a row before it is pooled (zp_global_score), and the row goes to `out`.
+struct CarriedScores {
+  const void* cache = nullptr;
+  int64_t c_sl = 0, c_sp = 0;        // elements; slots of Hkv heads
+  float decay = 0.f;
+  int method = 0;
+  void* out = nullptr;
+};
+// zp_select_topk of rows that zp_attention_score_parts left, as partials or scores.
+bool zp_select_takes_parts(int64_t Tn, int BS, int pool_kernel_size);
+int zp_select_topk_parts(const void* scores, const ScoreParts& parts, const CarriedScores& carried, const void* redundancy,
+                         uint8_t* flag_out, const int32_t* block_table, const uint8_t* compressed, int32_t L, int32_t B,
+                         int32_t NB, int32_t BS, int32_t Hkv, int32_t num_pages, int32_t pool_kernel_size,
+                         int32_t continues_pooling, int32_t pool_mode, int32_t max_norm_red, double redudancy_lambda,
+                         int32_t sink_len, int32_t window, int32_t mask_pad, int32_t k, int32_t dtype, void* stream);
 // gather.hip, library-internal: K/V compaction and the carried scores' compaction in one launch
 // where the shapes allow it (zp_compress_kv followed by zp_compress_score otherwise); the
 // arguments of the two.

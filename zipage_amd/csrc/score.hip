@@ -1788,14 +1788,15 @@ int64_t zp_attention_score_workspace_floor(int32_t L, int32_t B, int32_t NB, int
   return sweep_workspace(L, B, NB, BS, Hkv, Hq, W);
 }
 
-extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
-                                  const int32_t* seq_idx, const int32_t* block_table,
-                                  void* scores_out, void* logits_out, int32_t L, int32_t B,
-                                  int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
-                                  int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl,
-                                  int64_t k_sp, int64_t q_sl, int64_t q_ss, float softmax_scale,
-                                  int32_t reduced, int32_t dtype, void* workspace,
-                                  int64_t workspace_bytes, void* stream) {
+// left: where the partials of one sweep are all that is asked for, see ScoreParts.
+static int attention_score(const void* k_cache, const void* query_cache,
+                           const int32_t* seq_idx, const int32_t* block_table,
+                           void* scores_out, void* logits_out, int32_t L, int32_t B,
+                           int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
+                           int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl,
+                           int64_t k_sp, int64_t q_sl, int64_t q_ss, float softmax_scale,
+                           int32_t reduced, int32_t dtype, void* workspace,
+                           int64_t workspace_bytes, ScoreParts* left, void* stream) {
   ZP_REQUIRE(k_cache && query_cache && seq_idx && block_table && scores_out,
              "attention_score: null pointer");
   ZP_REQUIRE(L >= 0 && B >= 0 && NB > 0 && BS > 0 && Hkv > 0 && Hq > 0 && D > 0 && W > 0,
@@ -1855,6 +1856,10 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
   hipStream_t st = (hipStream_t)stream;
   a.n_items = L * B * Hkv;
   a.part = (float*)workspace;
+  auto leave = [&] {
+    if (left) *left = ScoreParts{a.part, a.RB, W, a.reduce_max, Gp};
+    return left != nullptr;
+  };
   const int64_t tiled = tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype);
   const bool straight = BS == 256 && !a.reduce_max && (Gp == 2 || Gp == 4);
   const int64_t walks = (int64_t)a.n_items * (resident32 ? (W * Gp + 15) / 16 : RB);
@@ -1895,7 +1900,8 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
       return ZP_EHIP;                                                                            \
     }                                                                                            \
     hipLaunchKernelGGL(fn, dim3(units), dim3(kThreads), smem, st, a);                            \
-    hipLaunchKernelGGL((score_combine_kernel<TT, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, \
+    if (!leave())                                                                                \
+      hipLaunchKernelGGL((score_combine_kernel<TT, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, \
                        block_table, B, NB, BS, Hkv, RB, W, num_pages, a.reduce_max, Gp);         \
   } while (0)
     if (dtype == ZP_BF16) ZP_RESIDENT_LAUNCH(BF16);
@@ -1918,7 +1924,8 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
       return ZP_EHIP;
     }
     hipLaunchKernelGGL(fn, dim3(units), dim3(kThreads), smem, st, a);
-    hipLaunchKernelGGL((score_combine_kernel<F32, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
+    if (!leave())
+      hipLaunchKernelGGL((score_combine_kernel<F32, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
                        B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max, Gp);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
@@ -1945,4 +1952,24 @@ extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
 #undef ZP_SCORE_LAUNCH
   ZP_LAUNCH_CHECK();
   return ZP_OK;
+}
+
+extern "C" int zp_attention_score(const void* k_cache, const void* query_cache,
+                                  const int32_t* seq_idx, const int32_t* block_table,
+                                  void* scores_out, void* logits_out, int32_t L, int32_t B,
+                                  int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
+                                  int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl,
+                                  int64_t k_sp, int64_t q_sl, int64_t q_ss, float softmax_scale,
+                                  int32_t reduced, int32_t dtype, void* workspace,
+                                  int64_t workspace_bytes, void* stream) {
+  return attention_score(k_cache, query_cache, seq_idx, block_table, scores_out, logits_out, L, B, NB, BS, Hkv, Hq, D, W, num_pages,
+                         max_seqs, k_sl, k_sp, q_sl, q_ss, softmax_scale, reduced, dtype, workspace, workspace_bytes, nullptr, stream);
+}
+int zp_attention_score_parts(const void* k_cache, const void* query_cache, const int32_t* seq_idx, const int32_t* block_table,
+                             void* scores_out, int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
+                             int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl, int64_t k_sp, int64_t q_sl,
+                             int64_t q_ss, float softmax_scale, int32_t reduced, int32_t dtype, void* workspace,
+                             int64_t workspace_bytes, ScoreParts* left, void* stream) {
+  return attention_score(k_cache, query_cache, seq_idx, block_table, scores_out, nullptr, L, B, NB, BS, Hkv, Hq, D, W, num_pages,
+                         max_seqs, k_sl, k_sp, q_sl, q_ss, softmax_scale, reduced, dtype, workspace, workspace_bytes, left, stream);
 }

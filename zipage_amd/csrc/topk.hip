@@ -8,6 +8,7 @@
 // exclusive scan over index-ordered per-thread chunks decides.
 #include "common.h"
 #include <limits.h>
+#include <type_traits>
 
 namespace {
 
@@ -191,6 +192,11 @@ struct SelectArgs {
   float lam, one_minus_lam;
   int sink_len, window, mask_pad, k, low_bit;
 };
+struct LeftArgs : SelectArgs {        // a row as the scorer left it: see ScoreParts; and the scores of earlier steps
+  ScoreParts parts;
+  CarriedScores carried;
+  int num_pages;
+};
 
 // Row -> LDS as fp32, 16 bytes per thread per step when the row allows it.
 template <typename T>
@@ -216,6 +222,78 @@ __device__ __forceinline__ void stage_row(const void* __restrict__ src, int64_t 
     }
   } else {
     for (int t = threadIdx.x; t < Tn; t += kThreads) row[t] = Elem<T>::ld(src, base + t);
+  }
+}
+
+// The same row (of at most kPer tokens a thread) as the scorer left it, PARTS: in partials, with the scores of earlier steps, rounded
+// where launches of their own would.  Bound by the partials' way from memory: all tokens' loads of four blocks are side by side (one
+// token's after another's, 64 bf16 sequences 14.0 us, now 13.5; 256 without earlier scores 32.0, now 24.6; 4 with 13.4, now 9.6).
+constexpr int kPer = 10;             // tokens of a thread whose keys stay in registers
+template <typename T, bool PARTS>
+__device__ __forceinline__ void stage_left(const LeftArgs& p, uint32_t r, int b, int Tn, float* __restrict__ row) {
+  constexpr int kPieces = (kPer + 3) / 4, kBlocks = 4;      // of four tokens; whose loads are side by side
+  const int h = (int)(r % (uint32_t)p.Hkv), l = (int)(r / ((uint32_t)p.Hkv * (uint32_t)p.B));
+  const bool again = p.carried.cache && p.compressed[b] != 0;
+  typedef float f4 __attribute__((ext_vector_type(4)));
+  auto join = [&](const f4& x, const f4& o) {
+    return p.parts.rmax ? f4{fmaxf(x.x, o.x), fmaxf(x.y, o.y), fmaxf(x.z, o.z), fmaxf(x.w, o.w)} : x + o;
+  };
+  f4 v[kPieces];
+  int at[kPieces], code[kPieces];
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    at[u] = min((u * kThreads + (int)threadIdx.x) * 4, Tn - 4);
+    code[u] = p.table[(int64_t)b * p.NB + at[u] / p.BS];
+  }
+  if constexpr (PARTS) {
+    const float* const part = p.parts.part + (int64_t)r * p.parts.RB * Tn;
+    for (int r0 = 0; r0 < p.parts.RB; r0 += kBlocks) {
+      f4 x[kPieces][kBlocks];
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+        for (int k = 0; k < kBlocks; ++k)
+          x[u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)min(r0 + k, p.parts.RB - 1) * Tn + at[u]));
+#pragma unroll
+      for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+        for (int k = 0; k < kBlocks; ++k) {
+          if (r0 + k >= p.parts.RB) break;
+          v[u] = r0 + k == 0 ? x[u][k] : join(v[u], x[u][k]);
+        }
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < kPieces; ++u) {
+    const int t = (u * kThreads + (int)threadIdx.x) * 4;
+    if (t >= Tn) break;
+    const int pid = page_is_pad(code[u]) ? -1 : page_id(code[u]);
+    const bool there = pid >= 0 && pid < p.num_pages;
+    if constexpr (PARTS) {
+      if (!p.parts.rmax)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[u][i] = Elem<T>::rnd(v[u][i] / (float)p.parts.W);
+      if (!there) v[u] = f4{0.f, 0.f, 0.f, 0.f};
+    } else {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[u][i] = Elem<T>::ld(p.scores, (int64_t)r * Tn + t + i);
+    }
+    if (again && there && !page_is_last(code[u])) {
+      const int64_t from = l * p.carried.c_sl + pid * p.carried.c_sp + (int64_t)(t % p.BS) * p.Hkv + h;
+      float old[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) old[i] = Elem<T>::ld(p.carried.cache, from + i * p.Hkv);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float o = old[i] * p.carried.decay;
+        v[u][i] = Elem<T>::rnd(p.carried.method == ZP_ACTIVATE_MAX ? fmaxf(v[u][i], o) : v[u][i] + o);
+      }
+    }
+    if (p.carried.out && (PARTS || again)) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) Elem<T>::st(p.carried.out, (int64_t)r * Tn + t + i, v[u][i]);
+    }
+    *(f4*)(row + t) = v[u];
   }
 }
 
@@ -269,8 +347,8 @@ __device__ __forceinline__ void write_flags(const uint8_t* fl, uint8_t* __restri
 // are straight-line code.
 constexpr int kSelHalf = 3;
 constexpr int kSelPad = 4;   // floats in front of the row (keeps it 16-byte aligned)
-template <typename T, int PER, int POOLK, bool RED>
-__global__ __launch_bounds__(kThreads) void select_reg_kernel(SelectArgs p) {
+template <typename T, int PER, int POOLK, bool RED, typename Args>
+__global__ __launch_bounds__(kThreads) void select_reg_kernel(Args p) {
   extern __shared__ float sel_smem[];
   __shared__ __align__(16) int hist[RadixPlan<LowBit<T>::v>::words];
   __shared__ int scan_lds[kWaves];
@@ -286,7 +364,9 @@ __global__ __launch_bounds__(kThreads) void select_reg_kernel(SelectArgs p) {
   // every global read of the prologue is issued before the first wait
   const uint8_t was_compressed = p.compressed[b];
   for (int i = tid; i < p.NB + 2; i += kThreads) trow[i] = i < p.NB ? p.table[(int64_t)b * p.NB + i] : -1;
-  stage_row<T>(p.scores, base, Tn, row);
+  if constexpr (std::is_same_v<Args, SelectArgs>) stage_row<T>(p.scores, base, Tn, row);
+  else if (p.parts.part) stage_left<T, true>(p, r, b, Tn, row);
+  else stage_left<T, false>(p, r, b, Tn, row);
   {
     const float neutral = POOLK > 0 ? -INFINITY : 0.f;
     if (tid < kSelPad) row[tid - kSelPad] = neutral;
@@ -502,13 +582,18 @@ extern "C" int zp_topk_mask(const void* scores, uint8_t* flag_out, int32_t rows,
   return ZP_OK;
 }
 
-extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* redundancy,
-                              uint8_t* flag_out, const int32_t* block_table,
-                              const uint8_t* compressed, int32_t L, int32_t B, int32_t NB,
-                              int32_t BS, int32_t Hkv, int32_t pool_kernel_size,
-                              int32_t continues_pooling, int32_t pool_mode, int32_t max_norm_red,
-                              double redudancy_lambda, int32_t sink_len, int32_t window,
-                              int32_t mask_pad, int32_t k, int32_t dtype, void* stream) {
+bool zp_select_takes_parts(int64_t Tn, int BS, int pool_kernel_size) {
+  return Tn <= kPer * kThreads && BS >= kPer && BS % 4 == 0 && pool_kernel_size <= 2 * kSelHalf + 1;
+}
+
+static int select_topk(const void* scores, void* scores_out, const void* redundancy,
+                       uint8_t* flag_out, const int32_t* block_table,
+                       const uint8_t* compressed, int32_t L, int32_t B, int32_t NB,
+                       int32_t BS, int32_t Hkv, int32_t pool_kernel_size,
+                       int32_t continues_pooling, int32_t pool_mode, int32_t max_norm_red,
+                       double redudancy_lambda, int32_t sink_len, int32_t window,
+                       int32_t mask_pad, int32_t k, int32_t dtype, const ScoreParts& parts, const CarriedScores& carried,
+                       int32_t num_pages, void* stream) {
   ZP_REQUIRE(L >= 0 && B >= 0 && NB > 0 && BS > 0 && Hkv > 0, "select_topk: bad dims");
   const int64_t Tn = (int64_t)NB * BS;
   ZP_REQUIRE(k >= 0 && k <= Tn, "select_topk: k=%d out of range for a row of %lld", k, (long long)Tn);
@@ -521,9 +606,10 @@ extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* 
   ZP_REQUIRE(dtype >= ZP_BF16 && dtype <= ZP_F32, "select_topk: unknown dtype tag %d", dtype);
   ZP_REQUIRE(Tn * 8 <= 150 * 1024, "select_topk: row of %lld tokens exceeds LDS", (long long)Tn);
   if (L == 0 || B == 0) return ZP_OK;
-  ZP_REQUIRE(scores && flag_out && block_table && compressed, "select_topk: null pointer");
+  ZP_REQUIRE((scores || parts.part) && flag_out && block_table && compressed, "select_topk: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  SelectArgs p;
+  LeftArgs p;
+  p.parts = parts; p.carried = carried; p.num_pages = num_pages;
   p.scores = scores; p.scores_out = scores_out; p.red = redundancy; p.flag = flag_out;
   p.table = block_table; p.compressed = compressed;
   p.B = B; p.NB = NB; p.BS = BS; p.Hkv = Hkv; p.ksize = pool_kernel_size;
@@ -532,10 +618,10 @@ extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* 
   p.sink_len = sink_len; p.window = window; p.mask_pad = mask_pad; p.k = k;
   p.low_bit = dtype == ZP_BF16 ? 16 : (dtype == ZP_F16 ? 13 : 0);
   dim3 grid((unsigned)((int64_t)L * B * Hkv));
-  constexpr int PER = 10;
+  constexpr int PER = kPer;
   const bool in_regs = Tn <= PER * kThreads && BS >= PER && pool_kernel_size <= 2 * kSelHalf + 1;
   const size_t smem = in_regs ? ((size_t)Tn + PER + 2 * kSelPad + NB + 2) * 4 : (size_t)Tn * 8;
-#define ZP_SELECT_LAUNCH(KERNEL)                                                                  \
+#define ZP_SELECT_LAUNCH(KERNEL, ARGS)                                                            \
   do {                                                                                            \
     if (smem > 64 * 1024 &&                                                                       \
         hipFuncSetAttribute((const void*)KERNEL, hipFuncAttributeMaxDynamicSharedMemorySize,      \
@@ -543,12 +629,12 @@ extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* 
       zp_set_error("select_topk: cannot reserve %zu bytes of LDS", smem);                         \
       return ZP_EHIP;                                                                             \
     }                                                                                             \
-    hipLaunchKernelGGL(KERNEL, grid, dim3(kThreads), smem, st, p);                                \
+    hipLaunchKernelGGL(KERNEL, grid, dim3(kThreads), smem, st, ARGS);                                \
   } while (0)
 #define ZP_SELECT_REG(POOLK)                                                                      \
   do {                                                                                            \
-    if (redundancy) ZP_SELECT_LAUNCH((select_reg_kernel<T, PER, POOLK, true>));                   \
-    else ZP_SELECT_LAUNCH((select_reg_kernel<T, PER, POOLK, false>));                             \
+    if (redundancy) ZP_SELECT_LAUNCH((select_reg_kernel<T, PER, POOLK, true, Args>), *args);      \
+    else ZP_SELECT_LAUNCH((select_reg_kernel<T, PER, POOLK, false, Args>), *args);                \
   } while (0)
 #define ZP_SELECT_REG_ALL()                                                                       \
   do {                                                                                            \
@@ -559,13 +645,42 @@ extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* 
     else ZP_SELECT_REG(3);                                                                        \
   } while (0)
   if (in_regs) {
-    ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_REG_ALL());
+    auto launch = [&](auto* args) -> int {
+      using Args = std::remove_pointer_t<decltype(args)>;
+      ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_REG_ALL());
+      return ZP_OK;
+    };
+    const int rc = parts.part || carried.cache ? launch(&p) : launch((SelectArgs*)&p);
+    if (rc != ZP_OK) return rc;
   } else {
-    ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_LAUNCH((select_lds_kernel<T>)));
+    ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_LAUNCH((select_lds_kernel<T>), p));
   }
 #undef ZP_SELECT_REG_ALL
 #undef ZP_SELECT_REG
 #undef ZP_SELECT_LAUNCH
   ZP_LAUNCH_CHECK();
   return ZP_OK;
+}
+
+extern "C" int zp_select_topk(const void* scores, void* scores_out, const void* redundancy,
+                              uint8_t* flag_out, const int32_t* block_table,
+                              const uint8_t* compressed, int32_t L, int32_t B, int32_t NB,
+                              int32_t BS, int32_t Hkv, int32_t pool_kernel_size,
+                              int32_t continues_pooling, int32_t pool_mode, int32_t max_norm_red,
+                              double redudancy_lambda, int32_t sink_len, int32_t window,
+                              int32_t mask_pad, int32_t k, int32_t dtype, void* stream) {
+  ZP_REQUIRE(scores || L == 0 || B == 0, "select_topk: null pointer");
+  return select_topk(scores, scores_out, redundancy, flag_out, block_table, compressed, L, B, NB, BS, Hkv, pool_kernel_size,
+                     continues_pooling, pool_mode, max_norm_red, redudancy_lambda, sink_len, window, mask_pad, k, dtype, {}, {}, 0,
+                     stream);
+}
+int zp_select_topk_parts(const void* scores, const ScoreParts& parts, const CarriedScores& carried, const void* redundancy,
+                         uint8_t* flag_out, const int32_t* block_table, const uint8_t* compressed, int32_t L, int32_t B,
+                         int32_t NB, int32_t BS, int32_t Hkv, int32_t num_pages, int32_t pool_kernel_size,
+                         int32_t continues_pooling, int32_t pool_mode, int32_t max_norm_red, double redudancy_lambda,
+                         int32_t sink_len, int32_t window, int32_t mask_pad, int32_t k, int32_t dtype, void* stream) {
+  ZP_REQUIRE(zp_select_takes_parts((int64_t)NB * BS, BS, pool_kernel_size), "select_topk: rows too long to be added up here");
+  return select_topk(scores, nullptr, redundancy, flag_out, block_table, compressed, L, B, NB, BS, Hkv, pool_kernel_size,
+                     continues_pooling, pool_mode, max_norm_red, redudancy_lambda, sink_len, window, mask_pad, k, dtype, parts,
+                     carried, num_pages, stream);
 }
