@@ -72,6 +72,11 @@ int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32
 /* The same for up to 256 rows. */
 int zp_row_tiles_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
                         int64_t out_stride, int32_t dtype, void* stream);
+/* The same in parts of the contraction, whose fp32 sums lie in the workspace (zp_split_rows_workspace bytes, 16-byte aligned) on
+   the way: at most 256 rows. */
+int64_t zp_split_rows_workspace(int32_t n, int32_t K, int32_t M);
+int zp_split_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
+                         int64_t out_stride, int32_t dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* What an attention does beyond the softmax of scaled products; NULL stands for {0, 1}.
  * softcap > 0: scores s (after the scale) enter the softmax as softcap * tanh(s / softcap).

@@ -346,6 +346,48 @@ def test_products_of_row_tiles(dev, dtype, n, K, M):
         _lib.call_models("zp_few_rows_linear", x.data_ptr(), w.data_ptr(), out.data_ptr(), n, *args)
 
 
+# every tile size, in one part and in several; a contraction that ends inside a stage, and parts of unequal length; rows and outputs
+# that end inside a tile; the largest number of parts
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 127, 129, 192, 193, 256])
+@pytest.mark.parametrize("K,M", [(32, 4), (96, 516), (1056, 1540), (4128, 512), (2080, 4100), (1024, 6148), (160, 24580), (3072, 132)])
+def test_products_in_parts(dev, dtype, n, K, M):
+    from zipage_amd import _lib
+    wide = _rand(n, K + 24, seed=1, dtype=dtype).to(dev)
+    x, w = wide[:, 8:8 + K], (_rand(M, K, seed=2).float() * K ** -0.5).to(dtype).to(dev)
+    out = torch.full((n + 1, M + 4), 7.0, dtype=dtype, device=dev)
+    size = _lib.size("zp_split_rows_workspace", n, K, M)
+    room = torch.full((size // 4 + 4,), 7.0, device=dev)
+    args = lambda n, size: (x.data_ptr(), w.data_ptr(), out.data_ptr(), n, K, M, x.stride(0), out.stride(0), _lib.dtype_tag(x),
+                            room.data_ptr(), size, _lib.stream_ptr(x))
+    _lib.call_models("zp_split_rows_linear", *args(n, size))
+    assert bool((out[:n, M:] == 7).all()) and bool((out[n:] == 7).all()) and bool((room[size // 4:] == 7).all())
+    want = x.double() @ w.double().T                           # bounds as for few rows
+    bits = 2.0 ** (-8 if dtype == BF16 else -11)
+    assert bool(((out[:n, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
+    if size:
+        with pytest.raises(RuntimeError, match="workspace"):
+            _lib.call_models("zp_split_rows_linear", *args(n, size - 16))
+    with pytest.raises(RuntimeError, match="at most 256"):
+        _lib.call_models("zp_split_rows_linear", *args(257, size))
+
+
+def test_products_in_parts_under_capture(dev):
+    """Through the entry point, in a graph that is replayed on new rows."""
+    from zipage_amd.layers import linear
+    x, w = _rand(40, 5120, seed=3).to(dev), (_rand(2048, 5120, seed=4).float() / 72).to(BF16).to(dev)
+    linear(x, w)
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g):
+        y = linear(x, w)
+    for seed in range(3):
+        x.copy_(_rand(40, 5120, seed=seed).to(dev))
+        g.replay()
+        assert torch.equal(y, linear(x, w))
+        want = x.double() @ w.double().T
+        assert bool(((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -20).all())
+
+
 @pytest.fixture
 def few_rows_calls(monkeypatch):
     """Says whether the kernel for few rows was called since it last did."""

@@ -105,3 +105,18 @@ def test_which_sizes_are_few_rows(n, k, m, few):
 def test_which_sizes_are_row_tiles(n, k, m, tiles):
     from zipage_amd.layers.linear import _few_rows, _row_tiles
     assert _row_tiles(n, k, m) == tiles and not (_row_tiles(n, k, m) and _few_rows(n, k, m))
+
+
+# each line of the rule from both sides
+@pytest.mark.parametrize("n,k,m,split", [(16, 12288, 4096, False), (17, 12288, 4096, True), (32, 4608, 4096, False), (32, 12288, 4868, False),
+                                         (32, 8192, 1980, False), (24, 4096, 24576, True), (24, 4096, 151936, True), (24, 992, 151936, False),
+                                         (64, 1024, 151936, True), (65, 1024, 151936, False), (112, 4096, 151936, True), (113, 4096, 151936, False),
+                                         (33, 4096, 6144, True), (33, 4096, 10244, False), (48, 3072, 1024, True), (48, 3072, 2048, False),
+                                         (48, 2528, 1024, False), (64, 8192, 1024, False), (64, 8224, 1024, True), (65, 4096, 4096, False),
+                                         (89, 4096, 4096, True), (65, 4096, 6144, True), (128, 12288, 1020, False), (128, 4096, 24576, True),
+                                         (129, 4096, 24576, False), (129, 4096, 6144, True), (192, 4096, 4096, True), (193, 4096, 4096, False),
+                                         (256, 4096, 6144, True), (256, 12288, 4096, True), (257, 12288, 4096, False), (256, 4064, 6144, False),
+                                         (100, 6160, 4096, False), (100, 6144, 4098, False)])
+def test_which_sizes_are_split(n, k, m, split):
+    from zipage_amd.layers.linear import _split_rows
+    assert _split_rows(n, k, m) == split

@@ -159,10 +159,11 @@ MODEL_LIBS = {
         "zp_gather_rows": [ptr, ptr, ptr, i32, i32, i64, ptr],
         "zp_few_rows_linear": [ptr, ptr, ptr, i32, i32, i32, i64, i64, i32, ptr],
         "zp_row_tiles_linear": [ptr, ptr, ptr, i32, i32, i32, i64, i64, i32, ptr],
+        "zp_split_rows_linear": [ptr, ptr, ptr, i32, i32, i32, i64, i64, i32, ptr, i64, ptr],
         "zp_run_attention": [ptr, ptr, ptr, ptr, ptr, ptr, ptr, form_ptr, i32, i32, i32, i32, i32, i32, i32, i32, i64,
                              i64, i64, i64, i64, i64, f32, f32, i32, ptr],
         "zp_causal_attention": [ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i64, i64, i64, i64, i64, i64, f32, i32, ptr],
-    }, {}),
+    }, {"zp_split_rows_workspace": [i32, i32, i32]}),
     "latent": ({
         "zp_latent_norm_store": [ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i32, i32, i32, i64,
                                  f32, i32, ptr],

@@ -62,6 +62,37 @@ def _row_tiles(n: int, k: int, m: int) -> bool:
     return k <= 2048 or n <= 128 and (n > 96 and k <= 3072 or n > 112 and k <= 4096)
 
 
+def _split_rows(n: int, k: int, m: int) -> bool:
+    """The same for 17 to 256 rows, in parts of the contraction, before the two above: where the library's tiles leave most of the chip
+    idle (us of both: 64 rows, 12 288 -> 4096 25.5 and 36.3, 4096 -> 6144 17.2 and 17.6; 128 rows 31.1 and 66.0, 21.1 and 25.0; 192 rows 37
+    and 89, 25.0 and 33.3; 256 rows 41 and 53, 28 and 39.5; 4096 -> 4096 17.3 and 23.5 for 128 rows, 21.6 and 31.5 for 192), and up to 64
+    rows outputs of many rounds of workgroups (64 rows, 4096 -> 151 936 227 and 262; 48 rows, 1024 -> 151 936 66 and 77; 96 rows 259 and 273).
+    The library's choices are uneven, so the lines are drawn where 95 % of random sizes are no slower (300 sizes: 1.35 times as fast on
+    average): it is good at 6144 and 8192 -> 1280 and fewer (32 to 128 rows, 10.9 and 9.7), at contractions of 4096 of some rows (80 rows,
+    -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
+    its tiles fill the chip (256 rows, 4096 -> 24 576 64 and 62; but 128 rows 45.3 and 48.3)."""
+    if not 16 < n <= 256 or k % 32 or m % 4 or m < 512:
+        return False
+    if m >= 73728:
+        return k >= 1024 and n <= 64 or k >= 2048 and n <= 112 and m >= 131072
+    if k < 2560 or m < 1280 and 6144 <= k <= 8192:
+        return False
+    if n <= 32:
+        return 21504 <= m <= 25600 or k > 4608 and (1984 if k <= 8192 else 1280) <= m <= 4864
+    if n <= 64:
+        return m <= 10240 if k >= 4096 else m <= 1280 or 2816 <= m <= 8192
+    if n <= 128:
+        if 21120 <= m <= 24576:
+            return 3072 <= k <= 12288
+        least = 1024 if k >= 5376 else 2432 if k >= 4480 else 3968 if n > 88 else 5632
+        return k >= 4096 and least <= m <= 12288
+    if k < 4096 or not 1024 <= m <= 12288:
+        return False
+    if n <= 192:
+        return k >= 5888 or 2816 <= m <= (6656 if k < 4608 else 12288)
+    return k >= 7168 or m >= 5888
+
+
 def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether something beside the product looks at the call, which only the library's passes through torch's dispatcher:
     gradients of either mode, vmap and its like, autocast, modes, subclasses, tracing and compilation; or another device than the current
@@ -75,12 +106,20 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """F.linear(x, w) without a bias."""
     if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 == w.dim() and x.layout == w.layout == torch.strided:
         (n, k), (m, wk), (stride, one) = x.shape, w.shape, x.stride()
-        if k == wk and x.dtype == w.dtype in _FEW_TYPES and (_few_rows(n, k, m) or _row_tiles(n, k, m)) and one == 1 and \
-                k <= stride <= 1 << 23 and stride % 8 == 0 and w.is_contiguous() and w.device == x.device:
+        if k == wk and x.dtype == w.dtype in _FEW_TYPES and one == 1 and k <= stride <= 1 << 23 and stride % 8 == 0 and w.is_contiguous() and \
+                w.device == x.device:
             at, w_at = x.data_ptr(), w.data_ptr()
-            if (at | w_at) % 16 == 0:
-                out = x.new_empty(n, m)
-                _lib.call_models("zp_few_rows_linear" if n <= 64 else "zp_row_tiles_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, _lib.dtype_tag(x), _lib.stream_ptr(x))
+            split = _split_rows(n, k, m) and stride <= 1 << 22
+            if (at | w_at) % 16 == 0 and (split or _few_rows(n, k, m) or _row_tiles(n, k, m)):
+                out, tag, stream = x.new_empty(n, m), _lib.dtype_tag(x), _lib.stream_ptr(x)
+                if split:
+                    size = _lib.size("zp_split_rows_workspace", n, k, m)
+                    room = x.new_empty(size // 2) if size else None
+                    _lib.call_models("zp_split_rows_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, tag, room.data_ptr() if size else None,
+                                     size, stream)
+                else:
+                    _lib.call_models("zp_few_rows_linear" if n <= 64 else "zp_row_tiles_linear", at, w_at, out.data_ptr(), n, k, m, stride, m,
+                                     tag, stream)
                 return out
     return F.linear(x, w)
 
