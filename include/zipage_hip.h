@@ -330,6 +330,15 @@ int zp_paged_decode_attention(const void* q, const void* k_cache, const void* v_
                               int32_t BS, int32_t NB, int32_t num_pages,
                               int64_t k_stride_page, int64_t v_stride_page,
                               float softmax_scale, int32_t dtype, void* stream);
+/* The same where few sequences leave CUs idle: each context in several parts, whose sums lie in the workspace
+ * (zp_paged_decode_workspace bytes, none where it says 0; 16-byte aligned) on the way. */
+int64_t zp_paged_decode_workspace(int32_t B, int32_t Hq, int32_t Hkv, int32_t D, int32_t BS, int32_t NB);
+int zp_paged_decode_parts(const void* q, const void* k_cache, const void* v_cache,
+                          const int32_t* block_tables, const int32_t* context_lens,
+                          void* out, int32_t B, int32_t Hq, int32_t Hkv, int32_t D,
+                          int32_t BS, int32_t NB, int32_t num_pages,
+                          int64_t k_stride_page, int64_t v_stride_page,
+                          float softmax_scale, int32_t dtype, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* ---- fused elementwise pieces of the decoder layer (between the GEMMs and the cache kernels).
  * The reference takes RMSNorm and SiluAndMul from its nanovllm dependency (imports at

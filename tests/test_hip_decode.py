@@ -115,3 +115,36 @@ def test_store_kvcache_empty(dev):
     key = torch.zeros(0, 2, 64, device=dev, dtype=torch.bfloat16)
     store_kvcache(key, key.clone(), k_cache, v_cache, torch.zeros(0, device=dev, dtype=torch.int32))
     assert not k_cache.any()
+
+
+# one part and several of each context: groups at the line and one past it, tables on both sides of 1024 tokens, contexts that leave
+# parts empty or end inside one, that are longer than one slice of the logits, and none
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("B,Hq,Hkv,D,BS,NB", [(16, 32, 8, 128, 256, 4), (17, 32, 8, 128, 256, 4), (8, 16, 8, 128, 256, 9), (8, 16, 8, 128, 64, 15),
+                                              (1, 8, 8, 64, 64, 33), (1, 8, 1, 128, 256, 65), (3, 16, 2, 96, 48, 70), (32, 8, 4, 128, 128, 9),
+                                              (33, 8, 8, 128, 64, 20), (2, 4, 4, 8, 16, 200)])
+def test_paged_decode_in_parts(dev, dtype, B, Hq, Hkv, D, BS, NB):
+    from zipage_amd import _lib
+    from zipage_amd.layers import paged_decode_attention
+    g = torch.Generator().manual_seed(B * NB)
+    k, v = ((torch.randn(B * NB, BS, Hkv, D, generator=g)).to(dtype).to(dev) for _ in range(2))
+    q = torch.randn(B, Hq, D, generator=g).to(dtype).to(dev)
+    tables = torch.randperm(B * NB, generator=g).int().view(B, NB).contiguous().to(dev)
+    most = NB * BS
+    lens = ([most, 1, 0, most // 2 + 1, 64, 65, most - 1, 300] * B)[:B]
+    ctx = torch.tensor([min(n, most) for n in lens], dtype=torch.int32, device=dev)
+    whole = torch.empty_like(q)
+    _lib.call("zp_paged_decode_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), tables.data_ptr(), ctx.data_ptr(), whole.data_ptr(),
+              B, Hq, Hkv, D, BS, NB, B * NB, k.stride(0), v.stride(0), D ** -0.5, _lib.dtype_tag(q), _lib.stream_ptr(q))
+    got = paged_decode_attention(q, k, v, ctx, tables, D ** -0.5)
+    bits = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for b, n in enumerate(ctx.tolist()):
+        if n == 0:
+            assert not got[b].any() and not whole[b].any()
+            continue
+        kk, vv = (c[tables[b].long()].reshape(-1, Hkv, D)[:n].double().cpu().repeat_interleave(Hq // Hkv, 1) for c in (k, v))
+        w = ((kk * q[b].double().cpu()).sum(-1) * D ** -0.5).softmax(0)
+        want = (w[..., None] * vv).sum(0)
+        # the result's rounding, and each weight's: its share of the values' absolute sum
+        bound = bits * (want.abs() + (w[..., None] * vv.abs()).sum(0)) + 2.0 ** -16
+        assert bool(((got[b].double().cpu() - want).abs() <= bound).all()) and bool(((whole[b].double().cpu() - want).abs() <= bound).all())

@@ -50,6 +50,8 @@ SIGNATURES = {
     "zp_store_kvcache": [ptr, ptr, ptr, ptr, ptr, i32, i32, i64, i64, i64, i32, ptr],
     "zp_paged_decode_attention": [ptr, ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i32, i32, i32,
                                   i64, i64, f32, i32, ptr],
+    "zp_paged_decode_parts": [ptr, ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i32, i32, i32,
+                              i64, i64, f32, i32, ptr, i64, ptr],
     "zp_add_rms_norm": [ptr, ptr, ptr, ptr, i32, i32, i64, i64, i64, f32, i32, ptr],
     "zp_silu_and_mul": [ptr, ptr, i32, i32, i64, i64, i32, ptr],
     "zp_qk_norm_rope_store": [ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, i32, i32,
@@ -88,6 +90,7 @@ I64_RETURNING = {
     "zp_attention_score_workspace_for": [i32, i32, i32, i32, i32, i32, i32, i32],
     "zp_attention_score_workspace_few": [i32, i32, i32, i32, i32, i32, i32, i32],
     "zp_redundancy_raw_workspace": [i32, i32, i32, i32, i32],
+    "zp_paged_decode_workspace": [i32, i32, i32, i32, i32, i32],
 }
 EXPORTS = sorted(list(SIGNATURES) + list(I64_RETURNING) + ["zp_abi_version", "zp_last_error"])
 

@@ -72,6 +72,8 @@ struct DecodeArgs {
   int B, Hq, Hkv, G, D, BS, NB, num_pages;
   int bs_shift;        // log2(BS) when BS is a power of two, else -1
   int chunk;           // tokens per slice when the context is walked in slices (multiple of 128)
+  int splits;          // of each context, a workgroup each
+  float* part;         // splits > 1: (B, Hq, splits, D) sums, then (B, Hq, splits) maxima and weights
   int64_t k_sp, v_sp;  // page strides in elements
   float scale;
 };
@@ -82,10 +84,9 @@ struct DecodeArgs {
 #define ZP_DEC_LOAD(ptr) __builtin_nontemporal_load(ptr)
 #endif
 constexpr int kMaxTablePages = 256;     // block-table entries per sequence (the LDS logits cap the context first)
-constexpr int kGroups = kThreads / 8;  // token rows in flight per step of the workgroup
 constexpr int kUnroll = 4;             // rows per lane group and loop trip (must be even)
 
-// One workgroup per (sequence, kv head); the G query heads of the group share the K/V stream.
+// One workgroup per (sequence, kv head), or SPLIT: per part of one's context; the G query heads of the group share the K/V stream.
 // Eight lanes own one token row: lane `sub` holds the 16-byte pieces `sub` and `sub + 8` of the
 // head vector, so one load instruction of the wave covers eight rows, each a full 128-byte line.
 //   pass 1: logits = q.k on packed 16-bit pairs, reduced over the 8 lanes, scaled, to LDS (fp32)
@@ -93,16 +94,22 @@ constexpr int kUnroll = 4;             // rows per lane group and loop trip (mus
 //           packed in pairs (token t, token t + 32) over the logit word of t
 //   pass 3: out += p.v with two tokens per dot2 (the pair above), fp32 accumulate; the row
 //           groups are summed at the end and scaled by 1 / sum(p).
-template <typename T, int G, bool CHUNKED>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4 && !CHUNKED ? 4 : 2, 4))) void paged_decode_kernel(DecodeArgs p) {
+template <typename T, int G, bool CHUNKED, bool SPLIT, int THREADS>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(G <= 4 && !CHUNKED ? 4 : 2, 4))) void paged_decode_kernel(DecodeArgs p) {
+  constexpr int kThreads = THREADS, kWaves = THREADS / 64;
+  constexpr int kGroups = THREADS / 8;   // token rows in flight per step of the workgroup
   extern __shared__ __align__(16) float lds[];
   __shared__ float red[kWaves * G];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int grp = tid >> 3, sub = tid & 7;
-  const int h = blockIdx.x % p.Hkv, b = blockIdx.x / p.Hkv;
+  const int split = SPLIT ? blockIdx.x % p.splits : 0, item = SPLIT ? blockIdx.x / p.splits : blockIdx.x;
+  const int h = item % p.Hkv, b = item / p.Hkv;
   int Tn = p.ctx[b];
   Tn = max(0, min(Tn, p.NB * p.BS));
-  const int Tpad = CHUNKED ? p.chunk : ((p.NB * p.BS + 63) & ~63);   // LDS row of one head's logits
+  // tokens of one of the splits, at most; and of this sequence's
+  const int most = SPLIT ? (p.NB * p.BS + p.splits - 1) / p.splits : p.NB * p.BS;
+  const int per = SPLIT ? ((Tn + p.splits - 1) / p.splits + 63) & ~63 : Tn, first = split * per;
+  const int Tpad = CHUNKED ? p.chunk : ((most + 63) & ~63);   // LDS row of one head's logits
   float* logit = lds;                            // [G][Tpad]
   uint32_t* pw = (uint32_t*)lds;                 // packed p pairs over the same words
   const int pieces = p.D / 8;                    // 16-byte pieces per head vector (<= 16)
@@ -187,6 +194,19 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4
         }
       }
     }
+    // rows of V: those of the first trip are asked for before the softmax where a workgroup makes few trips
+    constexpr int kPairs = 4, kRows = THREADS / 16;
+    auto pair_at = [&](int u) { return (u * kRows >> 5) * 64 + (u * kRows & 31) + g16; };   // its partner is 32 further
+    u32x4 vx[kPairs], vy[kPairs];
+    auto fetch_v = [&](int t0, u32x4* x, u32x4* y) {
+#pragma unroll
+      for (int u = 0; u < kPairs; ++u) {
+        const int t = c0 + t0 + pair_at(u);
+        x[u] = ZP_DEC_LOAD((const u32x4*)(row_base(p.v, p.v_sp, t) + offV));
+        y[u] = ZP_DEC_LOAD((const u32x4*)(row_base(p.v, p.v_sp, t + 32) + offV));
+      }
+    };
+    if constexpr (SPLIT) fetch_v(0, vx, vy);
     __syncthreads();
     // ---- pass 2: softmax statistics per head, p packed in pairs (t, t + 32)
     {
@@ -238,26 +258,17 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4
         m_run[g] = mx[g];
       }
     }
-    // ---- pass 3: P.V, two tokens per dot2; a trip covers two 64-token blocks, and row group
-    // `g16` takes the pairs j = g16 and j = g16 + 16 of each.
+    // ---- pass 3: P.V, two tokens per dot2; a trip covers kPairs pairs (of 32 in a 64-token block) of each of the row
+    // groups, `g16` of them side by side.
     {
-      constexpr int kPairs = 4;
-      u32x4 vx[kPairs], vy[kPairs], nx[kPairs], ny[kPairs];
-      auto fetch_v = [&](int t0, u32x4* x, u32x4* y) {
+      u32x4 nx[kPairs], ny[kPairs];
+      if constexpr (!SPLIT) fetch_v(0, vx, vy);
+      for (int t0 = 0; t0 < Tc; t0 += kRows * kPairs * 2) {
+        const bool more = t0 + kRows * kPairs * 2 < Tc;
+        if (more) fetch_v(t0 + kRows * kPairs * 2, nx, ny);
 #pragma unroll
         for (int u = 0; u < kPairs; ++u) {
-          const int t = c0 + t0 + (u >> 1) * 64 + (u & 1) * 16 + g16;
-          x[u] = ZP_DEC_LOAD((const u32x4*)(row_base(p.v, p.v_sp, t) + offV));
-          y[u] = ZP_DEC_LOAD((const u32x4*)(row_base(p.v, p.v_sp, t + 32) + offV));
-        }
-      };
-      fetch_v(0, vx, vy);
-      for (int t0 = 0; t0 < Tc; t0 += 16 * kPairs * 2) {
-        const bool more = t0 + 16 * kPairs * 2 < Tc;
-        if (more) fetch_v(t0 + 16 * kPairs * 2, nx, ny);
-#pragma unroll
-        for (int u = 0; u < kPairs; ++u) {
-          const int t = t0 + (u >> 1) * 64 + (u & 1) * 16 + g16;  // partner is t + 32
+          const int t = t0 + pair_at(u);
           if (t < Tc) {
             uint32_t pp[G];
 #pragma unroll
@@ -287,7 +298,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4
       __syncthreads();   // the next slice's logits overwrite this slice's p
     }
   } else {
-    if (Tn > 0) slice(0, Tn);   // one pass: nothing is carried, the accumulators start at pass 3
+    const int Tc = min(per, Tn - first);
+    if (Tc > 0) slice(first, Tc);   // one pass: nothing is carried, the accumulators start at pass 3
   }
   float inv[G];
 #pragma unroll
@@ -311,12 +323,43 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4
       for (int i = 0; i < 8; ++i) part[(wave * G + g) * 128 + s16 * 8 + i] = acc[g][i];
   }
   __syncthreads();
+  if constexpr (SPLIT)
+    if (tid < G) {
+      float* const ml = p.part + (int64_t)p.B * p.Hq * p.splits * p.D + (((int64_t)b * p.Hq + h * G + tid) * p.splits + split) * 2;
+#pragma unroll
+      for (int g = 0; g < G; ++g)
+        if (tid == g) ml[0] = m_run[g], ml[1] = l_run[g];
+    }
   for (int e = tid; e < G * p.D; e += kThreads) {
     const int g = e / p.D, d = e - g * p.D;
     float s = 0.f;
 #pragma unroll
     for (int w = 0; w < kWaves; ++w) s += part[(w * G + g) * 128 + d];
-    Elem<T>::st(p.out, ((int64_t)b * p.Hq + h * G + g) * p.D + d, s * inv[g]);
+    if constexpr (SPLIT) p.part[(((int64_t)b * p.Hq + h * G + g) * p.splits + split) * p.D + d] = s;
+    else Elem<T>::st(p.out, ((int64_t)b * p.Hq + h * G + g) * p.D + d, s * inv[g]);
+  }
+}
+
+// Adds up the splits of one (sequence, head), each at the largest maximum.
+template <typename T>
+__global__ __launch_bounds__(64) void paged_combine_kernel(DecodeArgs p) {
+  const int64_t item = blockIdx.x;
+  const float* const ml = p.part + (int64_t)p.B * p.Hq * p.splits * p.D + item * p.splits * 2;
+  const int s0 = min((int)threadIdx.x, p.splits - 1);          // at most 64 of them
+  const float m = ml[2 * s0], mx = wave_max(m);
+  const float f = mx == -INFINITY || (int)threadIdx.x >= p.splits ? 0.f : __expf(m - mx), l = wave_sum(f * ml[2 * s0 + 1]);
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  for (int d = threadIdx.x * 2; d < p.D; d += 128) {
+    const float* const from = p.part + item * p.splits * p.D + d;
+    float2 r = {0.f, 0.f};
+#pragma unroll 8
+    for (int s = 0; s < p.splits; ++s) {
+      const float2 x = *(const float2*)(from + s * p.D);
+      const float w = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), s));
+      r.x += x.x * w; r.y += x.y * w;
+    }
+    Elem<T>::st(p.out, item * p.D + d, r.x * inv);
+    Elem<T>::st(p.out, item * p.D + d + 1, r.y * inv);
   }
 }
 
@@ -325,26 +368,46 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(G <= 4
 constexpr int kSingleSliceBytes = 72 * 1024;
 constexpr int kSliceTokens = 2048;
 
-template <typename T, int G>
-int launch_decode(DecodeArgs a, hipStream_t st) {
-  const int Tpad = (a.NB * a.BS + 63) & ~63;
-  const size_t part = sizeof(float) * kWaves * G * 128;
-  const bool chunked = sizeof(float) * (size_t)G * Tpad > kSingleSliceBytes;
-  a.chunk = chunked ? kSliceTokens : 0;
-  size_t smem = sizeof(float) * (size_t)G * (chunked ? kSliceTokens : Tpad);
+// Workgroups on a CU: one of 512 threads where all have a CU to themselves, for what then bounds it is bytes in flight (8
+// sequences of about 2150 tokens, 32 heads over 8 of 128 54 us with 256 threads, 40 with 512 and 42 with 1024); more are better
+// off with four of 256 (64 sequences of 450 28 and 30, 40 of 2150 77 and 80; 256 of 2150 357 and 361).
+constexpr int kCUs = 256;
+int decode_threads(const DecodeArgs& a) { return (int64_t)a.B * a.Hkv <= kCUs ? 512 : 256; }
+// Parts of a context: what makes a workgroup per CU, of 256 tokens and more, for a CU reads no more than 34 GB/s whatever is in flight.
+// us with one part: 8 sequences of about 1900 tokens, 32 heads over 8 39 -> 24, 16 heads 33 -> 21; 16 sequences 40 -> 31 and 35 -> 28; one
+// 37 -> 17; 12 of 900 25.2 -> 20.7.  More than fill the chip are slower (8 sequences in 8 parts 29), as are two parts of 24
+// sequences (43 -> 48); tables of fewer than 1024 tokens gain 1 to 3 us and lose as much of the host's time to a launch.
+int decode_splits(int B, int Hkv, int BS, int NB) {
+  const int64_t groups = (int64_t)B * Hkv, tokens = (int64_t)NB * BS;
+  if (2 * groups > kCUs || tokens < 1024) return 1;
+  const int64_t s = kCUs / groups < tokens / 256 ? kCUs / groups : tokens / 256;
+  return (int)(s < 64 ? s : 64);
+}
+template <typename T, int G, bool CHUNKED, bool SPLIT, int THREADS>
+int launch_decode(const DecodeArgs& a, size_t smem, hipStream_t st) {
+  const size_t part = sizeof(float) * (THREADS / 64) * G * 128;
   if (part > smem) smem = part;
-  const void* fn = chunked ? (const void*)paged_decode_kernel<T, G, true>
-                           : (const void*)paged_decode_kernel<T, G, false>;
-  if (smem > 64 * 1024 &&
-      hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
+  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)paged_decode_kernel<T, G, CHUNKED, SPLIT, THREADS>,
+                                              hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem) != hipSuccess) {
     zp_set_error("paged_decode_attention: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  const dim3 grid((unsigned)(a.B * a.Hkv));
-  if (chunked) hipLaunchKernelGGL((paged_decode_kernel<T, G, true>), grid, dim3(kThreads), smem, st, a);
-  else hipLaunchKernelGGL((paged_decode_kernel<T, G, false>), grid, dim3(kThreads), smem, st, a);
+  hipLaunchKernelGGL((paged_decode_kernel<T, G, CHUNKED, SPLIT, THREADS>), dim3((unsigned)(a.B * a.Hkv * a.splits)), dim3(THREADS), smem, st, a);
+  if (SPLIT) hipLaunchKernelGGL((paged_combine_kernel<T>), dim3((unsigned)(a.B * a.Hq)), dim3(64), 0, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
+}
+template <typename T, int G>
+int launch_decode(DecodeArgs a, hipStream_t st) {
+  const int Tpad = ((a.NB * a.BS + a.splits - 1) / a.splits + 63) & ~63;
+  const bool chunked = sizeof(float) * (size_t)G * Tpad > kSingleSliceBytes;
+  a.chunk = chunked ? kSliceTokens : 0;
+  if (chunked) a.splits = 1;
+  const size_t smem = sizeof(float) * (size_t)G * (chunked ? kSliceTokens : Tpad);
+  if (chunked) return launch_decode<T, G, true, false, 256>(a, smem, st);
+  if (a.splits > 1) return launch_decode<T, G, false, true, 512>(a, smem, st);
+  if (decode_threads(a) == 512) return launch_decode<T, G, false, false, 512>(a, smem, st);
+  return launch_decode<T, G, false, false, 256>(a, smem, st);
 }
 
 template <typename T>
@@ -398,12 +461,14 @@ extern "C" int zp_store_kvcache(const void* key, const void* value, void* k_cach
   return ZP_OK;
 }
 
-extern "C" int zp_paged_decode_attention(const void* q, const void* k_cache, const void* v_cache,
+static int64_t splits_bytes(int B, int Hq, int D, int splits) { return (int64_t)B * Hq * splits * (D + 2) * 4; }
+static int paged_decode(const void* q, const void* k_cache, const void* v_cache,
                                          const int32_t* block_tables, const int32_t* context_lens,
                                          void* out, int32_t B, int32_t Hq, int32_t Hkv, int32_t D,
                                          int32_t BS, int32_t NB, int32_t num_pages,
                                          int64_t k_stride_page, int64_t v_stride_page,
-                                         float softmax_scale, int32_t dtype, void* stream) {
+                                         float softmax_scale, int32_t dtype, void* workspace, int64_t workspace_bytes, int splits,
+                                         void* stream) {
   ZP_REQUIRE(q && k_cache && v_cache && block_tables && context_lens && out,
              "paged_decode_attention: null pointer");
   ZP_REQUIRE(B >= 0 && Hq > 0 && Hkv > 0 && D > 0 && BS > 0 && NB > 0,
@@ -422,15 +487,44 @@ extern "C" int zp_paged_decode_attention(const void* q, const void* k_cache, con
                  (k_stride_page * 2) % 16 == 0 && (v_stride_page * 2) % 16 == 0,
              "paged_decode_attention: tensors must be 16-byte aligned");
   if (B == 0) return ZP_OK;
+  ZP_REQUIRE(splits == 1 || (workspace && (uintptr_t)workspace % 16 == 0 && workspace_bytes >= splits_bytes(B, Hq, D, splits)),
+             "paged_decode_attention: workspace of %lld bytes", (long long)workspace_bytes);
   DecodeArgs a;
   a.q = (const char*)q; a.k = (const char*)k_cache; a.v = (const char*)v_cache;
   a.table = block_tables; a.ctx = context_lens; a.out = out;
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.G = Hq / Hkv; a.D = D; a.BS = BS; a.NB = NB;
   a.num_pages = num_pages; a.k_sp = k_stride_page; a.v_sp = v_stride_page; a.scale = softmax_scale;
+  a.splits = splits; a.part = (float*)workspace;
   a.bs_shift = -1;
   if ((BS & (BS - 1)) == 0)
     for (a.bs_shift = 0; (1 << a.bs_shift) < BS; ++a.bs_shift) {}
   hipStream_t st = (hipStream_t)stream;
   if (dtype == ZP_BF16) return dispatch_group<BF16>(a, st);
   return dispatch_group<F16>(a, st);
+}
+
+extern "C" int zp_paged_decode_attention(const void* q, const void* k_cache, const void* v_cache,
+                                         const int32_t* block_tables, const int32_t* context_lens,
+                                         void* out, int32_t B, int32_t Hq, int32_t Hkv, int32_t D,
+                                         int32_t BS, int32_t NB, int32_t num_pages,
+                                         int64_t k_stride_page, int64_t v_stride_page,
+                                         float softmax_scale, int32_t dtype, void* stream) {
+  return paged_decode(q, k_cache, v_cache, block_tables, context_lens, out, B, Hq, Hkv, D, BS, NB, num_pages, k_stride_page,
+                      v_stride_page, softmax_scale, dtype, nullptr, 0, 1, stream);
+}
+extern "C" int64_t zp_paged_decode_workspace(int32_t B, int32_t Hq, int32_t Hkv, int32_t D, int32_t BS, int32_t NB) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || D <= 0 || BS <= 0 || NB <= 0) return 0;
+  const int splits = decode_splits(B, Hkv, BS, NB);
+  return splits > 1 ? splits_bytes(B, Hq, D, splits) : 0;
+}
+extern "C" int zp_paged_decode_parts(const void* q, const void* k_cache, const void* v_cache,
+                                         const int32_t* block_tables, const int32_t* context_lens,
+                                         void* out, int32_t B, int32_t Hq, int32_t Hkv, int32_t D,
+                                         int32_t BS, int32_t NB, int32_t num_pages,
+                                         int64_t k_stride_page, int64_t v_stride_page,
+                                         float softmax_scale, int32_t dtype, void* workspace,
+                                         int64_t workspace_bytes, void* stream) {
+  const int splits = B > 0 && Hq > 0 && Hkv > 0 && BS > 0 && NB > 0 ? decode_splits(B, Hkv, BS, NB) : 1;
+  return paged_decode(q, k_cache, v_cache, block_tables, context_lens, out, B, Hq, Hkv, D, BS, NB, num_pages, k_stride_page,
+                      v_stride_page, softmax_scale, dtype, workspace, workspace_bytes, splits, stream);
 }

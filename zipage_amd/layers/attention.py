@@ -47,9 +47,12 @@ def paged_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     assert block_tables.is_contiguous() and context_lens.is_contiguous()
     assert q.dtype == k_cache.dtype == v_cache.dtype
     out = torch.empty_like(q)
-    _lib.call("zp_paged_decode_attention", _lib.dev_ptr(q), _lib.dev_ptr(k_cache),
+    NB = block_tables.shape[1]
+    size = _lib.size("zp_paged_decode_workspace", B, Hq, Hkv, D, BS, NB)
+    ws = q.new_empty(size // 2) if size else None
+    _lib.call("zp_paged_decode_parts", _lib.dev_ptr(q), _lib.dev_ptr(k_cache),
               _lib.dev_ptr(v_cache), _lib.dev_ptr(block_tables), _lib.dev_ptr(context_lens),
-              _lib.dev_ptr(out), B, Hq, Hkv, D, BS, block_tables.shape[1], num_pages,
+              _lib.dev_ptr(out), B, Hq, Hkv, D, BS, NB, num_pages,
               k_cache.stride(0), v_cache.stride(0), float(softmax_scale), _lib.dtype_tag(q),
-              _lib.stream_ptr(q))
+              _lib.dev_ptr(ws), size, _lib.stream_ptr(q))
     return out
