@@ -1129,6 +1129,34 @@ __device__ __forceinline__ int half_max_i(int v) {
   return max(v, lane_xor16(v));
 }
 
+// The largest of each of sixteen values over the 32 lanes of a wave half, left in x[0] of lane i for value r (returned), i and i + 16
+// alike: each step halves the values that a lane still has, so they take fifty instructions instead of 112.
+__device__ __forceinline__ int sixteen_half_max(int (&x)[16], int lane) {
+#define ZP_DPP(V, CTRL) __builtin_amdgcn_update_dpp(0, V, CTRL, 0xf, 0xf, false)
+  const bool b0 = lane & 1, b1 = lane & 2, b2 = lane & 4, b3 = lane & 8;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {      // quad_perm [1,0,3,2]: lane ^ 1
+    const int lo = max(x[2 * i], ZP_DPP(x[2 * i], 0xB1)), hi = max(x[2 * i + 1], ZP_DPP(x[2 * i + 1], 0xB1));
+    x[i] = b0 ? hi : lo;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {      // quad_perm [2,3,0,1]: lane ^ 2
+    const int lo = max(x[2 * i], ZP_DPP(x[2 * i], 0x4E)), hi = max(x[2 * i + 1], ZP_DPP(x[2 * i + 1], 0x4E));
+    x[i] = b1 ? hi : lo;
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {      // lane ^ 8
+    const int lo = max(x[2 * i], dpp_row_ror<8>(x[2 * i])), hi = max(x[2 * i + 1], dpp_row_ror<8>(x[2 * i + 1]));
+    x[i] = b3 ? hi : lo;
+  }
+  // row_half_mirror of quad_perm [3,2,1,0]: lane ^ 4
+  const int lo = max(x[0], ZP_DPP(ZP_DPP(x[0], 0x1B), 0x141)), hi = max(x[1], ZP_DPP(ZP_DPP(x[1], 0x1B), 0x141));
+#undef ZP_DPP
+  const int v = b2 ? hi : lo;
+  x[0] = max(v, lane_xor16(v));
+  return (lane & 3) | (b3 ? 4 : 0) | (b2 ? 8 : 0);
+}
+
 // The 16-bit MFMA of the cache dtype: products of cache elements are exact in fp32.
 typedef _Float16 f16x8_t __attribute__((ext_vector_type(8)));
 template <typename T> struct Mfma16;
@@ -1226,7 +1254,8 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
   float* l_rn = l_sum2 + 2 * kPageRows;                // 1 / norm
   int* l_col = (int*)(l_rn + kPageRows);
   int* l_bexp = l_col + kPageRows;                     // [kPageWaves] scale exponent of a block's rn pieces
-  int* l_code = l_bexp + kPageWaves;                   // [NB] the block table row
+  int* l_any2 = l_bexp + kPageWaves;                   // [2] whether a key of the page has a claim
+  int* l_code = l_any2 + 2;                            // [NB] the block table row
 
   const int tid = threadIdx.x;
 #ifdef ZP_PAGE_STAMP
@@ -1310,6 +1339,7 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
     const int64_t obase = rowbase + (int64_t)jp * p.BS;
     const int tix = wave * 64 + lane;
     if (tix < kPageRows) { l_col[tix] = -1; l_corr[tix] = 0ull; }
+    if (tix == 0) l_any2[par] = 0;
     ZP_PSTAMP();   // 1
 
     // ---- norms from the diagonal of the Gram matrix: wave a multiplies its own block (a, a) as
@@ -1448,22 +1478,25 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
       for (int r = 0; r < 16; ++r) dcol[r] = -1;
       const int nd = nrb / 2 + ((nrb & 1) || a < nrb / 2 ? 1 : 0);   // distances 0 .. nd-1
       // what a tile feeds: the last column over the threshold of the keys on both of its sides
+      bool dense = false;             // the last tile had claims: the next is likely to, and nothing asks first
       auto scan = [&](const f32x16_t& acc, int cb, bool off_diagonal) {
         const int cslot = cb * 32 + col;
         const float rn_col = l_rn[cslot];
         // most tiles hold no entry over the threshold, and one maximum decides.  With a positive
         // threshold only positive products matter, and those are at most the largest product
         // times the largest row factor: that bound needs no multiplication per entry.
-        if (thr_lo > 0.f) {
+        if (thr_lo > 0.f && !dense) {
           float amax = 0.f;
 #pragma unroll
           for (int r = 0; r < 16; ++r) amax = fmaxf(amax, acc[r]);
           if (!__any(amax * rn_max * rn_col > thr_lo)) return;
         }
-        float big = -INFINITY;
+        if (!dense) {
+          float big = -INFINITY;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) big = fmaxf(big, acc[r] * rn_row[r]);
-        if (!__any(big * rn_col > thr_lo)) return;
+          for (int r = 0; r < 16; ++r) big = fmaxf(big, acc[r] * rn_row[r]);
+          if (!__any(big * rn_col > thr_lo)) return;
+        }
         // row side: key (a, r) sees column cslot; column side (off the diagonal block, where both
         // (i, j) and (j, i) are computed): key cslot sees the rows of block a, whose index grows
         // with r inside a lane, so the last hit is the largest
@@ -1474,7 +1507,8 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
           dcol[r] = max(dcol[r], over ? cslot : -1);
           rlast = over ? r : rlast;
         }
-        if (off_diagonal && __any(rlast >= 0)) {
+        dense = __any(rlast >= 0);
+        if (off_diagonal && dense) {
           int ci = rlast < 0 ? -1 : a * 32 + (rlast >> 2) * 8 + half * 4 + (rlast & 3);
           ci = max(ci, lane_xor32(ci));
           if (half == 0 && ci >= 0) atomicMax(&l_col[cslot], ci);
@@ -1507,12 +1541,9 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
 #pragma unroll
       for (int r = 0; r < 16; ++r) mine |= dcol[r] >= 0;
       if (__any(mine)) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int c = half_max_i(dcol[r]);
-          if (col == 0 && c >= 0)
-            atomicMax(&l_col[a * 32 + (r >> 2) * 8 + half * 4 + (r & 3)], c);
-        }
+        const int r = sixteen_half_max(dcol, lane);
+        if (lane == 0) l_any2[par] = 1;
+        if ((lane & 16) == 0 && dcol[0] >= 0) atomicMax(&l_col[a * 32 + (r >> 2) * 8 + half * 4 + (r & 3)], dcol[0]);
       }
     }
     ZP_PSTAMP();   // 5: tiles of wave 0
@@ -1520,6 +1551,39 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
     __syncthreads();
     ZP_PSTAMP();   // 6: tiles of all waves, key sum planes
 
+    // ---- value of every key's claimed entry, subtracted from the row it was taken from.  Several
+    // keys may claim from one row: the values are added as 2^-32 fixed point with integer atomics,
+    // which is exact for a cosine above 2^-8 and does not depend on the order of the additions.
+    // Two lanes per key: theirs are the pieces of its row that the tiles were multiplied with, and those of the row it claims
+    // from, which is still in LDS, so a wave is done with its 32 keys at once; the sixteen pieces' sums are added as a
+    // tree, pieces eight apart first.  With both rows from the cache, four keys at a time: 64 rows of 9 pages whose keys nearly all
+    // have a claim 163 us, now 114; without claims 75 either way.
+    if (__builtin_amdgcn_readfirstlane(l_any2[par]) != 0) {
+      const int key = wave * 32 + col;
+      const int cl = wave < nrb ? l_col[key] : -1;
+      // cl == key: with a negative threshold the zeroed diagonal entry itself can be the claim; its
+      // value is 0, nothing to hand back
+      const bool claimed = cl >= 0 && cl != key;
+      if (__any(claimed)) {
+        const int c = claimed ? cl : key;
+        const char* crow = k_pl + (c >> 2) * kPgGrp + (c & 3) * 64 + half * 16;
+        float t[KSB];
+#pragma unroll
+        for (int s = 0; s < KSB; ++s) {
+          float ej[8], ec[8];
+          Unpack<T>::run(__builtin_bit_cast(vec16, ak[s]), ej);
+          Unpack<T>::run(*(const vec16*)(crow + (s >> 1) * 256 + (s & 1) * 32), ec);
+          t[s] = 0.f;
+#pragma unroll
+          for (int e = 0; e < 8; ++e) t[s] = fmaf(ej[e], ec[e], t[s]);
+        }
+        static_assert(KSB == 8, "sixteen pieces");
+        float v = ((t[0] + t[4]) + (t[2] + t[6])) + ((t[1] + t[5]) + (t[3] + t[7]));
+        v += lane_xor32(v);
+        if (claimed && half == 0) atomicAdd(&l_corr[c], to_fixed32(v * (l_rn[key] * l_rn[c])));
+      }
+      __syncthreads();
+    }
     // ---- nothing below reads the page in LDS: the next page of the row is requested now and
     // lands while this one finishes
     const int nj = next_valid(jp + p.parts);
@@ -1548,46 +1612,6 @@ __global__ __launch_bounds__(kPageThreads, 4) void gram_page_kernel(GramArgs p) 
           v.z = t[4 * q + 2] * rn_row[4 * q + 2] - v.z;
           v.w = t[4 * q + 3] * rn_row[4 * q + 3] - v.w;
           *dst = v;
-        }
-      }
-    }
-    // ---- value of every key's claimed entry, subtracted from the row it was taken from.  Several
-    // keys may claim from one row: the values are added as 2^-32 fixed point with integer atomics,
-    // which is exact for a cosine above 2^-8 and does not depend on the order of the additions.
-    // Wave w looks at the keys 32 w .. 32 w + 31 at once (most have no claim) and then handles the
-    // ones that have, four at a time with sixteen lanes per key; the two key rows come from
-    // global memory (the cache: the page was read a moment ago).
-    {
-      static_assert(PIECES == 16, "sixteen lanes per key");
-      const int key = wave * 32 + col;
-      const int cl = key < p.BS ? l_col[key] : -1;
-      // cl == key: with a negative threshold the zeroed diagonal entry itself can be the claim; its
-      // value is 0, nothing to hand back
-      unsigned todo = (unsigned)__builtin_amdgcn_ballot_w64(half == 0 && cl >= 0 && cl != key);
-      const int q = lane >> 4, piece = lane & 15;
-      while (todo) {
-        unsigned m = todo;           // the q-th lowest key with a claim goes to lane group q
-#pragma unroll
-        for (int i = 0; i < 3; ++i) m = i < q ? m & (m - 1) : m;
-        const int jl = m ? __builtin_ctz(m) : -1;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) todo &= todo - 1;
-        const int c = __builtin_amdgcn_ds_bpermute((jl < 0 ? 0 : jl) << 2, cl);
-        if (jl >= 0) {               // uniform over the 16 lanes of a key
-          const int j = wave * 32 + jl;
-          u32x4 kj = u32x4{0u, 0u, 0u, 0u}, kc = kj;
-          if (piece < dpieces) {
-            kj = *(const u32x4*)(page + (int64_t)j * k_row + piece * 16);
-            kc = *(const u32x4*)(page + (int64_t)c * k_row + piece * 16);
-          }
-          float ej[8], ec[8];
-          Unpack<T>::run(vec16{kj.x, kj.y, kj.z, kj.w}, ej);
-          Unpack<T>::run(vec16{kc.x, kc.y, kc.z, kc.w}, ec);
-          float t = 0.f;
-#pragma unroll
-          for (int e = 0; e < 8; ++e) t = fmaf(ej[e], ec[e], t);
-          t = pieces_sum<PIECES>(t);
-          if (piece == 0) atomicAdd(&l_corr[c], to_fixed32(t * (l_rn[j] * l_rn[c])));
         }
       }
     }
@@ -2601,8 +2625,8 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
   if constexpr (T::bytes == 2 && !RAW) {
     // the block table row sits in LDS
     const size_t smem = (size_t)kPgBytes + 4 * kDmax * 2 + 4 * kPageRows * 2 +
-                        (size_t)kPageRows * (2 * 8 + 2 * 4 + 4 + 4) + sizeof(int) * (kPageWaves + a.NB);
-    if (a.BS <= kPageRows && a.BS % 32 == 0 && smem <= 80 * 1024) {
+                        (size_t)kPageRows * (2 * 8 + 2 * 4 + 4 + 4) + sizeof(int) * (kPageWaves + 2 + a.NB);
+    if (a.BS <= kPageRows && a.BS % 32 == 0 && smem <= 80 * 1024 + 8) {
       const GramArgs w = page_walks(a, L, 2);
       grid = dim3((unsigned)((int64_t)L * a.B * a.Hkv * w.parts));
       if (hipFuncSetAttribute((const void*)gram_page_kernel<T>,
