@@ -260,7 +260,7 @@ RAW_ORACLE_ROUNDING = "reference"
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("bs,d", [(256, 128), (192, 128), (64, 64), (128, 40), (256, 72)])
 def test_pages_of_many_and_of_no_claims(dev, dtype, bs, d):
     """Pages whose keys nearly all have a claim (one or six directions, cosines of 0.9 and more within one), with few such keys and with none
@@ -276,18 +276,19 @@ def test_pages_of_many_and_of_no_claims(dev, dtype, bs, d):
             axes = torch.linalg.qr(torch.randn(d, d, generator=g))[0][:directions] * d ** 0.5
             near = axes[torch.randint(0, directions, (bs,), generator=g)] + 0.2 * torch.randn(bs, d, generator=g)
             k[0, p, :, h] = torch.where(torch.rand(bs, 1, generator=g) < share, near, k[0, p, :, h])
-    k = _clear_of_norm_boundaries(k.to(dtype))
+    if dtype != torch.float32:
+        k = _clear_of_norm_boundaries(k.to(dtype))
     enc = encode_block_table([[0, 3, 6, 9, 12], [1, 2, 5, 4], [13, 7, 8, 10, 11]])
     kw = dict(threshold=0.7, temperature=0.4, return_logits=True)
     wl, wr = O.lightning_redudancy_score(k, enc, **kw)
     gl, gr = (t.cpu() for t in K.lightning_redudancy_score(k.to(dev), enc.to(dev), **kw))
     # a sum of up to bs cosines in fp32 on both sides, however much of it cancels, and one rounding of it; and of the softmax, whose
-    # exponents the sums' last places move
-    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    # exponents the sums' last places move.  fp32 cosines carry an error of 2^-23 themselves.
+    eps = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11, torch.float32: 2.0 ** -22}[dtype]
     for got, want, places in ((gl, wl, 1), (gr, wr, 4)):
         got, want = got.double(), want.double()
         there = torch.isfinite(want)
         assert torch.equal(there, torch.isfinite(got))
         got, want = got[there], want[there]
-        assert bool(((got - want).abs() <= places * 2 * eps * torch.maximum(got.abs(), want.abs()) + bs * 2.0 ** -22).all())
-    assert float((gl == wl).float().mean()) > 0.9
+        assert bool(((got - want).abs() <= places * 2 * eps * torch.maximum(got.abs(), want.abs()) + bs * 2.0 ** -21).all())
+    assert dtype == torch.float32 or float((gl == wl).float().mean()) > 0.9
