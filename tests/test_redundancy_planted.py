@@ -292,3 +292,27 @@ def test_pages_of_many_and_of_no_claims(dev, dtype, bs, d):
         got, want = got[there], want[there]
         assert bool(((got - want).abs() <= places * 2 * eps * torch.maximum(got.abs(), want.abs()) + bs * 2.0 ** -21).all())
     assert dtype == torch.float32 or float((gl == wl).float().mean()) > 0.9
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bs,lengths", [(64, [16, 1, 7]), (64, [17, 2]), (64, [66, 65]), (128, [5, 16, 2])])
+def test_raw_fp32_rows_of_many_pages(dev, bs, lengths):
+    """Tables on both sides of sixteen pages (the sums of pairs of pages) and of 64, rows shorter than they are, and a claim at most keys."""
+    from zipage_amd import kernel as K
+    from oracle.zipage_oracle import encode_block_table
+    g = torch.Generator().manual_seed(bs + lengths[0])
+    pages, heads, d = sum(lengths), 1, 32
+    axes = torch.linalg.qr(torch.randn(d, d, generator=g))[0][:5] * d ** 0.5
+    k = axes[torch.randint(0, 5, (1, pages, bs, heads), generator=g)] + 0.2 * torch.randn(1, pages, bs, heads, d, generator=g)
+    order = torch.randperm(pages, generator=g).tolist()
+    enc = encode_block_table([[order.pop() for _ in range(n)] for n in lengths])
+    kw = dict(threshold=0.7, temperature=0.4, return_logits=True)
+    wl, wr = O.raw_redudancy_score(k, enc, **kw)
+    gl, gr = (t.cpu() for t in K.raw_redudancy_score(k.to(dev), enc.to(dev), **kw))
+    # up to bs * pages cosines in fp32 on both sides, each with an error of 2^-23, and the softmax of their sums
+    for got, want in ((gl, wl), (gr, wr)):
+        got, want = got.double(), want.double()
+        there = torch.isfinite(want)
+        assert torch.equal(there, torch.isfinite(got))
+        got, want = got[there], want[there]
+        assert bool(((got - want).abs() <= 2.0 ** -18 * torch.maximum(got.abs(), want.abs()) + bs * max(lengths) * 2.0 ** -21).all())
