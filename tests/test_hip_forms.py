@@ -372,6 +372,7 @@ def test_products_in_parts(dev, dtype, n, K, M):
         _lib.call_models("zp_split_rows_linear", *args(257, size))
 
 
+@torch.inference_mode()
 def test_products_in_parts_under_capture(dev):
     """Through the entry point, in a graph that is replayed on new rows."""
     from zipage_amd.layers import linear
