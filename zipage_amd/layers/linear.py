@@ -67,6 +67,8 @@ def _split_rows(n: int, k: int, m: int) -> bool:
     idle (us of both: 64 rows, 12 288 -> 4096 25.5 and 36.3, 4096 -> 6144 17.2 and 17.6; 128 rows 31.1 and 66.0, 21.1 and 25.0; 192 rows 37
     and 89, 25.0 and 33.3; 256 rows 41 and 53, 28 and 39.5; 4096 -> 4096 17.3 and 23.5 for 128 rows, 21.6 and 31.5 for 192), and up to 64
     rows outputs of many rounds of workgroups (64 rows, 4096 -> 151 936 227 and 262; 48 rows, 1024 -> 151 936 66 and 77; 96 rows 259 and 273).
+    Outputs that make one full round of them, in one part: up to 128 rows, 4096 -> 32 768 54 and 61 (64 rows), 51 and 67 (24), 58 and 64 (128),
+    2560 -> 32 512 33 and 44.
     The library's choices are uneven, so the lines are drawn where 95 % of random sizes are no slower (300 sizes: 1.35 times as fast on
     average): it is good at 6144 and 8192 -> 1280 and fewer (32 to 128 rows, 10.9 and 9.7), at contractions of 4096 of some rows (80 rows,
     -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
@@ -75,6 +77,8 @@ def _split_rows(n: int, k: int, m: int) -> bool:
         return False
     if m >= 73728:
         return k >= 1024 and n <= 64 or k >= 2048 and n <= 112 and m >= 131072
+    if n <= 128 and 26880 <= m <= 32768:
+        return 2048 <= k <= 12288
     if k < 2560 or m < 1280 and 6144 <= k <= 8192:
         return False
     if n <= 32:
