@@ -117,7 +117,7 @@ def test_which_sizes_are_row_tiles(n, k, m, tiles):
                                          (129, 4096, 24576, False), (129, 4096, 6144, True), (192, 4096, 4096, True), (193, 4096, 4096, False),
                                          (256, 4096, 6144, True), (256, 12288, 4096, True), (257, 12288, 4096, False), (256, 4064, 6144, False),
                                          (128, 4096, 32768, True), (129, 4096, 32768, False), (24, 2048, 26880, True), (64, 2016, 32768, False),
-                                         (64, 4096, 26876, False), (64, 4096, 32772, False), (100, 6160, 4096, False), (100, 6144, 4098, False)])
+                                         (64, 4096, 26876, False), (64, 4096, 32772, False), (255, 4096, 6144, False), (224, 4096, 6144, True), (100, 6160, 4096, False), (100, 6144, 4098, False)])
 def test_which_sizes_are_split(n, k, m, split):
     from zipage_amd.layers.linear import _split_rows
     assert _split_rows(n, k, m) == split

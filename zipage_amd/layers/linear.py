@@ -71,7 +71,7 @@ def _split_rows(n: int, k: int, m: int) -> bool:
     2560 -> 32 512 33 and 44.
     The library's choices are uneven, so the lines are drawn where 95 % of random sizes are no slower (300 sizes: 1.35 times as fast on
     average): it is good at 6144 and 8192 -> 1280 and fewer (32 to 128 rows, 10.9 and 9.7), at contractions of 4096 of some rows (80 rows,
-    -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
+    -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0; 255, -> 6144 28.0 and 26.3, but 224 26.6 and 36.2), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
     its tiles fill the chip (256 rows, 4096 -> 24 576 64 and 62; but 128 rows 45.3 and 48.3)."""
     if not 16 < n <= 256 or k % 32 or m % 4 or m < 512:
         return False
@@ -94,7 +94,7 @@ def _split_rows(n: int, k: int, m: int) -> bool:
         return False
     if n <= 192:
         return k >= 5888 or 2816 <= m <= (6656 if k < 4608 else 12288)
-    return k >= 7168 or m >= 5888
+    return k >= 7168 or m >= 5888 and (k > 4608 or n % 32 == 0)
 
 
 def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
