@@ -351,6 +351,9 @@ int zp_paged_decode_parts(const void* q, const void* k_cache, const void* v_cach
 int zp_add_rms_norm(const void* x, void* residual, const void* weight, void* out,
                     int32_t n, int32_t hidden, int64_t x_stride, int64_t r_stride,
                     int64_t out_stride, float eps, int32_t dtype, void* stream);
+/* The same of a product that is left in parts, (parts, n, hidden) fp32, whose sum is rounded to the dtype first. */
+int zp_add_rms_norm_parts(const float* planes, int32_t parts, void* residual, const void* weight, void* out, int32_t n,
+                          int32_t hidden, int64_t r_stride, int64_t out_stride, float eps, int32_t dtype, void* stream);
 
 /* out = silu(gate_up[:, :I]) * gate_up[:, I:]  (SiluAndMul, zipage/models/qwen3.py:108-111). */
 int zp_silu_and_mul(const void* gate_up, void* out, int32_t n, int32_t intermediate,

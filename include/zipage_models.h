@@ -73,7 +73,7 @@ int zp_few_rows_linear(const void* x, const void* w, void* out, int32_t n, int32
 int zp_row_tiles_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
                         int64_t out_stride, int32_t dtype, void* stream);
 /* The same in parts of the contraction, whose fp32 sums lie in the workspace (zp_split_rows_workspace bytes, 16-byte aligned) on
-   the way: at most 256 rows. */
+   the way: at most 256 rows.  A null `out` leaves it at the parts, (parts, n, M) where there is a workspace. */
 int64_t zp_split_rows_workspace(int32_t n, int32_t K, int32_t M);
 int zp_split_rows_linear(const void* x, const void* w, void* out, int32_t n, int32_t K, int32_t M, int64_t x_stride,
                          int64_t out_stride, int32_t dtype, void* workspace, int64_t workspace_bytes, void* stream);

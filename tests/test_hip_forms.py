@@ -372,6 +372,26 @@ def test_products_in_parts(dev, dtype, n, K, M):
         _lib.call_models("zp_split_rows_linear", *args(257, size))
 
 
+@pytest.mark.parametrize("dtype", [BF16, torch.float16])
+@pytest.mark.parametrize("n,K,M", [(17, 12288, 4096), (40, 4096, 1024), (100, 6144, 2048), (256, 8192, 1288), (40, 128, 4096), (5, 4096, 4096)])
+def test_norms_of_products_in_parts(dev, dtype, n, K, M):
+    """The norm that adds the parts up: what the product and the norm after it give; products that are made whole stay what they are."""
+    from zipage_amd.layers import linear, linear_parts, rms_norm, rms_norm_parts
+    x, w = _rand(n, K, seed=1, dtype=dtype).to(dev), (_rand(M, K, seed=2).float() * K ** -0.5).to(dtype).to(dev)
+    weight, resid = _rand(M, seed=3, dtype=dtype).to(dev), _rand(n, M, seed=4, dtype=dtype).to(dev)
+    parts, whole = linear_parts(x, w), linear(x, w)
+    assert parts.dim() == (3 if 16 < n and K > 128 else 2)
+    if parts.dim() == 2:
+        assert torch.equal(parts, whole)
+        return
+    want, got = rms_norm(whole, weight, 1e-6, resid.clone()), rms_norm_parts(parts, weight, 1e-6, resid.clone())
+    assert torch.equal(want[1].view(torch.int16), got[1].view(torch.int16))
+    # fp16: one instruction may multiply and round to 16 bits, or two, which round a value beside a tie twice: a unit in the last place
+    # (2^-10) before the weight, and the rounding after it; bf16 has no such instruction
+    assert bool(((want[0].double() - got[0].double()).abs() <= (2.0 ** -9 if dtype == torch.float16 else 0.0) * want[0].double().abs()).all())
+    assert float((want[0] == got[0]).float().mean()) > 0.999
+
+
 @torch.inference_mode()
 def test_products_in_parts_under_capture(dev):
     """Through the entry point, in a graph that is replayed on new rows."""

@@ -53,6 +53,7 @@ SIGNATURES = {
     "zp_paged_decode_parts": [ptr, ptr, ptr, ptr, ptr, ptr, i32, i32, i32, i32, i32, i32, i32,
                               i64, i64, f32, i32, ptr, i64, ptr],
     "zp_add_rms_norm": [ptr, ptr, ptr, ptr, i32, i32, i64, i64, i64, f32, i32, ptr],
+    "zp_add_rms_norm_parts": [ptr, i32, ptr, ptr, ptr, i32, i32, i64, i64, f32, i32, ptr],
     "zp_silu_and_mul": [ptr, ptr, i32, i32, i64, i64, i32, ptr],
     "zp_qk_norm_rope_store": [ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, ptr, i32, i32,
                               i32, i32, i32, i64, i64, i32, i32, i64, i64, f32, i32, ptr],

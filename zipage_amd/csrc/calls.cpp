@@ -74,7 +74,7 @@ PyMethodDef entries[] = {
     ZP_ENTRY(zp_compress_layers_workspace_few), ZP_ENTRY(zp_compress_layers), ZP_ENTRY(zp_static_scratch_init),
     ZP_ENTRY(zp_compress_layers_static), ZP_ENTRY(zp_store_kvcache), ZP_ENTRY(zp_paged_decode_attention),
     ZP_ENTRY(zp_paged_decode_workspace), ZP_ENTRY(zp_paged_decode_parts),
-    ZP_ENTRY(zp_add_rms_norm), ZP_ENTRY(zp_silu_and_mul), ZP_ENTRY(zp_qk_norm_rope_store), ZP_ENTRY(zp_embed_norm),
+    ZP_ENTRY(zp_add_rms_norm), ZP_ENTRY(zp_add_rms_norm_parts), ZP_ENTRY(zp_silu_and_mul), ZP_ENTRY(zp_qk_norm_rope_store), ZP_ENTRY(zp_embed_norm),
     ZP_ENTRY(zp_residual_norm), ZP_ENTRY(zp_normed_powers), ZP_ENTRY(zp_xielu), ZP_ENTRY(zp_relu_square), ZP_ENTRY(zp_softcap),
     ZP_ENTRY(zp_gather_rows), ZP_ENTRY(zp_few_rows_linear), ZP_ENTRY(zp_row_tiles_linear), ZP_ENTRY(zp_split_rows_linear),
     ZP_ENTRY(zp_split_rows_workspace), ZP_ENTRY(zp_run_attention), ZP_ENTRY(zp_causal_attention),

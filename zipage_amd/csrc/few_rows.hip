@@ -310,7 +310,7 @@ template <typename T, int TT, int MT> int launch_split(SplitArgs a, hipStream_t 
   }
   const int64_t total = (int64_t)a.parts * a.col_tiles * a.row_tiles;
   hipLaunchKernelGGL((split_rows_kernel<T, TT, MT>), dim3((unsigned)((total + 7) / 8 * 8)), dim3(512), smem, st, a);
-  if (a.parts > 1)
+  if (a.parts > 1 && a.out)
     hipLaunchKernelGGL((split_sum_kernel<T>), dim3((unsigned)(((int64_t)a.n * a.M + 1023) / 1024)), dim3(256), 0, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
@@ -364,8 +364,9 @@ extern "C" int zp_split_rows_linear(const void* x, const void* w, void* out, int
     return ZP_EUNSUPPORTED;
   }
   if (n == 0) return ZP_OK;
-  ZP_REQUIRE(x && w && out && aligned16(x) && aligned16(w) && ((uintptr_t)out & 7) == 0, "split_rows_linear: null or unaligned pointer");
   const SplitPlan p = split_plan(n, K, M);
+  ZP_REQUIRE(x && w && (out || p.parts > 1) && aligned16(x) && aligned16(w) && ((uintptr_t)out & 7) == 0,
+             "split_rows_linear: null or unaligned pointer");
   ZP_REQUIRE(p.parts == 1 || (workspace && aligned16(workspace) && workspace_bytes >= (int64_t)p.parts * n * M * 4),
              "split_rows_linear: workspace of %lld bytes", (long long)workspace_bytes);
   SplitArgs a;

@@ -14,8 +14,8 @@ import torch
 import torch.nn.functional as F
 
 from zipage_amd.kernel import store_query_cache
-from zipage_amd.layers import (causal_attention, gather_rows, linear, paged_decode_attention, qk_norm_rope_store, rms_norm,
-                               silu_and_mul, step_product)
+from zipage_amd.layers import (causal_attention, gather_rows, linear, linear_parts, paged_decode_attention,
+                               qk_norm_rope_store, rms_norm, rms_norm_parts, silu_and_mul, step_product)
 
 from .inputs import plan_prompts
 
@@ -77,6 +77,15 @@ class StepContext:
     # the same portions for recurrent layers: those attended one by one, and the runs
     segments: Segments | None = None
     run_segments: Segments | None = None
+
+
+def _parts(product):
+    """What a product that only `_add_norm` reads is made with."""
+    return linear_parts if product is linear else product
+
+
+def _add_norm(hidden, weight, eps, resid):
+    return (rms_norm if hidden.dim() == 2 else rms_norm_parts)(hidden, weight, eps, resid)
 
 
 class Qwen3:
@@ -204,7 +213,7 @@ class Qwen3:
                                    ctx.query_slot_mapping)
             o = paged_decode_attention(q, kc, vc, ctx.context_lens, ctx.block_tables,
                                        self.scale).view(N, q_sz)
-        return product(o, p["wo"])
+        return _parts(product)(o, p["wo"])
 
     # ------------------------------------------------------------------ forward
     @torch.inference_mode()
@@ -220,11 +229,11 @@ class Qwen3:
             if resid is None:
                 resid, h = hidden, rms_norm(hidden, p["ln1"], s.eps)
             else:
-                h, resid = rms_norm(hidden, p["ln1"], s.eps, resid)
+                h, resid = _add_norm(hidden, p["ln1"], s.eps, resid)
             hidden = self._attention(li, p, h, pos32, ctx, plan)
-            h, resid = rms_norm(hidden, p["ln2"], s.eps, resid)
-            hidden = product(silu_and_mul(product(h, p["wgu"])), p["wd"])
-        h, _ = rms_norm(hidden, self.final_norm, s.eps, resid)
+            h, resid = _add_norm(hidden, p["ln2"], s.eps, resid)
+            hidden = _parts(product)(silu_and_mul(product(h, p["wgu"])), p["wd"])
+        h, _ = _add_norm(hidden, self.final_norm, s.eps, resid)
         return h
 
     @torch.inference_mode()

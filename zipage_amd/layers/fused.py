@@ -20,6 +20,17 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.
     return out if residual is None else (out, residual)
 
 
+def rms_norm_parts(planes: torch.Tensor, weight: torch.Tensor, eps: float, residual: torch.Tensor):
+    """`rms_norm` of a product that `linear_parts` left in parts, (parts, N, hidden) fp32: their sum is rounded as the product is."""
+    parts, N, H = planes.shape
+    assert planes.is_contiguous() and planes.dtype == torch.float32 and weight.is_contiguous() and weight.numel() == H
+    assert residual.shape == (N, H) and residual.stride(1) == 1 and residual.dtype == weight.dtype
+    out = torch.empty((N, H), dtype=residual.dtype, device=residual.device)
+    _lib.call("zp_add_rms_norm_parts", _lib.dev_ptr(planes), parts, _lib.dev_ptr(residual), _lib.dev_ptr(weight), _lib.dev_ptr(out), N, H,
+              residual.stride(0), out.stride(0), float(eps), _lib.dtype_tag(residual), _lib.stream_ptr(residual))
+    return out, residual
+
+
 def silu_and_mul(gate_up: torch.Tensor) -> torch.Tensor:
     """SiluAndMul of the dependency (zipage/models/qwen3.py:108-111): silu(x[:, :I]) * x[:, I:]."""
     N, two_i = gate_up.shape

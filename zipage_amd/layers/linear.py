@@ -106,8 +106,7 @@ def _seen_by_others(x: torch.Tensor, w: torch.Tensor) -> bool:
             or (x.requires_grad or w.requires_grad) and torch.is_grad_enabled() or x.device.index != _current_device())
 
 
-def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
-    """F.linear(x, w) without a bias."""
+def _linear(x: torch.Tensor, w: torch.Tensor, parts: bool) -> torch.Tensor:
     if x.is_cuda and not _seen_by_others(x, w) and x.dim() == 2 == w.dim() and x.layout == w.layout == torch.strided:
         (n, k), (m, wk), (stride, one) = x.shape, w.shape, x.stride()
         if k == wk and x.dtype == w.dtype in _FEW_TYPES and one == 1 and k <= stride <= 1 << 23 and stride % 8 == 0 and w.is_contiguous() and \
@@ -115,17 +114,32 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
             at, w_at = x.data_ptr(), w.data_ptr()
             split = _split_rows(n, k, m) and stride <= 1 << 22
             if (at | w_at) % 16 == 0 and (split or _few_rows(n, k, m) or _row_tiles(n, k, m)):
-                out, tag, stream = x.new_empty(n, m), _lib.dtype_tag(x), _lib.stream_ptr(x)
+                tag, stream = _lib.dtype_tag(x), _lib.stream_ptr(x)
+                size = _lib.size("zp_split_rows_workspace", n, k, m) if split else 0
+                parts = parts and size > 0
+                out = None if parts else x.new_empty(n, m)
                 if split:
-                    size = _lib.size("zp_split_rows_workspace", n, k, m)
-                    room = x.new_empty(size // 2) if size else None
-                    _lib.call_models("zp_split_rows_linear", at, w_at, out.data_ptr(), n, k, m, stride, m, tag, room.data_ptr() if size else None,
-                                     size, stream)
+                    room = x.new_empty(size // (4 * n * m), n, m, dtype=torch.float32) if size else None
+                    _lib.call_models("zp_split_rows_linear", at, w_at, None if parts else out.data_ptr(), n, k, m, stride, m, tag,
+                                     room.data_ptr() if size else None, size, stream)
+                    if parts:
+                        return room
                 else:
                     _lib.call_models("zp_few_rows_linear" if n <= 64 else "zp_row_tiles_linear", at, w_at, out.data_ptr(), n, k, m, stride, m,
                                      tag, stream)
                 return out
     return F.linear(x, w)
+
+
+def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """F.linear(x, w) without a bias."""
+    return _linear(x, w, False)
+
+
+def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
+    """`linear`, but a product that is made in parts of the contraction stays in them, (parts, n, m) fp32, for what adds them up itself: their
+    sum in this order, rounded, is the product."""
+    return _linear(x, w, True)
 
 
 def step_product(ctx):
