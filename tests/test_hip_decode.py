@@ -148,3 +148,34 @@ def test_paged_decode_in_parts(dev, dtype, B, Hq, Hkv, D, BS, NB):
         # the result's rounding, and each weight's: its share of the values' absolute sum
         bound = bits * (want.abs() + (w[..., None] * vv.abs()).sum(0)) + 2.0 ** -16
         assert bool(((got[b].double().cpu() - want).abs() <= bound).all()) and bool(((whole[b].double().cpu() - want).abs() <= bound).all())
+
+
+# tokens whose scores are -inf weigh nothing, wherever they lie: a part's only one, all of a part at the beginning, in the middle and at
+# the end, and whole parts side by side; a context of such tokens alone has no softmax
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("Hq,Hkv,D,BS,NB", [(8, 8, 64, 64, 33), (8, 2, 128, 128, 17), (4, 1, 128, 256, 8)])
+def test_paged_decode_of_parts_without_scores(dev, dtype, Hq, Hkv, D, BS, NB):
+    from zipage_amd import _lib
+    from zipage_amd.layers import paged_decode_attention
+    gone = [(129, 128, 129), (129, 0, 64), (200, 64, 128), (2047, 0, 1025), (2000, 1000, 2000), (65, 1, 64), (70, 0, 70), (0, 0, 0)]
+    B, g = len(gone), torch.Generator().manual_seed(NB)
+    k, v = ((torch.randn(B * NB, BS, Hkv, D, generator=g)).to(dtype).to(dev) for _ in range(2))
+    q = torch.randn(B, Hq, D, generator=g).to(dtype).to(dev)
+    q[..., 9] = 1.0
+    tables = torch.randperm(B * NB, generator=g).int().view(B, NB).contiguous().to(dev)
+    for b, (_, lo, hi) in enumerate(gone):
+        for t in range(lo, hi):
+            k[tables[b, t // BS], t % BS, :, 9] = -float("inf")
+    ctx = torch.tensor([n for n, _, _ in gone], dtype=torch.int32, device=dev)
+    assert _lib.size("zp_paged_decode_workspace", B, Hq, Hkv, D, BS, NB) > 0
+    got = paged_decode_attention(q, k, v, ctx, tables, D ** -0.5)
+    bits = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for b, (n, lo, hi) in enumerate(gone):
+        if hi - lo == n:
+            assert bool(got[b].isnan().all()) if n else not got[b].any()
+            continue
+        kk, vv = (c[tables[b].long()].reshape(-1, Hkv, D)[:n].double().cpu().repeat_interleave(Hq // Hkv, 1) for c in (k, v))
+        w = ((kk * q[b].double().cpu()).sum(-1) * D ** -0.5).softmax(0)
+        want = (w[..., None] * vv).sum(0)
+        bound = bits * (want.abs() + (w[..., None] * vv.abs()).sum(0)) + 2.0 ** -16      # as above
+        assert bool(((got[b].double().cpu() - want).abs() <= bound).all()), b

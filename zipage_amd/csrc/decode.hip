@@ -229,12 +229,14 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(G <= 4 
       const int npairs = ((Tc + 63) >> 6) * 32;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
+        // scores of -inf only, beside a part with others: weights of 0, not of exp(-inf + inf)
+        const float ms = SPLIT && mx[g] == -INFINITY ? 0.f : mx[g];
         float s = 0.f;
         for (int pi = tid; pi < npairs; pi += kThreads) {
           const int t = (pi >> 5) * 64 + (pi & 31);
           // each token belongs to exactly one pair, so the packed word can overwrite logit[t]
-          const float e0 = t < Tc ? __expf(logit[g * Tpad + t] - mx[g]) : 0.f;
-          const float e1 = t + 32 < Tc ? __expf(logit[g * Tpad + t + 32] - mx[g]) : 0.f;
+          const float e0 = t < Tc ? __expf(logit[g * Tpad + t] - ms) : 0.f;
+          const float e1 = t + 32 < Tc ? __expf(logit[g * Tpad + t + 32] - ms) : 0.f;
           s += e0 + e1;
           pw[g * Tpad + t] = pack2<T>(e0, e1);
         }
@@ -348,7 +350,8 @@ __global__ __launch_bounds__(64) void paged_combine_kernel(DecodeArgs p) {
   const int s0 = min((int)threadIdx.x, p.splits - 1);          // at most 64 of them
   const float m = ml[2 * s0], mx = wave_max(m);
   const float f = mx == -INFINITY || (int)threadIdx.x >= p.splits ? 0.f : __expf(m - mx), l = wave_sum(f * ml[2 * s0 + 1]);
-  const float inv = l > 0.f ? 1.f / l : 0.f;
+  // a context of such scores alone has no softmax, as in one part; one without tokens is 0
+  const float inv = l > 0.f ? 1.f / l : mx == -INFINITY && p.ctx[item / p.Hq] > 0 ? NAN : 0.f;
   for (int d = threadIdx.x * 2; d < p.D; d += 128) {
     const float* const from = p.part + item * p.splits * p.D + d;
     float2 r = {0.f, 0.f};
