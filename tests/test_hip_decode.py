@@ -179,3 +179,32 @@ def test_paged_decode_of_parts_without_scores(dev, dtype, Hq, Hkv, D, BS, NB):
         want = (w[..., None] * vv).sum(0)
         bound = bits * (want.abs() + (w[..., None] * vv.abs()).sum(0)) + 2.0 ** -16      # as above
         assert bool(((got[b].double().cpu() - want).abs() <= bound).all()), b
+
+
+# the same of slices of a long context in one part: the first, a middle one, the last, all but the last, and all
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_paged_decode_of_slices_without_scores(dev, dtype, Hq=8, Hkv=1, D=128, BS=256, NB=20):
+    from zipage_amd import _lib
+    gone = [(5000, 0, 2048), (5000, 2048, 4096), (4500, 4096, 4500), (5120, 0, 4096), (3000, 100, 3000), (2100, 0, 2100), (0, 0, 0)]
+    B, g = len(gone), torch.Generator().manual_seed(NB)
+    k, v = ((torch.randn(B * NB, BS, Hkv, D, generator=g)).to(dtype) for _ in range(2))
+    q = torch.randn(B, Hq, D, generator=g).to(dtype)
+    q[..., 9] = 1.0
+    tables = torch.randperm(B * NB, generator=g).int().view(B, NB).contiguous()
+    for b, (_, lo, hi) in enumerate(gone):
+        t = torch.arange(lo, hi)
+        k[tables[b, t // BS].long(), t % BS, :, 9] = -float("inf")
+    q, k, v, tables, ctx = (t.to(dev) for t in (q, k, v, tables, torch.tensor([n for n, _, _ in gone], dtype=torch.int32)))
+    got = torch.empty_like(q)
+    _lib.call("zp_paged_decode_attention", q.data_ptr(), k.data_ptr(), v.data_ptr(), tables.data_ptr(), ctx.data_ptr(), got.data_ptr(),
+              B, Hq, Hkv, D, BS, NB, B * NB, k.stride(0), v.stride(0), D ** -0.5, _lib.dtype_tag(q), _lib.stream_ptr(q))
+    bits = 2.0 ** (-8 if dtype == torch.bfloat16 else -11)
+    for b, (n, lo, hi) in enumerate(gone):
+        if hi - lo == n:
+            assert bool(got[b].isnan().all()) if n else not got[b].any()
+            continue
+        kk, vv = (c[tables[b].long()].reshape(-1, Hkv, D)[:n].double().cpu().repeat_interleave(Hq // Hkv, 1) for c in (k, v))
+        w = ((kk * q[b].double().cpu()).sum(-1) * D ** -0.5).softmax(0)
+        want = (w[..., None] * vv).sum(0)
+        bound = bits * (want.abs() + (w[..., None] * vv.abs()).sum(0)) + 2.0 ** -16      # as above
+        assert bool(((got[b].double().cpu() - want).abs() <= bound).all()), b

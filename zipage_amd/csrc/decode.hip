@@ -229,8 +229,8 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(G <= 4 
       const int npairs = ((Tc + 63) >> 6) * 32;
 #pragma unroll
       for (int g = 0; g < G; ++g) {
-        // scores of -inf only, beside a part with others: weights of 0, not of exp(-inf + inf)
-        const float ms = SPLIT && mx[g] == -INFINITY ? 0.f : mx[g];
+        // scores of -inf only, beside a part or slice with others: weights of 0, not of exp(-inf + inf)
+        const float ms = (SPLIT || CHUNKED) && mx[g] == -INFINITY ? 0.f : mx[g];
         float s = 0.f;
         for (int pi = tid; pi < npairs; pi += kThreads) {
           const int t = (pi >> 5) * 64 + (pi & 31);
@@ -250,7 +250,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(G <= 4 
         for (int w = 0; w < kWaves; ++w) s += red[w * G + g];
         if (CHUNKED) {
           // earlier slices were accumulated against a smaller maximum: bring them to this one
-          const float f = __expf(m_run[g] - mx[g]);   // exp(-inf) = 0 on the first slice
+          const float f = mx[g] == -INFINITY ? 0.f : __expf(m_run[g] - mx[g]);   // exp(-inf) = 0 on the first slice
           l_run[g] = l_run[g] * f + s;
 #pragma unroll
           for (int i = 0; i < 8; ++i) acc[g][i] *= f;
@@ -305,7 +305,10 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(G <= 4 
   }
   float inv[G];
 #pragma unroll
-  for (int g = 0; g < G; ++g) inv[g] = l_run[g] > 0.f ? 1.f / l_run[g] : 0.f;
+  for (int g = 0; g < G; ++g) {
+    inv[g] = l_run[g] > 0.f ? 1.f / l_run[g] : 0.f;
+    if (CHUNKED && m_run[g] == -INFINITY && Tn > 0) inv[g] = NAN;   // no softmax, as in one slice
+  }
   // sum the 4 row groups of each wave (lanes with equal piece), then the waves through LDS
 #pragma unroll
   for (int g = 0; g < G; ++g)
