@@ -393,6 +393,14 @@ def test_norms_of_products_in_parts(dev, dtype, n, K, M):
 
 
 @torch.inference_mode()
+@pytest.mark.parametrize("n", [0, 8, 40, 65, 256])
+def test_products_without_outputs(dev, n):
+    from zipage_amd.layers import linear, linear_parts
+    x, w = _rand(n, 1024, seed=1).to(dev), torch.empty(0, 1024, dtype=BF16, device=dev)
+    assert linear(x, w).shape == linear_parts(x, w).shape == (n, 0)
+
+
+@torch.inference_mode()
 def test_products_in_parts_under_capture(dev):
     """Through the entry point, in a graph that is replayed on new rows."""
     from zipage_amd.layers import linear

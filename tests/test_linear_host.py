@@ -121,3 +121,10 @@ def test_which_sizes_are_row_tiles(n, k, m, tiles):
 def test_which_sizes_are_split(n, k, m, split):
     from zipage_amd.layers.linear import _split_rows
     assert _split_rows(n, k, m) == split
+
+
+@pytest.mark.parametrize("n", [0, 1, 16, 17, 32, 64, 65, 128, 256])
+@pytest.mark.parametrize("k,m", [(1024, 0), (4096, 0), (0, 1024), (0, 0)])
+def test_products_of_nothing_stay_with_the_library(n, k, m):
+    from zipage_amd.layers.linear import _few_rows, _row_tiles, _split_rows
+    assert not (_few_rows(n, k, m) or _row_tiles(n, k, m) or _split_rows(n, k, m))

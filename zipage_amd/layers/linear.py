@@ -36,7 +36,7 @@ def _few_rows(n: int, k: int, m: int) -> bool:
     -> 8192 11.2 and 14.6, -> 9216 17.0 and 14.1; 4096 -> 4096 10.4 and 13.6, -> 6144 16.5 and 15.4).
     Up to 64, since each workgroup reads all rows: 48 rows, 1024 -> 4096 6.6 and 11.3, 3072 -> 1024 11.3 and 11.7, but -> 2048
     11.4 and 10.3, -> 256 10.6 and 9.3; 64 -> 8192 4.0 and 3.8."""
-    if n <= 0 or k <= 0 or k % 32 or m % 4 or k > 1 << 23:
+    if n <= 0 or k <= 0 or m <= 0 or k % 32 or m % 4 or k > 1 << 23:
         return False
     if n <= 16:
         if k > 4096:
@@ -54,7 +54,7 @@ def _row_tiles(n: int, k: int, m: int) -> bool:
     short ones, since a CU has one workgroup with them (256 rows, 1536 -> 4096 12.7 and 11.2, 2048 -> 4096 18.1 and 13.2); longer
     contractions up to 128 rows, where the library's tiles leave most of the chip idle (128 rows, 4096 -> 4096 18.2 and 23.5, 3072 ->
     4096 14.9 and 20.2; 100 rows 17.7 and 16.5, 13.6 and 16.5; 4096 -> 6144 25.4 and 25.3)."""
-    if not 64 < n <= 256 or k % 32 or m % 4 or k < 96:
+    if not 64 < n <= 256 or m <= 0 or k % 32 or m % 4 or k < 96:
         return False
     tiles = lambda outs: -(-n // 64) * -(-m // outs)
     if tiles(32) > 256 and (tiles(64) > 256 or k > (2048 if n <= 128 else 1024)):
