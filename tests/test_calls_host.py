@@ -1,6 +1,7 @@
 """Calls through native code: the same conversions as ctypes makes, for every entry point."""
 import ctypes
 
+import numpy as np
 import pytest
 import torch
 
@@ -51,3 +52,39 @@ def test_addresses_of_tensors():
         _lib.dev_ptr(torch.zeros(3))
     with pytest.raises(AttributeError):
         _lib.dev_ptr(3)
+
+
+class _Numbers(ctypes.Structure):
+    _fields_ = [("a", ctypes.c_int64), ("b", ctypes.c_int64)]
+
+
+def test_what_stands_for_a_pointer():
+    calls, seen = _lib.load_calls(), []
+    back = ctypes.CFUNCTYPE(ctypes.c_int32, *[ctypes.c_void_p] * 3, ctypes.c_int32, ctypes.c_int32, ctypes.c_int64,
+                            ctypes.c_void_p)(lambda *a: (seen.append(a[0]), 0)[1])
+    gather = calls.entry("zp_gather_rows", ctypes.cast(back, ctypes.c_void_p).value)
+    call = lambda o: (gather(o, 0, 0, 0, 0, 0, 0), seen.pop())[1]
+    held, numbers = (ctypes.c_int64 * 3)(5, 6, 7), _Numbers(1, 2)
+    at = ctypes.addressof(held)
+    for o, want in ((None, None), (0, None), (at, at), (held, at), (ctypes.byref(held), at), (ctypes.byref(held, 8), at + 8),
+                    (ctypes.c_void_p(at), at), (ctypes.c_void_p(), None), (ctypes.cast(held, ctypes.POINTER(ctypes.c_int64)), at),
+                    (numbers, ctypes.addressof(numbers))):
+        assert call(o) == want, o
+    # what ctypes refuses for an address stays refused: a number that is not Python's, and what merely has a buffer
+    for o in (np.int64(at), np.array([at]), bytearray(8), memoryview(b"12345678"), torch.zeros(2), 1.5, [at], ctypes.c_int64(at)):
+        with pytest.raises(TypeError):
+            gather(o, 0, 0, 0, 0, 0, 0)
+    assert not seen
+
+
+def test_what_stands_for_a_structure():
+    calls, seen = _lib.load_calls(), []
+    back = ctypes.CFUNCTYPE(ctypes.c_int32, ctypes.c_void_p, ctypes.c_int32, ctypes.c_void_p)(lambda *a: (seen.append(a[0]), 0)[1])
+    scan = calls.entry("zp_linear_scan", ctypes.cast(back, ctypes.c_void_p).value)
+    args = _lib.LinearArgs()
+    for o in (args, ctypes.byref(args)):
+        assert scan(o, 0, 0) == 0 and seen.pop() == ctypes.addressof(args)
+    for o in (ctypes.addressof(args), _Numbers(), ctypes.byref(_Numbers()), _lib.AttentionForm(), ctypes.c_void_p(ctypes.addressof(args))):
+        with pytest.raises(TypeError):
+            scan(o, 0, 0)
+    assert not seen

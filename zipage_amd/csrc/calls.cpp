@@ -15,6 +15,42 @@
 
 namespace {
 
+PyObject *held_types, *pointer_types, *cast, *void_pointer;      // of ctypes
+// Where a ctypes structure, union or array lies, or what a ctypes pointer or reference points to; the caller holds it.  Nothing else
+// that has a buffer: a NumPy number would pass its own address.  `record`: bytes of the structure that is wanted, 0: any.
+bool address(PyObject* o, void*& v, size_t record) {
+  const int held = PyObject_IsInstance(o, held_types), other = held ? 0 : PyObject_IsInstance(o, pointer_types);
+  if (held < 0 || other < 0) return false;
+  if (!held && !other) return PyErr_Format(PyExc_TypeError, "%s in a pointer's place", Py_TYPE(o)->tp_name), false;
+  PyObject* to = o;
+  if (other) {
+    PyObject* const p = PyObject_CallFunctionObjArgs(cast, o, void_pointer, nullptr);
+    if (!p) return false;
+    PyObject* const value = PyObject_GetAttrString(p, "value");
+    Py_DECREF(p);
+    if (!value) return false;
+    v = value == Py_None ? nullptr : PyLong_AsVoidPtr(value);
+    Py_DECREF(value);
+    if (!v && PyErr_Occurred()) return false;
+    if (!record) return true;
+    to = PyObject_GetAttrString(o, "_obj");
+    if (!to) return PyErr_Format(PyExc_TypeError, "%s in a structure's place", Py_TYPE(o)->tp_name), false;
+  }
+  Py_buffer b;
+  const bool there = PyObject_GetBuffer(to, &b, PyBUF_SIMPLE) == 0;
+  if (other) Py_DECREF(to);
+  if (!there) return false;
+  const size_t bytes = (size_t)b.len;
+  if (held) v = b.buf;
+  PyBuffer_Release(&b);
+  if (record && (bytes == 0 || bytes % record)) return PyErr_Format(PyExc_TypeError, "%zu bytes instead of a structure's %zu", bytes, record), false;
+  return true;
+}
+
+template <class T> constexpr size_t record_bytes() {
+  if constexpr (std::is_class<T>::value) return sizeof(T);
+  else return 0;
+}
 template <class T> bool from(PyObject* o, T& v) {
   if constexpr (std::is_floating_point<T>::value) {
     const double x = PyFloat_AsDouble(o);
@@ -24,22 +60,20 @@ template <class T> bool from(PyObject* o, T& v) {
     const long long x = PyLong_AsLongLong(o);
     v = (T)x;
     return x != -1 || !PyErr_Occurred();
-  } else if (o == Py_None) {
-    v = nullptr;
-    return true;
-  } else if (PyLong_Check(o)) {
-    v = (T)PyLong_AsVoidPtr(o);
-    return v || !PyErr_Occurred();
-  } else {                                       // a ctypes structure or array, or one by reference, which the caller holds
-    PyObject* const by = PyObject_CheckBuffer(o) ? nullptr : PyObject_GetAttrString(o, "_obj");
-    if (!by) PyErr_Clear();
-    Py_buffer b;
-    const bool there = PyObject_GetBuffer(by ? by : o, &b, PyBUF_SIMPLE) == 0;
-    Py_XDECREF(by);
-    if (!there) return false;
-    v = (T)b.buf;
-    PyBuffer_Release(&b);
-    return true;
+  } else {
+    constexpr size_t record = record_bytes<std::remove_cv_t<std::remove_pointer_t<T>>>();
+    if (o == Py_None) {
+      v = nullptr;
+      return true;
+    }
+    if (!record && PyLong_Check(o)) {
+      v = (T)PyLong_AsVoidPtr(o);
+      return v || !PyErr_Occurred();
+    }
+    void* at = nullptr;
+    const bool there = address(o, at, record);
+    v = (T)at;
+    return there;
   }
 }
 
@@ -127,5 +161,21 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "zipage_calls", nullptr, -1, method
 PyMODINIT_FUNC PyInit_zipage_calls() {
   is_cuda = PyUnicode_InternFromString("is_cuda");
   data_ptr = PyUnicode_InternFromString("data_ptr");
-  return is_cuda && data_ptr ? PyModule_Create(&module) : nullptr;
+  PyObject* const ctypes = PyImport_ImportModule("ctypes");
+  PyObject* const inner = ctypes ? PyImport_ImportModule("_ctypes") : nullptr;
+  if (!inner) return nullptr;
+  cast = PyObject_GetAttrString(ctypes, "cast");
+  void_pointer = PyObject_GetAttrString(ctypes, "c_void_p");
+  PyObject* const some = void_pointer ? PyObject_CallNoArgs(void_pointer) : nullptr;
+  PyObject* const by = some ? PyObject_CallMethod(ctypes, "byref", "O", some) : nullptr;
+  if (!cast || !by) return nullptr;
+  held_types = Py_BuildValue("(NNN)", PyObject_GetAttrString(ctypes, "Structure"), PyObject_GetAttrString(ctypes, "Union"),
+                             PyObject_GetAttrString(ctypes, "Array"));
+  pointer_types = Py_BuildValue("(NNOO)", PyObject_GetAttrString(inner, "_Pointer"), PyObject_GetAttrString(inner, "CFuncPtr"), void_pointer,
+                                (PyObject*)Py_TYPE(by));
+  Py_DECREF(by);
+  Py_DECREF(some);
+  Py_DECREF(inner);
+  Py_DECREF(ctypes);
+  return held_types && pointer_types && is_cuda && data_ptr ? PyModule_Create(&module) : nullptr;
 }
