@@ -1,11 +1,15 @@
 """Calls through native code: the same conversions as ctypes makes, for every entry point."""
 import ctypes
+import importlib.machinery
+import importlib.util
+import subprocess
 
 import numpy as np
 import pytest
 import torch
 
 from zipage_amd import _lib
+from zipage_amd.build import calls_command
 
 
 def test_every_entry_point_is_there():
@@ -88,3 +92,11 @@ def test_what_stands_for_a_structure():
         with pytest.raises(TypeError):
             scan(o, 0, 0)
     assert not seen
+
+
+def test_built_for_another_python(tmp_path):
+    path = str(tmp_path / "zipage_calls.so")
+    subprocess.run([*calls_command(path), '-DZP_PYTHON="3.99."', "-O0"], check=True)
+    loader = importlib.machinery.ExtensionFileLoader("zipage_calls", path)
+    with pytest.raises(ImportError, match="Python 3.99.x"):
+        importlib.util.module_from_spec(importlib.util.spec_from_loader("zipage_calls", loader))

@@ -69,6 +69,11 @@ def _run(cmd, verbose):
         print(err, file=sys.stderr)
 
 
+def calls_command(out: str) -> list[str]:
+    return [shutil.which("g++") or shutil.which("hipcc") or "/opt/rocm/bin/hipcc", "-O2", "-std=c++17", "-fPIC", "-shared",
+            "-I" + sysconfig.get_path("include"), os.path.join(CSRC, "calls.cpp"), "-o", out]
+
+
 def build(verbose: bool = True, jobs: int | None = None, libs: tuple[str, ...] = LIBS) -> str:
     """Compile the sources of ``libs`` to object files (in parallel) and link the shared objects."""
     from concurrent.futures import ThreadPoolExecutor
@@ -77,8 +82,7 @@ def build(verbose: bool = True, jobs: int | None = None, libs: tuple[str, ...] =
     work, links = [], []
     for lib in libs:
         if lib == CALLS_LIB:
-            work.append([shutil.which("g++") or hipcc, "-O2", "-std=c++17", "-fPIC", "-shared", "-I" + sysconfig.get_path("include"),
-                         os.path.join(CSRC, "calls.cpp"), "-o", lib + ".tmp"])
+            work.append(calls_command(lib + ".tmp"))
             links.append((lib, None))
             continue
         models = lib in MODEL_SOURCES

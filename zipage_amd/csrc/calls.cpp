@@ -153,12 +153,22 @@ PyObject* pointer(PyObject*, PyObject* t) {
   return PyObject_CallMethodNoArgs(t, data_ptr);
 }
 
+#ifndef ZP_PYTHON
+#define ZP_TEXT_OF(x) #x
+#define ZP_TEXT(x) ZP_TEXT_OF(x)
+#define ZP_PYTHON ZP_TEXT(PY_MAJOR_VERSION) "." ZP_TEXT(PY_MINOR_VERSION) "."
+#endif
+constexpr char kPython[] = ZP_PYTHON;
+
 PyMethodDef methods[] = {{"entry", entry, METH_VARARGS, nullptr}, {"pointer", pointer, METH_O, nullptr}, {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "zipage_calls", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 
 }  // namespace
 
 PyMODINIT_FUNC PyInit_zipage_calls() {
+  // objects are laid out as in the Python that this was compiled against
+  if (std::strncmp(Py_GetVersion(), kPython, sizeof(kPython) - 1) != 0)
+    return PyErr_Format(PyExc_ImportError, "libzipage_calls.so is for Python %sx, this is %.20s: build it again", kPython, Py_GetVersion());
   is_cuda = PyUnicode_InternFromString("is_cuda");
   data_ptr = PyUnicode_InternFromString("data_ptr");
   PyObject* const ctypes = PyImport_ImportModule("ctypes");
