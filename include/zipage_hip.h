@@ -38,7 +38,9 @@ enum { ZP_REDUCE_MEAN = 0, ZP_REDUCE_MAX = 1 };    /* attention_score `reduced` 
 enum { ZP_ACTIVATE_MAX = 0, ZP_ACTIVATE_SUM = 1 }; /* global_score `activate_method` */
 enum { ZP_POOL_MAX = 0, ZP_POOL_AVG = 1 };
 
-/* ABI version of this header; bumped on any signature change. */
+/* ABI version of this header and of zipage_models.h; bumped on any change of a signature or a structure.  A library of another
+ * version takes other arguments. */
+#define ZP_ABI_VERSION 5
 int zp_abi_version(void);
 /* Message of the last error raised on the calling thread ("" if none). */
 const char* zp_last_error(void);

@@ -3,6 +3,7 @@ No compute calls: this runs without a GPU."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -126,3 +127,38 @@ def test_room_for_pieces_of_runs_follows_the_rows():
             room = size(rows, runs, heads) - blocks(rows, runs, heads)
             assert room == min(384, (rows // 64 + runs) * heads) * state
         assert size(2048, 8, 32) == blocks(2048, 8, 32)                                   # 256 pairs
+
+
+def test_version_is_the_headers():
+    from zipage_amd import _lib
+    text = open(os.path.join(ROOT, "include", "zipage_hip.h")).read()
+    assert _lib.ABI_VERSION == int(re.search(r"#define ZP_ABI_VERSION (\d+)", text)[1])
+    for lib in (_lib.load(), *(_lib.load_models(name) for name in _lib.MODEL_LIBS)):
+        assert lib.zp_abi_version() == _lib.ABI_VERSION
+
+
+def test_library_of_another_version_is_refused(tmp_path):
+    from zipage_amd import _lib
+    path = str(tmp_path / "old.so")
+    source = f"int zp_abi_version(void) {{ return {_lib.ABI_VERSION - 1}; }}"
+    subprocess.run(["gcc", "-shared", "-fPIC", "-x", "c", "-", "-o", path], input=source, text=True, check=True)
+    with pytest.raises(RuntimeError, match=f"ABI version {_lib.ABI_VERSION - 1}"):
+        _lib._open(path, {}, {})
+
+
+def test_structures_are_as_long_as_the_headers(tmp_path):
+    from zipage_amd import _lib
+    here = {"zp_compress_config": _lib.CompressConfigC, "zp_branch": _lib.Branch, "zp_segments": _lib.Segments, "zp_mlstm": _lib.MlstmArgs,
+            "zp_delta": _lib.DeltaArgs, "zp_linear": _lib.LinearArgs, "zp_attention_form": _lib.AttentionForm, "zp_store_form": _lib.StoreForm}
+    headers = "".join(open(os.path.join(ROOT, "include", h)).read() for h in ("zipage_hip.h", "zipage_models.h"))
+    records = [n for n in re.findall(r"^} (zp_\w+);", headers, re.M)]
+    assert sorted(records) == sorted(here)
+    # the last field of each too: what lies behind the others has their sizes and places
+    last = lambda t: t._fields_[-1][0]
+    body = "".join(f'printf("%zu %zu\\n", sizeof({n}), offsetof({n}, {last(here[n])}));' for n in records)
+    source = f'#include <stddef.h>\n#include <stdio.h>\n#include "zipage_hip.h"\n#include "zipage_models.h"\nint main(void) {{ {body} return 0; }}'
+    exe = str(tmp_path / "sizes")
+    subprocess.run(["gcc", "-I", os.path.join(ROOT, "include"), "-x", "c", "-", "-o", exe], input=source, text=True, check=True)
+    out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split("\n")
+    for n, line in zip(records, out):
+        assert [int(v) for v in line.split()] == [ctypes.sizeof(here[n]), getattr(here[n], last(here[n])).offset], n

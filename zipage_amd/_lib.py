@@ -206,6 +206,7 @@ MODEL_LIBS = {
 MODEL_EXPORTS = {lib: sorted([*calls, *sizes]) for lib, (calls, sizes) in MODEL_LIBS.items()}
 _LIB_OF = {name: lib for lib, names in MODEL_EXPORTS.items() for name in names}
 
+ABI_VERSION = 5                          # ZP_ABI_VERSION
 CALLS_PATH = os.path.join(_HERE, "libzipage_calls.so")
 _lib = None
 _models: dict[str, C.CDLL] = {}
@@ -219,13 +220,15 @@ def _open(path: str, signatures: dict, i64_returning: dict) -> C.CDLL:
             f"{path} is missing: build it with `python -m zipage_amd.build` "
             "(there is no CPU fallback for the HIP kernels)")
     lib = C.CDLL(path)
+    lib.zp_abi_version.argtypes, lib.zp_abi_version.restype = [], i32
+    if lib.zp_abi_version() != ABI_VERSION:
+        raise RuntimeError(f"{path} has ABI version {lib.zp_abi_version()} instead of {ABI_VERSION}: build it with `python -m zipage_amd.build`")
     for name, args in signatures.items():
         fn = getattr(lib, name)
         fn.argtypes, fn.restype = args, i32
     for name, args in i64_returning.items():
         fn = getattr(lib, name)
         fn.argtypes, fn.restype = args, i64
-    lib.zp_abi_version.argtypes, lib.zp_abi_version.restype = [], i32
     lib.zp_last_error.argtypes, lib.zp_last_error.restype = [], C.c_char_p
     return lib
 
