@@ -288,3 +288,22 @@ def test_recurrent_models_share_no_prefix():
                 done.append(p.seq)
         sched.postprocess(done, None, advance=True)
     assert ran == 3 * 72 and sched.pool.num_free == 24 and sched.pool.reserved == 0
+
+
+def test_experts_chosen_by_another_route():
+    from zipage_amd.layers import Experts
+
+    class Chosen(Exception):
+        pass
+
+    def choose(h):
+        raise Chosen
+
+    class Other(Experts):
+        route = staticmethod(choose)
+    m = Experts(64, 4, 2, 32, 7.0)
+    m.route = choose
+    for experts in (m, Other(64, 4, 2, 32, 7.0)):
+        experts.router = torch.zeros(4, 64)
+        with pytest.raises(Chosen):
+            experts.forward(torch.zeros(3, 64))

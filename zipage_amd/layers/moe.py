@@ -182,5 +182,9 @@ class Experts:
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         """h (N, padded width) -> planes (slots, N, padded width) that `residual_norm` adds up in fp32."""
-        plan, weights = self.routed(h)
+        if type(self).route is Experts.route and "route" not in vars(self):
+            plan, weights = self.routed(h)
+        else:                                         # another choice of experts
+            ids, weights, counts = self.route(h)
+            plan = Plan(ids, counts, self.experts, self.shared_ff is not None, h.dtype)
         return self.down_planes(self.gate_up_rows(h, plan, weights), plan)
