@@ -738,3 +738,22 @@ def test_command_line(dev, engines, tmp_path, capsys, monkeypatch):
     C.close("ends", read(0), full[[0, 32]], F32, whole=full)
     C.close("ends", read(2), torch.stack([other[2], full[39]]), F32, whole=full)
     C.close("ends", read(3), full[:1], F32, whole=full)
+
+
+def test_experts_read_the_plan_as_it_is(dev):
+    """Tensors that take the place of a plan's own are the ones that count."""
+    from zipage_amd.layers import Experts
+    from zipage_amd.layers.moe import Plan
+    E, n = 5, 40
+    m = Experts(64, E, 2, 32, 7.0)
+    m.load(_expert_weights(E, 64, 32, None, BF16), BF16, dev)
+    h = _rand(dev, BF16, n, 64, seed=2)
+    ids_, weights, counts = m.route(h)
+    p = Plan(ids_, counts, E, False, BF16)
+    want = m.gate_up_rows(h, p, weights)
+    planes = m.down_planes(want, p)
+    own = p.ntiles
+    p.sorted, p.tiles, p.ntiles = p.sorted.clone(), p.tiles.clone(), p.ntiles.clone()
+    own.zero_()                                              # no tiles
+    assert torch.equal(m.gate_up_rows(h, p, weights), want) and torch.equal(m.down_planes(want, p), planes)
+    assert torch.equal(m.forward(h), planes)

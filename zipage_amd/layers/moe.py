@@ -9,13 +9,16 @@ from zipage_amd import _lib
 from .linear import fit, pad_to_multiple
 
 
+def _small_linear(x: torch.Tensor, w: torch.Tensor, out: int):
+    assert x.stride(1) == 1 and w.is_contiguous() and w.dtype == x.dtype and w.shape[1] == x.shape[1]
+    _lib.call_models("zp_small_linear", _lib.dev_ptr(x), _lib.dev_ptr(w), out, x.shape[0], x.shape[1], w.shape[0], x.stride(0),
+                     _lib.dtype_tag(x), _lib.stream_ptr(x))
+
+
 def small_linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     """x (N, K), w (M, K) -> (N, M) in fp32, for products with few outputs."""
-    N, K = x.shape
-    assert x.stride(1) == 1 and w.is_contiguous() and w.dtype == x.dtype and w.shape[1] == K
-    out = torch.empty((N, w.shape[0]), dtype=torch.float32, device=x.device)
-    _lib.call_models("zp_small_linear", _lib.dev_ptr(x), _lib.dev_ptr(w), _lib.dev_ptr(out), N, K, w.shape[0],
-                     x.stride(0), _lib.dtype_tag(x), _lib.stream_ptr(x))
+    out = torch.empty((x.shape[0], w.shape[0]), dtype=torch.float32, device=x.device)
+    _small_linear(x, w, _lib.dev_ptr(out))
     return out
 
 
@@ -36,32 +39,41 @@ def moe_select(logits: torch.Tensor, experts: int, top: int, groups: int = 1, ke
 
 
 class Plan:
-    """Assignments (token * slots + slot) in the order of their experts, and row tiles over them."""
+    """Assignments (token * slots + slot) in the order of their experts, and row tiles over them: `sorted`, `tiles` and `ntiles`."""
 
     def __init__(self, ids: torch.Tensor, counts: torch.Tensor, experts: int, shared: bool, dtype):
         N, top = ids.shape
-        dev = ids.device
-        self._size(N, experts, top, shared, dtype)
-        self.sorted = torch.empty(N * self.slots, dtype=torch.int32, device=dev)
-        self.tiles = torch.empty((self.max_tiles, 4), dtype=torch.int32, device=dev)
-        self.ntiles = torch.empty(1, dtype=torch.int32, device=dev)
-        size = _lib.size("zp_moe_plan_workspace", N, experts, top)
-        ws = torch.empty(size, dtype=torch.uint8, device=dev)
-        self.sorted_at, self.tiles_at, self.ntiles_at = (_lib.dev_ptr(t) for t in (self.sorted, self.tiles, self.ntiles))
-        _lib.call_models("zp_moe_plan", _lib.dev_ptr(ids), _lib.dev_ptr(counts), self.sorted_at, self.tiles_at, self.ntiles_at, N, experts,
-                         top, self.shared, self.rows, self.max_tiles, _lib.dev_ptr(ws), size, _lib.stream_ptr(ids))
+        self._allocate(N, experts, top, shared, dtype, ids.device)
+        self.sorted = torch.narrow(self.held, 0, self.places[0] // 4, N * self.slots)
+        self.tiles = torch.narrow(self.held, 0, self.places[1] // 4, self.max_tiles * 4).view(-1, 4)
+        self.ntiles = torch.narrow(self.held, 0, self.places[2] // 4, 1)
+        self._make(_lib.dev_ptr(ids), _lib.dev_ptr(counts), _lib.stream_ptr(ids))
 
-    @classmethod
-    def of(cls, n: int, experts: int, top: int, shared: bool, dtype):
-        """One of that size, whose three addresses the caller sets."""
-        plan = cls.__new__(cls)
-        plan._size(n, experts, top, shared, dtype)
-        return plan
-
-    def _size(self, n: int, experts: int, top: int, shared: bool, dtype):
+    def _allocate(self, n: int, experts: int, top: int, shared: bool, dtype, device, *before: int) -> list[int]:
+        """One allocation of all, each 16-byte aligned; the addresses of those of `before` words that the caller wants in it too."""
         self.n, self.experts, self.top, self.shared, self.slots = n, experts, top, int(shared), top + int(shared)
         self.rows = _lib.size("zp_moe_tile_rows", n, experts, top, _lib._DTYPES[dtype])
         self.max_tiles = _lib.size("zp_moe_max_tiles", n, experts, top, self.shared, self.rows)
+        self.room = _lib.size("zp_moe_plan_workspace", n, experts, top)
+        at, total = [], 0
+        for words in (*before, n * self.slots, self.max_tiles * 4, 1, -(-self.room // 4)):
+            at.append(4 * total)
+            total += -(-words // 4) * 4
+        self.held, self.places = torch.empty(total, dtype=torch.int32, device=device), at[len(before):]
+        self.sorted = self.tiles = self.ntiles = None
+        start = _lib.dev_ptr(self.held)
+        return [start + a for a in at[:len(before)]]
+
+    def _make(self, ids: int, counts: int, stream: int):
+        _lib.call_models("zp_moe_plan", ids, counts, *self.addresses(), self.n, self.experts, self.top, self.shared, self.rows, self.max_tiles,
+                         _lib.dev_ptr(self.held) + self.places[3], self.room, stream)
+
+    def addresses(self) -> tuple:
+        """Of the three, as they are now."""
+        if self.sorted is not None:
+            return _lib.dev_ptr(self.sorted), _lib.dev_ptr(self.tiles), _lib.dev_ptr(self.ntiles)
+        start = _lib.dev_ptr(self.held)
+        return start + self.places[0], start + self.places[1], start + self.places[2]
 
 
 def tile_order(w: torch.Tensor) -> torch.Tensor:
@@ -142,20 +154,12 @@ class Experts:
         """`route` and the plan of it, with one allocation instead of eight, which take 1.7 us of host time each (9 tokens, 32 experts
         of 1024 wide: 54 -> 41 us): the plan, and the address of the weights, which it holds."""
         N, E, top, M = h.shape[0], self.experts, self.top, self.router.shape[0]
-        assert h.stride(1) == 1 and h.dtype == self.router.dtype and h.shape[1] == self.router.shape[1]
-        plan = Plan.of(N, E, top, self.shared_ff is not None, h.dtype)
-        ws = _lib.size("zp_moe_plan_workspace", N, E, top)
-        at, total = [], 0
-        for n in (N * M, N * top, N * top, E + 1, N * plan.slots, plan.max_tiles * 4, 1, ws // 4):
-            at.append(4 * total)
-            total += -(-n // 4) * 4                   # 16-byte aligned
-        plan.held = torch.empty(total, dtype=torch.int32, device=h.device)
-        logits, ids, weights, counts, plan.sorted_at, plan.tiles_at, plan.ntiles_at, ws_at = (_lib.dev_ptr(plan.held) + a for a in at)
-        tag, stream = _lib.dtype_tag(h), _lib.stream_ptr(h)
-        _lib.call_models("zp_small_linear", _lib.dev_ptr(h), _lib.dev_ptr(self.router), logits, N, h.shape[1], M, h.stride(0), tag, stream)
+        plan = Plan.__new__(Plan)
+        logits, ids, weights, counts = plan._allocate(N, E, top, self.shared_ff is not None, h.dtype, h.device, N * M, N * top, N * top, E + 1)
+        _small_linear(h, self.router, logits)
+        stream = _lib.stream_ptr(h)
         _lib.call_models("zp_moe_select", logits, ids, weights, counts, N, E, top, self.groups, self.keep, self.score, M, stream)
-        _lib.call_models("zp_moe_plan", ids, counts, plan.sorted_at, plan.tiles_at, plan.ntiles_at, N, E, top, plan.shared, plan.rows,
-                         plan.max_tiles, ws_at, ws, stream)
+        plan._make(ids, counts, stream)
         return plan, weights
 
     def gate_up_rows(self, h: torch.Tensor, plan: Plan, weights: torch.Tensor | int) -> torch.Tensor:
@@ -166,8 +170,8 @@ class Experts:
         ff = max(self.ff_p, self.shared_p)
         act = torch.empty((plan.n * plan.slots, ff), dtype=h.dtype, device=h.device)
         _lib.call_models("zp_moe_gate_up", _lib.dev_ptr(h), _lib.dev_ptr(self.gate_up), _lib.dev_ptr(self.shared_gate_up),
-                         _lib.dev_ptr(act), plan.sorted_at, plan.tiles_at, plan.ntiles_at, weights, plan.n, self.experts, self.top, plan.shared, plan.rows, plan.max_tiles,
-                         self.width_p, self.ff_p, self.shared_p, h.stride(0), ff, self.act, self.limit, self.shared_limit,
+                         _lib.dev_ptr(act), *plan.addresses(), weights, plan.n, self.experts, self.top, plan.shared, plan.rows,
+                         plan.max_tiles, self.width_p, self.ff_p, self.shared_p, h.stride(0), ff, self.act, self.limit, self.shared_limit,
                          _lib.dtype_tag(h), _lib.stream_ptr(h))
         return act
 
@@ -175,9 +179,8 @@ class Experts:
         """(slots, N, width) parts of the output, to be added up."""
         out = torch.empty((plan.slots, plan.n, self.width_p), dtype=act.dtype, device=act.device)
         _lib.call_models("zp_moe_down", _lib.dev_ptr(act), _lib.dev_ptr(self.down), _lib.dev_ptr(self.shared_down),
-                         _lib.dev_ptr(out), plan.sorted_at, plan.tiles_at, plan.ntiles_at,
-                         plan.n, self.experts, self.top, plan.shared, plan.rows, plan.max_tiles, self.ff_p, self.shared_p,
-                         self.width_p, act.stride(0), self.width_p, _lib.dtype_tag(act), _lib.stream_ptr(act))
+                         _lib.dev_ptr(out), *plan.addresses(), plan.n, self.experts, self.top, plan.shared, plan.rows, plan.max_tiles,
+                         self.ff_p, self.shared_p, self.width_p, act.stride(0), self.width_p, _lib.dtype_tag(act), _lib.stream_ptr(act))
         return out
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
