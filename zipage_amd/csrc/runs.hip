@@ -36,8 +36,8 @@ struct TilesArgs {
   const uint16_t* gate;   // token rows of g_st elements, head h at h * V; or null
   int64_t g_st;
   const float2* turns;    // one map: (q_rows, V / 2) cos and sin, results turn back by them; or null
-  const zp_f32x4* q_turns;   // one map: (q_half / 2) planes of (q_rows, 2) cos and sin by which queries turn, or null: they are
-  int64_t q_plane;           // as they come; rows from a plane to the next
+  const zp_f32x4* q_turns;   // TURN: (q_half / 2) planes of (q_rows, 2) cos and sin by which queries turn; otherwise null
+  int64_t q_plane;           // rows from a plane to the next
   int q_half;
   bool rising;            // a run's tiles come in the order of their keys; otherwise those with many keys first
   int few_tiles;          // tiles of keys up to which a workgroup takes the form that stages no tile ahead
@@ -120,7 +120,9 @@ constexpr int long_step(int DKS, int VCB, int MAPS, bool SHARED, int CAP) {
 // Column tile t of a wave: 16 queries, map t % MAPS of the head (differential attention has two, over the same
 // values; elsewhere there is one).  SHARED: the last P elements of every head's key are the row of a.ks.
 // FINE: softmax weights enter the value product as two bf16 planes (17 bits), elsewhere as one.
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
+// TURN: queries come as projected (see turn_queries); a form of its own, for the branch alone costs the flow 2.5 % where nothing turns
+// (16 prompts of 256 to 768 tokens, 32 heads of 128 over 8, 95.5 us without it, 97.7 with it).
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep, bool TURN>
 __device__ __forceinline__ void run_tile(const TilesArgs& a, char* lds_raw, int h, int tile) {
   typedef TileStage<DKS, VCB, MAPS> Stage;
   constexpr bool kTurns = MAPS == 1 && !SHARED && CAP == kNoCap;
@@ -166,16 +168,16 @@ __device__ __forceinline__ void run_tile(const TilesArgs& a, char* lds_raw, int 
         qf[t][ks] = (*(const u32x4*)(q + (c < DT ? c : 0)) & kept) ^ flip;
         if (c >= DT) qf[t][ks] = u32x4{0u, 0u, 0u, 0u};
       }
-      if constexpr (kTurns && DKS <= 4 && VCB == 1)
-        if (a.q_turns) {                                      // the sign above goes through a turn unchanged
-          const zp_f32x4* const turns = a.q_turns + g * 4 * a.q_plane + q0 + qi;
-          if constexpr (DKS == 4) {
-            if (a.q_half == 64) turn_queries<2, 32>(qf[t], turns, a.q_plane);
-            else turn_queries<1, 32>(qf[t], turns, a.q_plane);
-          } else {
-            turn_queries<1, 32>(qf[t], turns, a.q_plane);
-          }
+      if constexpr (TURN) {                                   // the sign above goes through a turn unchanged
+        static_assert(kTurns && DKS <= 4 && VCB == 1, "heads of at most 128");
+        const zp_f32x4* const turns = a.q_turns + g * 4 * a.q_plane + q0 + qi;
+        if constexpr (DKS == 4) {
+          if (a.q_half == 64) turn_queries<2, 32>(qf[t], turns, a.q_plane);
+          else turn_queries<1, 32>(qf[t], turns, a.q_plane);
+        } else {
+          turn_queries<1, 32>(qf[t], turns, a.q_plane);
         }
+      }
     }
     f32x4 o[kT][VCB * 8];
     float m[kT], l[kT];
@@ -407,10 +409,10 @@ __device__ __forceinline__ void run_tile(const TilesArgs& a, char* lds_raw, int 
   }
 }
 
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep, bool TURN>
 __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(TilesArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
-  run_tile<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>(a, lds_raw, blockIdx.x % a.H, blockIdx.x / a.H);   // one head's tiles share an L2 when H % 8 == 0
+  run_tile<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep, TURN>(a, lds_raw, blockIdx.x % a.H, blockIdx.x / a.H);   // one head's tiles share an L2 when H % 8 == 0
 }
 
 // ------------------------------------------------------------------ heads of at most 128, one map, no cap
@@ -476,9 +478,9 @@ __device__ __forceinline__ void flow_out(const TilesArgs& a, int h, int64_t row,
     }
 }
 
-// FINE as above.  A wave's 32 queries are the columns of 32 x 32 products: lane l32 of either half holds one query's scores
+// FINE and TURN as above.  A wave's 32 queries are the columns of 32 x 32 products: lane l32 of either half holds one query's scores
 // for keys 8 (i / 4) + 4 half + i % 4 of a tile of 32, which are its operand elements of the products with values.
-template <int KS, int VB, bool FINE>
+template <int KS, int VB, bool FINE, bool TURN>
 __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef typename FlowStage<KS, VB>::K KL;
@@ -506,7 +508,7 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
   const int lo = first_seen(rel + w0, a.window, a.chunk), lo_last = first_seen(rel + w0 + 31, a.window, a.chunk);
   const int tiles = (last - first) / kTileK + 1;
   if constexpr (VB == 4)
-    if (tiles <= a.few_tiles) return run_tile<KS / 2, 1, 2, 1, false, kNoCap, FINE, 32>(a, lds_raw, h, tile);
+    if (tiles <= a.few_tiles) return run_tile<KS / 2, 1, 2, 1, false, kNoCap, FINE, 32, TURN>(a, lds_raw, h, tile);
   // tiles that queries of the wave see; none: they begin behind the last one
   const int seen0 = w0 < nq ? (lo - first) / kTileK : tiles + 1;
   const int seen1 = w0 < nq ? (rel + min(w0 + 32, nq) - 1 - first) / kTileK : tiles + 1;
@@ -557,7 +559,7 @@ __global__ __launch_bounds__(256, 2) void run_flow_kernel(TilesArgs a) {
       qf[ks] = *(const u32x4*)(q + (c < a.D ? c : 0));
       if (c >= a.D) qf[ks] = u32x4{0u, 0u, 0u, 0u};
     }
-    if (a.q_turns) {
+    if constexpr (TURN) {
       const zp_f32x4* const turns = a.q_turns + half * 4 * a.q_plane + q0 + qi;
       if constexpr (KS == 8) {
         if (a.q_half == 64) turn_queries<4, 16>(qf, turns, a.q_plane);
@@ -753,16 +755,16 @@ inline int few_tiles(const TilesArgs& a) {
   const int64_t groups = (int64_t)a.T * a.H;
   return groups >= 1024 ? 2 : groups >= 512 ? 1 : 0;
 }
-template <int KS, int VB, bool FINE> int launch_flow(const TilesArgs& args, hipStream_t st) {
+template <int KS, int VB, bool FINE, bool TURN> int launch_flow(const TilesArgs& args, hipStream_t st) {
   constexpr int flow = FlowStage<KS, VB>::kBytes, steps = VB == 4 ? TileStage<KS / 2, 1, 1>::kBytes : 0, smem = flow > steps ? flow : steps;
-  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)run_flow_kernel<KS, VB, FINE>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)run_flow_kernel<KS, VB, FINE, TURN>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               smem) != hipSuccess) {
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
   TilesArgs a = args;
   a.few_tiles = few_tiles(a);
-  hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE>), flow_grid(a), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((run_flow_kernel<KS, VB, FINE, TURN>), flow_grid(a), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -775,36 +777,39 @@ inline bool flow_takes(const TilesArgs& a) {
   return a.D <= 128 && a.V <= 128 && (a.V <= 64 || !few_keys(a)) && a.kv_st < 1 << 24 && a.v_st < 1 << 24 && grid.y < 65536 &&
          grid.z < 65536;
 }
-template <bool FINE> int launch_flow(const TilesArgs& a, hipStream_t st) {
-  if (a.V <= 64) return a.D <= 64 ? launch_flow<4, 2, FINE>(a, st) : launch_flow<8, 2, FINE>(a, st);
-  return a.D <= 64 ? launch_flow<4, 4, FINE>(a, st) : launch_flow<8, 4, FINE>(a, st);
+template <bool FINE, bool TURN> int launch_flow(const TilesArgs& a, hipStream_t st) {
+  if (a.V <= 64) return a.D <= 64 ? launch_flow<4, 2, FINE, TURN>(a, st) : launch_flow<8, 2, FINE, TURN>(a, st);
+  return a.D <= 64 ? launch_flow<4, 4, FINE, TURN>(a, st) : launch_flow<8, 4, FINE, TURN>(a, st);
 }
 
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep>
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE, int kStep, bool TURN>
 int launch_steps(const TilesArgs& a, hipStream_t st) {
   constexpr int smem = TileStage<DKS, VCB, MAPS>::kBytes;
   if (smem > 64 * 1024 &&
-      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>,
+      hipFuncSetAttribute((const void*)run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep, TURN>,
                           hipFuncAttributeMaxDynamicSharedMemorySize, smem) != hipSuccess) {
     zp_set_error("run_attention: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep>), dim3((unsigned)a.T * a.H),
+  hipLaunchKernelGGL((run_tiles_kernel<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kStep, TURN>), dim3((unsigned)a.T * a.H),
                      dim3(64 * TileStage<DKS, VCB, MAPS>::kWaves), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
-template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false>
+template <int DKS, int VCB, int kQT, int MAPS, bool SHARED, int CAP, bool FINE = false, bool TURN = false>
 int launch_run_tiles(const TilesArgs& a, hipStream_t st) {
   constexpr int kLong = long_step(DKS, VCB, MAPS, SHARED, CAP);
-  if (few_keys(a)) return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, 32>(a, st);
-  return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kLong>(a, st);
+  if (few_keys(a)) return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, 32, TURN>(a, st);
+  return launch_steps<DKS, VCB, kQT, MAPS, SHARED, CAP, FINE, kLong, TURN>(a, st);
 }
 
 template <bool SHARED, int CAP> int launch_one_map(const TilesArgs& a, hipStream_t st) {
   const int dk = (a.D + a.P + 31) / 32;
-  if constexpr (!SHARED && CAP == kNoCap)
-    if (flow_takes(a)) return launch_flow<false>(a, st);
+  if constexpr (!SHARED && CAP == kNoCap) {
+    if (flow_takes(a)) return a.q_turns ? launch_flow<false, true>(a, st) : launch_flow<false, false>(a, st);
+    if (a.q_turns)                                             // heads of at most 128
+      return dk <= 2 ? launch_run_tiles<2, 1, 2, 1, false, kNoCap, false, true>(a, st) : launch_run_tiles<4, 1, 2, 1, false, kNoCap, false, true>(a, st);
+  }
   if (a.V <= 128) {
     if (dk <= 2) return launch_run_tiles<2, 1, 2, 1, SHARED, CAP>(a, st);
     if (dk <= 4) return launch_run_tiles<4, 1, 2, 1, SHARED, CAP>(a, st);
@@ -903,6 +908,6 @@ extern "C" int zp_causal_attention(const void* q, const void* k, const void* v, 
   TilesArgs a = {(const uint16_t*)q, (const uint16_t*)k, (const uint16_t*)v, nullptr, (uint16_t*)out, tiles, nullptr, T, H, HK,
                  D, 0, D, 0, 0, q_rows, k_rows, q_stride, k_stride, v_stride, 0, out_stride, scale, 1.f, 0.f, 0.f, 0.f, D,
                  nullptr, 0, nullptr, nullptr, 0, 0, false};
-  if (flow_takes(a)) return launch_flow<true>(a, (hipStream_t)stream);
+  if (flow_takes(a)) return launch_flow<true, false>(a, (hipStream_t)stream);
   return launch_run_tiles<4, 1, 2, 1, false, kNoCap, true>(a, (hipStream_t)stream);
 }
