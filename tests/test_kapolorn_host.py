@@ -307,3 +307,16 @@ def test_experts_chosen_by_another_route():
         experts.router = torch.zeros(4, 64)
         with pytest.raises(Chosen):
             experts.forward(torch.zeros(3, 64))
+
+
+def test_rows_that_may_share_memory():
+    from zipage_amd.layers.grouped import _overlap
+    buf = torch.zeros(9, 40)
+    rows = lambda lo, hi, a=0, b=40: buf[lo:hi, a:b]
+    # one behind the other, whatever lies next to what
+    for a, b in ((rows(0, 4), rows(4, 9)), (rows(0, 4, 8, 40), rows(4, 9)), (rows(0, 4), rows(4, 9, 8)), (rows(0, 1), rows(1, 2)),
+                 (rows(3, 4, 0, 8), rows(3, 4, 8, 40)), (rows(0, 0), rows(0, 9)), (rows(2, 2), rows(1, 3))):
+        assert not _overlap(a, b) and not _overlap(b, a)
+    # rows that are the same, lie in each other or between each other
+    for a, b in ((rows(0, 4), rows(3, 9)), (rows(0, 9), rows(4, 5)), (rows(0, 9, 0, 8), rows(0, 9, 8, 40)), (rows(0, 4, 0, 8), rows(3, 5, 0, 8))):
+        assert _overlap(a, b) and _overlap(b, a)

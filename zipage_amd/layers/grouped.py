@@ -93,8 +93,8 @@ def grouped_rows_attention(q: torch.Tensor, cache: torch.Tensor, heads: int, kv_
 
 def _overlap(a: torch.Tensor, b: torch.Tensor) -> bool:
     """Whether two tensors of rows may share memory."""
-    end = lambda t: t.data_ptr() + (t.shape[0] * t.stride(0) + t.shape[1]) * t.element_size()
-    return a.data_ptr() < end(b) and b.data_ptr() < end(a)
+    end = lambda t: t.data_ptr() + ((t.shape[0] - 1) * t.stride(0) + t.shape[1]) * t.element_size()
+    return a.numel() > 0 and b.numel() > 0 and a.data_ptr() < end(b) and b.data_ptr() < end(a)
 
 
 class GroupedAttention:
