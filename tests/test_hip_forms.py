@@ -5,6 +5,7 @@ import torch
 from oracle import kapolorn_oracle as K
 from oracle import rutevik_oracle as R
 from oracle import zipage_oracle as O
+from zipage_amd.sight import Chunk
 
 pytestmark = pytest.mark.gpu
 BF16 = torch.bfloat16
@@ -322,6 +323,53 @@ def test_products_of_few_rows(dev, dtype, n, K, M):
     # rounding to 8 or 11 bits, and K terms in fp32, each sum within 2^-24 sqrt(K) of its terms' root of squares
     bits = 2.0 ** (-8 if dtype == BF16 else -11)
     assert bool(((out[:, :M].double() - want).abs() <= bits * want.abs() + 2.0 ** -20).all())
+
+
+# a mixer whose runs turn their queries, against the same with stored ones: whole prompts, portions that look back on pages, both beside
+# decoded tokens; values that turn too; heads as long as what turns and longer
+@pytest.mark.parametrize("H,G,D,V,rot,turning,sight", [(4, 2, 64, 64, 64, False, None), (4, 1, 128, 128, 128, True, 100),
+                                                       (2, 2, 96, 64, 64, True, Chunk(64)), (2, 1, 128, 48, 64, False, 100)])
+@pytest.mark.parametrize("portions", [[(0, 150), (0, 33)], [(70, 140), (5, 20)], [(40, 1), (0, 129), (99, 1), (64, 64)]])
+def test_mixers_turn_queries_late(dev, monkeypatch, H, G, D, V, rot, turning, sight, portions):
+    from zipage_amd.engine.inputs import Runs, plan_portions
+    from zipage_amd.engine.qwen3 import StepContext
+    from zipage_amd.engine.sequence import Portion, Sequence
+    from zipage_amd.layers import GroupedAttention, Rotary, grouped
+    mix = GroupedAttention(32, H, G, D, V, D ** -0.5, sight, Rotary(5e5, rot, interleaved=turning), turn_values=turning)
+    mix.load({k: _rand(*t, seed=i) for i, (k, t) in enumerate(mix.shapes().items())}, BF16, dev, 32)
+    assert mix._turns_late(1 << 20) and not mix._turns_late(200)
+    BS, work, free = 16, [], iter(torch.randperm(80, generator=torch.Generator().manual_seed(D)).tolist())
+    for start, count in portions:
+        seq = Sequence([0] * (start + count), block_size=BS)
+        seq.block_table = [next(free) for _ in range(-(-(start + count) // BS))]
+        work.append(Portion(seq, start, count))
+    plan = plan_portions(work, BS, [sight], 16)
+    t = lambda a: None if a is None else torch.as_tensor(a).to(dev)
+    ctx = StepContext(False, t(plan.slots), None, t(plan.context_lens), t(plan.tables), table_rows=t(plan.table_rows),
+                      runs={k: Runs(t(r.tiles), t(r.key_slots)) for k, r in plan.runs.items()})
+    N, singles, asked = len(plan.positions), len(plan.context_lens), []
+    held = _rand(80, BS, mix.row, seed=1).to(dev)
+    wide = _rand(N, mix.columns + mix.out_columns, seed=2).to(dev)
+    attention = grouped.run_attention
+    monkeypatch.setattr(grouped, "run_attention", lambda *a, form=None, **k: (asked.append(form is not None and bool(form.q_turns)),
+                                                                              attention(*a, form=form, **k)))
+
+    def go(late, proj, out):
+        monkeypatch.setattr(GroupedAttention, "_turns_late", lambda self, n: late)
+        cache = held.clone()
+        mix.attend(proj, t(plan.positions), cache, ctx, out)
+        return out.clone(), cache
+    proj = wide[:, :mix.columns]
+    want, cache = go(False, proj, torch.full((N, mix.out_columns), float("nan"), dtype=BF16, device=dev))
+    got, other = go(True, proj, torch.full((N, mix.out_columns), float("nan"), dtype=BF16, device=dev))
+    assert asked == [False, True] and torch.equal(cache, other) and torch.equal(got[:singles], want[:singles])
+    # as above
+    assert (got != want).float().mean() < 1e-3 and (got.float() - want.float()).abs().max() <= 2.0 ** -6 * want.float().abs().max()
+    # results beside the projections, between them, and where the queries are
+    for both, at in ((wide.clone(), mix.columns), (wide.clone(), 0)):
+        again, other = go(True, both[:, :mix.columns], both[:, at:at + mix.out_columns])
+        assert torch.equal(again, want) and torch.equal(cache, other)
+    assert asked == [False, True, False, False]
 
 
 # up to 256 rows: each of the four tile sizes at the most outputs that make 256 workgroups with it and at more; rows that leave one,
