@@ -772,11 +772,14 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   t.z = min(t.z - tile % a.split * per, per);
   if (t.z <= 0) return;
   constexpr int kPart = kTiles / 4;
-  if constexpr (HALVES == 2 && UP) return expert_tile<UP, HALVES, HT, kTiles>(a, lds_raw, t, cb);
-  if (t.z > 48 * kPart) expert_tile<UP, HALVES, HT, 4 * kPart>(a, lds_raw, t, cb);
-  else if (t.z > 32 * kPart) expert_tile<UP, HALVES, HT, 3 * kPart>(a, lds_raw, t, cb);
-  else if (HALVES == 2 || t.z > 16 * kPart) expert_tile<UP, HALVES, HT, 2 * kPart>(a, lds_raw, t, cb);
-  else if constexpr (HALVES == 1) expert_tile<UP, HALVES, HT, kPart>(a, lds_raw, t, cb);
+  if constexpr (HALVES == 2 && UP) {
+    expert_tile<UP, HALVES, HT, kTiles>(a, lds_raw, t, cb);
+  } else {
+    if (t.z > 48 * kPart) expert_tile<UP, HALVES, HT, 4 * kPart>(a, lds_raw, t, cb);
+    else if (t.z > 32 * kPart) expert_tile<UP, HALVES, HT, 3 * kPart>(a, lds_raw, t, cb);
+    else if (HALVES == 2 || t.z > 16 * kPart) expert_tile<UP, HALVES, HT, 2 * kPart>(a, lds_raw, t, cb);
+    else if constexpr (HALVES == 1) expert_tile<UP, HALVES, HT, kPart>(a, lds_raw, t, cb);
+  }
 }
 
 template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, hipStream_t st) {

@@ -1857,7 +1857,7 @@ static int attention_score(const void* k_cache, const void* query_cache,
   a.n_items = L * B * Hkv;
   a.part = (float*)workspace;
   auto leave = [&] {
-    if (left) *left = ScoreParts{a.part, a.RB, W, a.reduce_max, Gp};
+    if (left) *left = ScoreParts{a.part, a.RB, W, a.reduce_max};
     return left != nullptr;
   };
   const int64_t tiled = tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype);
