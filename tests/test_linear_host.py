@@ -128,3 +128,24 @@ def test_which_sizes_are_split(n, k, m, split):
 def test_products_of_nothing_stay_with_the_library(n, k, m):
     from zipage_amd.layers.linear import _few_rows, _row_tiles, _split_rows
     assert not (_few_rows(n, k, m) or _row_tiles(n, k, m) or _split_rows(n, k, m))
+
+
+# where either kernel was slower than the library: from both sides of the lines that keep these sizes there
+@pytest.mark.parametrize("n,k,m,tiles", [(65, 288, 8192, False), (65, 320, 8192, True), (65, 288, 4096, True), (69, 2016, 7620, True), (69, 2048, 7620, False),
+                                         (69, 2048, 4096, True), (112, 2048, 4100, False), (113, 2048, 4100, True), (129, 288, 4096, False),
+                                         (120, 4096, 1024, True), (120, 4096, 1028, False), (120, 4064, 1776, True), (128, 4096, 2176, False),
+                                         (128, 4096, 2180, True), (127, 4096, 3964, False), (127, 4096, 3968, True)])
+def test_which_sizes_are_no_row_tiles(n, k, m, tiles):
+    from zipage_amd.layers.linear import _row_tiles
+    assert _row_tiles(n, k, m) == tiles
+
+
+@pytest.mark.parametrize("n,k,m,split", [(48, 8192, 29952, True), (48, 8224, 29952, False), (49, 4608, 29952, True), (49, 4640, 29952, False),
+                                         (128, 4608, 32256, True), (128, 4640, 32256, False), (32, 5120, 24576, True), (32, 5152, 24576, False),
+                                         (128, 8192, 24576, True), (128, 8224, 24576, False), (32, 5120, 120000, True), (33, 5088, 120000, True),
+                                         (33, 5120, 120000, False), (80, 4096, 151936, False), (81, 4096, 151936, True), (96, 4096, 140000, True),
+                                         (97, 4096, 140000, False), (97, 4096, 147456, True), (144, 5888, 1788, False), (144, 5888, 1792, True),
+                                         (144, 6656, 1280, True), (80, 8192, 1660, False), (80, 8192, 1664, True), (81, 8192, 1280, True), (80, 8224, 1280, True)])
+def test_which_sizes_stay_whole(n, k, m, split):
+    from zipage_amd.layers.linear import _split_rows
+    assert _split_rows(n, k, m) == split

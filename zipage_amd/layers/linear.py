@@ -34,8 +34,9 @@ def _few_rows(n: int, k: int, m: int) -> bool:
     contraction that is worth a workgroup's beginning (128 -> 32 768 6.6 and 6.2, 1024 -> 65 536 29 and 27.5).
     Up to 32: as far as one round of workgroups goes (24 rows, 1024 -> 16 384 9.5 and 13.0, -> 20 480 15.1 and 14.4; 2048
     -> 8192 11.2 and 14.6, -> 9216 17.0 and 14.1; 4096 -> 4096 10.4 and 13.6, -> 6144 16.5 and 15.4).
-    Up to 64, since each workgroup reads all rows: 48 rows, 1024 -> 4096 6.6 and 11.3, 3072 -> 1024 11.3 and 11.7, but -> 2048
-    11.4 and 10.3, -> 256 10.6 and 9.3; 64 -> 8192 4.0 and 3.8."""
+    Up to 64, since each workgroup reads all rows: 48 rows, 1024 -> 4096 6.6 and 11.3, 3072 -> 1024 11.3 and 11.7 (which parts of the
+    contraction take first, unless rows lie more than 2^22 elements apart), but -> 2048 11.4 and 10.3, -> 256 10.6 and 9.3; 64 -> 8192
+    4.0 and 3.8."""
     if n <= 0 or k <= 0 or m <= 0 or k % 32 or m % 4 or k > 1 << 23:
         return False
     if n <= 16:
@@ -50,14 +51,19 @@ def _few_rows(n: int, k: int, m: int) -> bool:
 def _row_tiles(n: int, k: int, m: int) -> bool:
     """The same for 65 to 256 rows, in tiles of up to 64 x 64: what makes one round of workgroups, over contractions that are not much
     longer than their beginning and end (us of both: 65 to 128 rows, 1024 -> 4096 7.7 and 12.0, 2048 -> 1024 6.5 and 8.3, 2048 -> 4096
-    11.4 and 12.8, 128 -> 2048 4.1 and 4.0; 129 to 256, 1024 -> 4096 9.8 and 12.4, 2048 -> 2048 10.5 and 11.8).  The largest tiles for
-    short ones, since a CU has one workgroup with them (256 rows, 1536 -> 4096 12.7 and 11.2, 2048 -> 4096 18.1 and 13.2); longer
-    contractions up to 128 rows, where the library's tiles leave most of the chip idle (128 rows, 4096 -> 4096 18.2 and 23.5, 3072 ->
-    4096 14.9 and 20.2; 100 rows 17.7 and 16.5, 13.6 and 16.5; 4096 -> 6144 25.4 and 25.3)."""
+    11.4 and 12.8, 128 -> 2048 4.1 and 4.0; 129 to 256, 1024 -> 4096 9.8 and 12.4, 2048 -> 2048 10.5 and 11.8).  The largest tiles,
+    of which a CU has one workgroup, neither for long contractions (256 rows, 1536 -> 4096 12.7 and 11.2, 2048 -> 4096 18.1 and 13.2; 69
+    rows, 2048 -> 7620 15.3 and 14.6) nor for so short ones that writing decides (95 rows, 160 -> 5188 5.6 and 4.8).  Longer
+    contractions up to 128 rows, where the library's tiles leave most of the chip idle (128 rows, 3072 -> 4096 14.9 and 20.2; 100 rows 13.6
+    and 16.5; 113 to 128 rows, up to 4064 -> 1024 to 4096 1.3 to 1.6 times as fast), but not of 4096, whose rows the library reads better
+    (120 rows, -> 1776 14.2 and 12.8; 128, -> 2560 1.4 times as fast again).  Of these sizes 96 % of random ones are no more than 2 %
+    slower, on average they are 1.29 times as fast (13 700 of them)."""
     if not 64 < n <= 256 or m <= 0 or k % 32 or m % 4 or k < 96:
         return False
     tiles = lambda outs: -(-n // 64) * -(-m // outs)
-    if tiles(32) > 256 and (tiles(64) > 256 or k > (2048 if n <= 128 else 1024)):
+    if tiles(32) > 256 and (tiles(64) > 256 or not 320 <= k <= (1024 if n > 128 else 2048 if n > 112 else 2016)):
+        return False
+    if k == 4096 and 1024 < m <= (2176 if n == 128 else 3964):
         return False
     return k <= 2048 or n <= 128 and (n > 96 and k <= 3072 or n > 112 and k <= 4096)
 
@@ -68,32 +74,35 @@ def _split_rows(n: int, k: int, m: int) -> bool:
     and 89, 25.0 and 33.3; 256 rows 41 and 53, 28 and 39.5; 4096 -> 4096 17.3 and 23.5 for 128 rows, 21.6 and 31.5 for 192), and up to 64
     rows outputs of many rounds of workgroups (64 rows, 4096 -> 151 936 227 and 262; 48 rows, 1024 -> 151 936 66 and 77; 96 rows 259 and 273).
     Outputs that make one full round of them, in one part: up to 128 rows, 4096 -> 32 768 54 and 61 (64 rows), 51 and 67 (24), 58 and 64 (128),
-    2560 -> 32 512 33 and 44.
-    The library's choices are uneven, so the lines are drawn where 95 % of random sizes are no slower (300 sizes: 1.35 times as fast on
-    average): it is good at 6144 and 8192 -> 1280 and fewer (32 to 128 rows, 10.9 and 9.7), at contractions of 4096 of some rows (80 rows,
-    -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0; 255, -> 6144 28.0 and 26.3, but 224 26.6 and 36.2), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
-    its tiles fill the chip (256 rows, 4096 -> 24 576 64 and 62; but 128 rows 45.3 and 48.3)."""
+    2560 -> 32 512 33 and 44; longer contractions stream weights as fast in the library (96 rows, 9728 -> 29 952 138 and 118; 128 rows,
+    11 776 -> 32 256 189 and 152).
+    The library's choices are uneven, so the lines are drawn where nearly all random sizes are no slower: it is good at 6144 and 8192 -> 1280
+    and fewer (32 to 128 rows, 10.9 and 9.7; 144 to 184 rows to 1664, 20 and 17), at contractions of 4096 of some rows (80 rows,
+    -> 3392 17.0 and 16.2; 256 rows, -> 4096 24.1 and 22.0; 255, -> 6144 28.0 and 26.3, but 224 26.6 and 36.2), of 80 and 112 rows to many outputs
+    (80 rows, 2432 -> 132 352 182 and 144), at fewer than 2560 to 4096 (160 rows, 2560 -> 1216 14.3 and 9.6) and wherever
+    its tiles fill the chip (256 rows, 4096 -> 24 576 64 and 62; but 128 rows 45.3 and 48.3).  Of these sizes 98 % of random ones are no
+    more than 2 % slower, on average they are 1.44 times as fast (17 300 of them)."""
     if not 16 < n <= 256 or k % 32 or m % 4 or m < 512:
         return False
     if m >= 73728:
-        return k >= 1024 and n <= 64 or k >= 2048 and n <= 112 and m >= 131072
+        return 1024 <= k and (n <= 32 or n <= 64 and k <= 5088) or k >= 2048 and 80 < n <= (112 if m >= 147456 else 96) and m >= 131072
     if n <= 128 and 26880 <= m <= 32768:
-        return 2048 <= k <= 12288
-    if k < 2560 or m < 1280 and 6144 <= k <= 8192:
+        return 2048 <= k <= (8192 if n <= 48 else 4608)
+    if k < 2560 or m < (1664 if 64 < n <= 80 and k == 8192 else 1280) and 6144 <= k <= 8192:
         return False
     if n <= 32:
-        return 21504 <= m <= 25600 or k > 4608 and (1984 if k <= 8192 else 1280) <= m <= 4864
+        return k <= 5120 and 21504 <= m <= 25600 or k > 4608 and (1984 if k <= 8192 else 1280) <= m <= 4864
     if n <= 64:
         return m <= 10240 if k >= 4096 else m <= 1280 or 2816 <= m <= 8192
     if n <= 128:
         if 21120 <= m <= 24576:
-            return 3072 <= k <= 12288
+            return 3072 <= k <= 8192
         least = 1024 if k >= 5376 else 2432 if k >= 4480 else 3968 if n > 88 else 5632
         return k >= 4096 and least <= m <= 12288
     if k < 4096 or not 1024 <= m <= 12288:
         return False
     if n <= 192:
-        return k >= 5888 or 2816 <= m <= (6656 if k < 4608 else 12288)
+        return k >= 6656 or k >= 5888 and m >= 1792 or 2816 <= m <= (6656 if k < 4608 else 12288)
     return k >= 7168 or m >= 5888 and (k > 4608 or n % 32 == 0)
 
 
