@@ -29,8 +29,9 @@ struct FewArgs {
   int64_t x_st, o_st;
 };
 
-// 16 * TT rows of x (tiles of them side by side, which share W in the L2) and 16 * MT of W per workgroup, four waves that share the contraction.  Both pass through LDS in stages of
-// 128 elements of every row, a step of 32 for each wave: loads of whole cache lines, for the L1 takes four to five cycles for
+// 16 * TT rows of x (TILES: tiles of them side by side, which share W in the L2; otherwise these are all, and the division that finds
+// a tile, 0.1 to 0.4 us, is saved) and 16 * MT of W per workgroup, four waves that share the contraction.  Both pass through LDS in
+// stages of 128 elements of every row, a step of 32 for each wave: loads of whole cache lines, for the L1 takes four to five cycles for
 // every line touched, whole or in part.  A row's sixteen pieces lie in the order of (piece ^ row).  Bound by the weights'
 // stream: what counts is bytes in flight, so the ring takes what LDS there is, for two workgroups where the tiles are small.
 // Weights from memory, us (the library): 16 rows, 1024 -> 4096 4.4 (7.6), 2048 -> 1024 5.5 (11.0), 3072 -> 1024 6.7 (12.0), 4096
@@ -40,7 +41,7 @@ template <int TT, int MT> struct FewTile {
   static constexpr int kLoads = TT + MT, kBytes = kLoads * 4096;       // of a wave; of a stage
   static constexpr int kRing = kLoads <= 2 ? 9 : kLoads == 3 ? 6 : kLoads == 4 ? 9 : kLoads == 5 ? 7 : kLoads == 6 ? 6 : 5;
 };
-template <typename T, int TT, int MT>
+template <typename T, int TT, int MT, bool TILES>
 __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
   extern __shared__ __align__(16) char lds_raw[];
   typedef FewTile<TT, MT> Tile;
@@ -48,7 +49,8 @@ __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
   static_assert((R - 2) * L < 64, "loads that a wait can count");
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int row_tiles = (a.n + 16 * TT - 1) / (16 * TT), n0 = (int)(blockIdx.x % row_tiles) * 16 * TT, rows = min(16 * TT, a.n - n0);
+  const int row_tiles = TILES ? (a.n + 16 * TT - 1) / (16 * TT) : 1;
+  const int n0 = TILES ? (int)(blockIdx.x % row_tiles) * 16 * TT : 0, rows = TILES ? min(16 * TT, a.n - n0) : a.n;
   const int m0 = (int)(blockIdx.x / row_tiles) * 16 * MT, steps = a.K / 32, stages = (steps + 3) / 4;
   const int x_row = (int)a.x_st * 2;                     // bytes
   const u32x4 xr = rows_from(a.x + n0 * a.x_st, (uint32_t)(rows - 1) * x_row + a.K * 2);
@@ -115,14 +117,14 @@ __global__ __launch_bounds__(256, 2) void few_rows_kernel(FewArgs a) {
   }
 }
 
-template <typename T, int TT, int MT> int launch_few(const FewArgs& a, hipStream_t st) {
+template <typename T, int TT, int MT, bool TILES = false> int launch_few(const FewArgs& a, hipStream_t st) {
   constexpr int ring = FewTile<TT, MT>::kRing * FewTile<TT, MT>::kBytes, sums = TT * MT * 4096, smem = ring > sums ? ring : sums;
-  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)few_rows_kernel<T, TT, MT>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  if (smem > 64 * 1024 && hipFuncSetAttribute((const void*)few_rows_kernel<T, TT, MT, TILES>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               smem) != hipSuccess) {
     zp_set_error("few_rows_linear: cannot reserve %d bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((few_rows_kernel<T, TT, MT>), dim3((unsigned)((a.M + 16 * MT - 1) / (16 * MT) * ((a.n + 16 * TT - 1) / (16 * TT)))), dim3(256), smem, st, a);
+  hipLaunchKernelGGL((few_rows_kernel<T, TT, MT, TILES>), dim3((unsigned)((a.M + 16 * MT - 1) / (16 * MT) * ((a.n + 16 * TT - 1) / (16 * TT)))), dim3(256), smem, st, a);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -146,10 +148,10 @@ template <typename T> int launch_few(const FewArgs& a, hipStream_t st) {
 // -> 4096 10.1 (11.9), 512 -> 3072 7.4 (9.0), 1024 -> 768 6.0 (8.1), 128 -> 4096 5.5 (5.5).
 template <typename T> int launch_row_tiles(const FewArgs& a, hipStream_t st) {
   const auto groups = [&](int rows, int outs) { return (int64_t)((a.n + rows - 1) / rows) * ((a.M + outs - 1) / outs); };
-  if (groups(32, 16) <= kCUs) return launch_few<T, 2, 1>(a, st);
-  if (groups(32, 32) <= kCUs) return launch_few<T, 2, 2>(a, st);
-  if (groups(64, 32) <= kCUs) return launch_few<T, 4, 2>(a, st);
-  return launch_few<T, 4, 4>(a, st);
+  if (groups(32, 16) <= kCUs) return launch_few<T, 2, 1, true>(a, st);
+  if (groups(32, 32) <= kCUs) return launch_few<T, 2, 2, true>(a, st);
+  if (groups(64, 32) <= kCUs) return launch_few<T, 4, 2, true>(a, st);
+  return launch_few<T, 4, 4, true>(a, st);
 }
 
 
