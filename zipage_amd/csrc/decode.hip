@@ -377,13 +377,14 @@ constexpr int kSliceTokens = 2048;
 // Workgroups on a CU: one of 512 threads where all have a CU to themselves, for what then bounds it is bytes in flight (8
 // sequences of about 2150 tokens, 32 heads over 8 of 128 54 us with 256 threads, 40 with 512 and 42 with 1024); more are better
 // off with four of 256 (64 sequences of 450 28 and 30, 40 of 2150 77 and 80; 256 of 2150 357 and 361), and so are contexts of up
-// to 128 tokens, of which the second four waves have nothing (8 sequences of 73 12.6 and 15.1, 16 of 68 8.0 and 9.3; of 200 10.1 and
-// 9.5), with groups of eight heads up to 450 (4 of 400 13.5 and 14.0).  The longest context ends in the tables' last column.
+// to 128 tokens, of which the second four waves have nothing (8 sequences of 73, 64 heads over 8 of 128 12.6 and 15.1, 16 of 69, 32 over 8 of
+// 64 8.1 and 9.4; but 14 of 255, 16 over 8 9.2 and 8.5), with groups of eight heads up to 450 (6 of 393, 64 over 8 19.4 and 20.2).
+// The longest context ends in the tables' last column.
 constexpr int kCUs = 256;
 int decode_threads(const DecodeArgs& a) {
   return (int64_t)a.B * a.Hkv <= kCUs && (int64_t)(a.NB - 1) * a.BS >= (a.G > 4 ? 448 : 128) ? 512 : 256;
 }
-// Parts of a context: what makes a workgroup per CU, of 256 tokens and more, for a workgroup that has a CU to itself reads 25 to 34 GB/s.
+// Parts of a context: what makes a workgroup per CU, of 256 tokens and more, for a workgroup that has a CU to itself reads about 25 GB/s.
 // us with one part: 8 sequences of about 1900 tokens, 32 heads over 8 39 -> 24, 16 heads 33 -> 21; 16 sequences 40 -> 31 and 35 -> 28; one
 // 37 -> 17; 12 of 900 25.2 -> 20.7.  More than fill the chip are slower (8 sequences in 8 parts 29), as are two parts of 24
 // sequences (43 -> 48); tables of fewer than 1024 tokens gain 1 to 3 us and lose as much of the host's time to a launch.
