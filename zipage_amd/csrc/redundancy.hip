@@ -1947,10 +1947,11 @@ void gram_raw_kernel(GramArgs p) {
 // fragment read from LDS feeds two products; the column tiles go from global memory straight into
 // LDS (wave w requests rows 32 w .. 32 w + 31 of a tile, the layout of `gram_page_kernel`), two
 // buffers, one barrier per tile, the request for tile t + 1 under the products of tile t.  Two
-// workgroups per compute unit (two waves per SIMD, 256 registers each).
+// workgroups per compute unit (two waves per SIMD, 256 registers each).  PARTS: a workgroup has some of
+// a page's tiles (see tile_parts); where it has all, first and last tile are known, which is 2 to 3 % of the kernel.
 constexpr int kRawTile = 128;
 constexpr int kRawTileBytes = (kRawTile / 4) * kPgGrp;
-template <typename T>
+template <typename T, bool PARTS>
 __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   static_assert(T::bytes == 2, "16-bit caches only");
   typedef typename Mfma16<T>::V frag_t;
@@ -1972,7 +1973,8 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, col = lane & 31;
-  const unsigned pages = gridDim.x / p.parts, page = blockIdx.x % pages, part = blockIdx.x / pages;
+  const int pages = PARTS ? gridDim.x / p.parts : gridDim.x;
+  const int page = PARTS ? blockIdx.x % pages : blockIdx.x, part = PARTS ? blockIdx.x / pages : 0;
   const int jp = page % p.NB;
   const int h = (page / p.NB) % p.Hkv;
   const int b = (page / (p.NB * p.Hkv)) % p.B;
@@ -1995,7 +1997,8 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int nv = nvalid_s, ia = mine_s;
   const int nd = nv / 2 + (((nv & 1) || ia < nv / 2) ? 1 : 0);   // page distances 0 .. nd-1
   const int tiles_per_page = p.BS / TNc;
-  const int from = nd * tiles_per_page * part / p.parts, to = nd * tiles_per_page * (part + 1) / p.parts;   // its tiles
+  const int from = PARTS ? nd * tiles_per_page * part / p.parts : 0;                       // its tiles
+  const int to = PARTS ? nd * tiles_per_page * (part + 1) / p.parts : nd * tiles_per_page;
   const int k_row = p.Hkv * p.D * 2;
   const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2;
   const float* rn_all = p.ws_val + obase;           // written by raw_prep_kernel
@@ -2736,7 +2739,9 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
       zp_set_error("redundancy: a row of %d tokens exceeds LDS", a.NB * a.BS);
       return ZP_EUNSUPPORTED;
     }
-    if (hipFuncSetAttribute(wide ? (const void*)gram_raw_wide_kernel<T> : fn,
+    const GramArgs cut = tile_parts(a, grid.x), claims = claim_parts(a, grid.x);
+    const void* const wide_fn = cut.parts > 1 ? (const void*)gram_raw_wide_kernel<T, true> : (const void*)gram_raw_wide_kernel<T, false>;
+    if (hipFuncSetAttribute(wide ? wide_fn : fn,
                             hipFuncAttributeMaxDynamicSharedMemorySize, (int)(wide ? smemw : smem1)) != hipSuccess ||
         hipFuncSetAttribute((const void*)raw_chain_kernel<T>, hipFuncAttributeMaxDynamicSharedMemorySize,
                             (int)smem2) != hipSuccess) {
@@ -2744,8 +2749,8 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
       return ZP_EHIP;
     }
     hipLaunchKernelGGL((raw_prep_kernel<T>), grid, dim3(kThreads), 0, st, a);
-    const GramArgs cut = tile_parts(a, grid.x), claims = claim_parts(a, grid.x);
-    if (wide) hipLaunchKernelGGL((gram_raw_wide_kernel<T>), dim3(grid.x * cut.parts), dim3(256), smemw, st, cut);
+    if (wide && cut.parts > 1) hipLaunchKernelGGL((gram_raw_wide_kernel<T, true>), dim3(grid.x * cut.parts), dim3(256), smemw, st, cut);
+    else if (wide) hipLaunchKernelGGL((gram_raw_wide_kernel<T, false>), grid, dim3(256), smemw, st, cut);
     else if (tn == 128) hipLaunchKernelGGL((gram_raw_kernel<T, 128>), grid, dim3(512), smem1, st, a);
     else hipLaunchKernelGGL((gram_raw_kernel<T, TN>), grid, dim3(512), smem1, st, a);
     hipLaunchKernelGGL((raw_claim_value_kernel<T>), dim3(grid.x * claims.parts), dim3(kThreads), 0, st, claims);
