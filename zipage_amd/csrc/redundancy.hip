@@ -2185,37 +2185,46 @@ __global__ __launch_bounds__(kThreads) void raw_claim_value_kernel(GramArgs p) {
   const bool pok = piece < p.D / 8;
   const int64_t k_row = (int64_t)p.Hkv * p.D * 2;
   const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2 + (pok ? piece : 0) * 16;
-  for (int slot = part * GROUPS + g; slot < p.BS; slot += GROUPS * p.parts) {
-    const int64_t oi = obase + (int64_t)jp * p.BS + slot;
-    const int c = p.ws_col[oi];
-    if (c < 0 || c >= Tn) continue;     // uniform over the 16 lanes of a key
-    if (c == jp * p.BS + slot) {        // negative threshold: the zeroed diagonal entry was claimed
-      if (piece == 0) p.ws_val[oi] = 0.f;
-      continue;
-    }
-    const int cp = c / p.BS, cs = c - cp * p.BS;
-    const int ccode = p.table[(int64_t)b * p.NB + cp];
-    const int cpid = page_is_pad(ccode) ? -1 : page_id(ccode);
-    if (cpid < 0 || cpid >= p.num_pages) continue;
-    u32x4 ra = *(const u32x4*)(kbase + (int64_t)rpid * p.k_sp * 2 + (int64_t)slot * k_row);
-    u32x4 rc = *(const u32x4*)(kbase + (int64_t)cpid * p.k_sp * 2 + (int64_t)cs * k_row);
-    if (!pok) { ra = u32x4{0u, 0u, 0u, 0u}; rc = ra; }
-    float ea[8], ec[8];
-    Unpack<T>::run(vec16{ra.x, ra.y, ra.z, ra.w}, ea);
-    Unpack<T>::run(vec16{rc.x, rc.y, rc.z, rc.w}, ec);
-    float sa = 0.f, sc = 0.f, t = 0.f;
+  // The claims of all keys are asked for at once; one after the other, each waits for memory, and where there are none that is all there
+  // is to do (2880 pages without claims 12.3 us, now 6.6; with claims of half of the keys 60 and 59).
+  __shared__ int l_claim[kThreads];
+  for (int s0 = 0; s0 < p.BS; s0 += kThreads) {
+    const int n = min(kThreads, p.BS - s0), mine = tid < n ? p.ws_col[obase + (int64_t)jp * p.BS + s0 + tid] : -1;
+    if (s0 > 0) __syncthreads();
+    l_claim[tid] = mine;
+    if (!__syncthreads_or(mine >= 0)) continue;
+    for (int i = part * GROUPS + g; i < n; i += GROUPS * p.parts) {
+      const int slot = s0 + i, c = l_claim[i];
+      const int64_t oi = obase + (int64_t)jp * p.BS + slot;
+      if (c < 0 || c >= Tn) continue;     // uniform over the 16 lanes of a key
+      if (c == jp * p.BS + slot) {        // negative threshold: the zeroed diagonal entry was claimed
+        if (piece == 0) p.ws_val[oi] = 0.f;
+        continue;
+      }
+      const int cp = c / p.BS, cs = c - cp * p.BS;
+      const int ccode = p.table[(int64_t)b * p.NB + cp];
+      const int cpid = page_is_pad(ccode) ? -1 : page_id(ccode);
+      if (cpid < 0 || cpid >= p.num_pages) continue;
+      u32x4 ra = *(const u32x4*)(kbase + (int64_t)rpid * p.k_sp * 2 + (int64_t)slot * k_row);
+      u32x4 rc = *(const u32x4*)(kbase + (int64_t)cpid * p.k_sp * 2 + (int64_t)cs * k_row);
+      if (!pok) { ra = u32x4{0u, 0u, 0u, 0u}; rc = ra; }
+      float ea[8], ec[8];
+      Unpack<T>::run(vec16{ra.x, ra.y, ra.z, ra.w}, ea);
+      Unpack<T>::run(vec16{rc.x, rc.y, rc.z, rc.w}, ec);
+      float sa = 0.f, sc = 0.f, t = 0.f;
 #pragma unroll
-    for (int q = 0; q < 8; ++q) {
-      sa = fmaf(ea[q], ea[q], sa);
-      sc = fmaf(ec[q], ec[q], sc);
-      t = fmaf(ea[q], ec[q], t);
+      for (int q = 0; q < 8; ++q) {
+        sa = fmaf(ea[q], ea[q], sa);
+        sc = fmaf(ec[q], ec[q], sc);
+        t = fmaf(ea[q], ec[q], t);
+      }
+      sa = pieces_sum<PIECES>(sa);
+      sc = pieces_sum<PIECES>(sc);
+      t = pieces_sum<PIECES>(t);
+      const float rna = __builtin_amdgcn_rcpf(fmaxf(Elem<T>::rnd(sqrtf(sa)), epsr));
+      const float rnc = __builtin_amdgcn_rcpf(fmaxf(Elem<T>::rnd(sqrtf(sc)), epsr));
+      if (piece == 0) p.ws_val[oi] = t * rna * rnc;
     }
-    sa = pieces_sum<PIECES>(sa);
-    sc = pieces_sum<PIECES>(sc);
-    t = pieces_sum<PIECES>(t);
-    const float rna = __builtin_amdgcn_rcpf(fmaxf(Elem<T>::rnd(sqrtf(sa)), epsr));
-    const float rnc = __builtin_amdgcn_rcpf(fmaxf(Elem<T>::rnd(sqrtf(sc)), epsr));
-    if (piece == 0) p.ws_val[oi] = t * rna * rnc;
   }
 }
 
@@ -2663,10 +2672,12 @@ GramArgs tile_parts(GramArgs a, int64_t pages) {
   }
   return a;
 }
-// The keys of a page, whose claims are looked up one after the other (us with 1, 2, 4 and 8 workgroups: 80 pages 15.5, 9.4, 6.0, 5.0;
-// 320 21.1, 13.2, 9.7, 10.2; 1152 28.5, 25.4, 23.8, 26.9; 2880 53.0, 49.8, 52.3, 61.9).
+// The keys of a page, whose claims are looked up one after the other, go to several workgroups where all of them run at once, six on a
+// CU: more take longer to launch than the claims of most pages (us with 1, 2, 4 and 8 workgroups, without claims and with claims of
+// half of the keys: 72 pages of 256 4.5, 4.5, 4.6, 4.4 and 12.7, 7.8, 5.7, 5.0; 288 4.6, 4.6, 4.9, 5.5 and 16.6, 11.2, 9.4, 10.2; 576 4.7,
+// 4.6, 5.5, 8.8 and 21.0, 15.2, 14.8, 15.9; 1728 4.6, 7.2, 12.4, 23 and 36.8, 35.9, 33.6, 39.4).
 GramArgs claim_parts(GramArgs a, int64_t pages) {
-  a.parts = pages <= 256 ? 8 : pages <= 2048 ? 4 : pages <= INT32_MAX / 2 ? 2 : 1;
+  for (a.parts = 8; a.parts > 1 && pages * a.parts > 1536; a.parts /= 2) {}
   return a;
 }
 
