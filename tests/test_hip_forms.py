@@ -517,7 +517,7 @@ def test_products_of_few_rows_keep_tangents(dev, few_rows_calls):
 
 
 # ------------------------------------------------------------------ raw redundancy of few sequences
-# pages of few sequences are worked on in parts (five, three, two; the claims' in eight and four), of twelve whole: the same bits.  Odd and
+# pages of few sequences are worked on in parts (five, three, two; the claims' in eight, four and two), of twelve whole: the same bits.  Odd and
 # even numbers of pages, padding, near copies of keys in their own page, in others and across the parts' edges
 @pytest.mark.parametrize("dtype", [BF16, torch.float16])
 @pytest.mark.parametrize("BS,pages", [(128, (9, 9, 8, 9)), (256, (3, 4, 4, 1)), (384, (2, 1, 2, 2))])
