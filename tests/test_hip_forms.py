@@ -169,6 +169,40 @@ def test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act, shared_
     assert float(err) < 2.0 ** -8 and bool(torch.isfinite(got).all())
 
 
+# averages of 8, 9, 16, 17 and 48 rows; tiles that eight XCDs cannot have as many of each, over several blocks of columns;
+# launches of few rows that are no multiple of eight workgroups; a shared expert of one to three tiles of 16
+@pytest.mark.parametrize("n,width,E,top,ff", [(40, 96, 5, 1, 544), (45, 96, 5, 1, 544), (80, 544, 5, 1, 800), (85, 544, 5, 1, 800),
+                                              (240, 800, 5, 1, 288), (130, 800, 11, 2, 1056), (7, 160, 5, 1, 32), (17, 160, 5, 1, 96),
+                                              (33, 288, 6, 1, 160), (48, 96, 9, 1, 352)])
+@pytest.mark.parametrize("act", ["clamped", "silu"])
+def test_experts_among_xcds(dev, n, width, E, top, ff, act):
+    test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act)
+
+
+def test_experts_of_many_weights_spread_over_xcds(dev):
+    """Few rows against 380 MB of weights: every expert as by itself, whose weights are one XCD's share."""
+    from zipage_amd.layers import Experts
+    from zipage_amd.layers.moe import Plan
+    E, n, W, ff = 7, 24, 4096, 3328
+    m = Experts(W, E, 1, ff, 7.0)
+    m.random(BF16, dev, torch.Generator(device=dev).manual_seed(1))
+    plan = lambda ids_, experts: Plan(ids_, torch.zeros(experts + 1, dtype=torch.int32, device=dev), experts, False, BF16)
+    h, ids_ = _rand(n, W, seed=2).to(dev), (torch.arange(n, device=dev) * 5 % E).to(torch.int32)[:, None]
+    p, one = plan(ids_, E), torch.ones(n, 1, device=dev)
+    act = m.gate_up_rows(h, p, one)
+    down, order = m.down_planes(act, p)[0], p.sorted.long()
+    assert p.rows == 16
+    for e in range(E):
+        mine = (ids_[:, 0] == e).nonzero()[:, 0]
+        alone = Experts(W, 1, 1, ff, 7.0)
+        alone.gate_up, alone.down, alone.shared_gate_up, alone.shared_down = m.gate_up[e:e + 1], m.down[e:e + 1], None, None
+        q = plan(torch.zeros(len(mine), 1, dtype=torch.int32, device=dev), 1)
+        a = alone.gate_up_rows(h[mine].contiguous(), q, one)
+        at = (order[:, None] == mine[q.sorted.long()]).nonzero()
+        assert torch.equal(act[at[at[:, 1].argsort(), 0]], a)
+        assert torch.equal(down[mine], alone.down_planes(a, q)[0])
+
+
 # 256-row tiles whose contraction leaves 0 to 3 steps behind the loop, which takes four at a time, in either product; a
 # shared expert that has fewer steps than the loop takes
 @pytest.mark.parametrize("n,width,ff,shared_ff", [(530, 2560, 48, 0), (530, 2592, 48, 0), (530, 2624, 48, 0), (530, 2656, 48, 0),

@@ -380,6 +380,7 @@ struct ExpertArgs {
   int act;
   float limit, limit_shared;
   int split;              // parts in which expert_tiles_kernel takes a tile
+  bool together;          // expert_rows_kernel: an XCD takes a contiguous share of the launch, see launch_experts
 };
 
 // ZP_GATE_CLAMPED: w g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
@@ -417,7 +418,8 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tile = blockIdx.x % a.max_tiles, cb = blockIdx.x / a.max_tiles;
+  const int at = a.together ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const int tile = at % a.max_tiles, cb = at / a.max_tiles;
   if (tile >= *a.ntiles) return;
   const int4 t = *(const int4*)(a.tiles + (int64_t)tile * 4);
   const bool shared = t.x == a.E;
@@ -756,15 +758,15 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   constexpr int kTiles = HT * HALVES, kGroup = 8;
   extern __shared__ __align__(16) char lds_raw[];
   // An XCD takes a contiguous share of the (tile, column block) pairs, eight tiles at a time, column block by column
-  // block, so that what is in flight on it shares rows of x and of W in its L2.
+  // block, so that what is in flight on it shares rows of x and of W in its L2.  Shares are of pairs, not of tiles: 33 tiles in
+  // shares of five left the last XCD and half of another without work (8 experts and a shared one of 3 x 4096 x 14336, 180
+  // tokens 792 -> 644 us; 3200 tokens of 3 of 32 of 3 x 4096 x 3072 1194 -> 1153).
   const int nt = *a.ntiles * a.split;
   const int Mx = max(a.M, a.M_shared) * (UP ? 2 : 1), cols = (Mx + 16 * kBlockW - 1) / (16 * kBlockW);
-  const int share = (nt + 7) / 8 * cols, i_xcd = blockIdx.x >> 3;
-  if (i_xcd >= share) return;
-  const int lin = (blockIdx.x & 7) * share + i_xcd;
-  const int tg = lin / (kGroup * cols), rem = lin - tg * kGroup * cols;
-  const int tile = tg * kGroup + rem % kGroup, cb = rem / kGroup;
-  if (tile >= nt) return;
+  const int pairs = nt * cols, share = (pairs + 7) / 8, i_xcd = blockIdx.x >> 3, lin = (blockIdx.x & 7) * share + i_xcd;
+  if (i_xcd >= share || lin >= pairs) return;
+  const int tg = lin / (kGroup * cols), rem = lin - tg * kGroup * cols, in_group = min(kGroup, nt - tg * kGroup);
+  const int tile = tg * kGroup + rem % in_group, cb = rem / in_group;
   int4 t = *(const int4*)(a.tiles + (int64_t)(tile / a.split) * 4);
   // a part of a larger tile
   const int per = a.split > 1 ? ((t.z + a.split - 1) / a.split + 15) & ~15 : kTiles * 16;
@@ -804,12 +806,18 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
   const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
   const bool wide = rows == 16 && dtype == ZP_BF16 && a.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
                     (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
-  const int64_t grid = grid_of(wide ? kWideW : kNarrowW);
+  const int64_t grid = (grid_of(wide ? kWideW : kNarrowW) + 7) / 8 * 8;      // shares of eight XCDs; behind the last tile of W nothing is done
   if (grid >= (1ll << 31)) {
     zp_set_error("moe: too many tiles");
     return ZP_EUNSUPPORTED;
   }
-#define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, a)
+  // The shared expert's tiles read the same weights: on one XCD, one after the other, they find them in its L2 (64 tokens of 3 of
+  // 32 experts and a shared one of 3 x 4096 x 3072: 475 -> 425 us, 53: 432 -> 416, 32: 441 -> 417; 24, with two such tiles, 383
+  // and 386).  Without one, weights that the last-level cache holds gain too (3 x 1024 x 768, 4 of 32, 17 tokens 43.9 -> 41.5);
+  // those from memory come faster spread over all (3 x 4096 x 3072, 17 tokens 347, 360 in shares; 64: 383, 390).
+  ExpertArgs b = a;
+  b.together = a.slots > a.top || (int64_t)a.E * a.w_expert * (dtype == ZP_BF16 ? 2 : 4) < 320ll << 20;
+#define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, b)
 #define ZP_EXPERT_ROWS(T)                            \
   do {                                               \
     if (rows == 16) ZP_EXPERTS(T, 1, kNarrowW);      \
@@ -825,11 +833,17 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
   return ZP_OK;
 }
 
-// Rows per tile: enough for the average expert.
+// Rows per tile: enough for the average expert.  From 17 rows of bf16 on tokens go through LDS: read by every wave for itself, 64
+// rows take more lines of the L1 than the weights that they meet (tiles of 128 and, before, of 64: 3 of 32 experts and a shared
+// one of 3 x 4096 x 3072, 200 tokens 490 and 542 us, 256 496 and 673, 480 515 and 694; of 3 x 1024 x 768, 200 51 and 60, 480 53
+// and 68; 8 of 128 of 3 x 2048 x 768, 320 tokens 234 and 261).  With up to 16, tiles of 32 lose up to 4 % without a shared expert
+// (100 tokens of 4 of 32, 437 and 453) and win up to 9 % with one, whose tile of 128 rows starts a second round of workgroups (96
+// tokens 512 and 470).  Launches of that form address x in 31 bits, so many tokens over many experts stay with tiles of 64.
+constexpr int kMostStaged = 16384;
 int tile_rows(int n, int E, int top, int dtype) {
   const int64_t avg = ((int64_t)n * top + E - 1) / E;
   if (dtype == ZP_BF16 && avg > 512) return kBigRows;
-  if (dtype == ZP_BF16 && avg > 48) return 128;
+  if (dtype == ZP_BF16 && (avg > 48 || (avg > 16 && n <= kMostStaged))) return 128;
   return avg <= 8 ? 16 : (avg <= 16 ? 32 : 64);       // a second tile reads an expert's weights again
 }
 int tile_bound(int n, int E, int top, int shared, int rows) {
@@ -968,7 +982,7 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
     }
   }
   ExpertArgs a = {x, w, w_shared, out, sorted, tiles, ntiles, weights, n, E, top, top + shared, max_tiles, K, K_shared,
-                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1};
+                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false};
   return up ? launch_experts<true>(a, rows, dtype, (hipStream_t)stream)
             : launch_experts<false>(a, rows, dtype, (hipStream_t)stream);
 }
