@@ -714,6 +714,38 @@ def _run_segments(dev, counts):
     return rows, types.SimpleNamespace(segments=None, run_segments=seg)
 
 
+# Blocks of 16 tokens go in pairs: one block, a second one of one token to all, a third; channels that forget little, some that
+# leave the range of a reciprocal within a block, and all of them.
+@pytest.mark.parametrize("bias,spread", [(-3.0, 1.0), (-2.0, 6.0), (12.0, 1.0)])
+@pytest.mark.parametrize("H,G,D,V,taps", [(2, 1, 128, 128, 4), (3, 3, 64, 64, 2), (2, 1, 32, 96, 8), (1, 1, 128, 32, 1), (2, 2, 64, 128, 3)])
+def test_delta_runs_in_pairs_of_blocks(dev, H, G, D, V, taps, bias, spread):
+    import types
+    from zipage_amd.engine.qwen3 import Segments
+    from zipage_amd.layers import ChannelDelta
+    counts, W = [1, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 97], 64
+    m, n, rows = ChannelDelta(W, H, G, D, V, taps, 1e-3), len(counts), sum(counts)
+    shapes = m.shapes(8, 8)
+    w = {k: _rand(*s, seed=i) * s[-1] ** -0.5 for i, (k, s) in enumerate(shapes.items())}
+    w["dt_bias"] = (bias + spread * _rand(H * D, seed=52).float()).to(BF16)
+    into, _ = m.load(w, BF16, dev, W)
+    proj = (_rand(rows, W, seed=60).to(dev).float() @ into.to(dev).float().T).to(BF16)
+    t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
+    seg = Segments(t([sum(counts[:i]) for i in range(n)]), t(counts), t(list(range(n, 0, -1))),
+                   t([0 if i % 2 or c < taps else 333 for i, c in enumerate(counts)]), longest=max(counts))
+
+    def scan(runs):
+        state = m.allocate(n + 1, BF16, dev)
+        state[0].copy_((0.1 * _rand(*state[0].shape, seed=61).float()).to(dev))
+        state[1].copy_(_rand(*state[1].shape, seed=62))
+        out = torch.empty(rows, m.out_columns, dtype=BF16, device=dev)
+        m.scan(proj, state, types.SimpleNamespace(segments=None if runs else seg, run_segments=seg if runs else None), out)
+        return out.float(), state[0].double()
+    (got, gs), (want, ws) = scan(True), scan(False)
+    # as in pieces of runs: sums of up to 100 terms in fp32, exponentials of another function; rows rounded to 2^-9
+    assert float((gs - ws).norm() / ws.norm()) < 2.0 ** -15
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -8 and bool(torch.isfinite(got).all())
+
+
 # operands enter the bf16 matrix cores in three planes: the state has to stay as good as fp32's
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 128, 128), (2, 2, 32, 96), (3, 1, 64, 32), (1, 1, 128, 64)])
 def test_delta_state_of_runs(dev, H, G, D, V):

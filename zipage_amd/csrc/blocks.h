@@ -75,6 +75,7 @@ struct PlanePairs {
     ll = u32x4{p.lo.x, p.lo.y, p.lo.x, p.lo.y};
     hm = u32x4{p.hi.x, p.hi.y, p.mid.x, p.mid.y};
   }
+  __device__ __forceinline__ PlanePairs(const u32x4 (&p)[4]) : hh(p[0]), mm(p[1]), ll(p[2]), hm(p[3]) {}
   __device__ __forceinline__ void add(const u32x4& left, const uint2& lo, f32x4& c) const {
     c = mfma_bf16(left, ll, c);
     c = mfma_bf16(u32x4{lo.x, lo.y, lo.x, lo.y}, hm, c);
@@ -182,7 +183,7 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 }
 
 // ------------------------------------------------------------------ runs in pieces
-// A head walks its blocks one after the other, 2.5 us each whatever else the chip does, and a few heads leave most CUs idle.
+// A head walks its blocks one after the other, 2.4 us each, and a few heads leave most CUs idle.
 // The state behind a piece of a run is (what the piece keeps) * (the state before it) + what the piece adds to none, so few
 // heads walk their runs in pieces side by side:
 //
@@ -190,13 +191,14 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 //   states   the states between pieces, from the first to the last
 //   blocks   as without pieces, each from its state on
 //
-// Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) allow.  Where the sums and the two
+// Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) and the chain of states between them
+// allow.  Where the sums and the two
 // launches cost more than what is saved, runs stay whole (PieceCost): a block of the sums takes 0.3 of one with rows (0.8 for the
-// delta rule), the launches 19 us (15 for the delta rule, whose blocks are the longer ones), states of the delta rule 2.4 us a
+// delta rule), the launches 19 us (17 for the delta rule, whose blocks are the longer ones), states of the delta rule 5.7 us a
 // piece (matrix memory, 8 heads, a prompt of 155 tokens: whole 41.8 us, in pieces 42.8; linear attention, 32 heads, 200
 // tokens: 53, 46).  Whole scans: linear attention, 32 heads of 128,
 // 4 prompts of 500 to 2048 tokens 374 -> 287 us; 16 heads, 8 prompts of 2048, retention 429 -> 332 and matrix memory 369
-// -> 285; retention, a prompt of 700 126 -> 45; delta rule, 32 heads, a prompt of 2048 477 -> 269, two of about 1250 384 -> 314.
+// -> 285; retention, a prompt of 700 126 -> 45; delta rule, 32 heads, a prompt of 2048 477 -> 269 (now 227), two of about 1250 384 -> 314 (262).
 constexpr int kPieceGroups = 256, kPieceStates = 384, kLeastPiece = 4;
 struct Pieces {
   int blocks = 0, most = 1;      // of a piece, 0: runs are whole; pieces of the longest run at most
@@ -212,16 +214,19 @@ inline int64_t most_states(int64_t rows, int64_t segments, int64_t heads, const 
   const int64_t states = piece_slots(rows, segments, kLeastPiece) * heads;
   return states < kPieceStates ? states : kPieceStates;
 }
-// Runs stay whole, too, where `room` states are not enough.
-inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest, const PieceCost& cost, int64_t room) {
+// Runs stay whole, too, where `room` states are not enough.  `step`: blocks that are walked together.
+inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t longest, const PieceCost& cost, int step, int64_t room) {
   Pieces p;
   const int64_t all = (longest + kBlock - 1) / kBlock;
   if (!few_heads(segments, heads)) return p;
-  for (int64_t m = kLeastPiece; m < all; ++m) {
+  int64_t best = all * 10;
+  for (int64_t m = kLeastPiece; m < all; m += step) {
     const int64_t most = (all + m - 1) / m, slots = piece_slots(rows, segments, m), pieces = segments * most < slots ? segments * most : slots;
-    if (pieces * heads > kPieceGroups || (pieces - segments) * heads * cost.groups > kPieceGroups || slots * heads > kPieceStates) continue;
-    if (m * (10 + cost.sum) + cost.fixed + most * cost.state < all * 10 && slots * heads <= room) p.blocks = (int)m, p.most = (int)most;
-    return p;
+    const int64_t took = m * (10 + cost.sum) + cost.fixed + most * cost.state;
+    if (pieces * heads > kPieceGroups || (pieces - segments) * heads * cost.groups > kPieceGroups || slots * heads > kPieceStates ||
+        slots * heads > room || took >= best) continue;
+    best = took;
+    p.blocks = (int)m, p.most = (int)most;
   }
   return p;
 }

@@ -1,14 +1,12 @@
-// Gated delta rule (delta.hip) over long runs, 16 tokens at a time.  With G_t the product of the block's
+// Gated delta rule (delta.hip) over long runs, blocks of 16 tokens, two at a time.  With G_t the product of the block's
 // decays up to token t, per key channel, a block is
 //
 //   A[t, s] = beta_t sum_c k_t k_s G_t / G_s (s < t),   P[t, s] = sum_c q_t k_s G_t / G_s (s <= t)
-//   (1 + A) [U0 | W] = beta [V | G k],   U = U0 - W S,   O = (G q) S + P U
+//   (1 + A) [V0 | W] = beta [V | G k],   U = V0 - W S,   O = (G q) S + P U
 //   S <- G_15 S + sum_s (G_15 / G_s) k_s u_s^T
 //
-// delta_prepare computes everything without S for all blocks at once and leaves it in the order of the
-// matrix operands; ratios of decays are running products of the decays themselves, so nothing is divided
-// and nothing overflows.  delta_blocks walks a head's blocks with S in registers.  All fp32; projections in
-// bfloat16.
+// delta_prepare computes everything without S for all pairs of blocks at once and leaves it in the order of the matrix
+// operands.  delta_blocks walks a head's pairs with S in registers.  All fp32; projections in bfloat16.
 #include "blocks.h"
 
 namespace {
@@ -22,30 +20,73 @@ struct RunArgs {
   Pieces pieces;
 };
 
-// [-W | G q] and the keys as left operands, U0 as a result tile, P's planes, the block's decays; whole KBs
-__host__ __device__ inline constexpr int block_floats(int dk, int dv) {
-  return (kBlock * (3 * dk + dv) + kPairFloats + dk + 255) / 256 * 256;
+// Two blocks after one another are one step of the chain, which splits the state once for both and meets once (a block at a
+// time, 160 heads 3.2 us for 16 tokens, now 2.4): with D the decays of a whole block and S the state before both,
+//
+//   U0 = V0 - W0 S,   U1 = V1 - W1 D0 S - (W1 K0^T) U0,   S <- D1 D0 S + D1 K0^T U0 + K1^T U1
+//   O0 = Q0 S + P0 U0,   O1 = Q1 D0 S + (Q1 K0^T) U0 + P1 U1      (Q: G q, K: keys with the decays behind them)
+//
+// A pair in memory, whole KBs: tiles of [64 lanes][4] of -W0, Q0, -W1 D0, Q1 D0 (16 columns each, left operands) and, by 16
+// rows, of D1 K0 and K1; V0 and V1 as result tiles; planes of P0, P1, -W1 K0^T, Q1 K0^T; D0 D1.
+__host__ __device__ inline constexpr int small_floats(int dk) { return 4 * kPairFloats + dk; }
+__host__ __device__ inline constexpr int pair_floats(int dk, int dv) {
+  return (2 * kBlock * (3 * dk + dv) + small_floats(dk) + 255) / 256 * 256;
 }
+__device__ __forceinline__ int64_t pair_slot(int row0, const Segment& sg, int seg, int b) { return (sg.row - row0) / (2 * kBlock) + seg + b; }
 
+// A pair of blocks: 256 threads each, and the products of the second with the first.  Bound by vector issue (four fifths of its
+// time).  A and P as products of G k and G q with k / G on the matrix cores take less of it than a walk down the tokens that
+// multiplies decays as it goes (160 heads of 2037 tokens at most 271 -> 234 us), which is left for channels that forget more
+// than 1 / G can hold.
+constexpr int kPrepareLd = 132;                // floats of a row: reads across tokens meet no conflicts, offsets are constants
+constexpr int kPrepareHalf = kBlock * 4 * kPrepareLd + 6 * kBlock * kBlock + kBlock + 128 + 4;
+constexpr float kLeastDecay = 0x1p-60f;        // of a channel within a block, for its reciprocal
+// From the bits that each of a row of 16 lanes forgets to the decays up to it: sums over two lanes, their powers, products of
+// these (fewer roundings than products of all, and relative ones).  Eight side by side, as a lane that is moved has to be
+// written two instructions before.
+__device__ __forceinline__ void running_decays(f32x4 (&x)[2]) {
+#ifdef __HIP_DEVICE_COMPILE__
+#define ZP_MOVED(op, i, n) "v_" op "_f32_dpp %" #i ", %" #i ", %" #i " row_shr:" #n " row_mask:0xf bank_mask:0xf\n\t"
+#define ZP_ALL(op, n)                                                                                              \
+  ZP_MOVED(op, 0, n) ZP_MOVED(op, 1, n) ZP_MOVED(op, 2, n) ZP_MOVED(op, 3, n) ZP_MOVED(op, 4, n) ZP_MOVED(op, 5, n) \
+  ZP_MOVED(op, 6, n) ZP_MOVED(op, 7, n)
+#define ZP_EIGHT "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
+  float v[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = x[i >> 2][i & 3];
+  asm volatile("s_nop 1\n\t" ZP_ALL("add", 1) : ZP_EIGHT);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = __builtin_amdgcn_exp2f(-v[i]);
+  asm volatile("s_nop 1\n\t" ZP_ALL("mul", 2) ZP_ALL("mul", 4) ZP_ALL("mul", 8) "s_nop 1" : ZP_EIGHT);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) x[i >> 2][i & 3] = v[i];
+#undef ZP_EIGHT
+#undef ZP_ALL
+#undef ZP_MOVED
+#endif
+}
 template <int TAPS>
-__global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
+__global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
   const zp_delta& a = ra.d;
-  constexpr int ld = 132;                      // every row: reads across tokens meet no conflicts, offsets are constants
+  constexpr int ld = kPrepareLd;
   const int dk = a.dk, dv = a.dv, taps = a.taps;
   const Segment sg = segment_of(a.seg, blockIdx.z);
-  const int t0 = blockIdx.x * kBlock;
-  if (t0 >= sg.count || sg.row < ra.row0) return;
-  const int cnt = min(kBlock, sg.count - t0);
+  const int half = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8), t0 = (2 * blockIdx.x + half) * kBlock;
+  if ((int)blockIdx.x * 2 * kBlock >= sg.count || sg.row < ra.row0) return;
+  const int cnt = max(min(kBlock, sg.count - t0), 0);          // of the second block: maybe none
   const int h = blockIdx.y, hk = h / (a.heads / a.kv_heads);
-  float* const qs = lds;                       // [16][ld], later G q
-  float* const ks = qs + kBlock * ld;
-  float* const gs = ks + kBlock * ld;          // decays, later -W
+  float* const qs = lds + half * kPrepareHalf;                 // [16][ld], later G q
+  float* const ks = qs + kBlock * ld;          // later G k, then -W
+  float* const gs = ks + kBlock * ld;          // bits forgotten, later keys with the decays behind them
   float* const vs = gs + kBlock * ld;
   float* const As = vs + kBlock * ld;          // [16][16]
-  float* const Ps = As + kBlock * kBlock;      // [16][16]
-  float* const beta = Ps + kBlock * kBlock;
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  float* const Ps = As + kBlock * kBlock;      // [16][16]; both over parts of them, [3][2][64][4]
+  float* const beta = As + 6 * kBlock * kBlock;
+  float* const decays = beta + kBlock;         // [dk] of the whole block
+  int* const forgets = (int*)(lds + kPrepareHalf - 4);         // of either block
+  float* const other_decays = decays + (half ? -kPrepareHalf : kPrepareHalf);
+  const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = 2 * dk + dv;
   const char* const tail = (const char*)a.conv_state + ((int64_t)sg.slot * a.heads + h) * (taps - 1) * cw * 2;
   const int channels = 2 * a.kv_heads * dk + a.heads * dv;
@@ -57,20 +98,21 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
   f32x4 z[2], zb[2];
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
-    const int i = tid + u * 256, t = min(i >> piece_bits, cnt - 1), c = (i & ((1 << piece_bits) - 1)) * 4;
-    z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t0 + t) * a.low_stride + h * dk + c);
+    const int i = tid + u * 256, t = min(t0 + (i >> piece_bits), sg.count - 1), c = (i & ((1 << piece_bits) - 1)) * 4;
+    z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t) * a.low_stride + h * dk + c);
     zb[u] = *(const f32x4*)(a.dt_bias + h * dk + c);
   }
   const float b_in = tid < cnt ? Elem<BF16>::ld(a.in, (int64_t)(sg.row + t0 + tid) * a.in_stride + a.b_at + h) : 0.f;
-  const float rate = __expf(a.a_log[h]);
+  const float rate = expf(a.a_log[h]) * 1.44269504088896f;
   // ---- convolutions: a thread's two channels, the block's 16 tokens from a sliding window.  Rows behind the run's end read
   // as zero, and those before its beginning too, unless they come from the history.
   const int row_bytes = (int)a.in_stride * 2;
   const __amdgpu_buffer_rsrc_t rows = __builtin_amdgcn_make_buffer_rsrc(
       (void*)((const char*)a.in + (int64_t)(sg.row + t0) * row_bytes), 0, cnt * row_bytes, 0x00020000);
   const __amdgpu_buffer_rsrc_t before = __builtin_amdgcn_make_buffer_rsrc(
-      (void*)((const char*)a.in + (int64_t)(sg.row + t0 - (TAPS - 1)) * row_bytes), 0, t0 > 0 ? (TAPS - 1) * row_bytes : 0, 0x00020000);
-  if (const int c = 2 * tid; c < cw) {         // at most 384 channels
+      (void*)((const char*)a.in + (int64_t)(sg.row + t0 - (TAPS - 1)) * row_bytes), 0, t0 > 0 && cnt > 0 ? (TAPS - 1) * row_bytes : 0, 0x00020000);
+  // at most 384 channels, which leave a wave of each half without work: not those on one SIMD
+  if (const int c = 2 * ((tid + 64 * (blockIdx.x + 2 * half)) & 255); c < cw) {
     const int at = place(c);
     uint32_t x[kBlock + TAPS - 1];             // two channels' bf16
 #pragma unroll
@@ -112,14 +154,14 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
   for (int u = 0; u < 2; ++u) {
     const int i = tid + u * 256, t = i >> piece_bits, c = (i & ((1 << piece_bits) - 1)) * 4;
     if (t < kBlock) {
-      f32x4 g;
+      f32x4 bits;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) g[e] = t < cnt ? __expf(-rate * fast_softplus(z[u][e] + zb[u][e])) : 1.f;
-      *(f32x4*)(gs + t * ld + c) = g;
+      for (int e = 0; e < 4; ++e) bits[e] = t < cnt ? rate * fast_softplus(z[u][e] + zb[u][e]) : 0.f;
+      *(f32x4*)(gs + t * ld + c) = bits;
     }
   }
   if (tid < kBlock) beta[tid] = tid < cnt ? fast_sigmoid(b_in) : 0.f;
-  if (tid < 2 * kBlock * kBlock / 4) *(f32x4*)(As + tid * 4) = f32x4{0.f, 0.f, 0.f, 0.f};       // and Ps behind it
+  if (threadIdx.x == 0) *forgets = 0;
   __syncthreads();
   // ---- unit vectors: a wave its four tokens, 16 lanes each
   {
@@ -147,62 +189,159 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
     }
   }
   __syncthreads();
-  // ---- A and P: 16 lanes walk k_s down the tokens from s on, in pieces of four channels.  A wave takes four
-  // neighbours, so that it starts at the first of them; which four changes with the block, as the waves' shares differ (all
-  // tokens for every s: 1135 us for 8 prompts of 2048 tokens, 32 heads, with the kernel below, now 1100).
-  {
-    const int first = 4 * ((wave + blockIdx.x) & 3), l16 = lane & 15, s = first + (lane >> 4), pieces = dk / 4;
-    int at[2];
-    f32x4 kk[2];
+  // ---- A and P on the matrix cores, 32 channels a wave: rows G_t k_t and G_t q_t with k_s / G_s
+  const int tiles = dk / 16, waves = dk / 32, row_at = (lane & 15) * ld + wave * 32 + (lane >> 4) * 4;
+  float* const to = ra.ws + (pair_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * pair_floats(dk, dv);
+  float* const oU = to + 6 * kBlock * dk + half * kBlock * dv;
+  float* const oSmall = to + 6 * kBlock * dk + 2 * kBlock * dv;
+  auto put_small = [&](int i, const f32x4& v) {
+    const Planes x(v);
+    *(u32x4*)(oSmall + i * kPairFloats + lane * 4) = u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y};
+    *(uint2*)(oSmall + i * kPairFloats + 256 + lane * 2) = x.lo;
+  };
+  auto split = [](const f32x4 (&v)[2], u32x4 (&o)[3]) {
+    const Planes x(v[0]), y(v[1]);
+    o[0] = u32x4{x.hi.x, x.hi.y, y.hi.x, y.hi.y};
+    o[1] = u32x4{x.mid.x, x.mid.y, y.mid.x, y.mid.y};
+    o[2] = u32x4{x.lo.x, x.lo.y, y.lo.x, y.lo.y};
+  };
+  auto products = [](const u32x4 (&l)[3], const u32x4 (&r)[2][3], f32x4 (&y)[2]) {      // the smallest first
+    y[0] = y[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 2; i >= 0; --i)
+#pragma unroll
+      for (int j = 2 - i; j >= 0; --j)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) y[u] = mfma_bf16(l[i], r[u][j], y[u]);
+  };
+  f32x4 Gq[2], Gk[2], behind[2], y[2];         // behind: keys with the decays behind them
+  if (wave < waves) {
+    f32x4 G[2], over[2];
+    u32x4 left[3], rows2[2][3];
+    float least = 1.f;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      const int pc = l16 + 16 * p;
-      at[p] = min(pc, pieces - 1) * 4;
-      kk[p] = *(const f32x4*)(ks + s * ld + at[p]);
-      if (pc >= pieces) kk[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+      G[p] = *(const f32x4*)(gs + row_at + 16 * p);
+      Gk[p] = *(const f32x4*)(ks + row_at + 16 * p);
+      Gq[p] = *(const f32x4*)(qs + row_at + 16 * p);
     }
-    // Two tokens at a time, four sums over 16 lanes: lanes 8 .. 15 keep those of P, of each eight the upper half the second
-    // token's (eleven additions and choices instead of sixteen additions, one store instead of four).
-    const bool is_p = l16 & 8, second = l16 & 4;
-    float* const to = (is_p ? Ps : As) + s;
-    auto tokens = [&](int t, bool all) {       // all: they lie behind the four
-      float sa[2], sp[2];
+    running_decays(G);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = pa;
+    for (int p = 0; p < 2; ++p) {
 #pragma unroll
-        for (int p = 0; p < 2; ++p) {
-          const f32x4 gt = *(const f32x4*)(gs + (t + u) * ld + at[p]);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) kk[p][e] *= all || t + u > s ? gt[e] : 1.f;
-          pa += kk[p] * *(const f32x4*)(ks + (t + u) * ld + at[p]);
-          pp += kk[p] * *(const f32x4*)(qs + (t + u) * ld + at[p]);
-        }
-        sa[u] = (pa[0] + pa[1]) + (pa[2] + pa[3]);
-        sp[u] = (pp[0] + pp[1]) + (pp[2] + pp[3]);
-        sa[u] += dpp_row_ror<8>(sa[u]);
-        sp[u] += dpp_row_ror<8>(sp[u]);
-        sa[u] = is_p ? sp[u] : sa[u];
-        sa[u] += half_row_mirror(sa[u]);
+      for (int e = 0; e < 4; ++e) {
+        const float whole = dpp_moved<0x15f>(G[p][e]);         // of the row's last lane
+        over[p][e] = Gk[p][e] * __builtin_amdgcn_rcpf(G[p][e]);
+        behind[p][e] = over[p][e] * whole;
+        least = fminf(least, whole);
       }
-      const float x = quad_sum(second ? sa[1] : sa[0]);
-      const int mine = t + second;
-      const float by = is_p ? 1.f : beta[mine];
-      if (all || (is_p ? mine >= s : mine > s)) to[mine * kBlock] = x * by;
-    };
+      Gk[p] *= G[p];
+      Gq[p] *= G[p];
+      if ((lane & 15) == 15) *(f32x4*)(decays + wave * 32 + 16 * p + (lane >> 4) * 4) = G[p];
+    }
+    if (least < kLeastDecay) *forgets = 1;
+    split(over, left);
+    split(Gk, rows2[0]);
+    split(Gq, rows2[1]);
+    products(left, rows2, y);
+    if (wave > 0)
 #pragma unroll
-    for (int u = 0; u < 4; u += 2) tokens(first + u, false);
+      for (int u = 0; u < 2; ++u) *(f32x4*)(As + (((wave - 1) * 2 + u) * 64 + lane) * 4) = y[u];
+  }
+  const int t_row = lane & 15, s_first = lane >> 4 << 2;       // of A and P: row t, from column s on
+  auto rows_to_lds = [&] {
+    if (wave < waves)
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        *(f32x4*)(ks + row_at + 16 * p) = Gk[p];
+        *(f32x4*)(gs + row_at + 16 * p) = behind[p];
+        *(f32x4*)(qs + row_at + 16 * p) = Gq[p];
+      }
+  };
+  __syncthreads();
+  if (!__builtin_amdgcn_readfirstlane(*forgets)) {
+    rows_to_lds();
+    if (wave == 0) {
+      for (int j = 1; j < waves; ++j)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) y[u] += *(const f32x4*)(As + (((j - 1) * 2 + u) * 64 + lane) * 4);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        y[0][r] *= beta[t_row];                                // those of A from t on are not read
+        if (s_first + r > t_row) y[1][r] = 0.f;
+      }
+      *(f32x4*)(As + t_row * kBlock + s_first) = y[0];
+      put_small(half, y[1]);
+    }
+  } else {
+    if (tid < kBlock * kBlock / 4) *(f32x4*)(Ps + tid * 4) = f32x4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+    // 16 lanes walk k_s down the tokens from s on, in pieces of four channels.  A wave takes four neighbours, so that it
+    // starts at the first of them.
+    {
+      const int turn = (wave + blockIdx.x) & 3, first = 4 * (half ? 3 - turn : turn), l16 = lane & 15, s = first + (lane >> 4), pieces = dk / 4;
+      int at[2];
+      f32x4 kk[2];
+#pragma unroll
+      for (int p = 0; p < 2; ++p) {
+        const int pc = l16 + 16 * p;
+        at[p] = min(pc, pieces - 1) * 4;
+        kk[p] = *(const f32x4*)(ks + s * ld + at[p]);
+        if (pc >= pieces) kk[p] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+      // Two tokens at a time, four sums over 16 lanes: lanes 8 .. 15 keep those of P, of each eight the upper half the second
+      // token's (eleven additions and choices instead of sixteen additions, one store instead of four).
+      const bool is_p = l16 & 8, second = l16 & 4;
+      float* const to = (is_p ? Ps : As) + s;
+      auto tokens = [&](int t, bool all) {       // all: they lie behind the four
+        float sa[2], sp[2];
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = pa;
+#pragma unroll
+          for (int p = 0; p < 2; ++p) {
+            const f32x4 gt = *(const f32x4*)(gs + (t + u) * ld + at[p]);      // bits
+#pragma unroll
+            for (int e = 0; e < 4; ++e) kk[p][e] *= all || t + u > s ? __builtin_amdgcn_exp2f(-gt[e]) : 1.f;
+            pa += kk[p] * *(const f32x4*)(ks + (t + u) * ld + at[p]);
+            pp += kk[p] * *(const f32x4*)(qs + (t + u) * ld + at[p]);
+          }
+          sa[u] = (pa[0] + pa[1]) + (pa[2] + pa[3]);
+          sp[u] = (pp[0] + pp[1]) + (pp[2] + pp[3]);
+          sa[u] += dpp_row_ror<8>(sa[u]);
+          sp[u] += dpp_row_ror<8>(sp[u]);
+          sa[u] = is_p ? sp[u] : sa[u];
+          sa[u] += half_row_mirror(sa[u]);
+        }
+        const float x = quad_sum(second ? sa[1] : sa[0]);
+        const int mine = t + second;
+        const float by = is_p ? 1.f : beta[mine];
+        if (all || (is_p ? mine >= s : mine > s)) to[mine * kBlock] = x * by;
+      };
+#pragma unroll
+      for (int u = 0; u < 4; u += 2) tokens(first + u, false);
 #pragma unroll 1
-    for (int t = first + 4; t < kBlock; t += 2) tokens(t, true);
+      for (int t = first + 4; t < kBlock; t += 2) tokens(t, true);
+    }
+    // what is forgotten behind a token lies at the right of its lane
+    if (wave < waves)
+#pragma unroll
+      for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          float R = dpp_moved<0x101>(gs[row_at + 16 * p + e]);     // row_shl:1, zeros behind the last
+          R += dpp_moved<0x101>(R);
+          R += dpp_moved<0x102>(R);
+          R += dpp_moved<0x104>(R);
+          R += dpp_moved<0x108>(R);
+          behind[p][e] = ks[row_at + 16 * p + e] * __builtin_amdgcn_exp2f(-R);
+        }
+    __syncthreads();
+    rows_to_lds();
+    if (wave == 3) put_small(half, *(const f32x4*)(Ps + t_row * kBlock + s_first));
   }
   __syncthreads();
-  // ---- columns: forward substitution, and the block's decays.  A thread reads and writes its own column only.
-  const int64_t base = (block_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * block_floats(dk, dv);
-  float* const oWQ = ra.ws + base;             // [2][dk / 16][64 lanes][4]
-  float* const oK = oWQ + 2 * kBlock * dk;     // [dk / 16][64][4]
-  float* const oU = oK + kBlock * dk;          // [dv / 16][64][4]
-  float* const oP = oU + kBlock * dv;          // [64][hi 4, mid 4], [64][lo 4]
-  float* const oG = oP + kPairFloats;          // [dk]
+  // ---- columns: forward substitution.  A thread reads and writes its own column only.
   float w[kBlock];
   auto substitute = [&](int t, float b) {      // w_t = b - sum_{s < t} A[t, s] w_s
     float x[4] = {b, 0.f, 0.f, 0.f};
@@ -216,47 +355,62 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
     w[t] = (x[0] + x[1]) + (x[2] + x[3]);
     if (t % 2 == 1) __builtin_amdgcn_sched_barrier(0);
   };
-  for (int c = tid; c < dk; c += 256) {
-    float G = 1.f;
+  if (tid < dk + dv) {                         // at most 256
+    const bool key = tid < dk;
+    const int c = key ? tid : tid - dk;
+    const float* const column = (key ? ks : vs) + c;
 #pragma unroll
-    for (int t = 0; t < kBlock; ++t) {
-      G *= gs[t * ld + c];
-      qs[t * ld + c] *= G;
-      substitute(t, beta[t] * ks[t * ld + c] * G);
-    }
-    oG[c] = G;
-    asm volatile("" ::: "memory");            // keys and decays are read again rather than kept
-    float R = 1.f;
+    for (int t = 0; t < kBlock; ++t) substitute(t, beta[t] * column[t * ld]);
+    if (key) {
+      const float D = other_decays[c], by = half ? 1.f : D;
+      if (!half) oSmall[4 * kPairFloats + c] = decays[c] * D;
+      float* const oK = to + (4 * tiles + 2 * (c >> 4) + half) * 256 + (c & 15) * 4;
 #pragma unroll
-    for (int g = 3; g >= 0; --g) {
-      f32x4 x;
+      for (int g = 0; g < 4; ++g) {
+        f32x4 x;
 #pragma unroll
-      for (int r = 3; r >= 0; --r) {
-        const int t = 4 * g + r;
-        x[r] = ks[t * ld + c] * R;
-        R *= gs[t * ld + c];
-        gs[t * ld + c] = -w[t];
+        for (int r = 0; r < 4; ++r) {
+          x[r] = gs[(4 * g + r) * ld + c] * by;
+          ks[(4 * g + r) * ld + c] = -w[4 * g + r];
+        }
+        *(f32x4*)(oK + g * 64) = x;
       }
-      *(f32x4*)(oK + ((c >> 4) * 64 + g * 16 + (c & 15)) * 4) = x;
-      __builtin_amdgcn_sched_barrier(0);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *(f32x4*)(oU + ((c >> 4) * 64 + g * 16 + (c & 15)) * 4) = f32x4{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
     }
-  }
-  for (int v = (tid + 256 - dk) % 256; v < dv; v += 256) {      // on the threads the keys leave free, as far as they go
-#pragma unroll
-    for (int t = 0; t < kBlock; ++t) substitute(t, beta[t] * vs[t * ld + v]);
-#pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *(f32x4*)(oU + ((v >> 4) * 64 + g * 16 + (v & 15)) * 4) = f32x4{w[4 * g], w[4 * g + 1], w[4 * g + 2], w[4 * g + 3]};
-  }
-  if (tid < 64) {
-    const Planes x(*(const f32x4*)(Ps + (tid & 15) * kBlock + (tid >> 4) * 4));
-    *(u32x4*)(oP + tid * 4) = u32x4{x.hi.x, x.hi.y, x.mid.x, x.mid.y};
-    *(uint2*)(oP + 256 + tid * 2) = x.lo;
   }
   __syncthreads();
-  for (int i = tid; i < 2 * kBlock * dk / 4; i += 256) {       // lane (g, row) of tile kt: columns 16 kt + 4 g ..
-    const int tile = i >> 6, l = i & 63, kt = tile & (dk / 16 - 1);
-    *(f32x4*)(oWQ + i * 4) = *(const f32x4*)((tile < dk / 16 ? gs : qs) + (l & 15) * ld + kt * 16 + (l >> 4) * 4);
+  // ---- -W and G q, as left operands hold them; the second block's with the first one's keys, transposed like these
+  float* const part = lds + kPrepareHalf + 3 * kBlock * ld;    // over the second block's values: [dk / 32][2][64][4]
+  if (wave < waves) {
+    f32x4 W[2], Q[2], K[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      W[p] = *(const f32x4*)(ks + row_at + 16 * p);
+      Q[p] = *(const f32x4*)(qs + row_at + 16 * p);
+      K[p] = *(const f32x4*)(lds + 2 * kBlock * ld + row_at + 16 * p);
+      const f32x4 D = *(const f32x4*)(other_decays + wave * 32 + 16 * p + (lane >> 4) * 4);
+      float* const o = to + (2 * half * tiles + 2 * wave + p) * 256 + lane * 4;
+      *(f32x4*)o = half ? W[p] * D : W[p];
+      *(f32x4*)(o + tiles * 256) = half ? Q[p] * D : Q[p];
+    }
+    if (half) {
+      u32x4 left[3], rows2[2][3];
+      split(K, left);
+      split(W, rows2[0]);
+      split(Q, rows2[1]);
+      products(left, rows2, y);
+#pragma unroll
+      for (int u = 0; u < 2; ++u) *(f32x4*)(part + ((wave * 2 + u) * 64 + lane) * 4) = y[u];
+    }
+  }
+  __syncthreads();
+  if (half && wave < 2) {
+    f32x4 x = *(const f32x4*)(part + (wave * 64 + lane) * 4);
+    for (int j = 1; j < waves; ++j) x += *(const f32x4*)(part + ((j * 2 + wave) * 64 + lane) * 4);
+    put_small(2 + wave, x);
   }
 }
 
@@ -267,7 +421,7 @@ __global__ __launch_bounds__(256, 4) void delta_prepare_kernel(RunArgs ra) {
 __host__ __device__ inline constexpr int piece_floats(int dk) { return 2 * dk * dk; }
 
 // From sums to the states before the pieces, in place; a wave 16 columns.  The products are those of the blocks, M split by
-// all waves together while the piece before is worked on: 2.4 us a piece.
+// all waves together while the piece before is worked on: 5.7 us a piece.
 template <int KT>
 __global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float planes[];              // [rows / 16][pairs of columns / 16][3][64 lanes][4]
@@ -345,29 +499,34 @@ __global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
   }
 }
 
-// A head's blocks, one after the other, a wave 16 columns of the state.  On the fp32 matrix cores the products would be the
-// bound (208 of 32 cycles a block on each SIMD, which keep its vector units idle as well), so operands are split into
-// three bf16 planes: the products that count take a quarter of that, beside the vector units.  The state is split
-// where it is updated, what comes from memory by all waves together, a block ahead and under the products with the state;
-// rows are normed and stored behind the next meeting of the waves, which the norm needs too.  What bounds it now is a wave's
-// chain of work: two per SIMD are all there are (twice the columns per wave, one per SIMD: 2 to 12 % more time in all).
-// 8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1161 -> 1106 us, one of them 566 -> 491; error of the
-// state against 64 bits 4.0e-7 -> 3.6e-7 of its size.
+// A head's pairs of blocks, one after the other, a wave 16 columns of the state.  On the fp32 matrix cores the products would be
+// the bound, so operands are split into three bf16 planes: the products that count take a quarter of that, beside the vector
+// units.  The state is split where it is updated; what comes from memory passes through registers, asked for a pair ahead, and
+// is split into LDS by all waves together under the products with the state; rows are normed and stored in the next pair.
+// What bounds it: of 11 300 cycles a pair and SIMD the products take 5100, vector issue 6200 beside them, LDS 4300, and the
+// younger of its two waves the rest.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1033 -> 936 us, 5 of
+// 1640 to 2037 717 -> 621, one 256 -> 227; 7 of 625 to 1499 with 16 heads 415 -> 355; error of the state against 64 bits 3.3e-7 ->
+// 3.0e-7 of its size.
 // SUMS: no state comes in and no rows go out; every second workgroup takes what the piece keeps, where values are none.
+template <int KT, int NW> struct PairStage {
+  static constexpr int kTiles = 6 * KT, kPlanes = kTiles * 384, kSmall = small_floats(16 * KT);      // floats in LDS
+  static constexpr int kMine = (kTiles + NW - 1) / NW, kRing = kMine <= 6 ? kMine : kMine % 6 == 0 ? 6 : kMine % 4 == 0 ? 4 : 3;      // a wave's tiles; asked for ahead
+  static constexpr int kPieces = (kSmall / 4 + 64 * NW - 1) / (64 * NW);     // a thread's 16 bytes of the small ones
+  static constexpr int kBytes = (2 * kPlanes + 2 * kSmall + 4 * NW * kBlock) * 4;
+  static_assert(kMine % kRing == 0, "places of the ring are constants");
+};
 template <int KT, int NW, bool SUMS>
 __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
+  typedef PairStage<KT, NW> Stage;
   const zp_delta& a = ra.d;
-  constexpr int dk = 16 * KT, dv = 16 * NW, size = block_floats(dk, dv), J = KT / 2;
-  constexpr int kSplit = 3 * kBlock * dk, kRest = size - kSplit;      // floats of a block: operands to be split, the others
-  constexpr int kP = kBlock * dv, kG = kP + kPairFloats;              // in the rest, behind U0
-  constexpr int kPlanes = 3 * KT * 384, kMine = ((SUMS ? 2 : 3) * KT + NW - 1) / NW;    // floats of a block's planes; tiles of a wave
+  constexpr int dk = 16 * KT, dv = 16 * NW, size = pair_floats(dk, dv), J = KT / 2;
+  constexpr int kMine = Stage::kMine, kRing = Stage::kRing, kPlanes = Stage::kPlanes, kSmall = Stage::kSmall, kPieces = Stage::kPieces;
   const int tid = threadIdx.x, lane = tid & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  float* const split = lds;                    // [2][kSplit]
-  float* const rest = split + 2 * kSplit;      // [3][kRest]
-  float* const planes = rest + 3 * kRest;      // [2][kPlanes]
-  float* const red = planes + 2 * kPlanes;     // [2][NW * 16]
+  float* const planes = lds;                   // [2][pairs of tiles][3][64 lanes][4]
+  float* const small = planes + 2 * kPlanes;   // [2][kSmall]
+  float* const red = small + 2 * kSmall;       // [2][2][NW * 16]
   const bool keeps = SUMS && blockIdx.x & 1;
   const int id = SUMS ? blockIdx.x >> 1 : blockIdx.x, most = ra.pieces.most - SUMS, unit = id / most, h = unit % a.heads, seg = unit / a.heads;
   const Segment whole = segment_of(a.seg, seg);
@@ -391,44 +550,51 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     load_state<KT, 1>(S, state, dv, col0, sg.start == 0);
   }
   const float nrm = a.norm[h * dv + col0 + l16] * a.out_scale;
-  const float* const base = ra.ws + (block_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
+  const float* const base = ra.ws + (pair_slot(ra.row0, sg, seg, 0) * a.heads + h) * size;
   const int64_t stride = (int64_t)a.heads * size;
-  const int blocks = (sg.count + kBlock - 1) / kBlock;
-  auto tile_at = [](int i) { return SUMS && i >= KT ? i + KT : i; };      // without those of G q
-  auto request = [&](int b) {                  // a block behind the last: nothing is read
-    const StageLoads from(base + b * stride, b < blocks ? size * 4 : 0);
-    constexpr int kKBs = size / 256 - (SUMS ? KT : 0);
-#pragma unroll
-    for (int u = 0; u < (kKBs + NW - 1) / NW; ++u) {
-      const int i = tile_at(min(wave + u * NW, kKBs - 1));         // the last may come twice
-      float* const to = i < kSplit / 256 ? split + (b & 1) * kSplit + i * 256 : rest + b % 3 * kRest + (i * 256 - kSplit);
-      from.ld(to, lane * 16, i * 1024);
-    }
-  };
-  // Planes of a block's tiles: for pairs of those of -W and of G q [3][64 lanes][two tiles' 4], for those of keys
-  // [64][hi 4, mid 4], [64][lo 4].  A wave's tile u; the last may be made twice.
-  auto tile_of = [&](int b, int u) {
-    return *(const f32x4*)(split + (b & 1) * kSplit + tile_at(min(wave + u * NW, (SUMS ? 2 : 3) * KT - 1)) * 256 + lane * 4);
-  };
-  auto put_planes = [&](int b, int u, const f32x4& x) {
-    const int i = tile_at(min(wave + u * NW, (SUMS ? 2 : 3) * KT - 1));
-    const int key = i >= 2 * KT;               // multiplied, not branched on: the products beside stay in one stretch
-    float* const to = planes + (b & 1) * kPlanes + (i >> 1) * 768 + (i & 1) * (2 + 382 * key) + lane * 4;
-    const Planes p(x);
+  const int pairs = (sg.count + 2 * kBlock - 1) / (2 * kBlock);
+  auto at_pair = [&](int b) { return base + min(b, pairs - 1) * stride; };     // behind the last: it again, and nobody looks
+  // A wave's tile u of a pair: on its way through registers, then its planes in LDS.  The last may come twice.
+  auto tile_index = [&](int u) { return min(wave + u * NW, Stage::kTiles - 1); };
+  f32x4 raw[kRing], rest[kPieces], values[2];
+  auto ask = [&](int b, int u) { raw[u % kRing] = *(const f32x4*)(at_pair(b) + tile_index(u) * 256 + lane * 4); };
+  auto put = [&](int b, int u) {
+    const int i = tile_index(u);
+    float* const to = planes + (b & 1) * kPlanes + (i >> 1) * 768 + (i & 1) * 2 + lane * 4;
+    const Planes p(raw[u % kRing]);
     *(uint2*)to = p.hi;
-    *(uint2*)(to + 256 - 254 * key) = p.mid;
-    *(uint2*)(to + 512 - (256 + lane * 2) * key) = p.lo;
+    *(uint2*)(to + 256) = p.mid;
+    *(uint2*)(to + 512) = p.lo;
   };
-  f32x4 done = {0.f, 0.f, 0.f, 0.f};
-  uint16_t gate[4] = {0, 0, 0, 0};
+  auto next_tile = [&](int b, int u) {         // put tile u of pair b, ask for the one kRing further
+    put(b, u);
+    if (u + kRing < kMine) ask(b, u + kRing);
+    else ask(b + 1, u + kRing - kMine);
+  };
+  auto ask_values = [&](int b) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) values[i] = *(const f32x4*)(at_pair(b) + 6 * kBlock * dk + i * kBlock * dv + wave * 256 + lane * 4);
+  };
+  auto ask_rest = [&](int b) {
+    const float* const p = at_pair(b) + 2 * kBlock * (3 * dk + dv);
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) rest[u] = *(const f32x4*)(p + min(tid + u * 64 * NW, kSmall / 4 - 1) * 4);
+  };
+  auto put_rest = [&](int b) {
+#pragma unroll
+    for (int u = 0; u < kPieces; ++u) *(f32x4*)(small + (b & 1) * kSmall + min(tid + u * 64 * NW, kSmall / 4 - 1) * 4) = rest[u];
+  };
+  f32x4 done[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+  uint16_t gate[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   const float inv_v = 1.f / (float)a.vdim;
   const int out_at = (4 * g * (int)a.out_stride + h * dv + col0 + l16) * 2;
   const int low_at = (4 * g * (int)a.low_stride + a.g_at + h * dv + col0 + l16) * 2;
-  auto finish = [&](int b, int r, const f32x4& ss) {               // row r of block b, whose squares are ss; none of block -1
-    const int cnt = b < 0 ? 0 : min(kBlock, sg.count - b * kBlock);
-    const BlockRows out(a.out, sg.row + b * kBlock, cnt, a.out_stride);
-    const float rs = __builtin_amdgcn_rsqf(ss[r] * inv_v + a.eps);
-    out.st(out_at + r * (int)a.out_stride * 2, 0, done[r] * rs * nrm * fast_sigmoid(bf16_bits_to_float(gate[r])));
+  auto rows_of = [&](int b) { return b < 0 ? 0 : min(2 * kBlock, sg.count - b * 2 * kBlock); };
+  auto finish = [&](int b, int r, const f32x4& ss) {               // row 16 (r / 4) + 4 g + r % 4 of pair b; none of pair -1
+    const BlockRows out(a.out, sg.row + b * 2 * kBlock, rows_of(b), a.out_stride);
+    const float rs = __builtin_amdgcn_rsqf(ss[r & 3] * inv_v + a.eps);
+    out.st(out_at + (r / 4 * kBlock + (r & 3)) * (int)a.out_stride * 2, 0,
+           done[r / 4][r & 3] * rs * nrm * fast_sigmoid(bf16_bits_to_float(gate[r])));
   };
   u32x4 sp[3][J];                              // the state's planes, pairs of tiles
   auto split_state = [&](int kt) {
@@ -438,113 +604,157 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     sp[1][kt >> 1][at] = x.mid.x, sp[1][kt >> 1][at + 1] = x.mid.y;
     sp[2][kt >> 1][at] = x.lo.x, sp[2][kt >> 1][at + 1] = x.lo.y;
   };
-  request(0);
-  __builtin_amdgcn_s_waitcnt(0);               // the state is there: the loop's first use of it must not wait in every pass
+  auto meet = [] {                             // LDS alone: what comes from memory and goes there stays on its way
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
 #pragma unroll
-  for (int kt = 0; kt < KT; ++kt) split_state(kt);
-  wait_and_meet();
-  request(1);
+  for (int u = 0; u < kRing; ++u) ask(0, u);
+  ask_rest(0);
+  ask_values(0);
 #pragma unroll
-  for (int u = 0; u < kMine; ++u) put_planes(0, u, tile_of(0, u));
+  for (int kt = 0; kt < (J > 1 ? KT - 2 : KT); ++kt) split_state(kt);      // the last two beside the first products
+#pragma unroll
+  for (int u = 0; u < kMine; ++u) next_tile(0, u);
+  put_rest(0);
+  ask_rest(1);
 #pragma unroll 1
-  for (int b = 0; b < blocks; ++b) {
-    wait_and_meet();
-    const float* const mine = rest + b % 3 * kRest;
+  for (int b = 0; b < pairs; ++b) {
+    meet();
+    const float* const mine = small + (b & 1) * kSmall;
     const float* const pl = planes + (b & 1) * kPlanes + lane * 4;
     u32x4 W[2][3], Q[2][3];
-    auto operands = [&](int j) {
+    auto operands = [&](int n) {
 #pragma unroll
       for (int i = 0; i < 3; ++i) {
-        W[j & 1][i] = *(const u32x4*)(pl + (j * 3 + i) * 256);
-        if constexpr (!SUMS) Q[j & 1][i] = *(const u32x4*)(pl + ((J + j) * 3 + i) * 256);
+        W[n & 1][i] = *(const u32x4*)(pl + ((n / J * 2 * J + n % J) * 3 + i) * 256);
+        if constexpr (!SUMS) Q[n & 1][i] = *(const u32x4*)(pl + (((n / J * 2 + 1) * J + n % J) * 3 + i) * 256);
       }
     };
     operands(0);
-    f32x4 U = *(const f32x4*)(mine + wave * 256 + lane * 4), O = {0.f, 0.f, 0.f, 0.f};
-    if (keeps) U = f32x4{0.f, 0.f, 0.f, 0.f};
-    f32x4 tile = tile_of(b + 1, 0), ss;
-    if constexpr (!SUMS) ss = block_squares_total<NW>(red + ((b - 1) & 1) * NW * kBlock);
-    request(b + 2);
-    const int cnt = min(kBlock, sg.count - b * kBlock);
-    const BlockRows low(a.low, sg.row + b * kBlock, cnt, a.low_stride);
-    uint16_t next[4];
+    f32x4 U[2] = {values[0], values[1]}, O[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+    if (keeps) U[0] = U[1] = f32x4{0.f, 0.f, 0.f, 0.f};
+    ask_values(b + 1);
+    f32x4 ss;
+    const BlockRows low(a.low, sg.row + b * 2 * kBlock, rows_of(b), a.low_stride);
+    uint16_t next[8];
     if constexpr (!SUMS)
 #pragma unroll
-    for (int r = 0; r < 4; ++r) next[r] = low.ld(low_at + r * (int)a.low_stride * 2, 0);
+      for (int r = 0; r < 8; ++r) next[r] = low.ld(low_at + (r / 4 * kBlock + (r & 3)) * (int)a.low_stride * 2, 0);
     __builtin_amdgcn_sched_barrier(0);
-    u32x4 K[2][2];
-    uint2 Kl[2][2];
+    u32x4 left[2], up[3], u0[4], K[2][2][3];   // up: planes of U0 and U1, one contraction of 32
+    uint2 left_lo[2];
     f32x4 dec[2][2];
+    auto small_operands = [&](int i, int k) {
+      left[0] = *(const u32x4*)(mine + i * kPairFloats + lane * 4);
+      left_lo[0] = *(const uint2*)(mine + i * kPairFloats + 256 + lane * 2);
+      left[1] = *(const u32x4*)(mine + k * kPairFloats + lane * 4);
+      left_lo[1] = *(const uint2*)(mine + k * kPairFloats + 256 + lane * 2);
+    };
     auto keys = [&](int j) {
 #pragma unroll
       for (int i = 0; i < 2; ++i) {
-        const float* const at = planes + (b & 1) * kPlanes + (2 * KT + 2 * j + i) * 384;
-        K[j & 1][i] = *(const u32x4*)(at + lane * 4);
-        Kl[j & 1][i] = *(const uint2*)(at + 256 + lane * 2);
-        dec[j & 1][i] = *(const f32x4*)(mine + kG + 16 * (2 * j + i) + 4 * g);
+#pragma unroll
+        for (int k = 0; k < 3; ++k) K[j & 1][i][k] = *(const u32x4*)(pl + ((4 * J + 2 * j + i) * 3 + k) * 256);
+        dec[j & 1][i] = *(const f32x4*)(mine + 4 * kPairFloats + 16 * (2 * j + i) + 4 * g);
       }
     };
+    // What follows from U0: its planes, the second block's U and O.  Within the second half where that is long enough.
+    auto split_first = [&] {
+      const PlanePairs u(U[0]);
+      u0[0] = u.hh, u0[1] = u.mm, u0[2] = u.ll, u0[3] = u.hm;
+      up[0][0] = u.hh[0], up[0][1] = u.hh[1], up[1][0] = u.mm[0], up[1][1] = u.mm[1], up[2][0] = u.ll[0], up[2][1] = u.ll[1];
+    };
+    auto cross = [&] {
+      const PlanePairs u(u0);
+      if constexpr (SUMS) u.add(left[0], left_lo[0], U[1]);
+      else u.add(left, left_lo, U[1], O[1]);
+    };
+    constexpr bool kLate = J < 4;
 #pragma unroll
-    for (int j = 0; j < J; ++j) {              // beside: the block before is finished, the next one's planes are made
-      if (j + 1 < J) operands(j + 1);
+    for (int n = 0; n < 2 * J; ++n) {          // beside: the pair before is finished, the next one's planes are made
+      const int half = n / J;
+      if (n + 1 < 2 * J) operands(n + 1);
       else keys(0);
+      if constexpr (!SUMS)
+        if (n % J == 0) ss = block_squares_total<NW>(red + (((b - 1) & 1) * 2 + half) * NW * kBlock);
+      if (!kLate && n == J + 1) small_operands(2, 3);
 #pragma unroll
       for (int i = 2; i >= 0; --i)             // the smallest products first
 #pragma unroll
         for (int k = 2 - i; k >= 0; --k) {
-          U = mfma_bf16(W[j & 1][i], sp[k][j], U);
-          if constexpr (!SUMS) O = mfma_bf16(Q[j & 1][i], sp[k][j], O);
+          U[half] = mfma_bf16(W[n & 1][i], sp[k][n % J], U[half]);
+          if constexpr (!SUMS) O[half] = mfma_bf16(Q[n & 1][i], sp[k][n % J], O[half]);
         }
+      if (J > 1 && n == 0) {
+        split_state(KT - 2);
+        split_state(KT - 1);
+      }
       if constexpr (!SUMS)
 #pragma unroll
-        for (int r = j * 4 / J; r < (j + 1) * 4 / J; ++r) finish(b - 1, r, ss);
+        for (int r = n * 8 / (2 * J); r < (n + 1) * 8 / (2 * J); ++r) finish(b - 1, r, ss);
 #pragma unroll
-      for (int u = j * kMine / J; u < (j + 1) * kMine / J; ++u) {
-        put_planes(b + 1, u, tile);
-        if (u + 1 < kMine) tile = tile_of(b + 1, u + 1);
-      }
+      for (int u = n * kMine / (2 * J); u < (n + 1) * kMine / (2 * J); ++u) next_tile(b + 1, u);
+      if (!kLate && n == J) split_first();
+      if (!kLate && n == J + 2) cross();
       spread_over_products<SUMS ? 6 : 12, 4>();
     }
-    u32x4 P;
-    uint2 Pl;
+    if constexpr (kLate) {
+      small_operands(2, 3);
+      split_first();
+      cross();
+    }
+    put_rest(b + 1);
+    ask_rest(b + 2);
     if constexpr (!SUMS) {
 #pragma unroll
-      for (int r = 0; r < 4; ++r) gate[r] = next[r];
-      P = *(const u32x4*)(mine + kP + lane * 4);
-      Pl = *(const uint2*)(mine + kP + 256 + lane * 2);
+      for (int r = 0; r < 8; ++r) gate[r] = next[r];
+      small_operands(0, 1);
     }
-    const PlanePairs u(U);
-    __builtin_amdgcn_sched_barrier(0);
     S[0][0] *= dec[0][0];
     S[1][0] *= dec[0][1];
+    const PlanePairs u1(U[1]);
+    up[0][2] = u1.hh[0], up[0][3] = u1.hh[1], up[1][2] = u1.mm[0], up[1][3] = u1.mm[1], up[2][2] = u1.ll[0], up[2][3] = u1.ll[1];
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int j = 0; j < J; ++j) {              // beside: two tiles before are split, the next two decay
+    for (int j = 0; j < J; ++j) {              // beside: two tiles before are split, the next two decay, rows are squared
       if (j + 1 < J) {
         keys(j + 1);
         S[2 * j + 2][0] *= dec[(j + 1) & 1][0];
         S[2 * j + 3][0] *= dec[(j + 1) & 1][1];
       }
-      u.add(K[j & 1], Kl[j & 1], S[2 * j][0], S[2 * j + 1][0]);
+      if constexpr (!SUMS)
+        if (j == 0) {
+          PlanePairs(u0).add(left[0], left_lo[0], O[0]);
+          u1.add(left[1], left_lo[1], O[1]);
+        }
+#pragma unroll
+      for (int i = 2; i >= 0; --i)
+#pragma unroll
+        for (int k = 2 - i; k >= 0; --k)
+#pragma unroll
+          for (int t = 0; t < 2; ++t) S[2 * j + t][0] = mfma_bf16(K[j & 1][t][i], up[k], S[2 * j + t][0]);
       if (j > 0) {
         split_state(2 * j - 2);
         split_state(2 * j - 1);
       }
-      spread_over_products<8, 5>();
+      if constexpr (!SUMS)
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          if (j == min(i + 1, J - 1)) {
+            f32x4 o[1] = {O[i]};
+            block_squares<1>(o, red + ((b & 1) * 2 + i) * NW * kBlock, wave);
+            done[i] = O[i];
+          }
+      spread_over_products<12, 4>();
     }
-    if constexpr (!SUMS) u.add(P, Pl, O);
-    split_state(KT - 2);
-    split_state(KT - 1);
-#pragma unroll
-    for (int i = 0; i < 3; ++i)                // here, not behind the squares
-#pragma unroll
-      for (int j = 0; j < J; ++j) settle(sp[i][j]);
-    if constexpr (!SUMS) {
-      f32x4 o[1] = {O};
-      block_squares<1>(o, red + (b & 1) * NW * kBlock, wave);
-      done = O;
+    if constexpr (J == 1) {
+      split_state(KT - 2);
+      split_state(KT - 1);
     }
   }
-  wait_and_meet();
+  meet();
   if constexpr (SUMS) {
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
@@ -558,9 +768,12 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     }
     return;
   }
-  const f32x4 ss = block_squares_total<NW>(red + ((blocks - 1) & 1) * NW * kBlock);
 #pragma unroll
-  for (int r = 0; r < 4; ++r) finish(blocks - 1, r, ss);
+  for (int i = 0; i < 2; ++i) {
+    const f32x4 ss = block_squares_total<NW>(red + (((pairs - 1) & 1) * 2 + i) * NW * kBlock);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) finish(pairs - 1, 4 * i + r, ss);
+  }
   if (!piece.last) return;
   store_state<KT, 1>(S, state, dv, col0);
   // the last inputs of the head's convolutions (runs are longer than a filter)
@@ -583,8 +796,7 @@ template <typename F> int launch_kernel(F* kernel, int64_t groups, int threads, 
   return ZP_OK;
 }
 template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
-  constexpr int kSplit = 3 * kBlock * 16 * KT;
-  constexpr int smem = (3 * block_floats(16 * KT, 16 * NW) - kSplit + 2 * 3 * KT * 384 + 2 * NW * kBlock) * 4;
+  constexpr int smem = PairStage<KT, NW>::kBytes;
   const int64_t units = (int64_t)ra.d.seg.n * ra.d.heads;
   if constexpr (KT == NW)
     if (ra.pieces.blocks) {
@@ -605,14 +817,14 @@ template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
 
 template <int TAPS> int launch_prepare(const RunArgs& ra, int longest, hipStream_t st) {
   const zp_delta& a = ra.d;
-  const size_t smem = sizeof(float) * (kBlock * 4 * 132 + 2 * kBlock * kBlock + kBlock);
+  const size_t smem = sizeof(float) * 2 * kPrepareHalf;
   if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)delta_prepare_kernel<TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)smem) != hipSuccess) {
     zp_set_error("delta_runs: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((delta_prepare_kernel<TAPS>), dim3((unsigned)((longest + kBlock - 1) / kBlock), (unsigned)a.heads, (unsigned)a.seg.n),
-                     dim3(256), smem, st, ra);
+  hipLaunchKernelGGL((delta_prepare_kernel<TAPS>), dim3((unsigned)((longest + 2 * kBlock - 1) / (2 * kBlock)), (unsigned)a.heads, (unsigned)a.seg.n),
+                     dim3(512), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
 }
@@ -630,16 +842,16 @@ int launch_runs(const RunArgs& ra, int longest, hipStream_t st) {
 
 }  // namespace
 
-static int64_t blocks_bytes(int64_t rows, int64_t segments, int64_t heads, int dk, int dv) {
-  return (rows / kBlock + segments) * heads * block_floats(dk, dv) * 4;
+static int64_t pairs_bytes(int64_t rows, int64_t segments, int64_t heads, int dk, int dv) {
+  return (rows / (2 * kBlock) + segments) * heads * pair_floats(dk, dv) * 4;
 }
 
-constexpr PieceCost kCost = {2, 8, 60, 10};
+constexpr PieceCost kCost = {2, 8, 72, 24};
 
 // With room for the states between pieces of few heads' runs, whatever the longest run.
 extern "C" int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk, int32_t dv) {
   if (rows < 0 || segments < 0 || heads <= 0 || dk <= 0 || dv <= 0) return -1;
-  return blocks_bytes(rows, segments, heads, dk, dv) +
+  return pairs_bytes(rows, segments, heads, dk, dv) +
          (dk == dv && dk <= 128 ? most_states(rows, segments, heads, kCost) * piece_floats(dk) * 4 : 0);
 }
 
@@ -661,10 +873,10 @@ extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t lo
                  a.seg.rows && a.seg.counts && a.seg.slots && a.seg.starts && aligned16(a.state) && aligned16(a.in) && aligned16(a.low) &&
                  aligned16(a.dt_bias) && aligned16(workspace),
              "delta_runs: null or unaligned pointer");
-  const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk, a.dv);
+  const int64_t rows = a.seg.num_rows - first_row, whole = pairs_bytes(rows, a.seg.n, a.heads, a.dk, a.dv);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "delta_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, first_row, {}};
-  if (a.dk == a.dv) ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk));
+  if (a.dk == a.dv) ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, 2, (workspace_bytes - whole) / 4 / piece_floats(a.dk));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   return launch_runs(ra, longest, (hipStream_t)stream);

@@ -482,7 +482,7 @@ extern "C" int zp_linear_runs(const zp_linear* args, int32_t first_row, int32_t 
   const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads, a.dk);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "linear_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, first_row, {}};
-  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
+  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, 1, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   hipStream_t st = (hipStream_t)stream;

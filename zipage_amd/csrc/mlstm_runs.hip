@@ -516,7 +516,7 @@ extern "C" int zp_mlstm_runs(const zp_mlstm* args, int32_t first_row, int32_t lo
   const int64_t rows = a.seg.num_rows - first_row, whole = blocks_bytes(rows, a.seg.n, a.heads);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "mlstm_runs: workspace too small");
   RunArgs ra = {a, (float*)workspace, nullptr, first_row, {}};
-  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
+  ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, 1, (workspace_bytes - whole) / 4 / piece_floats(a.dk, a.dv));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.scal = (float4*)(ra.aux + ((int64_t)(a.seg.num_rows - first_row) / kBlock + a.seg.n) * a.heads * kAux);
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
