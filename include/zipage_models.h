@@ -268,6 +268,14 @@ int zp_delta_scan(const zp_delta* args, int32_t dtype, void* stream);
 int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32_t heads, int32_t dk, int32_t dv);
 int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
                   int64_t workspace_bytes, int32_t dtype, void* stream);
+/* The same with the rows of `low`, which is not read, made on the way: the products, rounded to bfloat16, of the `rank` columns
+ * of `in` from low_at on with low_weights (heads * (dk + dv), rank) bfloat16, whose first heads * dk rows, those of the
+ * decays, are zero from column a_rank on and the others, the gates', before it.  They lie as [rows / 16][columns / 32][4 pieces of 8
+ * columns][16 rows], zeros behind `rank`.  low_at, a_rank and rank multiples of 8; a_rank and what the gates read, from a_rank
+ * / 32 * 32 on, up to 128 columns. */
+int zp_delta_runs_projected(const zp_delta* args, const void* low_weights, int32_t low_at, int32_t a_rank, int32_t rank,
+                            int32_t first_row, int32_t longest, void* workspace, int64_t workspace_bytes, int32_t dtype,
+                            void* stream);
 
 /* ------------------------------------------------------------------ libzipage_linear.so */
 

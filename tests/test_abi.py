@@ -162,3 +162,13 @@ def test_structures_are_as_long_as_the_headers(tmp_path):
     out = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split("\n")
     for n, line in zip(records, out):
         assert [int(v) for v in line.split()] == [ctypes.sizeof(here[n]), getattr(here[n], last(here[n])).offset], n
+
+
+def test_delta_products_of_other_ranks_are_refused():
+    from zipage_amd import _lib
+    lib = _lib.load_models("recurrent")
+    args = _lib.DeltaArgs(in_stride=4096)
+    call = lambda at, a_rank, rank: lib.zp_delta_runs_projected(ctypes.byref(args), ctypes.c_void_p(16), at, a_rank, rank, 0, 16, None, 0, 0, None)
+    for at, a_rank, rank in ((4, 8, 16), (8, 8, 20), (0, 136, 144), (0, 16, 144), (0, 128, 264)):
+        assert call(at, a_rank, rank) == 3, (at, a_rank, rank)             # ZP_EUNSUPPORTED
+    assert call(4000, 64, 128) == 1 and call(0, 16, 8) == 1 and call(-8, 8, 16) == 1

@@ -715,19 +715,22 @@ def _run_segments(dev, counts):
 
 
 # Blocks of 16 tokens go in pairs: one block, a second one of one token to all, a third; channels that forget little, some that
-# leave the range of a reciprocal within a block, and all of them.
+# leave the range of a reciprocal within a block, and all of them.  Low-rank products of ranks that share a step of 32 columns, that
+# fill the most that the kernels make, and that are left to the library.
 @pytest.mark.parametrize("bias,spread", [(-3.0, 1.0), (-2.0, 6.0), (12.0, 1.0)])
-@pytest.mark.parametrize("H,G,D,V,taps", [(2, 1, 128, 128, 4), (3, 3, 64, 64, 2), (2, 1, 32, 96, 8), (1, 1, 128, 32, 1), (2, 2, 64, 128, 3)])
-def test_delta_runs_in_pairs_of_blocks(dev, H, G, D, V, taps, bias, spread):
+@pytest.mark.parametrize("H,G,D,V,taps,ranks", [(2, 1, 128, 128, 4, (128, 128)), (3, 3, 64, 64, 2, (40, 72)), (2, 1, 32, 96, 8, (8, 8)),
+                                                (1, 1, 128, 32, 1, (136, 8)), (2, 2, 64, 128, 3, (100, 16))])
+def test_delta_runs_in_pairs_of_blocks(dev, H, G, D, V, taps, ranks, bias, spread):
     import types
     from zipage_amd.engine.qwen3 import Segments
     from zipage_amd.layers import ChannelDelta
     counts, W = [1, 15, 16, 17, 31, 32, 33, 48, 49, 64, 65, 97], 64
     m, n, rows = ChannelDelta(W, H, G, D, V, taps, 1e-3), len(counts), sum(counts)
-    shapes = m.shapes(8, 8)
+    shapes = m.shapes(*ranks)
     w = {k: _rand(*s, seed=i) * s[-1] ** -0.5 for i, (k, s) in enumerate(shapes.items())}
     w["dt_bias"] = (bias + spread * _rand(H * D, seed=52).float()).to(BF16)
     into, _ = m.load(w, BF16, dev, W)
+    assert (m.low_tiles is None) == (max(ranks) > 128)
     proj = (_rand(rows, W, seed=60).to(dev).float() @ into.to(dev).float().T).to(BF16)
     t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
     seg = Segments(t([sum(counts[:i]) for i in range(n)]), t(counts), t(list(range(n, 0, -1))),

@@ -187,6 +187,7 @@ MODEL_LIBS = {
         "zp_mlstm_runs": [C.POINTER(MlstmArgs), i32, i32, ptr, i64, i32, ptr],
         "zp_delta_scan": [C.POINTER(DeltaArgs), i32, ptr],
         "zp_delta_runs": [C.POINTER(DeltaArgs), i32, i32, ptr, i64, i32, ptr],
+        "zp_delta_runs_projected": [C.POINTER(DeltaArgs), ptr, i32, i32, i32, i32, i32, ptr, i64, i32, ptr],
     }, {"zp_mlstm_runs_workspace": [i32, i32, i32], "zp_delta_runs_workspace": [i32, i32, i32, i32, i32]}),
     "linear": ({
         "zp_linear_scan": [C.POINTER(LinearArgs), i32, ptr],

@@ -115,7 +115,7 @@ PyMethodDef entries[] = {
     ZP_ENTRY(zp_latent_norm_store), ZP_ENTRY(zp_rotate_heads), ZP_ENTRY(zp_headwise_linear), ZP_ENTRY(zp_latent_rows_workspace),
     ZP_ENTRY(zp_latent_rows_attention), ZP_ENTRY(zp_rotary_store), ZP_ENTRY(zp_grouped_rows_workspace),
     ZP_ENTRY(zp_grouped_rows_attention), ZP_ENTRY(zp_mlstm_scan), ZP_ENTRY(zp_mlstm_runs_workspace), ZP_ENTRY(zp_mlstm_runs),
-    ZP_ENTRY(zp_delta_scan), ZP_ENTRY(zp_delta_runs_workspace), ZP_ENTRY(zp_delta_runs), ZP_ENTRY(zp_linear_scan),
+    ZP_ENTRY(zp_delta_scan), ZP_ENTRY(zp_delta_runs_workspace), ZP_ENTRY(zp_delta_runs), ZP_ENTRY(zp_delta_runs_projected), ZP_ENTRY(zp_linear_scan),
     ZP_ENTRY(zp_linear_runs_workspace), ZP_ENTRY(zp_linear_runs), ZP_ENTRY(zp_small_linear), ZP_ENTRY(zp_moe_select),
     ZP_ENTRY(zp_moe_tile_rows), ZP_ENTRY(zp_moe_max_tiles), ZP_ENTRY(zp_moe_plan_workspace), ZP_ENTRY(zp_moe_plan),
     ZP_ENTRY(zp_moe_gate_up), ZP_ENTRY(zp_moe_down),

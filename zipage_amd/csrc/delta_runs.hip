@@ -18,7 +18,12 @@ struct RunArgs {
   float* ws;
   int row0;      // first token row of the first segment
   Pieces pieces;
+  // PROJECTED: the decays' and the gates' pre-activations are products made here, of `rank` columns of a.in from low_at on, the
+  // first a_rank of them for the decays, with rows (heads * (dk + dv), rank) as [rows / 16][columns / 32][64 lanes][8]
+  const uint16_t* low_weights;
+  int low_at, rank, a_rank;
 };
+constexpr int kLowSteps = 4, kLowRank = 256;   // of 32 columns for either product; columns in all
 
 // Two blocks after one another are one step of the chain, which splits the state once for both and meets once (a block at a
 // time, 160 heads 3.2 us for 16 tokens, now 2.4): with D the decays of a whole block and S the state before both,
@@ -27,11 +32,13 @@ struct RunArgs {
 //   O0 = Q0 S + P0 U0,   O1 = Q1 D0 S + (Q1 K0^T) U0 + P1 U1      (Q: G q, K: keys with the decays behind them)
 //
 // A pair in memory, whole KBs: tiles of [64 lanes][4] of -W0, Q0, -W1 D0, Q1 D0 (16 columns each, left operands) and, by 16
-// rows, of D1 K0 and K1; V0 and V1 as result tiles; planes of P0, P1, -W1 K0^T, Q1 K0^T; D0 D1.
+// rows, of D1 K0 and K1; V0 and V1 as result tiles; planes of P0, P1, -W1 K0^T, Q1 K0^T; D0 D1; the gates' pre-activations
+// as result tiles in bfloat16.
 __host__ __device__ inline constexpr int small_floats(int dk) { return 4 * kPairFloats + dk; }
 __host__ __device__ inline constexpr int pair_floats(int dk, int dv) {
-  return (2 * kBlock * (3 * dk + dv) + small_floats(dk) + 255) / 256 * 256;
+  return (2 * kBlock * (3 * dk + dv) + small_floats(dk) + kBlock * dv + 255) / 256 * 256;
 }
+__host__ __device__ inline constexpr int gates_at(int dk, int dv) { return 2 * kBlock * (3 * dk + dv) + small_floats(dk); }
 __device__ __forceinline__ int64_t pair_slot(int row0, const Segment& sg, int seg, int b) { return (sg.row - row0) / (2 * kBlock) + seg + b; }
 
 // A pair of blocks: 256 threads each, and the products of the second with the first.  Bound by vector issue (four fifths of its
@@ -65,7 +72,7 @@ __device__ __forceinline__ void running_decays(f32x4 (&x)[2]) {
 #undef ZP_MOVED
 #endif
 }
-template <int TAPS>
+template <int TAPS, bool PROJECTED>
 __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float lds[];
   const zp_delta& a = ra.d;
@@ -93,14 +100,48 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   auto place = [&](int c) -> int {
     return c < dk ? hk * dk + c : (c < 2 * dk ? a.kv_heads * dk + hk * dk + c - dk : 2 * a.kv_heads * dk + h * dv + c - 2 * dk);
   };
-  // ---- requests first: the decays' pre-activations (two pieces a thread at most), the step sizes'
+  const int tiles = dk / 16, wave8 = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), l16 = lane & 15, g4 = lane >> 4;
+  float* const to = ra.ws + (pair_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * pair_floats(dk, dv);
+  // ---- requests first: the decays' pre-activations (two pieces a thread at most), the step sizes'; or what they are products of
   const int piece_bits = 31 - __builtin_clz(dk / 4);           // pieces of four channels: 8, 16 or 32 a row
   f32x4 z[2], zb[2];
+  u32x4 low[2], wa[kLowSteps], wg[kLowSteps];
+  const int g_step = ra.a_rank >> 5;                           // the gates' first step; they share it with the decays where that ends inside
+  if constexpr (PROJECTED) {
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
-    const int i = tid + u * 256, t = min(t0 + (i >> piece_bits), sg.count - 1), c = (i & ((1 << piece_bits) - 1)) * 4;
-    z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t) * a.low_stride + h * dk + c);
-    zb[u] = *(const f32x4*)(a.dt_bias + h * dk + c);
+    for (int u = 0; u < 2; ++u) {                              // rows of up to 32 pieces of 16 bytes
+      const int i = tid + u * 256, t = min(t0 + (i >> 5), sg.count - 1), c = (i & 31) * 8;
+      low[u] = u32x4{0u, 0u, 0u, 0u};
+      if (c < ra.rank) low[u] = *(const u32x4*)((const uint16_t*)a.in + (int64_t)(sg.row + t) * a.in_stride + ra.low_at + c);
+    }
+    const int steps = (ra.rank + 31) >> 5;
+    auto weights = [&](int tile, int step, bool there) {
+      u32x4 v = {0u, 0u, 0u, 0u};
+      if (there && step < steps) v = *(const u32x4*)(ra.low_weights + ((int64_t)tile * steps + step) * 512 + lane * 8);
+      return v;
+    };
+#pragma unroll
+    for (int i = 0; i < kLowSteps; ++i) {
+      wa[i] = weights(h * tiles + wave8, i, wave8 < tiles && i * 32 < ra.a_rank);
+      wg[i] = weights(a.heads * tiles + h * (dv / 16) + wave8, g_step + i, wave8 < dv / 16);
+    }
+  } else {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int i = tid + u * 256, t = min(t0 + (i >> piece_bits), sg.count - 1), c = (i & ((1 << piece_bits) - 1)) * 4;
+      z[u] = load4<BF16>(a.low, (int64_t)(sg.row + t) * a.low_stride + h * dk + c);
+      zb[u] = *(const f32x4*)(a.dt_bias + h * dk + c);
+    }
+    if (wave8 < dv / 16)
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const int first = (2 * blockIdx.x + k) * kBlock;
+        const BlockRows rows(a.low, sg.row + first, min(max(sg.count - first, 0), kBlock), a.low_stride);
+        uint32_t v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = rows.ld((4 * g4 + r) * (int)a.low_stride * 2 + (a.g_at + h * dv + wave8 * 16 + l16) * 2, 0);
+        *(uint2*)(to + gates_at(dk, dv) + ((k * (dv / 16) + wave8) * 64 + lane) * 2) = uint2{v[0] | v[1] << 16, v[2] | v[3] << 16};
+      }
   }
   const float b_in = tid < cnt ? Elem<BF16>::ld(a.in, (int64_t)(sg.row + t0 + tid) * a.in_stride + a.b_at + h) : 0.f;
   const float rate = expf(a.a_log[h]) * 1.44269504088896f;
@@ -112,16 +153,17 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   const __amdgpu_buffer_rsrc_t before = __builtin_amdgcn_make_buffer_rsrc(
       (void*)((const char*)a.in + (int64_t)(sg.row + t0 - (TAPS - 1)) * row_bytes), 0, t0 > 0 && cnt > 0 ? (TAPS - 1) * row_bytes : 0, 0x00020000);
   // at most 384 channels, which leave a wave of each half without work: not those on one SIMD
-  if (const int c = 2 * ((tid + 64 * (blockIdx.x + 2 * half)) & 255); c < cw) {
+  const int c = 2 * ((tid + 64 * (blockIdx.x + 2 * half)) & 255);
+  uint32_t x[kBlock + TAPS - 1];               // two channels' bf16
+  float f[2][TAPS];                            // f[.][j]: j tokens back
+  if (c < cw) {
     const int at = place(c);
-    uint32_t x[kBlock + TAPS - 1];             // two channels' bf16
 #pragma unroll
     for (int i = 0; i < kBlock + TAPS - 1; ++i)
       x[i] = (uint32_t)(i < TAPS - 1 ? __builtin_amdgcn_raw_buffer_load_b32(before, at * 2, i * row_bytes, 0)
                                      : __builtin_amdgcn_raw_buffer_load_b32(rows, at * 2, (i - (TAPS - 1)) * row_bytes, 0));
-    float f[2][TAPS];
 #pragma unroll
-    for (int j = 0; j < TAPS; ++j)                            // f[.][j]: j tokens back
+    for (int j = 0; j < TAPS; ++j)
 #pragma unroll
       for (int e = 0; e < 2; ++e) f[e][j] = a.filters[(int64_t)max(taps - 1 - j, 0) * channels + at + e];
 #pragma unroll
@@ -133,6 +175,38 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
       for (int i = 0; i < TAPS - 1; ++i)
         if (i >= TAPS - taps) x[i] = *(const uint32_t*)(tail + ((int64_t)(taps - TAPS + i) * cw + c) * 2);
     }
+  }
+  if constexpr (PROJECTED) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) *(u32x4*)((char*)qs + ((tid + u * 256) >> 5) * ld * 4 + (tid & 31) * 16) = low[u];
+    __syncthreads();
+    // A wave 16 channels of decays and 16 of gates, of both blocks.  The library's product of rows that are half zeros takes as
+    // long as this does in all for many tokens and a launch more (8 prompts of 2048 tokens, 32 heads 936 -> 917 us, 2 of about 1250
+    // 261 -> 240, one of 110, 16 heads 42.3 -> 38.7); weights row by row, which touch twice as many lines, 944.
+    const f32x4 bias = wave8 < tiles ? *(const f32x4*)(a.dt_bias + h * dk + wave8 * 16 + g4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const char* const rows = (const char*)(lds + k * kPrepareHalf) + l16 * ld * 4 + g4 * 16;
+      f32x4 x = {0.f, 0.f, 0.f, 0.f}, y = x;
+#pragma unroll
+      for (int i = 0; i < kLowSteps; ++i) {
+        x = mfma_bf16(wa[i], *(const u32x4*)(rows + i * 64), x);
+        y = mfma_bf16(*(const u32x4*)(rows + (g_step + i) * 64), wg[i], y);
+      }
+      if (wave8 < dv / 16)
+        *(uint2*)(to + gates_at(dk, dv) + ((k * (dv / 16) + wave8) * 64 + lane) * 2) = uint2{pack_bf16(y[0], y[1]), pack_bf16(y[2], y[3])};
+      if (wave8 < tiles) {
+        const uint32_t lo = pack_bf16(x[0], x[1]), hi = pack_bf16(x[2], x[3]);     // as rows `low` would hold them
+        x = f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)} + bias;
+        const bool there = (2 * (int)blockIdx.x + k) * kBlock + l16 < sg.count;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) x[e] = there ? rate * fast_softplus(x[e]) : 0.f;
+        *(f32x4*)(lds + k * kPrepareHalf + 2 * kBlock * ld + l16 * ld + wave8 * 16 + g4 * 4) = x;
+      }
+    }
+    __syncthreads();                           // the rows are used up
+  }
+  if (c < cw) {
     float* const dst = c < dk ? qs + c : (c < 2 * dk ? ks + c - dk : vs + c - 2 * dk);
 #pragma unroll
     for (int t = 0; t < kBlock; ++t) {
@@ -150,6 +224,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     }
     for (int t = cnt; t < kBlock; ++t) *(float2*)(dst + t * ld) = float2{0.f, 0.f};
   }
+  if constexpr (!PROJECTED)
 #pragma unroll
   for (int u = 0; u < 2; ++u) {
     const int i = tid + u * 256, t = i >> piece_bits, c = (i & ((1 << piece_bits) - 1)) * 4;
@@ -165,7 +240,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   __syncthreads();
   // ---- unit vectors: a wave its four tokens, 16 lanes each
   {
-    const int t = wave * 4 + (lane >> 4), l16 = lane & 15, pieces = dk / 4;
+    const int t = wave * 4 + (lane >> 4), pieces = dk / 4;
     f32x4 q[2], k[2], q2 = {0.f, 0.f, 0.f, 0.f}, k2 = q2;
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -190,8 +265,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   }
   __syncthreads();
   // ---- A and P on the matrix cores, 32 channels a wave: rows G_t k_t and G_t q_t with k_s / G_s
-  const int tiles = dk / 16, waves = dk / 32, row_at = (lane & 15) * ld + wave * 32 + (lane >> 4) * 4;
-  float* const to = ra.ws + (pair_slot(ra.row0, sg, blockIdx.z, blockIdx.x) * a.heads + h) * pair_floats(dk, dv);
+  const int waves = dk / 32, row_at = (lane & 15) * ld + wave * 32 + (lane >> 4) * 4;
   float* const oU = to + 6 * kBlock * dk + half * kBlock * dv;
   float* const oSmall = to + 6 * kBlock * dk + 2 * kBlock * dv;
   auto put_small = [&](int i, const f32x4& v) {
@@ -279,7 +353,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     // 16 lanes walk k_s down the tokens from s on, in pieces of four channels.  A wave takes four neighbours, so that it
     // starts at the first of them.
     {
-      const int turn = (wave + blockIdx.x) & 3, first = 4 * (half ? 3 - turn : turn), l16 = lane & 15, s = first + (lane >> 4), pieces = dk / 4;
+      const int turn = (wave + blockIdx.x) & 3, first = 4 * (half ? 3 - turn : turn), s = first + (lane >> 4), pieces = dk / 4;
       int at[2];
       f32x4 kk[2];
 #pragma unroll
@@ -504,8 +578,8 @@ __global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
 // units.  The state is split where it is updated; what comes from memory passes through registers, asked for a pair ahead, and
 // is split into LDS by all waves together under the products with the state; rows are normed and stored in the next pair.
 // What bounds it: of 11 300 cycles a pair and SIMD the products take 5100, vector issue 6200 beside them, LDS 4300, and the
-// younger of its two waves the rest.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1033 -> 936 us, 5 of
-// 1640 to 2037 717 -> 621, one 256 -> 227; 7 of 625 to 1499 with 16 heads 415 -> 355; error of the state against 64 bits 3.3e-7 ->
+// younger of its two waves the rest.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1033 -> 917 us, 5 of
+// 1640 to 2037 717 -> 598, one 256 -> 214; 7 of 625 to 1499 with 16 heads 415 -> 344; error of the state against 64 bits 3.3e-7 ->
 // 3.0e-7 of its size.
 // SUMS: no state comes in and no rows go out; every second workgroup takes what the piece keeps, where values are none.
 template <int KT, int NW> struct PairStage {
@@ -585,16 +659,16 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     for (int u = 0; u < kPieces; ++u) *(f32x4*)(small + (b & 1) * kSmall + min(tid + u * 64 * NW, kSmall / 4 - 1) * 4) = rest[u];
   };
   f32x4 done[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  uint16_t gate[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+  uint2 gate[2] = {{0, 0}, {0, 0}};
   const float inv_v = 1.f / (float)a.vdim;
   const int out_at = (4 * g * (int)a.out_stride + h * dv + col0 + l16) * 2;
-  const int low_at = (4 * g * (int)a.low_stride + a.g_at + h * dv + col0 + l16) * 2;
   auto rows_of = [&](int b) { return b < 0 ? 0 : min(2 * kBlock, sg.count - b * 2 * kBlock); };
   auto finish = [&](int b, int r, const f32x4& ss) {               // row 16 (r / 4) + 4 g + r % 4 of pair b; none of pair -1
     const BlockRows out(a.out, sg.row + b * 2 * kBlock, rows_of(b), a.out_stride);
     const float rs = __builtin_amdgcn_rsqf(ss[r & 3] * inv_v + a.eps);
+    const uint32_t two = r & 2 ? gate[r / 4].y : gate[r / 4].x;
     out.st(out_at + (r / 4 * kBlock + (r & 3)) * (int)a.out_stride * 2, 0,
-           done[r / 4][r & 3] * rs * nrm * fast_sigmoid(bf16_bits_to_float(gate[r])));
+           done[r / 4][r & 3] * rs * nrm * fast_sigmoid(__uint_as_float(r & 1 ? two & 0xffff0000u : two << 16)));
   };
   u32x4 sp[3][J];                              // the state's planes, pairs of tiles
   auto split_state = [&](int kt) {
@@ -637,11 +711,10 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     if (keeps) U[0] = U[1] = f32x4{0.f, 0.f, 0.f, 0.f};
     ask_values(b + 1);
     f32x4 ss;
-    const BlockRows low(a.low, sg.row + b * 2 * kBlock, rows_of(b), a.low_stride);
-    uint16_t next[8];
+    uint2 next[2];
     if constexpr (!SUMS)
 #pragma unroll
-      for (int r = 0; r < 8; ++r) next[r] = low.ld(low_at + (r / 4 * kBlock + (r & 3)) * (int)a.low_stride * 2, 0);
+      for (int i = 0; i < 2; ++i) next[i] = *(const uint2*)(at_pair(b) + gates_at(dk, dv) + ((i * NW + wave) * 64 + lane) * 2);
     __builtin_amdgcn_sched_barrier(0);
     u32x4 left[2], up[3], u0[4], K[2][2][3];   // up: planes of U0 and U1, one contraction of 32
     uint2 left_lo[2];
@@ -709,7 +782,7 @@ __global__ __launch_bounds__(64 * NW, 2) void delta_blocks_kernel(RunArgs ra) {
     ask_rest(b + 2);
     if constexpr (!SUMS) {
 #pragma unroll
-      for (int r = 0; r < 8; ++r) gate[r] = next[r];
+      for (int i = 0; i < 2; ++i) gate[i] = next[i];
       small_operands(0, 1);
     }
     S[0][0] *= dec[0][0];
@@ -815,15 +888,15 @@ template <int KT> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   }
 }
 
-template <int TAPS> int launch_prepare(const RunArgs& ra, int longest, hipStream_t st) {
+template <int TAPS, bool PROJECTED> int launch_prepare(const RunArgs& ra, int longest, hipStream_t st) {
   const zp_delta& a = ra.d;
   const size_t smem = sizeof(float) * 2 * kPrepareHalf;
-  if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)delta_prepare_kernel<TAPS>, hipFuncAttributeMaxDynamicSharedMemorySize,
+  if (smem > 60 * 1024 && hipFuncSetAttribute((const void*)delta_prepare_kernel<TAPS, PROJECTED>, hipFuncAttributeMaxDynamicSharedMemorySize,
                                               (int)smem) != hipSuccess) {
     zp_set_error("delta_runs: cannot reserve %zu bytes of LDS", smem);
     return ZP_EHIP;
   }
-  hipLaunchKernelGGL((delta_prepare_kernel<TAPS>), dim3((unsigned)((longest + 2 * kBlock - 1) / (2 * kBlock)), (unsigned)a.heads, (unsigned)a.seg.n),
+  hipLaunchKernelGGL((delta_prepare_kernel<TAPS, PROJECTED>), dim3((unsigned)((longest + 2 * kBlock - 1) / (2 * kBlock)), (unsigned)a.heads, (unsigned)a.seg.n),
                      dim3(512), smem, st, ra);
   ZP_LAUNCH_CHECK();
   return ZP_OK;
@@ -831,7 +904,8 @@ template <int TAPS> int launch_prepare(const RunArgs& ra, int longest, hipStream
 
 int launch_runs(const RunArgs& ra, int longest, hipStream_t st) {
   const zp_delta& a = ra.d;
-  const int rc = a.taps <= 4 ? launch_prepare<4>(ra, longest, st) : launch_prepare<kMaxTaps>(ra, longest, st);
+  const int rc = ra.low_weights ? (a.taps <= 4 ? launch_prepare<4, true>(ra, longest, st) : launch_prepare<kMaxTaps, true>(ra, longest, st))
+                                : (a.taps <= 4 ? launch_prepare<4, false>(ra, longest, st) : launch_prepare<kMaxTaps, false>(ra, longest, st));
   if (rc != ZP_OK) return rc;
   switch (a.dk) {
     case 32: return launch_blocks<2>(ra, st);
@@ -855,29 +929,47 @@ extern "C" int64_t zp_delta_runs_workspace(int32_t rows, int32_t segments, int32
          (dk == dv && dk <= 128 ? most_states(rows, segments, heads, kCost) * piece_floats(dk) * 4 : 0);
 }
 
-extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
-                             int64_t workspace_bytes, int32_t dtype, void* stream) {
+static int delta_runs(const zp_delta* args, const void* low_weights, int low_at, int a_rank, int rank, int first_row, int longest,
+                      void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
   ZP_REQUIRE(args, "delta_runs: null arguments");
   const zp_delta& a = *args;
   ZP_REQUIRE(a.seg.n >= 0 && a.heads > 0 && a.kv_heads > 0 && a.heads % a.kv_heads == 0 && a.vdim > 0 && a.vdim <= a.dv &&
                  a.seg.num_slots > 0 && a.out_stride >= (int64_t)a.heads * a.dv && first_row >= 0 && longest >= 0 &&
                  first_row <= a.seg.num_rows, "delta_runs: bad dims");
   if (dtype != ZP_BF16 || (a.dk != 32 && a.dk != 64 && a.dk != 128) || a.dv % 32 || a.dv > 128 || a.taps < 1 || a.taps > kMaxTaps || a.heads > 65535 ||
-      a.seg.n > 65535 || a.in_stride % 8 || a.low_stride % 8 || a.out_stride >= (1 << 24) || a.low_stride >= (1 << 24)) {
+      a.seg.n > 65535 || a.in_stride % 8 || a.out_stride >= (1 << 24) || (!low_weights && (a.low_stride % 8 || a.low_stride >= (1 << 24)))) {
     zp_set_error("delta_runs: bfloat16, head sizes %d (32, 64, 128) and %d (a multiple of 32, <= 128), %d taps (1 .. %d) unsupported",
                  a.dk, a.dv, a.taps, kMaxTaps);
     return ZP_EUNSUPPORTED;
   }
   if (a.seg.n == 0 || longest == 0) return ZP_OK;
-  ZP_REQUIRE(a.in && a.low && a.filters && a.a_log && a.dt_bias && a.norm && a.state && (a.conv_state || a.taps == 1) && a.out &&
-                 a.seg.rows && a.seg.counts && a.seg.slots && a.seg.starts && aligned16(a.state) && aligned16(a.in) && aligned16(a.low) &&
+  ZP_REQUIRE(a.in && (a.low || low_weights) && a.filters && a.a_log && a.dt_bias && a.norm && a.state && (a.conv_state || a.taps == 1) && a.out &&
+                 a.seg.rows && a.seg.counts && a.seg.slots && a.seg.starts && aligned16(a.state) && aligned16(a.in) && (low_weights ? aligned16(low_weights) : aligned16(a.low)) &&
                  aligned16(a.dt_bias) && aligned16(workspace),
              "delta_runs: null or unaligned pointer");
   const int64_t rows = a.seg.num_rows - first_row, whole = pairs_bytes(rows, a.seg.n, a.heads, a.dk, a.dv);
   ZP_REQUIRE(workspace && workspace_bytes >= whole, "delta_runs: workspace too small");
-  RunArgs ra = {a, (float*)workspace, first_row, {}};
+  RunArgs ra = {a, (float*)workspace, first_row, {}, (const uint16_t*)low_weights, low_at, rank, a_rank};
   if (a.dk == a.dv) ra.pieces = pieces_of(rows, a.seg.n, a.heads, longest, kCost, 2, (workspace_bytes - whole) / 4 / piece_floats(a.dk));
   ra.pieces.states = (float*)workspace + whole / 4;
   ra.d.seg.max_count = longest;               // no segment has more blocks than were prepared
   return launch_runs(ra, longest, (hipStream_t)stream);
+}
+
+extern "C" int zp_delta_runs(const zp_delta* args, int32_t first_row, int32_t longest, void* workspace,
+                             int64_t workspace_bytes, int32_t dtype, void* stream) {
+  return delta_runs(args, nullptr, 0, 0, 0, first_row, longest, workspace, workspace_bytes, dtype, stream);
+}
+
+extern "C" int zp_delta_runs_projected(const zp_delta* args, const void* low_weights, int32_t low_at, int32_t a_rank, int32_t rank,
+                                       int32_t first_row, int32_t longest, void* workspace, int64_t workspace_bytes, int32_t dtype,
+                                       void* stream) {
+  ZP_REQUIRE(args && low_weights && low_at >= 0 && a_rank >= 0 && rank >= a_rank && low_at + (int64_t)rank <= args->in_stride,
+             "delta_runs: bad low-rank products");
+  if (low_at % 8 || rank % 8 || rank > kLowRank || (a_rank + 31) / 32 > kLowSteps || (rank + 31) / 32 - a_rank / 32 > kLowSteps) {
+    zp_set_error("delta_runs: low-rank products of %d and %d columns from column %d on unsupported (multiples of 8, up to 128)", a_rank,
+                 rank - a_rank, low_at);
+    return ZP_EUNSUPPORTED;
+  }
+  return delta_runs(args, low_weights, low_at, a_rank, rank, first_row, longest, workspace, workspace_bytes, dtype, stream);
 }

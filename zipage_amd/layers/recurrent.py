@@ -7,8 +7,8 @@ import torch
 
 from zipage_amd import _lib
 
-from .linear import fit, pad_to_multiple, step_product
-from .moe import small_linear
+from .linear import _seen_by_others, fit, pad_to_multiple, step_product
+from .moe import small_linear, tile_order
 from .rotary import Rotary
 
 
@@ -136,12 +136,16 @@ class ChannelDelta:
         ra_p, rg_p = pad_to_multiple(ra, 8), pad_to_multiple(rg, 8)
         self.b_at = self.channels
         self.low_at = self.b_at + pad_to_multiple(H, 8)
-        self.low_rank = ra_p + rg_p
+        self.a_rank, self.low_rank = ra_p, ra_p + rg_p
         self.columns = self.low_at + self.low_rank
         low = torch.zeros(H * (Dp + Vp), self.low_rank, dtype=w["a2"].dtype)
         low[:H * Dp, :ra] = fit(w["a2"].view(H, D, ra), H, Dp, ra).flatten(0, 1)
         low[H * Dp:, ra_p:ra_p + rg] = fit(w["g2"].view(H, V, rg), H, Vp, rg).flatten(0, 1)
         self.low = low.to(device=device, dtype=dtype).contiguous()
+        # once more in the order that the blocked kernels read, where they make these products themselves
+        self.low_tiles = None
+        if dtype == torch.bfloat16 and self.can_run and self.low_rank <= 256 and max(ra_p, self.low_rank - ra_p // 32 * 32) <= 128:
+            self.low_tiles = tile_order(fit(self.low, len(self.low), pad_to_multiple(self.low_rank, 32)))
         into = torch.cat([rows(w["q"], G, D, Dp), rows(w["k"], G, D, Dp), rows(w["v"], H, V, Vp),
                           fit(w["b"], pad_to_multiple(H, 8), padded_width), fit(w["a1"], ra_p, padded_width),
                           fit(w["g1"], rg_p, padded_width)])
@@ -164,15 +168,20 @@ class ChannelDelta:
         S, tail = state
         H, D = self.heads, self.dim_p
         assert proj.stride(1) == out.stride(1) == 1 and proj.dtype == out.dtype == tail.dtype and S.is_contiguous()
-        low = step_product(ctx)(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
+        blocks = self.can_run and proj.dtype == torch.bfloat16
+        # runs by the blocked kernels make the low-rank products on their way, where nothing else looks at them
+        projected = ctx.run_segments is not None and blocks and self.low_tiles is not None and self.low_tiles.device == proj.device and \
+            not _seen_by_others(proj, self.low)
+        low = None if projected and ctx.segments is None else \
+            step_product(ctx)(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
         tag, stream = _lib.dtype_tag(proj), _lib.stream_ptr(proj)
-        for segments, runs in ((ctx.segments, False), (ctx.run_segments, self.can_run and proj.dtype == torch.bfloat16)):
+        for segments, runs in ((ctx.segments, False), (ctx.run_segments, blocks)):
             if segments is None:
                 continue
             args = _lib.DeltaArgs(
                 _segments(segments, S.shape[0], proj.shape[0]), _lib.dev_ptr(proj), _lib.dev_ptr(low),
                 _lib.dev_ptr(self.filters), _lib.dev_ptr(self.a_log), _lib.dev_ptr(self.dt_bias), _lib.dev_ptr(self.norm),
-                _lib.dev_ptr(S), _lib.dev_ptr(tail), _lib.dev_ptr(out), proj.stride(0), low.stride(0), out.stride(0), H,
+                _lib.dev_ptr(S), _lib.dev_ptr(tail), _lib.dev_ptr(out), proj.stride(0), 0 if low is None else low.stride(0), out.stride(0), H,
                 self.kv_heads, D, self.vdim_p, self.vdim, self.taps, self.b_at, H * D, self.dim ** -0.5, self.eps,
                 self.out_scale)
             if not runs:
@@ -180,8 +189,11 @@ class ChannelDelta:
                 continue
             size = _lib.load_models("recurrent").zp_delta_runs_workspace(proj.shape[0] - segments.first_row, segments.counts.numel(), H, D, self.vdim_p)
             ws = torch.empty(size, dtype=torch.uint8, device=proj.device)
-            _lib.call_models("zp_delta_runs", args, segments.first_row, segments.longest,
-                             _lib.dev_ptr(ws), size, tag, stream)
+            if projected:
+                _lib.call_models("zp_delta_runs_projected", args, _lib.dev_ptr(self.low_tiles), self.low_at, self.a_rank, self.low_rank,
+                                 segments.first_row, segments.longest, _lib.dev_ptr(ws), size, tag, stream)
+            else:
+                _lib.call_models("zp_delta_runs", args, segments.first_row, segments.longest, _lib.dev_ptr(ws), size, tag, stream)
 
 
 class LinearAttention:
