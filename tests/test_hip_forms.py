@@ -1015,3 +1015,31 @@ def test_prompts_keep_the_librarys_products(dev, few_rows_calls, tmp_path, model
         assert not few_rows_calls(), [len(t) for _, t, _ in step]
     eng.feed([(a, toks[30:31], []), (b, toks[20:21], [])])
     assert few_rows_calls()
+
+
+# ------------------------------------------------------------------ redundancy over all pairs, 16 bit
+# Pages of one or two tiles of 128 keys are their own first tiles, larger ones read their rows apart and take several rounds; pages
+# that are no whole tiles take the general form.  Rows of a multiple of eight share an XCD; few pages go in parts.  Chains of 16, 8,
+# 24, 32 and 12 chunks a page, whose ends fall anywhere among the 32 that are taken at a time.
+@pytest.mark.parametrize("dtype,BS,D,Hkv,pages,thr", [
+    (BF16, 256, 128, 3, (5, 2), 0.5), (BF16, 256, 64, 8, (4, 1), 0.5), (torch.float16, 128, 128, 4, (7, 3), 0.3), (BF16, 384, 96, 1, (3,), 0.5),
+    (torch.float16, 512, 32, 2, (2, 3), 0.9), (BF16, 192, 128, 2, (3, 5), 0.5), (BF16, 256, 128, 8, (4, 3) * 8, 0.5), (BF16, 128, 128, 8, (9,) * 6, 0.5),
+    (BF16, 256, 128, 8, (4, 3) * 8, 0.0)])
+def test_all_pairs_forms(dev, dtype, BS, D, Hkv, pages, thr):
+    from tests.test_redundancy_planted import _clear_of_norm_boundaries, _close_in_ulps
+    from zipage_amd.kernel import raw_redudancy_score
+    g = torch.Generator().manual_seed(BS + D)
+    order = torch.randperm(sum(pages), generator=g).tolist()
+    tables = [[order.pop() for _ in range(n)] for n in pages]
+    enc = O.encode_block_table(tables)
+    k = torch.randn((1, sum(pages), BS, Hkv, D), generator=g)
+    for t in tables:                                 # a quarter of a sequence's keys are another one's direction, some of them longer
+        rows = k[0, t].reshape(-1, Hkv, D)
+        n = rows.shape[0] // 4
+        to, src = torch.randperm(rows.shape[0], generator=g)[:n], torch.randint(rows.shape[0], (n,), generator=g)
+        rows[to] = rows[src] * torch.where(torch.rand(n, 1, 1, generator=g) < 0.2, 4.0, 1.0)
+        k[0, t] = rows.view(len(t), BS, Hkv, D)
+    k = _clear_of_norm_boundaries(k.to(dtype))
+    want, scale = O.raw_redudancy_logits(k, enc, thr, return_partial_max=True)
+    got, _ = raw_redudancy_score(k.to(dev), enc.to(dev), threshold=thr, temperature=0.4, return_logits=True)
+    _close_in_ulps(got, want, dtype, ulps=1, frac_exact=0.95, chain_scale=scale)

@@ -29,13 +29,13 @@ PAGE_PHASES = ["row set-up (first page only), claim slots cleared",
                "barrier",
                "store"]
 CHAIN_PHASES = ["table lookup, page list, key loads",
-                "claims of the round gathered",
                 "first planes",
-                "corrections cleared (all tiles)",
-                "corrections added",
-                "products and epilogue",
-                "next planes stored, serial chain",
-                "barrier behind the chain"]
+                "barrier: planes and corrections",
+                "products, corrections taken off",
+                "barrier behind the products",
+                "next planes and corrections stored",
+                "serial chain",
+                "(none)"]
 
 
 def main():

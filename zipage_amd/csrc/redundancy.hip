@@ -1213,6 +1213,16 @@ template <> struct Split3<BF16> {
     o[1] = (uint16_t)(__float_as_uint(m) >> 16);
     o[2] = (uint16_t)(__float_as_uint(l) >> 16);
   }
+  // two floats, their pieces side by side
+  __device__ static __forceinline__ void two(float x, float y, uint32_t* o) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const zp_f32x2 v = {x, y};
+      o[i] = __builtin_bit_cast(uint32_t, __builtin_convertvector(v, zp_bf16x2));
+      x -= __uint_as_float(o[i] << 16);
+      y -= __uint_as_float(o[i] & 0xffff0000u);
+    }
+  }
 };
 template <> struct Split3<F16> {
   __device__ static __forceinline__ void run(float v, uint16_t* o) {
@@ -1220,6 +1230,13 @@ template <> struct Split3<F16> {
     const float r1 = v - f16_bits_to_float(o[0]);
     o[1] = float_to_f16_bits(r1);
     o[2] = float_to_f16_bits(r1 - f16_bits_to_float(o[1]));
+  }
+  __device__ static __forceinline__ void two(float x, float y, uint32_t* o) {
+    uint16_t a[3], b[3];
+    run(x, a);
+    run(y, b);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) o[i] = (uint32_t)a[i] | ((uint32_t)b[i] << 16);
   }
 };
 
@@ -1942,13 +1959,29 @@ void gram_raw_kernel(GramArgs p) {
   }
 }
 
+// Pages of a row, whose keys and chunk sums each of them reads, on one XCD, one after the other.
+__device__ __forceinline__ unsigned row_of_page(unsigned id, unsigned pages, unsigned NB, int& jp) {
+  const unsigned rows = pages / NB;
+  if (rows % 8 != 0) { jp = id % NB; return id / NB; }
+  jp = (id >> 3) % NB;
+  return (id >> 3) / NB * 8 + (id & 7);
+}
+
 // The same for pages that are whole 128-key tiles, built like the page kernel of the lightning
 // variant: four waves, each with TWO row blocks of the row page in registers (64 rows), so a B
 // fragment read from LDS feeds two products; the column tiles go from global memory straight into
 // LDS (wave w requests rows 32 w .. 32 w + 31 of a tile, the layout of `gram_page_kernel`), two
-// buffers, one barrier per tile, the request for tile t + 1 under the products of tile t.  Two
-// workgroups per compute unit (two waves per SIMD, 256 registers each).  PARTS: a workgroup has some of
+// buffers, one barrier per tile, the request for tile t + 1 beside the products of tile t, a load at a
+// time.  Two workgroups per compute unit (two waves per SIMD, 256 registers each).  PARTS: a workgroup has some of
 // a page's tiles (see tile_parts); where it has all, first and last tile are known, which is 2 to 3 % of the kernel.
+// Of 7200 cycles a tile (two workgroups on a CU) its products take 2048; the rest is the other workgroup's products, the look at
+// the largest ones, and 1800 of waits, barriers and claims.  48 sequences of 2049 to 2560 tokens, 8 heads: 395 -> 343 us, 378 -> 328
+// without claims; 23 of two layers whose keys are copies of one another 361 -> 337; 2 sequences 23.4 -> 21.0.  A page's own rows
+// come in whole lines with its first tiles and the claims of a block and its transpose are worked out once; requests one by one,
+// fragments of the next columns before the look at these, no division per tile: request and claims 10 900 -> 5200 cycles a page,
+// products 63 800 -> 51 500.  Rows on one XCD halve what L2 misses, at no change in time.  Tried: the products of two column blocks
+// in turns, with the maxima of one beside the other's (registers for the row factors go, 357 and 337); claims by ballots and LDS
+// atomics (680 against 507 where half of the keys have copies).
 constexpr int kRawTile = 128;
 constexpr int kRawTileBytes = (kRawTile / 4) * kPgGrp;
 template <typename T, bool PARTS>
@@ -1973,12 +2006,13 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5, col = lane & 31;
-  const int pages = PARTS ? gridDim.x / p.parts : gridDim.x;
-  const int page = PARTS ? blockIdx.x % pages : blockIdx.x, part = PARTS ? blockIdx.x / pages : 0;
-  const int jp = page % p.NB;
-  const int h = (page / p.NB) % p.Hkv;
-  const int b = (page / (p.NB * p.Hkv)) % p.B;
-  const int l = page / (p.NB * p.Hkv * p.B);
+  const unsigned pages = PARTS ? gridDim.x / p.parts : gridDim.x;
+  const int part = PARTS ? blockIdx.x / pages : 0;
+  int jp;
+  const unsigned row = row_of_page(PARTS ? blockIdx.x % pages : blockIdx.x, pages, p.NB, jp);
+  const int h = row % p.Hkv;
+  const int b = row / p.Hkv % p.B;
+  const int l = row / p.Hkv / p.B;
   const int Tn = p.NB * p.BS;
   const int64_t obase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
 
@@ -1986,61 +2020,52 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   int rpid = page_is_pad(code) ? -1 : page_id(code);
   if (rpid >= p.num_pages) rpid = -1;
   if (rpid < 0) return;
-  list_valid_pages(p.table + (int64_t)b * p.NB, p.NB, p.num_pages, jp, vpage, vidx, nullptr, &nvalid_s, &mine_s);
   const int dpieces = p.D / 8;
-  if (dpieces < PIECES) {   // head dims below 128 leave the upper pieces of every LDS row at zero
-    for (int i = tid; i < 2 * kRawTileBytes / 4; i += kThreads) ((uint32_t*)smem)[i] = 0u;
+  const int k_row = p.Hkv * p.D * 2;
+  const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2;
+  // rows of a page -> LDS, a wave 32 of a tile: eight instructions of four rows; past the end of a head's rows come zeros
+  const int st_g = (lane >> 4) * 4 + (lane & 3), st_r = (lane >> 2) & 3;
+  const int st_voff = st_g < dpieces ? st_r * k_row + st_g * 16 : 0x40000000;
+  auto rows_of = [&](int pid, int toff) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(kbase + (int64_t)pid * p.k_sp * 2 + (int64_t)(toff + wave * 32) * k_row), 0, 32 * k_row, 0x00020000);
+  };
+  auto stage = [&](const __amdgpu_buffer_rsrc_t& rs, char* buf, int i) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(buf + (wave * 8 + i) * kPgGrp), 16, st_voff, i * 4 * k_row, 0, 0);
+  };
+  auto stage_all = [&](const __amdgpu_buffer_rsrc_t& rs, char* buf) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) stage(rs, buf, i);
+  };
+  // A page of at most two tiles is its own first ones: its rows are asked for before anything else.
+  const int tiles_per_page = p.BS / TNc;
+  const bool own = part == 0 && tiles_per_page <= 2;
+  if (own) {
+    stage_all(rows_of(rpid, 0), buf0);
+    if (tiles_per_page == 2) stage_all(rows_of(rpid, TNc), buf1);
   }
+  list_valid_pages(p.table + (int64_t)b * p.NB, p.NB, p.num_pages, jp, vpage, vidx, nullptr, &nvalid_s, &mine_s);
   if (tid < 2 * TNc) l_cside[tid] = -1;
   for (int i = tid; i < p.BS; i += kThreads) l_rnrow[i] = p.ws_val[obase + (int64_t)jp * p.BS + i];
   __syncthreads();
   const int nv = nvalid_s, ia = mine_s;
   const int nd = nv / 2 + (((nv & 1) || ia < nv / 2) ? 1 : 0);   // page distances 0 .. nd-1
-  const int tiles_per_page = p.BS / TNc;
   const int from = PARTS ? nd * tiles_per_page * part / p.parts : 0;                       // its tiles
   const int to = PARTS ? nd * tiles_per_page * (part + 1) / p.parts : nd * tiles_per_page;
-  const int k_row = p.Hkv * p.D * 2;
-  const char* kbase = p.k + (l * p.k_sl) * 2 + (int64_t)h * p.D * 2;
   const float* rn_all = p.ws_val + obase;           // written by raw_prep_kernel
-
-  auto tile_page = [&](int tile, int& d, int& toff) {
-    d = tile / tiles_per_page;
-    toff = (tile - d * tiles_per_page) * TNc;
-    const int ic = ia + d;
-    return ic < nv ? ic : ic - nv;
-  };
-  // tile -> LDS: eight instructions of four rows per wave; 1 / norm of the tile's keys to a register
-  const int st_g = (lane >> 4) * 4 + (lane & 3), st_r = (lane >> 2) & 3;
-  const int st_voff = st_r * k_row + st_g * 16;
-  float pre_rn = 0.f;
-  auto request = [&](int tile, char* buf) {
-    int d, toff;
-    const int ic = tile_page(tile, d, toff);
-    const int pid = __builtin_amdgcn_readfirstlane(vpage[ic]);
-    const char* src = kbase + (int64_t)pid * p.k_sp * 2 + (int64_t)(toff + wave * 32) * k_row;
-    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, 32 * k_row, 0x00020000);
-    if (st_g < dpieces) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(buf + (wave * 8 + i) * kPgGrp), 16, st_voff,
-                                                 i * 4 * k_row, 0, 0);
-    }
-    if (tid < TNc) pre_rn = rn_all[vidx[ic] * p.BS + toff + tid];
-  };
+  float pre_rn = 0.f;                               // of the next tile's key `tid`
   // Hands the column-side claims of a finished tile to the keys of its page and clears the slot.
-  auto flush_cside = [&](int tile) {
+  auto flush_cside = [&](int tile, int64_t at) {
     if (tid < TNc) {
-      int d, toff;
-      const int ic = tile_page(tile, d, toff);
       int* slot = l_cside + (tile & 1) * TNc + tid;
       const int v = *slot;
       if (v >= 0) {
-        atomicMax(p.ws_col + obase + (int64_t)vidx[ic] * p.BS + toff + tid, v);
+        atomicMax(p.ws_col + at + tid, v);
         *slot = -1;
       }
     }
   };
   const float thr_lo = p.threshold - fabsf(p.threshold) * 1e-5f - 1e-30f;
+  const bool bounded = p.threshold > 0.f;           // the largest product of a tile bounds its entries
   // fragment of k-step s of this lane's row of a 32-row block: base + (s / 2) * 256 + (s % 2) * 32
   const int rd_off = (col >> 2) * kPgGrp + (col & 3) * 64 + half * 16;
 
@@ -2048,117 +2073,158 @@ __global__ __launch_bounds__(256, 2) void gram_raw_wide_kernel(GramArgs p) {
   const int NR = (row_blocks + 2 * kWaves - 1) / (2 * kWaves);
   for (int rr = 0; rr < NR; ++rr) {
     const int rb0 = (rr * kWaves + wave) * 2;          // this wave's two row blocks: rb0, rb0 + 1
-    const bool act0 = rb0 < row_blocks, act1 = rb0 + 1 < row_blocks;
-    // ---- A fragments: this lane's two key rows as stored; lane (row, half) holds k = 16 s + 8 half + i
-    frag_t ak0[KSB], ak1[KSB];
-    {
-      const char* src0 = kbase + (int64_t)rpid * p.k_sp * 2 + (int64_t)((act0 ? rb0 : 0) * 32 + col) * k_row;
-      const char* src1 = kbase + (int64_t)rpid * p.k_sp * 2 + (int64_t)((act1 ? rb0 + 1 : 0) * 32 + col) * k_row;
+    const bool act = rb0 < row_blocks;
+    int d = from / tiles_per_page, toff = (from - d * tiles_per_page) * TNc, ic = ia + d < nv ? ia + d : ia + d - nv;
+    int64_t before_at = 0;                             // the keys of the tile before
+    int there = own && rr == 0 ? tiles_per_page : from;          // tiles that were asked for
+    if (there == from && from < to) {
+      stage_all(rows_of(__builtin_amdgcn_readfirstlane(vpage[ic]), toff), from & 1 ? buf1 : buf0);
+      if (tid < TNc) pre_rn = rn_all[vidx[ic] * p.BS + toff + tid];
+      ++there;
+    }
+    // ---- A fragments: this lane's two key rows as stored; lane (row, half) holds k = 16 s + 8 half + i.  Rows in LDS were asked
+    // for in whole lines
+    frag_t ak[2][KSB];
+    if (own) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __syncthreads();
 #pragma unroll
-      for (int s = 0; s < KSB; ++s) {
-        const int pc = 2 * s + half;
-        u32x4 v0 = u32x4{0u, 0u, 0u, 0u}, v1 = v0;
-        if (pc < dpieces) {
-          v0 = *(const u32x4*)(src0 + pc * 16);
-          v1 = *(const u32x4*)(src1 + pc * 16);
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int s = 0; s < KSB; ++s)
+          ak[g][s] = *(const frag_t*)(smem + (act ? rb0 + g : 0) * 8 * kPgGrp + rd_off + (s >> 1) * 256 + (s & 1) * 32);
+    } else {
+#pragma unroll
+      for (int g = 0; g < 2; ++g) {
+        const char* src = kbase + (int64_t)rpid * p.k_sp * 2 + (int64_t)((act ? rb0 + g : 0) * 32 + col) * k_row;
+#pragma unroll
+        for (int s = 0; s < KSB; ++s) {
+          const int pc = 2 * s + half;
+          u32x4 v = u32x4{0u, 0u, 0u, 0u};
+          if (pc < dpieces) v = *(const u32x4*)(src + pc * 16);
+          ak[g][s] = __builtin_bit_cast(frag_t, v);
         }
-        ak0[s] = __builtin_bit_cast(frag_t, v0);
-        ak1[s] = __builtin_bit_cast(frag_t, v1);
       }
     }
-    float rn_row0[16], rn_row1[16];
+    float rn_row[2][16], rn_most[2];                   // of the rows whose products this lane has
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const float4 v0 = *(const float4*)(l_rnrow + (act0 ? rb0 : 0) * 32 + half * 4 + g * 8);
-      const float4 v1 = *(const float4*)(l_rnrow + (act1 ? rb0 + 1 : 0) * 32 + half * 4 + g * 8);
-      rn_row0[4 * g] = v0.x; rn_row0[4 * g + 1] = v0.y; rn_row0[4 * g + 2] = v0.z; rn_row0[4 * g + 3] = v0.w;
-      rn_row1[4 * g] = v1.x; rn_row1[4 * g + 1] = v1.y; rn_row1[4 * g + 2] = v1.z; rn_row1[4 * g + 3] = v1.w;
+    for (int g = 0; g < 2; ++g) {
+      rn_most[g] = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float4 v = *(const float4*)(l_rnrow + (act ? rb0 + g : 0) * 32 + half * 4 + q * 8);
+        rn_row[g][4 * q] = v.x, rn_row[g][4 * q + 1] = v.y, rn_row[g][4 * q + 2] = v.z, rn_row[g][4 * q + 3] = v.w;
+        rn_most[g] = fmaxf(rn_most[g], fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w)));
+      }
     }
-    int dcol0[16], dcol1[16];
-#pragma unroll
-    for (int r = 0; r < 16; ++r) { dcol0[r] = -1; dcol1[r] = -1; }
 
-    if (from < to) request(from, (from & 1) ? buf1 : buf0);
+    int dcol[2][16];
+#pragma unroll
+    for (int g = 0; g < 2; ++g)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) dcol[g][r] = -1;
     for (int tile = from; tile < to; ++tile) {
-      char* cur = (tile & 1) ? buf1 : buf0;
-      char* nxt = (tile & 1) ? buf0 : buf1;
+      char* const cur = (tile & 1) ? buf1 : buf0;
+      char* const nxt = (tile & 1) ? buf0 : buf1;
+      const int jc = vidx[ic];
+      int toff1 = toff + TNc, d1 = d, ic1 = ic;        // the next one
+      if (toff1 == p.BS) toff1 = 0, ++d1, ic1 = ic + 1 < nv ? ic + 1 : 0;
+      const int next_pid = __builtin_amdgcn_readfirstlane(vpage[ic1]), next_idx = vidx[ic1];
       // this wave's share of the tile (and its A fragments, the first time) has landed; after the
       // barrier so has everybody's, and everybody is done with the tile before
       asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      if (tid < TNc) l_rn[(tile & 1) * TNc + tid] = pre_rn;
+      if (tid < TNc) l_rn[(tile & 1) * TNc + tid] = d == 0 ? l_rnrow[toff + tid] : pre_rn;
       __syncthreads();
-      if (tile + 1 < to) request(tile + 1, nxt);
-      if (tile > from) flush_cside(tile - 1);   // its slot is next written two tiles from now
-      int d, toff;
-      const int ic = tile_page(tile, d, toff);
-      const int jc = vidx[ic];
-      // what a tile of 32 x 32 products feeds: the last column over the threshold of its rows and
-      // (other pages only: inside a page both (i, j) and (j, i) are computed) the last row over
-      // the threshold of its columns
-      auto scan = [&](f32x16_t& acc, int rb, const float* rn_row, int* dcol, int st, float rn_col) {
-        const int cslot = toff + st * 32 + col;
-        const int cidx = jc * p.BS + cslot;
-        if (d == 0) {
+      const bool ask = there < to && there == tile + 1;
+      const __amdgpu_buffer_rsrc_t next = rows_of(next_pid, toff1);
+      if (ask) {
+        if (tid < TNc) pre_rn = rn_all[next_idx * p.BS + toff1 + tid];
+        ++there;
+      }
+      if (tile > from) flush_cside(tile - 1, before_at);   // its slot is next written two tiles from now
+      before_at = obase + (int64_t)jc * p.BS + toff;
+      const int tile_d = d, tile_off = toff;
+      d = d1, toff = toff1, ic = ic1;
+      // blocks of columns that lie below both row blocks' diagonals have been seen
+      const int first = !act ? NSUB : tile_d == 0 ? min(max(rb0 - (tile_off >> 5), 0), NSUB) : 0;
+      const bool beside = ask && first == 0;           // loads one by one beside the products: eight in a row hold a wave
+      if (ask && !beside) stage_all(next, nxt);
+      if (first == NSUB) continue;
+      // What a tile of 32 x 32 products feeds: the last column over the threshold of its rows and the last row over the
+      // threshold of its columns.  Inside a page blocks below the diagonal are the transposes of those above it.
+      auto claims = [&](f32x16_t& acc, int g, int st, float rn_col) {
+        const int rb = rb0 + g, cb = (tile_off >> 5) + st;
+        if (tile_d == 0 && cb <= rb) {
+          if (cb < rb) return;
           // the page against itself: a key against itself counts as 0
 #pragma unroll
           for (int r = 0; r < 16; ++r)
-            if (rb * 32 + (r >> 2) * 8 + half * 4 + (r & 3) == cslot) acc[r] = 0.f;
+            if ((r >> 2) * 8 + half * 4 + (r & 3) == col) acc[r] = 0.f;
         }
-        // most tiles hold no entry over the threshold: one maximum decides
-        float big = -INFINITY;
-#pragma unroll
-        for (int r = 0; r < 16; ++r) big = fmaxf(big, acc[r] * rn_row[r]);
-        if (!__any(big * rn_col > thr_lo)) return;
+        const int cidx = jc * p.BS + tile_off + st * 32 + col;
         int rlast = -1;
 #pragma unroll
         for (int r = 0; r < 16; ++r) {
-          const bool over = acc[r] * (rn_row[r] * rn_col) > p.threshold;
-          dcol[r] = max(dcol[r], over ? cidx : -1);
+          const bool over = acc[r] * (rn_row[g][r] * rn_col) > p.threshold;
+          dcol[g][r] = max(dcol[g][r], over ? cidx : -1);
           rlast = over ? r : rlast;
         }
-        if (d != 0 && __any(rlast >= 0)) {
+        if ((tile_d != 0 || cb != rb) && __any(rlast >= 0)) {
           int ci = rlast < 0 ? -1 : jp * p.BS + rb * 32 + (rlast >> 2) * 8 + half * 4 + (rlast & 3);
           ci = max(ci, lane_xor32(ci));
           if (half == 0 && ci >= 0) atomicMax(&l_cside[(tile & 1) * TNc + st * 32 + col], ci);
         }
       };
-      if (act0) {
+      // Two row blocks against 32 columns at a time.  Fragments leave LDS kAhead ahead of their products, those of the next
+      // columns too.  Most tiles hold no entry over the threshold: their largest product, as integers, which order what is
+      // positive, and the largest row factor decide.
+      constexpr int kAhead = 3, kRing = 4;
+      static_assert(KSB % kRing == 0, "places of the ring are constants");
+      frag_t bk[kRing];
+      const char* brow = cur + first * 8 * kPgGrp + rd_off;
+      auto fragment = [&](int s) { bk[s % kRing] = *(const frag_t*)(brow + (s >> 1) * 256 + (s & 1) * 32); };
+#pragma unroll
+      for (int s = 0; s < kAhead; ++s) fragment(s);
 #pragma unroll 1
-        for (int st = 0; st < NSUB; ++st) {
-          f32x16_t acc0, acc1;
+      for (int st = first; st < NSUB; ++st) {
+        const float rn_col = l_rn[(tile & 1) * TNc + st * 32 + col];
+        f32x16_t acc[2];
 #pragma unroll
-          for (int r = 0; r < 16; ++r) { acc0[r] = 0.f; acc1[r] = 0.f; }
-          const char* brow = cur + st * 8 * kPgGrp + rd_off;
-          const float rn_col = l_rn[(tile & 1) * TNc + st * 32 + col];
+        for (int g = 0; g < 2; ++g)
 #pragma unroll
-          for (int s0 = 0; s0 < KSB; s0 += 4) {
-            frag_t bk[4];
+          for (int r = 0; r < 16; ++r) acc[g][r] = 0.f;
 #pragma unroll
-            for (int s = 0; s < 4; ++s) bk[s] = *(const frag_t*)(brow + ((s0 + s) >> 1) * 256 + ((s0 + s) & 1) * 32);
+        for (int s = 0; s < KSB; ++s) {
+          if (s + kAhead == KSB && st + 1 < NSUB) brow += 8 * kPgGrp;      // behind the last columns they come again
+          fragment((s + kAhead) % KSB);
 #pragma unroll
-            for (int s = 0; s < 4; ++s) {
-              acc0 = Mfma16<T>::run(ak0[s0 + s], bk[s], acc0);
-              acc1 = Mfma16<T>::run(ak1[s0 + s], bk[s], acc1);
-            }
-          }
-          scan(acc0, rb0, rn_row0, dcol0, st, rn_col);
-          if (act1) scan(acc1, rb0 + 1, rn_row1, dcol1, st, rn_col);
+          for (int g = 0; g < 2; ++g) acc[g] = Mfma16<T>::run(ak[g][s], bk[s % kRing], acc[g]);
+          if (beside && (s == 2 || s == 5)) stage(next, nxt, 2 * st + (s == 5));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int g = 0; g < 2; ++g) {
+          int big = -1;
+#pragma unroll
+          for (int r = 0; r < 16; ++r) big = max(big, __float_as_int(acc[g][r]));
+          if (!bounded || __any(!(__int_as_float(big) * rn_most[g] * rn_col <= thr_lo))) claims(acc[g], g, st, rn_col);
         }
       }
     }
     __syncthreads();   // everybody is done with the last tile
-    if (from < to) flush_cside(to - 1);
+    if (from < to) flush_cside(to - 1, before_at);
     bool any_mine = false;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) any_mine |= dcol0[r] >= 0 || dcol1[r] >= 0;
+    for (int r = 0; r < 16; ++r) any_mine |= dcol[0][r] >= 0 || dcol[1][r] >= 0;
     if (__any(any_mine)) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int c0 = half_max_i(dcol0[r]), c1 = half_max_i(dcol1[r]);
-        const int64_t row = obase + (int64_t)jp * p.BS + rb0 * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
-        if (act0 && col == 0 && c0 >= 0) atomicMax(p.ws_col + row, c0);
-        if (act1 && col == 0 && c1 >= 0) atomicMax(p.ws_col + row + 32, c1);
-      }
+      for (int g = 0; g < 2; ++g)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) {
+          const int c = half_max_i(dcol[g][r]);
+          const int64_t at = obase + (int64_t)jp * p.BS + (rb0 + g) * 32 + (r >> 2) * 8 + half * 4 + (r & 3);
+          if (act && col == 0 && c >= 0) atomicMax(p.ws_col + at, c);
+        }
     }
     __syncthreads();   // the claim slots are clear again before the next round writes them
   }
@@ -2237,9 +2303,20 @@ __global__ __launch_bounds__(kThreads) void raw_claim_value_kernel(GramArgs p) {
 // with s_chunk the sum of the chunk's normalised keys from raw_prep_kernel.  The dot products of
 // a page's 256 keys with 32 chunks at a time run on the matrix cores: the keys as stored (exact
 // 16-bit products), s_chunk split into three 16-bit planes (together its full fp32 mantissa).
-// One workgroup per valid page; wave w owns keys 32 w .. 32 w + 31.
+// One workgroup per valid page.  A wave has 64 keys as the columns of two products, so a fragment of the planes read from LDS
+// feeds both (with 32, LDS was as busy as the matrix cores), and one exchange between its halves leaves every lane with one
+// key's 32 chunk sums in order: the chain runs in registers, on all lanes.  What it replaces went through LDS, half of the
+// threads walked the chain of a tile behind a barrier, and the claims of a row went through a list.  48 sequences of 2049 to 2560
+// tokens, 8 heads: 274 -> 183 us; 2 of them 26.5 -> 17.7.  Bound by what a page does one after the other: of 42 000 cycles (two
+// workgroups on a CU) the table, the keys and the first planes take 16 000, the products 12 000 (7100 of them the matrix
+// cores'), splitting and corrections 9000.
 // chunk sums are below 16 + 1 in magnitude: 2^-26 fixed point fits 32 bits, and integer atomics
 // make the sum of several claims independent of their order
+// Chunks that raw_chain_kernel takes at a time; words of a key's corrections, 16 bytes of neighbours in different banks; bytes of
+// LDS: a round's 256 keys, and then planes and corrections.
+constexpr int kChainTile = 32, kChainLd = kChainTile + 4;
+constexpr int kChainBytes = 256 / 4 * kPgGrp;
+static_assert(3 * kChainTile * ROWH + 256 * kChainLd * 4 <= kChainBytes, "planes and corrections fit where the keys were");
 __device__ __forceinline__ int to_fixed26(float v) { return (int)(v * 67108864.f); }
 __device__ __forceinline__ float from_fixed26(int w) { return (float)w * (1.f / 67108864.f); }
 
@@ -2254,32 +2331,30 @@ extern "C" int zp_debug_chain_stamps(long long* dst, int n_groups) {
 #endif
 
 template <typename T>
-__global__ __launch_bounds__(512, 4) void raw_chain_kernel(GramArgs p) {
+__global__ __launch_bounds__(256, 2) void raw_chain_kernel(GramArgs p) {
   static_assert(T::bytes == 2, "16-bit caches only");
   typedef typename Mfma16<T>::V frag_t;
-  constexpr int kT = 512, kW = 8, KSB = kDmax / 16, CT = 32;     // CT chunks per tile
-  constexpr int KEYS = kW * 32;                                     // keys per round
+  constexpr int kT = 256, KSB = kDmax / 16, CT = kChainTile;     // CT chunks per tile
+  constexpr int KEYS = kT;                                          // keys per round
   extern __shared__ __align__(16) char smem[];
   char* planes = smem;                                   // [3][CT] rows of ROWH bytes
-  int* cl = (int*)(smem + 3 * CT * ROWH);                // [CT][KEYS] corrections, then chunk sums
-  int* vidx = cl + CT * KEYS;                            // [NB] logical page of the n-th valid page
-  int* vord = vidx + p.NB;                               // [NB] inverse (-1: pad)
-  // the claims taken from this round's keys, gathered once per round: (chunk << 16 | key) and value
-  uint32_t* lst_key = (uint32_t*)(vord + p.NB);          // [NB * BS]
-  float* lst_val = (float*)(lst_key + (size_t)p.NB * p.BS);
-  __shared__ int nvalid_s, nlist_s;
+  int* cl = (int*)(smem + 3 * CT * ROWH);                // [KEYS][kChainLd] corrections
+  int* vidx = (int*)(smem + kChainBytes);                // [NB] logical page of the n-th valid page
+  int* chunk_of = vidx + p.NB;                           // [NB * BS / 16] logical chunk of the n-th one of the valid pages
+  __shared__ int nvalid_s, mine_s, corrected[2];         // corrected: whether a tile has any
 
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int tid = threadIdx.x, lane = tid & 63;
   const int half = lane >> 5, col = lane & 31;
 #ifdef ZP_PAGE_STAMP
   long long acc_[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   long long last_ = clock64();
   const long long wall0 = wall_clock64();
 #endif
-  const int jp = blockIdx.x % p.NB;
-  const int h = (blockIdx.x / p.NB) % p.Hkv;
-  const int b = (blockIdx.x / (p.NB * p.Hkv)) % p.B;
-  const int l = blockIdx.x / (p.NB * p.Hkv * p.B);
+  int jp;
+  const unsigned row = row_of_page(blockIdx.x, gridDim.x, p.NB, jp);
+  const int h = row % p.Hkv;
+  const int b = row / p.Hkv % p.B;
+  const int l = row / p.Hkv / p.B;
   const int Tn = p.NB * p.BS;
   const int64_t obase = (((int64_t)l * p.B + b) * p.Hkv + h) * Tn;
 
@@ -2290,180 +2365,204 @@ __global__ __launch_bounds__(512, 4) void raw_chain_kernel(GramArgs p) {
     for (int s = tid; s < p.BS; s += kT) Elem<T>::st(p.r_out, obase + (int64_t)jp * p.BS + s, -INFINITY);
     return;
   }
-  list_valid_pages(p.table + (int64_t)b * p.NB, p.NB, p.num_pages, jp, nullptr, vidx, vord, &nvalid_s, nullptr);
-  __syncthreads();
   const int cpp = p.BS / kChunk;
-  const int nchunks = nvalid_s * cpp;
-  const int ntiles = (nchunks + CT - 1) / CT;
-  const int my_ord = vord[jp];
   const int dpieces = p.D / 8;
-  const int64_t k_row = (int64_t)p.Hkv * p.D * 2;
+  const int k_row = p.Hkv * p.D * 2;
   const char* kpage = p.k + (l * p.k_sl + (int64_t)rpid * p.k_sp) * 2 + (int64_t)h * p.D * 2;
   const float* chunk_all = p.ws_chunk + (obase / kChunk) * kDmax;
+  // ---- the wave's 64 keys in whole lines into LDS, where planes and corrections will lie: rows of 256 bytes asked for as
+  // operands touch each line four times, which takes three times as long
+  const int st_g = (lane >> 4) * 4 + (lane & 3), st_r = (lane >> 2) & 3;
+  char* const keys = smem + (tid >> 6) * 16 * kPgGrp;
+  auto stage_keys = [&](int first) {
+    const int left = p.BS - first;
+    if (left <= 0 || st_g >= dpieces) return;
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc((void*)(kpage + (int64_t)first * k_row), 0, min(left, 64) * k_row, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < 16; ++i)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(keys + i * kPgGrp), 16, st_r * k_row + st_g * 16, i * 4 * k_row, 0, 0);
+  };
+  const int wave64 = __builtin_amdgcn_readfirstlane(tid & ~63);
+  stage_keys(wave64);
+  list_valid_pages(p.table + (int64_t)b * p.NB, p.NB, p.num_pages, jp, nullptr, vidx, nullptr, &nvalid_s, &mine_s);
+  __syncthreads();
+  const int nchunks = nvalid_s * cpp;
+  const int ntiles = (nchunks + CT - 1) / CT;
+  const int my_ord = mine_s;
+  for (int i = tid; i < nchunks; i += kT) chunk_of[i] = vidx[i / cpp] * cpp + i % cpp;
+  __syncthreads();
 
   const int rounds = (p.BS + KEYS - 1) / KEYS;
   for (int rr = 0; rr < rounds; ++rr) {
-    const int key0 = rr * KEYS;                       // first slot of this round
-    const int slot = key0 + wave * 32 + col;          // this lane's key (both halves of the wave)
+    const int key0 = rr * KEYS, row0 = jp * p.BS + key0;   // first slot of this round
+    const int slot = key0 + tid;                           // the key whose chain this lane walks
     const bool live = slot < p.BS;
-    // ---- B fragments: the key as stored; lane (key, half) holds k = 16 s + 8 half + i
-    frag_t bk[KSB];
-    float ssq = 0.f;
-    {
-      const char* src = kpage + (int64_t)(live ? slot : 0) * k_row;
+    // What a tile needs is requested one tile ahead: its chunk sums (CT x kDmax floats), which are split into the three planes
+    // once the tile before is done with them, and the claims of its CT * kChunk keys, whose values are corrections where
+    // they were taken from this round's keys.
+    constexpr int kSums = CT * (kDmax / 4) / kT, kClaims = CT * kChunk / kT;
+    float4 pv[kSums];
+    int from[kClaims];
+    float value[kClaims];
+    auto request = [&](int tile) {
+#pragma unroll
+      for (int u = 0; u < kSums; ++u) {
+        const int i = tid + u * kT;
+        const int vc = tile * CT + i / (kDmax / 4), q4 = i % (kDmax / 4);
+        pv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (vc < nchunks) pv[u] = *(const float4*)(chunk_all + (int64_t)chunk_of[vc] * kDmax + q4 * 4);
+      }
+#pragma unroll
+      for (int u = 0; u < kClaims; ++u) {
+        const int i = tid + u * kT, vc = tile * CT + i / kChunk;
+        from[u] = -1;
+        if (vc < nchunks) {
+          const int64_t t = obase + (int64_t)chunk_of[vc] * kChunk + i % kChunk;
+          from[u] = p.ws_col[t] - row0;
+          value[u] = p.ws_val[t];
+        }
+      }
+    };
+    // the next tile's planes, the corrections of its entries
+    auto store = [&](int tile, int own_chunk, float diag) {
+#pragma unroll
+      for (int u = 0; u < kSums; ++u) {
+        const int i = tid + u * kT;
+        const int m = i / (kDmax / 4), q4 = i % (kDmax / 4);
+        uint32_t lo[3], hi[3];
+        Split3<T>::two(pv[u].x, pv[u].y, lo);
+        Split3<T>::two(pv[u].z, pv[u].w, hi);
+#pragma unroll
+        for (int pl = 0; pl < 3; ++pl) *(uint2*)(planes + (pl * CT + m) * ROWH + q4 * 8) = make_uint2(lo[pl], hi[pl]);
+      }
+      bool any = false;
+#pragma unroll
+      for (int u = 0; u < kClaims; ++u)
+        if (from[u] >= 0 && from[u] < KEYS && key0 + from[u] < p.BS) {
+          atomicAdd(&cl[from[u] * kChainLd + (tid + u * kT) / kChunk], to_fixed26(value[u]));
+          any = true;
+        }
+      const int own = own_chunk - tile * CT;
+      if (live && own >= 0 && own < CT) {
+        atomicAdd(&cl[tid * kChainLd + own], to_fixed26(diag));
+        any = true;
+      }
+      if (any) corrected[tile & 1] = 1;
+    };
+    request(0);
+    const float rn = live ? p.ws_sum[obase + row0 + tid] : 0.f;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");      // this wave's keys are in LDS
+    ZP_CSTAMP(0);   // table lookup, page list, first requests
+    // ---- B fragments: keys as stored; lane (col, half) holds k = 16 s + 8 half + i of keys col and col + 32 of the wave's 64
+    frag_t bk[2][KSB];
+    float ssq[2];
+#pragma unroll
+    for (int g = 0; g < 2; ++g) {
+      const bool there = key0 + wave64 + g * 32 + col < p.BS;
+      const char* src = keys + (g * 8 + (col >> 2)) * kPgGrp + (col & 3) * 64 + half * 16;
+      ssq[g] = 0.f;
 #pragma unroll
       for (int s = 0; s < KSB; ++s) {
-        const int pc = 2 * s + half;
-        u32x4 v = u32x4{0u, 0u, 0u, 0u};
-        if (live && pc < dpieces) v = *(const u32x4*)(src + pc * 16);
-        bk[s] = __builtin_bit_cast(frag_t, v);
+        u32x4 v = *(const u32x4*)(src + (s >> 1) * 256 + (s & 1) * 32);
+        if (!there || 2 * s + half >= dpieces) v = u32x4{0u, 0u, 0u, 0u};
+        bk[g][s] = __builtin_bit_cast(frag_t, v);
         float e[8];
         Unpack<T>::run(vec16{v.x, v.y, v.z, v.w}, e);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) ssq = fmaf(e[q], e[q], ssq);
+        for (int q = 0; q < 8; ++q) ssq[g] = fmaf(e[q], e[q], ssq[g]);
       }
-      ssq += lane_xor32(ssq);
+      ssq[g] += lane_xor32(ssq[g]);
     }
-    ZP_CSTAMP(0);   // set-up, key loads issued
-    const float rn = live ? p.ws_sum[obase + (int64_t)jp * p.BS + slot] : 0.f;
-    const float diag = ssq * rn * rn;                 // S_ii, the entry the reference zeroes
+    const float diag = (half ? ssq[1] : ssq[0]) * rn * rn;    // S_ii, the entry the reference zeroes
     const int own_chunk = my_ord * cpp + slot / kChunk;
-    float part = 0.f, total = 0.f;                    // chain state of key `tid` (tid < KEYS)
-    // every key of the sequence claims at most one entry: one pass over the claims keeps those
-    // taken from this round's keys, with the chunk of the claiming key (the order of the list does
-    // not matter, the values are added as fixed point)
+    float part = 0.f, total = 0.f;                    // chain state of this lane's key
+    __syncthreads();                                  // everyone has its keys
+    for (int i = tid; i < KEYS * kChainLd / 4; i += kT) ((int4*)cl)[i] = make_int4(0, 0, 0, 0);
+    if (tid == 0) corrected[0] = 0;
     __syncthreads();
-    if (tid == 0) nlist_s = 0;
-    __syncthreads();
-    for (int t0 = tid; t0 < Tn; t0 += 4 * kT) {      // four independent loads in flight per thread
-      int cw[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = t0 + u * kT;
-        cw[u] = t < Tn ? p.ws_col[obase + t] : -1;
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const int t = t0 + u * kT;
-        if (t >= Tn) continue;
-        const int jt = t / p.BS;
-        const int ord = vord[jt];
-        if (ord < 0) continue;
-        const int cc = cw[u] - (jp * p.BS + key0);   // the row key t claimed from
-        if (cc >= 0 && cc < KEYS && key0 + cc < p.BS) {
-          const int i = atomicAdd(&nlist_s, 1);
-          lst_key[i] = (uint32_t)(ord * cpp + (t - jt * p.BS) / kChunk) << 16 | (uint32_t)cc;
-          lst_val[i] = p.ws_val[obase + t];
-        }
-      }
-    }
-    __syncthreads();
-    const int nlist = nlist_s;
-    ZP_CSTAMP(1);   // claims gathered
-
-    // the chunk sums of a tile (CT chunks x kDmax floats, two float4 per thread) are requested one
-    // tile ahead and split into the three planes once the tile before is done with them
-    static_assert(CT * (kDmax / 4) == 2 * kT, "two float4 of a tile's chunk sums per thread");
-    float4 pv[2];
-    auto request_planes = [&](int tile) {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int i = tid + u * kT;
-        const int m = i / (kDmax / 4), q4 = i - m * (kDmax / 4);
-        const int vc = tile * CT + m;
-        pv[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-        if (vc < nchunks) {
-          const int vp = vc / cpp, c = vc - vp * cpp;
-          pv[u] = *(const float4*)(chunk_all + ((int64_t)vidx[vp] * cpp + c) * kDmax + q4 * 4);
-        }
-      }
-    };
-    auto store_planes = [&]() {
-#pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        const int i = tid + u * kT;
-        const int m = i / (kDmax / 4), q4 = i - m * (kDmax / 4);
-        const float f[4] = {pv[u].x, pv[u].y, pv[u].z, pv[u].w};
-        uint16_t o[4][3];
-#pragma unroll
-        for (int q = 0; q < 4; ++q) Split3<T>::run(f[q], o[q]);
-#pragma unroll
-        for (int pl = 0; pl < 3; ++pl) {
-          uint2 w;
-          w.x = (uint32_t)o[0][pl] | ((uint32_t)o[1][pl] << 16);
-          w.y = (uint32_t)o[2][pl] | ((uint32_t)o[3][pl] << 16);
-          *(uint2*)(planes + (pl * CT + m) * ROWH + q4 * 8) = w;
-        }
-      }
-    };
-    if (ntiles > 0) { request_planes(0); store_planes(); }
-    if (ntiles > 1) request_planes(1);
-    ZP_CSTAMP(2);   // first planes
+    store(0, own_chunk, diag);
+    if (ntiles > 1) request(1);
+    ZP_CSTAMP(1);   // first planes
+    int cm = 0;                              // where the next chunk lies inside its page
     for (int tile = 0; tile < ntiles; ++tile) {
-      const int c0 = tile * CT;
-      // ---- corrections of this tile (its three planes are in LDS)
-      for (int i = tid; i < CT * KEYS / 4; i += kT) ((int4*)cl)[i] = make_int4(0, 0, 0, 0);
-      __syncthreads();
-      ZP_CSTAMP(3);   // corrections cleared
-      if (half == 0 && live && own_chunk >= c0 && own_chunk < c0 + CT)
-        atomicAdd(&cl[(own_chunk - c0) * KEYS + wave * 32 + col], to_fixed26(diag));
-      for (int i = tid; i < nlist; i += kT) {
-        const uint32_t w = lst_key[i];
-        const int vc = (int)(w >> 16);
-        if (vc >= c0 && vc < c0 + CT)
-          atomicAdd(&cl[(vc - c0) * KEYS + (int)(w & 0xffffu)], to_fixed26(lst_val[i]));
-      }
-      __syncthreads();
-      ZP_CSTAMP(4);   // corrections added
+      __syncthreads();                       // the tile's planes and corrections are in LDS
+      const bool some = corrected[tile & 1] != 0;
+      if (tid == 0) corrected[(tile + 1) & 1] = 0;
+      ZP_CSTAMP(2);   // barrier
       // ---- chunk sums of the tile: A = planes (rows = chunks), B = keys
-      {
-        f32x16_t acc;
+      f32x16_t acc[2];
 #pragma unroll
-        for (int r = 0; r < 16; ++r) acc[r] = 0.f;
+      for (int g = 0; g < 2; ++g)
 #pragma unroll
-        for (int pl = 2; pl >= 0; --pl) {
-          const char* arow = planes + (pl * CT + col) * ROWH + half * 16;
+        for (int r = 0; r < 16; ++r) acc[g][r] = 0.f;
+      // fragments leave LDS kAhead ahead of their products, the smallest plane first
+      constexpr int kAhead = 4, kFrags = 3 * KSB;
+      frag_t a[kAhead + 1];
+      auto fragment = [&](int n) { a[n % (kAhead + 1)] = *(const frag_t*)(planes + ((2 - n / KSB) * CT + col) * ROWH + half * 16 + n % KSB * 32); };
 #pragma unroll
-          for (int s = 0; s < KSB; ++s) acc = Mfma16<T>::run(*(const frag_t*)(arow + s * 32), bk[s], acc);
-        }
+      for (int n = 0; n < kAhead; ++n) fragment(n);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int m = (r >> 2) * 8 + half * 4 + (r & 3);
-          int* slot_p = &cl[m * KEYS + wave * 32 + col];
-          *slot_p = __float_as_int(acc[r] * rn - from_fixed26(*slot_p));
+      for (int n = 0; n < kFrags; ++n) {
+        if (n + kAhead < kFrags) fragment(n + kAhead);
+        acc[0] = Mfma16<T>::run(a[n % (kAhead + 1)], bk[0][n % KSB], acc[0]);
+        acc[1] = Mfma16<T>::run(a[n % (kAhead + 1)], bk[1][n % KSB], acc[1]);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      // lane (col, half) has chunks 8 (r / 4) + 4 half + r % 4 of keys col and col + 32; now all of them of one key
+      float v[CT];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const auto both = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[0][r]), __float_as_uint(acc[1][r]), false, false);
+        const int m = (r >> 2) * 8 + (r & 3);
+        v[m] = __uint_as_float(both[0]) * rn;
+        v[m + 4] = __uint_as_float(both[1]) * rn;
+      }
+      if (some) {
+#pragma unroll
+        for (int m = 0; m < CT; m += 4) {
+          int4* const at = (int4*)(cl + tid * kChainLd + m);
+          const int4 c = *at;
+          v[m] -= from_fixed26(c.x);
+          v[m + 1] -= from_fixed26(c.y);
+          v[m + 2] -= from_fixed26(c.z);
+          v[m + 3] -= from_fixed26(c.w);
+          *at = make_int4(0, 0, 0, 0);
         }
       }
-      __syncthreads();
-      ZP_CSTAMP(5);   // products
-      // the products are done with this tile's planes: the next tile's go in, the one after is requested
+      ZP_CSTAMP(3);   // products
+      __syncthreads();                       // everyone is done with the planes and this lane's corrections are clear
+      ZP_CSTAMP(4);   // barrier
       if (tile + 1 < ntiles) {
-        store_planes();
-        if (tile + 2 < ntiles) request_planes(tile + 2);
+        store(tile + 1, own_chunk, diag);
+        if (tile + 2 < ntiles) request(tile + 2);
       }
-      // ---- the reference's chain: one cache-dtype partial sum per column page
-      if (tid < KEYS) {
-        int cm = c0 % cpp;                     // where the tile's first chunk lies inside its page
-        const int mend = min(CT, nchunks - c0);
-        for (int m0 = 0; m0 < mend; m0 += 8) {   // eight chunk sums read ahead of the serial chain
-          float v[8];
+      ZP_CSTAMP(5);   // next planes stored
+      // ---- the reference's chain: one cache-dtype partial sum per column page.  Behind the last chunk there are zeros.
+      auto page_ends = [&](int chunks) {
+        if (cm == 0) { total += part; part = 0.f; }
+        cm += chunks;
+        if (cm >= cpp) cm = 0;
+      };
+      if (cpp % 8 == 0) {
 #pragma unroll
-          for (int u = 0; u < 8; ++u) v[u] = m0 + u < mend ? __int_as_float(cl[(m0 + u) * KEYS + tid]) : 0.f;
+        for (int m = 0; m < CT; ++m) {
+          if (m % 8 == 0) page_ends(8);
+          part = Elem<T>::rnd(part + v[m]);
+        }
+      } else {
 #pragma unroll
-          for (int u = 0; u < 8; ++u) {
-            if (m0 + u < mend) {
-              if (cm == 0) { total += part; part = 0.f; }
-              part = Elem<T>::rnd(part + v[u]);
-              cm = cm + 1 == cpp ? 0 : cm + 1;
-            }
-          }
+        for (int m = 0; m < CT; ++m) {
+          page_ends(1);
+          part = Elem<T>::rnd(part + v[m]);
         }
       }
-      ZP_CSTAMP(6);   // next planes stored, chain of thread 0
-      __syncthreads();
-      ZP_CSTAMP(7);   // barrier behind the chain
+      ZP_CSTAMP(6);   // chain
     }
-    if (tid < KEYS && key0 + tid < p.BS)
-      Elem<T>::st(p.r_out, obase + (int64_t)jp * p.BS + key0 + tid, total + part);
+    if (live) Elem<T>::st(p.r_out, obase + row0 + tid, total + part);
+    if (rr + 1 < rounds) {
+      __syncthreads();                       // everyone is done with the planes
+      stage_keys(key0 + KEYS + wave64);
+    }
   }
 #ifdef ZP_PAGE_STAMP
   if (tid == 0 && blockIdx.x < (1 << 16)) {
@@ -2744,9 +2843,8 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
     const size_t smemw = 2 * (size_t)kRawTileBytes + sizeof(int) * 4 * kRawTile + sizeof(float) * a.BS +
                          sizeof(int) * 2 * a.NB;
     const bool wide = tn == 128 && smemw <= 80 * 1024;
-    const size_t smem2 = 3 * 32 * (size_t)ROWH + sizeof(int) * 32 * 256 + sizeof(int) * 2 * a.NB +
-                         (size_t)a.NB * a.BS * 8;   // + the round's claim list
-    if (smem2 > 160 * 1024) {
+    const size_t smem2 = kChainBytes + sizeof(int) * (a.NB + a.NB * a.BS / kChunk);
+    if (58880 + (size_t)a.NB * (8 + a.BS * 8) > 160 * 1024) {   // rows of up to 13 120 tokens
       zp_set_error("redundancy: a row of %d tokens exceeds LDS", a.NB * a.BS);
       return ZP_EUNSUPPORTED;
     }
@@ -2765,7 +2863,7 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
     else if (tn == 128) hipLaunchKernelGGL((gram_raw_kernel<T, 128>), grid, dim3(512), smem1, st, a);
     else hipLaunchKernelGGL((gram_raw_kernel<T, TN>), grid, dim3(512), smem1, st, a);
     hipLaunchKernelGGL((raw_claim_value_kernel<T>), dim3(grid.x * claims.parts), dim3(kThreads), 0, st, claims);
-    hipLaunchKernelGGL((raw_chain_kernel<T>), grid, dim3(512), smem2, st, a);
+    hipLaunchKernelGGL((raw_chain_kernel<T>), grid, dim3(256), smem2, st, a);
     ZP_LAUNCH_CHECK();
     return ZP_OK;
   }
