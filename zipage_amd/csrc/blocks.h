@@ -194,7 +194,7 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 // Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) and the chain of states between them
 // allow.  Where the sums and the two
 // launches cost more than what is saved, runs stay whole (PieceCost): a block of the sums takes 0.3 of one with rows (0.8 for the
-// delta rule), the launches 19 us (17 for the delta rule, whose blocks are the longer ones), states of the delta rule 5.7 us a
+// delta rule), the launches 19 us (17 for the delta rule, whose blocks are the longer ones), states of the delta rule 4.3 us a
 // piece (matrix memory, 8 heads, a prompt of 155 tokens: whole 41.8 us, in pieces 42.8; linear attention, 32 heads, 200
 // tokens: 53, 46).  Whole scans: linear attention, 32 heads of 128,
 // 4 prompts of 500 to 2048 tokens 374 -> 287 us; 16 heads, 8 prompts of 2048, retention 429 -> 332 and matrix memory 369

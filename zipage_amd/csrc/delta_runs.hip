@@ -494,33 +494,36 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
 // it, then M as a left operand, [rows / 16][columns / 16][64 lanes][4].
 __host__ __device__ inline constexpr int piece_floats(int dk) { return 2 * dk * dk; }
 
-// From sums to the states before the pieces, in place; a wave 16 columns.  The products are those of the blocks, M split by
-// all waves together while the piece before is worked on: 5.7 us a piece.
-template <int KT>
-__global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
+// From sums to the states before the pieces, in place; a wave 16 columns, a workgroup half of them, which splits all of M: 4.3 us
+// a piece.  With all columns in one workgroup the products and reads of eight waves take 5.7; with a quarter, the splitting by two
+// waves 5.0 (a prompt of 700 tokens, 16 heads, in six pieces 34.2, 25.9 and 30.1 us; the whole scan 106 -> 98).
+template <int KT, int NW>
+__global__ __launch_bounds__(64 * NW, 1) void delta_states_kernel(RunArgs ra) {
   extern __shared__ __align__(16) float planes[];              // [rows / 16][pairs of columns / 16][3][64 lanes][4]
-  constexpr int dk = 16 * KT, J = KT / 2;
+  constexpr int dk = 16 * KT, J = KT / 2, kParts = KT / NW;
   const zp_delta& a = ra.d;
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int h = blockIdx.x % a.heads, seg = blockIdx.x / a.heads;
+  const int unit = blockIdx.x / kParts, h = unit % a.heads, seg = unit / a.heads, mine = blockIdx.x % kParts * NW + wave;
   const Segment whole = segment_of(a.seg, seg);
   if (whole.count <= 0 || whole.row < ra.row0) return;
-  f32x4 S[KT][1], x[KT], add[KT];
-  load_state<KT, 1>(S, a.state + ((int64_t)whole.slot * a.heads + h) * ((int64_t)dk * dk), dk, wave * 16, whole.start == 0);
+  f32x4 S[KT][1], x[kParts][KT], add[KT];
+  load_state<KT, 1>(S, a.state + ((int64_t)whole.slot * a.heads + h) * ((int64_t)dk * dk), dk, mine * 16, whole.start == 0);
   const int tokens = ra.pieces.blocks * kBlock, count = (whole.count + tokens - 1) / tokens;
   const int64_t stride = (int64_t)a.heads * piece_floats(dk);
   float* const at = ra.pieces.states + Piece(ra.pieces, ra.row0, whole, seg, 0).slot * stride + (int64_t)h * piece_floats(dk) + lane * 4;
-  auto load = [&](int c) {                                     // this wave's columns of M, for all waves
+  auto load = [&](int c) {                                     // this wave's share of M's columns, for all waves
 #pragma unroll
-    for (int t = 0; t < KT; ++t) x[t] = *(const f32x4*)(at + c * stride + dk * dk + (t * KT + wave) * 256);
+    for (int u = 0; u < kParts; ++u)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) x[u][t] = *(const f32x4*)(at + c * stride + dk * dk + (t * KT + wave + u * NW) * 256);
   };
   auto meet = [] {                                             // LDS alone: what comes from memory and goes there stays on its way
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  auto load_sums = [&](int c, int t) { add[t] = *(const f32x4*)(at + c * stride + (wave * KT + t) * 256); };
+  auto load_sums = [&](int c, int t) { add[t] = *(const f32x4*)(at + c * stride + (mine * KT + t) * 256); };
   if (count > 1) {
     load(0);
 #pragma unroll
@@ -533,18 +536,21 @@ __global__ __launch_bounds__(64 * KT, 2) void delta_states_kernel(RunArgs ra) {
     meet();                                                    // the planes before these are used up
     if (more) {
 #pragma unroll
-      for (int t = 0; t < KT; ++t) {
-        const Planes p(x[t]);
-        float* const to = planes + (t * J + (wave >> 1)) * 768 + lane * 4 + (wave & 1) * 2;
-        *(uint2*)to = p.hi;
-        *(uint2*)(to + 256) = p.mid;
-        *(uint2*)(to + 512) = p.lo;
-      }
+      for (int u = 0; u < kParts; ++u)
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+          const Planes p(x[u][t]);
+          const int column = wave + u * NW;
+          float* const to = planes + (t * J + (column >> 1)) * 768 + lane * 4 + (column & 1) * 2;
+          *(uint2*)to = p.hi;
+          *(uint2*)(to + 256) = p.mid;
+          *(uint2*)(to + 512) = p.lo;
+        }
       load(min(c + 1, count - 2));
     }
 #pragma unroll
     for (int kt = 0; kt < KT; ++kt) {
-      *(f32x4*)(at + c * stride + (wave * KT + kt) * 256) = S[kt][0];
+      *(f32x4*)(at + c * stride + (mine * KT + kt) * 256) = S[kt][0];
       const Planes p(S[kt][0]);
       const int e = (kt & 1) * 2;
       sp[0][kt >> 1][e] = p.hi.x, sp[0][kt >> 1][e + 1] = p.hi.y;
@@ -874,7 +880,7 @@ template <int KT, int NW> int launch_blocks(const RunArgs& ra, hipStream_t st) {
   if constexpr (KT == NW)
     if (ra.pieces.blocks) {
       int rc = launch_kernel(delta_blocks_kernel<KT, NW, true>, units * (ra.pieces.most - 1) * 2, 64 * NW, smem, ra, st);
-      if (rc == ZP_OK) rc = launch_kernel(delta_states_kernel<KT>, units, 64 * KT, KT * KT / 2 * 3072, ra, st);
+      if (rc == ZP_OK) rc = launch_kernel(delta_states_kernel<KT, KT / 2>, units * 2, 32 * KT, KT * KT / 2 * 3072, ra, st);
       if (rc != ZP_OK) return rc;
     }
   return launch_kernel(delta_blocks_kernel<KT, NW, false>, units * ra.pieces.most, 64 * NW, smem, ra, st);
@@ -920,6 +926,8 @@ static int64_t pairs_bytes(int64_t rows, int64_t segments, int64_t heads, int dk
   return (rows / (2 * kBlock) + segments) * heads * pair_floats(dk, dv) * 4;
 }
 
+// A piece as dear as when its states took 5.7 us: with 18, shorter pieces of 500 and 700 tokens, 16 heads, take 93 and 101 us instead
+// of 86 and 98, what begins and ends them being paid more often.
 constexpr PieceCost kCost = {2, 8, 72, 24};
 
 // With room for the states between pieces of few heads' runs, whatever the longest run.
