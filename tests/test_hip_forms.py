@@ -108,6 +108,33 @@ def test_scores_of_few_sequences(dev, dtype, group, W, BS, D, reduced, B):
     torch.testing.assert_close(many[:, :3].cpu().float(), want.float(), rtol=2.0 ** -6 if dtype != torch.float32 else 1e-4, atol=1e-6)
 
 
+# Units of groups of two and four, up to 128 of them, go in halves of their rows where the selection adds up what they leave and there is
+# room for it: the flags of whole units.
+@pytest.mark.parametrize("dtype,L,B,Hkv,G,W", [(BF16, 1, 1, 8, 4, 32), (BF16, 1, 5, 8, 2, 32), (torch.float16, 1, 3, 8, 4, 32), (BF16, 1, 16, 8, 2, 16),
+                                               (torch.float16, 1, 4, 8, 4, 28), (BF16, 2, 4, 4, 3, 20), (BF16, 1, 9, 5, 4, 5), (BF16, 1, 17, 8, 2, 16)])
+@pytest.mark.parametrize("carry", [False, True])
+def test_scores_in_halves_of_units(dev, monkeypatch, dtype, L, B, Hkv, G, W, carry):
+    from zipage_amd import _lib
+    from zipage_amd.compress import CompressConfig, compress_layers
+    BS, D, budget = 256, 128, 2
+    g = torch.Generator().manual_seed(B * 8 + W)
+    counts = [3 + (b * 3 + 4) % 7 for b in range(B)]
+    pages = torch.randperm(sum(counts), generator=g).tolist()
+    tables = [[pages.pop() for _ in range(n)] for n in counts]
+    enc, target = O.encode_block_table(tables).to(dev), torch.tensor([t[:budget + 1] for t in tables], dtype=torch.int32, device=dev)
+    k, v = (_rand(L, sum(counts), BS, Hkv, D, seed=i, dtype=dtype).to(dev) for i in (1, 2))
+    q = _rand(L, B, W, Hkv * G, D, seed=3, std=2.0, dtype=dtype).to(dev)
+    old = torch.rand((L, sum(counts), BS, Hkv), generator=g).to(dtype).to(dev) if carry else None
+    cfg = CompressConfig(budget_blocks=budget, query_cache_len=W, enable_pooling=True, pooling_size=5, use_global_score=carry)
+    seq, again = torch.arange(B, dtype=torch.int32, device=dev), torch.full((B,), carry, device=dev)
+    run = lambda: [t for x in [(k.clone(), v.clone(), None if old is None else old.clone())]
+                   for t in (compress_layers(x[0], x[1], q, x[2], seq, enc, again, target, cfg), *x) if t is not None]
+    halves, size = run(), _lib.size
+    monkeypatch.setattr(_lib, "size", lambda name, *a: size(name.replace("_layers_workspace_few", "_layers_workspace"), *a))
+    for got, want in zip(halves, run()):
+        assert torch.equal(got, want)
+
+
 # ------------------------------------------------------------------ redundancy inside pages
 # workgroups walk whole rows where 512 of them (fp32: 256), or a multiple, are at least 90 % full (461 rows on), and
 # take a page each otherwise.  Same bits for a sequence alone, in a batch that is walked and in one

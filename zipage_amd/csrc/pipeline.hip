@@ -380,6 +380,8 @@ extern "C" int zp_compress_layers_static(void* k_cache, void* v_cache, const voi
   Plan p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr);
   // the logits of few sequences always fit (at most 16 MB of 23 in all)
   if (p.total > (int64_t)ZP_STATIC_SCRATCH_BYTES)
+    p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr, Scratch::one_sweep);
+  if (p.total > (int64_t)ZP_STATIC_SCRATCH_BYTES)
     p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr, Scratch::floor);
   ZP_REQUIRE(p.total <= (int64_t)ZP_STATIC_SCRATCH_BYTES,
              "compress_layers_static: this chunk needs %lld bytes of scratch, the library's array "

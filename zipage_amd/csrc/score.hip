@@ -836,6 +836,20 @@ __device__ __forceinline__ float group_window_reduce(float (&pv)[16], int Gp, bo
   return red;
 }
 
+// The same of half of the rows, in groups of two or four, as far as group_window_reduce adds them up before the halves of the
+// wave: (first half's + second half's rows) of one half of the wave + those of the other are its sums.
+template <typename T, int GP> __device__ __forceinline__ float half_window_sum(const float (&pv)[8]) {
+  float t[8 / GP];
+#pragma unroll
+  for (int q = 0; q < 8 / GP; ++q)
+    t[q] = exp2_hw(GP == 4 ? vmax4(pv[4 * q], pv[4 * q + 1], pv[4 * q + 2 < 8 ? 4 * q + 2 : 0], pv[4 * q + 3 < 8 ? 4 * q + 3 : 0])
+                           : vmax(pv[2 * q], pv[2 * q + 1]));
+#pragma unroll
+  for (int q = 0; q < 8 / GP; q += 2) Rnd<T>::pair(t[q], t[q + 1]);
+  if constexpr (GP == 4) return t[0] + t[1];
+  else return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
 // Every wave builds the list of usable pages for itself (no LDS, no barrier): `code` is table entry `lane`, a ballot ranks
 // the usable ones, and a lane permute leaves entry n of the list in lane n as (page id, table index | last << 30).  Returns
 // their number.
@@ -853,12 +867,15 @@ __device__ __forceinline__ int list_pages(int code, int num_pages, int2& mine) {
 
 // TPP: 128-token tiles per page when known at compile time (0: from the arguments); with it
 // the page of every unrolled tile is a constant and its id comes from a lane of a register.
-template <typename T, int GPC, int RMAXC, int TPP>
+// SPLIT 2: a workgroup multiplies all 32 rows of a unit and goes on with half of them; see kSplitUnits.
+template <typename T, int GPC, int RMAXC, int TPP, int SPLIT>
 __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p) {
   typedef Mma<T> M;
   typedef typename M::Frag Frag;
   typedef Pack2<T> P2;
   constexpr int KS = M::KS;   // 8 contraction steps of 16
+  constexpr int R = 16 / SPLIT;                // rows of a lane
+  static_assert(SPLIT == 1 || (SPLIT == 2 && RMAXC == 0 && (GPC == 2 || GPC == 4)), "halves whose windows are added up");
   const int GpV = GPC > 0 ? GPC : p.Gp;
   const int gsV = GPC == 8 ? 3 : GPC == 4 ? 2 : GPC == 2 ? 1 : p.gs;
   const bool rmaxV = RMAXC >= 0 ? (RMAXC != 0) : (p.reduce_max != 0);
@@ -885,8 +902,9 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   // of an item get consecutive ids ON ONE XCD, so they run at the same time behind one L2 and
   // the item's keys leave HBM once
   const int xcd = blockIdx.x & 7, loc = blockIdx.x >> 3;
-  const int rb = loc % p.RB;
-  const int item = (loc / p.RB) * 8 + xcd;
+  const int part_of = SPLIT == 1 ? 0 : loc % SPLIT, unit = loc / SPLIT;
+  const int rb = unit % p.RB;
+  const int item = (unit / p.RB) * 8 + xcd;
   if (item >= p.n_items) return;
   const int h = item % p.Hkv;
   const int b = (item / p.Hkv) % p.B;
@@ -953,7 +971,7 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   // ---- A fragments: the 32 query rows of this block, in registers for the whole sweep
   Frag afrag[KS];
   {
-    const int mrow = rb * 32 + col;
+    const int mrow = rb * 32 + ((col + part_of * (32 / SPLIT)) & 31);      // this part's rows first
     const int a_w = mrow >> gsV, a_g = mrow & (GpV - 1);
     const bool a_ok = seq_ok && a_w < p.W && a_g < p.G;
     const char* qrow = p.q + ((int64_t)l * p.q_sl + (int64_t)seq * p.q_ss +
@@ -972,11 +990,11 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(afrag[s]));
 
   ZP_STAMP();
-  const int row0 = rb * 32 + half * 4;   // rows of this lane: row0 + (r/4)*8 + r%4
-  uint32_t lg[kResTiles * 8];
-  float run[16];
+  const int row0 = rb * 32 + part_of * (32 / SPLIT) + half * 4;   // rows of this lane: row0 + (r/4)*8 + r%4
+  uint32_t lg[kResTiles * (R / 2)];
+  float run[R];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) run[r] = -INFINITY;
+  for (int r = 0; r < R; ++r) run[r] = -INFINITY;
 
   // ---- the sweep: products, causal mask, running maximum, rounded logits into registers.
   // Software-pipelined inside the wave: the products of block it+1 are issued before the
@@ -1023,16 +1041,16 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
       if (((vs >> 30) & 1) && (toff + 31 > p.BS - p.W)) {   // causal mask: tail of the last page
         const int slot = toff + col;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+        for (int r = 0; r < R; ++r) {
           const int w = (row0 + (r >> 2) * 8 + (r & 3)) >> gsV;
           if (slot > p.BS - p.W + w) acc[r] = -INFINITY;
         }
       }
 #pragma unroll
-      for (int r = 0; r < 16; ++r) run[r] = vmax(run[r], acc[r]);
+      for (int r = 0; r < R; ++r) run[r] = vmax(run[r], acc[r]);
 #pragma unroll
-      for (int r = 0; r < 16; r += 2)
-        lg[it * 8 + (r >> 1)] = P2::pack(acc[r] * p.scale, acc[r + 1] * p.scale);
+      for (int r = 0; r < R; r += 2)
+        lg[it * (R / 2) + (r >> 1)] = P2::pack(acc[r] * p.scale, acc[r + 1] * p.scale);
       if (it + 1 < ntiles) acc_cur = acc_next;
     }
   }
@@ -1040,16 +1058,16 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   ZP_STAMP();
   // ---- row maximum over the lanes of a row and the four waves
   auto row_slot = [&](int r) { return (r >> 2) * 8 + half * 4 + (r & 3); };
-  float mx[16];
+  float mx[R];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < R; ++r) {
     const float v = half_max(run[r]);
     run[r] = v;
     if (col == 0) stat[wave * 32 + row_slot(r)] = v;
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < R; ++r) {
     float v = run[r];
 #pragma unroll
     for (int w2 = 1; w2 < kWaves; ++w2) v = fmaxf(v, stat[((wave + w2) % kWaves) * 32 + row_slot(r)]);
@@ -1060,31 +1078,31 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
   ZP_STAMP();
   // ---- x = rounded(logit - max) back into the registers, row sums of exp(x)
 #pragma unroll
-  for (int r = 0; r < 16; ++r) run[r] = 0.f;
+  for (int r = 0; r < R; ++r) run[r] = 0.f;
 #pragma unroll
   for (int it = 0; it < kResTiles; ++it) {
     if (it < ntiles) {
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const uint32_t w = lg[it * 8 + q];
+      for (int q = 0; q < R / 2; ++q) {
+        const uint32_t w = lg[it * (R / 2) + q];
         const uint32_t x = P2::pack(P2::lo(w) - mx[2 * q], P2::hi(w) - mx[2 * q + 1]);
-        lg[it * 8 + q] = x;
+        lg[it * (R / 2) + q] = x;
         run[2 * q] += exp_neg(P2::lo(x));
         run[2 * q + 1] += exp_neg(P2::hi(x));
       }
     }
   }
   ZP_STAMP();
-  float cl[16];
+  float cl[R];
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < R; ++r) {
     const float v = half_sum(run[r]);
     run[r] = v;
     if (col == 0) stat[wave * 32 + row_slot(r)] = v;
   }
   __syncthreads();
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
+  for (int r = 0; r < R; ++r) {
     // the four waves' sums are added in wave order, whichever wave does it
     float v = stat[row_slot(r)];
 #pragma unroll
@@ -1096,22 +1114,25 @@ __global__ __launch_bounds__(kThreads, 2) void score_resident_kernel(ScoreArgs p
 
   ZP_STAMP();
   // ---- output: p = 2^(x log2(e) - log2(sum)), group maximum, this block's share of the window sum
-  float* part = p.part + ((int64_t)item * p.RB + rb) * Tn + wtok + col;
+  // SPLIT: by halves of the wave, and of the rows within
+  float* part = p.part + ((int64_t)(item * p.RB + rb) * (SPLIT * SPLIT) + (SPLIT > 1 ? half * SPLIT + part_of : 0)) * Tn + wtok + col;
 #pragma unroll
   for (int it = 0; it < kResTiles; ++it) {
     if (it < ntiles) {
-      float pv[16];
+      float pv[R];
 #pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const uint32_t x = lg[it * 8 + q];
+      for (int q = 0; q < R / 2; ++q) {
+        const uint32_t x = lg[it * (R / 2) + q];
         pv[2 * q] = __builtin_fmaf(P2::lo(x), 1.44269504088896340736f, cl[2 * q]);
         pv[2 * q + 1] = __builtin_fmaf(P2::hi(x), 1.44269504088896340736f, cl[2 * q + 1]);
       }
-      const float red = group_window_reduce<T>(pv, GpV, rmaxV);
+      float red;
+      if constexpr (SPLIT == 1) red = group_window_reduce<T>(pv, GpV, rmaxV);
+      else red = half_window_sum<T, GPC>(pv);
       const int vp = tile_page(it);
       const int j = page_word(myinfo.y, vp) & 0xffff;
       const int toff = (it - vp * tiles_per_page) * 128;
-      if (half == 0) __builtin_nontemporal_store(red, part + j * p.BS + toff);
+      if (SPLIT > 1 || half == 0) __builtin_nontemporal_store(red, part + j * p.BS + toff);
     }
   }
   ZP_STAMP();
@@ -1808,6 +1829,21 @@ static int64_t tiled_need(int L, int B, int NB, int BS, int Hkv, int Hq, int W, 
   return units * NB * BS * (64 + (dtype == ZP_F32 ? 4 : 8) * 4);      // logits, and partials of a unit's quarters
 }
 
+// Units of which not every other CU has one go in halves of their rows, where the epilogue is a straight line and the selection adds
+// up what they leave: a workgroup's vector work is what a unit takes 24 us for, and half of it leaves the same bits, as rows are
+// apart up to the sums over windows; all products are made twice, which the matrix cores have time for.  Whole steps of 9 and 10
+// pages, us whole (or in tiles) and in halves: groups of four, window 32, 96 units 48.2 and 43.5, 128 50.6 and 46.6, but 192 59.5 and
+// 64.9; groups of two, window 16, 128 units 88.8 and 83.1, 256 139.1 and 140.8.  Against tiles, which the keys' blocks of a row are
+// spread in as well, where an item has two units: 32 of them 37.9 and 39.2 (tiles first), 48 42.0 and 41.1, 64 47.1 and 44.6; four: 32 39.2
+// and 35.7, 64 42.1 and 41.0; one: 16 35.5 and 38.3, 64 57.1 and 57.3.
+constexpr int64_t kSplitUnits = 128;      // of two workgroups
+static int64_t split_need(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype, bool reduce_max) {
+  const int64_t whole = dtype == ZP_F32 ? 0 : resident_need(L, B, NB, BS, Hkv, Hq, W, dtype);
+  if (!whole || reduce_max || BS != 256) return 0;
+  const int Gp = pow2_ceil(Hq / Hkv);
+  return (Gp == 2 || Gp == 4) && (int64_t)L * B * Hkv * ((W * Gp + 31) / 32) <= kSplitUnits ? 4 * whole : 0;
+}
+
 extern "C" int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                                     int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype) {
   if (Hkv <= 0 || Hq <= 0 || L < 0 || B < 0 || NB <= 0 || BS <= 0 || W <= 0) return 0;
@@ -1820,7 +1856,7 @@ extern "C" int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_
 extern "C" int64_t zp_attention_score_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                                     int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype) {
   const int64_t usual = zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, dtype);
-  return usual <= 0 ? usual : std::max(usual, tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype));
+  return usual <= 0 ? usual : std::max({usual, tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype), split_need(L, B, NB, BS, Hkv, Hq, W, dtype, false)});
 }
 
 extern "C" int64_t zp_attention_score_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS,
@@ -1905,13 +1941,16 @@ static int attention_score(const void* k_cache, const void* query_cache,
   a.n_items = L * B * Hkv;
   a.part = (float*)workspace;
   auto leave = [&] {
-    if (left) *left = ScoreParts{a.part, a.RB, W, a.reduce_max};
+    if (left) *left = ScoreParts{a.part, a.RB, W, a.reduce_max, 1};
     return left != nullptr;
   };
   const int64_t tiled = tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype);
   const bool straight = BS == 256 && !a.reduce_max && (Gp == 2 || Gp == 4);
   const int64_t walks = (int64_t)a.n_items * (resident32 ? (W * Gp + 15) / 16 : RB);
-  if ((resident || resident32) && tiled && workspace_bytes >= tiled && !(straight && NB <= kShortPages && walks > kFewUnitsShort)) {
+  const int64_t split = split_need(L, B, NB, BS, Hkv, Hq, W, dtype, a.reduce_max);
+  const bool halves = resident && left && split && workspace_bytes >= split;
+  if ((resident || resident32) && tiled && workspace_bytes >= tiled && !(straight && NB <= kShortPages && walks > kFewUnitsShort) &&
+      !(halves && RB >= 2 && walks >= (RB >= 4 ? 32 : 33))) {
     if (resident32) a.RB = (W * Gp + 15) / 16;
     a.tiles = NB * (BS / (resident ? 128 : 64));
     a.lg = (char*)workspace + walks * NB * BS * (resident ? 32 : 16);
@@ -1933,22 +1972,25 @@ static int attention_score(const void* k_cache, const void* query_cache,
   }
   if (resident) {
     const size_t smem = (size_t)kWaves * 2 * kSubBytes + sizeof(float) * kWaves * 32;
-    const unsigned units = (unsigned)(((int64_t)a.n_items + 7) / 8 * 8 * RB);
+    const unsigned units = (unsigned)(((int64_t)a.n_items + 7) / 8 * 8 * RB * (halves ? 2 : 1));
     const dim3 cgrid((unsigned)a.n_items, (unsigned)((NB * BS / 4 + 255) / 256));
     // The common groups get straight-line epilogues (groups of two, window 32, the whole compression step: 1 sequence
     // 53 -> 42 us, 64 sequences 330 -> 312, 200 1039 -> 1009).
 #define ZP_RESIDENT_LAUNCH(TT)                                                                   \
   do {                                                                                           \
-    void (*fn)(ScoreArgs) = score_resident_kernel<TT, 0, -1, 0>;                                 \
-    if (Gp == 4 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 4, 0, 2>;          \
-    else if (Gp == 2 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 2, 0, 2>;     \
+    void (*fn)(ScoreArgs) = score_resident_kernel<TT, 0, -1, 0, 1>;                              \
+    if (halves && Gp == 4) fn = score_resident_kernel<TT, 4, 0, 2, 2>;                           \
+    else if (halves) fn = score_resident_kernel<TT, 2, 0, 2, 2>;                                 \
+    else if (Gp == 4 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 4, 0, 2, 1>;  \
+    else if (Gp == 2 && !a.reduce_max && BS == 256) fn = score_resident_kernel<TT, 2, 0, 2, 1>;  \
     if (hipFuncSetAttribute((const void*)fn, hipFuncAttributeMaxDynamicSharedMemorySize,         \
                             (int)smem) != hipSuccess) {                                          \
       zp_set_error("attention_score: cannot reserve %zu bytes of LDS", smem);                    \
       return ZP_EHIP;                                                                            \
     }                                                                                            \
     hipLaunchKernelGGL(fn, dim3(units), dim3(kThreads), smem, st, a);                            \
-    if (!leave())                                                                                \
+    if (leave()) left->shares = halves ? 4 : 1;                                                  \
+    else                                                                                         \
       hipLaunchKernelGGL((score_combine_kernel<TT, 1>), cgrid, dim3(256), 0, st, a.part, scores_out, \
                        block_table, B, NB, BS, Hkv, RB, W, num_pages, a.reduce_max, Gp);         \
   } while (0)

@@ -246,19 +246,28 @@ __device__ __forceinline__ void stage_left(const LeftArgs& p, uint32_t r, int b,
     code[u] = p.table[(int64_t)b * p.NB + at[u] / p.BS];
   }
   if constexpr (PARTS) {
-    const float* const part = p.parts.part + (int64_t)r * p.parts.RB * Tn;
-    for (int r0 = 0; r0 < p.parts.RB; r0 += kBlocks) {
+    const int rows = p.parts.RB * p.parts.shares;
+    const float* const part = p.parts.part + (int64_t)r * rows * Tn;
+    for (int r0 = 0; r0 < rows; r0 += kBlocks) {
       f4 x[kPieces][kBlocks];
 #pragma unroll
       for (int u = 0; u < kPieces; ++u)
 #pragma unroll
         for (int k = 0; k < kBlocks; ++k)
-          x[u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)min(r0 + k, p.parts.RB - 1) * Tn + at[u]));
+          x[u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)min(r0 + k, rows - 1) * Tn + at[u]));
+      if (p.parts.shares == kBlocks) {                        // sums
+#pragma unroll
+        for (int u = 0; u < kPieces; ++u) {
+          const f4 block = (x[u][0] + x[u][1]) + (x[u][2] + x[u][3]);
+          v[u] = r0 == 0 ? block : v[u] + block;
+        }
+        continue;
+      }
 #pragma unroll
       for (int u = 0; u < kPieces; ++u)
 #pragma unroll
         for (int k = 0; k < kBlocks; ++k) {
-          if (r0 + k >= p.parts.RB) break;
+          if (r0 + k >= rows) break;
           v[u] = r0 + k == 0 ? x[u][k] : join(v[u], x[u][k]);
         }
     }
