@@ -114,12 +114,13 @@ __global__ __launch_bounds__(NT) void compact_kernel(CompactArgs p) {
   const int l = item / (p.Hkv * p.B);
 
   // a thread's flags are asked for with the tables, where a few registers hold them, and not twice one after the other (two fp32
-  // sequences 17.6 -> 16.9 us, eight bfloat16 ones 29.3 -> 28.5)
+  // sequences 17.6 -> 16.9 us, eight bfloat16 ones 29.3 -> 28.5).  Not where keys and values share workgroups, which are enough of them to
+  // hide it (256 bfloat16 sequences 823 us, and 827)
   const int chunk = (T + NT - 1) / NT;
   const int s0 = min(tid * chunk, T), s1 = min(s0 + chunk, T);
   const uint8_t* f = p.flag + (((int64_t)l * p.B + b) * p.Hkv + h) * (int64_t)T;
   constexpr int kHeld = kWide ? 4 : 12;
-  const bool holds = chunk <= kHeld;
+  const bool holds = !HAS_B && chunk <= kHeld;
   uint8_t held[kHeld];
   if (holds)
 #pragma unroll
