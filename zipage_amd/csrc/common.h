@@ -45,7 +45,7 @@ int64_t zp_attention_score_workspace_floor(int32_t L, int32_t B, int32_t NB, int
 struct ScoreParts {
   const float* part = nullptr;
   int RB = 0, W = 0, rmax = 0;
-  int shares = 1;                    // of a block: 4 are added up in pairs first
+  int shares = 1;                    // of a block, or 4, sums that are added up in pairs first
 };
 int zp_attention_score_parts(const void* k_cache, const void* query_cache, const int32_t* seq_idx, const int32_t* block_table,
                              void* scores_out, int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,

@@ -1963,8 +1963,10 @@ static int attention_score(const void* k_cache, const void* query_cache,
     ZP_DISPATCH_DTYPE(dtype, {
       if (BS == 256) ZP_TILED_LAUNCH(T::bytes == 2 ? 2 : 4);
       else ZP_TILED_LAUNCH(0);
-      hipLaunchKernelGGL((score_combine_kernel<T, T::bytes == 2 ? 8 : 4>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
-                         B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max, Gp);
+      if (T::bytes == 4 && !a.reduce_max && Gp < 8 && leave()) left->shares = 4;      // sums in pairs, as of halves
+      else
+        hipLaunchKernelGGL((score_combine_kernel<T, T::bytes == 2 ? 8 : 4>), cgrid, dim3(256), 0, st, a.part, scores_out, block_table,
+                           B, NB, BS, Hkv, a.RB, W, num_pages, a.reduce_max, Gp);
     });
 #undef ZP_TILED_LAUNCH
     ZP_LAUNCH_CHECK();

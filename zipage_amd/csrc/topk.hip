@@ -197,6 +197,8 @@ struct LeftArgs : SelectArgs {        // a row as the scorer left it: see ScoreP
   CarriedScores carried;
   int num_pages;
 };
+struct SharesArgs : LeftArgs {};      // of blocks in shares; apart, as two of these are on their way at once, for which a full chip's rows
+                                      // have no registers (whole steps of 256 bf16 sequences 1300 us, 1308 with both in one kernel)
 
 // Row -> LDS as fp32, 16 bytes per thread per step when the row allows it.
 template <typename T>
@@ -229,7 +231,7 @@ __device__ __forceinline__ void stage_row(const void* __restrict__ src, int64_t 
 // where launches of their own would.  Bound by the partials' way from memory: all tokens' loads of four blocks are side by side (one
 // token's after another's, 64 bf16 sequences 14.0 us, now 13.5; 256 without earlier scores 32.0, now 24.6; 4 with 13.4, now 9.6).
 constexpr int kPer = 10;             // tokens of a thread whose keys stay in registers
-template <typename T, bool PARTS>
+template <typename T, int PARTS>        // 0: none, 1: of a block, 2: of its four shares
 __device__ __forceinline__ void stage_left(const LeftArgs& p, uint32_t r, int b, int Tn, float* __restrict__ row) {
   constexpr int kPieces = (kPer + 3) / 4, kBlocks = 4;      // of four tokens; whose loads are side by side
   const int h = (int)(r % (uint32_t)p.Hkv), l = (int)(r / ((uint32_t)p.Hkv * (uint32_t)p.B));
@@ -245,31 +247,45 @@ __device__ __forceinline__ void stage_left(const LeftArgs& p, uint32_t r, int b,
     at[u] = min((u * kThreads + (int)threadIdx.x) * 4, Tn - 4);
     code[u] = p.table[(int64_t)b * p.NB + at[u] / p.BS];
   }
-  if constexpr (PARTS) {
-    const int rows = p.parts.RB * p.parts.shares;
-    const float* const part = p.parts.part + (int64_t)r * rows * Tn;
-    for (int r0 = 0; r0 < rows; r0 += kBlocks) {
+  if constexpr (PARTS == 1) {
+    const float* const part = p.parts.part + (int64_t)r * p.parts.RB * Tn;
+    for (int r0 = 0; r0 < p.parts.RB; r0 += kBlocks) {
       f4 x[kPieces][kBlocks];
 #pragma unroll
       for (int u = 0; u < kPieces; ++u)
 #pragma unroll
         for (int k = 0; k < kBlocks; ++k)
-          x[u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)min(r0 + k, rows - 1) * Tn + at[u]));
-      if (p.parts.shares == kBlocks) {                        // sums
-#pragma unroll
-        for (int u = 0; u < kPieces; ++u) {
-          const f4 block = (x[u][0] + x[u][1]) + (x[u][2] + x[u][3]);
-          v[u] = r0 == 0 ? block : v[u] + block;
-        }
-        continue;
-      }
+          x[u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)min(r0 + k, p.parts.RB - 1) * Tn + at[u]));
 #pragma unroll
       for (int u = 0; u < kPieces; ++u)
 #pragma unroll
         for (int k = 0; k < kBlocks; ++k) {
-          if (r0 + k >= rows) break;
+          if (r0 + k >= p.parts.RB) break;
           v[u] = r0 + k == 0 ? x[u][k] : join(v[u], x[u][k]);
         }
+    }
+  }
+  if constexpr (PARTS == 2) {           // sums: of a block's shares in pairs, then of blocks
+    const int rows = p.parts.RB * kBlocks;
+    const float* const part = p.parts.part + (int64_t)r * rows * Tn;
+    f4 x[2][kPieces][kBlocks];
+    for (int r0 = 0; r0 < rows; r0 += 2 * kBlocks) {
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        if (r0 + n * kBlocks < rows)
+#pragma unroll
+          for (int u = 0; u < kPieces; ++u)
+#pragma unroll
+            for (int k = 0; k < kBlocks; ++k)
+              x[n][u][k] = __builtin_nontemporal_load((const f4*)(part + (int64_t)(r0 + n * kBlocks + k) * Tn + at[u]));
+#pragma unroll
+      for (int n = 0; n < 2; ++n)
+        if (r0 + n * kBlocks < rows)
+#pragma unroll
+          for (int u = 0; u < kPieces; ++u) {
+            const f4 block = (x[n][u][0] + x[n][u][1]) + (x[n][u][2] + x[n][u][3]);
+            v[u] = r0 + n == 0 ? block : v[u] + block;
+          }
     }
   }
 #pragma unroll
@@ -278,8 +294,8 @@ __device__ __forceinline__ void stage_left(const LeftArgs& p, uint32_t r, int b,
     if (t >= Tn) break;
     const int pid = page_is_pad(code[u]) ? -1 : page_id(code[u]);
     const bool there = pid >= 0 && pid < p.num_pages;
-    if constexpr (PARTS) {
-      if (!p.parts.rmax)
+    if constexpr (PARTS > 0) {
+      if (PARTS == 2 || !p.parts.rmax)
 #pragma unroll
         for (int i = 0; i < 4; ++i) v[u][i] = Elem<T>::rnd(v[u][i] / (float)p.parts.W);
       if (!there) v[u] = f4{0.f, 0.f, 0.f, 0.f};
@@ -374,8 +390,9 @@ __global__ __launch_bounds__(kThreads) void select_reg_kernel(Args p) {
   const uint8_t was_compressed = p.compressed[b];
   for (int i = tid; i < p.NB + 2; i += kThreads) trow[i] = i < p.NB ? p.table[(int64_t)b * p.NB + i] : -1;
   if constexpr (std::is_same_v<Args, SelectArgs>) stage_row<T>(p.scores, base, Tn, row);
-  else if (p.parts.part) stage_left<T, true>(p, r, b, Tn, row);
-  else stage_left<T, false>(p, r, b, Tn, row);
+  else if constexpr (std::is_same_v<Args, SharesArgs>) stage_left<T, 2>(p, r, b, Tn, row);
+  else if (p.parts.part) stage_left<T, 1>(p, r, b, Tn, row);
+  else stage_left<T, 0>(p, r, b, Tn, row);
   {
     const float neutral = POOLK > 0 ? -INFINITY : 0.f;
     if (tid < kSelPad) row[tid - kSelPad] = neutral;
@@ -617,7 +634,7 @@ static int select_topk(const void* scores, void* scores_out, const void* redunda
   if (L == 0 || B == 0) return ZP_OK;
   ZP_REQUIRE((scores || parts.part) && flag_out && block_table && compressed, "select_topk: null pointer");
   hipStream_t st = (hipStream_t)stream;
-  LeftArgs p;
+  SharesArgs p;
   p.parts = parts; p.carried = carried; p.num_pages = num_pages;
   p.scores = scores; p.scores_out = scores_out; p.red = redundancy; p.flag = flag_out;
   p.table = block_table; p.compressed = compressed;
@@ -659,7 +676,7 @@ static int select_topk(const void* scores, void* scores_out, const void* redunda
       ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_REG_ALL());
       return ZP_OK;
     };
-    const int rc = parts.part || carried.cache ? launch(&p) : launch((SelectArgs*)&p);
+    const int rc = parts.part && parts.shares > 1 ? launch(&p) : parts.part || carried.cache ? launch((LeftArgs*)&p) : launch((SelectArgs*)&p);
     if (rc != ZP_OK) return rc;
   } else {
     ZP_DISPATCH_DTYPE(dtype, ZP_SELECT_LAUNCH((select_lds_kernel<T>), p));
