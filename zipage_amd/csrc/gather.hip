@@ -116,15 +116,15 @@ __global__ __launch_bounds__(NT) void compact_kernel(CompactArgs p) {
   // a thread's flags are asked for with the tables, where a few registers hold them, and not twice one after the other (two fp32
   // sequences 17.6 -> 16.9 us, eight bfloat16 ones 29.3 -> 28.5).  Not where keys and values share workgroups, which are enough of them to
   // hide it (256 bfloat16 sequences 823 us, and 827)
-  const int chunk = (T + NT - 1) / NT;
-  const int s0 = min(tid * chunk, T), s1 = min(s0 + chunk, T);
-  const uint8_t* f = p.flag + (((int64_t)l * p.B + b) * p.Hkv + h) * (int64_t)T;
-  constexpr int kHeld = kWide ? 4 : 12;
-  const bool holds = !HAS_B && chunk <= kHeld;
+  constexpr int kHeld = HAS_B ? 1 : kWide ? 4 : 12;
   uint8_t held[kHeld];
-  if (holds)
+  if constexpr (!HAS_B) {
+    const int per = (T + NT - 1) / NT, from = min(tid * per, T);
+    const uint8_t* f = p.flag + (((int64_t)l * p.B + b) * p.Hkv + h) * (int64_t)T;
+    if (per <= kHeld)
 #pragma unroll
-    for (int i = 0; i < kHeld; ++i) held[i] = f[min(s0 + i, T - 1)];
+      for (int i = 0; i < kHeld; ++i) held[i] = f[min(from + i, T - 1)];
+  }
   for (int i = tid; i < p.NB; i += NT) {
     int code = p.table[(int64_t)b * p.NB + i];
     int pid = page_is_pad(code) ? -1 : page_id(code);
@@ -137,26 +137,33 @@ __global__ __launch_bounds__(NT) void compact_kernel(CompactArgs p) {
   __syncthreads();
 
   // ---- phase 1: ordered survivor list
+  const int chunk = (T + NT - 1) / NT;
+  const int s0 = min(tid * chunk, T), s1 = min(s0 + chunk, T);
+  const uint8_t* f = p.flag + (((int64_t)l * p.B + b) * p.Hkv + h) * (int64_t)T;
   int cnt = 0;
-  uint32_t kept = 0;
   auto page_of = [&](int s) { return POW2 ? (s >> p.bs_shift) : (s / p.BS); };
-  if (holds) {
+  auto list_flags = [&] {
+    for (int s = s0; s < s1; ++s) cnt += (f[s] != 0 && tab[page_of(s)] >= 0) ? 1 : 0;
+    int total;
+    int off = block_exclusive_scan<NT>(cnt, &total, scan_lds);
+    for (int s = s0; s < s1; ++s)
+      if (f[s] != 0 && tab[page_of(s)] >= 0) list[off++] = (uint16_t)s;
+    return total;
+  };
+  int total;
+  if constexpr (HAS_B) {
+    total = list_flags();
+  } else if (chunk > kHeld) {
+    total = list_flags();
+  } else {
+    uint32_t kept = 0;
 #pragma unroll
     for (int i = 0; i < kHeld; ++i)
       if (s0 + i < s1 && held[i] != 0 && tab[page_of(s0 + i)] >= 0) kept |= 1u << i;
-    cnt = __popc(kept);
-  } else {
-    for (int s = s0; s < s1; ++s) cnt += (f[s] != 0 && tab[page_of(s)] >= 0) ? 1 : 0;
-  }
-  int total;
-  int off = block_exclusive_scan<NT>(cnt, &total, scan_lds);
-  if (holds) {
+    int off = block_exclusive_scan<NT>(__popc(kept), &total, scan_lds);
 #pragma unroll
     for (int i = 0; i < kHeld; ++i)
       if (kept >> i & 1) list[off++] = (uint16_t)(s0 + i);
-  } else {
-    for (int s = s0; s < s1; ++s)
-      if (f[s] != 0 && tab[page_of(s)] >= 0) list[off++] = (uint16_t)s;
   }
   __syncthreads();
   const int cap = p.target_width * p.BS;
