@@ -16,8 +16,8 @@ def _rand(*shape, seed, std=1.0, dtype=BF16):
 
 
 # ------------------------------------------------------------------ compaction
-# pairs of (row, tensor): up to 512 take workgroups of sixteen waves, up to 256 workgroups are cut by columns of at
-# least 128 bytes; 513 and more take the general form
+# pairs of (row, tensor): up to 512 take workgroups of sixteen waves, up to 256 workgroups are cut by columns; 513 and
+# more take the general form
 @pytest.mark.parametrize("dtype,L,B,Hkv,D", [(torch.float32, 1, 1, 1, 256), (torch.float32, 1, 1, 8, 128), (BF16, 1, 1, 2, 128),
                                              (BF16, 2, 8, 8, 128), (torch.float16, 1, 32, 8, 64), (BF16, 1, 33, 8, 64),
                                              (BF16, 1, 2, 3, 48), (torch.float32, 1, 16, 8, 64)])
@@ -42,6 +42,29 @@ def test_compaction_of_few_rows(dev, dtype, L, B, Hkv, D, style):
     compress_kv(gk, gv, flag.to(dev), enc.to(dev), target.to(dev))
     assert torch.equal(gk.cpu().view(torch.uint8), wk.view(torch.uint8))
     assert torch.equal(gv.cpu().view(torch.uint8), wv.view(torch.uint8))
+
+
+# columns of 32 bytes where a row's workgroups share an XCD, which multiples of eight pairs do, and of whole lines elsewhere;
+# rounds of half as many pieces up to 8192 of them: exactly as many, and a page more
+@pytest.mark.parametrize("dtype,Hkv,D,width", [(BF16, 4, 128, 128), (BF16, 4, 128, 129), (torch.float32, 4, 128, 64), (BF16, 3, 128, 32),
+                                               (BF16, 3, 128, 33), (torch.float32, 12, 64, 61), (torch.float16, 8, 32, 40)])
+def test_compaction_in_parts_of_lines(dev, dtype, Hkv, D, width):
+    from zipage_amd.kernel import compress_kv
+    BS, NB = 32, width + 2
+    g = torch.Generator().manual_seed(width)
+    table = torch.randperm(NB + 3, generator=g).tolist()
+    enc = O.encode_block_table([table[:NB]])
+    target = torch.tensor([[table[NB]] + table[1:width]], dtype=torch.int32)
+    k, v = (_rand(1, NB + 3, BS, Hkv, D, seed=s, dtype=dtype) for s in (1, 2))
+    flag = torch.zeros(1, 1, Hkv, NB * BS, dtype=torch.bool)
+    for h in range(Hkv):                                                 # the first of as many as there is room for
+        flag[0, 0, h, torch.randperm(NB * BS, generator=g)[:width * BS - 7 * h]] = True
+    flag = flag.view(1, 1, Hkv, NB, BS)
+    wk, wv = k.clone(), v.clone()
+    O.compress_kv(wk, wv, flag, enc, target)
+    gk, gv = k.to(dev), v.to(dev)
+    compress_kv(gk, gv, flag.to(dev), enc.to(dev), target.to(dev))
+    assert torch.equal(gk.cpu().view(torch.uint8), wk.view(torch.uint8)) and torch.equal(gv.cpu().view(torch.uint8), wv.view(torch.uint8))
 
 
 # the list of 65 536 tokens and its pages, which fill the LDS but for 16 or 64 bytes: the former leaves no room for the

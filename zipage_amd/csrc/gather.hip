@@ -104,8 +104,9 @@ __global__ __launch_bounds__(NT) void compact_kernel(CompactArgs p) {
   // works on one head's 256-byte slice of the token rows.  Measured against giving each XCD a
   // contiguous range of items (all heads of a sequence on one XCD: 2.5 % slower) and against
   // rotating the head index by the sequence index (4 % slower), inside one allocation.
-  const int part = kWide ? (int)blockIdx.x % p.parts : 0;
-  const int unit = kWide ? (int)blockIdx.x / p.parts : (int)blockIdx.x;
+  const int pairs = 2 * p.n_items;             // wide: column ranges of a pair are a multiple of 8 apart where pairs are, on one XCD
+  const int part = kWide ? (int)blockIdx.x / pairs : 0;
+  const int unit = kWide ? (int)blockIdx.x % pairs : (int)blockIdx.x;
   const int which = (!HAS_B && p.split_kv && unit >= p.n_items) ? 1 : 0;
   const int item = unit - which * p.n_items;
   if (item >= p.n_items) return;
@@ -284,18 +285,29 @@ inline bool aligned_to(int64_t v, int n) { return (v % n) == 0; }
 
 // Few rows leave most of the chip idle, and a row is a chain of rounds (2 048 fp32 vectors of one tensor: sixteen
 // of 64 KB).  So up to kWideUnits (row, tensor) pairs get workgroups of sixteen waves, and a pair is cut into column
-// ranges of at least a cache line while that leaves at most one workgroup per CU.  Whole steps of one layer, general
+// ranges while that leaves at most one workgroup per CU.  Whole steps of one layer, general
 // -> wide form: 1 fp32 sequence of 8 heads 110 -> 59 us, 8 of them 130 -> 99, 32 of them (512 pairs) 323 -> 314; 1
 // bfloat16 sequence 64 -> 42, 16 of them 101 -> 91, 32 of them 171 -> 163.  At 1 024 pairs the general form has four
 // workgroups per CU and the wide one is within 1 % either way; cutting beyond 256 workgroups loses 1-3 %.
 // Returns the column ranges, 0: the general form, also for the longest lists, which leave no room for the sums of sixteen
 // waves beside them.
-constexpr int kWideUnits = 512, kWideGrid = 256, kLinePieces = 8, kLds = 160 * 1024;
+// Ranges are less than a line where a pair's meet in one L2: a workgroup's time is its rounds and the lines that it asks its
+// L1 for, and the latter are spread over more of them (compaction of one bf16 sequence 11.8 us in lines; 10.1 in halves, 8.8 in
+// quarters; two 13.5, 11.2, 10.9; one fp32 14.6, 13.6, 13.3; with halves on different XCDs one bf16 13.5, two 17.1).
+constexpr int kWideUnits = 512, kWideGrid = 256, kLinePieces = 8, kLeastPieces = 2, kLds = 160 * 1024;
 inline int wide_parts(int64_t pairs, int lpv, size_t lds) {
   if (pairs > kWideUnits || lds + kWideThreads / 64 * sizeof(int) > kLds) return 0;
+  const int least = pairs % 8 ? kLinePieces : kLeastPieces;
   int parts = 1;
-  while (pairs * parts * 2 <= kWideGrid && lpv % (parts * 2 * kLinePieces) == 0) parts *= 2;
+  while (pairs * parts * 2 <= kWideGrid && lpv % (parts * 2 * least) == 0) parts *= 2;
   return parts;
+}
+
+// Rounds of half as many pieces where one takes all: loads of those that are not there are made all the same (columns of quarter
+// lines, one bf16 sequence 10.3 us, now 8.8, one fp32 14.9, 13.1).
+template <int CES> int launch_wide(const CompactArgs& a, int L, hipStream_t st) {
+  if ((int64_t)a.target_width * a.BS * a.lpv <= kWideThreads * kCompactR) return launch_compact_impl<u32x4, kCompactR, false, true, CES, kWideThreads>(a, L, st);
+  return launch_compact_impl<u32x4, 2 * kCompactR, false, true, CES, kWideThreads>(a, L, st);
 }
 
 // ------------------------------------------------------------------ query ring store
@@ -373,10 +385,9 @@ int compress_kv_impl(void* key, void* value, const uint8_t* flag, const int32_t*
     a.lpv /= parts;
     a.lpv_shift = log2_exact(a.lpv);
     a.bs_shift = log2_exact(BS);
-    if (!score_cache || !fused) return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 0, kWideThreads>(a, L, st);
+    if (!score_cache || !fused) return launch_wide<0>(a, L, st);
     *fused = true;
-    if (es == 4) return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 4, kWideThreads>(a, L, st);
-    return launch_compact_impl<u32x4, 2 * kCompactR, false, true, 2, kWideThreads>(a, L, st);
+    return es == 4 ? launch_wide<4>(a, L, st) : launch_wide<2>(a, L, st);
   }
   switch (piece) {
     case 16:
