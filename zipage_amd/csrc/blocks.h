@@ -220,7 +220,7 @@ inline Pieces pieces_of(int64_t rows, int64_t segments, int64_t heads, int64_t l
   const int64_t all = (longest + kBlock - 1) / kBlock;
   if (!few_heads(segments, heads)) return p;
   int64_t best = all * 10;
-  for (int64_t m = kLeastPiece; m < all; m += step) {
+  for (int64_t m = kLeastPiece; m < all && m * (10 + cost.sum) + cost.fixed < best; m += step) {      // longer ones only take longer
     const int64_t most = (all + m - 1) / m, slots = piece_slots(rows, segments, m), pieces = segments * most < slots ? segments * most : slots;
     const int64_t took = m * (10 + cost.sum) + cost.fixed + most * cost.state;
     if (pieces * heads > kPieceGroups || (pieces - segments) * heads * cost.groups > kPieceGroups || slots * heads > kPieceStates ||
