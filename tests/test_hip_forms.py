@@ -836,6 +836,47 @@ def test_delta_state_of_runs(dev, H, G, D, V):
         assert float(err) < 2.0 ** -19, float(err)
 
 
+# Channels that forget `bits` a token, or hardly anything but 5 to 14 at every sixteenth: A, P and what the state gets of a key are
+# sums of running products, which carry no rounding of what was forgotten before.  Low-rank products of one term each, which are exact.
+@pytest.mark.parametrize("bits", [0.05, 0.5, 3.0, 8.0, "spikes"])
+def test_delta_state_of_channels_that_forget(dev, bits):
+    from zipage_amd.layers import ChannelDelta
+    H, G, D, V, W, taps, rank, counts = 4, 2, 128, 128, 64, 4, 64, [160, 96, 47]
+    m, n, g = ChannelDelta(W, H, G, D, V, taps, 1e-6), sum(counts), torch.Generator().manual_seed(3)
+    r = lambda *s, std=1.0: (torch.randn(*s, generator=g) * std).to(BF16)
+    w = {k: r(*s) for k, s in m.shapes(rank, rank).items()} | {k: r(*m.shapes(rank, rank)[k], std=.5) for k in ("q.conv", "k.conv", "v.conv")}
+    w |= {"A_log": torch.zeros(H, dtype=BF16), "dt_bias": torch.zeros(H * D, dtype=BF16), "a2": torch.zeros(H * D, rank, dtype=BF16)}
+    column = torch.randint(rank, (H * D,), generator=g)
+    w["a2"][torch.arange(H * D), column] = 1
+    m.load(w, BF16, dev, W)
+    P = r(n, m.columns, std=.5)
+    if bits == "spikes":
+        forgets = torch.where(torch.rand(n, rank, generator=g) < 1 / 16, 5 + 9 * torch.rand(n, rank, generator=g), 0.01)
+    else:
+        forgets = bits * torch.exp(.3 * torch.randn(n, rank, generator=g))
+    P[:, m.low_at:m.low_at + rank] = torch.log(torch.expm1(forgets.double() * 0.6931471805599453)).to(BF16)      # softplus gives it back
+    state = m.allocate(len(counts), BF16, dev)
+    rows, ctx = _run_segments(dev, counts)
+    m.scan(P.to(dev), state, ctx, torch.empty(n, H * V, dtype=BF16, device=dev))
+    P, head = P.double(), torch.arange(H) // (H // G)
+    decay = torch.exp(-torch.nn.functional.softplus(P[:, m.low_at:m.low_at + rank]))[:, column].view(n, H, D)
+    for i, c in enumerate(counts):
+        p, gg = P[rows[i]:rows[i] + c], decay[rows[i]:rows[i] + c]
+        conv = lambda f, t, k: K.short_conv(p[:, f:t], w[k + ".conv"].double())
+        k = K.unit(conv(G * D, 2 * G * D, "k").view(c, G, D))[:, head]
+        v = conv(2 * G * D, 2 * G * D + H * V, "v").view(c, H, V)
+        beta, S = torch.sigmoid(p[:, m.b_at:m.b_at + H]), torch.zeros(H, D, V, dtype=torch.float64)
+        for t in range(c):
+            S = gg[t][:, :, None] * S
+            u = beta[t][:, None] * (v[t] - (S * k[t][:, :, None]).sum(1))
+            S = S + k[t][:, :, None] * u[:, None, :]
+        # Roundings of 2^-24 by the products, decays and unit vectors of the tokens that a state remembers: one or two of them where
+        # channels forget 3 bits and more, each with a unit vector, a step size, a value and a few decays (1.1e-7 measured for 3 bits; 5.9e-7
+        # with quotients of decays).
+        err = float((state[0][i].double().cpu().view(H, D, V) - S).norm() / S.norm())
+        assert err < (2.0 ** -22 if bits in (3.0, 8.0) else 2.0 ** -20), err
+
+
 # linear attention and matrix memory likewise; rows of values, and of the memory's keys, are bf16 as they come
 @pytest.mark.parametrize("H,D,V", [(2, 128, 128), (2, 32, 96), (3, 64, 32), (1, 128, 64)])
 @pytest.mark.parametrize("mixer", ["linear", "memory"])

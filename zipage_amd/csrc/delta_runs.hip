@@ -42,35 +42,35 @@ __host__ __device__ inline constexpr int gates_at(int dk, int dv) { return 2 * k
 __device__ __forceinline__ int64_t pair_slot(int row0, const Segment& sg, int seg, int b) { return (sg.row - row0) / (2 * kBlock) + seg + b; }
 
 // A pair of blocks: 256 threads each, and the products of the second with the first.  Bound by vector issue (four fifths of its
-// time).  A and P as products of G k and G q with k / G on the matrix cores take less of it than a walk down the tokens that
-// multiplies decays as it goes (160 heads of 2037 tokens at most 271 -> 234 us), which is left for channels that forget more
-// than 1 / G can hold.
+// time).  Ratios of decays are running products of the decays behind a token, A and P sums in fp32.  As products of G k and G q with
+// k / G on the matrix cores they take less of it (8 prompts of 2048 tokens, 32 heads 899 us in all, now 945; one of 110, 16 heads 39.0 and
+// 40.4), but quotients carry the roundings of what both have in common: where channels forget 3 bits a token, the state was 2.7e-7 of its
+// norm off 64 bits, now 1.1e-7.
 constexpr int kPrepareLd = 132;                // floats of a row: reads across tokens meet no conflicts, offsets are constants
-constexpr int kPrepareHalf = kBlock * 4 * kPrepareLd + 6 * kBlock * kBlock + kBlock + 128 + 4;
-constexpr float kLeastDecay = 0x1p-60f;        // of a channel within a block, for its reciprocal
-// From the bits that each of a row of 16 lanes forgets to the decays up to it: sums over two lanes, their powers, products of
-// these (fewer roundings than products of all, and relative ones).  Eight side by side, as a lane that is moved has to be
-// written two instructions before.
-__device__ __forceinline__ void running_decays(f32x4 (&x)[2]) {
+constexpr int kPrepareHalf = kBlock * 4 * kPrepareLd + 6 * kBlock * kBlock + kBlock + 128;
+// A lane of 16, one of each row, gets its left neighbour's times its own decay; the first keeps its own.  Eight side by side, as a
+// lane that is moved has to be written two instructions before.
+__device__ __forceinline__ void to_next_token(float (&x)[8], const float (&g)[8]) {
 #ifdef __HIP_DEVICE_COMPILE__
-#define ZP_MOVED(op, i, n) "v_" op "_f32_dpp %" #i ", %" #i ", %" #i " row_shr:" #n " row_mask:0xf bank_mask:0xf\n\t"
-#define ZP_ALL(op, n)                                                                                              \
-  ZP_MOVED(op, 0, n) ZP_MOVED(op, 1, n) ZP_MOVED(op, 2, n) ZP_MOVED(op, 3, n) ZP_MOVED(op, 4, n) ZP_MOVED(op, 5, n) \
-  ZP_MOVED(op, 6, n) ZP_MOVED(op, 7, n)
-#define ZP_EIGHT "+v"(v[0]), "+v"(v[1]), "+v"(v[2]), "+v"(v[3]), "+v"(v[4]), "+v"(v[5]), "+v"(v[6]), "+v"(v[7])
-  float v[8];
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = x[i >> 2][i & 3];
-  asm volatile("s_nop 1\n\t" ZP_ALL("add", 1) : ZP_EIGHT);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = __builtin_amdgcn_exp2f(-v[i]);
-  asm volatile("s_nop 1\n\t" ZP_ALL("mul", 2) ZP_ALL("mul", 4) ZP_ALL("mul", 8) "s_nop 1" : ZP_EIGHT);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) x[i >> 2][i & 3] = v[i];
-#undef ZP_EIGHT
-#undef ZP_ALL
+#define ZP_MOVED(i, by) "v_mul_f32_dpp %" #i ", %" #i ", %" #by " row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
+  asm("s_nop 1\n\t" ZP_MOVED(0, 8) ZP_MOVED(1, 9) ZP_MOVED(2, 10) ZP_MOVED(3, 11) ZP_MOVED(4, 12) ZP_MOVED(5, 13) ZP_MOVED(6, 14) ZP_MOVED(7, 15)
+      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
+      : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(g[4]), "v"(g[5]), "v"(g[6]), "v"(g[7]));
 #undef ZP_MOVED
 #endif
+}
+// The left neighbour's of 16, the first's one.
+__device__ __forceinline__ float before_or_one(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0x3f800000, __builtin_bit_cast(int, x), 0x111, 0xf, 0xf, false));
+}
+// Sums over the wave's four groups of 16 lanes; group g has that of x[g].
+__device__ __forceinline__ float sums_of_groups(const float (&x)[4]) {
+  auto bits = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+  auto value = [](uint32_t v) { return __builtin_bit_cast(float, v); };
+  const auto a = __builtin_amdgcn_permlane16_swap(bits(x[0]), bits(x[1]), false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(bits(x[2]), bits(x[3]), false, false);
+  const auto c = __builtin_amdgcn_permlane32_swap(bits(value(a[0]) + value(a[1])), bits(value(b[0]) + value(b[1])), false, false);
+  return value(c[0]) + value(c[1]);
 }
 template <int TAPS, bool PROJECTED>
 __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
@@ -85,13 +85,12 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   const int h = blockIdx.y, hk = h / (a.heads / a.kv_heads);
   float* const qs = lds + half * kPrepareHalf;                 // [16][ld], later G q
   float* const ks = qs + kBlock * ld;          // later G k, then -W
-  float* const gs = ks + kBlock * ld;          // bits forgotten, later keys with the decays behind them
+  float* const gs = ks + kBlock * ld;          // decays, later keys with those behind them
   float* const vs = gs + kBlock * ld;
   float* const As = vs + kBlock * ld;          // [16][16]
   float* const Ps = As + kBlock * kBlock;      // [16][16]; both over parts of them, [3][2][64][4]
   float* const beta = As + 6 * kBlock * kBlock;
   float* const decays = beta + kBlock;         // [dk] of the whole block
-  int* const forgets = (int*)(lds + kPrepareHalf - 4);         // of either block
   float* const other_decays = decays + (half ? -kPrepareHalf : kPrepareHalf);
   const int tid = threadIdx.x & 255, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int cw = 2 * dk + dv;
@@ -144,7 +143,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
       }
   }
   const float b_in = tid < cnt ? Elem<BF16>::ld(a.in, (int64_t)(sg.row + t0 + tid) * a.in_stride + a.b_at + h) : 0.f;
-  const float rate = expf(a.a_log[h]) * 1.44269504088896f;
+  const float rate = expf(a.a_log[h]) * 1.44269504088896f;      // in bits
   // ---- convolutions: a thread's two channels, the block's 16 tokens from a sliding window.  Rows behind the run's end read
   // as zero, and those before its beginning too, unless they come from the history.
   const int row_bytes = (int)a.in_stride * 2;
@@ -181,8 +180,8 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     for (int u = 0; u < 2; ++u) *(u32x4*)((char*)qs + ((tid + u * 256) >> 5) * ld * 4 + (tid & 31) * 16) = low[u];
     __syncthreads();
     // A wave 16 channels of decays and 16 of gates, of both blocks.  The library's product of rows that are half zeros takes as
-    // long as this does in all for many tokens and a launch more (8 prompts of 2048 tokens, 32 heads 936 -> 917 us, 2 of about 1250
-    // 261 -> 240, one of 110, 16 heads 42.3 -> 38.7); weights row by row, which touch twice as many lines, 944.
+    // long as this does in all for many tokens and a launch more (8 prompts of 2048 tokens, 32 heads 19 us of 936, 2 of about 1250
+    // 21 of 261, one of 110, 16 heads 3.6 of 42.3); weights row by row, which touch twice as many lines, cost 27 of the first.
     const f32x4 bias = wave8 < tiles ? *(const f32x4*)(a.dt_bias + h * dk + wave8 * 16 + g4 * 4) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < 2; ++k) {
@@ -200,7 +199,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
         x = f32x4{__uint_as_float(lo << 16), __uint_as_float(lo & 0xffff0000u), __uint_as_float(hi << 16), __uint_as_float(hi & 0xffff0000u)} + bias;
         const bool there = (2 * (int)blockIdx.x + k) * kBlock + l16 < sg.count;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) x[e] = there ? rate * fast_softplus(x[e]) : 0.f;
+        for (int e = 0; e < 4; ++e) x[e] = there ? __builtin_amdgcn_exp2f(-rate * fast_softplus(x[e])) : 1.f;
         *(f32x4*)(lds + k * kPrepareHalf + 2 * kBlock * ld + l16 * ld + wave8 * 16 + g4 * 4) = x;
       }
     }
@@ -229,14 +228,13 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   for (int u = 0; u < 2; ++u) {
     const int i = tid + u * 256, t = i >> piece_bits, c = (i & ((1 << piece_bits) - 1)) * 4;
     if (t < kBlock) {
-      f32x4 bits;
+      f32x4 g;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) bits[e] = t < cnt ? rate * fast_softplus(z[u][e] + zb[u][e]) : 0.f;
-      *(f32x4*)(gs + t * ld + c) = bits;
+      for (int e = 0; e < 4; ++e) g[e] = t < cnt ? __builtin_amdgcn_exp2f(-rate * fast_softplus(z[u][e] + zb[u][e])) : 1.f;
+      *(f32x4*)(gs + t * ld + c) = g;
     }
   }
   if (tid < kBlock) beta[tid] = tid < cnt ? fast_sigmoid(b_in) : 0.f;
-  if (threadIdx.x == 0) *forgets = 0;
   __syncthreads();
   // ---- unit vectors: a wave its four tokens, 16 lanes each
   {
@@ -264,7 +262,9 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     }
   }
   __syncthreads();
-  // ---- A and P on the matrix cores, 32 channels a wave: rows G_t k_t and G_t q_t with k_s / G_s
+  // ---- A and P: a wave 32 channels, a lane one token's of them.  Keys go down the tokens, from lane to lane, and decay on the way:
+  // after d moves a lane has k_s with the decays behind s, s = t - d, for A[t, s] and P[t, s], and the last lane what the state gets of
+  // k_s.  One comes in before the first token, and once it has reached a lane, that has the decays up to it.
   const int waves = dk / 32, row_at = (lane & 15) * ld + wave * 32 + (lane >> 4) * 4;
   float* const oU = to + 6 * kBlock * dk + half * kBlock * dv;
   float* const oSmall = to + 6 * kBlock * dk + 2 * kBlock * dv;
@@ -288,131 +288,69 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) y[u] = mfma_bf16(l[i], r[u][j], y[u]);
   };
-  f32x4 Gq[2], Gk[2], behind[2], y[2];         // behind: keys with the decays behind them
+  f32x4 y[2];                                  // A and P, distances 4 u + lane / 16 in element u
   if (wave < waves) {
-    f32x4 G[2], over[2];
-    u32x4 left[3], rows2[2][3];
-    float least = 1.f;
+    float k[8], q[8], g[8], x[8];              // of this lane's own elements, all three, which nobody else reads
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
-      G[p] = *(const f32x4*)(gs + row_at + 16 * p);
-      Gk[p] = *(const f32x4*)(ks + row_at + 16 * p);
-      Gq[p] = *(const f32x4*)(qs + row_at + 16 * p);
+      const f32x4 kp = *(const f32x4*)(ks + row_at + 16 * p), qp = *(const f32x4*)(qs + row_at + 16 * p), gp = *(const f32x4*)(gs + row_at + 16 * p);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) k[4 * p + e] = kp[e], q[4 * p + e] = qp[e], g[4 * p + e] = gp[e], x[4 * p + e] = kp[e];
     }
-    running_decays(G);
+    auto put = [](float* at, const float (&v)[8]) {
+      *(f32x4*)at = f32x4{v[0], v[1], v[2], v[3]};
+      *(f32x4*)(at + 16) = f32x4{v[4], v[5], v[6], v[7]};
+    };
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
+    for (int u = 0; u < 4; ++u) {
+      float sa[4], sp[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float whole = dpp_moved<0x15f>(G[p][e]);         // of the row's last lane
-        over[p][e] = Gk[p][e] * __builtin_amdgcn_rcpf(G[p][e]);
-        behind[p][e] = over[p][e] * whole;
-        least = fminf(least, whole);
+      for (int j = 0; j < 4; ++j) {
+        const int d = 4 * u + j;
+        if (d == 1)
+#pragma unroll
+          for (int i = 0; i < 8; ++i) x[i] = before_or_one(x[i]) * g[i];
+        if (d > 1) to_next_token(x, g);
+        if ((lane & 15) == 15) put(gs + row_at - d * ld, x);
+        sa[j] = sp[j] = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (d > 0) sa[j] += x[i] * k[i];
+          sp[j] += x[i] * q[i];
+        }
       }
-      Gk[p] *= G[p];
-      Gq[p] *= G[p];
-      if ((lane & 15) == 15) *(f32x4*)(decays + wave * 32 + 16 * p + (lane >> 4) * 4) = G[p];
+      y[0][u] = sums_of_groups(sa);
+      y[1][u] = sums_of_groups(sp);
     }
-    if (least < kLeastDecay) *forgets = 1;
-    split(over, left);
-    split(Gk, rows2[0]);
-    split(Gq, rows2[1]);
-    products(left, rows2, y);
     if (wave > 0)
 #pragma unroll
       for (int u = 0; u < 2; ++u) *(f32x4*)(As + (((wave - 1) * 2 + u) * 64 + lane) * 4) = y[u];
+    to_next_token(x, g);                       // the decays up to the lane's token
+    if ((lane & 15) == 15) put(decays + wave * 32 + (lane >> 4) * 4, x);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) k[i] *= x[i], q[i] *= x[i];
+    put(ks + row_at, k);
+    put(qs + row_at, q);
   }
-  const int t_row = lane & 15, s_first = lane >> 4 << 2;       // of A and P: row t, from column s on
-  auto rows_to_lds = [&] {
-    if (wave < waves)
-#pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        *(f32x4*)(ks + row_at + 16 * p) = Gk[p];
-        *(f32x4*)(gs + row_at + 16 * p) = behind[p];
-        *(f32x4*)(qs + row_at + 16 * p) = Gq[p];
-      }
-  };
   __syncthreads();
-  if (!__builtin_amdgcn_readfirstlane(*forgets)) {
-    rows_to_lds();
-    if (wave == 0) {
-      for (int j = 1; j < waves; ++j)
+  if (wave == 0) {
+    for (int j = 1; j < waves; ++j)
 #pragma unroll
-        for (int u = 0; u < 2; ++u) y[u] += *(const f32x4*)(As + (((j - 1) * 2 + u) * 64 + lane) * 4);
+      for (int u = 0; u < 2; ++u) y[u] += *(const f32x4*)(As + (((j - 1) * 2 + u) * 64 + lane) * 4);
+    asm volatile("" ::: "memory");             // the parts are read before rows of A and P lie there
+    const int t = lane & 15, g4 = lane >> 4;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        y[0][r] *= beta[t_row];                                // those of A from t on are not read
-        if (s_first + r > t_row) y[1][r] = 0.f;
+    for (int u = 0; u < 4; ++u)
+      if (const int d = 4 * u + g4; d <= t) {  // A's with itself is not read
+        As[t * kBlock + t - d] = y[0][u] * beta[t];
+        Ps[t * kBlock + t - d] = y[1][u];
       }
-      *(f32x4*)(As + t_row * kBlock + s_first) = y[0];
-      put_small(half, y[1]);
-    }
-  } else {
-    if (tid < kBlock * kBlock / 4) *(f32x4*)(Ps + tid * 4) = f32x4{0.f, 0.f, 0.f, 0.f};
-    __syncthreads();
-    // 16 lanes walk k_s down the tokens from s on, in pieces of four channels.  A wave takes four neighbours, so that it
-    // starts at the first of them.
-    {
-      const int turn = (wave + blockIdx.x) & 3, first = 4 * (half ? 3 - turn : turn), s = first + (lane >> 4), pieces = dk / 4;
-      int at[2];
-      f32x4 kk[2];
+    asm volatile("" ::: "memory");
+    f32x4 P = *(const f32x4*)(Ps + t * kBlock + 4 * g4);
 #pragma unroll
-      for (int p = 0; p < 2; ++p) {
-        const int pc = l16 + 16 * p;
-        at[p] = min(pc, pieces - 1) * 4;
-        kk[p] = *(const f32x4*)(ks + s * ld + at[p]);
-        if (pc >= pieces) kk[p] = f32x4{0.f, 0.f, 0.f, 0.f};
-      }
-      // Two tokens at a time, four sums over 16 lanes: lanes 8 .. 15 keep those of P, of each eight the upper half the second
-      // token's (eleven additions and choices instead of sixteen additions, one store instead of four).
-      const bool is_p = l16 & 8, second = l16 & 4;
-      float* const to = (is_p ? Ps : As) + s;
-      auto tokens = [&](int t, bool all) {       // all: they lie behind the four
-        float sa[2], sp[2];
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-          f32x4 pa = {0.f, 0.f, 0.f, 0.f}, pp = pa;
-#pragma unroll
-          for (int p = 0; p < 2; ++p) {
-            const f32x4 gt = *(const f32x4*)(gs + (t + u) * ld + at[p]);      // bits
-#pragma unroll
-            for (int e = 0; e < 4; ++e) kk[p][e] *= all || t + u > s ? __builtin_amdgcn_exp2f(-gt[e]) : 1.f;
-            pa += kk[p] * *(const f32x4*)(ks + (t + u) * ld + at[p]);
-            pp += kk[p] * *(const f32x4*)(qs + (t + u) * ld + at[p]);
-          }
-          sa[u] = (pa[0] + pa[1]) + (pa[2] + pa[3]);
-          sp[u] = (pp[0] + pp[1]) + (pp[2] + pp[3]);
-          sa[u] += dpp_row_ror<8>(sa[u]);
-          sp[u] += dpp_row_ror<8>(sp[u]);
-          sa[u] = is_p ? sp[u] : sa[u];
-          sa[u] += half_row_mirror(sa[u]);
-        }
-        const float x = quad_sum(second ? sa[1] : sa[0]);
-        const int mine = t + second;
-        const float by = is_p ? 1.f : beta[mine];
-        if (all || (is_p ? mine >= s : mine > s)) to[mine * kBlock] = x * by;
-      };
-#pragma unroll
-      for (int u = 0; u < 4; u += 2) tokens(first + u, false);
-#pragma unroll 1
-      for (int t = first + 4; t < kBlock; t += 2) tokens(t, true);
-    }
-    // what is forgotten behind a token lies at the right of its lane
-    if (wave < waves)
-#pragma unroll
-      for (int p = 0; p < 2; ++p)
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          float R = dpp_moved<0x101>(gs[row_at + 16 * p + e]);     // row_shl:1, zeros behind the last
-          R += dpp_moved<0x101>(R);
-          R += dpp_moved<0x102>(R);
-          R += dpp_moved<0x104>(R);
-          R += dpp_moved<0x108>(R);
-          behind[p][e] = ks[row_at + 16 * p + e] * __builtin_amdgcn_exp2f(-R);
-        }
-    __syncthreads();
-    rows_to_lds();
-    if (wave == 3) put_small(half, *(const f32x4*)(Ps + t_row * kBlock + s_first));
+    for (int r = 0; r < 4; ++r)
+      if (4 * g4 + r > t) P[r] = 0.f;
+    put_small(half, P);
   }
   __syncthreads();
   // ---- columns: forward substitution.  A thread reads and writes its own column only.
@@ -584,9 +522,10 @@ __global__ __launch_bounds__(64 * NW, 1) void delta_states_kernel(RunArgs ra) {
 // units.  The state is split where it is updated; what comes from memory passes through registers, asked for a pair ahead, and
 // is split into LDS by all waves together under the products with the state; rows are normed and stored in the next pair.
 // What bounds it: of 11 300 cycles a pair and SIMD the products take 5100, vector issue 6200 beside them, LDS 4300, and the
-// younger of its two waves the rest.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1033 -> 917 us, 5 of
-// 1640 to 2037 717 -> 598, one 256 -> 214; 7 of 625 to 1499 with 16 heads 415 -> 344; error of the state against 64 bits 3.3e-7 ->
-// 3.0e-7 of its size.
+// younger of its two waves the rest.  8 prompts of 2048 tokens, 32 heads of 128 x 128, with the kernel above: 1017 -> 945 us, 5 of
+// 1640 to 2037 717 -> 621, one 261 -> 217; 7 of 625 to 1499 with 16 heads 417 -> 357; error of the state against 64 bits, where channels
+// forget 0.01, 1 and 3 bits a token, 3.9e-7 -> 3.7e-7, 1.7e-7 -> 1.4e-7 and 1.3e-7 -> 1.1e-7 of its norm.  All products are six of the planes;
+// with eight in the update of the state, 3.694e-7 instead of 3.695e-7, 1.437e-7 and 1.142e-7, and 1 to 2 % longer.
 // SUMS: no state comes in and no rows go out; every second workgroup takes what the piece keeps, where values are none.
 template <int KT, int NW> struct PairStage {
   static constexpr int kTiles = 6 * KT, kPlanes = kTiles * 384, kSmall = small_floats(16 * KT);      // floats in LDS
