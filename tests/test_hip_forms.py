@@ -799,6 +799,48 @@ def test_delta_runs_in_pairs_of_blocks(dev, H, G, D, V, taps, ranks, bias, sprea
     assert float((got - want).norm() / want.norm()) < 2.0 ** -8 and bool(torch.isfinite(got).all())
 
 
+# Decoded tokens and short portions beside runs: a row's low-rank products are made once, by the library for portions and by the kernels for
+# runs, which get what they would of a step of their own; by the library for all rows where the portions' may be any.
+@pytest.mark.parametrize("short,known", [((1, 1, 1), True), ((3, 15), True), ((3, 15), False), ((), True)])
+def test_delta_steps_of_runs_and_portions(dev, monkeypatch, short, known):
+    import types
+    from zipage_amd import _lib
+    from zipage_amd.engine.qwen3 import Segments
+    from zipage_amd.layers import ChannelDelta, recurrent
+    H, G, D, taps, W, counts = 4, 2, 128, 4, 64, [*short, 64, 100]
+    m, n, rows, first = ChannelDelta(W, H, G, D, D, taps, 1e-3), len(counts), sum(counts), sum(short)
+    into, _ = m.load({k: _rand(*s, seed=i) * s[-1] ** -0.5 for i, (k, s) in enumerate(m.shapes(128, 128).items())}, BF16, dev, W)
+    proj = (_rand(rows, W, seed=60).to(dev).float() @ into.to(dev).float().T).to(BF16)
+    t = lambda a: torch.tensor(a, dtype=torch.int32, device=dev)
+
+    def segments(i, j, **kw):
+        return Segments(t([sum(counts[:k]) for k in range(i, j)]), t(counts[i:j]), t(list(range(i, j))), t([7] * (j - i)), **kw) if j > i else None
+    portions = segments(0, len(short), end=first if known else 0)
+    runs = segments(len(short), n, first_row=first, longest=max(counts))
+
+    def scan(portions, runs, tiles=True):
+        calls, call, product = [], _lib.call_models, recurrent.step_product
+        with monkeypatch.context() as patch:
+            patch.setattr(_lib, "call_models", lambda name, *a: (calls.append(name), call(name, *a)))
+            patch.setattr(recurrent, "step_product", lambda ctx: lambda x, w: (calls.append(x.shape[0]), product(ctx)(x, w))[1])
+            patch.setattr(m, "low_tiles", m.low_tiles if tiles else None)
+            state = m.allocate(n, BF16, dev)
+            state[0].copy_((0.1 * _rand(*state[0].shape, seed=61).float()).to(dev))
+            out = torch.empty(rows, m.out_columns, dtype=BF16, device=dev)
+            m.scan(proj, state, types.SimpleNamespace(segments=portions, run_segments=runs), out)
+        return calls, out, state[0]
+    calls, got, gs = scan(portions, runs)
+    made = known or not short
+    assert calls == ([first if known else rows, "zp_delta_scan"] if short else []) + ["zp_delta_runs_projected" if made else "zp_delta_runs"]
+    _, alone, state = scan(None, runs, made)
+    assert torch.equal(got[first:], alone[first:]) and torch.equal(gs[len(short):], state[len(short):])
+    if short:
+        _, other, state = scan(portions, None)
+        # pre-activations that another order of sums rounds to the next bf16 value, one in some hundred
+        assert float((got[:first] - other[:first]).float().norm() / other[:first].float().norm()) < 2.0 ** -7
+        assert float((gs[:len(short)] - state[:len(short)]).norm() / state[:len(short)].norm()) < 2.0 ** -9
+
+
 # operands enter the bf16 matrix cores in three planes: the state has to stay as good as fp32's
 @pytest.mark.parametrize("H,G,D,V", [(2, 1, 128, 128), (2, 2, 32, 96), (3, 1, 64, 32), (1, 1, 128, 64)])
 def test_delta_state_of_runs(dev, H, G, D, V):

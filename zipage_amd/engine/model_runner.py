@@ -229,7 +229,7 @@ class ModelRunner:
         ids, rows, pos, slots, ctx_lens, table_rows = (next(d) for _ in range(6))
         tables = next(d).view(plan.tables.shape)
         seg, k = [next(d) for _ in range(4)], plan.short
-        segments = Segments(*(a[:k] for a in seg)) if k else None
+        segments = Segments(*(a[:k] for a in seg), end=int(plan.segments[0, k]) if k < len(portions) else 0) if k else None
         long = Segments(*(a[k:] for a in seg), first_row=int(plan.segments[0, k]),
                         longest=int(plan.segments[1, k:].max())) if k < len(portions) else None
         runs = {}

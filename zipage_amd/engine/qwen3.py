@@ -49,7 +49,8 @@ QWEN3_0_6B = Qwen3Shape(28, 1024, 16, 8, 128, 3072, 151936)
 class Segments:
     """The portions of a step as recurrent layers read them, int32 arrays: first token row (None: the
     portion's index), tokens (at most `max_count` when that is set; 0: inert), state slot, position of
-    the first token.  Long runs also name the first row of all and the length of the longest."""
+    the first token.  Long runs also name the first row of all and the length of the longest; short portions a row that all of
+    theirs lie before, where the host knows one (0: they may be any)."""
     rows: torch.Tensor | None
     counts: torch.Tensor
     slots: torch.Tensor
@@ -57,6 +58,7 @@ class Segments:
     max_count: int = 0
     first_row: int = 0
     longest: int = 0
+    end: int = 0
 
 
 @dataclass

@@ -153,7 +153,8 @@ def linear_parts(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 def step_product(ctx):
     """What a step's layers multiply with: `linear` where every sequence has one token.  What a step holds of a prompt may be few rows as
-    well, and keeps the library's products, as the same rows of a whole prompt do, so that both round alike."""
+    well, and keeps the library's products, as the same rows of a whole prompt do, so that both round alike.  (All but the low-rank
+    products of the delta rule: a step of runs alone makes them in the blocked kernels, whose order of fp32 sums is their own.)"""
     segments = getattr(ctx, "segments", None)
     prompts = getattr(ctx, "is_prefill", False) or getattr(ctx, "runs", None) or getattr(ctx, "run_segments", None) is not None or \
         segments is not None and segments.max_count != 1

@@ -169,17 +169,23 @@ class ChannelDelta:
         H, D = self.heads, self.dim_p
         assert proj.stride(1) == out.stride(1) == 1 and proj.dtype == out.dtype == tail.dtype and S.is_contiguous()
         blocks = self.can_run and proj.dtype == torch.bfloat16
-        # runs by the blocked kernels make the low-rank products on their way, where nothing else looks at them
-        projected = ctx.run_segments is not None and blocks and self.low_tiles is not None and self.low_tiles.device == proj.device and \
-            not _seen_by_others(proj, self.low)
-        low = None if projected and ctx.segments is None else \
-            step_product(ctx)(proj[:, self.low_at:self.low_at + self.low_rank], self.low)
+        # runs by the blocked kernels make the low-rank products on their way, where nothing else looks at them; the library makes them for
+        # short portions, or for all rows where these may be any: once for a row (8 prompts of 2048 tokens and 32 decoded ones, 32 heads
+        # 1016 us; 1133 with the runs' from the library too, 1111 before the kernels made them)
+        end = 0 if ctx.segments is None else getattr(ctx.segments, "end", 0) or proj.shape[0]
+        projected = ctx.run_segments is not None and blocks and end < proj.shape[0] and self.low_tiles is not None and \
+            self.low_tiles.device == proj.device and not _seen_by_others(proj, self.low)
+        at, low = slice(self.low_at, self.low_at + self.low_rank), None
+        if not projected:
+            end = proj.shape[0]
+        if end:
+            low = step_product(ctx)(proj[:end, at], self.low)
         tag, stream = _lib.dtype_tag(proj), _lib.stream_ptr(proj)
         for segments, runs in ((ctx.segments, False), (ctx.run_segments, blocks)):
             if segments is None:
                 continue
             args = _lib.DeltaArgs(
-                _segments(segments, S.shape[0], proj.shape[0]), _lib.dev_ptr(proj), _lib.dev_ptr(low),
+                _segments(segments, S.shape[0], proj.shape[0] if runs else end), _lib.dev_ptr(proj), _lib.dev_ptr(low),
                 _lib.dev_ptr(self.filters), _lib.dev_ptr(self.a_log), _lib.dev_ptr(self.dt_bias), _lib.dev_ptr(self.norm),
                 _lib.dev_ptr(S), _lib.dev_ptr(tail), _lib.dev_ptr(out), proj.stride(0), 0 if low is None else low.stride(0), out.stride(0), H,
                 self.kv_heads, D, self.vdim_p, self.vdim, self.taps, self.b_at, H * D, self.dim ** -0.5, self.eps,
