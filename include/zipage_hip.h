@@ -66,7 +66,7 @@ int zp_store_query(const void* query, void* query_cache, const int32_t* slot_map
  * positive scale and at most 2560 tokens per sequence that scratch lets the library keep the
  * logits in registers and sweep K once (fp32 window partials per block of 32 query rows -- 16
  * for fp32 caches -- go through the scratch); zp_attention_score_workspace_few(..., dtype) bytes,
- * which are more for calls with at most 128 such blocks, let it spread a block's tokens or rows over the
+ * which are more for calls with at most 64 such blocks, let it spread a block's tokens over the
  * chip, with the same bits; with less scratch (NULL is fine up to 128 window x
  * group rows) the same entry point sweeps K three times (twice for fp32 caches).  The kernels
  * round at the same points and differ only in the fp32 order of the row sums (fp32 caches: also
@@ -255,7 +255,8 @@ enum {
  * stages' own scratch, and the keep flags when flag_in_workspace != 0); -1 on bad arguments.  More
  * sequences need more, so what serves the largest batch serves every other.  With
  * zp_compress_layers_workspace_few() bytes, which are more for few sequences, their scores are
- * spread over the chip (see zp_attention_score): the same bits, sooner. */
+ * spread over the chip (see zp_attention_score; up to 128 blocks of rows, whose rows are spread where
+ * the selection adds up what they leave): the same bits, sooner. */
 int64_t zp_compress_layers_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv,
                                      int32_t Hq, int32_t W, int32_t dtype,
                                      const zp_compress_config* cfg, int32_t flag_in_workspace);

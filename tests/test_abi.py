@@ -112,6 +112,28 @@ def test_a_workspace_for_the_largest_batch_serves_every_other():
             assert few[0] > sizes[0] and few[-1] == sizes[-1] and all(f >= s for f, s in zip(few, sizes))
 
 
+def test_room_for_halves_of_blocks_only_where_they_are_used():
+    """Blocks of rows go in halves where the selection adds them up: not in the scorer's own call, nor for maxima over the window, nor where
+    carried scores are looked at in between."""
+    from zipage_amd import _lib
+    from zipage_amd.compress import CompressConfig, c_config
+    lib = _lib.load()
+    size = lambda name, batch, cc=(), heads=32, dtype=0: getattr(lib, name)(1, batch, 9, 256, 8, heads, 32, dtype, *cc)
+    for batch in (3, 4):                                                     # 96 and 128 blocks, too many for tiles
+        assert size("zp_attention_score_workspace_few", batch) == size("zp_attention_score_workspace_for", batch)
+    room = {}
+    for name, kw in (("sums", {}), ("max", dict(reduced="max")), ("carried", dict(use_global_score=True, decay_factor=0.8)),
+                     ("max norm", dict(use_global_score=True, decay_factor=0.8, max_norm=True)),
+                     ("atomic", dict(use_global_score=True, decay_factor=0.8))):
+        config = c_config(CompressConfig(budget_blocks=8, query_cache_len=32, **kw))
+        config.deterministic_carry = name != "atomic"
+        cc = (ctypes.byref(config), 0)
+        for batch in (4, 5):
+            room[name, batch] = size("zp_compress_layers_workspace_few", batch, cc) - size("zp_compress_layers_workspace", batch, cc)
+    partials = 4 * 9 * 256 * 8 * 4 * 4                                       # of 128 blocks
+    assert {k: v for k, v in room.items() if v} == {("sums", 4): 3 * partials, ("carried", 4): 3 * partials}
+
+
 def test_room_for_pieces_of_runs_follows_the_rows():
     """Blocks of 16 tokens alone where no run can be cut, as many states as rows, runs and heads can ask for beyond, and never more
     than 384."""

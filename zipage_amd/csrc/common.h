@@ -47,6 +47,9 @@ struct ScoreParts {
   int RB = 0, W = 0, rmax = 0;
   int shares = 1;                    // of a block, or 4, sums that are added up in pairs first
 };
+// Scratch with which it leaves them, that of zp_attention_score_workspace_few() and the halves' share of what is left.
+int64_t zp_attention_score_workspace_parts(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t W, int32_t reduced,
+                                           int32_t dtype);
 int zp_attention_score_parts(const void* k_cache, const void* query_cache, const int32_t* seq_idx, const int32_t* block_table,
                              void* scores_out, int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t D,
                              int32_t W, int32_t num_pages, int32_t max_seqs, int64_t k_sl, int64_t k_sp, int64_t q_sl,

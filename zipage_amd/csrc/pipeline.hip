@@ -20,7 +20,7 @@ inline int64_t align_up(int64_t v) { return (v + kAlign - 1) / kAlign * kAlign; 
 struct Plan {
   int64_t scores, scores2, red, flag, score_ws, raw_ws, total;   // byte offsets; -1 = unused
   int64_t score_ws_bytes, raw_ws_bytes;
-  bool one_launch_select;
+  bool one_launch_select, from_parts;
 };
 
 // Rows the one-launch selection holds in LDS (zp_select_topk's own limit).
@@ -37,6 +37,13 @@ Plan make_plan(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype,
   int64_t off = 0;
   auto take = [&](int64_t bytes) { const int64_t o = off; off += align_up(bytes); return o; };
   p.one_launch_select = select_fits((int64_t)NB * BS);
+  // The one-launch selection adds up what the scorer leaves of a row, and carries the scores of earlier steps, where nothing
+  // else looks at the row in between.  Selection, sums and carried scores of one layer: 64 bf16 sequences 8.8 + 4.8 + 8.8 us, now
+  // 13.5; 256 without earlier scores 16.6 + 18.0, now 24.6; 4 sequences 6.8 + 4.4 + 6.0, now 9.6; and the launches' gaps.  It adds up
+  // whole blocks and blocks in four shares (16-bit halves, fp32 quarters); the eight of 16-bit tiles are still summed by a launch of
+  // their own: in the selection one sequence takes 49.4 us instead of 47.3.
+  p.from_parts = p.one_launch_select && !(c->use_global_score && (c->max_norm || !c->deterministic_carry)) &&
+                 zp_select_takes_parts((int64_t)NB * BS, BS, c->pooling_size);
   p.scores = take(n * es);
   // the separate stages: pooling needs distinct in / out buffers, and the mask epilogue works in
   // place, which must not touch the scores the carried-score compaction reads later
@@ -47,7 +54,8 @@ Plan make_plan(int L, int B, int NB, int BS, int Hkv, int Hq, int W, int dtype,
   p.flag = own_flag ? take(n) : -1;
   p.score_ws_bytes = scratch == Scratch::floor ? zp_attention_score_workspace_floor(L, B, NB, BS, Hkv, Hq, W)
                      : scratch == Scratch::one_sweep ? zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, dtype)
-                                                     : zp_attention_score_workspace_few(L, B, NB, BS, Hkv, Hq, W, dtype);
+                     : p.from_parts ? zp_attention_score_workspace_parts(L, B, NB, BS, Hkv, Hq, W, c->reduced, dtype)
+                                    : zp_attention_score_workspace_few(L, B, NB, BS, Hkv, Hq, W, dtype);
   p.score_ws = p.score_ws_bytes ? take(p.score_ws_bytes) : -1;
   p.raw_ws_bytes = (c->use_redundancy && !c->lightning) ? zp_redundancy_raw_workspace(L, B, NB, BS, Hkv) : 0;
   p.raw_ws = p.raw_ws_bytes ? take(p.raw_ws_bytes) : -1;
@@ -156,24 +164,17 @@ int run_layers(void* k_cache, void* v_cache, const void* query_cache, void* scor
     ZP_REQUIRE(score_cache, "compress_layers: use_global_score needs a score cache");
     ZP_REQUIRE(c_ss == Hkv && c_sh == 1, "compress_layers: score cache must be (slot, head) contiguous");
   }
-  // The one-launch selection adds up what the scorer leaves of a row, and carries the scores of earlier steps, where nothing
-  // else looks at the row in between.  Selection, sums and carried scores of one layer: 64 bf16 sequences 8.8 + 4.8 + 8.8 us, now
-  // 13.5; 256 without earlier scores 16.6 + 18.0, now 24.6; 4 sequences 6.8 + 4.4 + 6.0, now 9.6; and the launches' gaps.  Few
-  // sequences' scores, whose partials are four and eight times as many, are still summed by a launch of their own: in here
-  // one sequence takes 49.4 us instead of 47.3.
-  const bool from_parts = p.one_launch_select && !(glob && (c->max_norm || !c->deterministic_carry)) &&
-                          zp_select_takes_parts((int64_t)NB * BS, BS, c->pooling_size);
   ScoreParts parts;
   CarriedScores carry;
   t.start(ZP_STAGE_ATTENTION_SCORE);
   rc = zp_attention_score_parts(k_cache, query_cache, seq_idx, block_table, scores, L, B, NB,
                                 BS, Hkv, Hq, D, W, num_pages, max_seqs, k_sl, k_sp, q_sl, q_ss, scale,
                                 c->reduced, dtype, p.score_ws >= 0 ? ws + p.score_ws : nullptr,
-                                p.score_ws_bytes, from_parts ? &parts : nullptr, stream);
+                                p.score_ws_bytes, p.from_parts ? &parts : nullptr, stream);
   if (rc != ZP_OK) return rc;
   t.stop(ZP_STAGE_ATTENTION_SCORE);
 
-  if (glob && from_parts) {               // inside the selection
+  if (glob && p.from_parts) {             // inside the selection
     carry = CarriedScores{score_cache, c_sl, c_sp, c->decay_factor, c->activate_method, scores};
     t.start(ZP_STAGE_GLOBAL_SCORE);
     t.stop(ZP_STAGE_GLOBAL_SCORE);

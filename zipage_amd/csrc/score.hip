@@ -1856,7 +1856,13 @@ extern "C" int64_t zp_attention_score_workspace_for(int32_t L, int32_t B, int32_
 extern "C" int64_t zp_attention_score_workspace_few(int32_t L, int32_t B, int32_t NB, int32_t BS,
                                                     int32_t Hkv, int32_t Hq, int32_t W, int32_t dtype) {
   const int64_t usual = zp_attention_score_workspace_for(L, B, NB, BS, Hkv, Hq, W, dtype);
-  return usual <= 0 ? usual : std::max({usual, tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype), split_need(L, B, NB, BS, Hkv, Hq, W, dtype, false)});
+  return usual <= 0 ? usual : std::max(usual, tiled_need(L, B, NB, BS, Hkv, Hq, W, dtype));
+}
+
+int64_t zp_attention_score_workspace_parts(int32_t L, int32_t B, int32_t NB, int32_t BS, int32_t Hkv, int32_t Hq, int32_t W, int32_t reduced,
+                                           int32_t dtype) {
+  const int64_t few = zp_attention_score_workspace_few(L, B, NB, BS, Hkv, Hq, W, dtype);
+  return few <= 0 ? few : std::max(few, split_need(L, B, NB, BS, Hkv, Hq, W, dtype, reduced == ZP_REDUCE_MAX));
 }
 
 extern "C" int64_t zp_attention_score_workspace(int32_t L, int32_t B, int32_t NB, int32_t BS,
