@@ -134,6 +134,22 @@ def test_room_for_halves_of_blocks_only_where_they_are_used():
     assert {k: v for k, v in room.items() if v} == {("sums", 4): 3 * partials, ("carried", 4): 3 * partials}
 
 
+def test_room_for_few_sequences_fits_the_librarys_scratch():
+    from zipage_amd import _lib
+    from zipage_amd.compress import CompressConfig, c_config
+    lib = _lib.load()
+    header = open(os.path.join(ROOT, "include", "zipage_hip.h")).read()
+    most = int(re.search(r"ZP_STATIC_SCRATCH_BYTES \((\d+)u << 20\)", header).group(1)) << 20
+    for kw in (dict(), dict(use_redudancy=True, use_global_score=True, decay_factor=0.8), dict(reduced="max")):
+        cc = (ctypes.byref(c_config(CompressConfig(budget_blocks=1, query_cache_len=16, **kw))), 1)
+        for dtype in (0, 2):
+            for NB, BS in ((40, 64), (20, 128), (10, 256), (1, 2560)):           # 2560 tokens
+                for group in (1, 2, 4, 8):
+                    for rows in range(1, 130):
+                        size = [getattr(lib, "zp_compress_layers_workspace" + few)(1, rows, NB, BS, 1, group, 16, dtype, *cc) for few in ("_few", "")]
+                        assert size[0] == size[1] or size[0] <= most
+
+
 def test_room_for_pieces_of_runs_follows_the_rows():
     """Blocks of 16 tokens alone where no run can be cut, as many states as rows, runs and heads can ask for beyond, and never more
     than 384."""

@@ -379,9 +379,8 @@ extern "C" int zp_compress_layers_static(void* k_cache, void* v_cache, const voi
                  target_block_table && strides, "compress_layers_static: null pointer");
   if (L == 0 || B == 0) return ZP_OK;
   Plan p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr);
-  // the logits of few sequences always fit (at most 16 MB of 23 in all)
-  if (p.total > (int64_t)ZP_STATIC_SCRATCH_BYTES)
-    p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr, Scratch::one_sweep);
+  // what few sequences ask for beside one sweep's always fits: the logits and partials of 64 blocks of rows are at most 16 MB, of 23 in all, the
+  // halves of 128 blocks 5, of 21
   if (p.total > (int64_t)ZP_STATIC_SCRATCH_BYTES)
     p = make_plan(L, B, NB, BS, Hkv, Hq, W, dtype, cfg, flag_out == nullptr, Scratch::floor);
   ZP_REQUIRE(p.total <= (int64_t)ZP_STATIC_SCRATCH_BYTES,
