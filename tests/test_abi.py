@@ -150,6 +150,16 @@ def test_room_for_few_sequences_fits_the_librarys_scratch():
                         assert size[0] == size[1] or size[0] <= most
 
 
+@pytest.mark.parametrize("NB,BS", [(52, 256), (26, 512), (202, 64), (1, 13120)])
+def test_rows_beyond_the_limit_of_all_pairs_are_refused(NB, BS):
+    from zipage_amd import _lib
+    lib, p = _lib.load(), ctypes.c_void_p(4096)
+    for dtype in (0, 1):
+        size = lib.zp_redundancy_raw_workspace(1, 1, NB, BS, 1)
+        assert lib.zp_redundancy_raw(p, p, p, None, 1, 1, NB, BS, 1, 128, NB, NB * BS * 128, BS * 128, 0.5, 0.4, dtype, p, size, None) == 3
+        assert b"at most 13120 tokens and pages" in lib.zp_last_error()
+
+
 def test_room_for_pieces_of_runs_follows_the_rows():
     """Blocks of 16 tokens alone where no run can be cut, as many states as rows, runs and heads can ask for beyond, and never more
     than 384."""

@@ -1153,11 +1153,11 @@ def test_prompts_keep_the_librarys_products(dev, few_rows_calls, tmp_path, model
 # ------------------------------------------------------------------ redundancy over all pairs, 16 bit
 # Pages of one or two tiles of 128 keys are their own first tiles, larger ones read their rows apart and take several rounds; pages
 # that are no whole tiles take the general form.  Rows of a multiple of eight share an XCD; few pages go in parts.  Chains of 16, 8,
-# 24, 32 and 12 chunks a page, whose ends fall anywhere among the 32 that are taken at a time.
+# 24, 32 and 12 chunks a page, whose ends fall anywhere among the 32 that are taken at a time.  The longest row of pages of 256.
 @pytest.mark.parametrize("dtype,BS,D,Hkv,pages,thr", [
     (BF16, 256, 128, 3, (5, 2), 0.5), (BF16, 256, 64, 8, (4, 1), 0.5), (torch.float16, 128, 128, 4, (7, 3), 0.3), (BF16, 384, 96, 1, (3,), 0.5),
     (torch.float16, 512, 32, 2, (2, 3), 0.9), (BF16, 192, 128, 2, (3, 5), 0.5), (BF16, 256, 128, 8, (4, 3) * 8, 0.5), (BF16, 128, 128, 8, (9,) * 6, 0.5),
-    (BF16, 256, 128, 8, (4, 3) * 8, 0.0)])
+    (BF16, 256, 128, 8, (4, 3) * 8, 0.0), (BF16, 256, 64, 1, (51,), 0.5)])
 def test_all_pairs_forms(dev, dtype, BS, D, Hkv, pages, thr):
     from tests.test_redundancy_planted import _clear_of_norm_boundaries, _close_in_ulps
     from zipage_amd.kernel import raw_redudancy_score

@@ -2317,6 +2317,9 @@ __global__ __launch_bounds__(kThreads) void raw_claim_value_kernel(GramArgs p) {
 // LDS: a round's 256 keys, and then planes and corrections.
 constexpr int kChainTile = 32, kChainLd = kChainTile + 4;
 constexpr int kChainBytes = 256 / 4 * kPgGrp;
+// Tokens and pages of a row that 16-bit caches take.  A limit of the interface: the claims of a row once lay in the LDS, now a row's pages and
+// chunks do, a twentieth of it here, and longer rows are not tested.
+constexpr int kMostRawTokens = 13120;
 static_assert(3 * kChainTile * ROWH + 256 * kChainLd * 4 <= kChainBytes, "planes and corrections fit where the keys were");
 __device__ __forceinline__ int to_fixed26(float v) { return (int)(v * 67108864.f); }
 __device__ __forceinline__ float from_fixed26(int w) { return (float)w * (1.f / 67108864.f); }
@@ -2845,8 +2848,8 @@ int launch_gram(const GramArgs& a, int L, hipStream_t st) {
                          sizeof(int) * 2 * a.NB;
     const bool wide = tn == 128 && smemw <= 80 * 1024;
     const size_t smem2 = kChainBytes + sizeof(int) * (a.NB + a.NB * a.BS / kChunk);
-    if (58880 + (size_t)a.NB * (8 + a.BS * 8) > 160 * 1024) {   // rows of up to 13 120 tokens
-      zp_set_error("redundancy: a row of %d tokens exceeds LDS", a.NB * a.BS);
+    if ((int64_t)a.NB * (a.BS + 1) > kMostRawTokens) {
+      zp_set_error("redundancy: a row of %d pages of %d tokens (16-bit caches: at most %d tokens and pages)", a.NB, a.BS, kMostRawTokens);
       return ZP_EUNSUPPORTED;
     }
     const GramArgs cut = tile_parts(a, grid.x), claims = claim_parts(a, grid.x);
