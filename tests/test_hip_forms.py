@@ -229,6 +229,24 @@ def test_experts_among_xcds(dev, n, width, E, top, ff, act):
     test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act)
 
 
+# 17 to 48 rows on average whose tokens lie so far apart that the staged form cannot address them: tiles of 128 in two parts, which are both
+# there, and where the second has one row
+@pytest.mark.parametrize("n,E,top,shared_ff", [(85, 5, 1, 0), (240, 5, 1, 96), (65, 2, 1, 0), (194, 6, 1, 32)])
+def test_experts_of_tokens_far_apart(dev, n, E, top, shared_ff):
+    from zipage_amd.layers import Experts
+    W, ff = 544, 96
+    m = Experts(W, E, top, ff, 7.0, shared_ff=shared_ff or None)
+    m.random(BF16, dev, torch.Generator(device=dev).manual_seed(1))
+    ids = (torch.arange(n * top, device=dev) % (E - 1)).to(torch.int32).view(n, top)
+    weights = torch.rand(n, top, device=dev, generator=torch.Generator(device=dev).manual_seed(2))
+    m.route = lambda h: (ids, weights, torch.zeros(E + 1, dtype=torch.int32, device=dev))
+    h = torch.empty(n, -(-2 ** 30 // n) + 8 & -8, dtype=BF16, device=dev)[:, :W]
+    h.copy_(_rand(n, W, seed=3))
+    want, got = m.forward(h.contiguous()).float(), m.forward(h).float()
+    # the same products, whose sums are split over other waves: roundings of activations and of rows, a bf16 step of 2^-8 where they differ
+    assert float((got - want).norm() / want.norm()) < 2.0 ** -9 and bool(torch.isfinite(got).all())
+
+
 def test_experts_of_many_weights_spread_over_xcds(dev):
     """Few rows against 380 MB of weights: every expert as by itself, whose weights are one XCD's share."""
     from zipage_amd.layers import Experts

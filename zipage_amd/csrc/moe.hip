@@ -381,6 +381,7 @@ struct ExpertArgs {
   float limit, limit_shared;
   int split;              // parts in which expert_tiles_kernel takes a tile
   bool together;          // expert_rows_kernel: an XCD takes a contiguous share of the launch, see launch_experts
+  int halves;             // expert_rows_kernel: 1 where tiles are of 128 rows and it takes them in two parts
 };
 
 // ZP_GATE_CLAMPED: w g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
@@ -420,8 +421,14 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int at = a.together ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int tile = at % a.max_tiles, cb = at / a.max_tiles;
-  if (tile >= *a.ntiles) return;
-  const int4 t = *(const int4*)(a.tiles + (int64_t)tile * 4);
+  if (tile >> a.halves >= *a.ntiles) return;
+  int4 t = *(const int4*)(a.tiles + (int64_t)(tile >> a.halves) * 4);
+  if constexpr (MT == 4) {
+    const int before = (tile & a.halves) * 64;
+    t.y += before;
+    t.z = min(t.z - before, 64);
+    if (t.z <= 0) return;
+  }
   const bool shared = t.x == a.E;
   const int wtiles = (shared ? a.M_shared : a.M) / 16 * (UP ? 2 : 1), K = shared ? a.K_shared : a.K;
   const int w0 = cb * kRowsW;
@@ -784,8 +791,9 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   }
 }
 
-template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, hipStream_t st) {
-  if (rows == 128 || rows == kBigRows) {
+// staged: tokens through LDS, tiles of 128 and 256 rows
+template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged, int dtype, hipStream_t st) {
+  if (staged) {
     const int Mx = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
     const bool big = rows == kBigRows && a.K >= kBigContraction;
     ExpertArgs b = a;
@@ -803,8 +811,11 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
     return ZP_OK;
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
-  const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
-  const bool wide = rows == 16 && dtype == ZP_BF16 && a.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
+  ExpertArgs b = a;
+  b.halves = rows == 128;
+  b.max_tiles <<= b.halves;
+  const auto grid_of = [&](int tiles_w) { return (int64_t)b.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
+  const bool wide = rows == 16 && dtype == ZP_BF16 && b.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
                     (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
   const int64_t grid = (grid_of(wide ? kWideW : kNarrowW) + 7) / 8 * 8;      // shares of eight XCDs; behind the last tile of W nothing is done
   if (grid >= (1ll << 31)) {
@@ -815,7 +826,6 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, int dtype, 
   // 32 experts and a shared one of 3 x 4096 x 3072: 475 -> 425 us, 53: 432 -> 416, 32: 441 -> 417; 24, with two such tiles, 383
   // and 386).  Without one, weights that the last-level cache holds gain too (3 x 1024 x 768, 4 of 32, 17 tokens 43.9 -> 41.5);
   // those from memory come faster spread over all (3 x 4096 x 3072, 17 tokens 347, 360 in shares; 64: 383, 390).
-  ExpertArgs b = a;
   b.together = a.slots > a.top || (int64_t)a.E * a.w_expert * (dtype == ZP_BF16 ? 2 : 4) < 320ll << 20;
 #define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, b)
 #define ZP_EXPERT_ROWS(T)                            \
@@ -974,17 +984,20 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
   ZP_REQUIRE(aligned16(x) && aligned16(w) && aligned16(w_shared) && aligned16(out) && aligned16(tiles) &&
                  x_stride >= (K > K_shared ? K : K_shared) && out_stride >= (M > M_shared ? M : M_shared),
              "moe experts: unaligned or overlapping rows");
-  if (rows >= 128) {              // 31-bit byte offsets into x and into a block of W
+  bool staged = rows >= 128;
+  if (staged) {                   // 31-bit byte offsets into x and into a block of W
     const int64_t xr = up ? n : rows, kx = K > K_shared ? K : K_shared;
-    if (xr * x_stride * 2 >= (1ll << 31) || kx * 512 >= (1ll << 31)) {
+    staged = xr * x_stride * 2 < (1ll << 31) && kx * 512 < (1ll << 31);
+    // few rows per expert, whose tiles were of 64 rows once, are read where they lie
+    if (!staged && (rows != 128 || (int64_t)n * top > 48ll * E)) {
       zp_set_error("moe experts: %lld rows of %lld elements in one step", (long long)xr, (long long)x_stride);
       return ZP_EUNSUPPORTED;
     }
   }
   ExpertArgs a = {x, w, w_shared, out, sorted, tiles, ntiles, weights, n, E, top, top + shared, max_tiles, K, K_shared,
-                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false};
-  return up ? launch_experts<true>(a, rows, dtype, (hipStream_t)stream)
-            : launch_experts<false>(a, rows, dtype, (hipStream_t)stream);
+                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false, 0};
+  return up ? launch_experts<true>(a, rows, staged, dtype, (hipStream_t)stream)
+            : launch_experts<false>(a, rows, staged, dtype, (hipStream_t)stream);
 }
 
 extern "C" int zp_moe_gate_up(const void* x, const void* w, const void* w_shared, void* out, const int32_t* sorted,
