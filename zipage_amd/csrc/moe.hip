@@ -824,9 +824,14 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged
   }
   // The shared expert's tiles read the same weights: on one XCD, one after the other, they find them in its L2 (64 tokens of 3 of
   // 32 experts and a shared one of 3 x 4096 x 3072: 475 -> 425 us, 53: 432 -> 416, 32: 441 -> 417; 24, with two such tiles, 383
-  // and 386).  Without one, weights that the last-level cache holds gain too (3 x 1024 x 768, 4 of 32, 17 tokens 43.9 -> 41.5);
-  // those from memory come faster spread over all (3 x 4096 x 3072, 17 tokens 347, 360 in shares; 64: 383, 390).
-  b.together = a.slots > a.top || (int64_t)a.E * a.w_expert * (dtype == ZP_BF16 ? 2 : 4) < 320ll << 20;
+  // and 386; tiles of 32, 100 tokens 536 -> 529, 170 563 -> 552; fp32, 64 tokens 994 -> 811, 128 1391 -> 1107, tiles of 64, 200 1944 -> 1813,
+  // 4000 12 510 -> 12 170).  Without one, weights that the last-level cache holds gain too (3 x 1024 x 768, 4 of 32, 17 tokens 43.9 -> 41.5; fp32
+  // 61 -> 52); those from memory come as fast or faster spread over all (3 x 4096 x 3072, 17 tokens 347, 360 in shares; 64: 383, 390).  The
+  // line lies low: launches of 256 MB are 10 to 15 % faster in shares, of 384 to 640 MB 6 % faster to 3 % slower, of 768 to 1280 MB 1 % faster to 2 %
+  // slower.  Tiles of 64 in bf16, of many tokens over hundreds of experts, stay spread: 16 500 tokens of 1 of 512 and a shared one, 3 x 1024 x 768
+  // 858 us, 883 in shares, 3 x 768 x 320 without one 285 and 306 (but 3 x 512 x 256 185 and 168).
+  b.together = (dtype == ZP_F32 || rows <= 32) &&
+               (a.slots > a.top || (int64_t)a.E * a.w_expert * (dtype == ZP_BF16 ? 2 : 4) < 320ll << 20);
 #define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, b)
 #define ZP_EXPERT_ROWS(T)                            \
   do {                                               \
