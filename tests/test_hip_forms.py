@@ -229,12 +229,22 @@ def test_experts_among_xcds(dev, n, width, E, top, ff, act):
     test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act)
 
 
-# 17 to 48 rows on average whose tokens lie so far apart that the staged form cannot address them: tiles of 128 in two parts, which are both
-# there, and where the second has one row
-@pytest.mark.parametrize("n,E,top,shared_ff", [(85, 5, 1, 0), (240, 5, 1, 96), (65, 2, 1, 0), (194, 6, 1, 32)])
+# Tiles of 64 rows, staged where tiles and 256 rows of W make 128 workgroups: both products, the first alone (exactly as many), neither;
+# averages of 17 to 48, experts of more than one tile; contractions that leave each remainder of what the loop takes
+@pytest.mark.parametrize("n,width,E,top,ff", [(600, 1056, 32, 1, 544), (1000, 992, 32, 1, 512), (816, 768, 48, 1, 352), (700, 1088, 64, 2, 544),
+                                              (272, 2048, 16, 1, 1056), (272, 1024, 16, 1, 512)])
+@pytest.mark.parametrize("act", ["clamped", "silu"])
+def test_experts_staged_in_tiles_of_64(dev, n, width, E, top, ff, act):
+    from zipage_amd import _lib
+    assert _lib.size("zp_moe_tile_rows", n, E, top, 0) == 64
+    test_experts_by_rows_and_contraction(dev, n, width, E, top, ff, act)
+
+
+# tokens that lie so far apart that the staged form cannot address them are read where they lie
+@pytest.mark.parametrize("n,E,top,shared_ff", [(160, 8, 1, 0), (384, 8, 1, 96), (200, 9, 1, 0), (60, 8, 4, 32)])
 def test_experts_of_tokens_far_apart(dev, n, E, top, shared_ff):
     from zipage_amd.layers import Experts
-    W, ff = 544, 96
+    W, ff = 544, 2048
     m = Experts(W, E, top, ff, 7.0, shared_ff=shared_ff or None)
     m.random(BF16, dev, torch.Generator(device=dev).manual_seed(1))
     ids = (torch.arange(n * top, device=dev) % (E - 1)).to(torch.int32).view(n, top)

@@ -381,7 +381,6 @@ struct ExpertArgs {
   float limit, limit_shared;
   int split;              // parts in which expert_tiles_kernel takes a tile
   bool together;          // expert_rows_kernel: an XCD takes a contiguous share of the launch, see launch_experts
-  int halves;             // expert_rows_kernel: 1 where tiles are of 128 rows and it takes them in two parts
 };
 
 // ZP_GATE_CLAMPED: w g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
@@ -421,14 +420,8 @@ __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int at = a.together ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int tile = at % a.max_tiles, cb = at / a.max_tiles;
-  if (tile >> a.halves >= *a.ntiles) return;
-  int4 t = *(const int4*)(a.tiles + (int64_t)(tile >> a.halves) * 4);
-  if constexpr (MT == 4) {
-    const int before = (tile & a.halves) * 64;
-    t.y += before;
-    t.z = min(t.z - before, 64);
-    if (t.z <= 0) return;
-  }
+  if (tile >= *a.ntiles) return;
+  const int4 t = *(const int4*)(a.tiles + (int64_t)tile * 4);
   const bool shared = t.x == a.E;
   const int wtiles = (shared ? a.M_shared : a.M) / 16 * (UP ? 2 : 1), K = shared ? a.K_shared : a.K;
   const int w0 = cb * kRowsW;
@@ -791,13 +784,13 @@ __global__ __launch_bounds__(256, HALVES == 2 ? 1 : 2) void expert_tiles_kernel(
   }
 }
 
-// staged: tokens through LDS, tiles of 128 and 256 rows
+// staged: tokens through LDS, tiles of 64 (see tile_rows), 128 and 256 rows
 template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged, int dtype, hipStream_t st) {
   if (staged) {
     const int Mx = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
     const bool big = rows == kBigRows && a.K >= kBigContraction;
     ExpertArgs b = a;
-    b.split = big ? 1 : rows / 128;
+    b.split = big || rows < 128 ? 1 : rows / 128;
     const int64_t grid = (int64_t)((b.max_tiles * b.split + 7) / 8) * 8 * ((Mx + 16 * kBlockW - 1) / (16 * kBlockW));
     const void* const fn = big ? (const void*)expert_tiles_kernel<UP, 2, 8> : (const void*)expert_tiles_kernel<UP, 1, 8>;
     const int smem = big ? 4 * 32 * 1024 : 3 * 16 * 1024;
@@ -812,10 +805,8 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
   ExpertArgs b = a;
-  b.halves = rows == 128;
-  b.max_tiles <<= b.halves;
-  const auto grid_of = [&](int tiles_w) { return (int64_t)b.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
-  const bool wide = rows == 16 && dtype == ZP_BF16 && b.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
+  const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
+  const bool wide = rows == 16 && dtype == ZP_BF16 && a.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
                     (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
   const int64_t grid = (grid_of(wide ? kWideW : kNarrowW) + 7) / 8 * 8;      // shares of eight XCDs; behind the last tile of W nothing is done
   if (grid >= (1ll << 31)) {
@@ -848,17 +839,20 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged
   return ZP_OK;
 }
 
-// Rows per tile: enough for the average expert.  From 17 rows of bf16 on tokens go through LDS: read by every wave for itself, 64
-// rows take more lines of the L1 than the weights that they meet (tiles of 128 and, before, of 64: 3 of 32 experts and a shared
-// one of 3 x 4096 x 3072, 200 tokens 490 and 542 us, 256 496 and 673, 480 515 and 694; of 3 x 1024 x 768, 200 51 and 60, 480 53
-// and 68; 8 of 128 of 3 x 2048 x 768, 320 tokens 234 and 261).  With up to 16, tiles of 32 lose up to 4 % without a shared expert
-// (100 tokens of 4 of 32, 437 and 453) and win up to 9 % with one, whose tile of 128 rows starts a second round of workgroups (96
-// tokens 512 and 470).  Launches of that form address x in 31 bits, so many tokens over many experts stay with tiles of 64.
-constexpr int kMostStaged = 16384;
+// Rows per tile: enough for the average expert.  bf16 tiles of 64 go through LDS as those of 128 do, where that makes workgroups for half of
+// the CUs: read by every wave for itself, 64 rows take more lines of the L1 than the weights that they meet.  Staged and direct, us of whole
+// layers: 3 of 32 experts and a shared one of 3 x 4096 x 3072, 200 tokens 480 and 533, 256 482 and 650, 480 493 and 683; of 3 x 1024 x 768, 200 40 and
+// 54, 480 45 and 61; 8 of 128 of 3 x 2048 x 768, 320 tokens 226 and 251; 2 of 8 and a shared one of 3 x 4096 x 14 336, 180 tokens 623 and 1133.
+// Of 1710 random products (1 to 256 experts, contractions of 32 to 14 336) those of 128 workgroups and more took 0.75 times as long staged, 23 in a
+// thousand of them more than 2 % longer, 13 % at most (just above a round of 256); of those below, more than half were slower, up to 1.7 times
+// (4 experts and a shared one of 3 x 4096 x 256, 96 tokens, the layer 48 and 33).  Tiles of 128 from 17 rows on do as well where they are staged, but
+// leave the direct form with parts that mostly are not there (up to 15 % of small layers).  With up to 16 rows, tiles of 32 lose up to 4 % without
+// a shared expert (100 tokens of 4 of 32, 437 and 453).  The staged form addresses x in 31 bits; rows too far apart are read where they lie.
+constexpr int kStagedGroups = 128;
 int tile_rows(int n, int E, int top, int dtype) {
   const int64_t avg = ((int64_t)n * top + E - 1) / E;
   if (dtype == ZP_BF16 && avg > 512) return kBigRows;
-  if (dtype == ZP_BF16 && (avg > 48 || (avg > 16 && n <= kMostStaged))) return 128;
+  if (dtype == ZP_BF16 && avg > 48) return 128;
   return avg <= 8 ? 16 : (avg <= 16 ? 32 : 64);       // a second tile reads an expert's weights again
 }
 int tile_bound(int n, int E, int top, int shared, int rows) {
@@ -989,18 +983,20 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
   ZP_REQUIRE(aligned16(x) && aligned16(w) && aligned16(w_shared) && aligned16(out) && aligned16(tiles) &&
                  x_stride >= (K > K_shared ? K : K_shared) && out_stride >= (M > M_shared ? M : M_shared),
              "moe experts: unaligned or overlapping rows");
-  bool staged = rows >= 128;
+  bool staged = rows >= 64 && dtype == ZP_BF16;
   if (staged) {                   // 31-bit byte offsets into x and into a block of W
     const int64_t xr = up ? n : rows, kx = K > K_shared ? K : K_shared;
     staged = xr * x_stride * 2 < (1ll << 31) && kx * 512 < (1ll << 31);
-    // few rows per expert, whose tiles were of 64 rows once, are read where they lie
-    if (!staged && (rows != 128 || (int64_t)n * top > 48ll * E)) {
+    if (rows == 64) {
+      const int64_t of_w = std::max(M, shared ? M_shared : 0) * (up ? 2ll : 1ll), with = E + (shared ? (n + 63) / 64 : 0);
+      staged = staged && with * of_w >= kStagedGroups * 16 * kBlockW;
+    } else if (!staged) {
       zp_set_error("moe experts: %lld rows of %lld elements in one step", (long long)xr, (long long)x_stride);
       return ZP_EUNSUPPORTED;
     }
   }
   ExpertArgs a = {x, w, w_shared, out, sorted, tiles, ntiles, weights, n, E, top, top + shared, max_tiles, K, K_shared,
-                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false, 0};
+                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false};
   return up ? launch_experts<true>(a, rows, staged, dtype, (hipStream_t)stream)
             : launch_experts<false>(a, rows, staged, dtype, (hipStream_t)stream);
 }
