@@ -380,7 +380,6 @@ struct ExpertArgs {
   int act;
   float limit, limit_shared;
   int split;              // parts in which expert_tiles_kernel takes a tile
-  bool together;          // expert_rows_kernel: an XCD takes a contiguous share of the launch, see launch_experts
 };
 
 // ZP_GATE_CLAMPED: w g sigmoid(1.702 g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
@@ -413,12 +412,13 @@ template <typename T> __device__ __forceinline__ float gated(int act, float w, f
 constexpr int kNarrowW = 4, kWideW = 8;                // 16-row tiles of W
 constexpr int kWideGrid = 1280, kWideTiles = 40, kWideRows = 6;    // workgroups, token tiles and average rows from which on
                                                                    // 128 rows of W are better
-template <typename T, int MT, bool UP, int kRowsW>
+// TOGETHER: an XCD takes a contiguous share of the launch, see launch_experts
+template <typename T, int MT, bool UP, int kRowsW, bool TOGETHER>
 __global__ __launch_bounds__(256) void expert_rows_kernel(ExpertArgs a) {
   __shared__ __align__(16) float part[4][kRowsW * MT * 256];
   const int lane = threadIdx.x & 63, l16 = lane & 15, g = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int at = a.together ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  const uint32_t at = TOGETHER ? (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3) : blockIdx.x;
   const int tile = at % a.max_tiles, cb = at / a.max_tiles;
   if (tile >= *a.ntiles) return;
   const int4 t = *(const int4*)(a.tiles + (int64_t)tile * 4);
@@ -804,7 +804,6 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged
     return ZP_OK;
   }
   const int Mw = (a.M > a.M_shared ? a.M : a.M_shared) * (UP ? 2 : 1);
-  ExpertArgs b = a;
   const auto grid_of = [&](int tiles_w) { return (int64_t)a.max_tiles * ((Mw + 16 * tiles_w - 1) / (16 * tiles_w)); };
   const bool wide = rows == 16 && dtype == ZP_BF16 && a.max_tiles >= kWideTiles && grid_of(kWideW) >= kWideGrid &&
                     (int64_t)a.n * a.top >= (int64_t)kWideRows * a.E;
@@ -821,9 +820,16 @@ template <bool UP> int launch_experts(const ExpertArgs& a, int rows, bool staged
   // line lies low: launches of 256 MB are 10 to 15 % faster in shares, of 384 to 640 MB 6 % faster to 3 % slower, of 768 to 1280 MB 1 % faster to 2 %
   // slower.  Tiles of 64 in bf16, of many tokens over hundreds of experts, stay spread: 16 500 tokens of 1 of 512 and a shared one, 3 x 1024 x 768
   // 858 us, 883 in shares, 3 x 768 x 320 without one 285 and 306 (but 3 x 512 x 256 185 and 168).
-  b.together = (dtype == ZP_F32 || rows <= 32) &&
+  // A share of fewer than eight column blocks would be a part of one, and some XCD's tiles ones that are not there (up to 256 columns, 48 experts, 91
+  // tokens, 64 x 4096 10.8 us, 15.7 in shares; fp32, 135 tokens, 256 x 2048 33 and 45).  The two orders are kernels of their own: what the choice
+  // cost small launches was more than it gave them (2 of 3 x 256 x 2048, 48 tokens, down 12.8 us, 14.5).
+  const bool together = (dtype == ZP_F32 || rows <= 32) && Mw > 7 * 16 * kNarrowW &&
                (a.slots > a.top || (int64_t)a.E * a.w_expert * (dtype == ZP_BF16 ? 2 : 4) < 320ll << 20);
-#define ZP_EXPERTS(T, MT, KW) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW>), dim3((unsigned)grid), dim3(256), 0, st, b)
+#define ZP_EXPERTS(T, MT, KW)                                                                                               \
+  do {                                                                                                                      \
+    if (together) hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW, true>), dim3((unsigned)grid), dim3(256), 0, st, a); \
+    else hipLaunchKernelGGL((expert_rows_kernel<T, MT, UP, KW, false>), dim3((unsigned)grid), dim3(256), 0, st, a);         \
+  } while (0)
 #define ZP_EXPERT_ROWS(T)                            \
   do {                                               \
     if (rows == 16) ZP_EXPERTS(T, 1, kNarrowW);      \
@@ -996,7 +1002,7 @@ static int experts(bool up, const void* x, const void* w, const void* w_shared, 
     }
   }
   ExpertArgs a = {x, w, w_shared, out, sorted, tiles, ntiles, weights, n, E, top, top + shared, max_tiles, K, K_shared,
-                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1, false};
+                  M, shared ? M_shared : 0, x_stride, out_stride, (int64_t)M * K * (up ? 2 : 1), act, limit, limit_shared, 1};
   return up ? launch_experts<true>(a, rows, staged, dtype, (hipStream_t)stream)
             : launch_experts<false>(a, rows, staged, dtype, (hipStream_t)stream);
 }
