@@ -207,6 +207,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
   }
   if (c < cw) {
     float* const dst = c < dk ? qs + c : (c < 2 * dk ? ks + c - dk : vs + c - 2 * dk);
+    if (cnt > 0)
 #pragma unroll
     for (int t = 0; t < kBlock; ++t) {
       float2 y = {0.f, 0.f};
@@ -262,10 +263,10 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     }
   }
   __syncthreads();
-  // ---- A and P: a wave 32 channels, a lane one token's of them.  Keys go down the tokens, from lane to lane, and decay on the way:
+  // ---- A and P: a wave 32 channels (of fewer than 128, some of the distances too), a lane one token's of them.  Keys go down the tokens, from lane to lane, and decay on the way:
   // after d moves a lane has k_s with the decays behind s, s = t - d, for A[t, s] and P[t, s], and the last lane what the state gets of
   // k_s.  One comes in before the first token, and once it has reached a lane, that has the decays up to it.
-  const int waves = dk / 32, row_at = (lane & 15) * ld + wave * 32 + (lane >> 4) * 4;
+  const int waves = dk / 32, mine = wave & (waves - 1), from = wave & -waves, row_at = (lane & 15) * ld + mine * 32 + (lane >> 4) * 4;
   float* const oU = to + 6 * kBlock * dk + half * kBlock * dv;
   float* const oSmall = to + 6 * kBlock * dk + 2 * kBlock * dv;
   auto put_small = [&](int i, const f32x4& v) {
@@ -288,8 +289,15 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) y[u] = mfma_bf16(l[i], r[u][j], y[u]);
   };
-  f32x4 y[2];                                  // A and P, distances 4 u + lane / 16 in element u
-  if (wave < waves) {
+  f32x4 y[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};       // A and P, distances 4 u + lane / 16 in element u
+  if (cnt == 0) {                              // a second block without tokens leaves the SIMDs to the first (beside zeros for keys and queries)
+    if (waves < 4) __syncthreads();
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+      *(f32x4*)(gs + row_at + 16 * p) = f32x4{0.f, 0.f, 0.f, 0.f};
+      if ((lane & 15) == 15) *(f32x4*)(decays + mine * 32 + 16 * p + (lane >> 4) * 4) = f32x4{1.f, 1.f, 1.f, 1.f};
+    }
+  } else {
     float k[8], q[8], g[8], x[8];              // of this lane's own elements, all three, which nobody else reads
 #pragma unroll
     for (int p = 0; p < 2; ++p) {
@@ -297,12 +305,14 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) k[4 * p + e] = kp[e], q[4 * p + e] = qp[e], g[4 * p + e] = gp[e], x[4 * p + e] = kp[e];
     }
+    if (waves < 4) __syncthreads();            // others read them too
     auto put = [](float* at, const float (&v)[8]) {
       *(f32x4*)at = f32x4{v[0], v[1], v[2], v[3]};
       *(f32x4*)(at + 16) = f32x4{v[4], v[5], v[6], v[7]};
     };
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
+    for (int u = 0; u < 4; ++u) {              // those before its first only move, and behind its last nothing does
+      if (u >= from + waves) continue;
       float sa[4], sp[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -311,6 +321,7 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
 #pragma unroll
           for (int i = 0; i < 8; ++i) x[i] = before_or_one(x[i]) * g[i];
         if (d > 1) to_next_token(x, g);
+        if (u < from) continue;
         if ((lane & 15) == 15) put(gs + row_at - d * ld, x);
         sa[j] = sp[j] = 0.f;
 #pragma unroll
@@ -319,22 +330,26 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
           sp[j] += x[i] * q[i];
         }
       }
+      if (u < from) continue;
       y[0][u] = sums_of_groups(sa);
       y[1][u] = sums_of_groups(sp);
     }
-    if (wave > 0)
+    if (from + waves == 4) {
+      to_next_token(x, g);                     // the decays up to the lane's token
+      if ((lane & 15) == 15) put(decays + mine * 32 + (lane >> 4) * 4, x);
 #pragma unroll
-      for (int u = 0; u < 2; ++u) *(f32x4*)(As + (((wave - 1) * 2 + u) * 64 + lane) * 4) = y[u];
-    to_next_token(x, g);                       // the decays up to the lane's token
-    if ((lane & 15) == 15) put(decays + wave * 32 + (lane >> 4) * 4, x);
-#pragma unroll
-    for (int i = 0; i < 8; ++i) k[i] *= x[i], q[i] *= x[i];
-    put(ks + row_at, k);
-    put(qs + row_at, q);
+      for (int i = 0; i < 8; ++i) k[i] *= x[i], q[i] *= x[i];
+      put(ks + row_at, k);
+      put(qs + row_at, q);
+    }
   }
+  if (wave > 0)
+#pragma unroll
+    for (int u = 0; u < 2; ++u) *(f32x4*)(As + (((wave - 1) * 2 + u) * 64 + lane) * 4) = y[u];
   __syncthreads();
   if (wave == 0) {
-    for (int j = 1; j < waves; ++j)
+#pragma unroll
+    for (int j = 1; j < 4; ++j)
 #pragma unroll
       for (int u = 0; u < 2; ++u) y[u] += *(const f32x4*)(As + (((j - 1) * 2 + u) * 64 + lane) * 4);
     asm volatile("" ::: "memory");             // the parts are read before rows of A and P lie there
@@ -371,8 +386,13 @@ __global__ __launch_bounds__(512, 4) void delta_prepare_kernel(RunArgs ra) {
     const bool key = tid < dk;
     const int c = key ? tid : tid - dk;
     const float* const column = (key ? ks : vs) + c;
+    if (cnt > 0) {
 #pragma unroll
-    for (int t = 0; t < kBlock; ++t) substitute(t, beta[t] * column[t * ld]);
+      for (int t = 0; t < kBlock; ++t) substitute(t, beta[t] * column[t * ld]);
+    } else {
+#pragma unroll
+      for (int t = 0; t < kBlock; ++t) w[t] = 0.f;
+    }
     if (key) {
       const float D = other_decays[c], by = half ? 1.f : D;
       if (!half) oSmall[4 * kPairFloats + c] = decays[c] * D;
