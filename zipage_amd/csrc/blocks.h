@@ -183,22 +183,21 @@ __device__ __forceinline__ int64_t block_slot(int row0, const Segment& sg, int s
 }
 
 // ------------------------------------------------------------------ runs in pieces
-// A head walks its blocks one after the other, 2.4 us each, and a few heads leave most CUs idle.
-// The state behind a piece of a run is (what the piece keeps) * (the state before it) + what the piece adds to none, so few
-// heads walk their runs in pieces side by side:
+// A head walks its blocks one after the other, 2.4 us each, and a few heads leave most CUs idle.  The state behind a piece of a
+// run is (what the piece keeps) * (the state before it) + what the piece adds to none, so few heads walk their runs in pieces
+// side by side:
 //
 //   sums     what each piece but the last adds and keeps: nothing waits for a state
 //   states   the states between pieces, from the first to the last
 //   blocks   as without pieces, each from its state on
 //
 // Workgroups fill a CU, so pieces are as short as 256 of them (and kLeastPiece blocks) and the chain of states between them
-// allow.  Where the sums and the two
-// launches cost more than what is saved, runs stay whole (PieceCost): a block of the sums takes 0.3 of one with rows (0.8 for the
-// delta rule), the launches 19 us (17 for the delta rule, whose blocks are the longer ones), states of the delta rule 4.3 us a
-// piece (matrix memory, 8 heads, a prompt of 155 tokens: whole 41.8 us, in pieces 42.8; linear attention, 32 heads, 200
-// tokens: 53, 46).  Whole scans: linear attention, 32 heads of 128,
-// 4 prompts of 500 to 2048 tokens 374 -> 287 us; 16 heads, 8 prompts of 2048, retention 429 -> 332 and matrix memory 369
-// -> 285; retention, a prompt of 700 126 -> 45; delta rule, 32 heads, a prompt of 2048 477 -> 269 (now 227), two of about 1250 384 -> 314 (262).
+// allow.  Where the sums and the two launches cost more than what is saved, runs stay whole (PieceCost): a block of the sums takes
+// 0.3 of one with rows (0.8 for the delta rule), the launches 19 us (17 for the delta rule), states of the delta rule 4.3 us a piece,
+// reckoned as 5.7 (matrix memory, 8 heads, a prompt of 155 tokens: whole 41.8 us, in pieces 42.8; linear attention, 32 heads, 200
+// tokens: 53, 46).  Whole scans, before pieces and now: linear attention, 32 heads of 128, 4 prompts of 500 to 2048 tokens 374 and 287 us; 16
+// heads, 8 prompts of 2048, retention 429 and 332, matrix memory 369 and 285; retention, a prompt of 700 126 and 45; delta rule, 32 heads, a
+// prompt of 2048 477 and 217, two of about 1250 384 and 238.
 constexpr int kPieceGroups = 256, kPieceStates = 384, kLeastPiece = 4;
 struct Pieces {
   int blocks = 0, most = 1;      // of a piece, 0: runs are whole; pieces of the longest run at most
