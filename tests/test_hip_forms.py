@@ -793,7 +793,7 @@ def _run_segments(dev, counts):
 
 
 # Blocks of 16 tokens go in pairs: one block, a second one of one token to all, a third; channels that forget little, some that
-# leave the range of a reciprocal within a block, and all of them.  Low-rank products of ranks that share a step of 32 columns, that
+# forget everything within a block, and all of them.  Low-rank products of ranks that share a step of 32 columns, that
 # fill the most that the kernels make, and that are left to the library.
 @pytest.mark.parametrize("bias,spread", [(-3.0, 1.0), (-2.0, 6.0), (12.0, 1.0)])
 @pytest.mark.parametrize("H,G,D,V,taps,ranks", [(2, 1, 128, 128, 4, (128, 128)), (3, 3, 64, 64, 2, (40, 72)), (2, 1, 32, 96, 8, (8, 8)),

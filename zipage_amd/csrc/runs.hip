@@ -421,8 +421,9 @@ __global__ __launch_bounds__(64 * tile_waves(MAPS), 2) void run_tiles_kernel(Til
 // wide ones there is room for the exponentials, and for 128 value columns (16 x 16, those of a head of 128 did not pay).
 // Rows go from memory into LDS without passing through registers, one load at a time between the products: eight in a row
 // held a wave for 870 cycles a tile.  Queries and the first keys are asked for together.
-// Bound by the vector issue (300 of 3390 cycles a tile and SIMD pair are waits) at the clock that the power limit leaves
-// (1.9 GHz); a tenth of the time a CU has one workgroup or none.  Heads of 128, 32 over 8 of keys and values, 8 prompts of
+// Of the cycles of a launch that turns its queries (window of 1024 below, 629 000 at 2.0 to 2.3 GHz) the vector units issue in 44 % and
+// the matrix cores are busy in 35 %; its waves, two per SIMD, wait in 35 % of theirs, and a tenth of the time a CU has one workgroup
+// or none.  Heads of 128, 32 over 8 of keys and values, 8 prompts of
 // 2048 tokens: window of 1024 309 -> 278 us, all keys 371 -> 327; one prompt 52 -> 44, of 300 tokens 12.7 -> 10.6; heads of
 // 64: 198 -> 181, 240 -> 216, 33 -> 29, 9.0 -> 8.2; causal with weights of 17 bits 452 -> 448, one prompt of 300 14.7 -> 12.5.
 // Tried: eight waves of two heads that share their rows, in turns at the matrix cores and the vector units (322 us: a wave
