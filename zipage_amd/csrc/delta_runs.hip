@@ -54,7 +54,7 @@ __device__ __forceinline__ void to_next_token(float (&x)[8], const float (&g)[8]
 #ifdef __HIP_DEVICE_COMPILE__
 #define ZP_MOVED(i, by) "v_mul_f32_dpp %" #i ", %" #i ", %" #by " row_shr:1 row_mask:0xf bank_mask:0xf\n\t"
   asm("s_nop 1\n\t" ZP_MOVED(0, 8) ZP_MOVED(1, 9) ZP_MOVED(2, 10) ZP_MOVED(3, 11) ZP_MOVED(4, 12) ZP_MOVED(5, 13) ZP_MOVED(6, 14) ZP_MOVED(7, 15)
-      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
+      : "+&v"(x[0]), "+&v"(x[1]), "+&v"(x[2]), "+&v"(x[3]), "+&v"(x[4]), "+&v"(x[5]), "+&v"(x[6]), "+&v"(x[7])
       : "v"(g[0]), "v"(g[1]), "v"(g[2]), "v"(g[3]), "v"(g[4]), "v"(g[5]), "v"(g[6]), "v"(g[7]));
 #undef ZP_MOVED
 #endif
